@@ -1,4 +1,5 @@
-"""ctypes binding of libcbk_hip.so (the C ABI declared in include/cbk.h).
+"""Bindings of libcbk_hip.so: ctypes for the C ABI declared in include/cbk.h, and the extension
+module `_native` with the operators that are called per token.
 
 The library is the only compute path of this package: if it is not built, every operator
 raises instead of falling back to PyTorch."""
@@ -61,6 +62,24 @@ def lib():
             raise CbkError(f"ABI version {L.cbk_abi_version()} != 1")
         _lib = L
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The extension module with the operators (`_native.so`); raises if it has not been built."""
+    global _native
+    if _native is None:
+        lib()
+        try:
+            from . import _native as mod
+        except ImportError as e:
+            raise CbkError("cobalt_amd/_native.so is missing or does not load: build it with "
+                           f"`python -m cobalt_amd.build`. There is no PyTorch fallback. ({e})") from e
+        mod.set_error(CbkError)
+        _native = mod
+    return _native
 
 
 def check(rc: int, what: str):

@@ -1,4 +1,5 @@
-"""Builds libcbk_hip.so (the C-ABI HIP library) in-tree with hipcc for gfx950."""
+"""Builds libcbk_hip.so (the C-ABI HIP library, hipcc for gfx950) and _native.so (its operators for
+Python) in-tree."""
 import os
 import subprocess
 import sys
@@ -39,6 +40,30 @@ def build_lib(verbose=True, extra=()):
     return LIB
 
 
+NATIVE = os.path.join(HERE, "_native.so")
+
+
+def build_native(verbose=True):
+    """_native.so: the operators of ops.py as a CPython extension on torch's C++ API (host code,
+    linked to libcbk_hip.so beside it)."""
+    import sysconfig
+    from torch.utils import cpp_extension as X
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    inc = list(X.include_paths()) + [sysconfig.get_paths()["include"], os.path.join(rocm, "include")]
+    libs = X.library_paths()
+    cmd = (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
+           + [a for d in inc for a in ("-isystem", d)] + [os.path.join(CSRC, "cbk_torch.cpp"), "-o", NATIVE]
+           + ["-L" + d for d in libs + [HERE]] + ["-Wl,-rpath," + d for d in libs] + ["-Wl,-rpath,$ORIGIN"]
+           + ["-lcbk_hip", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-lamdhip64",
+              "-L" + os.path.join(rocm, "lib")])
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    out = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if out.returncode != 0:
+        raise RuntimeError("g++ failed on cbk_torch.cpp:\n" + out.stdout)
+    return NATIVE
+
+
 BENCH_LIB = os.path.join(HERE, "libcbk_bench.so")
 
 
@@ -56,5 +81,6 @@ def build_bench_lib(verbose=True):
 
 if __name__ == "__main__":
     build_lib()
+    build_native()
     build_bench_lib()
-    print("built", LIB, BENCH_LIB)
+    print("built", LIB, NATIVE, BENCH_LIB)

@@ -201,6 +201,29 @@ static DMat dense4_view(const DMat& m, uint8_t* ws, const Transient& t) {
   return d;
 }
 
+// Room for the part sums of cbk_gemv at M rows (see cbk_workspace_bytes); no other use of a
+// workspace in decode.  A q|k|v matrix runs as its ranges, one launch for all of them.
+static size_t decode_workspace(const DMat& m, int M) {
+  if (M < 1 || M > 16) return 0;
+  if (family_of(m.layout) == FAM_SPARSE) return gemv_stream_workspace(m, M);
+  if (m.cs_rows != 3) return gemv_fast_takes(m, 1) ? gemv_fast_workspace(m, M) : 0;
+  int lo[3], hi[3], row[3];
+  const int nr = fused_ranges(m, lo, hi, row);
+  size_t need = 0;
+  for (int i = 0; i < nr; ++i) {
+    const DMat r = row_range(m, lo[i], hi[i], row[i]);
+    if (gemv_fast_takes(r, 1)) need += gemv_fast_workspace(r, M);
+  }
+  return need;
+}
+
+// What cbk_gemv uses of a workspace at M rows, without what only the prefill kernel needs: the
+// operators that know they will decode ask for this.
+size_t decode_workspace_bytes(const cbk_desc* in, int M) {
+  DMat m;
+  return to_dmat(in, &m, false) ? 0 : decode_workspace(m, M);
+}
+
 }  // namespace cbk
 
 using namespace cbk;
@@ -244,13 +267,13 @@ size_t cbk_workspace_bytes(const cbk_desc* in, int M) {
   DMat m;
   if (to_dmat(in, &m, false)) return 0;
   if (family_of(m.layout) == FAM_SPARSE) {                          // cbk_gemm / cbk_linear above 16 rows: see Transient
-    if (M <= 16) return gemv_stream_workspace(m, M);                // part sums of long rows split by columns, else none
+    if (M <= 16) return decode_workspace(m, M);                     // part sums of long rows split by columns, else none
     if (!sparse_repackable(m)) return 0;
     const Transient t = transient_dense4(m);
     return t.end + gemm_big_workspace(dense4_view(m, nullptr, t), M);
   }
   // the most any of the three entry points asks for (cbk_gemm runs the prefill kernel at any M)
-  size_t need = (M >= 1 && M <= 16 && gemv_fast_takes(m, 1)) ? gemv_fast_workspace(m, M) : 0;
+  size_t need = decode_workspace(m, M);
   if (gemm_big_takes(m, M)) {
     const size_t b = gemm_big_workspace(m, M);
     return need > b ? need : b;
@@ -360,7 +383,7 @@ int cbk_gemv_batch(int n, const cbk_desc* descs, const void* const* xs, const in
   size_t off = 0;
   for (int i = 0; i < n; ++i) {
     // (cbk_gemv uses a workspace where it has one and computes the same bits without)
-    const size_t need = cbk_workspace_bytes(descs + i, M);
+    const size_t need = decode_workspace_bytes(descs + i, M);
     const bool room = need && workspace && off + need <= workspace_bytes;
     int rc = cbk_gemv(descs + i, xs[i], x_dtype, M, ldxs[i], ys[i], y_dtype, ldys[i], biases ? biases[i] : nullptr,
                       room ? (uint8_t*)workspace + off : nullptr, room ? need : 0, stream);

@@ -1,0 +1,312 @@
+// The operators of cobalt_amd/ops.py as a CPython extension: argument checks, output and scratch
+// allocation and the call into libcbk_hip.so.
+//
+// Why native: a decode call is one or two kernels of 5 to 20 us.  Through ctypes (descriptor built
+// field by field, workspace looked up, a dozen conversions) the host needed 16.7 us for one
+// CobaltLinear call of a 1024 x 4096 matrix at one row, three times its kernel, and about 20 us per
+// gemv_batch: eager decode ran at the speed of the interpreter.
+//
+// Scratch comes from torch's caching allocator on every call (about a microsecond, stream-ordered,
+// private to the graph when the call is captured) instead of a buffer kept per stream: calls from
+// several threads on one stream cannot meet in it, and it goes back when the call has been enqueued.
+#include <Python.h>
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <ATen/ATen.h>
+#include <ATen/EmptyTensor.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/InlineDeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include "../../include/cbk.h"
+
+namespace cbk {
+size_t decode_workspace_bytes(const cbk_desc*, int M);              // cbk_api.hip
+}
+
+namespace {
+
+PyObject* g_error = nullptr;                                        // cobalt_amd._lib.CbkError
+
+// One packed matrix: the image and where its arrays are in it.  The addresses are formed per
+// call, so a tensor whose storage is exchanged (module.to()) is followed.
+struct Matrix {
+  PyObject_HEAD
+  at::Tensor* blob;
+  cbk_desc d;
+  int64_t off[5];                                                   // data, row_off, scale, zero, col_scale; -1: none
+};
+
+void matrix_dealloc(PyObject* o) {
+  delete ((Matrix*)o)->blob;
+  Py_TYPE(o)->tp_free(o);
+}
+
+PyObject* matrix_new(PyTypeObject* t, PyObject* args, PyObject*) {
+  PyObject *blob, *offs, *ints;
+  if (!PyArg_ParseTuple(args, "OO!O!", &blob, &PyTuple_Type, &offs, &PyTuple_Type, &ints)) return nullptr;
+  if (!THPVariable_Check(blob) || PyTuple_GET_SIZE(offs) != 5 || PyTuple_GET_SIZE(ints) != 10) {
+    PyErr_SetString(PyExc_TypeError, "Matrix(blob tensor, 5 offsets, 10 integers)");
+    return nullptr;
+  }
+  Matrix* m = (Matrix*)t->tp_alloc(t, 0);
+  if (!m) return nullptr;
+  m->blob = new at::Tensor(THPVariable_Unpack(blob));
+  long long v[10];
+  for (int i = 0; i < 10; ++i) v[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(ints, i));
+  for (int i = 0; i < 5; ++i) m->off[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(offs, i));
+  if (PyErr_Occurred()) { Py_DECREF(m); return nullptr; }
+  m->d = cbk_desc{};
+  m->d.K = (int32_t)v[0]; m->d.N = (int32_t)v[1]; m->d.layout = (int32_t)v[2]; m->d.bits = (int32_t)v[3];
+  m->d.group = (int32_t)v[4]; m->d.keep = (int32_t)v[5]; m->d.cs_rows = (int32_t)v[6];
+  m->d.cs_split0 = (int32_t)v[7]; m->d.cs_split1 = (int32_t)v[8]; m->d.flags = (int32_t)v[9];
+  return (PyObject*)m;
+}
+
+PyTypeObject MatrixType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+cbk_desc desc_of(const Matrix* m) {
+  cbk_desc d = m->d;
+  const uint8_t* base = (const uint8_t*)m->blob->const_data_ptr();
+  auto at_off = [&](int i) -> const void* { return m->off[i] < 0 ? nullptr : base + m->off[i]; };
+  d.data = at_off(0); d.row_off = at_off(1); d.scale = at_off(2); d.zero = at_off(3); d.col_scale = at_off(4);
+  return d;
+}
+
+struct Fail {};                                                     // a Python exception has been set
+
+[[noreturn]] void fail(PyObject* type, const std::string& msg) {
+  PyErr_SetString(type, msg.c_str());
+  throw Fail{};
+}
+
+void check(int rc, const char* what) {
+  if (rc) fail(g_error, std::string(what) + " failed: " + cbk_strerror(rc) + " (status " + std::to_string(rc) + ")");
+}
+
+const Matrix* as_matrix(PyObject* o) {
+  if (Py_TYPE(o) != &MatrixType) fail(PyExc_TypeError, "a native matrix handle is expected");
+  return (const Matrix*)o;
+}
+
+// None -> undefined tensor
+at::Tensor as_tensor(PyObject* o, const char* what) {
+  if (o == Py_None) return at::Tensor();
+  if (!THPVariable_Check(o)) fail(PyExc_TypeError, std::string(what) + " must be a tensor");
+  return THPVariable_Unpack(o);
+}
+
+int dtype_code(at::ScalarType t) {
+  switch (t) {
+    case at::kFloat: return CBK_F32;
+    case at::kHalf: return CBK_F16;
+    case at::kBFloat16: return CBK_BF16T;
+    default:
+      fail(PyExc_TypeError, std::string("unsupported dtype ") + c10::toString(t) +
+                                "; the layer takes float16 / bfloat16 activations");
+  }
+}
+
+at::ScalarType out_type(PyObject* o, const at::Tensor& x) {
+  if (o == Py_None) return x.scalar_type();
+  if (!THPDtype_Check(o)) fail(PyExc_TypeError, "out_dtype must be a torch.dtype");
+  return ((THPDtype*)o)->scalar_type;
+}
+
+void require_gpu(const Matrix* m, const at::Tensor& x, const at::Tensor& bias) {
+  if (!m->blob->is_cuda())
+    fail(g_error, "the packed matrix must live on the GPU (PackedMatrix.to('cuda')); this package has no CPU execution path");
+  for (const at::Tensor* t : {&x, &bias})
+    if (t->defined() && t->device() != m->blob->device())
+      fail(g_error, "tensor on " + t->device().str() + ", packed matrix on " + m->blob->device().str());
+}
+
+// x as [M, N] rows of unit stride the kernels can read with 16-byte loads (a copy if it is not)
+struct Rows { at::Tensor keep; const void* p; int64_t M, ld; };
+Rows rows_of(const at::Tensor& x, int64_t N) {
+  if (x.dim() < 1 || x.size(-1) != N)
+    fail(PyExc_ValueError, "x has " + std::to_string(x.dim() ? x.size(-1) : 1) + " input features, the matrix has N=" + std::to_string(N));
+  Rows r;
+  r.M = x.numel() / N;
+  const bool flat = x.is_contiguous();
+  if (flat || (x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0 && x.stride(0) >= N)) {
+    r.p = x.const_data_ptr();
+    r.ld = flat || r.M <= 1 ? N : x.stride(0);
+    if (((uintptr_t)r.p & 15) == 0) return r;
+  }
+  at::Tensor t = x.reshape({-1, N});
+  if (t.stride(1) != 1 || (t.size(0) > 1 && (t.stride(0) % 8 || t.stride(0) < N)) || ((uintptr_t)t.const_data_ptr() & 15))
+    t = t.clone(at::MemoryFormat::Contiguous);
+  r.keep = t;
+  r.p = t.const_data_ptr();
+  r.ld = r.M > 1 ? t.stride(0) : N;
+  return r;
+}
+
+at::Tensor out_for(const at::Tensor& x, int64_t K, at::ScalarType dt) {
+  c10::SmallVector<int64_t, 6> shape(x.sizes().begin(), x.sizes().end());
+  shape.back() = K;
+  return at::empty(shape, x.options().dtype(dt).requires_grad(false).memory_format(at::MemoryFormat::Contiguous));
+}
+
+at::Tensor scratch(const at::Tensor& like, size_t bytes) {
+  return bytes ? at::empty({(int64_t)bytes}, like.options().dtype(at::kByte)) : at::Tensor();
+}
+
+void* stream_of(const at::Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+template <class F>
+PyObject* guarded(F&& f) {
+  HANDLE_TH_ERRORS
+  try {
+    at::AutoDispatchBelowADInplaceOrView no_autograd;
+    return f();
+  } catch (const Fail&) {
+    return nullptr;
+  }
+  END_HANDLE_TH_ERRORS
+}
+
+bool arity(Py_ssize_t n, Py_ssize_t want) {
+  if (n == want) return true;
+  PyErr_SetString(PyExc_TypeError, "wrong number of arguments");
+  return false;
+}
+
+// matmul(entry 0 gemv / 1 gemm / 2 linear, matrix, x, bias, out_dtype, workspace) -> y
+PyObject* py_matmul(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (!arity(n, 6)) return nullptr;
+  return guarded([&]() -> PyObject* {
+    const long entry = PyLong_AsLong(a[0]);
+    const Matrix* m = as_matrix(a[1]);
+    const at::Tensor x = as_tensor(a[2], "x");
+    at::Tensor bias = as_tensor(a[3], "bias");
+    at::Tensor ws = as_tensor(a[5], "workspace");
+    if (!x.defined()) fail(PyExc_TypeError, "x must be a tensor");
+    require_gpu(m, x, bias);
+    const cbk_desc d = desc_of(m);
+    const Rows r = rows_of(x, d.N);
+    const at::ScalarType odt = out_type(a[4], x);
+    at::Tensor y = out_for(x, d.K, odt);
+    if (r.M == 0) return THPVariable_Wrap(y);
+    const int xdt = dtype_code(x.scalar_type()), ydt = dtype_code(odt), M = (int)r.M;
+    if (bias.defined() && bias.scalar_type() != odt) bias = bias.to(odt);
+    const c10::DeviceGuard guard(x.device());
+    if (!ws.defined())
+      ws = scratch(x, entry == 0 || (entry == 2 && M <= 8) ? cbk::decode_workspace_bytes(&d, M) : cbk_workspace_bytes(&d, M));
+    auto fn = entry == 0 ? cbk_gemv : entry == 1 ? cbk_gemm : cbk_linear;
+    check(fn(&d, r.p, xdt, M, r.ld, y.mutable_data_ptr(), ydt, d.K, bias.defined() ? bias.const_data_ptr() : nullptr,
+             ws.defined() ? ws.mutable_data_ptr() : nullptr, ws.defined() ? ws.nbytes() : 0, stream_of(x)),
+          entry == 0 ? "cbk_gemv" : entry == 1 ? "cbk_gemm" : "cbk_linear");
+    return THPVariable_Wrap(y);
+  });
+}
+
+// linear_act(matrix, x, act, bias, out_dtype) -> y
+PyObject* py_linear_act(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (!arity(n, 5)) return nullptr;
+  return guarded([&]() -> PyObject* {
+    const Matrix* m = as_matrix(a[0]);
+    const at::Tensor x = as_tensor(a[1], "x");
+    const int act = (int)PyLong_AsLong(a[2]);
+    at::Tensor bias = as_tensor(a[3], "bias");
+    if (!x.defined()) fail(PyExc_TypeError, "x must be a tensor");
+    require_gpu(m, x, bias);
+    const cbk_desc d = desc_of(m);
+    const Rows r = rows_of(x, d.N);
+    if (d.K % 2) fail(PyExc_ValueError, "a gate/up matrix has an even number of rows");
+    const at::ScalarType odt = out_type(a[4], x);
+    at::Tensor y = out_for(x, d.K / 2, odt);
+    if (r.M == 0) return THPVariable_Wrap(y);
+    const int xdt = dtype_code(x.scalar_type()), ydt = dtype_code(odt), M = (int)r.M;
+    if (bias.defined() && bias.scalar_type() != odt) bias = bias.to(odt);
+    const c10::DeviceGuard guard(x.device());
+    const at::Tensor ws = scratch(x, cbk_linear_act_workspace_bytes(&d, M, ydt));
+    check(cbk_linear_act(&d, r.p, xdt, M, r.ld, y.mutable_data_ptr(), ydt, d.K / 2,
+                         bias.defined() ? bias.const_data_ptr() : nullptr, act,
+                         ws.defined() ? ws.mutable_data_ptr() : nullptr, ws.defined() ? ws.nbytes() : 0, stream_of(x)),
+          "cbk_linear_act");
+    return THPVariable_Wrap(y);
+  });
+}
+
+// gemv_batch(list of matrices, list of x, list of biases or None, out_dtype) -> list of y
+PyObject* py_gemv_batch(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  if (!arity(nargs, 4)) return nullptr;
+  return guarded([&]() -> PyObject* {
+    if (!PyList_Check(a[0]) || !PyList_Check(a[1]) || !(a[2] == Py_None || PyList_Check(a[2])))
+      fail(PyExc_TypeError, "lists of matrices, activations and biases are expected");
+    const Py_ssize_t n = PyList_GET_SIZE(a[0]);
+    if (n < 1 || PyList_GET_SIZE(a[1]) < n || (a[2] != Py_None && PyList_GET_SIZE(a[2]) < n))
+      fail(PyExc_ValueError, "one activation (and bias) per matrix is expected");
+    if (n > 8) check(CBK_ERR_SHAPE, "cbk_gemv_batch");
+    cbk_desc d[8];
+    at::Tensor x[8], y[8], b[8];
+    Rows r[8];
+    const void *xp[8], *bp[8];
+    void* yp[8];
+    int64_t ldx[8], ldy[8];
+    at::ScalarType odt = at::kHalf;
+    size_t need = 0;
+    for (Py_ssize_t i = 0; i < n; ++i) {
+      const Matrix* m = as_matrix(PyList_GET_ITEM(a[0], i));
+      x[i] = as_tensor(PyList_GET_ITEM(a[1], i), "x");
+      if (!x[i].defined()) fail(PyExc_TypeError, "x must be a tensor");
+      if (a[2] != Py_None) b[i] = as_tensor(PyList_GET_ITEM(a[2], i), "bias");
+      require_gpu(m, x[i], b[i]);
+      d[i] = desc_of(m);
+      r[i] = rows_of(x[i], d[i].N);
+      if (i == 0) odt = out_type(a[3], x[0]);
+      if (r[i].M != r[0].M || x[i].scalar_type() != x[0].scalar_type())
+        fail(PyExc_ValueError, "all activations of a batch share the row count and the dtype");
+      y[i] = out_for(x[i], d[i].K, odt);
+      if (b[i].defined() && b[i].scalar_type() != odt) b[i] = b[i].to(odt);
+      xp[i] = r[i].p; ldx[i] = r[i].ld;
+      yp[i] = y[i].mutable_data_ptr(); ldy[i] = d[i].K;
+      bp[i] = b[i].defined() ? b[i].const_data_ptr() : nullptr;
+      need += cbk::decode_workspace_bytes(&d[i], (int)r[0].M);
+    }
+    const c10::DeviceGuard guard(x[0].device());
+    const at::Tensor ws = scratch(x[0], need);
+    check(cbk_gemv_batch((int)n, d, xp, ldx, dtype_code(x[0].scalar_type()), (int)r[0].M, yp, ldy, dtype_code(odt), bp,
+                         ws.defined() ? ws.mutable_data_ptr() : nullptr, need, stream_of(x[0])),
+          "cbk_gemv_batch");
+    PyObject* out = PyList_New(n);
+    if (!out) throw Fail{};
+    for (Py_ssize_t i = 0; i < n; ++i) PyList_SET_ITEM(out, i, THPVariable_Wrap(y[i]));
+    return out;
+  });
+}
+
+PyObject* py_set_error(PyObject*, PyObject* e) {
+  Py_INCREF(e);
+  Py_XSETREF(g_error, e);
+  Py_RETURN_NONE;
+}
+
+PyMethodDef methods[] = {
+    {"matmul", (PyCFunction)(void (*)())py_matmul, METH_FASTCALL, nullptr},
+    {"linear_act", (PyCFunction)(void (*)())py_linear_act, METH_FASTCALL, nullptr},
+    {"gemv_batch", (PyCFunction)(void (*)())py_gemv_batch, METH_FASTCALL, nullptr},
+    {"set_error", py_set_error, METH_O, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__native(void) {
+  MatrixType.tp_name = "cobalt_amd._native.Matrix";
+  MatrixType.tp_basicsize = sizeof(Matrix);
+  MatrixType.tp_dealloc = matrix_dealloc;
+  MatrixType.tp_flags = Py_TPFLAGS_DEFAULT;
+  MatrixType.tp_new = matrix_new;
+  if (PyType_Ready(&MatrixType) < 0) return nullptr;
+  PyObject* m = PyModule_Create(&module_def);
+  if (!m) return nullptr;
+  g_error = PyExc_RuntimeError;
+  Py_INCREF(g_error);
+  Py_INCREF(&MatrixType);
+  if (PyModule_AddObject(m, "Matrix", (PyObject*)&MatrixType) < 0) return nullptr;
+  return m;
+}

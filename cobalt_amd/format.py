@@ -202,6 +202,31 @@ class PackedMatrix:
     flags: int = 0
     meta: dict = field(default_factory=dict)
 
+    def __setattr__(self, name, value):
+        object.__setattr__(self, name, value)
+        object.__setattr__(self, "_handle", None)                  # the native handle below describes the old values
+
+    def __getstate__(self):                                        # copies and pickles make a handle of their own
+        return {k: v for k, v in self.__dict__.items() if k != "_handle"}
+
+    def __setstate__(self, state):
+        for k, v in state.items():
+            setattr(self, k, v)
+
+    def native(self):
+        """The handle the extension module takes for this matrix, made at the first call after a
+        field was set."""
+        h = self._handle
+        if h is None:
+            from . import _lib
+            o = self.offs
+            h = _lib.native().Matrix(self.blob, (o["data"], o.get("row_off", -1), o["scale"], o["zero"],
+                                                 o["col_scale"] if self.cs_rows else -1),
+                                     (self.K, self.N, self.layout, self.bits, self.group, self.keep or 0, self.cs_rows,
+                                      self.cs_splits[0], self.cs_splits[1], self.flags))
+            object.__setattr__(self, "_handle", h)
+        return h
+
     @property
     def G(self) -> int:
         return self.N // self.group

@@ -188,7 +188,10 @@ class CobaltLinear(nn.Module):
         self._backend = backend
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return ops.linear(self._pm(), x, self.bias)
+        pm = self._pm_cache
+        if pm is None or pm.blob is not self._buffers["blob"]:
+            pm = self._pm()
+        return ops.linear(pm, x, self.bias)
 
     def forward_act(self, x: torch.Tensor, act: str) -> torch.Tensor:
         """For a gate/up matrix (rows 2i gate, 2i+1 up): act(gate(x)) * up(x), [.., out_features / 2]."""
