@@ -2,6 +2,7 @@
 // No allocation, no host synchronisation; the only global state is the scratch array of
 // cbk_gemm_static and its per-device address.
 #include <mutex>
+#include "cbk_internal.h"
 #include "cbk_device.h"
 
 namespace cbk {
@@ -24,7 +25,8 @@ int launch_gemm_big(const DMat&, const void*, int, int, int64_t, void*, int, int
                     hipStream_t, bool halves = false);
 size_t gemm_big_workspace(const DMat&, int M);
 int launch_pack(const DMat&, const void* mask, const void* q, const void* scale, const void* zero, int zero_f16,
-                int fix_zero, int* status, hipStream_t);
+                int fix_zero, int* status, const PackExtra* extra, hipStream_t);
+int launch_repack_dense4(const DMat& sparse, const DMat& dense4, hipStream_t);
 int launch_unpack(const DMat&, void* q, void* mask, hipStream_t);
 // The 256 x 256 tile kernel takes every call of the fixed-stride layouts: below 256 activation
 // rows part of its token tile is padding, and it is still several times faster than the
@@ -167,7 +169,7 @@ static int check_io(const void* x, int xdt, int M, int64_t ldx, const void* y, i
 // matrix-core kernel of its own.  A prefill call re-packs it, in the caller's workspace and for
 // the duration of the call, as the dense 4-bit layout in tiled order (pruned columns hold the
 // zero point, so every weight dequantises to the same value) and runs the prefill kernel on that:
-// two small kernels (image -> codes and bitmap, codes -> rows) in front of the matrix product.
+// one small kernel in front of the matrix product.
 // A pruned column of the dense image stores the zero point as its code, so this needs every zero
 // point to be a 4-bit code itself (CBK_FLAG_ZERO_ON_GRID: the host cannot look), and a fixed row
 // stride cannot carry row-fused column scales; such matrices, and calls without the workspace,
@@ -176,15 +178,13 @@ static inline bool sparse_repackable(const DMat& m) {
   return m.cs_rows <= 1 && (m.flags & CBK_FLAG_ZERO_ON_GRID) != 0;
 }
 struct Transient {
-  size_t q, mask, data, scale, zero, end;   // byte offsets in the workspace, 256-byte aligned
+  size_t data, scale, zero, end;            // byte offsets in the workspace, 256-byte aligned
 };
 static Transient transient_dense4(const DMat& m) {
   const size_t K16 = ((size_t)m.K + 15) / 16 * 16, stride = (size_t)m.N / 2;
   auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
   Transient t;
-  t.q = 0;
-  t.mask = up((size_t)m.K * m.N);
-  t.data = t.mask + up((size_t)m.K * (m.N / 8));
+  t.data = 0;
   t.scale = t.data + up(K16 * stride + 512);
   t.zero = t.scale + up(K16 * m.G * 2);
   t.end = t.zero + up(K16 * m.G);
@@ -222,6 +222,20 @@ static size_t decode_workspace(const DMat& m, int M) {
 size_t decode_workspace_bytes(const cbk_desc* in, int M) {
   DMat m;
   return to_dmat(in, &m, false) ? 0 : decode_workspace(m, M);
+}
+
+int pack_image(const cbk_desc* dst, const void* mask_bits, const void* q, const void* scale, const void* zero,
+               int zero_dtype, int fix_zero, int* status, const PackExtra* extra, void* stream) {
+  DMat m;
+  const int rc = to_dmat(dst, &m, true);
+  if (rc) return rc;
+  if (!q || !scale || !zero) return CBK_ERR_NULL;
+  if (zero_dtype != CBK_F16 && zero_dtype != CBK_U8) return CBK_ERR_DTYPE;
+  if (((uintptr_t)q & 15) || ((uintptr_t)mask_bits & 3) || ((uintptr_t)scale & 1) || ((uintptr_t)status & 3) ||
+      (zero_dtype == CBK_F16 && ((uintptr_t)zero & 1)))
+    return CBK_ERR_ALIGN;
+  return launch_pack(m, mask_bits, q, scale, zero, zero_dtype == CBK_F16, fix_zero != 0, status, extra,
+                     (hipStream_t)stream);
 }
 
 }  // namespace cbk
@@ -306,15 +320,7 @@ int cbk_dequant(const cbk_desc* in, int row0, int nrows, int with_col_scale, voi
 
 int cbk_pack(const cbk_desc* dst, const void* mask_bits, const void* q, const void* scale, const void* zero,
              int zero_dtype, int fix_zero, int* status, void* stream) {
-  DMat m;
-  const int rc = to_dmat(dst, &m, true);
-  if (rc) return rc;
-  if (!q || !scale || !zero) return CBK_ERR_NULL;
-  if (zero_dtype != CBK_F16 && zero_dtype != CBK_U8) return CBK_ERR_DTYPE;
-  if (((uintptr_t)q & 15) || ((uintptr_t)mask_bits & 3) || ((uintptr_t)scale & 1) || ((uintptr_t)status & 3) ||
-      (zero_dtype == CBK_F16 && ((uintptr_t)zero & 1)))
-    return CBK_ERR_ALIGN;
-  return launch_pack(m, mask_bits, q, scale, zero, zero_dtype == CBK_F16, fix_zero != 0, status, (hipStream_t)stream);
+  return pack_image(dst, mask_bits, q, scale, zero, zero_dtype, fix_zero, status, nullptr, stream);
 }
 
 int cbk_unpack(const cbk_desc* in, void* q, void* mask_bits, void* stream) {
@@ -431,9 +437,7 @@ int cbk_gemm(const cbk_desc* in, const void* x, int x_dtype, int M, int64_t ldx,
     }
     uint8_t* ws = (uint8_t*)workspace;
     const DMat d = dense4_view(m, ws, t);
-    rc = launch_unpack(m, ws + t.q, ws + t.mask, (hipStream_t)stream);
-    if (rc) return rc;
-    rc = launch_pack(d, ws + t.mask, ws + t.q, m.scale, m.zero, 0, 0, nullptr, (hipStream_t)stream);
+    rc = launch_repack_dense4(m, d, (hipStream_t)stream);
     if (rc) return rc;
     return launch_gemm_big(d, x, x_dtype, M, ldx, y, y_dtype, ldy, bias, ws + t.end, workspace_bytes - t.end,
                            (hipStream_t)stream);

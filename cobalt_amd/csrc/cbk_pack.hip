@@ -3,11 +3,16 @@
 // docs/FORMAT.md:83-122) and of the two bit-stream layouts of this library (include/cbk.h);
 // the destination is either the row-major order or the 16-row tiled order.
 //
-// One thread packs 256 columns of one row (128 at the end of a row whose length is an odd
-// multiple of 128): 8 mask blocks, whose code bits end on a byte boundary whatever the code
-// width and the survivors per block, so no two threads share a byte.  HBM-bound byte work:
-// it reads K*N code bytes and K*N/8 mask bytes and writes the packed rows once.
-#include "cbk_device.h"
+// A workgroup packs a slab of 4096 columns of sixteen rows (one tile of the tiled order).  A thread
+// takes a 32-column block at a time: survivors are moved together by byte permutes from a table
+// indexed by the mask byte, narrowed to the code width, and or-ed into the slab's image in LDS; the
+// image leaves in whole 16-byte units.  A slab's codes start on a 16-byte unit whatever the code
+// width and the survivors per block (128 blocks: 16 * keep * bits bytes).  Bound: reading K*N code
+// bytes.  One thread per 256 columns with byte stores, the form before, took 147 us for
+// 14336 x 4096 (plus 5 us to clear the destination, every byte of which is written here).
+#include <atomic>
+#include "cbk_internal.h"
+#include "cbk_octet.h"
 
 namespace cbk {
 
@@ -19,28 +24,12 @@ struct PackArgs {
   uint8_t* data;
   uint16_t* oscale;
   uint8_t* ozero;
-  int K, N, G, group, bits, keep, fam, tiled, zero_f16, fix_zero;
+  int K, N, G, group, keep, tiled, zero_f16, fix_zero;
   uint32_t stride;
-};
-
-__device__ inline uint8_t* dst_byte(const PackArgs& a, int k, uint32_t o) {
-  if (a.tiled) return a.data + (size_t)(k >> 4) * 16 * a.stride + ((size_t)(o >> 4) * 16 + (k & 15)) * 16 + (o & 15);
-  return a.data + (size_t)k * a.stride + o;
-}
-
-// LSB-first bit stream writer onto consecutive row bytes starting at byte `o`
-struct BitSink {
-  uint64_t acc = 0;
-  int n = 0;
-  uint32_t o;
-  __device__ inline void put(const PackArgs& a, int k, uint32_t code, int bits) {
-    acc |= (uint64_t)(code & ((1u << bits) - 1u)) << n;            // never into the neighbouring code
-    n += bits;
-    while (n >= 8) { *dst_byte(a, k, o++) = (uint8_t)acc; acc >>= 8; n -= 8; }
-  }
-  __device__ inline void flush(const PackArgs& a, int k) {
-    if (n > 0) { *dst_byte(a, k, o++) = (uint8_t)acc; acc = 0; n = 0; }
-  }
+  int krows;               // rows of the image: K, or K padded to a multiple of 16 in the tiled order
+  uint32_t tail;           // readable bytes behind the last row, zeroed
+  int* status;             // see below, or nullptr
+  PackExtra extra;         // all zero: rows, scale and zero point only
 };
 
 // The quantisation of one group as it is stored: the RAW one, or, when the RAW zero point is off
@@ -59,30 +48,32 @@ struct GroupQ {
   }
 };
 
-__device__ inline GroupQ group_quant(const PackArgs& a, int k, int g, const uint8_t* qrow_full, const uint8_t* mrow_full) {
+// sz: the group's scale and, in the upper half, its zero point as given.  q, m: codes and mask of one 32-column block of the group; the blocks of a group are in consecutive
+// lanes (four or two of them, all active), which agree on the hull by lane exchanges.
+__device__ inline GroupQ group_quant(const PackArgs& a, float nl, uint32_t sz, const uint32_t (&q)[8], uint32_t m) {
   GroupQ r;
-  const size_t gi = (size_t)k * a.G + g;
-  const float nl = (float)((1u << a.bits) - 1u);
-  r.s_out = a.scale[gi];
+  r.s_out = (uint16_t)sz;
   r.s_raw = h2f(r.s_out);
-  int zi;
-  if (a.zero_f16) zi = (int)rintf(h2f(((const uint16_t*)a.zero)[gi]));
-  else zi = (int)((const uint8_t*)a.zero)[gi];
+  const int zi = a.zero_f16 ? (int)rintf(h2f((uint16_t)(sz >> 16))) : (int)(sz >> 16);
   r.z_raw = (float)zi;
   r.redo = a.fix_zero && (zi < 0 || zi > (int)nl);
   r.z_out = (uint32_t)zi & 0xffu;
   r.s_new = r.s_raw; r.z_new = r.z_raw;
   if (!r.redo) return r;
-  float vmin = 3.4028234663852886e38f, vmax = -3.4028234663852886e38f;
-  bool any = false;
-  for (int j = g * a.group; j < (g + 1) * a.group; ++j) {
-    const bool kept = mrow_full ? ((mrow_full[j >> 3] >> (j & 7)) & 1u) != 0 : true;
-    if (!kept) continue;
-    const float v = __fmul_rn((float)qrow_full[j] - r.z_raw, r.s_raw);
-    vmin = fminf(vmin, v); vmax = fmaxf(vmax, v); any = true;
+  constexpr float BIG = 3.4028234663852886e38f;
+  float vmin = BIG, vmax = -BIG;
+#pragma unroll
+  for (int j = 0; j < 32; ++j) {
+    const float v = __fmul_rn((float)((q[j >> 2] >> (8 * (j & 3))) & 0xFFu) - r.z_raw, r.s_raw);
+    const bool kept = (m >> j) & 1u;
+    vmin = kept ? fminf(vmin, v) : vmin;
+    vmax = kept ? fmaxf(vmax, v) : vmax;
   }
-  if (!any) vmin = vmax = 0.f;
-  vmin = fminf(vmin, 0.f); vmax = fmaxf(vmax, 0.f);
+  for (int o = 1; o < a.group >> 5; o <<= 1) {
+    vmin = fminf(vmin, __shfl_xor(vmin, o));
+    vmax = fmaxf(vmax, __shfl_xor(vmax, o));
+  }
+  vmin = fminf(vmin, 0.f); vmax = fmaxf(vmax, 0.f);                // (a group without survivors: 0 and 0)
   r.s_new = fmaxf(__fdiv_rn(__fsub_rn(vmax, vmin), nl), 1e-12f);
   r.z_new = fminf(fmaxf(rintf(__fdiv_rn(-vmin, r.s_new)), 0.f), nl);
   r.z_out = (uint32_t)r.z_new;
@@ -90,181 +81,378 @@ __device__ inline GroupQ group_quant(const PackArgs& a, int k, int g, const uint
   return r;
 }
 
+constexpr int PK_ROWS = 16, PK_COLS = 4096, PK_THREADS = 512;
+
+// permute selectors that move the survivors of eight bytes together: output byte i takes the i-th
+// survivor (zero past the last)
+__device__ inline uint2 compress_selectors(uint32_t mb) {
+  uint32_t lo = 0x0C0C0C0Cu, hi = 0x0C0C0C0Cu, r = 0;
+#pragma unroll
+  for (uint32_t p = 0; p < 8; ++p) {
+    if ((mb >> p) & 1u) {
+      const uint32_t sh = 8 * (r & 3u), put = (p ^ 0x0Cu) << sh;   // 0x0C -> p
+      if (r < 4) lo ^= put; else hi ^= put;
+      ++r;
+    }
+  }
+  return make_uint2(lo, hi);
+}
+
+// eight bytes holding codes of `bits` bits -> 8 * bits bits, first code lowest
+template <int bits>
+__device__ inline uint64_t narrow8(uint32_t lo, uint32_t hi) {
+  if (bits == 8) return (uint64_t)lo | ((uint64_t)hi << 32);
+  auto four = [&](uint32_t x) -> uint32_t {                         // four bytes -> 4 * bits bits
+    const uint32_t mask = ((1u << bits) - 1u) * 0x00010001u;
+    const uint32_t y = (x & mask) | (((x >> 8) & mask) << bits);    // pairs at bits 0 and 16
+    return (y & ((1u << (2 * bits)) - 1u)) | ((y >> 16) << (2 * bits));
+  };
+  return (uint64_t)four(lo) | ((uint64_t)four(hi) << (4 * bits));
+}
+
 // status[0] |= 1: a block without exactly `keep` survivors; |= 2: a dense layout had to store a zero
 // point above 2^bits - 1 at a pruned column (its low bits are stored; the column no longer
 // dequantises to 0); status[1] += groups re-derived
-__global__ __launch_bounds__(256) void pack_rows_kernel(PackArgs a, int* status) {
-  const int units = (a.N + 255) >> 8;
-  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (id >= (int64_t)a.K * units) return;
-  const int k = (int)(id / units), u = (int)(id % units);
-  const int c0 = u << 8, nb = (a.N - c0 >= 256 ? 256 : a.N - c0) >> 5;     // 8 or 4 blocks
-  const uint8_t* qfull = a.q + (size_t)k * a.N;
-  const uint8_t* mfull = a.mask ? a.mask + (size_t)k * (a.N >> 3) : nullptr;
-  const uint8_t* qrow = qfull + c0;
-  const uint8_t* mrow = mfull ? mfull + (c0 >> 3) : nullptr;
-  const float nl = (float)((1u << a.bits) - 1u);
-  BitSink sink;
-  if (a.fam == FAM_DENSE) sink.o = (uint32_t)(c0 >> 3) * a.bits;
-  else sink.o = (uint32_t)(a.N >> 3) + (uint32_t)(c0 >> 5) * a.keep * a.bits / 8;   // c0/32 is a multiple of 8
-  bool wrong = false, off_grid = false;
-  int fixed = 0, g_now = -1;
-  GroupQ gq;
-  for (int t = 0; t < nb; ++t) {
-    const int g = (c0 + 32 * t) / a.group;
-    if (g != g_now) {                                              // groups are 64 or 128 columns: never across units
-      g_now = g;
-      gq = group_quant(a, k, g, qfull, mfull);
-      fixed += gq.redo ? 1 : 0;
-      const size_t mi = a.tiled ? ((size_t)(k >> 4) * a.G + g) * 16 + (k & 15) : (size_t)k * a.G + g;
+template <int FAM, int BITS>
+__global__ __launch_bounds__(PK_THREADS) void pack_rows_kernel(PackArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint32_t img[];   // [PK_ROWS][code bytes of a slab (+ its BLK6 high plane)]
+  __shared__ uint2 lut[256];
+  __shared__ uint32_t tot[4];                                      // status bits, groups re-derived, largest zero, survivors
+  const int tid = threadIdx.x;
+  constexpr bool dense = FAM == FAM_DENSE, blk6 = FAM == FAM_BLK6;
+  if (tid < 256) lut[tid] = compress_selectors((uint32_t)tid);
+  if (tid < 4) tot[tid] = 0;
+  const int slabs = (a.N + PK_COLS - 1) / PK_COLS;
+  const int rt = blockIdx.x / slabs, c0 = (blockIdx.x % slabs) * PK_COLS, k0 = rt * PK_ROWS;
+  const int cols = a.N - c0 < PK_COLS ? a.N - c0 : PK_COLS, nb = cols >> 5;
+  constexpr int pb = blk6 ? 4 : BITS;                               // bits per code of the code plane
+  const int cb = (dense ? 32 : a.keep) * pb;                       // code bits of a block
+  const uint32_t plane = (uint32_t)a.N >> 3;
+  const uint32_t cbytes = ((uint32_t)nb * cb + 127) / 128 * 16;    // code bytes of the slab's rows, whole units
+  const uint32_t hbytes = blk6 ? (uint32_t)nb * 4u : 0u;
+  const uint32_t pitch = (cbytes + hbytes) >> 2;                   // dwords per row of the image
+  for (uint32_t i = tid; i < PK_ROWS * pitch; i += PK_THREADS) img[i] = 0;
+  __syncthreads();
+  const float nl = (float)((1u << BITS) - 1u);
+  const uint32_t over = ~((uint32_t)nl * 0x01010101u);             // bits that no code of this width has
+  uint32_t st = 0, fixed = 0, zmax = 0, surv = 0;
+  // codes, mask, scale and zero point of the next block are in flight while one is packed
+  struct In { uint4 qa, qb; uint32_t m, sz; };
+  const int items = (a.K - k0 < PK_ROWS ? a.K - k0 : PK_ROWS) * nb;  // (padding rows have no blocks)
+  auto load = [&](int it) -> In {
+    it = it < items ? it : items - 1;
+    const int k = k0 + it / nb, c = c0 + 32 * (it % nb);
+    const size_t gi = (size_t)k * a.G + (uint32_t)c / (uint32_t)a.group;
+    const uint8_t* qp = a.q + (size_t)k * a.N + c;
+    In x;
+    x.qa = *(const uint4*)qp; x.qb = *(const uint4*)(qp + 16);
+    x.m = a.mask ? *(const uint32_t*)(a.mask + (size_t)k * plane + (c >> 3)) : 0xffffffffu;
+    x.sz = (uint32_t)a.scale[gi] | ((a.zero_f16 ? (uint32_t)((const uint16_t*)a.zero)[gi] : (uint32_t)((const uint8_t*)a.zero)[gi]) << 16);
+    return x;
+  };
+  In nx = load(tid);
+  for (int it = tid; it < items; it += PK_THREADS) {
+    const In cur = nx;
+    nx = load(it + PK_THREADS);
+    const int row = it / nb, t = it % nb, k = k0 + row;
+    const int c = c0 + 32 * t, g = (uint32_t)c / (uint32_t)a.group;
+    uint32_t q[8] = {cur.qa.x, cur.qa.y, cur.qa.z, cur.qa.w, cur.qb.x, cur.qb.y, cur.qb.z, cur.qb.w};
+    const uint32_t m = cur.m;
+    surv += (uint32_t)__popc(m);
+    const GroupQ gq = group_quant(a, nl, cur.sz, q, m);
+    if (c % a.group == 0) {                                        // the group's first block stores its quantisation
+      const size_t mi = a.tiled ? ((size_t)rt * a.G + g) * 16 + row : (size_t)k * a.G + g;
       a.oscale[mi] = gq.s_out;
       a.ozero[mi] = (uint8_t)gq.z_out;
+      fixed += gq.redo ? 1u : 0u;
+      zmax = zmax > gq.z_out ? zmax : gq.z_out;
     }
-    const uint32_t m = mrow ? *(const uint32_t*)(mrow + 4 * t) : 0xffffffffu;
-    __attribute__((aligned(16))) uint8_t c[32];
-    *(uint4*)(c) = *(const uint4*)(qrow + 32 * t);
-    *(uint4*)(c + 16) = *(const uint4*)(qrow + 32 * t + 16);
-    if (a.fam == FAM_DENSE) {
-      if (m != 0xffffffffu && gq.z_out > (uint32_t)nl) off_grid = true;
+    uint32_t any = 0;
 #pragma unroll
-      for (int j = 0; j < 32; ++j) sink.put(a, k, ((m >> j) & 1u) ? gq.code(c[j], nl) : gq.z_out, a.bits);
+    for (int i = 0; i < 8; ++i) any |= q[i] & over;
+    if (gq.redo || any) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        uint32_t w = 0;
+        for (int e = 0; e < 4; ++e) w |= gq.code((q[i] >> (8 * e)) & 0xFFu, nl) << (8 * e);
+        q[i] = w;
+      }
+    }
+    uint32_t* dst = img + row * pitch;
+    if (dense) {
+      if (m != 0xffffffffu && gq.z_out > (uint32_t)nl) st |= 2u;
+      const uint32_t z4 = (gq.z_out & (uint32_t)nl) * 0x01010101u;
+      uint64_t w[4];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t kp = bits_to_bytes(m >> (4 * i)) * 0xFFu;
+        q[i] = (q[i] & kp) | (z4 & ~kp);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] = narrow8<pb>(q[2 * i], q[2 * i + 1]);
+      uint32_t* d = dst + t * pb;                                  // a block is pb whole dwords
+      if (pb == 8) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { d[2 * i] = (uint32_t)w[i]; d[2 * i + 1] = (uint32_t)(w[i] >> 32); }
+      } else if (pb == 4) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d[i] = (uint32_t)w[i];
+      } else if (pb == 3) {
+        const uint64_t x = w[0] | (w[1] << 24), y = w[2] | (w[3] << 24);     // 48 bits each
+        d[0] = (uint32_t)x; d[1] = (uint32_t)(x >> 32) | ((uint32_t)y << 16); d[2] = (uint32_t)(y >> 16);
+      } else {
+        d[0] = (uint32_t)w[0] | ((uint32_t)w[1] << 16); d[1] = (uint32_t)w[2] | ((uint32_t)w[3] << 16);
+      }
       continue;
     }
-    const uint32_t blk = (uint32_t)(c0 >> 5) + t;
+    if (__popc(m) != a.keep) st |= 1u;
+    // survivors of the block, at most `keep` of them, as one bit string of at most 128 bits
+    uint64_t s0 = 0, s1 = 0;
+    uint32_t hw = 0;
+    int r = 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) *dst_byte(a, k, blk * 4 + i) = (uint8_t)(m >> (8 * i));
-    if (__popc(m) != a.keep) wrong = true;
-    if (a.fam == FAM_BLK6) {                                       // low nibbles, then 2 high bits: even survivors in
-      uint32_t lo[2] = {0, 0}, hw = 0;                             // the low half of the word, odd ones in the high half
-      int i = 0;
-#pragma unroll
-      for (int j = 0; j < 32; ++j)
-        if (((m >> j) & 1u) && i < 16) {
-          const uint32_t cd = gq.code(c[j], nl);
-          lo[i >> 3] |= (cd & 0xF) << (4 * (i & 7));
-          hw |= ((cd >> 4) & 3) << (2 * (i >> 1) + 16 * (i & 1));
-          ++i;
+    for (int b = 0; b < 4; ++b) {
+      const uint32_t mb = (m >> (8 * b)) & 0xFFu;
+      const uint2 sel = lut[mb];
+      uint32_t lo = perm(q[2 * b + 1], q[2 * b], sel.x), hi = perm(q[2 * b + 1], q[2 * b], sel.y);
+      if (blk6) {                                                  // high bit pairs: even survivors from bit 0, odd ones from bit 16
+        for (int i = 0; i < 8; ++i) {
+          const uint32_t cd = ((i < 4 ? lo : hi) >> (8 * (i & 3))) & 0xFFu;
+          const int e = r + i;
+          if (e < 16) hw |= (cd >> 4) << (2 * (e >> 1) + 16 * (e & 1));
         }
+        lo &= 0x0F0F0F0Fu; hi &= 0x0F0F0F0Fu;
+      }
+      const uint64_t w = narrow8<pb>(lo, hi);
+      const int at = r * pb;
+      if (at < 64) { s0 |= w << at; if (at) s1 |= w >> (64 - at); }
+      else if (at < 128) s1 |= w << (at - 64);
+      r += __popc(mb);
+    }
+    if (cb < 64) { s0 &= (1ull << (cb & 63)) - 1ull; s1 = 0; }            // (too many survivors: an error, but never into the next block)
+    else if (cb < 128) s1 &= (1ull << (cb & 63)) - 1ull;
+    const uint32_t bit = (uint32_t)t * cb, sh = bit & 31u;
+    uint32_t* d = dst + (bit >> 5);
+    const uint32_t x[4] = {(uint32_t)s0, (uint32_t)(s0 >> 32), (uint32_t)s1, (uint32_t)(s1 >> 32)};
+    const int nd = (int)(sh + cb + 31) >> 5;
+    if ((cb & 31) == 0) {                                          // whole dwords: nobody shares them
 #pragma unroll
-      for (int b = 0; b < 8; ++b) *dst_byte(a, k, (uint32_t)(a.N >> 3) + blk * 8 + b) = (uint8_t)(lo[b >> 2] >> (8 * (b & 3)));
-#pragma unroll
-      for (int b = 0; b < 4; ++b) *dst_byte(a, k, (uint32_t)(a.N * 3 >> 3) + blk * 4 + b) = (uint8_t)(hw >> (8 * b));
+      for (int i = 0; i < 4; ++i)
+        if (i < nd) d[i] = x[i];
     } else {
-      int i = 0;
 #pragma unroll
-      for (int j = 0; j < 32; ++j)
-        if (((m >> j) & 1u) && i < a.keep) { sink.put(a, k, gq.code(c[j], nl), a.bits); ++i; }
-      for (; i < a.keep; ++i) sink.put(a, k, 0, a.bits);           // too few survivors: keep the stream aligned
+      for (int i = 0; i < 5; ++i) {
+        if (i >= nd) break;
+        const uint32_t lo = i < 4 ? x[i] : 0u, pre = i > 0 ? x[i - 1] : 0u;
+        const uint32_t v = sh ? (lo << sh) | (pre >> (32 - sh)) : lo;
+        if (v) atomicOr(d + i, v);
+      }
+    }
+    if (blk6) dst[(cbytes >> 2) + t] = hw;
+  }
+  __syncthreads();
+  // the image, unit by unit: consecutive threads write the rows of a unit (tiled: a 256-byte run) or the units of a row
+  auto unit_addr = [&](int row, uint32_t o) -> uint4* {            // o: byte offset in the row, a multiple of 16
+    return a.tiled ? (uint4*)(a.data + (size_t)rt * 16 * a.stride + (size_t)o * 16 + row * 16)
+                   : (uint4*)(a.data + (size_t)(k0 + row) * a.stride + o);
+  };
+  const int rows = a.krows - k0 < PK_ROWS ? a.krows - k0 : PK_ROWS;
+  auto put = [&](uint32_t units, uint32_t o0, auto&& get) {
+    for (uint32_t i = tid; i < PK_ROWS * units; i += PK_THREADS) {
+      const int row = a.tiled ? (int)(i & 15u) : (int)(i / units);
+      const uint32_t u = a.tiled ? i >> 4 : i % units;
+      if (row < rows) *unit_addr(row, o0 + u * 16) = get(row, u);
+    }
+  };
+  put(cbytes >> 4, (dense ? 0u : plane) + (uint32_t)(c0 >> 5) * (uint32_t)cb / 8,
+      [&](int row, uint32_t u) { return *(const uint4*)(img + row * pitch + 4 * u); });
+  if (blk6) put(hbytes >> 4, plane * 3u + (uint32_t)(c0 >> 3),
+                [&](int row, uint32_t u) { return *(const uint4*)(img + row * pitch + (cbytes >> 2) + 4 * u); });
+  if (!dense)
+    put((uint32_t)cols >> 7, (uint32_t)(c0 >> 3), [&](int row, uint32_t u) {
+      if (k0 + row >= a.K) return make_uint4(0, 0, 0, 0);
+      if (!a.mask) return make_uint4(~0u, ~0u, ~0u, ~0u);
+      const uint32_t* p = (const uint32_t*)(a.mask + (size_t)(k0 + row) * plane + (c0 >> 3)) + 4 * u;
+      return make_uint4(p[0], p[1], p[2], p[3]);
+    });
+  // padding rows have no groups of their own; the bytes behind the last row
+  if (c0 == 0 && k0 + PK_ROWS > a.K && a.tiled)
+    for (int i = tid; i < (k0 + PK_ROWS - a.K) * a.G; i += PK_THREADS) {
+      const size_t mi = ((size_t)rt * a.G + i % a.G) * 16 + (a.K - k0) + i / a.G;
+      a.oscale[mi] = 0;
+      a.ozero[mi] = 0;
+    }
+  if (blockIdx.x == 0 && tid < (int)(a.tail >> 4)) ((uint4*)(a.data + (size_t)a.krows * a.stride))[tid] = make_uint4(0, 0, 0, 0);
+  for (uint32_t i = blockIdx.x * (uint32_t)PK_THREADS + tid; i < a.extra.cs_units; i += gridDim.x * (uint32_t)PK_THREADS)
+    ((uint4*)a.extra.cs_dst)[i] = ((const uint4*)a.extra.cs_src)[i];
+  if (blockIdx.x == 0)
+    for (int i = 0; i < 4; ++i)
+      if (tid < (int)a.extra.gap_bytes[i]) a.extra.gap[i][tid] = 0;
+  if (a.status || a.extra.counts) {                                       // one update per workgroup
+    if (st) atomicOr(&tot[0], st);
+    if (fixed) atomicAdd(&tot[1], fixed);
+    if (a.extra.counts) { atomicMax(&tot[2], zmax); atomicAdd(&tot[3], surv); }
+    __syncthreads();
+    if (tid == 0) {
+      if (a.status && tot[0]) atomicOr(a.status, (int)tot[0]);
+      if (a.status && tot[1]) atomicAdd(a.status + 1, (int)tot[1]);
+      if (a.extra.counts) {
+        uint32_t* c = a.extra.counts + (blockIdx.x % PACK_SLOTS) * PACK_SLOT_WORDS;
+        if (tot[0]) atomicOr(c, tot[0]);
+        if (tot[1]) atomicAdd(c + 1, tot[1]);
+        atomicMax(c + 2, tot[2]);
+        atomicAdd(c + 3, tot[3]);
+      }
     }
   }
-  sink.flush(a, k);
-  if (status) {
-    if (wrong) atomicOr(status, 1);
-    if (off_grid) atomicOr(status, 2);
-    if (fixed) atomicAdd(status + 1, fixed);
-  }
-}
-
-__global__ __launch_bounds__(256) void pack_clear_kernel(uint4* p, size_t n16) {
-  const size_t id = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (id < n16) p[id] = make_uint4(0, 0, 0, 0);
-}
-
-static void clear16(void* p, size_t bytes, hipStream_t st) {
-  hipLaunchKernelGGL(pack_clear_kernel, dim3((unsigned)((bytes / 16 + 255) / 256)), dim3(256), 0, st, (uint4*)p, bytes / 16);
 }
 
 // ------------------------------------------------------------------ the way back: image -> RAW
 // Codes (0 at a pruned column of a bitmap or survivor-stream layout, the stored code, i.e. the
 // zero point, at a pruned column of a dense layout) and the keep bitmap of any layout.
-// Fixed-stride layouts: one thread per (row, 32-column block); survivor streams: one thread
-// per (row, group), as in the dequantiser.
+// A thread per eight columns.
+template <int FAM, int BITS>
 __global__ __launch_bounds__(256) void unpack_fixed_kernel(DMat m, uint8_t* q, uint8_t* mask) {
-  const int NB = m.N / BLOCK;
-  const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= (int64_t)m.K * NB) return;
-  const int k = (int)(gid / NB), t = (int)(gid % NB);
-  int c[32];
-  const uint32_t keep = decode_block32(m, row_view(m, k), t, c);
-  uint32_t w[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-    w[i] = (uint32_t)c[4 * i] | ((uint32_t)c[4 * i + 1] << 8) | ((uint32_t)c[4 * i + 2] << 16) | ((uint32_t)c[4 * i + 3] << 24);
-  uint4* dst = (uint4*)(q + (size_t)k * m.N + t * BLOCK);
-  dst[0] = make_uint4(w[0], w[1], w[2], w[3]);
-  dst[1] = make_uint4(w[4], w[5], w[6], w[7]);
-  if (mask) *(uint32_t*)(mask + (size_t)k * (m.N >> 3) + t * 4) = keep;
+  __shared__ uint2 lut[256 * OCT_LUT_LANES];
+  if (FAM != FAM_DENSE) { octet_table(lut); __syncthreads(); }
+  const uint32_t n8 = (uint32_t)m.N >> 3;
+  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int rt = (int)(id / n8);
+  const uint32_t j8 = (uint32_t)(id % n8);
+  const int k1 = rt * 16 + 16 < m.K ? rt * 16 + 16 : m.K;
+#pragma unroll 4
+  for (int k = rt * 16; k < k1; ++k) {
+    const Octet o = octet_fixed<FAM, BITS>(m, row_view(m, k), j8, lut);
+    *(uint2*)(q + (size_t)k * m.N + 8 * (size_t)j8) = make_uint2(o.lo, o.hi);
+    if (mask) mask[(size_t)k * n8 + j8] = (uint8_t)o.keep;
+  }
 }
 
-__global__ __launch_bounds__(256) void unpack_sparse_kernel(DMat m, uint8_t* q, uint8_t* mask) {
-  const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= (int64_t)m.K * m.G) return;
-  const int k = (int)(gid / m.G), g = (int)(gid % m.G);
-  const uint8_t* row = m.data + m.row_off[k];
-  const uint32_t* bm = (const uint32_t*)row;
-  const bool has_goff = m.layout != CBK_SPARSE4;
-  const int hdr = ((m.N >> 3) + (has_goff ? ((m.G * 2 + 15) & ~15) : 0) + 15) & ~15;
-  uint32_t off = 0;
-  if (has_goff) {
-    off = ((const uint16_t*)(row + (m.N >> 3)))[g];
-  } else {
-    for (int gg = 0; gg < g; ++gg) {
-      int c = 0;
-      for (int i = 0; i < 4; ++i) c += __popc(bm[gg * 4 + i]);
-      off += (uint32_t)(c + 1) >> 1;
+// Survivor streams, a workgroup per four rows.  DENSE4: instead of bytes, the same row as dense 4-bit
+// codes in tiled order (a pruned column holds its group's zero point), which is how a prefill call
+// re-packs such a matrix; one pass over the stream instead of one to bytes and one back.
+template <bool DENSE4>
+__global__ __launch_bounds__(256) void unpack_sparse_kernel(DMat m, uint8_t* q, uint8_t* mask, uint16_t* oscale,
+                                                            uint8_t* ozero, int summed) {
+  extern __shared__ uint32_t goff[];
+  __shared__ uint2 lut[256 * OCT_LUT_LANES];
+  octet_table(lut);
+  const uint32_t hdr = stream_header(m), n8 = (uint32_t)m.N >> 3;
+  const int k0 = blockIdx.x * 4;
+  for (int k = k0; k < k0 + 4; ++k) {
+    uint8_t* tile = q + (size_t)(k >> 4) * 16 * (m.N >> 1) + (k & 15) * 16;  // DENSE4 only
+    if (k >= m.K) {                                                 // (DENSE4: the padding rows of the last tile)
+      if (!DENSE4 || k >= ((m.K + 15) & ~15)) break;
+      for (uint32_t j8 = threadIdx.x; j8 < n8; j8 += 256) *(uint32_t*)(tile + (size_t)(j8 >> 2) * 256 + (j8 & 3u) * 4) = 0;
+      for (int g = threadIdx.x; g < m.G; g += 256) {
+        oscale[((size_t)(k >> 4) * m.G + g) * 16 + (k & 15)] = 0;
+        ozero[((size_t)(k >> 4) * m.G + g) * 16 + (k & 15)] = 0;
+      }
+      continue;
     }
-  }
-  const uint8_t* codes = row + hdr + off;
-  int nib = 0;
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t keep = bm[g * 4 + i];
-    uint32_t w[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) w[e] = 0;
-#pragma unroll
-    for (int p = 0; p < 32; ++p) {
-      if ((keep >> p) & 1u) {
-        const uint32_t by = codes[nib >> 1];
-        const uint32_t c = (nib & 1) ? (by >> 4) : (by & 0xFu);
-        ++nib;
-        w[p >> 2] |= c << (8 * (p & 3));
+    const uint8_t* row = m.data + m.row_off[k];
+    __syncthreads();                                                // the table; the offsets of the row before
+    if (summed) {
+      if (threadIdx.x < 64) stream_offsets(m, row, goff);
+      __syncthreads();
+    }
+    for (uint32_t j8 = threadIdx.x; j8 < n8; j8 += 256) {
+      const Octet o = octet_stream(m, row, hdr, summed ? goff : nullptr, j8, lut);
+      if (!DENSE4) {
+        *(uint2*)(q + (size_t)k * m.N + 8 * (size_t)j8) = make_uint2(o.lo, o.hi);
+        if (mask) mask[(size_t)k * n8 + j8] = (uint8_t)o.keep;
+        continue;
+      }
+      const uint32_t g = j8 >> 4;
+      const size_t mi = (size_t)k * m.G + g;
+      const uint32_t z = m.zero[mi], z4 = (z & 0xFu) * 0x01010101u;
+      const uint32_t k0b = bits_to_bytes(o.keep) * 0xFFu, k1b = bits_to_bytes(o.keep >> 4) * 0xFFu;
+      *(uint32_t*)(tile + (size_t)(j8 >> 2) * 256 + (j8 & 3u) * 4) =
+          (uint32_t)narrow8<4>(o.lo | (z4 & ~k0b), o.hi | (z4 & ~k1b));
+      if ((j8 & 15u) == 0) {
+        oscale[((size_t)(k >> 4) * m.G + g) * 16 + (k & 15)] = m.scale[mi];
+        ozero[((size_t)(k >> 4) * m.G + g) * 16 + (k & 15)] = (uint8_t)z;
       }
     }
-    uint4* dst = (uint4*)(q + (size_t)k * m.N + g * 128 + i * 32);
-    dst[0] = make_uint4(w[0], w[1], w[2], w[3]);
-    dst[1] = make_uint4(w[4], w[5], w[6], w[7]);
-    if (mask) *(uint32_t*)(mask + (size_t)k * (m.N >> 3) + g * 16 + i * 4) = keep;
   }
+  if (DENSE4 && blockIdx.x == 0 && threadIdx.x < 32)                // readable bytes behind the last tile
+    ((uint4*)(q + (size_t)((m.K + 15) >> 4) * 16 * (m.N >> 1)))[threadIdx.x] = make_uint4(0, 0, 0, 0);
 }
 
 int launch_unpack(const DMat& m, void* q, void* mask, hipStream_t st) {
-  const bool sparse = family_of(m.layout) == FAM_SPARSE;
-  const int64_t items = (int64_t)m.K * (sparse ? m.G : m.N / BLOCK);
-  const dim3 grid((unsigned)((items + 255) / 256)), blk(256);
-  if (sparse) hipLaunchKernelGGL(unpack_sparse_kernel, grid, blk, 0, st, m, (uint8_t*)q, (uint8_t*)mask);
-  else hipLaunchKernelGGL(unpack_fixed_kernel, grid, blk, 0, st, m, (uint8_t*)q, (uint8_t*)mask);
+  const int fam = family_of(m.layout);
+  const dim3 blk(256);
+  uint8_t *qb = (uint8_t*)q, *mb = (uint8_t*)mask;
+  if (fam == FAM_SPARSE) {
+    const int summed = stream_sums(m) ? 1 : 0;
+    hipLaunchKernelGGL(unpack_sparse_kernel<false>, dim3((unsigned)((m.K + 3) / 4)), blk, summed ? (size_t)m.G * 4 : 0, st, m,
+                       qb, mb, nullptr, nullptr, summed);
+  } else {
+    const dim3 grid((unsigned)(((int64_t)((m.K + 15) / 16) * (m.N / 8) + 255) / 256));
+    if (fam == FAM_BLK6) hipLaunchKernelGGL((unpack_fixed_kernel<FAM_BLK6, 6>), grid, blk, 0, st, m, qb, mb);
+    else if (fam == FAM_DENSE) {
+      if (m.bits == 2) hipLaunchKernelGGL((unpack_fixed_kernel<FAM_DENSE, 2>), grid, blk, 0, st, m, qb, mb);
+      else if (m.bits == 3) hipLaunchKernelGGL((unpack_fixed_kernel<FAM_DENSE, 3>), grid, blk, 0, st, m, qb, mb);
+      else if (m.bits == 4) hipLaunchKernelGGL((unpack_fixed_kernel<FAM_DENSE, 4>), grid, blk, 0, st, m, qb, mb);
+      else hipLaunchKernelGGL((unpack_fixed_kernel<FAM_DENSE, 8>), grid, blk, 0, st, m, qb, mb);
+    } else {
+      if (m.bits == 2) hipLaunchKernelGGL((unpack_fixed_kernel<FAM_BLK, 2>), grid, blk, 0, st, m, qb, mb);
+      else if (m.bits == 3) hipLaunchKernelGGL((unpack_fixed_kernel<FAM_BLK, 3>), grid, blk, 0, st, m, qb, mb);
+      else hipLaunchKernelGGL((unpack_fixed_kernel<FAM_BLK, 4>), grid, blk, 0, st, m, qb, mb);
+    }
+  }
+  return hipGetLastError() == hipSuccess ? CBK_OK : CBK_ERR_HIP;
+}
+
+// A survivor-stream matrix as dense 4-bit rows in tiled order: d.data, d.scale, d.zero of the sizes
+// that layout has.
+int launch_repack_dense4(const DMat& m, const DMat& d, hipStream_t st) {
+  const int summed = stream_sums(m) ? 1 : 0;
+  hipLaunchKernelGGL(unpack_sparse_kernel<true>, dim3((unsigned)((m.K + 15) / 16 * 4)), dim3(256),
+                     summed ? (size_t)m.G * 4 : 0, st, m, (uint8_t*)d.data, nullptr, (uint16_t*)d.scale, (uint8_t*)d.zero, summed);
+  return hipGetLastError() == hipSuccess ? CBK_OK : CBK_ERR_HIP;
+}
+
+template <int FAM, int BITS>
+static int launch_pack_cfg(const PackArgs& a, int64_t blocks, size_t lds, hipStream_t st) {
+  auto kern = pack_rows_kernel<FAM, BITS>;
+  static std::atomic<int> configured{0};
+  if (!configured.load(std::memory_order_acquire)) {               // 64 KB for a slab of 8-bit codes, and the table
+    if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024) != hipSuccess)
+      return CBK_ERR_HIP;
+    configured.store(1, std::memory_order_release);
+  }
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(PK_THREADS), lds, st, a);
   return hipGetLastError() == hipSuccess ? CBK_OK : CBK_ERR_HIP;
 }
 
 int launch_pack(const DMat& m, const void* mask, const void* q, const void* scale, const void* zero, int zero_f16,
-                int fix_zero, int* status, hipStream_t st) {
+                int fix_zero, int* status, const PackExtra* extra, hipStream_t st) {
   const int fam = family_of(m.layout);
   if (fam == FAM_SPARSE) return CBK_ERR_UNSUPPORTED;
-  const int kr = m.tiled ? (m.K + 15) / 16 * 16 : m.K;
-  clear16((void*)m.data, (size_t)kr * m.stride + (m.tiled ? 512 : 64), st);      // rows + tail, a multiple of 16
-  if (m.tiled && kr != m.K) {                                      // entries of the padding rows
-    clear16((void*)m.scale, (size_t)kr * m.G * 2, st);
-    clear16((void*)m.zero, (size_t)kr * m.G, st);
-  }
   PackArgs a;
   a.mask = (const uint8_t*)mask; a.q = (const uint8_t*)q; a.scale = (const uint16_t*)scale; a.zero = zero;
   a.data = (uint8_t*)m.data; a.oscale = (uint16_t*)m.scale; a.ozero = (uint8_t*)m.zero;
-  a.K = m.K; a.N = m.N; a.G = m.G; a.group = m.group; a.bits = m.bits; a.keep = m.keep; a.fam = fam; a.tiled = m.tiled;
+  a.K = m.K; a.N = m.N; a.G = m.G; a.group = m.group; a.keep = m.keep; a.tiled = m.tiled;
   a.zero_f16 = zero_f16; a.fix_zero = fix_zero;
   a.stride = m.stride;
-  const int64_t items = (int64_t)m.K * ((m.N + 255) / 256);
-  hipLaunchKernelGGL(pack_rows_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, a, status);
-  return hipGetLastError() == hipSuccess ? CBK_OK : CBK_ERR_HIP;
+  a.krows = m.tiled ? (m.K + 15) / 16 * 16 : m.K;
+  a.tail = m.tiled ? 512 : 64;
+  a.status = status;
+  a.extra = extra ? *extra : PackExtra{};
+  const int64_t blocks = (int64_t)((m.K + PK_ROWS - 1) / PK_ROWS) * ((m.N + PK_COLS - 1) / PK_COLS);
+  const int cols = m.N < PK_COLS ? m.N : PK_COLS, pb = fam == FAM_BLK6 ? 4 : m.bits;
+  const size_t row = (size_t)((cols / 32) * (fam == FAM_DENSE ? 32 : m.keep) * pb + 127) / 128 * 16 +
+                     (fam == FAM_BLK6 ? (size_t)cols / 8 : 0);
+  if (fam == FAM_BLK6) return launch_pack_cfg<FAM_BLK6, 6>(a, blocks, PK_ROWS * row, st);
+  if (fam == FAM_DENSE)
+    return m.bits == 2 ? launch_pack_cfg<FAM_DENSE, 2>(a, blocks, PK_ROWS * row, st)
+         : m.bits == 3 ? launch_pack_cfg<FAM_DENSE, 3>(a, blocks, PK_ROWS * row, st)
+         : m.bits == 4 ? launch_pack_cfg<FAM_DENSE, 4>(a, blocks, PK_ROWS * row, st)
+                       : launch_pack_cfg<FAM_DENSE, 8>(a, blocks, PK_ROWS * row, st);
+  return m.bits == 2 ? launch_pack_cfg<FAM_BLK, 2>(a, blocks, PK_ROWS * row, st)
+       : m.bits == 3 ? launch_pack_cfg<FAM_BLK, 3>(a, blocks, PK_ROWS * row, st)
+                     : launch_pack_cfg<FAM_BLK, 4>(a, blocks, PK_ROWS * row, st);
 }
 
 }  // namespace cbk

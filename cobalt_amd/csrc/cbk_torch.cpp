@@ -18,11 +18,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/InlineDeviceGuard.h>
 #include <c10/hip/HIPStream.h>
-#include "../../include/cbk.h"
-
-namespace cbk {
-size_t decode_workspace_bytes(const cbk_desc*, int M);              // cbk_api.hip
-}
+#include "cbk_internal.h"
 
 namespace {
 
@@ -72,6 +68,11 @@ cbk_desc desc_of(const Matrix* m) {
   d.data = at_off(0); d.row_off = at_off(1); d.scale = at_off(2); d.zero = at_off(3); d.col_scale = at_off(4);
   return d;
 }
+
+struct GilRelease {
+  PyThreadState* s = PyEval_SaveThread();
+  ~GilRelease() { PyEval_RestoreThread(s); }
+};
 
 struct Fail {};                                                     // a Python exception has been set
 
@@ -278,6 +279,79 @@ PyObject* py_gemv_batch(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   });
 }
 
+// pack_raw(mask or None, q, scale, zero, col_scale or None, layout, bits, group, keep, fix_zero, tiled) ->
+//   (blob, offsets of data / scale / zero / col_scale (-1: none), cs_rows, data_bytes, status, groups re-derived,
+//    largest zero point, survivors in the mask)
+// The caller has checked shapes and devices.  One kernel writes every byte of the image and one copy
+// brings the figures back; the call waits for that copy.
+PyObject* py_pack_raw(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (!arity(n, 11)) return nullptr;
+  return guarded([&]() -> PyObject* {
+    at::Tensor mask = as_tensor(a[0], "mask"), q = as_tensor(a[1], "q"), scale = as_tensor(a[2], "scale"),
+               zero = as_tensor(a[3], "zero"), cs = as_tensor(a[4], "col_scale");
+    cbk_desc d{};
+    d.layout = (int)PyLong_AsLong(a[5]); d.bits = (int)PyLong_AsLong(a[6]);
+    d.group = (int)PyLong_AsLong(a[7]); d.keep = (int)PyLong_AsLong(a[8]);
+    const bool fix = PyObject_IsTrue(a[9]), tiled = PyObject_IsTrue(a[10]);
+    if (PyErr_Occurred()) throw Fail{};
+    const at::Device dev = q.device();
+    const c10::DeviceGuard guard(dev);
+    const int64_t K = q.size(0), N = q.size(1), G = N / d.group;
+    d.K = (int32_t)K; d.N = (int32_t)N; d.flags = tiled ? CBK_FLAG_TILED16 : 0;
+    q = (q.scalar_type() == at::kByte ? q : q.clamp(0, 255).to(at::kByte)).contiguous();
+    if (mask.defined()) mask = mask.to(dev).reshape({K, N / 8}).contiguous();
+    scale = scale.to(dev, at::kHalf).reshape({K, G}).contiguous();
+    zero = zero.to(dev).reshape({K, G});
+    zero = (zero.scalar_type() == at::kByte ? zero : zero.to(at::kHalf)).contiguous();
+    int64_t cs_rows = 0;
+    if (cs.defined()) {
+      cs = cs.to(dev, at::kHalf).reshape({-1, N}).contiguous();
+      if ((uintptr_t)cs.const_data_ptr() & 15) cs = cs.clone(at::MemoryFormat::Contiguous);
+      cs_rows = cs.size(0);
+    }
+    // the packing kernel reads q with 16-byte and the mask with 4-byte loads
+    if ((uintptr_t)q.const_data_ptr() & 15) q = q.clone(at::MemoryFormat::Contiguous);
+    if (mask.defined() && ((uintptr_t)mask.const_data_ptr() & 3)) mask = mask.clone(at::MemoryFormat::Contiguous);
+    const int64_t kr = tiled ? (K + 15) / 16 * 16 : K, stride = (int64_t)cbk_row_stride(&d);
+    const int64_t size[4] = {kr * stride + (tiled ? 512 : 64), kr * G * 2, kr * G, cs_rows * N * 2};
+    const int na = cs_rows ? 4 : 3;
+    int64_t off[4] = {0, 0, 0, -1}, pos = 0;
+    cbk::PackExtra x{};
+    for (int i = 0; i < na; ++i) { off[i] = pos; pos = (pos + size[i] + 255) / 256 * 256; }
+    const at::TensorOptions bytes = at::TensorOptions().dtype(at::kByte).device(dev);
+    at::Tensor blob = at::empty({pos}, bytes);
+    uint8_t* base = (uint8_t*)blob.mutable_data_ptr();
+    for (int i = 0; i < na; ++i) {
+      x.gap[i] = base + off[i] + size[i];
+      x.gap_bytes[i] = (uint32_t)((i + 1 < na ? off[i + 1] : pos) - off[i] - size[i]);
+    }
+    d.data = base + off[0]; d.scale = base + off[1]; d.zero = base + off[2];
+    if (cs_rows) {
+      x.cs_src = cs.const_data_ptr(); x.cs_dst = base + off[3]; x.cs_units = (uint32_t)(size[3] / 16);
+    }
+    at::Tensor counts = at::zeros({cbk::PACK_SLOTS * cbk::PACK_SLOT_WORDS}, bytes.dtype(at::kInt));
+    x.counts = (uint32_t*)counts.mutable_data_ptr();
+    check(cbk::pack_image(&d, mask.defined() ? mask.const_data_ptr() : nullptr, q.const_data_ptr(), scale.const_data_ptr(),
+                          zero.const_data_ptr(), zero.scalar_type() == at::kByte ? CBK_U8 : CBK_F16, fix ? 1 : 0, nullptr, &x,
+                          stream_of(q)),
+          "cbk_pack");
+    at::Tensor host;
+    {
+      const GilRelease other_threads_run;
+      host = counts.cpu();
+    }
+    const uint32_t* h = (const uint32_t*)host.const_data_ptr();
+    uint32_t status = 0, fixed = 0, zmax = 0;
+    unsigned long long surv = 0;
+    for (int i = 0; i < cbk::PACK_SLOTS; ++i, h += cbk::PACK_SLOT_WORDS) {
+      status |= h[0]; fixed += h[1]; surv += h[3];
+      zmax = zmax > h[2] ? zmax : h[2];
+    }
+    return Py_BuildValue("N(LLLL)LLIIIK", THPVariable_Wrap(blob), (long long)off[0], (long long)off[1], (long long)off[2],
+                         (long long)off[3], (long long)cs_rows, (long long)(kr * stride), status, fixed, zmax, surv);
+  });
+}
+
 PyObject* py_set_error(PyObject*, PyObject* e) {
   Py_INCREF(e);
   Py_XSETREF(g_error, e);
@@ -288,6 +362,7 @@ PyMethodDef methods[] = {
     {"matmul", (PyCFunction)(void (*)())py_matmul, METH_FASTCALL, nullptr},
     {"linear_act", (PyCFunction)(void (*)())py_linear_act, METH_FASTCALL, nullptr},
     {"gemv_batch", (PyCFunction)(void (*)())py_gemv_batch, METH_FASTCALL, nullptr},
+    {"pack_raw", (PyCFunction)(void (*)())py_pack_raw, METH_FASTCALL, nullptr},
     {"set_error", py_set_error, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -89,45 +89,18 @@ def pack_raw(mask_bits, q, scale, zero, col_scale, layout, bits=None, group=None
         raise NotImplementedError("the variable-length SPARSE4* layouts are read, not produced, by this package")
     if q.device.type != "cuda":
         raise _lib.CbkError("ops.pack_raw packs on the GPU; use format.pack_raw for tensors on the CPU")
-    dev = q.device
     K, N = q.shape
     if N % 128 or N % group:
         raise ValueError(f"N={N} must be a multiple of 128 and of the group size")
-    G = N // group
     nl = (1 << bits) - 1
-    mb = None if mask_bits is None else mask_bits.to(dev).reshape(K, N // 8).contiguous()
-    q8 = (q if q.dtype == torch.uint8 else q.clamp(0, 255).to(torch.uint8)).contiguous()
-    sc16 = scale.to(dev).to(torch.float16).reshape(K, G).contiguous()
-    z = zero.to(dev).reshape(K, G)
-    z = (z if z.dtype == torch.uint8 else z.to(torch.float16)).contiguous()
-    stride = F.row_stride(layout, N, bits, group, kpb or None)
-    kr = F._align(K, 16) if tiled else K
-    sizes = {"data": kr * stride + (F.TILED_TAIL if tiled else F.BLOB_TAIL), "scale": kr * G * 2, "zero": kr * G}
-    cs = None
-    if col_scale is not None:
-        cs = col_scale.to(dev).to(torch.float16).reshape(-1, N).contiguous()
-        sizes["col_scale"] = cs.numel() * 2
-    offs, pos = {}, 0
-    for name, n in sizes.items():
-        pos = F._align(pos, F.ARR_ALIGN)
-        offs[name] = pos
-        pos += n
-    blob = torch.zeros(F._align(pos, F.ARR_ALIGN), dtype=torch.uint8, device=dev)
-    if cs is not None:
-        blob[offs["col_scale"]: offs["col_scale"] + sizes["col_scale"]] = cs.reshape(-1).view(torch.uint8)
-    if layout in F._DENSE:
-        n_surv = K * N if mb is None else int(F.unpack_mask(mb, N).sum())
-    else:
-        n_surv = K * (N // F.BLOCK) * kpb
-    pm = PackedMatrix(blob, offs, K, N, layout, bits, group, kpb, 0 if cs is None else cs.shape[0], tuple(cs_splits),
-                      kr * stride, n_surv, 0, (F.FLAG_TILED16 if tiled else 0))
-    status = torch.zeros(2, dtype=torch.int32, device=dev)
-    d = pm.desc()
-    rc = _lib.lib().cbk_pack(ctypes.byref(d), mb.data_ptr() if mb is not None else None, q8.data_ptr(), sc16.data_ptr(),
-                             z.data_ptr(), 3 if z.dtype == torch.uint8 else F.F16, int(bool(fix_zero)), status.data_ptr(),
-                             _stream_ptr(dev))
-    _lib.check(rc, "cbk_pack")
-    wrong, pm.n_zero_fixed = (int(v) for v in status.tolist())
+    blob, (o_data, o_scale, o_zero, o_cs), cs_rows, data_bytes, wrong, n_fixed, z_max, n_mask = _lib.native().pack_raw(
+        mask_bits, q, scale, zero, col_scale, layout, bits, group, kpb, bool(fix_zero), tiled)
+    offs = {"data": o_data, "scale": o_scale, "zero": o_zero}
+    if cs_rows:
+        offs["col_scale"] = o_cs
+    n_surv = n_mask if layout in F._DENSE else K * (N // F.BLOCK) * kpb
+    pm = PackedMatrix(blob, offs, K, N, layout, bits, group, kpb, cs_rows, tuple(cs_splits), data_bytes, n_surv, n_fixed,
+                      (F.FLAG_TILED16 if tiled else 0) | F.zero_flags(z_max, bits))
     if wrong & 2:
         raise ValueError(f"{F.LAYOUT_NAME[layout]} stores the zero point as the code of a pruned column, and a zero point "
                          f"of this matrix is above {nl}: such a column would not dequantise to 0 (pack with fix_zero=True, "
@@ -135,7 +108,6 @@ def pack_raw(mask_bits, q, scale, zero, col_scale, layout, bits=None, group=None
     if wrong & 1:
         raise ValueError(f"{F.LAYOUT_NAME[layout]} needs exactly {kpb} survivors in every aligned block of "
                          f"{F.BLOCK} columns; the mask has a block with another count")
-    pm.flags |= F.zero_flags(int(pm.array("zero").max()), bits)
     return pm.validate()
 
 
