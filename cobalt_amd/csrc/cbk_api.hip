@@ -23,19 +23,47 @@ int launch_gemm(const DMat&, const void*, int, int, int64_t, void*, int, int64_t
                 hipStream_t);
 int launch_gemm_big(const DMat&, const void*, int, int, int64_t, void*, int, int64_t, const void*, void*, size_t,
                     hipStream_t, bool halves = false);
-size_t gemm_big_workspace(const DMat&, int M);
+size_t gemm_big_workspace(const DMat&, int M, bool least);
+double gemm_big_time(const DMat&, int M, bool act);
+bool gemm_skinny_takes(const DMat&);
+double gemm_skinny_time(const DMat&, int M);
+size_t gemm_skinny_workspace(const DMat&, int M, bool least);
+int launch_gemm_skinny(const DMat&, const void*, int, int, int64_t, void*, int, int64_t, const void*, int act, void*, size_t,
+                       hipStream_t);
 int launch_pack(const DMat&, const void* mask, const void* q, const void* scale, const void* zero, int zero_f16,
                 int fix_zero, int* status, const PackExtra* extra, hipStream_t);
 int launch_repack_dense4(const DMat& sparse, const DMat& dense4, hipStream_t);
 int launch_unpack(const DMat&, void* q, void* mask, hipStream_t);
-// The 256 x 256 tile kernel takes every call of the fixed-stride layouts: below 256 activation
-// rows part of its token tile is padding, and it is still several times faster than the
-// 128 x 128 kernel, which decodes through the generic reader (14336 x 4096 at 64 rows: 54 us
-// against 288 us).  That one stays for q|k|v matrices whose ranges are off the 16-row grid.
+// The 256 x 256 tile kernel takes every call of the fixed-stride layouts but q|k|v matrices whose
+// ranges do not start on its row tiles.
 static inline bool gemm_big_takes(const DMat& m, int M) {
   if (M < 1 || family_of(m.layout) == FAM_SPARSE) return false;
   return m.cs_rows <= 2 || (m.cs_split0 % 256 == 0 && (m.cs_split0 + m.cs_split1) % 256 == 0);
 }
+
+// Two kernels for the fixed-stride layouts: the one that decodes into the registers that multiply
+// (cbk_gemm_skinny.h: few tokens, small matrices) and the 256 x 256 tile (many tokens, whose weight
+// tiles are worth a trip through LDS).  Each knows what a call costs it; the crossover lies between
+// 100 and 600 activation rows, depending on how the matrix fills the chip.
+static inline bool skinny_is_faster(const DMat& m, int M, bool act) {
+  return gemm_skinny_takes(m) && (!gemm_big_takes(m, M) || gemm_skinny_time(m, M) < gemm_big_time(m, M, act));
+}
+// Workspace of run_gemm.  least: what it cannot do without, else what it makes use of.
+static size_t gemm_workspace(const DMat& m, int M, bool least) {
+  if (M < 1) return 0;
+  const size_t big = gemm_big_takes(m, M) ? gemm_big_workspace(m, M, least) : 0;
+  if (!skinny_is_faster(m, M, false)) return big;
+  const size_t sk = gemm_skinny_workspace(m, M, least);
+  return least && big && big < sk ? big : sk;
+}
+static int run_gemm(const DMat& m, const void* x, int xdt, int M, int64_t ldx, void* y, int ydt, int64_t ldy, const void* bias,
+                    void* ws, size_t ws_bytes, hipStream_t st) {
+  if (skinny_is_faster(m, M, false) && (!gemm_big_takes(m, M) || ws_bytes >= gemm_skinny_workspace(m, M, true)))
+    return launch_gemm_skinny(m, x, xdt, M, ldx, y, ydt, ldy, bias, -1, ws, ws_bytes, st);
+  return launch_gemm_big(m, x, xdt, M, ldx, y, ydt, ldy, bias, ws, ws_bytes, st);
+}
+// the matrices run_gemm takes whole
+static inline bool gemm_takes(const DMat& m, int M) { return M >= 1 && (gemm_big_takes(m, M) || gemm_skinny_takes(m)); }
 
 static inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
@@ -277,28 +305,31 @@ size_t cbk_stream_bytes(const cbk_desc* in, size_t sparse_data_bytes) {
   return (size_t)d.K * stride_of(d) + meta;
 }
 
-size_t cbk_workspace_bytes(const cbk_desc* in, int M) {
-  DMat m;
-  if (to_dmat(in, &m, false)) return 0;
+static size_t workspace_of(const DMat& m, int M, bool least) {
   if (family_of(m.layout) == FAM_SPARSE) {                          // cbk_gemm / cbk_linear above 16 rows: see Transient
-    if (M <= 16) return decode_workspace(m, M);                     // part sums of long rows split by columns, else none
+    if (M <= 16) return least ? 0 : decode_workspace(m, M);         // part sums of long rows split by columns, else none
     if (!sparse_repackable(m)) return 0;
     const Transient t = transient_dense4(m);
-    return t.end + gemm_big_workspace(dense4_view(m, nullptr, t), M);
+    return t.end + gemm_workspace(dense4_view(m, nullptr, t), M, least);
   }
   // the most any of the three entry points asks for (cbk_gemm runs the prefill kernel at any M)
-  size_t need = decode_workspace(m, M);
-  if (gemm_big_takes(m, M)) {
-    const size_t b = gemm_big_workspace(m, M);
+  size_t need = least ? 0 : decode_workspace(m, M);
+  if (gemm_takes(m, M)) {
+    const size_t b = gemm_workspace(m, M, least);
     return need > b ? need : b;
   }
   int lo[3], hi[3], row[3];
   const int nr = M >= 1 ? fused_ranges(m, lo, hi, row) : 0;
   for (int i = 0; i < nr; ++i) {                                    // run one after the other on the same bytes
-    const size_t b = gemm_big_workspace(row_range(m, lo[i], hi[i], row[i]), M);
+    const size_t b = gemm_workspace(row_range(m, lo[i], hi[i], row[i]), M, least);
     need = need > b ? need : b;
   }
   return need;
+}
+
+size_t cbk_workspace_bytes(const cbk_desc* in, int M) {
+  DMat m;
+  return to_dmat(in, &m, false) ? 0 : workspace_of(m, M, false);
 }
 
 size_t cbk_gemv_batch_workspace_bytes(int n, const cbk_desc* descs, int M) {
@@ -422,7 +453,7 @@ int cbk_gemm(const cbk_desc* in, const void* x, int x_dtype, int M, int64_t ldx,
       return cbk_gemv(in, x, x_dtype, M, ldx, y, y_dtype, ldy, bias, workspace, workspace_bytes, stream);
     const Transient t = transient_dense4(m);
     const bool room = workspace && !((uintptr_t)workspace & 255) &&
-                      workspace_bytes >= t.end + gemm_big_workspace(dense4_view(m, nullptr, t), M);
+                      workspace_bytes >= t.end + gemm_workspace(dense4_view(m, nullptr, t), M, true);
     if (!sparse_repackable(m) || !room) {
       // zero points that are no 4-bit codes, row-fused column scales, or no room for the dense
       // image: the row kernel, sixteen activation rows per pass, without a workspace
@@ -439,12 +470,10 @@ int cbk_gemm(const cbk_desc* in, const void* x, int x_dtype, int M, int64_t ldx,
     const DMat d = dense4_view(m, ws, t);
     rc = launch_repack_dense4(m, d, (hipStream_t)stream);
     if (rc) return rc;
-    return launch_gemm_big(d, x, x_dtype, M, ldx, y, y_dtype, ldy, bias, ws + t.end, workspace_bytes - t.end,
-                           (hipStream_t)stream);
+    return run_gemm(d, x, x_dtype, M, ldx, y, y_dtype, ldy, bias, ws + t.end, workspace_bytes - t.end, (hipStream_t)stream);
   }
-  if (gemm_big_takes(m, M))
-    return launch_gemm_big(m, x, x_dtype, M, ldx, y, y_dtype, ldy, bias, workspace, workspace_bytes,
-                           (hipStream_t)stream);
+  if (gemm_takes(m, M))
+    return run_gemm(m, x, x_dtype, M, ldx, y, y_dtype, ldy, bias, workspace, workspace_bytes, (hipStream_t)stream);
   int lo[3], hi[3], row[3];
   const int nr = fused_ranges(m, lo, hi, row);
   if (nr) {
@@ -453,9 +482,8 @@ int cbk_gemm(const cbk_desc* in, const void* x, int x_dtype, int M, int64_t ldx,
     const size_t ysz = y_dtype == CBK_F32 ? 4 : 2;
     for (int i = 0; i < nr; ++i) {
       const DMat s = row_range(m, lo[i], hi[i], row[i]);
-      rc = launch_gemm_big(s, x, x_dtype, M, ldx, (uint8_t*)y + (size_t)lo[i] * ysz, y_dtype, ldy,
-                           bias ? (const uint8_t*)bias + (size_t)lo[i] * ysz : nullptr, workspace, workspace_bytes,
-                           (hipStream_t)stream);
+      rc = run_gemm(s, x, x_dtype, M, ldx, (uint8_t*)y + (size_t)lo[i] * ysz, y_dtype, ldy,
+                    bias ? (const uint8_t*)bias + (size_t)lo[i] * ysz : nullptr, workspace, workspace_bytes, (hipStream_t)stream);
       if (rc) return rc;
     }
     return CBK_OK;
@@ -495,8 +523,8 @@ extern "C" {
 
 int cbk_gemm_static(const cbk_desc* in, const void* x, int x_dtype, int M, int64_t ldx, void* y, int y_dtype,
                     int64_t ldy, const void* bias, void* stream) {
-  if (cbk_workspace_bytes(in, M) > (size_t)CBK_STATIC_SCRATCH_BYTES) {
-    DMat m;
+  DMat m;
+  if (!to_dmat(in, &m, false) && workspace_of(m, M, true) > (size_t)CBK_STATIC_SCRATCH_BYTES) {
     const int rc = to_dmat(in, &m, true);
     return rc ? rc : CBK_ERR_WORKSPACE;                             // more scratch than the array holds
   }
@@ -522,10 +550,16 @@ static size_t act_mid_bytes(int K, int M, int y_dtype) {
   return (b + 255) & ~(size_t)255;
 }
 
+// act(gate) * up in the kernel that sums the column parts (cbk_gemm_skinny.h): no t in memory
+static bool act_fused(const DMat& m, int M) {
+  return M > 8 && family_of(m.layout) != FAM_SPARSE && m.cs_rows <= 2 && skinny_is_faster(m, M, true);
+}
+
 size_t cbk_linear_act_workspace_bytes(const cbk_desc* in, int M, int y_dtype) {
-  cbk_desc d;
-  if (M < 1 || canon(in, &d)) return 0;
-  return act_mid_bytes(d.K, M, y_dtype) + cbk_workspace_bytes(in, M);
+  DMat m;
+  if (M < 1 || to_dmat(in, &m, false)) return 0;
+  if (act_fused(m, M)) return gemm_skinny_workspace(m, M, false);
+  return act_mid_bytes(m.K, M, y_dtype) + workspace_of(m, M, false);
 }
 
 int cbk_linear_act(const cbk_desc* in, const void* x, int x_dtype, int M, int64_t ldx, void* y, int y_dtype,
@@ -539,9 +573,14 @@ int cbk_linear_act(const cbk_desc* in, const void* x, int x_dtype, int M, int64_
   if (!y) return CBK_ERR_NULL;
   if (M < 1 || ldy < m.K / 2) return CBK_ERR_SHAPE;
   if ((uintptr_t)y & (y_dtype == CBK_F32 ? 3 : 1)) return CBK_ERR_ALIGN;
-  const size_t mid = act_mid_bytes(m.K, M, y_dtype);
-  if (!workspace || ((uintptr_t)workspace & 255) || workspace_bytes < mid + cbk_workspace_bytes(in, M))
+  if (!workspace || ((uintptr_t)workspace & 255) || workspace_bytes < cbk_linear_act_workspace_bytes(in, M, y_dtype))
     return CBK_ERR_WORKSPACE;
+  if (act_fused(m, M)) {
+    rc = check_io(x, x_dtype, M, ldx, y, y_dtype, ldy, m.N, m.K / 2);
+    if (rc) return rc;
+    return launch_gemm_skinny(m, x, x_dtype, M, ldx, y, y_dtype, ldy, bias, act, workspace, workspace_bytes, (hipStream_t)stream);
+  }
+  const size_t mid = act_mid_bytes(m.K, M, y_dtype);
   const int tdt = act_mid_dtype(M, y_dtype);
   if (M > 8 && m.cs_rows == 2 && gemm_big_takes(m, M)) {
     // the tile kernel leaves t as two halves (gate outputs, then up outputs): a workgroup holds

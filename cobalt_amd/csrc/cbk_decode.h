@@ -110,6 +110,28 @@ struct CodeCfg {
   static constexpr int SEL_KIND = (BITS == 2) ? 1 : 0;
 };
 
+// The ND dwords that start `skew` bits (0..127) into the NL dwords of `raw`; DWORDS: the skew is a
+// multiple of 32.
+template <int NL, int ND, bool DWORDS>
+__device__ inline void skew_dwords(const uint32_t (&raw)[NL], uint32_t skew, uint32_t (&cw)[ND]) {
+  uint32_t t1[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i)
+    t1[i] = DWORDS ? raw[i] : __builtin_amdgcn_alignbit(i + 1 < NL ? raw[i + 1] : 0u, raw[i], skew);
+  // Shift by one and by two dwords with bitwise selects under a sign-extended bit of the skew.
+  // Written as C++ conditionals the compiler turns the two steps into one read of the array at
+  // a run-time index, which puts the array into scratch memory (a store and a load of every
+  // dword per chunk).  Not inline assembly either: the compiler inserts no wait states between
+  // an MFMA and an assembly statement that overwrites one of the MFMA's result registers.
+  const uint32_t m32 = (uint32_t)__builtin_amdgcn_sbfe((int)skew, 5, 1);
+  const uint32_t m64 = (uint32_t)__builtin_amdgcn_sbfe((int)skew, 6, 1);
+  uint32_t t2[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i) t2[i] = mask_select(m32, t1[i], i + 1 < NL ? t1[i + 1] : 0u);
+#pragma unroll
+  for (int i = 0; i < ND; ++i) cw[i] = mask_select(m64, t2[i], i + 2 < NL ? t2[i + 2] : 0u);
+}
+
 // Chunk code bits with their first bit at bit 0 of cw[0], from the NL dwords loaded as whole
 // 16-byte units around them; `chunk` is the chunk index the units were loaded for.
 template <class C>
@@ -118,23 +140,7 @@ __device__ inline void align_chunk_codes(const uint32_t (&raw)[C::NL], uint32_t 
 #pragma unroll
     for (int i = 0; i < C::ND; ++i) cw[i] = raw[i];
   } else {
-    const uint32_t skew = (chunk * C::CHB) & 127u;                // inside the first unit
-    uint32_t t1[C::NL];
-#pragma unroll
-    for (int i = 0; i < C::NL; ++i)
-      t1[i] = C::ALIGNED ? raw[i] : __builtin_amdgcn_alignbit(i + 1 < C::NL ? raw[i + 1] : 0u, raw[i], skew);
-    // Shift by one and by two dwords with bitwise selects under a sign-extended bit of the skew.
-    // Written as C++ conditionals the compiler turns the two steps into one read of the array at
-    // a run-time index, which puts the array into scratch memory (a store and a load of every
-    // dword per chunk).  Not inline assembly either: the compiler inserts no wait states between
-    // an MFMA and an assembly statement that overwrites one of the MFMA's result registers.
-    const uint32_t m32 = (uint32_t)__builtin_amdgcn_sbfe((int)skew, 5, 1);
-    const uint32_t m64 = (uint32_t)__builtin_amdgcn_sbfe((int)skew, 6, 1);
-    uint32_t t2[C::NL];
-#pragma unroll
-    for (int i = 0; i < C::NL; ++i) t2[i] = mask_select(m32, t1[i], i + 1 < C::NL ? t1[i + 1] : 0u);
-#pragma unroll
-    for (int i = 0; i < C::ND; ++i) cw[i] = mask_select(m64, t2[i], i + 2 < C::NL ? t2[i + 2] : 0u);
+    skew_dwords<C::NL, C::ND, C::ALIGNED>(raw, (chunk * C::CHB) & 127u, cw);
   }
 }
 

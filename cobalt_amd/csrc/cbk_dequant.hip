@@ -6,7 +6,7 @@
 // sixteen consecutive rows: the stores of a wavefront are 1 KB runs, the column scales stay in
 // registers over the rows, and in the tiled byte order the sixteen rows share the cache lines of
 // their units.  One thread per 32-column block with single-element stores, the form before, was
-// bound by those stores: 14336 x 4096 to fp16 300 us.
+// bound by those stores: 14336 x 4096 to fp16 300 us, now 28 us (5.1 TB/s).
 #include "cbk_octet.h"
 
 namespace cbk {
@@ -21,10 +21,15 @@ __device__ inline void store8(void* out, size_t at, const float (&w)[8], bool ve
     for (int i = 0; i < 8; ++i) store_out<ODT>(out, at + i, w[i]);
     return;
   }
-  uint4* d = (uint4*)((uint8_t*)out + at * ESZ);
+  // Non-temporal: the output is larger than what the caches keep, and left to them its lines push
+  // out each other (two outputs of 117 MB in turn: 43 us a pass, 28 us past the caches).
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  u4* d = (u4*)((uint8_t*)out + at * ESZ);
   if (ODT == CBK_F32) {
-    d[0] = make_uint4(__float_as_uint(w[0]), __float_as_uint(w[1]), __float_as_uint(w[2]), __float_as_uint(w[3]));
-    d[1] = make_uint4(__float_as_uint(w[4]), __float_as_uint(w[5]), __float_as_uint(w[6]), __float_as_uint(w[7]));
+    const u4 a = {__float_as_uint(w[0]), __float_as_uint(w[1]), __float_as_uint(w[2]), __float_as_uint(w[3])};
+    const u4 b = {__float_as_uint(w[4]), __float_as_uint(w[5]), __float_as_uint(w[6]), __float_as_uint(w[7])};
+    __builtin_nontemporal_store(a, d);
+    __builtin_nontemporal_store(b, d + 1);
   } else {
     uint32_t p[4];
 #pragma unroll
@@ -36,7 +41,8 @@ __device__ inline void store8(void* out, size_t at, const float (&w)[8], bool ve
         p[i] = __builtin_bit_cast(uint32_t, v);
       }
     }
-    *d = make_uint4(p[0], p[1], p[2], p[3]);
+    const u4 v = {p[0], p[1], p[2], p[3]};
+    __builtin_nontemporal_store(v, d);
   }
 }
 

@@ -165,7 +165,7 @@ __device__ inline void gb_epilogue(const GbArgs& a, v16f (&acc)[TI][4], uint8_t*
 // BITS 2 / 3 / 4: byte-permute decoder for (BITS, KEEP, GRP), KEEP = 0 for the dense layouts.
 // BITS 0: generic 32-column reader, any fixed-stride layout.
 // PAR 0: one col_scale vector.  1: gate/up matrix (GbArgs::par).  2: q|k|v matrix (GbArgs::vs0, vs1).
-// 3: one col_scale vector, column range split over several workgroups (GbArgs::nsplit).
+// 3: one vector or q|k|v, column range split over several workgroups (GbArgs::nsplit).
 // Three instantiations rather than run-time switches: the schedule of the main loop is tuned
 // to the instruction and measurably shifts with every value that is added to it.
 // TI: 32-token blocks per wavefront.  4: the 256-token tile described above.  2: a 128-token tile
@@ -235,7 +235,7 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
   const int wv = __builtin_amdgcn_readfirstlane(wave);
   const uint32_t xvo_e = (uint32_t)((lane >> 3) * Npad * 2 + (((lane & 7) ^ (lane >> 4)) * 16));
   const uint32_t xvo_o = (uint32_t)((lane >> 3) * Npad * 2 + (((lane & 7) ^ (4 + (lane >> 4))) * 16));
-  const int xv = PAR == 1 ? pp : PAR == 2 ? (r0 >= a.vs0 ? 1 : 0) + (r0 >= a.vs1 ? 1 : 0) : 0;   // which col_scale vector
+  const int xv = PAR == 1 ? pp : PAR >= 2 ? (r0 >= a.vs0 ? 1 : 0) + (r0 >= a.vs1 ? 1 : 0) : 0;   // which col_scale vector
   const uint8_t* xsb = (const uint8_t*)(a.xp + (size_t)xv * a.xps + (size_t)(t0 + 16 * TI * wv) * Npad + (size_t)s_begin * GB_K);
   const uint32_t xlds0 = (uint32_t)(uintptr_t)Xs + (uint32_t)wv * (2048u * TI);
   auto dma_x = [&](int s, int buf) {                              // stage s -> Xs[buf]
@@ -529,8 +529,8 @@ static int launch_big_par(const GbArgs& a, int blocks, hipStream_t st) {
 template <int BITS, int KEEP, int GRP, int TI>
 static int launch_big_ti(const GbArgs& a, int blocks, hipStream_t st) {
   if (a.par) return launch_big_par<BITS, KEEP, GRP, 1, TI>(a, blocks, st);
-  if (a.vs0 != 0x7fffffff) return launch_big_par<BITS, KEEP, GRP, 2, TI>(a, blocks, st);
   if (a.nsplit > 1) return launch_big_par<BITS, KEEP, GRP, 3, TI>(a, blocks, st);
+  if (a.vs0 != 0x7fffffff) return launch_big_par<BITS, KEEP, GRP, 2, TI>(a, blocks, st);
   return launch_big_par<BITS, KEEP, GRP, 0, TI>(a, blocks, st);
 }
 

@@ -2,6 +2,7 @@
 // and the dispatch over the per-code-width instantiations (cbk_gemm_big_b2/3/4.hip).  The
 // kernel itself is in cbk_gemm_big.h.
 #include "cbk_gemm_big.h"
+#include "cbk_prep.h"
 
 namespace cbk {
 
@@ -14,27 +15,20 @@ int launch_gemm_big_b6(const GbArgs&, int blocks, hipStream_t);
 // s_row is the power of two that brings the row's largest |x * col_scale| below 2^15 (1 for
 // nearly every row: only magnitudes beyond fp16's range need it); the GEMM kernel multiplies the
 // row's outputs by it.  Rows M..Mpad-1 and columns N..Npad-1 are zero.
-__device__ inline void prep8(const uint4 v, const uint4 c, int xdt, float (&a)[8]) {
-  const uint32_t xw[4] = {v.x, v.y, v.z, v.w}, cw[4] = {c.x, c.y, c.z, c.w};
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    if (xdt == CBK_F16) { a[2 * e] = h2f((uint16_t)(xw[e] & 0xffffu)); a[2 * e + 1] = h2f((uint16_t)(xw[e] >> 16)); }
-    else { a[2 * e] = bf2f((uint16_t)(xw[e] & 0xffffu)); a[2 * e + 1] = bf2f((uint16_t)(xw[e] >> 16)); }
-    a[2 * e] *= h2f((uint16_t)(cw[e] & 0xffffu)); a[2 * e + 1] *= h2f((uint16_t)(cw[e] >> 16));
-  }
-}
-
 // One workgroup of 1024 threads per row.  CH: 16-byte pieces of the row a thread keeps in
 // registers between the two passes (the row is read from memory once); 0 = any row length, the
 // second pass reads the row again.
 template <int CH>
 __global__ __launch_bounds__(1024) void gemm_prep_kernel(const uint16_t* x, int64_t ldx, const uint16_t* cs, int xdt,
-                                                         int M, int N, int Npad, uint16_t* out, float* row_scale) {
+                                                         int M, int N, int Npad, uint16_t* out, size_t out_vs, float* row_scale,
+                                                         int scale_vs) {
   constexpr int T = 1024;
   __shared__ float red[T / 64];
   const int row = blockIdx.x, tid = threadIdx.x;
   const int n8 = Npad >> 3, nv = N >> 3;                           // N is a multiple of 128
-  uint16_t* orow = out + (size_t)row * Npad;
+  cs = cs ? cs + (size_t)blockIdx.y * N : nullptr;                  // one column-scale vector per blockIdx.y
+  row_scale += (size_t)blockIdx.y * scale_vs;
+  uint16_t* orow = out + (size_t)blockIdx.y * out_vs + (size_t)row * Npad;
   if (row >= M) {
     for (int c8 = tid; c8 < n8; c8 += T) *(uint4*)(orow + c8 * 8) = make_uint4(0, 0, 0, 0);
     if (tid == 0) row_scale[row] = 1.f;
@@ -148,43 +142,42 @@ static bool gb_fast(const DMat& m) {
 //    take the 256-token tile unless the model below gives the 128-token tile the shorter time,
 //    which it does for small matrices (4096 x 4096 at 256 to 2048 rows: 16 to 128 tiles of 256
 //    tokens): twice the tiles, each 0.8 of the time.
-// Times in microseconds from measurements of this kernel: per 64-column stage 1.1 / 1.35 / 1.7
+// Times in microseconds from measurements of this kernel: per 64-column stage 1.1 / 1.25 / 1.7
 // for the three tiles (the 64-token stage is bound by the weight loads' latency), 8 - 10 per
-// workgroup outside the stage loop, 4 TB/s for the partial tiles.  Over 24 measured calls
+// workgroup outside the stage loop, 7 TB/s for the partial tiles, 4 for the reduction kernel.  Over 24 measured calls
 // (eight shapes, 256 / 512 / 2048 rows) the choice is within 2 % of the faster tile; always
 // taking the 256-token tile loses 6 % on average and up to 34 %.
 struct GbPlan { int ti, nsplit; double t; };
-static GbPlan gb_plan_ti(const DMat& m, int M, int ti) {
+static GbPlan gb_plan_ti(const DMat& m, int M, int ti, int max_split) {
   const int T = 64 * ti;
   const int tiles = ((M + T - 1) / T) * ((m.K + GB_R - 1) / GB_R);
   const int nst = gb_npad(m.N) / GB_K;
-  const double t_stage = ti == 1 ? 1.1 : ti == 2 ? 1.35 : 1.7, t_wg = ti == 1 ? 8.0 : 10.0;
+  const double t_stage = ti == 1 ? 1.1 : ti == 2 ? 1.25 : 1.7, t_wg = ti == 1 ? 8.0 : 10.0;
   GbPlan best{ti, 1, 0.0};
   double t1 = 0;
-  const bool may_split = m.cs_rows <= 1 && gb_fast(m);
-  for (int s = 1; s <= (may_split ? 16 : 1); ++s) {
+  const bool may_split = max_split > 1 && m.cs_rows != 2 && gb_fast(m);
+  for (int s = 1; s <= (may_split ? max_split : 1); ++s) {
     const int per = ((nst + s - 1) / s + 3) / 4 * 4;                // stages per part, a multiple of 4
     if (s > 1 && (s - 1) * per >= nst) continue;                    // a part would be empty
     const double rounds = (double)((tiles * s + 255) / 256);
     double t = rounds * (per * t_stage + t_wg);
-    if (s > 1) t += 2.0 * s * (double)M * m.K * 4 / 4.0e6 + 5.0;
+    if (s > 1) t += 2.0 * s * (double)M * m.K * 4 / 7.0e6 + 4.0;
     if (s == 1) { t1 = t; best.t = t; }
     else if (t < best.t) { best.nsplit = s; best.t = t; }
   }
   if (best.t > 0.93 * t1) { best.nsplit = 1; best.t = t1; }         // not worth a second kernel
   return best;
 }
-static GbPlan gb_plan(const DMat& m, int M) {
-  if (M <= 64) return gb_plan_ti(m, M, 1);
-  if (M <= 128) return gb_plan_ti(m, M, 2);
-  const GbPlan p4 = gb_plan_ti(m, M, 4), p2 = gb_plan_ti(m, M, 2);
+static GbPlan gb_plan(const DMat& m, int M, int max_split = 16) {
+  if (M <= 64) return gb_plan_ti(m, M, 1, max_split);
+  if (M <= 128) return gb_plan_ti(m, M, 2, max_split);
+  const GbPlan p4 = gb_plan_ti(m, M, 4, max_split), p2 = gb_plan_ti(m, M, 2, max_split);
   return p2.t < p4.t ? p2 : p4;
 }
 
 static inline size_t gb_kpad(int K) { return (size_t)(K + 7) / 8 * 8; }
 
-size_t gemm_big_workspace(const DMat& m, int M) {
-  const GbPlan plan = gb_plan(m, M);
+static size_t gb_space(const DMat& m, int M, const GbPlan& plan) {
   const size_t T = 64 * plan.ti, mpad = (size_t)(M + T - 1) / T * T;
   const size_t nv = m.cs_rows > 1 ? m.cs_rows : 1;
   size_t b = (nv * mpad * gb_npad(m.N) * 2 + 255) & ~(size_t)255;     // X', one per col_scale vector
@@ -192,6 +185,17 @@ size_t gemm_big_workspace(const DMat& m, int M) {
   const int ns = plan.nsplit;
   if (ns > 1) b += ((size_t)ns * M * gb_kpad(m.K) * 4 + 255) & ~(size_t)255;
   return b;
+}
+// least: without room for partial tiles, i.e. with the column range in one piece
+size_t gemm_big_workspace(const DMat& m, int M, bool least) { return gb_space(m, M, gb_plan(m, M, least ? 1 : 16)); }
+
+// What a call takes, for the choice between this kernel and the one in cbk_gemm_skinny.h: the plan's
+// time, 5 us for the preparation kernel and the launch, 3 more where a gate/up matrix needs the activation
+// kernel behind it (and that kernel's traffic).  Layouts without a decoder of their own are read at a
+// tenth of the rate.
+double gemm_big_time(const DMat& m, int M, bool act) {
+  const double t = gb_plan(m, M).t * (gb_fast(m) ? 1.0 : 10.0) + 5.0;
+  return act ? t + 3.0 + (double)M * m.K * (M <= 128 ? 9 : 5) / 5.0e6 : t;
 }
 
 // halves: a gate/up matrix's outputs as two halves of y (GbArgs::halves) instead of interleaved
@@ -202,9 +206,10 @@ int launch_gemm_big(const DMat& m, const void* x, int xdt, int M, int64_t ldx, v
   // q|k|v ranges off the row-tile grid: the caller passes them one by one
   if (m.cs_rows == 3 && (m.cs_split0 % GB_R || (m.cs_split0 + m.cs_split1) % GB_R)) return CBK_ERR_UNSUPPORTED;
   if (ydt != CBK_F32 && ydt != CBK_F16 && ydt != CBK_BF16T) return CBK_ERR_DTYPE;
-  if (!ws || ws_bytes < gemm_big_workspace(m, M)) return CBK_ERR_WORKSPACE;
+  GbPlan plan = gb_plan(m, M);
+  if (ws_bytes < gb_space(m, M, plan)) plan = gb_plan(m, M, 1);     // no room for partial tiles
+  if (!ws || ws_bytes < gb_space(m, M, plan)) return CBK_ERR_WORKSPACE;
   if ((uintptr_t)ws & 255) return CBK_ERR_ALIGN;
-  const GbPlan plan = gb_plan(m, M);
   const int T = 64 * plan.ti;
   const int Mpad = (M + T - 1) / T * T;
   const int Npad = gb_npad(m.N);
@@ -215,10 +220,8 @@ int launch_gemm_big(const DMat& m, const void* x, int xdt, int M, int64_t ldx, v
   float* row_scale = (float*)((uint8_t*)ws + xbytes);
   const int ch = (Npad / 8 + 1023) / 1024;                         // 16-byte pieces per thread of the row kernel
   auto prep = ch <= 1 ? gemm_prep_kernel<1> : ch <= 3 ? gemm_prep_kernel<3> : gemm_prep_kernel<0>;
-  for (int v = 0; v < nv; ++v)                                     // one X' per col_scale vector
-    hipLaunchKernelGGL(prep, dim3((unsigned)Mpad), dim3(1024), 0, st,
-                       (const uint16_t*)x, ldx, m.cs ? m.cs + (size_t)v * m.N : nullptr, xdt, M, m.N, Npad,
-                       (uint16_t*)ws + (size_t)v * Mpad * Npad, row_scale + (size_t)v * Mpad);
+  hipLaunchKernelGGL(prep, dim3((unsigned)Mpad, (unsigned)nv), dim3(1024), 0, st, (const uint16_t*)x, ldx, m.cs, xdt, M, m.N, Npad,
+                     (uint16_t*)ws, (size_t)Mpad * Npad, row_scale, Mpad);   // one X' per col_scale vector
   GbArgs a;
   a.m = m; a.xp = (const uint16_t*)ws; a.M = M; a.Npad = Npad; a.y = y; a.ydt = ydt; a.ldy = ldy; a.bias = bias;
   a.par = par; a.xps = (size_t)Mpad * Npad;

@@ -1,0 +1,510 @@
+// GEMM for calls of nine to a few hundred activation rows:  Y[M, K] = X[M, N] . W_hat[K, N]^T.
+//
+// What bounds such a call is decoding the weights once, in vector instructions per weight, so the kernel
+// is built around that.
+//  * A decoded octet of columns never leaves the registers of the lane that decoded it: the B operand of
+//    v_mfma_f32_32x32x16_f16 is, per lane, eight columns of one weight row, what one mask byte decodes
+//    to.  A wavefront owns 64 weight rows (two such operands) and up to 64 activation rows.  There is no
+//    weight tile in LDS and no barrier in the loop; two wavefronts per SIMD cover each other's waits.
+//  * Everything is a byte permute: codes to their columns, the zero point into the pruned columns (which
+//    so subtract to 0), bytes to halves (0x6400 | code is 1024 + code, exact).
+//  * Tiles of up to 64 tokens multiply these halves as they are.  Once per quantisation group the float32
+//    sum is corrected by -(1024 + zero) * sum(X' of the group), one more matrix step whose A operand is
+//    that sum (as two halves), and multiplied by the group's scale on its way into the result: 37 vector
+//    instructions per step of 16 columns x 64 rows where a subtraction and a multiplication per weight
+//    need 52, and weights that are not rounded at all; the cancellation costs 2^-24 * 1024 /
+//    |code - zero|, below the 2^-12 of rounding (code - zero) * scale to a half.  Tiles of 96 tokens have
+//    no registers for a second set of sums; they subtract and multiply per weight.
+//
+// k order.  A step is eight columns of the first half of a group (lanes 0-31) and eight of the second
+// (lanes 32-63): a lane walks half a group of its own row, nothing is loaded or ranked twice.  The
+// activations X' = fp16(x * col_scale / s_m) are written in that order by the preparation kernel, as
+// whole 1 KB fragments [group][step][32-token block][lane], and come from L2 straight into registers,
+// several steps ahead.  s_m is the power of two that brings a token's largest |x * col_scale| into
+// [128, 256): neither X' nor the sum of a group leaves the range of a half, and the scaling is exact.
+//
+// A workgroup is eight wavefronts: two row groups of 64 rows (for a gate/up matrix: the even and the
+// odd rows of 128) times four parts of the column range.  The parts are added through LDS in part
+// order, so results do not depend on timing; where the rows alone do not fill the chip the column
+// range is also split over workgroups, which leave float32 partial tiles for a second kernel.
+// Because gate and up of an output meet in that sum, act(gate) * up costs no pass of its own.
+#pragma once
+#include <atomic>
+#include <type_traits>
+#include "cbk_octet.h"
+
+namespace cbk {
+
+constexpr int SK_WC = 4, SK_WR = 2;            // column parts and row groups of a workgroup
+constexpr int SK_ROWS = 64;                    // weight rows per wavefront
+constexpr int SK_PITCH = 72;                   // floats per token row of a wavefront's tile in LDS: lanes l and l + 32 write
+                                               // four token rows apart, 288 floats = 32 banks
+constexpr int SK_LUT_LANES = 16;               // lane-private copies of the selector table (16 lanes read 256 bytes at a time)
+constexpr int SK_LUT = 256 * SK_LUT_LANES * 16;
+constexpr size_t SK_LDS = (size_t)SK_WC * SK_WR * 32 * SK_PITCH * 4 + SK_LUT;
+
+typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+
+struct SkArgs {
+  DMat m;
+  const uint16_t* xp;      // fragments of X' [vector][token tile][group][steps][TI][64][8]
+  const uint32_t* xc;      // sums of X' over a group, two halves each [vector][token tile][group][32 TI]
+  size_t xcs;              // their distance between two vectors
+  const float* row_scale;  // [vector][rss]
+  int rss;
+  size_t xps;              // halfs between the fragments of two col_scale vectors
+  int M;
+  void* y;
+  int ydt;
+  int64_t ldy;
+  const void* bias;
+  int tiles_t, tiles_r, nsplit;
+  int par;                 // gate/up matrix: row group w of a workgroup takes the rows of parity w, with vector w
+  int act;                 // par only: -1, or the activation of act(gate) * up (y is [M, K / 2])
+  int vs0, vs1;            // q|k|v matrix: rows from vs0 / vs1 on use vector 1 / 2 (multiples of 64)
+  float* part;             // nsplit > 1: partial tiles [nsplit][M][part_ld] instead of y
+  size_t part_stride;
+  int64_t part_ld;
+};
+
+__device__ inline float sk_act(int act, float g) {
+  if (act == CBK_ACT_SILU) return g / (1.f + __expf(-g));
+  const float k = 0.7978845608028654f;                              // sqrt(2 / pi)
+  return 0.5f * g * (1.f + tanhf(k * (g + 0.044715f * g * g * g)));
+}
+
+// four consecutive outputs
+__device__ inline void sk_store4(void* y, int ydt, size_t at, const float (&v)[4], int n, bool vec) {
+  if (ydt == CBK_F32) {
+    if (vec && n == 4) *(float4*)((float*)y + at) = make_float4(v[0], v[1], v[2], v[3]);
+    else for (int e = 0; e < 4; ++e) { if (e < n) ((float*)y)[at + e] = v[e]; }
+    return;
+  }
+  uint16_t h[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) h[e] = ydt == CBK_F16 ? f2h(v[e]) : f2bf(v[e]);
+  if (vec && n == 4) *(uint2*)((uint16_t*)y + at) = make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
+  else for (int e = 0; e < 4; ++e) { if (e < n) ((uint16_t*)y)[at + e] = h[e]; }
+}
+
+// What a lane reads of a row per group: half a group's columns, PBLK 32-column blocks.
+constexpr int sk_gcd(int a, int b) { return b ? sk_gcd(b, a % b) : a; }
+template <int BITS, int KEEP, int GRP, int TI>
+struct SkCfg {
+  static constexpr bool DENSE = KEEP == 0, HI2 = BITS == 6, B8 = BITS == 8;
+  static constexpr int PB = HI2 ? 4 : BITS;                         // bits per code in the stream
+  static constexpr int CB = (DENSE ? 32 : KEEP) * PB;               // code bits of a block
+  static constexpr int PBLK = GRP / 64, ST = GRP / 16;              // blocks per lane and steps per group
+  static constexpr int HB = PBLK * CB;                              // code bits of a lane's run
+  static constexpr int ND = (HB + 31) / 32;
+  static constexpr bool WHOLE = HB == 32 || HB == 64 || HB % 128 == 0;   // the run starts on a dword / 8 / 16 bytes of its own
+  static constexpr int UNITS = (128 - sk_gcd(HB, 128) + HB + 127) / 128; // else: 16-byte units that hold it at any skew
+  static constexpr int NL = WHOLE ? ND : 4 * UNITS;
+  static constexpr int SB = BITS == 3 ? 4 : PB;                     // stream code width after expansion
+  static constexpr int NW = ((DENSE ? 32 : KEEP) * SB + 31) / 32;   // dwords of a block's stream
+  static constexpr int NG = GRP == 64 ? 3 : 2;                      // groups in flight
+  static constexpr int RG = (DENSE ? 0 : PBLK) + NL + (HI2 ? PBLK : 0) + 2;   // registers of a group and row
+  // scale and zero point per group instead of per weight: where the registers hold a second set of sums
+  // (without spilling: read off the compiler's report)
+  static constexpr bool DEFER = TI == 1 || (TI == 2 && 2 * NG * RG <= (DENSE ? 40 : GRP == 128 ? 32 : 24));
+  static constexpr int NA = TI == 1 || (TI == 2 && !DEFER) ? 8 : 4; // activation fragments in flight (steps)
+  // order of the columns of an octet in a fragment: the order the codes come out of the stream
+  static constexpr int ORDER = !DENSE || B8 ? 0 : BITS == 2 ? 2 : 1;
+};
+
+// BITS 2 / 3 / 4 / 6 with KEEP survivors per 32 columns, or KEEP = 0 for dense 2 / 3 / 4 / 8-bit codes; any zero
+// point.  TI: 32-token blocks of the tile.
+template <int BITS, int KEEP, int GRP, int TI>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_skinny_kernel(SkArgs a) {
+  using C = SkCfg<BITS, KEEP, GRP, TI>;
+  constexpr bool BITMAP = !C::DENSE;
+  constexpr bool DEFER = C::DEFER;
+  constexpr int ST = C::ST, NG = C::NG, NA = C::NA;
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  float* red = (float*)smem;
+  uint4* lut = (uint4*)(smem + (size_t)SK_WC * SK_WR * 32 * SK_PITCH * 4);   // [256][copies]: selectors, byte masks
+  const DMat& m = a.m;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wave & 1, wc = wave >> 1, half = lane >> 5;
+  if (BITMAP) {
+    if (tid < 256) {
+      const uint2 e = make_selectors((uint32_t)tid, BITS == 2 ? 1 : 0);
+      // 6-bit: all ones in the pruned bytes; else the field of a code in the kept ones
+      constexpr uint32_t F = C::HI2 ? 0xFFu : C::SB == 4 ? 0x0Fu : 0x03u;
+      const uint32_t k0 = bits_to_bytes((uint32_t)tid) * F, k1 = bits_to_bytes((uint32_t)tid >> 4) * F;
+#pragma unroll
+      for (int j = 0; j < SK_LUT_LANES; ++j) lut[tid * SK_LUT_LANES + j] = make_uint4(e.x, e.y, C::HI2 ? ~k0 : k0, C::HI2 ? ~k1 : k1);
+    }
+    __syncthreads();
+  }
+  // XCD-aware order: workgroups of one XCD (blockIdx % 8) take neighbouring tiles: the parts and token tiles of a
+  // row range read the same weights
+  const int nb = a.tiles_t * a.tiles_r * a.nsplit, per = (nb + 7) >> 3;
+  const int lin = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || lin >= nb) return;
+  const int tt = lin % a.tiles_t, rest = lin / a.tiles_t, sp = rest % a.nsplit, tr = rest / a.nsplit;
+  const int kstep = a.par ? 2 : 1;
+  const int r0 = tr * (SK_ROWS * SK_WR) + (a.par ? wr : SK_ROWS * wr);       // first row of this wavefront
+  // its groups: the row's cut into nsplit * SK_WC parts
+  const int q = sp * SK_WC + wc, nq = a.nsplit * SK_WC;
+  const int g0 = (int)((int64_t)m.G * q / nq), g1 = (int)((int64_t)m.G * (q + 1) / nq);
+  const int xv = a.par ? wr : (r0 >= a.vs0 ? 1 : 0) + (r0 >= a.vs1 ? 1 : 0);
+
+  v16f tot[TI][2];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) tot[i][j][e] = 0.f;
+
+  if (g0 < g1) {
+    // Addresses: a scalar base that moves with the group plus a 32-bit offset per lane that does not.  The base row
+    // is inside the matrix even where the wavefront's rows are not (those are decoded and never stored).
+    const int rb = r0 < m.K ? r0 : m.K - 1;
+    const uint32_t ush = m.tiled ? 256u : 16u;                      // bytes between the 16-byte units of a row
+    const uint8_t* dbase = m.data + (m.tiled ? (size_t)(rb >> 4) * m.stride * 16 : (size_t)rb * m.stride);
+    const size_t mbase = m.tiled ? (size_t)(rb >> 4) * m.G * 16 : (size_t)rb * m.G;
+    uint32_t roff[2], moff[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int r = r0 + kstep * (32 * j + (lane & 31)), rc = r < m.K ? r : m.K - 1;
+      roff[j] = m.tiled ? (uint32_t)((rc >> 4) - (rb >> 4)) * m.stride * 16u + (uint32_t)(rc & 15) * 16u : (uint32_t)(rc - rb) * m.stride;
+      moff[j] = m.tiled ? (uint32_t)((rc >> 4) - (rb >> 4)) * (uint32_t)m.G * 16u + (uint32_t)(rc & 15) : (uint32_t)(rc - rb) * (uint32_t)m.G;
+    }
+    const uint32_t lut_lane = (uint32_t)(lane & (SK_LUT_LANES - 1)) * 16u;
+    struct Grp {
+      uint32_t m[BITMAP ? C::PBLK : 1];
+      uint32_t raw[C::NL];
+      uint32_t h2[C::HI2 ? C::PBLK : 1];
+      uint32_t z, s;
+    };
+    auto load_group = [&](int g, Grp (&w)[2]) {
+      g = g < g1 ? g : g1 - 1;
+      const uint32_t ug = (uint32_t)g;
+      // mask words (and, for one-dword runs, codes): 8 PBLK bytes per group and row, the upper half's behind the lower's
+      const uint32_t go8 = C::PBLK == 2 ? ug * ush : (ug >> 1) * ush + (ug & 1u) * 8u, lo8 = (uint32_t)half * (C::PBLK * 4u);
+      // first unit of a skewed run
+      const uint32_t uskew = ((2u * ug + (uint32_t)half) * (uint32_t)C::HB >> 7) * ush;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        if (BITMAP) {
+          const uint8_t* p = dbase + go8 + (roff[j] + lo8);
+          if (C::PBLK == 2) { const uint2 v = *(const uint2*)p; w[j].m[0] = v.x; w[j].m[C::PBLK - 1] = v.y; }
+          else w[j].m[0] = *(const uint32_t*)p;
+        }
+        if (C::HI2) {                                               // behind the mask and nibble planes
+          const uint2 v = *(const uint2*)(dbase + (size_t)(m.N * 3 >> 7) * ush + ug * ush + (roff[j] + (uint32_t)half * 8u));
+          w[j].h2[0] = v.x; w[j].h2[C::HI2 ? C::PBLK - 1 : 0] = v.y;
+        }
+        const uint8_t* cbase = dbase + (m.code_off >> 4) * ush;     // the mask plane is whole units
+        if constexpr (C::HB == 32) w[j].raw[0] = *(const uint32_t*)(cbase + go8 + (roff[j] + lo8));
+        else if constexpr (C::HB == 64) {
+          const uint2 v = *(const uint2*)(cbase + ug * ush + (roff[j] + (uint32_t)half * 8u));
+          w[j].raw[0] = v.x; w[j].raw[1] = v.y;
+        } else {
+#pragma unroll
+          for (int i = 0; i < C::NL / 4; ++i) {
+            const uint8_t* p = C::WHOLE ? cbase + (ug * (2 * C::HB / 128) + i) * ush + (roff[j] + (uint32_t)half * (C::HB / 128) * ush)
+                                        : cbase + i * ush + (roff[j] + uskew);
+            const uint4 v = *(const uint4*)p;
+            w[j].raw[4 * i] = v.x; w[j].raw[4 * i + 1] = v.y; w[j].raw[4 * i + 2] = v.z; w[j].raw[4 * i + 3] = v.w;
+          }
+        }
+        const size_t mg = mbase + (m.tiled ? ug * 16u : ug);
+        w[j].z = (m.zero + mg)[moff[j]];
+        w[j].s = (m.scale + mg)[moff[j]];
+      }
+    };
+    // activation fragments of step t and group sums of group g (counted from the wavefront's first)
+    const uint8_t* xb = (const uint8_t*)(a.xp + (size_t)xv * a.xps) + ((size_t)tt * m.G + g0) * (ST * TI * 1024);
+    const uint32_t* xcb = a.xc + (size_t)xv * a.xcs + ((size_t)tt * m.G + g0) * (TI * 32);
+    v8h af[NA][TI];
+    uint32_t xs[TI];
+    uint32_t lane16 = (uint32_t)lane * 16u;
+    asm("" : "+v"(lane16));                                         // keep it an offset of its own: scalar base + 32-bit offset loads
+    const int steps = (g1 - g0) * ST;
+    auto load_a = [&](int t, int buf) {
+      const uint8_t* p = xb + (size_t)((uint32_t)(t < steps ? t : steps - 1) * (TI * 1024u));
+#pragma unroll
+      for (int i = 0; i < TI; ++i) af[buf][i] = *(const v8h*)(p + i * 1024 + lane16);
+    };
+    auto load_sums = [&](int g) {
+      const uint32_t* p = xcb + (size_t)((uint32_t)(g < g1 - g0 ? g : g1 - g0 - 1) * (TI * 32u));
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+        if (DEFER) xs[i] = p[(uint32_t)(lane & 31) + i * 32u];
+    };
+    const uint32_t first_half = (uint32_t)half - 1u;                // all ones in lanes 0-31
+    Grp ring[NG][2];
+    load_sums(0);
+#pragma unroll
+    for (int u = 0; u < NG; ++u) load_group(g0 + u, ring[u]);
+#pragma unroll
+    for (int t = 0; t < NA - 1; ++t) load_a(t, t);
+
+    // T0: position of the group's first step in the ring of activation fragments
+    auto group = [&](int g, Grp (&w)[2], auto t0_tag, auto more_tag) {
+      constexpr int T0 = decltype(t0_tag)::value;
+      constexpr bool more = decltype(more_tag)::value;
+      uint32_t cw[2][C::ND], st[2][C::NW], z4[2];
+      h2_t off[2], sh[2];                                           // !DEFER: -(1024 + zero) and scale
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        if constexpr (C::WHOLE) {
+#pragma unroll
+          for (int i = 0; i < C::ND; ++i) cw[j][i] = w[j].raw[i];
+        } else {
+          skew_dwords<C::NL, C::ND, C::HB % 32 == 0>(w[j].raw, ((2u * (uint32_t)g + (uint32_t)half) * (uint32_t)C::HB) & 127u, cw[j]);
+        }
+        z4[j] = perm(0, w[j].z, 0);                                 // the zero point in every byte
+        const _Float16 n = (_Float16)(-1024.0f - (float)w[j].z), f = __builtin_bit_cast(_Float16, (uint16_t)w[j].s);
+        off[j] = h2_t{n, n}; sh[j] = h2_t{f, f};
+      }
+      uint4 sel[2][2];
+      auto rank = [](uint32_t mw, int jj) { return (uint32_t)__builtin_popcount(mw & ((1u << (8 * jj)) - 1u)); };
+      auto fetch = [&](int o, uint4 (&e)[2]) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          if (BITMAP)                                               // entry address: mask byte in byte 1, this lane's copy in byte 0
+            e[j] = *(const uint4*)((const uint8_t*)lut + perm(w[j].m[BITMAP ? o >> 2 : 0], lut_lane, 0x0C0C0400u + ((uint32_t)(o & 3) << 8)));
+      };
+      // octet o of both rows -> the B operands of a step
+      auto decode = [&](int o, const uint4 (&e)[2], v8h (&bf)[2]) {
+        const int blk = o >> 2, jj = o & 3;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const uint32_t k64 = 0x64646464u;
+          uint32_t h[4];
+          if constexpr (C::B8) {
+            const uint32_t b0 = cw[j][2 * o], b1 = cw[j][2 * o + 1];
+            h[0] = perm(k64, b0, 0x04010400u); h[1] = perm(k64, b0, 0x04030402u);
+            h[2] = perm(k64, b1, 0x04010400u); h[3] = perm(k64, b1, 0x04030402u);
+          } else {
+            if (jj == 0) {
+#pragma unroll
+              for (int k = 0; k < C::NW; ++k)
+                st[j][k] = BITS == 3 ? expand3to4(get32<C::ND>(cw[j], blk * C::CB + 24 * k)) : get32<C::ND>(cw[j], blk * C::CB + 32 * k);
+            }
+            uint32_t win = BITMAP ? (jj == 0 ? st[j][0] : window<C::NW>(st[j], rank(w[j].m[BITMAP ? blk : 0], jj) * C::SB))
+                                  : C::SB == 4 ? st[j][jj] : (st[j][jj >> 1] >> (16 * (jj & 1)));
+            if (C::SB == 2) { win &= 0xFFFFu; win |= win << 14; }   // bytes c0 c4 c1 c5; four bits up c2 c6 c3 c7
+            if (BITMAP) {
+              // even and odd codes in the low bits of their bytes, the neighbour's bits above them
+              uint32_t q0 = win, q1 = win >> 4, b0, b1;
+              if (C::HI2) {
+                uint32_t h0, h1;
+                hi2_pools(w[j].h2[C::HI2 ? blk : 0], jj == 0 ? 0u : rank(w[j].m[BITMAP ? blk : 0], jj), h0, h1);
+                b0 = perm((q1 & 0x0F0F0F0Fu) | h1, (q0 & 0x0F0F0F0Fu) | h0, e[j].x) | (e[j].z & z4[j]);
+                b1 = perm((q1 & 0x0F0F0F0Fu) | h1, (q0 & 0x0F0F0F0Fu) | h0, e[j].y) | (e[j].w & z4[j]);
+              } else {                                              // a kept column's field, the zero point elsewhere (it has no bits there
+                b0 = mask_select(e[j].z, z4[j], perm(q1, q0, e[j].x));   // in a kept column: it is a code itself)
+                b1 = mask_select(e[j].w, z4[j], perm(q1, q0, e[j].y));
+              }
+              h[0] = perm(k64, b0, 0x04010400u); h[1] = perm(k64, b0, 0x04030402u);
+              h[2] = perm(k64, b1, 0x04010400u); h[3] = perm(k64, b1, 0x04030402u);
+            } else {                                                // columns in stream order (SkCfg::ORDER)
+              constexpr uint32_t F = C::SB == 4 ? 0x0F0F0F0Fu : 0x03030303u;
+              const uint32_t q0 = win & F, q1 = (win >> 4) & F;
+              h[0] = perm(k64, q0, 0x04010400u); h[1] = perm(k64, q0, 0x04030402u);
+              h[2] = perm(k64, q1, 0x04010400u); h[3] = perm(k64, q1, 0x04030402u);
+            }
+          }
+          if (!DEFER) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              h[i] = __builtin_bit_cast(uint32_t, (h2_t)((__builtin_bit_cast(h2_t, h[i]) + off[j]) * sh[j]));
+          }
+          const uint4 hv = make_uint4(h[0], h[1], h[2], h[3]);
+          bf[j] = __builtin_bit_cast(v8h, hv);
+        }
+      };
+      v8h bf[2][2];
+      fetch(0, sel[0]);
+      if (ST > 1) fetch(1, sel[1]);
+      // -(1024 + zero) against the two halves of the group's sum, in the lanes of the first half only
+      v16f part[DEFER ? TI : 1][2];
+      if constexpr (DEFER) {
+        v8h bz[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const uint32_t nn = perm(0, (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)off[j][0]), 0x01000100u) & first_half;
+          bz[j] = __builtin_bit_cast(v8h, make_uint4(nn, 0, 0, 0));
+        }
+#pragma unroll
+        for (int i = 0; i < TI; ++i) {
+          const v8h az = __builtin_bit_cast(v8h, make_uint4(xs[i], 0, 0, 0));
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            v16f zero16;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) zero16[e] = 0.f;
+            part[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(az, bz[j], zero16, 0, 0, 0);
+          }
+        }
+        load_sums(g - g0 + 1);
+      }
+      decode(0, sel[0], bf[0]);
+      __builtin_amdgcn_sched_barrier(0);
+      // Step o multiplies octet o while octet o + 1 is decoded and the selectors of octet o + 2 are fetched
+      const int t0 = (g - g0) * ST;
+#pragma unroll
+      for (int o = 0; o < ST; ++o) {
+        load_a(t0 + o + NA - 1, (T0 + o + NA - 1) % NA);
+        if (o + 2 < ST) fetch(o + 2, sel[o & 1]);
+        if (o + 1 < ST) decode(o + 1, sel[(o + 1) & 1], bf[(o + 1) & 1]);
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            v16f& d = DEFER ? part[DEFER ? i : 0][j] : tot[i][j];
+            d = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[(T0 + o) % NA][i], bf[o & 1][j], d, 0, 0, 0);
+          }
+#pragma unroll
+        for (int k = 0; k < 2 * TI; ++k) {                          // a matrix instruction, then a slice of the decode
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, DEFER ? 18 / TI : 8, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      float sc[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) sc[j] = h2f((uint16_t)w[j].s);
+      if (more) load_group(g + NG, w);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (DEFER) {
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) tot[i][j][e] = fmaf(part[i][j][e], sc[j], tot[i][j][e]);
+      }
+    };
+    // No branch between the groups of a trip: where paths join, the compiler waits for every load in
+    // flight.  A trip is UG groups: whole turns of both rings.
+    constexpr int UG = NG == 3 && ST % NA ? 6 : NG;
+    static_assert(UG % NG == 0 && UG * ST % NA == 0, "both rings turn a whole number of times per trip");
+    using Yes = std::true_type; using No = std::false_type;
+    int g = g0;
+    for (; g + UG <= g1; g += UG) {
+      group(g, ring[0], std::integral_constant<int, 0>{}, Yes{});
+      group(g + 1, ring[1 % NG], std::integral_constant<int, ST % NA>{}, Yes{});
+      if constexpr (UG > 2) group(g + 2, ring[2 % NG], std::integral_constant<int, 2 * ST % NA>{}, Yes{});
+      if constexpr (UG > 3) {
+        group(g + 3, ring[3 % NG], std::integral_constant<int, 3 * ST % NA>{}, Yes{});
+        group(g + 4, ring[4 % NG], std::integral_constant<int, 4 * ST % NA>{}, Yes{});
+        group(g + 5, ring[5 % NG], std::integral_constant<int, 5 * ST % NA>{}, Yes{});
+      }
+    }
+    if (g < g1) group(g, ring[0], std::integral_constant<int, 0>{}, Yes{});
+    if constexpr (UG > 2) {
+      if (g + 1 < g1) group(g + 1, ring[1 % NG], std::integral_constant<int, ST % NA>{}, Yes{});
+    }
+    if constexpr (UG > 3) {
+      if (g + 2 < g1) group(g + 2, ring[2 % NG], std::integral_constant<int, 2 * ST % NA>{}, Yes{});
+      if (g + 3 < g1) group(g + 3, ring[3 % NG], std::integral_constant<int, 3 * ST % NA>{}, Yes{});
+      if (g + 4 < g1) group(g + 4, ring[4 % NG], std::integral_constant<int, 4 * ST % NA>{}, No{});
+    }
+  }
+
+  // ---- the four column parts through LDS, 32 tokens at a time.  D[r] of lane l: token 8 (r / 4) + 4 (l / 32) +
+  // r % 4 of the block, weight row l % 32 of the 32.  Then a thread owns four rows of both row groups of one token.
+  const int tok0 = tt * 32 * TI;
+  const int et = tid >> 4, eq = (tid & 15) * 4;
+  const size_t esz = a.ydt == CBK_F32 ? 4 : 2;
+  const int rg0 = tr * (SK_ROWS * SK_WR), rg1 = rg0 + SK_ROWS;
+  const int xg[2] = {a.par ? 0 : (rg0 >= a.vs0 ? 1 : 0) + (rg0 >= a.vs1 ? 1 : 0),       // vectors of the two row groups
+                     a.par ? 1 : (rg1 >= a.vs0 ? 1 : 0) + (rg1 >= a.vs1 ? 1 : 0)};
+#pragma unroll
+  for (int i = 0; i < TI; ++i) {
+    __syncthreads();                                                // the tile of the block before has been read
+    float* mine = red + (size_t)(wc * SK_WR + wr) * 32 * SK_PITCH;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        mine[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * SK_PITCH + 32 * j + (lane & 31)] = tot[i][j][r];
+    __syncthreads();
+    const int tok = tok0 + 32 * i + et;
+    if (tok >= a.M) continue;                                       // (no barrier is skipped: the next one is reached by all)
+    float v[2][4];
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const float s = a.row_scale[(size_t)xg[g] * a.rss + tok];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[g][e] = 0.f;
+#pragma unroll
+      for (int c = 0; c < SK_WC; ++c) {
+        const float4 f = *(const float4*)(red + (size_t)(c * SK_WR + g) * 32 * SK_PITCH + et * SK_PITCH + eq);
+        v[g][0] += f.x; v[g][1] += f.y; v[g][2] += f.z; v[g][3] += f.w;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[g][e] *= s;
+    }
+    const bool part = a.nsplit > 1;
+    void* y = part ? (void*)(a.part + (size_t)sp * a.part_stride) : a.y;
+    const int ydt = part ? (int)CBK_F32 : a.ydt;
+    const int64_t ld = part ? a.part_ld : a.ldy;
+    const size_t es = part ? 4 : esz;
+    if (!part && a.bias) {
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int k = a.par ? rg0 + 2 * (eq + e) + g : rg0 + SK_ROWS * g + eq + e;
+          if (k < m.K) v[g][e] += a.ydt == CBK_F32 ? ((const float*)a.bias)[k] : a.ydt == CBK_F16 ? h2f(((const uint16_t*)a.bias)[k]) : bf2f(((const uint16_t*)a.bias)[k]);
+        }
+    }
+    const bool vec = ((((uintptr_t)y) | (uintptr_t)(ld * (int64_t)es)) & (4 * es - 1)) == 0;
+    if (!a.par) {
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const int k = rg0 + SK_ROWS * g + eq;
+        sk_store4(y, ydt, (size_t)tok * ld + k, v[g], m.K - k, vec);
+      }
+    } else if (a.act >= 0 && !part) {
+      float o[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = sk_act(a.act, v[0][e]) * v[1][e];
+      const int k = (rg0 >> 1) + eq;
+      sk_store4(y, ydt, (size_t)tok * ld + k, o, (m.K >> 1) - k, vec);
+    } else {
+      const int k = rg0 + 2 * eq;
+      const float lo[4] = {v[0][0], v[1][0], v[0][1], v[1][1]}, hi[4] = {v[0][2], v[1][2], v[0][3], v[1][3]};
+      sk_store4(y, ydt, (size_t)tok * ld + k, lo, m.K - k, vec);
+      sk_store4(y, ydt, (size_t)tok * ld + k + 4, hi, m.K - k - 4, vec);
+    }
+  }
+}
+
+template <int BITS, int KEEP, int GRP, int TI>
+static int launch_skinny_ti(const SkArgs& a, int blocks, hipStream_t st) {
+  auto kern = gemm_skinny_kernel<BITS, KEEP, GRP, TI>;
+  static std::atomic<int> configured{0};
+  if (!configured.load(std::memory_order_acquire)) {
+    if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
+      return CBK_ERR_HIP;
+    configured.store(1, std::memory_order_release);
+  }
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(512), SK_LDS, st, a);
+  return hipGetLastError() == hipSuccess ? CBK_OK : CBK_ERR_HIP;
+}
+template <int BITS, int KEEP, int GRP>
+static int launch_skinny_cfg(const SkArgs& a, int ti, int blocks, hipStream_t st) {
+  return ti == 1 ? launch_skinny_ti<BITS, KEEP, GRP, 1>(a, blocks, st)
+       : ti == 2 ? launch_skinny_ti<BITS, KEEP, GRP, 2>(a, blocks, st) : launch_skinny_ti<BITS, KEEP, GRP, 3>(a, blocks, st);
+}
+template <int BITS>
+static int launch_skinny_bits(const SkArgs& a, int keep, int group, int ti, int blocks, hipStream_t st) {
+#define CBK_SK_CASE(KEEP)                                                             \
+  case KEEP: return group == 64 ? launch_skinny_cfg<BITS, KEEP, 64>(a, ti, blocks, st) \
+                                : launch_skinny_cfg<BITS, KEEP, 128>(a, ti, blocks, st);
+  switch (keep) {
+    CBK_SK_CASE(0) CBK_SK_CASE(10) CBK_SK_CASE(16) CBK_SK_CASE(23)
+    default: return CBK_ERR_UNSUPPORTED;
+  }
+#undef CBK_SK_CASE
+}
+
+}  // namespace cbk

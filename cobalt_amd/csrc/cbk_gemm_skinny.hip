@@ -1,0 +1,244 @@
+// Preparation kernel, reduction kernels, plan and dispatch of the GEMM in cbk_gemm_skinny.h.
+#include "cbk_gemm_skinny.h"
+#include "cbk_prep.h"
+
+namespace cbk {
+
+int launch_skinny_b2(const SkArgs&, int keep, int group, int ti, int blocks, hipStream_t);
+int launch_skinny_b3(const SkArgs&, int keep, int group, int ti, int blocks, hipStream_t);
+int launch_skinny_b4(const SkArgs&, int keep, int group, int ti, int blocks, hipStream_t);
+int launch_skinny_b68(const SkArgs&, int bits, int group, int ti, int blocks, hipStream_t);
+
+// X' = fp16(x * col_scale / s_row) in fragment order and the sums of X' over the quantisation groups
+// (see cbk_gemm_skinny.h), for every column-scale vector (blockIdx.z).  A workgroup takes 2048 columns
+// of four tokens, whose 16-byte pieces of the same eight columns are neighbours in that order (64-byte
+// writes).  Every workgroup finds the tokens' largest |x * col_scale| over the whole row by itself: the
+// row comes from L2, and the call does not wait for one workgroup per four tokens to work through long
+// rows (16 tokens of 16384 columns: 19 -> 4 us).  Tokens past M are left unwritten, their outputs are
+// never stored.
+__device__ inline float skinny_scale(float mx) {                   // the power of two that brings mx into [128, 256)
+  if (!(mx > 0.f) || !(mx <= 3.4028234663852886e38f)) return 1.f;
+  int e = (int)((__float_as_uint(mx) >> 23) & 0xffu) - 7;          // its biased exponent
+  e = e < 1 ? 1 : e;
+  return __uint_as_float((uint32_t)e << 23);
+}
+__global__ __launch_bounds__(1024) void skinny_prep_kernel(const uint16_t* x, int64_t ldx, const uint16_t* cs, int xdt,
+                                                           int M, int N, int group, int order, int ti, uint16_t* out,
+                                                           size_t xps, uint32_t* sums, size_t xcs, float* row_scale, int rss) {
+  __shared__ float red[16][4];
+  const int tid = threadIdx.x, tl = tid & 3, tok = blockIdx.x * 4 + tl, v = blockIdx.z;
+  const bool ok = tok < M;
+  const int n8 = N >> 3, G = N / group, st = group >> 4;            // N is a multiple of 128
+  const uint16_t* xr = x + (size_t)(ok ? tok : M - 1) * ldx;
+  const uint16_t* cv = cs ? cs + (size_t)v * N : nullptr;
+  const uint4 one = make_uint4(0x3c003c00u, 0x3c003c00u, 0x3c003c00u, 0x3c003c00u);
+  const int mine = blockIdx.y * 256 + (tid >> 2);                   // this thread's eight columns
+  const bool has = mine < n8;
+  const uint4 xm = has ? *(const uint4*)(xr + mine * 8) : make_uint4(0, 0, 0, 0);
+  const uint4 cm = has && cv ? *(const uint4*)(cv + mine * 8) : one;
+  float mx = 0.f;
+#pragma unroll 4
+  for (int c8 = tid >> 2; c8 < n8; c8 += 256) {
+    float a[8];
+    prep8(*(const uint4*)(xr + c8 * 8), cv ? *(const uint4*)(cv + c8 * 8) : one, xdt, a);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(a[e]));
+  }
+#pragma unroll
+  for (int o = 4; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+  if ((tid & 63) < 4) red[tid >> 6][tl] = mx;
+  __syncthreads();
+  float all = red[0][tl];
+#pragma unroll
+  for (int w = 1; w < 16; ++w) all = fmaxf(all, red[w][tl]);
+  const float s = skinny_scale(all), inv = 1.f / s;                 // powers of two
+  if (ok && tid < 4 && blockIdx.y == 0) row_scale[(size_t)v * rss + tok] = s;
+  if (!has) return;                                                 // (a wavefront's sixteen pieces are one 128-column chunk: all or none)
+  const int tile = tok / (32 * ti), i32 = tok % (32 * ti) / 32, l = tok & 31;
+  float a[8];
+  prep8(xm, cm, xdt, a);
+  uint16_t h[8];
+  float sum = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) { h[e] = f2h(a[e] * inv); sum += h2f(h[e]); }
+  uint32_t o[4];
+  if (order == 0) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = (uint32_t)h[2 * e] | ((uint32_t)h[2 * e + 1] << 16);
+  } else if (order == 1) {                                          // even columns, then odd ones
+    o[0] = (uint32_t)h[0] | ((uint32_t)h[2] << 16); o[1] = (uint32_t)h[4] | ((uint32_t)h[6] << 16);
+    o[2] = (uint32_t)h[1] | ((uint32_t)h[3] << 16); o[3] = (uint32_t)h[5] | ((uint32_t)h[7] << 16);
+  } else {                                                          // 0 4 1 5 2 6 3 7
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = (uint32_t)h[e] | ((uint32_t)h[e + 4] << 16);
+  }
+  const int col = mine * 8, g = col / group, w = col % group, hf = w / (group >> 1), t = w % (group >> 1) >> 3;
+  uint16_t* o0 = out + (size_t)v * xps + (((size_t)tile * G + g) * st + t) * (ti * 512) + i32 * 512 + hf * 256 + l * 8;
+  if (ok) *(uint4*)o0 = make_uint4(o[0], o[1], o[2], o[3]);
+#pragma unroll
+  for (int d = 4; d < 32; d <<= 1) sum += __shfl_xor(sum, d);       // eight pieces: 64 columns
+  if (group == 128) sum += __shfl_xor(sum, 32);
+  if (ok && w == 0) {
+    const uint16_t hi = f2h(sum), lo = f2h(sum - h2f(hi));
+    sums[(size_t)v * xcs + ((size_t)tile * G + g) * ti * 32 + i32 * 32 + l] = (uint32_t)hi | ((uint32_t)lo << 16);
+  }
+}
+
+// y = sum of the float32 partial tiles in part order (+ bias); ACT: act(gate) * up of the interleaved
+// gate / up sums.  Four outputs per thread.
+template <bool ACT>
+__global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* part, size_t part_stride, int64_t part_ld, int nsplit,
+                                                            int M, int K, const void* bias, void* y, int ydt, int64_t ldy,
+                                                            int act) {
+  constexpr int W = ACT ? 8 : 4;                                    // sums per thread
+  const int Ko = ACT ? K >> 1 : K, k4 = (Ko + 3) >> 2;
+  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (id >= (int64_t)M * k4) return;
+  const int tok = (int)(id / k4), o0 = (int)(id % k4) * 4, k0 = ACT ? 2 * o0 : o0;
+  float v[W];
+#pragma unroll
+  for (int e = 0; e < W; ++e) v[e] = 0.f;
+  const float* src = part + (size_t)tok * part_ld + k0;
+  for (int p = 0; p < nsplit; ++p)
+#pragma unroll
+    for (int h = 0; h < W / 4; ++h) {
+      const float4 f = ((const float4*)(src + (size_t)p * part_stride))[h];
+      v[4 * h] += f.x; v[4 * h + 1] += f.y; v[4 * h + 2] += f.z; v[4 * h + 3] += f.w;
+    }
+  if (bias)
+#pragma unroll
+    for (int e = 0; e < W; ++e)
+      if (k0 + e < K) v[e] += ydt == CBK_F32 ? ((const float*)bias)[k0 + e] : ydt == CBK_F16 ? h2f(((const uint16_t*)bias)[k0 + e]) : bf2f(((const uint16_t*)bias)[k0 + e]);
+  float o[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = ACT ? sk_act(act, v[ACT ? 2 * e : e]) * v[ACT ? 2 * e + 1 : e] : v[e];
+  const int esz = ydt == CBK_F32 ? 4 : 2;
+  const bool vec = (((uintptr_t)y | (uintptr_t)(ldy * esz)) & (4 * esz - 1)) == 0;
+  sk_store4(y, ydt, (size_t)tok * ldy + o0, o, Ko - o0, vec);
+}
+
+// ------------------------------------------------------------------ plan
+static inline size_t sk_up(size_t v) { return (v + 255) & ~(size_t)255; }
+
+// the matrices this kernel has a decoder for
+bool gemm_skinny_takes(const DMat& m) {
+  const int fam = family_of(m.layout);
+  if (fam == FAM_SPARSE || (m.group != 64 && m.group != 128)) return false;
+  if (m.cs_rows == 3 && (m.cs_split0 % SK_ROWS || (m.cs_split0 + m.cs_split1) % SK_ROWS)) return false;
+  // 32-bit offsets inside a wavefront's 128 rows
+  if ((uint64_t)m.stride * 160 >= (1ull << 32)) return false;
+  if (fam == FAM_DENSE) return true;
+  if (!(m.flags & CBK_FLAG_ZERO_ON_GRID)) return false;             // (a pruned column's zero point is decoded as a code)
+  if (fam == FAM_BLK6) return m.bits == 6 && m.keep == 16 && m.group == 128;
+  return m.keep == 10 || m.keep == 16 || m.keep == 23;
+}
+
+struct SkPlan { int ti, nsplit; double t; };
+// Times in microseconds, fitted to calls of ten shapes (1024 x 4096 to 43008 x 5376) at 16 to 1700 rows,
+// within a tenth of the measured ones: a group of a wavefront with two wavefronts per SIMD, by token tile
+// (codes that do not start on 16-byte units take a fifth longer), 5.5 to 10 per workgroup outside the
+// loop, 7.4 for the preparation kernel and the launches, 5.5 and the partial tiles at 4 TB/s for the
+// reduction kernel.
+static SkPlan sk_plan_ti(const DMat& m, int M, int ti, int max_split) {
+  const int tiles = ((M + 32 * ti - 1) / (32 * ti)) * ((m.K + SK_ROWS * SK_WR - 1) / (SK_ROWS * SK_WR));
+  static const double g128[3] = {1.7, 2.2, 2.8}, g64[3] = {1.17, 1.45, 1.53}, wg[3] = {5.5, 7.6, 10.0};
+  const bool skewed = family_of(m.layout) == FAM_BLK && (m.keep * m.bits * (m.group / 64)) % 32 != 0;
+  const double two = m.cs_rows == 2 ? 1.12 : 1.0;                   // (two sets of X' compete for L2)
+  const double t_group = (m.group == 128 ? g128 : g64)[ti - 1] * (skewed ? 1.2 : 1.0) * two, t_wg = wg[ti - 1] * two;
+  SkPlan best{ti, 1, 0};
+  for (int s = 1; s <= max_split; ++s) {
+    const int per = (m.G + SK_WC * s - 1) / (SK_WC * s);
+    double t = 7.4 + (double)((tiles * s + 255) / 256) * (per * t_group + t_wg);
+    if (s > 1) t += 2.0 * s * (double)M * m.K * 4 / 4.0e6 + 5.5;
+    if (s == 1 || t < best.t) { best.nsplit = s; best.t = t; }
+    if (SK_WC * s >= m.G) break;
+  }
+  return best;
+}
+static SkPlan sk_plan(const DMat& m, int M, int max_split = 16) {
+  SkPlan best = sk_plan_ti(m, M, 1, max_split);
+  for (int ti = 2; ti <= 3; ++ti) {
+    const SkPlan p = sk_plan_ti(m, M, ti, max_split);
+    if (p.t < best.t) best = p;
+  }
+  return best;
+}
+double gemm_skinny_time(const DMat& m, int M) { return sk_plan(m, M).t; }
+
+struct SkSpace { size_t x, sums, scale, part; int mpad; };
+static SkSpace sk_space(const DMat& m, int M, const SkPlan& p) {
+  SkSpace s;
+  s.mpad = (M + 32 * p.ti - 1) / (32 * p.ti) * (32 * p.ti);
+  const size_t nv = m.cs_rows > 1 ? m.cs_rows : 1;
+  s.x = sk_up(nv * s.mpad * m.N * 2);
+  s.sums = sk_up(nv * s.mpad * m.G * 4);
+  s.scale = sk_up(nv * s.mpad * 4);
+  s.part = p.nsplit > 1 ? sk_up((size_t)p.nsplit * M * ((m.K + 7) / 8 * 8) * 4) : 0;
+  return s;
+}
+static inline size_t sk_sum(const SkSpace& s) { return s.x + s.sums + s.scale + s.part; }
+// `room`: what the caller has, or (size_t)-1: the split is taken back where its partial tiles do not fit
+static SkPlan sk_fit(const DMat& m, int M, size_t room, SkSpace& s) {
+  SkPlan p = sk_plan(m, M);
+  s = sk_space(m, M, p);
+  if (sk_sum(s) > room) { p = sk_plan(m, M, 1); s = sk_space(m, M, p); }
+  return p;
+}
+size_t gemm_skinny_workspace(const DMat& m, int M, bool least) {
+  SkSpace s;
+  sk_fit(m, M, least ? 0 : (size_t)-1, s);
+  return sk_sum(s);
+}
+
+// act: -1, or CBK_ACT_*: y = act(gate) * up of a gate/up matrix, [M, K / 2]
+int launch_gemm_skinny(const DMat& m, const void* x, int xdt, int M, int64_t ldx, void* y, int ydt, int64_t ldy,
+                       const void* bias, int act, void* ws, size_t ws_bytes, hipStream_t st) {
+  if (!gemm_skinny_takes(m) || (act >= 0 && ((m.K & 1) || m.cs_rows == 3))) return CBK_ERR_UNSUPPORTED;
+  SkSpace sp;
+  const SkPlan plan = sk_fit(m, M, ws_bytes, sp);
+  if (!ws || ws_bytes < sk_sum(sp)) return CBK_ERR_WORKSPACE;
+  if ((uintptr_t)ws & 255) return CBK_ERR_ALIGN;
+  const int nv = m.cs_rows > 1 ? m.cs_rows : 1;
+  SkArgs a;
+  a.m = m; a.M = M; a.y = y; a.ydt = ydt; a.ldy = ldy; a.bias = bias;
+  a.xp = (const uint16_t*)ws;
+  a.xc = (const uint32_t*)((uint8_t*)ws + sp.x);
+  a.row_scale = (const float*)((uint8_t*)ws + sp.x + sp.sums);
+  a.par = m.cs_rows == 2 || act >= 0 ? 1 : 0;
+  a.act = act;
+  // (a gate/up matrix with one vector: both parities read the same X')
+  a.xps = nv > 1 ? (size_t)sp.mpad * m.N : 0;
+  a.xcs = nv > 1 ? (size_t)sp.mpad * m.G : 0;
+  a.rss = nv > 1 ? sp.mpad : 0;
+  a.vs0 = m.cs_rows == 3 ? m.cs_split0 : 0x7fffffff;
+  a.vs1 = m.cs_rows == 3 ? m.cs_split0 + m.cs_split1 : 0x7fffffff;
+  a.nsplit = plan.nsplit;
+  a.part = (float*)((uint8_t*)ws + sp.x + sp.sums + sp.scale);
+  a.part_ld = (m.K + 7) / 8 * 8;
+  a.part_stride = (size_t)M * a.part_ld;
+  a.tiles_t = sp.mpad / (32 * plan.ti);
+  a.tiles_r = (m.K + SK_ROWS * SK_WR - 1) / (SK_ROWS * SK_WR);
+  const int order = family_of(m.layout) != FAM_DENSE || m.bits == 8 ? 0 : m.bits == 2 ? 2 : 1;   // SkCfg::ORDER
+  hipLaunchKernelGGL(skinny_prep_kernel, dim3((unsigned)((M + 3) / 4), (unsigned)((m.N + 2047) / 2048), (unsigned)nv), dim3(1024),
+                     0, st, (const uint16_t*)x, ldx, m.cs, xdt, M, m.N, m.group, order, plan.ti, (uint16_t*)ws, a.xps,
+                     (uint32_t*)a.xc, a.xcs, (float*)a.row_scale, a.rss);
+  const int nb = a.tiles_t * a.tiles_r * a.nsplit, blocks = (nb + 7) / 8 * 8;
+  const int fam = family_of(m.layout), keep = fam == FAM_DENSE ? 0 : m.keep;
+  int rc;
+  if (m.bits == 8 || fam == FAM_BLK6) rc = launch_skinny_b68(a, m.bits, m.group, plan.ti, blocks, st);
+  else rc = m.bits == 2 ? launch_skinny_b2(a, keep, m.group, plan.ti, blocks, st)
+          : m.bits == 3 ? launch_skinny_b3(a, keep, m.group, plan.ti, blocks, st) : launch_skinny_b4(a, keep, m.group, plan.ti, blocks, st);
+  if (rc == CBK_OK && a.nsplit > 1) {
+    const int Ko = act >= 0 ? m.K / 2 : m.K;
+    const int64_t items = (int64_t)M * ((Ko + 3) / 4);
+    const dim3 grid((unsigned)((items + 255) / 256));
+    if (act >= 0) hipLaunchKernelGGL(skinny_reduce_kernel<true>, grid, dim3(256), 0, st, (const float*)a.part, a.part_stride,
+                                     a.part_ld, a.nsplit, M, m.K, bias, y, ydt, ldy, act);
+    else hipLaunchKernelGGL(skinny_reduce_kernel<false>, grid, dim3(256), 0, st, (const float*)a.part, a.part_stride,
+                            a.part_ld, a.nsplit, M, m.K, bias, y, ydt, ldy, act);
+    if (hipGetLastError() != hipSuccess) rc = CBK_ERR_HIP;
+  }
+  return rc;
+}
+
+}  // namespace cbk

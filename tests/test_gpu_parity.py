@@ -843,6 +843,29 @@ def test_gemm_every_kernel_configuration(case):
         assert torch.equal(y64, ops.gemm(pm, x[:50].to(DEV), out_dtype=torch.float32))
 
 
+@pytest.mark.parametrize("case", [(F.BLK1632_4, 4, 128, 16), (F.BLKC, 2, 64, 16), (F.BLKC, 3, 128, 23), (F.BLK1632_6, 6, 128, 16),
+                                  (F.DENSE4, 4, 128, 0), (F.DENSE8, 8, 128, 0), (F.DENSEB, 8, 64, 0), (F.DENSEB, 2, 64, 0)], ids=case_id)
+def test_gemm_token_tiles_of_32_64_and_96(case):
+    """The kernel of few tokens at the edges of its tiles: 32 / 64 / 96 tokens and one more, row groups of
+    64 and 128 and one more or less, one group of columns (fewer than the parts of a row), group counts
+    that are no multiple of what is in flight, both byte orders.  Against the oracle's float64 product:
+    two roundings to eleven bits, 2^-12 each, give 3e-4, so the layer tolerance holds with room; also for
+    activations of one sign, whose group sums are what 1024 + zero is taken off again from."""
+    for K, N, tiled in ((1, 128, True), (63, 384, False), (129, 1152, True), (191, 2304, False)):
+        raw = make_raw(case, K, N, seed=K + N)
+        pk = oracle_pack(case, raw)
+        pm = packed_from_oracle(case, pk, raw["col_scale"], K, N, DEV, tiled=tiled)
+        W = R.dequant(pk, K, N, case[0], col_scale=raw["col_scale"], **kw_of(case))
+        for M, dtype in ((9, torch.float16), (32, torch.bfloat16), (33, torch.float16), (64, torch.float16), (65, torch.bfloat16),
+                         (96, torch.float16), (97, torch.float16), (200, torch.bfloat16)):
+            x = acts(M, N, dtype, seed=M)
+            if M in (33, 96):
+                x = (x.float() * 0.05 + 1.0).to(dtype)
+            y = ops.gemm(pm, x.to(DEV), out_dtype=torch.float32)
+            err = rel_fro(_np(y), R.forward_ref(W, _np(x)))
+            assert err < TOL, f"{case_id(case)} {K}x{N} M={M}: {err}"
+
+
 def test_gemm_bias_dtype_and_prune_zero():
     case = (F.BLK1632_4, 4, 128, 16)
     K, N, M = 256, 2048, 300
