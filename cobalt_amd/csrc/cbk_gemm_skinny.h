@@ -20,8 +20,9 @@
 // (lanes 32-63): a lane walks half a group of its own row, nothing is loaded or ranked twice.  The
 // activations X' = fp16(x * col_scale / s_m) are written in that order by the preparation kernel, as
 // whole 1 KB fragments [group][step][32-token block][lane], and come from L2 straight into registers,
-// several steps ahead.  s_m is the power of two that brings a token's largest |x * col_scale| into
-// [128, 256): neither X' nor the sum of a group leaves the range of a half, and the scaling is exact.
+// several steps ahead.  s_m is the power of two that brings the largest |x * col_scale| of a token and
+// column part into [128, 256): neither X' nor the sum of a group leaves the range of a half, and the
+// scaling is exact.
 //
 // A workgroup is eight wavefronts: two row groups of 64 rows (for a gate/up matrix: the even and the
 // odd rows of 128) times four parts of the column range.  The parts are added through LDS in part
@@ -48,10 +49,10 @@ typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
 struct SkArgs {
   DMat m;
   const uint16_t* xp;      // fragments of X' [vector][token tile][group][steps][TI][64][8]
-  const uint32_t* xc;      // sums of X' over a group, two halves each [vector][token tile][group][32 TI]
+  const uint32_t* xc;      // sums of X' over the halves of a group, two halfs each [vector][token tile][group][2][32 TI]
   size_t xcs;              // their distance between two vectors
-  const float* row_scale;  // [vector][rss]
-  int rss;
+  const float* row_scale;  // [vector][part of the column range][rss]
+  int rss, rvs;            // floats between two parts / two vectors
   size_t xps;              // halfs between the fragments of two col_scale vectors
   int M;
   void* y;
@@ -126,17 +127,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const DMat& m = a.m;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = wave & 1, wc = wave >> 1, half = lane >> 5;
-  if (BITMAP) {
-    if (tid < 256) {
-      const uint2 e = make_selectors((uint32_t)tid, BITS == 2 ? 1 : 0);
-      // 6-bit: all ones in the pruned bytes; else the field of a code in the kept ones
-      constexpr uint32_t F = C::HI2 ? 0xFFu : C::SB == 4 ? 0x0Fu : 0x03u;
-      const uint32_t k0 = bits_to_bytes((uint32_t)tid) * F, k1 = bits_to_bytes((uint32_t)tid >> 4) * F;
-#pragma unroll
-      for (int j = 0; j < SK_LUT_LANES; ++j) lut[tid * SK_LUT_LANES + j] = make_uint4(e.x, e.y, C::HI2 ? ~k0 : k0, C::HI2 ? ~k1 : k1);
-    }
-    __syncthreads();
-  }
   // XCD-aware order: workgroups of one XCD (blockIdx % 8) take neighbouring tiles: the parts and token tiles of a
   // row range read the same weights
   const int nb = a.tiles_t * a.tiles_r * a.nsplit, per = (nb + 7) >> 3;
@@ -147,7 +137,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int r0 = tr * (SK_ROWS * SK_WR) + (a.par ? wr : SK_ROWS * wr);       // first row of this wavefront
   // its groups: the row's cut into nsplit * SK_WC parts
   const int q = sp * SK_WC + wc, nq = a.nsplit * SK_WC;
-  const int g0 = (int)((int64_t)m.G * q / nq), g1 = (int)((int64_t)m.G * (q + 1) / nq);
+  const int g0 = m.G * q / nq, g1 = m.G * (q + 1) / nq;
   const int xv = a.par ? wr : (r0 >= a.vs0 ? 1 : 0) + (r0 >= a.vs1 ? 1 : 0);
 
   v16f tot[TI][2];
@@ -158,6 +148,25 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
       for (int e = 0; e < 16; ++e) tot[i][j][e] = 0.f;
 
+  // Selector table, built while the first loads are in flight
+  auto build_table = [&]() {
+    if (BITMAP) {
+      if (tid < 256) {
+        const uint2 e = make_selectors((uint32_t)tid, BITS == 2 ? 1 : 0);
+        // 6-bit: all ones in the pruned bytes; else the field of a code in the kept ones
+        constexpr uint32_t F = C::HI2 ? 0xFFu : C::SB == 4 ? 0x0Fu : 0x03u;
+        const uint32_t k0 = bits_to_bytes((uint32_t)tid) * F, k1 = bits_to_bytes((uint32_t)tid >> 4) * F;
+#pragma unroll
+        for (int j = 0; j < SK_LUT_LANES; ++j) lut[tid * SK_LUT_LANES + j] = make_uint4(e.x, e.y, C::HI2 ? ~k0 : k0, C::HI2 ? ~k1 : k1);
+      }
+      // (a barrier over LDS only: __syncthreads() would wait for the loads in flight)
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    }
+  };
+
+  if (g0 >= g1) build_table();
   if (g0 < g1) {
     // Addresses: a scalar base that moves with the group plus a 32-bit offset per lane that does not.  The base row
     // is inside the matrix even where the wavefront's rows are not (those are decoded and never stored).
@@ -218,7 +227,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     };
     // activation fragments of step t and group sums of group g (counted from the wavefront's first)
     const uint8_t* xb = (const uint8_t*)(a.xp + (size_t)xv * a.xps) + ((size_t)tt * m.G + g0) * (ST * TI * 1024);
-    const uint32_t* xcb = a.xc + (size_t)xv * a.xcs + ((size_t)tt * m.G + g0) * (TI * 32);
+    const uint32_t* xcb = a.xc + (size_t)xv * a.xcs + ((size_t)tt * m.G + g0) * (2 * TI * 32);
     v8h af[NA][TI];
     uint32_t xs[TI];
     uint32_t lane16 = (uint32_t)lane * 16u;
@@ -230,12 +239,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int i = 0; i < TI; ++i) af[buf][i] = *(const v8h*)(p + i * 1024 + lane16);
     };
     auto load_sums = [&](int g) {
-      const uint32_t* p = xcb + (size_t)((uint32_t)(g < g1 - g0 ? g : g1 - g0 - 1) * (TI * 32u));
+      const uint32_t* p = xcb + (size_t)((uint32_t)(g < g1 - g0 ? g : g1 - g0 - 1) * (2u * TI * 32u));
 #pragma unroll
       for (int i = 0; i < TI; ++i)
-        if (DEFER) xs[i] = p[(uint32_t)(lane & 31) + i * 32u];
+        if (DEFER) xs[i] = p[(uint32_t)(lane & 31) + (uint32_t)half * (TI * 32u) + i * 32u];
     };
-    const uint32_t first_half = (uint32_t)half - 1u;                // all ones in lanes 0-31
     Grp ring[NG][2];
     load_sums(0);
 #pragma unroll
@@ -322,13 +330,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       v8h bf[2][2];
       fetch(0, sel[0]);
       if (ST > 1) fetch(1, sel[1]);
-      // -(1024 + zero) against the two halves of the group's sum, in the lanes of the first half only
+      // -(1024 + zero) against the sum of this lane's half of the group (as two halfs)
       v16f part[DEFER ? TI : 1][2];
       if constexpr (DEFER) {
         v8h bz[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          const uint32_t nn = perm(0, (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)off[j][0]), 0x01000100u) & first_half;
+          const uint32_t nn = perm(0, (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)off[j][0]), 0x01000100u);
           bz[j] = __builtin_bit_cast(v8h, make_uint4(nn, 0, 0, 0));
         }
 #pragma unroll
@@ -381,6 +389,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             for (int e = 0; e < 16; ++e) tot[i][j][e] = fmaf(part[i][j][e], sc[j], tot[i][j][e]);
       }
     };
+    build_table();
     // No branch between the groups of a trip: where paths join, the compiler waits for every load in
     // flight.  A trip is UG groups: whole turns of both rings.
     constexpr int UG = NG == 3 && ST % NA ? 6 : NG;
@@ -431,16 +440,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     float v[2][4];
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
-      const float s = a.row_scale[(size_t)xg[g] * a.rss + tok];
+      const float* s = a.row_scale + (size_t)xg[g] * a.rvs + (size_t)sp * SK_WC * a.rss + tok;
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[g][e] = 0.f;
 #pragma unroll
       for (int c = 0; c < SK_WC; ++c) {
         const float4 f = *(const float4*)(red + (size_t)(c * SK_WR + g) * 32 * SK_PITCH + et * SK_PITCH + eq);
-        v[g][0] += f.x; v[g][1] += f.y; v[g][2] += f.z; v[g][3] += f.w;
+        const float k = s[(size_t)c * a.rss];
+        v[g][0] = fmaf(f.x, k, v[g][0]); v[g][1] = fmaf(f.y, k, v[g][1]);
+        v[g][2] = fmaf(f.z, k, v[g][2]); v[g][3] = fmaf(f.w, k, v[g][3]);
       }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[g][e] *= s;
     }
     const bool part = a.nsplit > 1;
     void* y = part ? (void*)(a.part + (size_t)sp * a.part_stride) : a.y;

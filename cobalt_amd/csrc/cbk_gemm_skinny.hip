@@ -10,77 +10,100 @@ int launch_skinny_b4(const SkArgs&, int keep, int group, int ti, int blocks, hip
 int launch_skinny_b68(const SkArgs&, int bits, int group, int ti, int blocks, hipStream_t);
 
 // X' = fp16(x * col_scale / s_row) in fragment order and the sums of X' over the quantisation groups
-// (see cbk_gemm_skinny.h), for every column-scale vector (blockIdx.z).  A workgroup takes 2048 columns
-// of four tokens, whose 16-byte pieces of the same eight columns are neighbours in that order (64-byte
-// writes).  Every workgroup finds the tokens' largest |x * col_scale| over the whole row by itself: the
-// row comes from L2, and the call does not wait for one workgroup per four tokens to work through long
-// rows (16 tokens of 16384 columns: 19 -> 4 us).  Tokens past M are left unwritten, their outputs are
-// never stored.
+// (see cbk_gemm_skinny.h), for every column-scale vector (blockIdx.z) and every part of the column range
+// (blockIdx.y): a part is what one wavefront of the GEMM sums, so it has a scale per token of its own and
+// no workgroup needs to see a whole row.  A workgroup takes eight tokens, whose 16-byte pieces of the
+// same eight columns are a whole 128-byte line in that order.  Tokens past M are left unwritten, their
+// outputs are never stored.  CH: pieces of the part a thread keeps in registers between the range pass
+// and the write; 0 = any length, read twice.  (A scale per token over the whole row, found by one workgroup per
+// four tokens or by every workgroup again, and half lines: 48 rows of 14336 columns 9 us, 512 rows 31.)
 __device__ inline float skinny_scale(float mx) {                   // the power of two that brings mx into [128, 256)
   if (!(mx > 0.f) || !(mx <= 3.4028234663852886e38f)) return 1.f;
   int e = (int)((__float_as_uint(mx) >> 23) & 0xffu) - 7;          // its biased exponent
   e = e < 1 ? 1 : e;
   return __uint_as_float((uint32_t)e << 23);
 }
+template <int CH>
 __global__ __launch_bounds__(1024) void skinny_prep_kernel(const uint16_t* x, int64_t ldx, const uint16_t* cs, int xdt,
-                                                           int M, int N, int group, int order, int ti, uint16_t* out,
-                                                           size_t xps, uint32_t* sums, size_t xcs, float* row_scale, int rss) {
-  __shared__ float red[16][4];
-  const int tid = threadIdx.x, tl = tid & 3, tok = blockIdx.x * 4 + tl, v = blockIdx.z;
+                                                           int M, int N, int lg, int order, int ti, uint16_t* out,
+                                                           size_t xps, uint32_t* sums, size_t xcs, float* scale, int rss) {
+  __shared__ float red[16][8];
+  const int tid = threadIdx.x, tl = tid & 7, v = blockIdx.z, q = blockIdx.y, nq = gridDim.y;
+  const int tok = blockIdx.x * 8 + tl;
   const bool ok = tok < M;
-  const int n8 = N >> 3, G = N / group, st = group >> 4;            // N is a multiple of 128
+  // groups of 1 << lg columns; nothing per lane is divided (the four divisions by the group size alone took 6 us)
+  const int G = N >> lg, T8 = blockDim.x >> 3;
+  const int b8 = G * q / nq << (lg - 3), e8 = G * (q + 1) / nq << (lg - 3);
   const uint16_t* xr = x + (size_t)(ok ? tok : M - 1) * ldx;
   const uint16_t* cv = cs ? cs + (size_t)v * N : nullptr;
   const uint4 one = make_uint4(0x3c003c00u, 0x3c003c00u, 0x3c003c00u, 0x3c003c00u);
-  const int mine = blockIdx.y * 256 + (tid >> 2);                   // this thread's eight columns
-  const bool has = mine < n8;
-  const uint4 xm = has ? *(const uint4*)(xr + mine * 8) : make_uint4(0, 0, 0, 0);
-  const uint4 cm = has && cv ? *(const uint4*)(cv + mine * 8) : one;
+  uint4 xk[CH ? CH : 1], ck[CH ? CH : 1];
   float mx = 0.f;
-#pragma unroll 4
-  for (int c8 = tid >> 2; c8 < n8; c8 += 256) {
+  auto range = [&](const uint4 xq, const uint4 cq) {
     float a[8];
-    prep8(*(const uint4*)(xr + c8 * 8), cv ? *(const uint4*)(cv + c8 * 8) : one, xdt, a);
+    prep8(xq, cq, xdt, a);
 #pragma unroll
     for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(a[e]));
+  };
+  if (CH) {
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      const int c8 = b8 + (tid >> 3) + T8 * i;
+      xk[i] = make_uint4(0, 0, 0, 0); ck[i] = one;
+      if (c8 < e8) { xk[i] = *(const uint4*)(xr + c8 * 8); if (cv) ck[i] = *(const uint4*)(cv + c8 * 8); }
+    }
+#pragma unroll
+    for (int i = 0; i < CH; ++i) range(xk[i], ck[i]);
+  } else {
+    for (int c8 = b8 + (tid >> 3); c8 < e8; c8 += T8) range(*(const uint4*)(xr + c8 * 8), cv ? *(const uint4*)(cv + c8 * 8) : one);
   }
 #pragma unroll
-  for (int o = 4; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-  if ((tid & 63) < 4) red[tid >> 6][tl] = mx;
+  for (int o = 8; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+  if ((tid & 63) < 8) red[tid >> 6][tl] = mx;
   __syncthreads();
   float all = red[0][tl];
-#pragma unroll
-  for (int w = 1; w < 16; ++w) all = fmaxf(all, red[w][tl]);
+  for (int w = 1; w < (int)(blockDim.x >> 6); ++w) all = fmaxf(all, red[w][tl]);
   const float s = skinny_scale(all), inv = 1.f / s;                 // powers of two
-  if (ok && tid < 4 && blockIdx.y == 0) row_scale[(size_t)v * rss + tok] = s;
-  if (!has) return;                                                 // (a wavefront's sixteen pieces are one 128-column chunk: all or none)
-  const int tile = tok / (32 * ti), i32 = tok % (32 * ti) / 32, l = tok & 31;
-  float a[8];
-  prep8(xm, cm, xdt, a);
-  uint16_t h[8];
-  float sum = 0.f;
+  if (ok && tid < 8) scale[((size_t)v * nq + q) * rss + tok] = s;
+  const int t32 = blockIdx.x >> 2, tile = t32 / ti, i32 = t32 % ti, l = tok & 31;
+  uint16_t* o0 = out + (size_t)v * xps + ((size_t)tile * (N >> 4) * ti + i32) * 512 + l * 8;
+  uint32_t* s0 = sums + (size_t)v * xcs + (size_t)tile * G * 2 * ti * 32 + i32 * 32 + l;
+  auto emit = [&](int c8, const uint4 xq, const uint4 cq) {         // (the pieces of half a group emit together: its sum needs all of them)
+    float a[8];
+    prep8(xq, cq, xdt, a);
+    uint16_t h[8];
+    float sum = 0.f;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) { h[e] = f2h(a[e] * inv); sum += h2f(h[e]); }
-  uint32_t o[4];
-  if (order == 0) {
+    for (int e = 0; e < 8; ++e) { h[e] = f2h(a[e] * inv); sum += h2f(h[e]); }
+    uint32_t o[4];
+    if (order == 0) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = (uint32_t)h[2 * e] | ((uint32_t)h[2 * e + 1] << 16);
-  } else if (order == 1) {                                          // even columns, then odd ones
-    o[0] = (uint32_t)h[0] | ((uint32_t)h[2] << 16); o[1] = (uint32_t)h[4] | ((uint32_t)h[6] << 16);
-    o[2] = (uint32_t)h[1] | ((uint32_t)h[3] << 16); o[3] = (uint32_t)h[5] | ((uint32_t)h[7] << 16);
-  } else {                                                          // 0 4 1 5 2 6 3 7
+      for (int e = 0; e < 4; ++e) o[e] = (uint32_t)h[2 * e] | ((uint32_t)h[2 * e + 1] << 16);
+    } else if (order == 1) {                                        // even columns, then odd ones
+      o[0] = (uint32_t)h[0] | ((uint32_t)h[2] << 16); o[1] = (uint32_t)h[4] | ((uint32_t)h[6] << 16);
+      o[2] = (uint32_t)h[1] | ((uint32_t)h[3] << 16); o[3] = (uint32_t)h[5] | ((uint32_t)h[7] << 16);
+    } else {                                                        // 0 4 1 5 2 6 3 7
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = (uint32_t)h[e] | ((uint32_t)h[e + 4] << 16);
-  }
-  const int col = mine * 8, g = col / group, w = col % group, hf = w / (group >> 1), t = w % (group >> 1) >> 3;
-  uint16_t* o0 = out + (size_t)v * xps + (((size_t)tile * G + g) * st + t) * (ti * 512) + i32 * 512 + hf * 256 + l * 8;
-  if (ok) *(uint4*)o0 = make_uint4(o[0], o[1], o[2], o[3]);
+      for (int e = 0; e < 4; ++e) o[e] = (uint32_t)h[e] | ((uint32_t)h[e + 4] << 16);
+    }
+    const int run = c8 >> (lg - 4), t = c8 & ((1 << (lg - 4)) - 1);   // half group, step in it
+    if (ok) *(uint4*)(o0 + (size_t)((run >> 1 << (lg - 4)) + t) * (ti * 512) + (run & 1) * 256) = make_uint4(o[0], o[1], o[2], o[3]);
+    sum += __shfl_xor(sum, 8);                                      // the pieces of half a group: 32 or 64 columns
+    sum += __shfl_xor(sum, 16);
+    if (lg == 7) sum += __shfl_xor(sum, 32);
+    if (ok && t == 0) {
+      const uint16_t hi = f2h(sum), lo = f2h(sum - h2f(hi));
+      s0[(size_t)run * ti * 32] = (uint32_t)hi | ((uint32_t)lo << 16);
+    }
+  };
+  if (CH) {
 #pragma unroll
-  for (int d = 4; d < 32; d <<= 1) sum += __shfl_xor(sum, d);       // eight pieces: 64 columns
-  if (group == 128) sum += __shfl_xor(sum, 32);
-  if (ok && w == 0) {
-    const uint16_t hi = f2h(sum), lo = f2h(sum - h2f(hi));
-    sums[(size_t)v * xcs + ((size_t)tile * G + g) * ti * 32 + i32 * 32 + l] = (uint32_t)hi | ((uint32_t)lo << 16);
+    for (int i = 0; i < CH; ++i) {
+      const int c8 = b8 + (tid >> 3) + T8 * i;
+      if (c8 < e8) emit(c8, xk[i], ck[i]);
+    }
+  } else {
+    for (int c8 = b8 + (tid >> 3); c8 < e8; c8 += T8) emit(c8, *(const uint4*)(xr + c8 * 8), cv ? *(const uint4*)(cv + c8 * 8) : one);
   }
 }
 
@@ -171,8 +194,8 @@ static SkSpace sk_space(const DMat& m, int M, const SkPlan& p) {
   s.mpad = (M + 32 * p.ti - 1) / (32 * p.ti) * (32 * p.ti);
   const size_t nv = m.cs_rows > 1 ? m.cs_rows : 1;
   s.x = sk_up(nv * s.mpad * m.N * 2);
-  s.sums = sk_up(nv * s.mpad * m.G * 4);
-  s.scale = sk_up(nv * s.mpad * 4);
+  s.sums = sk_up(nv * s.mpad * m.G * 8);
+  s.scale = sk_up(nv * s.mpad * p.nsplit * SK_WC * 4);              // one per part of the column range
   s.part = p.nsplit > 1 ? sk_up((size_t)p.nsplit * M * ((m.K + 7) / 8 * 8) * 4) : 0;
   return s;
 }
@@ -208,8 +231,9 @@ int launch_gemm_skinny(const DMat& m, const void* x, int xdt, int M, int64_t ldx
   a.act = act;
   // (a gate/up matrix with one vector: both parities read the same X')
   a.xps = nv > 1 ? (size_t)sp.mpad * m.N : 0;
-  a.xcs = nv > 1 ? (size_t)sp.mpad * m.G : 0;
-  a.rss = nv > 1 ? sp.mpad : 0;
+  a.xcs = nv > 1 ? (size_t)sp.mpad * m.G * 2 : 0;
+  a.rss = sp.mpad;
+  a.rvs = nv > 1 ? a.rss * plan.nsplit * SK_WC : 0;
   a.vs0 = m.cs_rows == 3 ? m.cs_split0 : 0x7fffffff;
   a.vs1 = m.cs_rows == 3 ? m.cs_split0 + m.cs_split1 : 0x7fffffff;
   a.nsplit = plan.nsplit;
@@ -219,9 +243,13 @@ int launch_gemm_skinny(const DMat& m, const void* x, int xdt, int M, int64_t ldx
   a.tiles_t = sp.mpad / (32 * plan.ti);
   a.tiles_r = (m.K + SK_ROWS * SK_WR - 1) / (SK_ROWS * SK_WR);
   const int order = family_of(m.layout) != FAM_DENSE || m.bits == 8 ? 0 : m.bits == 2 ? 2 : 1;   // SkCfg::ORDER
-  hipLaunchKernelGGL(skinny_prep_kernel, dim3((unsigned)((M + 3) / 4), (unsigned)((m.N + 2047) / 2048), (unsigned)nv), dim3(1024),
-                     0, st, (const uint16_t*)x, ldx, m.cs, xdt, M, m.N, m.group, order, plan.ti, (uint16_t*)ws, a.xps,
-                     (uint32_t*)a.xc, a.xcs, (float*)a.row_scale, a.rss);
+  const int nq = plan.nsplit * SK_WC, p8 = (m.G + nq - 1) / nq * (m.group / 8);   // parts, 16-byte pieces of the longest
+  const int want = (2 * p8 + 63) / 64 * 64;                         // four pieces per thread
+  const int threads = want > 1024 ? 1024 : want, ch = (8 * p8 + threads - 1) / threads;
+  auto prep = ch <= 4 ? skinny_prep_kernel<4> : ch <= 8 ? skinny_prep_kernel<8> : skinny_prep_kernel<0>;
+  hipLaunchKernelGGL(prep, dim3((unsigned)((M + 7) / 8), (unsigned)nq, (unsigned)nv), dim3(threads), 0, st, (const uint16_t*)x,
+                     ldx, m.cs, xdt, M, m.N, m.group == 64 ? 6 : 7, order, plan.ti, (uint16_t*)ws, a.xps, (uint32_t*)a.xc, a.xcs,
+                     (float*)a.row_scale, a.rss);
   const int nb = a.tiles_t * a.tiles_r * a.nsplit, blocks = (nb + 7) / 8 * 8;
   const int fam = family_of(m.layout), keep = fam == FAM_DENSE ? 0 : m.keep;
   int rc;
