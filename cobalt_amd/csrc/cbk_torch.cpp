@@ -231,6 +231,25 @@ PyObject* py_linear_act(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// dequant(matrix, dtype, row0, nrows, with_col_scale) -> W_hat[row0 : row0 + nrows]
+PyObject* py_dequant(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (!arity(n, 5)) return nullptr;
+  return guarded([&]() -> PyObject* {
+    const Matrix* m = as_matrix(a[0]);
+    require_gpu(m, at::Tensor(), at::Tensor());
+    if (!THPDtype_Check(a[1])) fail(PyExc_TypeError, "dtype must be a torch.dtype");
+    const at::ScalarType dt = ((THPDtype*)a[1])->scalar_type;
+    const long long row0 = PyLong_AsLongLong(a[2]), nrows = PyLong_AsLongLong(a[3]);
+    const int cs = PyObject_IsTrue(a[4]);
+    if (PyErr_Occurred()) throw Fail{};
+    const cbk_desc d = desc_of(m);
+    at::Tensor out = at::empty({(int64_t)nrows, (int64_t)d.N}, m->blob->options().dtype(dt));
+    const c10::DeviceGuard guard(out.device());
+    check(cbk_dequant(&d, (int)row0, (int)nrows, cs, out.mutable_data_ptr(), dtype_code(dt), d.N, stream_of(out)), "cbk_dequant");
+    return THPVariable_Wrap(out);
+  });
+}
+
 // gemv_batch(list of matrices, list of x, list of biases or None, out_dtype) -> list of y
 PyObject* py_gemv_batch(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   if (!arity(nargs, 4)) return nullptr;
@@ -279,12 +298,13 @@ PyObject* py_gemv_batch(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   });
 }
 
-// pack_raw(mask or None, q, scale, zero, col_scale or None, layout, bits, group, keep, fix_zero, tiled) ->
-//   (blob, offsets of data / scale / zero / col_scale (-1: none), cs_rows, data_bytes, status, groups re-derived,
-//    largest zero point, survivors in the mask)
-// The caller has checked shapes and devices.  One kernel writes every byte of the image and one copy
-// brings the figures back; the call waits for that copy.
-PyObject* py_pack_raw(PyObject*, PyObject* const* a, Py_ssize_t n) {
+// pack_begin(mask or None, q, scale, zero, col_scale or None, layout, bits, group, keep, fix_zero, tiled) ->
+//   (blob, offsets of data / scale / zero / col_scale (-1: none), cs_rows, data_bytes, pending)
+// pack_end(pending) -> (status, groups re-derived, largest zero point, survivors in the mask)
+// The caller has checked shapes and devices.  One kernel writes every byte of the image; the figures
+// follow it to pinned memory.  pack_end waits for the stream: what the caller does in between costs
+// no time.
+PyObject* py_pack_begin(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!arity(n, 11)) return nullptr;
   return guarded([&]() -> PyObject* {
     at::Tensor mask = as_tensor(a[0], "mask"), q = as_tensor(a[1], "q"), scale = as_tensor(a[2], "scale"),
@@ -335,10 +355,23 @@ PyObject* py_pack_raw(PyObject*, PyObject* const* a, Py_ssize_t n) {
                           zero.const_data_ptr(), zero.scalar_type() == at::kByte ? CBK_U8 : CBK_F16, fix ? 1 : 0, nullptr, &x,
                           stream_of(q)),
           "cbk_pack");
-    at::Tensor host;
+    at::Tensor host = at::empty(counts.sizes(), at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+    host.copy_(counts, true);
+    return Py_BuildValue("N(LLLL)LLN", THPVariable_Wrap(blob), (long long)off[0], (long long)off[1], (long long)off[2],
+                         (long long)off[3], (long long)cs_rows, (long long)(kr * stride),
+                         THPVariable_Wrap(host));
+  });
+}
+
+// (the second argument is the device index)
+PyObject* py_pack_end(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (!arity(n, 2)) return nullptr;
+  return guarded([&]() -> PyObject* {
+    const at::Tensor host = as_tensor(a[0], "pending");
+    const int dev = (int)PyLong_AsLong(a[1]);
     {
       const GilRelease other_threads_run;
-      host = counts.cpu();
+      c10::hip::getCurrentHIPStream(dev).synchronize();
     }
     const uint32_t* h = (const uint32_t*)host.const_data_ptr();
     uint32_t status = 0, fixed = 0, zmax = 0;
@@ -347,8 +380,7 @@ PyObject* py_pack_raw(PyObject*, PyObject* const* a, Py_ssize_t n) {
       status |= h[0]; fixed += h[1]; surv += h[3];
       zmax = zmax > h[2] ? zmax : h[2];
     }
-    return Py_BuildValue("N(LLLL)LLIIIK", THPVariable_Wrap(blob), (long long)off[0], (long long)off[1], (long long)off[2],
-                         (long long)off[3], (long long)cs_rows, (long long)(kr * stride), status, fixed, zmax, surv);
+    return Py_BuildValue("IIIK", status, fixed, zmax, surv);
   });
 }
 
@@ -362,7 +394,9 @@ PyMethodDef methods[] = {
     {"matmul", (PyCFunction)(void (*)())py_matmul, METH_FASTCALL, nullptr},
     {"linear_act", (PyCFunction)(void (*)())py_linear_act, METH_FASTCALL, nullptr},
     {"gemv_batch", (PyCFunction)(void (*)())py_gemv_batch, METH_FASTCALL, nullptr},
-    {"pack_raw", (PyCFunction)(void (*)())py_pack_raw, METH_FASTCALL, nullptr},
+    {"dequant", (PyCFunction)(void (*)())py_dequant, METH_FASTCALL, nullptr},
+    {"pack_begin", (PyCFunction)(void (*)())py_pack_begin, METH_FASTCALL, nullptr},
+    {"pack_end", (PyCFunction)(void (*)())py_pack_end, METH_FASTCALL, nullptr},
     {"set_error", py_set_error, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -51,7 +51,13 @@ class CobaltLinear(nn.Module):
         """From the RAW per-matrix schema `<name>.{mask,q,scale,zero,col_scale}`
         (src/cobaltkernel/pack_cobalt.py:3-11); `tiled` asks for the decode kernel's byte order
         at once instead of the reference's row-major order."""
-        return cls(cls._pack(mask, q, scale, zero, col_scale, layout, bits, group, keep, cs_splits, tiled), bias, meta)
+        if not q.is_cuda:
+            return cls(cls._pack(mask, q, scale, zero, col_scale, layout, bits, group, keep, cs_splits, tiled), bias, meta)
+        job = ops.PackJob(mask, q, scale, zero, col_scale, layout, bits, group, keep, cs_splits=cs_splits, tiled=tiled)
+        self = cls(job.pm, bias, meta)                                # while the kernel runs
+        pm = job.finish()
+        self.cbk_meta[-2:] = torch.tensor([pm.n_survivors, pm.flags])
+        return self
 
     @classmethod
     def from_linear(cls, linear: nn.Module, X_cal: Optional[torch.Tensor] = None, H: Optional[torch.Tensor] = None,

@@ -9,7 +9,7 @@ from typing import Optional
 import torch
 
 from . import _lib
-from .format import PackedMatrix, dtype_code
+from .format import PackedMatrix
 
 def _stream_ptr(device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
@@ -34,14 +34,7 @@ def workspace_for(pm: PackedMatrix, M: int) -> Optional[torch.Tensor]:
 def dequant(pm: PackedMatrix, dtype=torch.float32, row0: int = 0, nrows: Optional[int] = None,
             with_col_scale: bool = True) -> torch.Tensor:
     """W_hat[row0:row0+nrows] as a dense tensor (bit-exact float32 formula, one cast)."""
-    _require_gpu(pm)
-    nrows = pm.K - row0 if nrows is None else nrows
-    out = torch.empty(nrows, pm.N, dtype=dtype, device=pm.blob.device)
-    d = pm.desc()
-    rc = _lib.lib().cbk_dequant(ctypes.byref(d), row0, nrows, int(with_col_scale), out.data_ptr(),
-                                dtype_code(dtype), pm.N, _stream_ptr(pm.blob.device))
-    _lib.check(rc, "cbk_dequant")
-    return out
+    return _lib.native().dequant(pm.native(), dtype, row0, pm.K - row0 if nrows is None else nrows, bool(with_col_scale))
 
 
 def gemv(pm, x, bias=None, out_dtype=None, workspace=None):
@@ -76,6 +69,47 @@ def gemv_batch(pms, xs, biases=None, out_dtype=None):
     return _lib.native().gemv_batch([pm.native() for pm in pms], list(xs), None if biases is None else list(biases), out_dtype)
 
 
+class PackJob:
+    """A matrix being packed on the GPU: `pm` describes it already (its zero-point flags and survivor
+    count are provisional), `finish()` waits for the kernel, raises if the arrays do not fit the
+    layout, and completes the description."""
+
+    def __init__(self, mask_bits, q, scale, zero, col_scale, layout, bits=None, group=None, keep=None, fix_zero=True,
+                 cs_splits=(0, 0), tiled=True):
+        from . import format as F
+        bits, group, kpb = F.canon(layout, bits, group, keep)
+        if layout in F._SPARSE:
+            raise NotImplementedError("the variable-length SPARSE4* layouts are read, not produced, by this package")
+        if q.device.type != "cuda":
+            raise _lib.CbkError("ops.pack_raw packs on the GPU; use format.pack_raw for tensors on the CPU")
+        K, N = q.shape
+        if N % 128 or N % group:
+            raise ValueError(f"N={N} must be a multiple of 128 and of the group size")
+        blob, (o_data, o_scale, o_zero, o_cs), cs_rows, data_bytes, self._pending = _lib.native().pack_begin(
+            mask_bits, q, scale, zero, col_scale, layout, bits, group, kpb, bool(fix_zero), tiled)
+        offs = {"data": o_data, "scale": o_scale, "zero": o_zero}
+        if cs_rows:
+            offs["col_scale"] = o_cs
+        self.pm = PackedMatrix(blob, offs, K, N, layout, bits, group, kpb, cs_rows, tuple(cs_splits), data_bytes,
+                               K * (N // F.BLOCK) * kpb, 0, F.FLAG_TILED16 if tiled else 0).validate()
+
+    def finish(self) -> PackedMatrix:
+        from . import format as F
+        pm = self.pm
+        wrong, pm.n_zero_fixed, z_max, n_mask = _lib.native().pack_end(self._pending, pm.blob.device.index)
+        if wrong & 2:
+            raise ValueError(f"{F.LAYOUT_NAME[pm.layout]} stores the zero point as the code of a pruned column, and a zero point "
+                             f"of this matrix is above {(1 << pm.bits) - 1}: such a column would not dequantise to 0 (pack with "
+                             f"fix_zero=True, or keep a bitmap layout)")
+        if wrong & 1:
+            raise ValueError(f"{F.LAYOUT_NAME[pm.layout]} needs exactly {pm.keep} survivors in every aligned block of "
+                             f"{F.BLOCK} columns; the mask has a block with another count")
+        if pm.layout in F._DENSE:
+            pm.n_survivors = n_mask
+        pm.flags |= F.zero_flags(z_max, pm.bits)
+        return pm
+
+
 def pack_raw(mask_bits, q, scale, zero, col_scale, layout, bits=None, group=None, keep=None, fix_zero=True,
              cs_splits=(0, 0), tiled=True) -> PackedMatrix:
     """RAW arrays on the GPU -> PackedMatrix on the GPU, written by the library's packing kernel
@@ -83,32 +117,7 @@ def pack_raw(mask_bits, q, scale, zero, col_scale, layout, bits=None, group=None
     src/cobaltkernel/pack_cobalt.py:55-87), in the tiled order the decode kernel streams (`tiled`)
     or the reference's row-major order.  Same arguments and same bytes as `format.pack_raw`
     (which is torch and runs anywhere)."""
-    from . import format as F
-    bits, group, kpb = F.canon(layout, bits, group, keep)
-    if layout in F._SPARSE:
-        raise NotImplementedError("the variable-length SPARSE4* layouts are read, not produced, by this package")
-    if q.device.type != "cuda":
-        raise _lib.CbkError("ops.pack_raw packs on the GPU; use format.pack_raw for tensors on the CPU")
-    K, N = q.shape
-    if N % 128 or N % group:
-        raise ValueError(f"N={N} must be a multiple of 128 and of the group size")
-    nl = (1 << bits) - 1
-    blob, (o_data, o_scale, o_zero, o_cs), cs_rows, data_bytes, wrong, n_fixed, z_max, n_mask = _lib.native().pack_raw(
-        mask_bits, q, scale, zero, col_scale, layout, bits, group, kpb, bool(fix_zero), tiled)
-    offs = {"data": o_data, "scale": o_scale, "zero": o_zero}
-    if cs_rows:
-        offs["col_scale"] = o_cs
-    n_surv = n_mask if layout in F._DENSE else K * (N // F.BLOCK) * kpb
-    pm = PackedMatrix(blob, offs, K, N, layout, bits, group, kpb, cs_rows, tuple(cs_splits), data_bytes, n_surv, n_fixed,
-                      (F.FLAG_TILED16 if tiled else 0) | F.zero_flags(z_max, bits))
-    if wrong & 2:
-        raise ValueError(f"{F.LAYOUT_NAME[layout]} stores the zero point as the code of a pruned column, and a zero point "
-                         f"of this matrix is above {nl}: such a column would not dequantise to 0 (pack with fix_zero=True, "
-                         f"or keep a bitmap layout)")
-    if wrong & 1:
-        raise ValueError(f"{F.LAYOUT_NAME[layout]} needs exactly {kpb} survivors in every aligned block of "
-                         f"{F.BLOCK} columns; the mask has a block with another count")
-    return pm.validate()
+    return PackJob(mask_bits, q, scale, zero, col_scale, layout, bits, group, keep, fix_zero, cs_splits, tiled).finish()
 
 
 def unpack(pm: PackedMatrix):
