@@ -22,9 +22,8 @@
 // to 16 column parts and the (tile, part) items are dealt round-robin to the wavefronts.  There
 // is no barrier per tile: the partial sums of a tile meet in an LDS slot and the wavefront that
 // arrives last adds them in part order, so results are run-to-run identical.
-// For 2 <= M <= 8 the headline configurations put the lane quarters on the four 32-column
-// blocks of one chunk instead of on four chunks (see block_split_capable below), so that
-// every MFMA serves four activation rows (M = 5..8: two MFMAs per decoded fragment, one weight
+// For 2 <= M <= 8 the lane quarters are put on the four 32-column blocks of one chunk instead of on
+// four chunks (see block_loads below), so that every MFMA serves four activation rows (M = 5..8: two MFMAs per decoded fragment, one weight
 // pass); sums are formed in the same order as for M = 1, so a row's result does not depend on M.
 // The activation digits and the byte-permute selector table live in LDS for the whole launch;
 // where the digits of all rows of a matrix do not fit (two to eight activation rows of a long
@@ -66,7 +65,7 @@ constexpr int NDIG = 3;                       // int8 digits per activation
 // row, digit) at the same column; row lengths are multiples of 128 bytes, and unpadded rows would
 // all start in the same LDS banks.
 constexpr int X_PAD = 16;
-constexpr int GV_MAX_M = 8;                     // 5..8 only in the block-per-quarter arrangement
+constexpr int GV_MAX_M = 8;                     // activation rows per pass over the weights
 constexpr int GV_MAX_BATCH = 8;               // matrices per launch
 
 // ------------------------------------------------------------------ kernel configuration
@@ -128,16 +127,18 @@ __host__ __device__ constexpr int frag_col(int bits, bool dense, int bi) {
 }
 
 // Two ways to lay a macro-step (16 rows x 512 columns) on the 16x16x64 MFMA.
-//  * quarter-per-chunk: lane quarter kq decodes chunk 4S + kq; one MFMA adds four different
-//    quantisation groups, so the A rows are (quarter, digit) and one activation row needs one
-//    pass.  Used for M = 1 and for every configuration below that cannot use the other way.
-//  * quarter-per-block: lane quarter kq decodes block kq (32 columns) of each of the four
-//    chunks; one MFMA covers 64 columns of a single group, the A rows are (activation row,
-//    digit), and up to four activation rows share every MFMA.  Needs group 128 and a block's
-//    code bits to be 4, 8 or 16 whole bytes.
-__host__ __device__ constexpr bool block_split_capable(int bits, int keep, int grp) {
+//  * quarter-per-chunk (M = 1, and M = 2 where the other way needs the turn): lane quarter kq decodes chunk 4S + kq; one MFMA adds four different
+//    quantisation groups, so the A rows are (quarter, digit) and one activation row needs one pass.
+//  * quarter-per-block (else): lane quarter kq decodes block kq (32 columns) of each of the four
+//    chunks; one MFMA covers 64 columns of one chunk, the A rows are (activation row, digit), and up
+//    to four activation rows share every MFMA.  Groups of 64 columns are the lower and the upper two
+//    quarters of a chunk: two MFMAs, each with an A operand that is zero in the other half.
+// A lane loads its own block where the block's code bits are 4, 8 or 16 whole bytes; in every other
+// code width it loads and aligns a whole chunk, as for M = 1, and the streams of the four blocks,
+// their masks (and high bits) change places between the lane quarters in registers.
+__host__ __device__ constexpr bool block_loads(int bits, int keep, int grp) {
   const int cb = (keep == 0 ? 32 : keep) * bits;
-  return grp == 128 && bits != 3 && (cb == 32 || cb == 64 || cb == 128);
+  return grp == 128 && bits != 3 && bits != 6 && (cb == 32 || cb == 64 || cb == 128);
 }
 
 // ------------------------------------------------------------------ activation prep
@@ -332,12 +333,204 @@ struct Loads {
   uint32_t h2[C::HI2 ? 4 : 1];   // BLK1632_6: the chunk's four dwords of high bits
 };
 
+// r0..r3 hold, in lane quarter q, the values (q, 0..3); afterwards register i holds (i, q): the upper
+// two quarters of r0 / r1 change places with the lower two of r2 / r3, then the odd quarters of r0 / r2
+// with the even ones of r1 / r3.  (Inline assembly as in quarter_sum.)
+__device__ inline void transpose4(uint32_t& r0, uint32_t& r1, uint32_t& r2, uint32_t& r3) {
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(r0), "+v"(r2));
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(r1), "+v"(r3));
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(r0), "+v"(r1));
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(r2), "+v"(r3));
+}
+
+// What the loads of a macro-step need of the position: the matrix's arrays, a scalar part that depends on
+// (tile, S) and a lane part.  Every address is one of the three base pointers plus a 32-bit offset (the
+// host admits only matrices whose arrays are smaller than 4 GB): one add per load, no 64-bit arithmetic.
+struct StepAt {
+  const uint8_t* data; const uint16_t* scale; const uint8_t* zero;
+  uint32_t so_t, so_g;       // scalar: start of the tile's rows, first scale / zero of the tile
+  uint32_t lane_off, sz_off; // this lane's row in them
+  uint32_t code_u0;
+  int ush, csh, NCH;
+};
+// quarter-per-block: block kq of the chunks S4 .. S4 + 3, one mask dword and CB / 8 code bytes each; the zero
+// point and scale of chunk S4 + kq, which the other quarters fetch from this lane
+template <class C>
+__device__ inline void load_blocks(const StepAt& p, int S4, int kq, Loads<C>& L) {
+  constexpr uint32_t BB = C::CB / 8;
+  const uint32_t voff_m = p.lane_off + (uint32_t)kq * 4u;
+  const uint32_t voff_c = p.lane_off + ((((uint32_t)kq * BB) >> 4) << p.ush) + (((uint32_t)kq * BB) & 15u);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    int chc = S4 + c;
+    chc = chc < p.NCH ? chc : p.NCH - 1;
+    if (!C::DENSE) L.mk[c] = *(const uint32_t*)(p.data + (p.so_t + ((uint32_t)chc << p.ush) + voff_m));
+    const uint8_t* cp = p.data + (p.so_t + ((p.code_u0 + (uint32_t)chc * (C::CHB / 128)) << p.ush) + voff_c);
+    if (C::CB == 32) {
+      L.raw[c] = *(const uint32_t*)cp;
+    } else if (C::CB == 64) {
+      const uint2 v = *(const uint2*)cp;
+      L.raw[2 * c] = v.x; L.raw[2 * c + 1] = v.y;
+    } else {
+      const uint4 v = *(const uint4*)cp;
+      L.raw[4 * c] = v.x; L.raw[4 * c + 1] = v.y; L.raw[4 * c + 2] = v.z; L.raw[4 * c + 3] = v.w;
+    }
+  }
+  const int klim = p.NCH - 1 - S4;                                  // chunks past N repeat chunk NCH - 1
+  const uint32_t chl = (uint32_t)(kq < klim ? kq : klim);
+  const uint32_t gv = p.so_g + ((uint32_t)S4 << p.csh) + p.sz_off + (chl << p.csh);
+  L.zraw = (uint32_t)p.zero[gv] | ((uint32_t)p.scale[gv] << 8);
+}
+// quarter-per-chunk: chunk S4 + kq whole
+template <class C>
+__device__ inline void load_chunk(const StepAt& p, int S4, int kq, Loads<C>& L) {
+  const int klim = p.NCH - 1 - S4;
+  const uint32_t chl = (uint32_t)(kq < klim ? kq : klim);
+  const uint32_t so_s = p.so_t + ((uint32_t)S4 << p.ush);           // scalar: unit S4 of the rows
+  if (!C::DENSE) {
+    const uint4 v = *(const uint4*)(p.data + (so_s + p.lane_off + (chl << p.ush)));
+    L.mk[0] = v.x; L.mk[1] = v.y; L.mk[2] = v.z; L.mk[3] = v.w;
+  }
+  // code bits of the chunk: bit ch*CHB of the code plane, fetched as whole 16-byte units
+  if (C::VEC16) {
+    const uint32_t so_c = p.so_t + ((p.code_u0 + (uint32_t)S4 * (C::CHB / 128)) << p.ush);
+    const uint32_t voff = p.lane_off + ((chl * (C::CHB / 128)) << p.ush);
+#pragma unroll
+    for (int i = 0; i < C::NL / 4; ++i) {
+      const uint4 v = *(const uint4*)(p.data + (so_c + ((uint32_t)i << p.ush) + voff));
+      L.raw[4 * i] = v.x; L.raw[4 * i + 1] = v.y; L.raw[4 * i + 2] = v.z; L.raw[4 * i + 3] = v.w;
+    }
+  } else {
+    const uint32_t u = (((uint32_t)S4 + chl) * (uint32_t)C::CHB) >> 7;
+    const uint32_t voff = p.lane_off + (u << p.ush);
+#pragma unroll
+    for (int i = 0; i < C::NL / 4; ++i) {
+      const uint4 v = *(const uint4*)(p.data + (p.so_t + ((p.code_u0 + (uint32_t)i) << p.ush) + voff));
+      L.raw[4 * i] = v.x; L.raw[4 * i + 1] = v.y; L.raw[4 * i + 2] = v.z; L.raw[4 * i + 3] = v.w;
+    }
+  }
+  if (C::HI2) {                                                     // unit ch of the plane behind mask and nibbles
+    const uint4 v = *(const uint4*)(p.data + (p.so_t + ((3u * (uint32_t)p.NCH + (uint32_t)S4 + chl) << p.ush) + p.lane_off));
+    L.h2[0] = v.x; L.h2[1] = v.y; L.h2[2] = v.z; L.h2[3] = v.w;
+  }
+  const uint32_t gv = p.so_g + ((uint32_t)(S4 * C::NGC) << p.csh) + p.sz_off + ((chl * C::NGC) << p.csh);
+  if (C::NGC == 1) {
+    L.zraw = p.zero[gv];
+    L.sc[0] = p.scale[gv];
+  } else {
+    const uint32_t gv1 = gv + (1u << p.csh);
+    L.zraw = (uint32_t)p.zero[gv] | ((uint32_t)p.zero[gv1] << 8);
+    L.sc[0] = p.scale[gv];
+    L.sc[C::NGC - 1] = p.scale[gv1];
+  }
+}
+
+// One macro-step in the quarter-per-block arrangement: adds 16 rows x 512 columns to the sums ysum[4 g + c]
+// of activation rows 4g + kq, chunk position c.  TURN: `cur` holds chunk 4S + kq as load_chunk left it, and
+// its blocks are turned into those of quarter-per-block here: four swaps per register of a block's stream and
+// mask, 12 to 24 of a step's ~ 350 instructions.  (A pass of quarter-per-chunk per row, five to eight rows in two
+// launches, 3-bit codes, 10 of 32 kept: 21504 x 5376 23.4 -> 21.3 us at M = 4, 45.6 -> 23.0 at M = 8; 5376 x 21504, rows
+// split by columns now, 35.2 -> 19.6 and 69.5 -> 21.4.)
+struct XDigits { uint32_t xq_off, z_off; const float* delta; int Ns, ch0, NCH, M; };   // staged digits and deltas
+template <class C, int BITS, int NG, bool TURN>
+__device__ inline void block_step(const Loads<C>& cur, const uint8_t* smem, const uint2* lut, uint32_t l16, int lane, int S,
+                                  const XDigits& x, float (&ysum)[4 * NG]) {
+  constexpr int NGC = C::NGC;
+  const int wr = lane & 15, kq = lane >> 4;
+  const int a_m = wr >> 2, a_dig = wr & 3;                          // activation row and digit of this lane's A row
+  uint32_t st4[4][C::NW], mk4[4], hw4[4];
+  if constexpr (TURN) {
+    uint32_t cw[C::ND];
+    const int chunk = 4 * S + kq;
+    align_chunk_codes<C>(cur.raw, (uint32_t)(chunk < x.NCH ? chunk : x.NCH - 1), cw);
+#pragma unroll
+    for (int jb = 0; jb < 4; ++jb) {
+      block_stream<C, BITS>(cw, jb, st4[jb]);
+      mk4[jb] = C::DENSE ? 0u : cur.mk[jb];
+      hw4[jb] = cur.h2[C::HI2 ? jb : 0];
+    }
+#pragma unroll
+    for (int k = 0; k < C::NW; ++k) transpose4(st4[0][k], st4[1][k], st4[2][k], st4[3][k]);
+    if (!C::DENSE) transpose4(mk4[0], mk4[1], mk4[2], mk4[3]);
+    if (C::HI2) transpose4(hw4[0], hw4[1], hw4[2], hw4[3]);
+  }
+  uint32_t zs[4][NGC];                                              // zero | scale << 8 of the groups of the chunks 4S .. 4S+3
+#pragma unroll
+  for (int g = 0; g < NGC; ++g) {
+    const uint32_t own = !TURN ? cur.zraw : ((cur.zraw >> (8 * g)) & 0xFFu) | (cur.sc[TURN ? g : 0] << 8);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) zs[c][g] = (uint32_t)__shfl((int)own, wr + 16 * c, 64);
+  }
+  // row group g holds activation rows 4g .. 4g+3: its A operand, and in the result lane
+  // quarter kq the three digit sums of activation row 4g + kq
+  bool a_on[NG];
+  uint32_t a_base[NG];
+  int dm[NG];                                                       // the activation rows this quarter sums
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    a_on[g] = a_dig < NDIG && a_m + 4 * g < x.M;
+    a_base[g] = x.xq_off + (uint32_t)(((a_m + 4 * g) * NDIG + a_dig) * (x.Ns + X_PAD) + kq * 32);
+    dm[g] = kq + 4 * g < x.M ? kq + 4 * g : 0;
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int chunk = 4 * S + c;
+    uint32_t aaddr[NG][NGC];
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int h = 0; h < NGC; ++h)
+        aaddr[g][h] = (a_on[g] && chunk < x.NCH && (NGC == 1 || (kq >> 1) == h)) ? a_base[g] + (uint32_t)(chunk - x.ch0) * 128u : x.z_off;
+    uint32_t rkc[4];
+    uint2 selc[4];
+    fetch_selectors<C>(TURN ? mk4[c] : cur.mk[c], lut, l16, rkc, selc);
+    uint32_t st[C::NW];
+#pragma unroll
+    for (int k = 0; k < C::NW; ++k) {
+      if constexpr (TURN) st[k] = st4[c][k];
+      else st[k] = cur.raw[c * C::NW + k];
+    }
+    const uint32_t z = (NGC == 1 || kq < 2 ? zs[c][0] : zs[c][NGC - 1]) & 0xFFu;
+    const uint32_t nz = 0x80808080u - z * 0x01010101u;
+    v4i acc[NG][NGC];
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int h = 0; h < NGC; ++h) acc[g][h] = (v4i){0, 0, 0, 0};
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      uint32_t bfrag[4];
+      decode_half<C, BITS>(st, rkc, selc, nz, half, bfrag, TURN && C::HI2 ? hw4[c] : 0u);
+      const v4i bv = (v4i){(int)bfrag[0], (int)bfrag[1], (int)bfrag[2], (int)bfrag[3]};
+#pragma unroll
+      for (int g = 0; g < NG; ++g)
+#pragma unroll
+        for (int h = 0; h < NGC; ++h) {
+          const v4i av = *(const v4i*)(smem + aaddr[g][h] + 16 * half);
+          acc[g][h] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bv, acc[g][h], 0, 0, 0);
+          asm("s_nop 1" : "+v"(acc[g][h]));                         // see the decode path of one activation row
+        }
+    }
+    // the 128 columns of the chunk are complete: rows 4 kq .. 4 kq + 2 of the result are the three digit
+    // sums of activation row 4g + kq
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const float dl = x.delta[dm[g] * (x.NCH + 4) + chunk];        // 0 past the last chunk
+#pragma unroll
+      for (int h = 0; h < NGC; ++h) {
+        const float f = fmaf((float)(acc[g][h][0] * 256 + acc[g][h][1]), 256.f, (float)acc[g][h][2]);
+        ysum[4 * g + c] = fmaf(f, h2f((uint16_t)(zs[c][h] >> 8)) * dl, ysum[4 * g + c]);
+      }
+    }
+  }
+}
+
 template <int BITS, int KEEP, int GRP, int MP>
 __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
   using C = Cfg<BITS, KEEP, GRP, MP>;
-  constexpr bool QB = (MP == 4 || MP == 8) && block_split_capable(BITS, KEEP, GRP);
+  static_assert(MP == 1 || MP == 2 || MP == 4 || MP == 8, "single activation rows, or row groups of four");
+  constexpr bool QB = MP >= 4, TURN = QB && !block_loads(BITS, KEEP, GRP);
   constexpr int NG = MP == 8 ? 2 : 1;                  // groups of four activation rows, one MFMA each per fragment
-  static_assert(MP <= 4 || QB, "more than four activation rows need the block-per-quarter arrangement");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);     // in a scalar register: positions are scalar work
@@ -470,80 +663,12 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
     auto issue = [&](int tile, int S, Loads<C>& L) {
       tile = tile < last_tile ? tile : last_tile;
       S = S < last_S ? S : last_S;
-      const int S4 = 4 * S;
       const int rlim = m_K - 1 - tile * 16;                         // rows past K repeat row K - 1
       const uint32_t wrc = (uint32_t)(wr < rlim ? wr : rlim);
-      const uint32_t lane_off = __umul24(wrc, lane_mul);
-      const int klim = NCH - 1 - S4;                                // chunks past N repeat chunk NCH - 1
-      const uint32_t chl = (uint32_t)(kq < klim ? kq : klim);
-      // Every address is one of the matrix's three base pointers plus a 32-bit offset (the host
-      // admits only matrices whose arrays are smaller than 4 GB): a scalar part that depends on
-      // (tile, S) and a lane part; one add per load, no 64-bit arithmetic per step.
-      const uint32_t so_t = (uint32_t)tile * tile_a;                 // scalar: start of the tile's rows
-      const uint32_t so_g = (uint32_t)tile * (uint32_t)(16 * m_G);   // scalar: first scale / zero of the tile
-      if constexpr (QB) {
-        // block kq of the chunks 4S .. 4S+3: one mask dword and CB / 8 code bytes each
-        constexpr uint32_t BB = C::CB / 8;
-        const uint32_t voff_m = lane_off + (uint32_t)kq * 4u;
-        const uint32_t voff_c = lane_off + ((((uint32_t)kq * BB) >> 4) << ush) + (((uint32_t)kq * BB) & 15u);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          int chc = S4 + c;
-          chc = chc < NCH ? chc : NCH - 1;
-          if (!C::DENSE) L.mk[c] = *(const uint32_t*)(m_data + (so_t + ((uint32_t)chc << ush) + voff_m));
-          const uint8_t* cp = m_data + (so_t + ((code_u0 + (uint32_t)chc * (C::CHB / 128)) << ush) + voff_c);
-          if (C::CB == 32) {
-            L.raw[c] = *(const uint32_t*)cp;
-          } else if (C::CB == 64) {
-            const uint2 v = *(const uint2*)cp;
-            L.raw[2 * c] = v.x; L.raw[2 * c + 1] = v.y;
-          } else {
-            const uint4 v = *(const uint4*)cp;
-            L.raw[4 * c] = v.x; L.raw[4 * c + 1] = v.y; L.raw[4 * c + 2] = v.z; L.raw[4 * c + 3] = v.w;
-          }
-        }
-        // zero point and scale of group 4S + kq; the other quarters fetch them from this lane
-        const uint32_t gv = so_g + ((uint32_t)S4 << csh) + __umul24(wrc, sz_mul) + (chl << csh);
-        L.zraw = (uint32_t)m_zero[gv] | ((uint32_t)m_scale[gv] << 8);
-        return;
-      }
-      const uint32_t so_s = so_t + ((uint32_t)S4 << ush);            // scalar: unit 4S of the rows
-      if (!C::DENSE) {
-        const uint4 v = *(const uint4*)(m_data + (so_s + lane_off + (chl << ush)));
-        L.mk[0] = v.x; L.mk[1] = v.y; L.mk[2] = v.z; L.mk[3] = v.w;
-      }
-      // code bits of the chunk: bit ch*CHB of the code plane, fetched as whole 16-byte units
-      if (C::VEC16) {
-        const uint32_t so_c = so_t + ((code_u0 + (uint32_t)S4 * (C::CHB / 128)) << ush);
-        const uint32_t voff = lane_off + ((chl * (C::CHB / 128)) << ush);
-#pragma unroll
-        for (int i = 0; i < C::NL / 4; ++i) {
-          const uint4 v = *(const uint4*)(m_data + (so_c + ((uint32_t)i << ush) + voff));
-          L.raw[4 * i] = v.x; L.raw[4 * i + 1] = v.y; L.raw[4 * i + 2] = v.z; L.raw[4 * i + 3] = v.w;
-        }
-      } else {
-        const uint32_t u = (((uint32_t)S4 + chl) * (uint32_t)C::CHB) >> 7;
-        const uint32_t voff = lane_off + (u << ush);
-#pragma unroll
-        for (int i = 0; i < C::NL / 4; ++i) {
-          const uint4 v = *(const uint4*)(m_data + (so_t + ((code_u0 + (uint32_t)i) << ush) + voff));
-          L.raw[4 * i] = v.x; L.raw[4 * i + 1] = v.y; L.raw[4 * i + 2] = v.z; L.raw[4 * i + 3] = v.w;
-        }
-      }
-      if (C::HI2) {                                                 // unit ch of the plane behind mask and nibbles
-        const uint4 v = *(const uint4*)(m_data + (so_t + ((3u * (uint32_t)NCH + (uint32_t)S4 + chl) << ush) + lane_off));
-        L.h2[0] = v.x; L.h2[1] = v.y; L.h2[2] = v.z; L.h2[3] = v.w;
-      }
-      const uint32_t gv = so_g + ((uint32_t)(S4 * C::NGC) << csh) + __umul24(wrc, sz_mul) + ((chl * C::NGC) << csh);
-      if (C::NGC == 1) {
-        L.zraw = m_zero[gv];
-        L.sc[0] = m_scale[gv];
-      } else {
-        const uint32_t gv1 = gv + (1u << csh);
-        L.zraw = (uint32_t)m_zero[gv] | ((uint32_t)m_zero[gv1] << 8);
-        L.sc[0] = m_scale[gv];
-        L.sc[C::NGC - 1] = m_scale[gv1];
-      }
+      const StepAt at{m_data, m_scale, m_zero, (uint32_t)tile * tile_a, (uint32_t)tile * (uint32_t)(16 * m_G),
+                      (uint32_t)__umul24(wrc, lane_mul), (uint32_t)__umul24(wrc, sz_mul), code_u0, ush, csh, NCH};
+      if constexpr (QB && !TURN) load_blocks<C>(at, 4 * S, kq, L);
+      else load_chunk<C>(at, 4 * S, kq, L);
     };
 
     // this wave's sequence of (tile, part, macro-step) positions: items wave, wave + 16, ...
@@ -602,59 +727,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
       // the compiler no longer spreads them over the decode, and every launch was 2-6 % slower)
       issue(t_lo + p1.tl, p1.S, tgt);
       if constexpr (QB) {
-        const int a_m = wr >> 2;                                    // activation row of this lane's A row
-        uint32_t zs[4];                                             // zero | scale << 8 of the groups 4S .. 4S+3
-#pragma unroll
-        for (int c = 0; c < 4; ++c) zs[c] = (uint32_t)__shfl((int)cur.zraw, wr + 16 * c, 64);
-        // row group g holds activation rows 4g .. 4g+3: its A operand, and in the result lane
-        // quarter kq the three digit sums of activation row 4g + kq
-        bool a_on[NG];
-        uint32_t a_base[NG];
-        int dm[NG];                                                 // the activation rows this quarter sums
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-          a_on[g] = a_dig < NDIG && a_m + 4 * g < h.M;
-          a_base[g] = xq_off + (uint32_t)(((a_m + 4 * g) * NDIG + a_dig) * (Ns + X_PAD) + kq * 32);
-          dm[g] = kq + 4 * g < h.M ? kq + 4 * g : 0;
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const int chunk = 4 * S + c;
-          uint32_t aaddr[NG];
-#pragma unroll
-          for (int g = 0; g < NG; ++g) aaddr[g] = (a_on[g] && chunk < NCH) ? a_base[g] + (uint32_t)(chunk - ch0) * 128u : z_off;
-          uint32_t rkc[4];
-          uint2 selc[4];
-          fetch_selectors<C>(cur.mk[c], lut, l16, rkc, selc);
-          uint32_t st[C::NW];
-#pragma unroll
-          for (int k = 0; k < C::NW; ++k) st[k] = cur.raw[c * C::NW + k];
-          const uint32_t z = zs[c] & 0xFFu;
-          const uint32_t nz = 0x80808080u - z * 0x01010101u;
-          v4i acc[NG];
-#pragma unroll
-          for (int g = 0; g < NG; ++g) acc[g] = (v4i){0, 0, 0, 0};
-#pragma unroll
-          for (int half = 0; half < 2; ++half) {
-            uint32_t bfrag[4];
-            decode_half<C, BITS>(st, rkc, selc, nz, half, bfrag);
-            const v4i bv = (v4i){(int)bfrag[0], (int)bfrag[1], (int)bfrag[2], (int)bfrag[3]};
-#pragma unroll
-            for (int g = 0; g < NG; ++g) {
-              const v4i av = *(const v4i*)(smem + aaddr[g] + 16 * half);
-              acc[g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bv, acc[g], 0, 0, 0);
-              asm("s_nop 1" : "+v"(acc[g]));                        // see the other decode path
-            }
-          }
-          // the 128 columns of group `chunk` are complete: rows 4 kq .. 4 kq + 2 of the result
-          // are the three digit sums of activation row 4g + kq
-#pragma unroll
-          for (int g = 0; g < NG; ++g) {
-            const float dl = delta[dm[g] * (NCH + 4) + chunk];      // 0 past the last chunk
-            const float f = fmaf((float)(acc[g][0] * 256 + acc[g][1]), 256.f, (float)acc[g][2]);
-            ysum[4 * g + c] = fmaf(f, h2f((uint16_t)(zs[c] >> 8)) * dl, ysum[4 * g + c]);
-          }
-        }
+        block_step<C, BITS, NG, TURN>(cur, smem, lut, l16, lane, S, XDigits{xq_off, z_off, delta, Ns, ch0, NCH, h.M}, ysum);
       } else
       {
         const int chunk = 4 * S + kq;
@@ -828,7 +901,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
 // deals the (tile, part) items of its slab to the wavefronts and writes the part sums to a
 // caller-provided buffer; a second small kernel adds the parts of every output in part order.
 // Same operations in the same order as for one activation row, so a row's result still does not
-// depend on M.  Block-per-quarter arrangement only.
+// depend on M.  Quarter-per-block arrangement.
 struct GsMat {             // one matrix of a column-split launch
   GvMat g;                 // spi, sk: the parts; sp: parts per slab
   int nslab, wps;          // column slabs, workgroups per slab
@@ -852,7 +925,8 @@ static_assert(sizeof(GsArgs) <= 4096 && sizeof(GvBatch) <= 4096, "kernel argumen
 template <int BITS, int KEEP, int GRP, int MP>
 __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
   using C = Cfg<BITS, KEEP, GRP, MP>;
-  static_assert((MP == 4 || MP == 8) && block_split_capable(BITS, KEEP, GRP), "block-per-quarter configurations only");
+  static_assert(MP == 4 || MP == 8, "row groups of four");
+  constexpr bool TURN = !block_loads(BITS, KEEP, GRP);
   constexpr int NG = MP / 4;                           // groups of four activation rows, one MFMA each per fragment
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -883,7 +957,6 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
   }
   const int wr = lane & 15, kq = lane >> 4;
   const uint32_t l16 = lane & (LUT_LANES - 1);
-  const int a_m = wr >> 2, a_dig = wr & 3;             // activation row and digit of this lane's A row
   const uint32_t xq_off = (uint32_t)((uint8_t*)xq - smem), z_off = (uint32_t)(zreg - smem);
 
   // this workgroup: slab sl, tiles [T_lo, T_hi)
@@ -903,39 +976,16 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
   const uint32_t tile_a = gm.tile_a, lane_mul = gm.lane_mul, sz_mul = gm.sz_mul, code_u0 = m.code_off >> 4;
   const int last_S = nS - 1, last_tile = T_hi - 1;
 
-  // loads of one (tile, macro-step) position: block kq of the chunks 4S .. 4S+3 of row wr
+  // loads of one (tile, macro-step) position
   auto issue = [&](int tile, int S, Loads<C>& L) {
     tile = tile < last_tile ? tile : last_tile;
     S = S < last_S ? S : last_S;
-    const int S4 = 4 * S;
     const int rlim = m_K - 1 - tile * 16;                           // rows past K repeat row K - 1
     const uint32_t wrc = (uint32_t)(wr < rlim ? wr : rlim);
-    const uint32_t lane_off = __umul24(wrc, lane_mul);
-    const int klim = NCH - 1 - S4;                                  // chunks past N repeat chunk NCH - 1
-    const uint32_t chl = (uint32_t)(kq < klim ? kq : klim);
-    const uint32_t so_t = (uint32_t)tile * tile_a;
-    const uint32_t so_g = (uint32_t)tile * (uint32_t)(16 * m_G);
-    constexpr uint32_t BB = C::CB / 8;
-    const uint32_t voff_m = lane_off + (uint32_t)kq * 4u;
-    const uint32_t voff_c = lane_off + ((((uint32_t)kq * BB) >> 4) << ush) + (((uint32_t)kq * BB) & 15u);
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      int chc = S4 + c;
-      chc = chc < NCH ? chc : NCH - 1;
-      if (!C::DENSE) L.mk[c] = *(const uint32_t*)(m_data + (so_t + ((uint32_t)chc << ush) + voff_m));
-      const uint8_t* cp = m_data + (so_t + ((code_u0 + (uint32_t)chc * (C::CHB / 128)) << ush) + voff_c);
-      if (C::CB == 32) {
-        L.raw[c] = *(const uint32_t*)cp;
-      } else if (C::CB == 64) {
-        const uint2 v = *(const uint2*)cp;
-        L.raw[2 * c] = v.x; L.raw[2 * c + 1] = v.y;
-      } else {
-        const uint4 v = *(const uint4*)cp;
-        L.raw[4 * c] = v.x; L.raw[4 * c + 1] = v.y; L.raw[4 * c + 2] = v.z; L.raw[4 * c + 3] = v.w;
-      }
-    }
-    const uint32_t gv = so_g + ((uint32_t)S4 << csh) + __umul24(wrc, sz_mul) + (chl << csh);
-    L.zraw = (uint32_t)m_zero[gv] | ((uint32_t)m_scale[gv] << 8);
+    const StepAt at{m_data, m_scale, m_zero, (uint32_t)tile * tile_a, (uint32_t)tile * (uint32_t)(16 * m_G),
+                    (uint32_t)__umul24(wrc, lane_mul), (uint32_t)__umul24(wrc, sz_mul), code_u0, ush, csh, NCH};
+    if constexpr (TURN) load_chunk<C>(at, 4 * S, kq, L);
+    else load_blocks<C>(at, 4 * S, kq, L);
   };
 
   // this wave's (tile, part, macro-step) positions: items wave, wave + 16, ... of the slab
@@ -979,54 +1029,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
       for (int p = 0; p < MP; ++p) ysum[p] = 0.f;
     }
     issue(T_lo + p1.tl, p1.S, tgt);
-    uint32_t zs[4];                                                 // zero | scale << 8 of the groups 4S .. 4S+3
-#pragma unroll
-    for (int c = 0; c < 4; ++c) zs[c] = (uint32_t)__shfl((int)cur.zraw, wr + 16 * c, 64);
-    bool a_on[NG];
-    uint32_t a_base[NG];
-    int dm[NG];                                                     // the activation rows this quarter sums
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      a_on[g] = a_dig < NDIG && a_m + 4 * g < M;
-      a_base[g] = xq_off + (uint32_t)(((a_m + 4 * g) * NDIG + a_dig) * (Ns + X_PAD) + kq * 32);
-      dm[g] = kq + 4 * g < M ? kq + 4 * g : 0;
-    }
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int chunk = 4 * S + c;
-      uint32_t aaddr[NG];
-#pragma unroll
-      for (int g = 0; g < NG; ++g) aaddr[g] = (a_on[g] && chunk < NCH) ? a_base[g] + (uint32_t)(chunk - ch0) * 128u : z_off;
-      uint32_t rkc[4];
-      uint2 selc[4];
-      fetch_selectors<C>(cur.mk[c], lut, l16, rkc, selc);
-      uint32_t st[C::NW];
-#pragma unroll
-      for (int k = 0; k < C::NW; ++k) st[k] = cur.raw[c * C::NW + k];
-      const uint32_t z = zs[c] & 0xFFu;
-      const uint32_t nz = 0x80808080u - z * 0x01010101u;
-      v4i acc[NG];
-#pragma unroll
-      for (int g = 0; g < NG; ++g) acc[g] = (v4i){0, 0, 0, 0};
-#pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        uint32_t bfrag[4];
-        decode_half<C, BITS>(st, rkc, selc, nz, half, bfrag);
-        const v4i bv = (v4i){(int)bfrag[0], (int)bfrag[1], (int)bfrag[2], (int)bfrag[3]};
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-          const v4i av = *(const v4i*)(smem + aaddr[g] + 16 * half);
-          acc[g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bv, acc[g], 0, 0, 0);
-          asm("s_nop 1" : "+v"(acc[g]));                            // see the main kernel
-        }
-      }
-#pragma unroll
-      for (int g = 0; g < NG; ++g) {
-        const float dl = delta[dm[g] * (NCH + 4) + chunk];          // 0 past the last chunk
-        const float f = fmaf((float)(acc[g][0] * 256 + acc[g][1]), 256.f, (float)acc[g][2]);
-        ysum[4 * g + c] = fmaf(f, h2f((uint16_t)(zs[c] >> 8)) * dl, ysum[4 * g + c]);
-      }
-    }
+    block_step<C, BITS, NG, TURN>(cur, smem, lut, l16, lane, S, XDigits{xq_off, z_off, delta, Ns, ch0, NCH, M}, ysum);
     if (S + 1 == s_end) {
       // the part is done: lane quarter kq holds activation row 4g + kq of weight row wr
 #pragma unroll
@@ -1308,7 +1311,7 @@ static int launch_stream_m(const DMat& m, const void* x, int64_t ldx, int xdt, v
 
 // ------------------------------------------------------------------ survivor-stream rows on the matrix cores
 // SPARSE4X / SPARSE4E (a code offset per group in the row) in 16-row tiles on the 16x16x64 int8
-// MFMA, block-per-quarter arrangement: lane (weight row wr, quarter kq) decodes block kq of each
+// MFMA, quarter-per-block arrangement: lane (weight row wr, quarter kq) decodes block kq of each
 // of the four groups of a 512-column step, one MFMA covers 64 columns of one group for up to four
 // activation rows, a second one the rows 4..7.  The rows of a tile have different lengths, so
 // every lane finds its codes itself: the group's mask words and code offset are loaded a step
@@ -1409,15 +1412,6 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_stream_mfma_kernel(SmArgs a) 
     g = g < m_G ? g : m_G - 1;                                      // groups past the row repeat the last one
     k.mk = ((const uint4*)row)[g];
     k.go = (uint32_t)((const uint16_t*)(row + go_off))[g];
-  };
-  // r0..r3 hold, in lane quarter q, the values (q, 0..3); afterwards register i holds (i, q):
-  // the upper two quarters of r0 / r1 change places with the lower two of r2 / r3, then the odd
-  // quarters of r0 / r2 with the even ones of r1 / r3.  (Inline assembly as in quarter_sum.)
-  auto transpose4 = [&](uint32_t& r0, uint32_t& r1, uint32_t& r2, uint32_t& r3) {
-    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(r0), "+v"(r2));
-    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(r1), "+v"(r3));
-    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(r0), "+v"(r1));
-    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(r2), "+v"(r3));
   };
   auto issue_codes = [&](const Pos& p, const SmMask& k, SmCodes& c) {
     const uint32_t cbase = p.ro + hdr;                              // the row's codes (16-byte aligned)
@@ -2155,7 +2149,6 @@ static bool keep_supported(int keep) { return keep == 10 || keep == 16 || keep =
 
 bool gemv_fast_takes(const DMat& m, int M) {
   if (M < 1 || M > GV_MAX_M) return false;
-  if (M > 4 && !block_split_capable(m.bits, family_of(m.layout) == FAM_DENSE ? 0 : m.keep, m.group)) return false;
   if (m.cs_rows == 3) return false;                              // the caller splits q|k|v into its ranges
   if (!(m.flags & CBK_FLAG_ZERO_LE_128)) return false;
   const int fam = family_of(m.layout);
@@ -2207,7 +2200,7 @@ static inline size_t main_x_budget(int M, int delta_cap, int sk_cap) {
 }
 
 // Rows whose digits (M * 3 * N bytes) stay within SPLIT_MIN_BYTES need no workspace; longer ones (two
-// to eight activation rows of a block-per-quarter configuration) are split over the workgroups by
+// to eight activation rows) are split over the workgroups by
 // columns when the caller provides room for the part sums: [tiles][parts <= 16][M][16] floats.
 constexpr size_t SPLIT_MIN_BYTES = 90 * 1024;  // digits of a row (M * 3 * N bytes) from which it is split (measured on both layer sets
                                                // at 56, 72, 90 and 112 KB: six rows of 5376 and eight of 4096 columns gain, seven of 4096 lose)
@@ -2219,7 +2212,7 @@ static inline int kernel_rows(const DMat& m, int M) {            // activation r
 
 size_t gemv_fast_workspace(const DMat& m, int M) {
   const int Mk = kernel_rows(m, M);
-  if (Mk < 2 || !block_split_capable(m.bits, family_of(m.layout) == FAM_DENSE ? 0 : m.keep, m.group)) return 0;
+  if (Mk < 2) return 0;
   const size_t digits = (size_t)Mk * NDIG * (m.N + X_PAD);
   if (digits <= SPLIT_MIN_BYTES) return 0;
   // what a call with this matrix alone would do
@@ -2257,14 +2250,11 @@ static int launch_cfg(const GvBatch& b, size_t lds, int blocks, hipStream_t st) 
 template <int BITS, int KEEP, int GRP>
 static int launch_mp(const GvBatch& b, size_t lds, int blocks, hipStream_t st) {
   if (b.h.M == 1) return launch_cfg<BITS, KEEP, GRP, 1>(b, lds, blocks, st);
-  if constexpr (!block_split_capable(BITS, KEEP, GRP)) {
+  // (two rows: a pass each costs less than turning the blocks, 21504 x 5376 3-bit keep 10: 19.7 against 20.7 us)
+  if constexpr (!block_loads(BITS, KEEP, GRP)) {
     if (b.h.M == 2) return launch_cfg<BITS, KEEP, GRP, 2>(b, lds, blocks, st);
   }
-  if constexpr (block_split_capable(BITS, KEEP, GRP)) {
-    if (b.h.M > 4) return launch_cfg<BITS, KEEP, GRP, 8>(b, lds, blocks, st);
-  } else {
-    if (b.h.M > 4) return CBK_ERR_UNSUPPORTED;
-  }
+  if (b.h.M > 4) return launch_cfg<BITS, KEEP, GRP, 8>(b, lds, blocks, st);
   return launch_cfg<BITS, KEEP, GRP, 4>(b, lds, blocks, st);
 }
 
@@ -2302,20 +2292,37 @@ static int gemv_blocks(const GvBatch& gb, int n, int tiles) {
 
 template <int BITS, int KEEP, int GRP, int MP>
 static int launch_split_cfg(const GsArgs& a, size_t lds, int blocks, int red_blocks, hipStream_t st) {
-  if constexpr ((MP == 4 || MP == 8) && block_split_capable(BITS, KEEP, GRP)) {
-    auto kern = gemv_split_kernel<BITS, KEEP, GRP, MP>;
-    static std::atomic<int> configured{0};
-    if (!configured.load(std::memory_order_acquire)) {
-      if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
-        return CBK_ERR_HIP;
-      configured.store(1, std::memory_order_release);
-    }
-    hipLaunchKernelGGL(kern, dim3(blocks), dim3(GV_THREADS), lds, st, a);
-    if (hipGetLastError() != hipSuccess) return CBK_ERR_HIP;
-    hipLaunchKernelGGL(gemv_split_reduce_kernel, dim3(red_blocks), dim3(GS_RED_THREADS), 0, st, a);
-    return hipGetLastError() == hipSuccess ? CBK_OK : CBK_ERR_HIP;
-  } else {
-    return CBK_ERR_UNSUPPORTED;
+  auto kern = gemv_split_kernel<BITS, KEEP, GRP, MP>;
+  static std::atomic<int> configured{0};
+  if (!configured.load(std::memory_order_acquire)) {
+    if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
+      return CBK_ERR_HIP;
+    configured.store(1, std::memory_order_release);
+  }
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(GV_THREADS), lds, st, a);
+  if (hipGetLastError() != hipSuccess) return CBK_ERR_HIP;
+  hipLaunchKernelGGL(gemv_split_reduce_kernel, dim3(red_blocks), dim3(GS_RED_THREADS), 0, st, a);
+  return hipGetLastError() == hipSuccess ? CBK_OK : CBK_ERR_HIP;
+}
+template <int BITS, int KEEP>
+static int launch_split_grp(const GsArgs& a, size_t lds, int blocks, int red_blocks, hipStream_t st) {
+  if constexpr (BITS != 6) {
+    if (a.mat[0].g.m.group == 64)
+      return a.h.M > 4 ? launch_split_cfg<BITS, KEEP, 64, 8>(a, lds, blocks, red_blocks, st)
+                       : launch_split_cfg<BITS, KEEP, 64, 4>(a, lds, blocks, red_blocks, st);
+  }
+  return a.h.M > 4 ? launch_split_cfg<BITS, KEEP, 128, 8>(a, lds, blocks, red_blocks, st)
+                   : launch_split_cfg<BITS, KEEP, 128, 4>(a, lds, blocks, red_blocks, st);
+}
+template <int BITS>
+static int launch_split_keep(const GsArgs& a, size_t lds, int blocks, int red_blocks, hipStream_t st) {
+  const DMat& m = a.mat[0].g.m;
+  switch (family_of(m.layout) == FAM_DENSE ? 0 : m.keep) {
+    case 0: return launch_split_grp<BITS, 0>(a, lds, blocks, red_blocks, st);
+    case 10: return launch_split_grp<BITS, 10>(a, lds, blocks, red_blocks, st);
+    case 16: return launch_split_grp<BITS, 16>(a, lds, blocks, red_blocks, st);
+    case 23: return launch_split_grp<BITS, 23>(a, lds, blocks, red_blocks, st);
+    default: return CBK_ERR_UNSUPPORTED;
   }
 }
 
@@ -2378,16 +2385,10 @@ static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt,
   a.h.xq_cap = xq_cap; a.h.delta_cap = delta_cap;
   const size_t lds = (size_t)LUT_BYTES + ZERO_BYTES + xq_cap + (size_t)delta_cap * 4;
   if (lds > 160 * 1024) return CBK_ERR_UNSUPPORTED;
-  const DMat& m = mats[0].m;
-  const int keep = family_of(m.layout) == FAM_DENSE ? 0 : m.keep;
-  const bool big = M > 4;
-  const int rb = th / GS_RED_THREADS;
-  if (m.group != 128) return CBK_ERR_UNSUPPORTED;
-  if (m.bits == 4 && keep == 16) return big ? launch_split_cfg<4, 16, 128, 8>(a, lds, wg, rb, st) : launch_split_cfg<4, 16, 128, 4>(a, lds, wg, rb, st);
-  if (m.bits == 4 && keep == 0) return big ? launch_split_cfg<4, 0, 128, 8>(a, lds, wg, rb, st) : launch_split_cfg<4, 0, 128, 4>(a, lds, wg, rb, st);
-  if (m.bits == 2 && keep == 16) return big ? launch_split_cfg<2, 16, 128, 8>(a, lds, wg, rb, st) : launch_split_cfg<2, 16, 128, 4>(a, lds, wg, rb, st);
-  if (m.bits == 2 && keep == 0) return big ? launch_split_cfg<2, 0, 128, 8>(a, lds, wg, rb, st) : launch_split_cfg<2, 0, 128, 4>(a, lds, wg, rb, st);
-  return CBK_ERR_UNSUPPORTED;
+  const int bits = mats[0].m.bits, rb = th / GS_RED_THREADS;
+  if (bits == 6) return launch_split_grp<6, 16>(a, lds, wg, rb, st);  // BLK1632_6: one configuration
+  return bits == 2 ? launch_split_keep<2>(a, lds, wg, rb, st) : bits == 3 ? launch_split_keep<3>(a, lds, wg, rb, st)
+       : bits == 4 ? launch_split_keep<4>(a, lds, wg, rb, st) : CBK_ERR_UNSUPPORTED;
 }
 
 // Distribution over the workgroups, LDS and launch of the matrices of `gb` (spi and sk set).
@@ -2491,14 +2492,13 @@ int launch_gemv_fast_batch(int n, const GvCall* calls, int xdt, int M, int ydt, 
     sk_cap = sk_cap > g.sk ? sk_cap : g.sk;
   }
   // Matrices for the column-split kernel (one launch pair for all of them, behind the others),
-  // where the configuration has one and the caller has left room for the part sums: rows whose
+  // where the caller has left room for the part sums: rows whose
   // digits do not fit the staging area of the main kernel, and, in launches of at most
   // SPLIT_MAX_TILES tiles, rows whose digits take more than SPLIT_MIN_BYTES of it (eight rows of
   // 5376 columns: every workgroup of the main kernel converts all of them before its first step
   // and is left with four reduction slots; gate,up of that shape 43 us there, 30 + 5 us split).
   // Otherwise the main kernel stages long rows slab by slab.
-  const DMat& m0 = gb.mat[0].m;
-  if (M > 1 && block_split_capable(m0.bits, family_of(m0.layout) == FAM_DENSE ? 0 : m0.keep, m0.group)) {
+  if (M > 1) {
     const size_t x_budget = main_x_budget(M, delta_cap, sk_cap);
     auto splits = [&](const GvMat& g) {
       const size_t digits = (size_t)M * NDIG * (g.m.N + X_PAD);

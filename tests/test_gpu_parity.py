@@ -489,6 +489,27 @@ def test_gemv_five_to_eight_rows_equal_single_rows(case):
             assert torch.equal(ops.gemv(pm, x, bias=bias, out_dtype=torch.float32), y)
 
 
+DECODE_CASES = [(F.BLK1632_6, 6, 128, 16)] + [(F.BLKC if k else F.DENSEB, b, g, k) for b in (2, 3, 4) for k in (0, 10, 16, 23) for g in (64, 128)]
+
+
+@pytest.mark.parametrize("case", DECODE_CASES, ids=case_id)
+def test_gemv_rows_do_not_depend_on_their_number(case):
+    """Two to eight activation rows share a pass over the weights in an arrangement of their own
+    (blocks turned between the lane quarters, two half-zero operands for groups of 64): row m is the
+    one-row result of row m bit for bit.  One column chunk, row tails, chunk counts off the four of a
+    step, rows split over the workgroups by columns (and the same without room for their part
+    sums), both byte orders."""
+    for (K, N, Ms) in ((16, 128, (2, 3, 8)), (33, 640, (2, 4, 5)), (7, 1664, (3, 7)), (40, 11136, (2, 4, 8))):
+        rows = F.synth_packed(K, N, case[0], case[1], case[2], case[3] or None, seed=K + N, device=DEV)
+        for pm in (rows, rows.to_tiled()):
+            for M in Ms:
+                x = acts(M, N, torch.float16, seed=M + N).to(DEV)
+                one = torch.cat([ops.gemv(pm, x[i:i + 1], out_dtype=torch.float32) for i in range(M)])
+                assert torch.equal(ops.gemv(pm, x, out_dtype=torch.float32), one), (K, N, M, pm is rows)
+                small = torch.empty(256, dtype=torch.uint8, device=DEV)
+                assert torch.equal(ops.gemv(pm, x, out_dtype=torch.float32, workspace=small), one), (K, N, M, pm is rows)
+
+
 @pytest.mark.parametrize("case", [(F.BLK1632_4, 4, 128, 16), (F.DENSE4, 4, 128, 0), (F.BLKC, 3, 128, 10)], ids=case_id)
 def test_gemv_rows_longer_than_the_staging_area(case):
     """Rows whose activation digits do not fit in LDS are staged and multiplied in column slabs, the
