@@ -127,19 +127,21 @@ __host__ __device__ constexpr int frag_col(int bits, bool dense, int bi) {
 }
 
 // Two ways to lay a macro-step (16 rows x 512 columns) on the 16x16x64 MFMA.
-//  * quarter-per-chunk (M = 1, and M = 2 where the other way needs the turn): lane quarter kq decodes chunk 4S + kq; one MFMA adds four different
+//  * quarter-per-chunk (M = 1, and M = 2 where the other way costs more): lane quarter kq decodes chunk 4S + kq; one MFMA adds four different
 //    quantisation groups, so the A rows are (quarter, digit) and one activation row needs one pass.
 //  * quarter-per-block (else): lane quarter kq decodes block kq (32 columns) of each of the four
 //    chunks; one MFMA covers 64 columns of one chunk, the A rows are (activation row, digit), and up
 //    to four activation rows share every MFMA.  Groups of 64 columns are the lower and the upper two
 //    quarters of a chunk: two MFMAs, each with an A operand that is zero in the other half.
-// A lane loads its own block where the block's code bits are 4, 8 or 16 whole bytes; in every other
+// A lane loads its own block where the block's code bits are 4, 8, 16 or 32 whole bytes; in every other
 // code width it loads and aligns a whole chunk, as for M = 1, and the streams of the four blocks,
 // their masks (and high bits) change places between the lane quarters in registers.
-__host__ __device__ constexpr bool block_loads(int bits, int keep, int grp) {
+__host__ __device__ constexpr bool block_loads(int bits, int keep) {
   const int cb = (keep == 0 ? 32 : keep) * bits;
-  return grp == 128 && bits != 3 && bits != 6 && (cb == 32 || cb == 64 || cb == 128);
+  return bits != 3 && bits != 6 && (cb == 32 || cb == 64 || cb == 128 || cb == 256);
 }
+// Digit order of a configuration inside a 16-column fragment (GvMat::order)
+__host__ __device__ constexpr int digit_order(int bits, bool dense) { return !dense || bits == 8 ? 0 : bits == 2 ? 2 : 1; }
 
 // ------------------------------------------------------------------ activation prep
 // x' = x * col_scale per 128-column chunk -> delta and three signed int8 digits per column:
@@ -283,6 +285,11 @@ __device__ inline void fetch_selectors(uint32_t mw, const uint2* lut, uint32_t l
 template <class C, int BITS>
 __device__ inline void decode_half(const uint32_t (&st)[C::NW], const uint32_t (&rk)[4], const uint2 (&sel4)[4],
                                    uint32_t nz, int half, uint32_t (&bfrag)[4], uint32_t hw = 0) {
+  if constexpr (BITS == 8) {                             // q - 128; the zero point is a second operand (zero8)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) bfrag[k] = st[4 * half + k] ^ 0x80808080u;
+    return;
+  }
 #pragma unroll
   for (int jj2 = 0; jj2 < 2; ++jj2) {
     const int jj = 2 * half + jj2;                       // mask byte inside the block
@@ -323,6 +330,16 @@ __device__ inline void decode_half(const uint32_t (&st)[C::NW], const uint32_t (
   }
 }
 
+// 8-bit codes: q - z needs nine bits, so the matrix instruction gets q - 128 and, in two more, the two halves of
+// 128 - z (-63 ... 64), into the same exact sums.  (The decode of such a fragment is four xors; sums of their own
+// for one constant z - 128 would take the registers that the second buffer of 32 dwords needs.)  On the row kernel below, a
+// wavefront per row: 21504 x 5376 at 1 / 8 rows 42.7 / 101 us, here 24.3 / 30; 5376 x 21504 53 / 346 and 28 / 28.
+__device__ inline v4i zero8(uint32_t z, int part) {
+  const int d = 128 - (int)z, h = part ? d - (d >> 1) : d >> 1;
+  const int b = (int)(((uint32_t)h & 0xFFu) * 0x01010101u);
+  return (v4i){b, b, b, b};
+}
+
 // ------------------------------------------------------------------ the decode kernel
 template <class C>
 struct Loads {
@@ -353,8 +370,24 @@ struct StepAt {
   uint32_t code_u0;
   int ush, csh, NCH;
 };
+// zero points and scales of chunk S4 + kq (chunks past N repeat chunk NCH - 1)
+template <class C>
+__device__ inline void load_meta(const StepAt& p, int S4, int kq, Loads<C>& L) {
+  const int klim = p.NCH - 1 - S4;
+  const uint32_t chl = (uint32_t)(kq < klim ? kq : klim);
+  const uint32_t gv = p.so_g + ((uint32_t)(S4 * C::NGC) << p.csh) + p.sz_off + ((chl * C::NGC) << p.csh);
+  if (C::NGC == 1) {
+    L.zraw = p.zero[gv];
+    L.sc[0] = p.scale[gv];
+  } else {
+    const uint32_t gv1 = gv + (1u << p.csh);
+    L.zraw = (uint32_t)p.zero[gv] | ((uint32_t)p.zero[gv1] << 8);
+    L.sc[0] = p.scale[gv];
+    L.sc[C::NGC - 1] = p.scale[gv1];
+  }
+}
 // quarter-per-block: block kq of the chunks S4 .. S4 + 3, one mask dword and CB / 8 code bytes each; the zero
-// point and scale of chunk S4 + kq, which the other quarters fetch from this lane
+// points and scales of chunk S4 + kq, which the other quarters fetch from this lane
 template <class C>
 __device__ inline void load_blocks(const StepAt& p, int S4, int kq, Loads<C>& L) {
   constexpr uint32_t BB = C::CB / 8;
@@ -372,14 +405,15 @@ __device__ inline void load_blocks(const StepAt& p, int S4, int kq, Loads<C>& L)
       const uint2 v = *(const uint2*)cp;
       L.raw[2 * c] = v.x; L.raw[2 * c + 1] = v.y;
     } else {
-      const uint4 v = *(const uint4*)cp;
-      L.raw[4 * c] = v.x; L.raw[4 * c + 1] = v.y; L.raw[4 * c + 2] = v.z; L.raw[4 * c + 3] = v.w;
+#pragma unroll
+      for (int i = 0; i < C::CB / 128; ++i) {
+        const uint4 v = *(const uint4*)(cp + ((uint32_t)i << p.ush));
+        const int o = (C::CB / 32) * c + 4 * i;
+        L.raw[o] = v.x; L.raw[o + 1] = v.y; L.raw[o + 2] = v.z; L.raw[o + 3] = v.w;
+      }
     }
   }
-  const int klim = p.NCH - 1 - S4;                                  // chunks past N repeat chunk NCH - 1
-  const uint32_t chl = (uint32_t)(kq < klim ? kq : klim);
-  const uint32_t gv = p.so_g + ((uint32_t)S4 << p.csh) + p.sz_off + (chl << p.csh);
-  L.zraw = (uint32_t)p.zero[gv] | ((uint32_t)p.scale[gv] << 8);
+  load_meta<C>(p, S4, kq, L);
 }
 // quarter-per-chunk: chunk S4 + kq whole
 template <class C>
@@ -413,16 +447,7 @@ __device__ inline void load_chunk(const StepAt& p, int S4, int kq, Loads<C>& L) 
     const uint4 v = *(const uint4*)(p.data + (p.so_t + ((3u * (uint32_t)p.NCH + (uint32_t)S4 + chl) << p.ush) + p.lane_off));
     L.h2[0] = v.x; L.h2[1] = v.y; L.h2[2] = v.z; L.h2[3] = v.w;
   }
-  const uint32_t gv = p.so_g + ((uint32_t)(S4 * C::NGC) << p.csh) + p.sz_off + ((chl * C::NGC) << p.csh);
-  if (C::NGC == 1) {
-    L.zraw = p.zero[gv];
-    L.sc[0] = p.scale[gv];
-  } else {
-    const uint32_t gv1 = gv + (1u << p.csh);
-    L.zraw = (uint32_t)p.zero[gv] | ((uint32_t)p.zero[gv1] << 8);
-    L.sc[0] = p.scale[gv];
-    L.sc[C::NGC - 1] = p.scale[gv1];
-  }
+  load_meta<C>(p, S4, kq, L);
 }
 
 // One macro-step in the quarter-per-block arrangement: adds 16 rows x 512 columns to the sums ysum[4 g + c]
@@ -457,7 +482,7 @@ __device__ inline void block_step(const Loads<C>& cur, const uint8_t* smem, cons
   uint32_t zs[4][NGC];                                              // zero | scale << 8 of the groups of the chunks 4S .. 4S+3
 #pragma unroll
   for (int g = 0; g < NGC; ++g) {
-    const uint32_t own = !TURN ? cur.zraw : ((cur.zraw >> (8 * g)) & 0xFFu) | (cur.sc[TURN ? g : 0] << 8);
+    const uint32_t own = ((cur.zraw >> (8 * g)) & 0xFFu) | (cur.sc[g] << 8);
 #pragma unroll
     for (int c = 0; c < 4; ++c) zs[c][g] = (uint32_t)__shfl((int)own, wr + 16 * c, 64);
   }
@@ -509,6 +534,13 @@ __device__ inline void block_step(const Loads<C>& cur, const uint8_t* smem, cons
           const v4i av = *(const v4i*)(smem + aaddr[g][h] + 16 * half);
           acc[g][h] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bv, acc[g][h], 0, 0, 0);
           asm("s_nop 1" : "+v"(acc[g][h]));                         // see the decode path of one activation row
+          if constexpr (BITS == 8) {
+#pragma unroll
+            for (int part = 0; part < 2; ++part) {
+              acc[g][h] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, zero8(z, part), acc[g][h], 0, 0, 0);
+              asm("s_nop 1" : "+v"(acc[g][h]));
+            }
+          }
         }
     }
     // the 128 columns of the chunk are complete: rows 4 kq .. 4 kq + 2 of the result are the three digit
@@ -529,7 +561,7 @@ template <int BITS, int KEEP, int GRP, int MP>
 __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
   using C = Cfg<BITS, KEEP, GRP, MP>;
   static_assert(MP == 1 || MP == 2 || MP == 4 || MP == 8, "single activation rows, or row groups of four");
-  constexpr bool QB = MP >= 4, TURN = QB && !block_loads(BITS, KEEP, GRP);
+  constexpr bool QB = MP >= 4, TURN = QB && !block_loads(BITS, KEEP);
   constexpr int NG = MP == 8 ? 2 : 1;                  // groups of four activation rows, one MFMA each per fragment
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -622,7 +654,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
     // waits for the weight loads as well; the conversion would start only once the first weights
     // have arrived instead of running while they are on their way.
     // (The second item only where its sixteen registers do not push the kernel into scratch.)
-    constexpr bool PRE2 = MP == 1 || (MP == 4 && QB);
+    constexpr bool PRE2 = BITS != 8 && (MP == 1 || (MP == 4 && QB));
     int xit = tid;
     XLoad xl, xl2;
     if (xit < xitems) stage_load(gm.x, gm.ldx, m.cs, N, col0, n16, xit, MP == 1, gm.par, xl);
@@ -701,7 +733,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
     // ---- stage: selector table and counters (once), activation digits and deltas of this matrix
     if (!first) __syncthreads();                                  // previous matrix fully consumed
     first = false;
-    constexpr int XORD = !C::DENSE ? 0 : (BITS == 2 ? 2 : 1);
+    constexpr int XORD = digit_order(BITS, C::DENSE);
     if (xit < xitems) stage_convert<XORD>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, xit, MP == 1, xq, delta, X_PAD);
     if (PRE2 && xit + GV_THREADS < xitems)
       stage_convert<XORD>(xl2, m.cs != nullptr, h.xdt, N, ch0, n16, xit + GV_THREADS, MP == 1, xq, delta, X_PAD);
@@ -769,6 +801,13 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
               // kernel (register allocations in which the accumulator chain changes registers)
               // returned run-to-run different sums on gfx950; with it every configuration is exact.
               asm("s_nop 1" : "+v"(acc[p]));
+              if constexpr (BITS == 8) {
+#pragma unroll
+                for (int part = 0; part < 2; ++part) {
+                  acc[p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, zero8(z, part), acc[p], 0, 0, 0);
+                  asm("s_nop 1" : "+v"(acc[p]));
+                }
+              }
             }
             // ---- end of a quantisation group: int32 -> float, times scale * delta
             if ((C::NGC == 2 && t == 3) || t == 7) {
@@ -926,7 +965,7 @@ template <int BITS, int KEEP, int GRP, int MP>
 __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
   using C = Cfg<BITS, KEEP, GRP, MP>;
   static_assert(MP == 4 || MP == 8, "row groups of four");
-  constexpr bool TURN = !block_loads(BITS, KEEP, GRP);
+  constexpr bool TURN = !block_loads(BITS, KEEP);
   constexpr int NG = MP / 4;                           // groups of four activation rows, one MFMA each per fragment
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1006,7 +1045,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
   Pos p1 = p0; bool v1 = v0 && advance(p1);
 
   // ---- stage the slab's digits (the activation loads go out before the first weight loads)
-  constexpr int XORD = !C::DENSE ? 0 : (BITS == 2 ? 2 : 1);
+  constexpr int XORD = digit_order(BITS, C::DENSE);
   const int n16 = Ns >> 4, xitems = M * n16;                        // a multiple of 8
   XLoad xl;
   if (tid < xitems) stage_load(gm.x, gm.ldx, m.cs, N, col0, n16, tid, false, gm.par, xl);
@@ -1953,7 +1992,8 @@ int launch_gemv_stream(const DMat& m, const void* x, int xdt, int M, int64_t ldx
 }
 
 // ------------------------------------------------------------------ 8-bit dense rows
-// DENSE8 (group 128) at one to eight activation rows per pass, on the same activation digits:
+// DENSE8 (group 128) rows or arrays too long for the matrix-core kernel (gemv_fast_takes), one to eight activation
+// rows per pass, on the same activation digits:
 // the codes are the bytes themselves, q - 128 is a signed byte (one xor), and
 //   sum_j (q_j - z) X_j = sum_j (q_j - 128) X_j - (z - 128) sum_j X_j
 // with the integer activations X of the group; their sum per 128-column chunk is formed once per
@@ -2150,13 +2190,13 @@ static bool keep_supported(int keep) { return keep == 10 || keep == 16 || keep =
 bool gemv_fast_takes(const DMat& m, int M) {
   if (M < 1 || M > GV_MAX_M) return false;
   if (m.cs_rows == 3) return false;                              // the caller splits q|k|v into its ranges
-  if (!(m.flags & CBK_FLAG_ZERO_LE_128)) return false;
   const int fam = family_of(m.layout);
+  // (q - z in a signed byte; 8-bit codes keep the zero point apart)
+  if (!(m.flags & CBK_FLAG_ZERO_LE_128) && !(fam == FAM_DENSE && m.bits == 8)) return false;
   if (fam == FAM_BLK) { if (!keep_supported(m.keep)) return false; }
-  else if (fam == FAM_DENSE) { if (m.bits == 8) return false; }
   else if (fam == FAM_BLK6) { if (m.bits != 6 || m.keep != 16 || m.group != 128) return false; }
-  else return false;
-  if (m.bits != 2 && m.bits != 3 && m.bits != 4 && fam != FAM_BLK6) return false;
+  else if (fam != FAM_DENSE) return false;
+  if (m.bits != 2 && m.bits != 3 && m.bits != 4 && fam != FAM_BLK6 && (fam != FAM_DENSE || m.bits != 8)) return false;
   // 32-bit offsets inside the kernel: every array of the matrix below 4 GB
   if ((uint64_t)((m.K + 15) / 16 * 16) * m.stride + 1024 >= (1ull << 32)) return false;
   if ((uint64_t)((m.K + 15) / 16 * 16) * m.G * 2 >= (1ull << 32)) return false;
@@ -2204,6 +2244,12 @@ static inline size_t main_x_budget(int M, int delta_cap, int sk_cap) {
 // columns when the caller provides room for the part sums: [tiles][parts <= 16][M][16] floats.
 constexpr size_t SPLIT_MIN_BYTES = 90 * 1024;  // digits of a row (M * 3 * N bytes) from which it is split (measured on both layer sets
                                                // at 56, 72, 90 and 112 KB: six rows of 5376 and eight of 4096 columns gain, seven of 4096 lose)
+// 8-bit codes at five to eight rows are split from two million weights on: two buffers of 32 dwords beside the sums of
+// eight rows spill registers in the main kernel (us at eight rows, main / split: 512 x 1024 7.1 / 8.0, 2048 x 2048
+// 9.4 / 8.0, 4096 x 4096 17.5 / 10.3, 1024 x 16384 39 / 11).
+static inline size_t split_min_bytes(const DMat& m, int M) {
+  return m.bits == 8 && M > 4 && (size_t)m.K * m.N >= (2u << 20) ? 0 : SPLIT_MIN_BYTES;
+}
 constexpr int SPLIT_MAX_TILES = 4096;          // (rows that fit are split only in launches of at most this many tiles)
 static inline int kernel_rows(const DMat& m, int M) {            // activation rows as the kernel counts them, per pass
   const int v = m.cs_rows == 2 ? 2 : 1;
@@ -2214,7 +2260,7 @@ size_t gemv_fast_workspace(const DMat& m, int M) {
   const int Mk = kernel_rows(m, M);
   if (Mk < 2) return 0;
   const size_t digits = (size_t)Mk * NDIG * (m.N + X_PAD);
-  if (digits <= SPLIT_MIN_BYTES) return 0;
+  if (digits <= split_min_bytes(m, Mk)) return 0;
   // what a call with this matrix alone would do
   const int ntiles = (m.K + 15) / 16, nS = (m.N / 128 + 3) / 4;
   int spi, sk;
@@ -2250,8 +2296,9 @@ static int launch_cfg(const GvBatch& b, size_t lds, int blocks, hipStream_t st) 
 template <int BITS, int KEEP, int GRP>
 static int launch_mp(const GvBatch& b, size_t lds, int blocks, hipStream_t st) {
   if (b.h.M == 1) return launch_cfg<BITS, KEEP, GRP, 1>(b, lds, blocks, st);
-  // (two rows: a pass each costs less than turning the blocks, 21504 x 5376 3-bit keep 10: 19.7 against 20.7 us)
-  if constexpr (!block_loads(BITS, KEEP, GRP)) {
+  // (two rows: a pass each costs less than turning the blocks or halving the operands, 21504 x 5376 3-bit keep 10: 19.7
+  // against 20.7 us)
+  if constexpr (!block_loads(BITS, KEEP) || GRP == 64) {
     if (b.h.M == 2) return launch_cfg<BITS, KEEP, GRP, 2>(b, lds, blocks, st);
   }
   if (b.h.M > 4) return launch_cfg<BITS, KEEP, GRP, 8>(b, lds, blocks, st);
@@ -2387,6 +2434,7 @@ static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt,
   if (lds > 160 * 1024) return CBK_ERR_UNSUPPORTED;
   const int bits = mats[0].m.bits, rb = th / GS_RED_THREADS;
   if (bits == 6) return launch_split_grp<6, 16>(a, lds, wg, rb, st);  // BLK1632_6: one configuration
+  if (bits == 8) return launch_split_grp<8, 0>(a, lds, wg, rb, st);
   return bits == 2 ? launch_split_keep<2>(a, lds, wg, rb, st) : bits == 3 ? launch_split_keep<3>(a, lds, wg, rb, st)
        : bits == 4 ? launch_split_keep<4>(a, lds, wg, rb, st) : CBK_ERR_UNSUPPORTED;
 }
@@ -2447,6 +2495,7 @@ static int launch_main_batch(GvBatch& gb, hipStream_t st) {
   if (lds > 160 * 1024) return CBK_ERR_UNSUPPORTED;
   const int bits = gb.mat[0].m.bits;
   if (bits == 6) return launch_mp<6, 16, 128>(gb, lds, blocks, st);   // BLK1632_6: one configuration
+  if (bits == 8) return launch_grp<8, 0>(gb, lds, blocks, st);
   return bits == 2 ? launch_keep<2>(gb, lds, blocks, st) : bits == 3 ? launch_keep<3>(gb, lds, blocks, st)
        : bits == 4 ? launch_keep<4>(gb, lds, blocks, st) : CBK_ERR_UNSUPPORTED;
 }
@@ -2469,7 +2518,7 @@ int launch_gemv_fast_batch(int n, const GvCall* calls, int xdt, int M, int ydt, 
     const bool dense = family_of(m.layout) == FAM_DENSE;
     GvMat& g = gb.mat[i];
     g.m = m; g.x = (const uint16_t*)calls[i].x; g.ldx = calls[i].ldx;
-    g.order = !dense ? 0 : (m.bits == 2 ? 2 : 1);
+    g.order = digit_order(m.bits, dense);
     g.par = par;
     g.y = calls[i].y; g.bias = calls[i].bias; g.ldy = calls[i].ldy;
     g.ntiles = (m.K + 15) / 16; g.nS = (m.N / 128 + 3) / 4; g.cost0 = cost;
@@ -2502,7 +2551,7 @@ int launch_gemv_fast_batch(int n, const GvCall* calls, int xdt, int M, int ydt, 
     const size_t x_budget = main_x_budget(M, delta_cap, sk_cap);
     auto splits = [&](const GvMat& g) {
       const size_t digits = (size_t)M * NDIG * (g.m.N + X_PAD);
-      return digits > x_budget || (digits > SPLIT_MIN_BYTES && tiles <= SPLIT_MAX_TILES);
+      return digits > x_budget || (digits > split_min_bytes(g.m, M) && tiles <= SPLIT_MAX_TILES);
     };
     GvMat split[GV_MAX_BATCH];
     int ns = 0;

@@ -489,7 +489,8 @@ def test_gemv_five_to_eight_rows_equal_single_rows(case):
             assert torch.equal(ops.gemv(pm, x, bias=bias, out_dtype=torch.float32), y)
 
 
-DECODE_CASES = [(F.BLK1632_6, 6, 128, 16)] + [(F.BLKC if k else F.DENSEB, b, g, k) for b in (2, 3, 4) for k in (0, 10, 16, 23) for g in (64, 128)]
+DECODE_CASES = [(F.BLK1632_6, 6, 128, 16), (F.DENSEB, 8, 64, 0), (F.DENSE8, 8, 128, 0)] + [
+    (F.BLKC if k else F.DENSEB, b, g, k) for b in (2, 3, 4) for k in (0, 10, 16, 23) for g in (64, 128)]
 
 
 @pytest.mark.parametrize("case", DECODE_CASES, ids=case_id)
