@@ -328,28 +328,14 @@ __global__ __launch_bounds__(256) void unpack_fixed_kernel(DMat m, uint8_t* q, u
   }
 }
 
-// Survivor streams, a workgroup per four rows.  DENSE4: instead of bytes, the same row as dense 4-bit
-// codes in tiled order (a pruned column holds its group's zero point), which is how a prefill call
-// re-packs such a matrix; one pass over the stream instead of one to bytes and one back.
-template <bool DENSE4>
-__global__ __launch_bounds__(256) void unpack_sparse_kernel(DMat m, uint8_t* q, uint8_t* mask, uint16_t* oscale,
-                                                            uint8_t* ozero, int summed) {
+// Survivor streams, a workgroup per four rows.
+__global__ __launch_bounds__(256) void unpack_sparse_kernel(DMat m, uint8_t* q, uint8_t* mask, int summed) {
   extern __shared__ uint32_t goff[];
   __shared__ uint2 lut[256 * OCT_LUT_LANES];
   octet_table(lut);
   const uint32_t hdr = stream_header(m), n8 = (uint32_t)m.N >> 3;
-  const int k0 = blockIdx.x * 4;
-  for (int k = k0; k < k0 + 4; ++k) {
-    uint8_t* tile = q + (size_t)(k >> 4) * 16 * (m.N >> 1) + (k & 15) * 16;  // DENSE4 only
-    if (k >= m.K) {                                                 // (DENSE4: the padding rows of the last tile)
-      if (!DENSE4 || k >= ((m.K + 15) & ~15)) break;
-      for (uint32_t j8 = threadIdx.x; j8 < n8; j8 += 256) *(uint32_t*)(tile + (size_t)(j8 >> 2) * 256 + (j8 & 3u) * 4) = 0;
-      for (int g = threadIdx.x; g < m.G; g += 256) {
-        oscale[((size_t)(k >> 4) * m.G + g) * 16 + (k & 15)] = 0;
-        ozero[((size_t)(k >> 4) * m.G + g) * 16 + (k & 15)] = 0;
-      }
-      continue;
-    }
+  const int k0 = blockIdx.x * 4, k1 = m.K - k0 < 4 ? m.K : k0 + 4;
+  for (int k = k0; k < k1; ++k) {
     const uint8_t* row = m.data + m.row_off[k];
     __syncthreads();                                                // the table; the offsets of the row before
     if (summed) {
@@ -358,25 +344,106 @@ __global__ __launch_bounds__(256) void unpack_sparse_kernel(DMat m, uint8_t* q, 
     }
     for (uint32_t j8 = threadIdx.x; j8 < n8; j8 += 256) {
       const Octet o = octet_stream(m, row, hdr, summed ? goff : nullptr, j8, lut);
-      if (!DENSE4) {
-        *(uint2*)(q + (size_t)k * m.N + 8 * (size_t)j8) = make_uint2(o.lo, o.hi);
-        if (mask) mask[(size_t)k * n8 + j8] = (uint8_t)o.keep;
-        continue;
+      *(uint2*)(q + (size_t)k * m.N + 8 * (size_t)j8) = make_uint2(o.lo, o.hi);
+      if (mask) mask[(size_t)k * n8 + j8] = (uint8_t)o.keep;
+    }
+  }
+}
+
+// A survivor-stream matrix as dense 4-bit rows in tiled order (a pruned column holds its group's zero
+// point), which is how a prefill call re-packs it: one pass over the stream.
+//
+// A workgroup takes a tile of sixteen rows; lane 16 b + r decodes block b (32 columns) of a group of row
+// r, so the sixteen rows' units of a block leave as 256 contiguous bytes, and the wavefronts walk
+// neighbouring groups together: the cache lines of the sixteen rows' masks and codes are read once.
+// (A thread per octet of four rows wrote four bytes at a time and looked its group's offset, mask words,
+// zero point and scale up for each.  A call of 21504 x 5376 at 128 rows 226 us, 99 now.)
+constexpr int RP_WIN = 256;                                         // groups whose offsets are summed at a time (SPARSE4)
+__global__ __launch_bounds__(1024) void repack_tile_kernel(DMat m, uint8_t* out, uint16_t* oscale, uint8_t* ozero) {
+  __shared__ uint2 lut[256 * OCT_LUT_LANES];
+  __shared__ uint32_t goff[16][RP_WIN + 1];                         // (+1: the sixteen rows of a group in different banks)
+  __shared__ uint32_t carry[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = (int)blockDim.x >> 6;
+  if (tid < 256) octet_table(lut);
+  const int r = lane & 15, b = lane >> 4, k = (int)blockIdx.x * 16 + r, kc = k < m.K ? k : m.K - 1;
+  const uint32_t hdr = stream_header(m);
+  const uint8_t* row = m.data + m.row_off[kc];
+  const bool sums = m.layout == CBK_SPARSE4;
+  uint8_t* tile = out + (size_t)blockIdx.x * 16 * (m.N >> 1);
+  for (int g0 = 0; g0 < m.G; g0 += RP_WIN) {
+    const int g1 = m.G - g0 < RP_WIN ? m.G : g0 + RP_WIN;
+    __syncthreads();                                                // the table; the offsets of the window before
+    if (sums) {
+      for (int rr = wave; rr < 16; rr += nw) {                      // a wavefront keeps its rows over the windows
+        const int kr = (int)blockIdx.x * 16 + rr;
+        const uint8_t* rp = m.data + m.row_off[kr < m.K ? kr : m.K - 1];
+        uint32_t base = g0 ? carry[rr] : 0u;
+        for (int gw = g0; gw < g1; gw += 64) {
+          const int g = gw + lane;
+          uint32_t c = 0;
+          if (g < g1) {
+            const uint4 w = *(const uint4*)(rp + (size_t)g * 16);
+            c = (uint32_t)(__popc(w.x) + __popc(w.y) + __popc(w.z) + __popc(w.w) + 1) >> 1;
+          }
+          uint32_t s = c;
+#pragma unroll
+          for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t v = (uint32_t)__shfl_up((int)s, o);
+            if (lane >= o) s += v;
+          }
+          if (g < g1) goff[rr][g - g0] = base + s - c;
+          base += (uint32_t)__shfl((int)s, 63);
+        }
+        if (lane == 0) carry[rr] = base;
       }
-      const uint32_t g = j8 >> 4;
-      const size_t mi = (size_t)k * m.G + g;
-      const uint32_t z = m.zero[mi], z4 = (z & 0xFu) * 0x01010101u;
-      const uint32_t k0b = bits_to_bytes(o.keep) * 0xFFu, k1b = bits_to_bytes(o.keep >> 4) * 0xFFu;
-      *(uint32_t*)(tile + (size_t)(j8 >> 2) * 256 + (j8 & 3u) * 4) =
-          (uint32_t)narrow8<4>(o.lo | (z4 & ~k0b), o.hi | (z4 & ~k1b));
-      if ((j8 & 15u) == 0) {
-        oscale[((size_t)(k >> 4) * m.G + g) * 16 + (k & 15)] = m.scale[mi];
-        ozero[((size_t)(k >> 4) * m.G + g) * 16 + (k & 15)] = (uint8_t)z;
+      __syncthreads();
+    }
+    struct Head { uint4 k; uint32_t off, z, sc; };
+    auto head = [&](int g) -> Head {
+      g = g < g1 ? g : g1 - 1;
+      Head h;
+      h.k = *(const uint4*)(row + (size_t)g * 16);
+      h.off = sums ? goff[r][g - g0] : ((const uint16_t*)(row + (m.N >> 3)))[g];
+      const size_t mi = (size_t)kc * m.G + g;
+      h.z = m.zero[mi]; h.sc = m.scale[mi];
+      return h;
+    };
+    Head nx = head(g0 + wave);
+    for (int g = g0 + wave; g < g1; g += nw) {
+      const Head h = nx;
+      const uint32_t c0 = (uint32_t)__popc(h.k.x), c1 = c0 + (uint32_t)__popc(h.k.y), c2 = c1 + (uint32_t)__popc(h.k.z);
+      const uint32_t mw = b == 0 ? h.k.x : b == 1 ? h.k.y : b == 2 ? h.k.z : h.k.w;
+      const uint32_t nib = 2u * (hdr + h.off) + (b == 0 ? 0u : b == 1 ? c0 : b == 2 ? c1 : c2);   // the block's first code
+      const uint32_t* cp = (const uint32_t*)row + (nib >> 3);
+      uint32_t e[5];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) e[i] = cp[i];                     // rows end in a readable tail
+      e[4] = 0;
+      if ((nib & 7u) + (uint32_t)__popc(mw) > 32u) e[4] = cp[4];
+      nx = head(g + nw);
+      uint32_t st[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) st[i] = __builtin_amdgcn_alignbit(e[i + 1], e[i], 4u * (nib & 7u));
+      const uint32_t z4 = (h.z & 0xFu) * 0x01010101u;
+      uint32_t w[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t before = i ? (uint32_t)__popc(mw & ((1u << (8 * i)) - 1u)) : 0u;
+        const Octet o = octet_from_nibbles(i ? window<4>(st, 4u * before) : st[0], (mw >> (8 * i)) & 0xFFu, lut);
+        const uint32_t lo = mask_select(bits_to_bytes(o.keep) * 0xFFu, z4, o.lo), hi = mask_select(bits_to_bytes(o.keep >> 4) * 0xFFu, z4, o.hi);
+        w[i] = (uint32_t)narrow8<4>(lo, hi);
+      }
+      const bool ok = k < m.K;                                      // (the padding rows of the last tile are zero)
+      *(uint4*)(tile + ((size_t)g * 4 + b) * 256 + r * 16) = ok ? make_uint4(w[0], w[1], w[2], w[3]) : make_uint4(0, 0, 0, 0);
+      if (b == 0) {
+        const size_t at = ((size_t)blockIdx.x * m.G + g) * 16 + r;
+        oscale[at] = (uint16_t)(ok ? h.sc : 0u);
+        ozero[at] = (uint8_t)(ok ? h.z : 0u);
       }
     }
   }
-  if (DENSE4 && blockIdx.x == 0 && threadIdx.x < 32)                // readable bytes behind the last tile
-    ((uint4*)(q + (size_t)((m.K + 15) >> 4) * 16 * (m.N >> 1)))[threadIdx.x] = make_uint4(0, 0, 0, 0);
+  if (blockIdx.x == 0 && tid < 32)                                  // readable bytes behind the last tile
+    ((uint4*)(out + (size_t)gridDim.x * 16 * (m.N >> 1)))[tid] = make_uint4(0, 0, 0, 0);
 }
 
 int launch_unpack(const DMat& m, void* q, void* mask, hipStream_t st) {
@@ -385,8 +452,7 @@ int launch_unpack(const DMat& m, void* q, void* mask, hipStream_t st) {
   uint8_t *qb = (uint8_t*)q, *mb = (uint8_t*)mask;
   if (fam == FAM_SPARSE) {
     const int summed = stream_sums(m) ? 1 : 0;
-    hipLaunchKernelGGL(unpack_sparse_kernel<false>, dim3((unsigned)((m.K + 3) / 4)), blk, summed ? (size_t)m.G * 4 : 0, st, m,
-                       qb, mb, nullptr, nullptr, summed);
+    hipLaunchKernelGGL(unpack_sparse_kernel, dim3((unsigned)((m.K + 3) / 4)), blk, summed ? (size_t)m.G * 4 : 0, st, m, qb, mb, summed);
   } else {
     const dim3 grid((unsigned)(((int64_t)((m.K + 15) / 16) * (m.N / 8) + 255) / 256));
     if (fam == FAM_BLK6) hipLaunchKernelGGL((unpack_fixed_kernel<FAM_BLK6, 6>), grid, blk, 0, st, m, qb, mb);
@@ -407,9 +473,10 @@ int launch_unpack(const DMat& m, void* q, void* mask, hipStream_t st) {
 // A survivor-stream matrix as dense 4-bit rows in tiled order: d.data, d.scale, d.zero of the sizes
 // that layout has.
 int launch_repack_dense4(const DMat& m, const DMat& d, hipStream_t st) {
-  const int summed = stream_sums(m) ? 1 : 0;
-  hipLaunchKernelGGL(unpack_sparse_kernel<true>, dim3((unsigned)((m.K + 15) / 16 * 4)), dim3(256),
-                     summed ? (size_t)m.G * 4 : 0, st, m, (uint8_t*)d.data, nullptr, (uint16_t*)d.scale, (uint8_t*)d.zero, summed);
+  // about 4096 wavefronts and more; a wavefront of a wide workgroup has a few groups only
+  const int tiles = (m.K + 15) / 16, threads = tiles >= 1024 ? 256 : tiles >= 512 ? 512 : 1024;
+  hipLaunchKernelGGL(repack_tile_kernel, dim3((unsigned)tiles), dim3(threads), 0, st, m, (uint8_t*)d.data, (uint16_t*)d.scale,
+                     (uint8_t*)d.zero);
   return hipGetLastError() == hipSuccess ? CBK_OK : CBK_ERR_HIP;
 }
 

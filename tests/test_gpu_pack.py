@@ -214,6 +214,18 @@ def test_survivor_streams_repacked_as_dense_rows(case):
     assert rel_fro(y.cpu().numpy(), R.forward_ref(W, acts(5, N, torch.float16, seed=5).float().numpy())) < 1e-3
 
 
+@pytest.mark.parametrize("layout", [F.SPARSE4, F.SPARSE4X], ids=["SPARSE4", "SPARSE4X"])
+@pytest.mark.parametrize("K,N", [(5, 128), (37, 33152), (8208, 384), (16400, 256)])
+def test_survivor_streams_repacked_inside_a_call(layout, K, N):
+    """The image a prefill call re-packs for itself equals the DENSE4 image made at load time: the same
+    kernel on it gives the same bits.  One group, more groups than are summed at a time, row tails,
+    and the widths of workgroup that few and many rows get."""
+    pm = F.synth_packed(K, N, layout, 4, 128, None, seed=K, device=DEV)
+    d4 = ops.transcode(pm, F.DENSE4)
+    x = acts(20, N, torch.float16, seed=3).to(DEV)
+    assert torch.equal(ops.linear(pm, x, out_dtype=torch.float32), ops.linear(d4, x, out_dtype=torch.float32))
+
+
 def test_survivor_stream_with_zero_points_off_the_code_grid():
     """A survivor-stream image may carry zero points that are no 4-bit codes (packed without the
     repair).  A dense layout cannot hold such a matrix (a pruned column stores the zero point as
