@@ -2192,11 +2192,15 @@ bool gemv_fast_takes(const DMat& m, int M) {
   if (m.cs_rows == 3) return false;                              // the caller splits q|k|v into its ranges
   const int fam = family_of(m.layout);
   // (q - z in a signed byte; 8-bit codes keep the zero point apart)
-  if (!(m.flags & CBK_FLAG_ZERO_LE_128) && !(fam == FAM_DENSE && m.bits == 8)) return false;
+  const bool dense8 = fam == FAM_DENSE && m.bits == 8;
+  if (!(m.flags & CBK_FLAG_ZERO_LE_128) && !dense8) return false;
+  // Row-major 8-bit rows stay on their row kernel, whose wavefront reads 2 KB of one row at a time: here sixteen rows
+  // give up a line each per load (one activation row, 21504 x 5376: 44 us against 25; tiled 24)
+  if (dense8 && !m.tiled && m.group == 128) return false;
   if (fam == FAM_BLK) { if (!keep_supported(m.keep)) return false; }
   else if (fam == FAM_BLK6) { if (m.bits != 6 || m.keep != 16 || m.group != 128) return false; }
   else if (fam != FAM_DENSE) return false;
-  if (m.bits != 2 && m.bits != 3 && m.bits != 4 && fam != FAM_BLK6 && (fam != FAM_DENSE || m.bits != 8)) return false;
+  if (m.bits != 2 && m.bits != 3 && m.bits != 4 && fam != FAM_BLK6 && !dense8) return false;
   // 32-bit offsets inside the kernel: every array of the matrix below 4 GB
   if ((uint64_t)((m.K + 15) / 16 * 16) * m.stride + 1024 >= (1ull << 32)) return false;
   if ((uint64_t)((m.K + 15) / 16 * 16) * m.G * 2 >= (1ull << 32)) return false;
