@@ -15,14 +15,16 @@ int launch_gemm_big_b6(const GbArgs&, int blocks, hipStream_t);
 // s_row is the power of two that brings the row's largest |x * col_scale| below 2^15 (1 for
 // nearly every row: only magnitudes beyond fp16's range need it); the GEMM kernel multiplies the
 // row's outputs by it.  Rows M..Mpad-1 and columns N..Npad-1 are zero.
-// One workgroup of 1024 threads per row.  CH: 16-byte pieces of the row a thread keeps in
+// One workgroup of T threads per row.  CH: 16-byte pieces of the row a thread keeps in
 // registers between the two passes (the row is read from memory once); 0 = any row length, the
-// second pass reads the row again.
-template <int CH>
-__global__ __launch_bounds__(1024) void gemm_prep_kernel(const uint16_t* x, int64_t ldx, const uint16_t* cs, int xdt,
+// second pass reads the row again.  Rows of up to 8192 columns take 256 threads, so that a CU has eight
+// of them in flight and a row's chain of load, exchange and store hides behind the others (1024 threads:
+// two in flight; 2 x 2048 rows of 5376 columns 23 -> 18 us); longer rows would need 200 registers
+// at that width (2048 rows of 21504 columns: 68 us, with 1024 threads 40).
+template <int CH, int T>
+__global__ __launch_bounds__(T) void gemm_prep_kernel(const uint16_t* x, int64_t ldx, const uint16_t* cs, int xdt,
                                                          int M, int N, int Npad, uint16_t* out, size_t out_vs, float* row_scale,
                                                          int scale_vs) {
-  constexpr int T = 1024;
   __shared__ float red[T / 64];
   const int row = blockIdx.x, tid = threadIdx.x;
   const int n8 = Npad >> 3, nv = N >> 3;                           // N is a multiple of 128
@@ -218,9 +220,10 @@ int launch_gemm_big(const DMat& m, const void* x, int xdt, int M, int64_t ldx, v
   const size_t xbytes = ((size_t)nv * Mpad * Npad * 2 + 255) & ~(size_t)255;
   const size_t sbytes = ((size_t)nv * Mpad * 4 + 255) & ~(size_t)255;
   float* row_scale = (float*)((uint8_t*)ws + xbytes);
-  const int ch = (Npad / 8 + 1023) / 1024;                         // 16-byte pieces per thread of the row kernel
-  auto prep = ch <= 1 ? gemm_prep_kernel<1> : ch <= 3 ? gemm_prep_kernel<3> : gemm_prep_kernel<0>;
-  hipLaunchKernelGGL(prep, dim3((unsigned)Mpad, (unsigned)nv), dim3(1024), 0, st, (const uint16_t*)x, ldx, m.cs, xdt, M, m.N, Npad,
+  const int p8 = Npad / 8, pt = p8 <= 1024 ? 256 : 1024, ch = (p8 + pt - 1) / pt;   // 16-byte pieces of a row, threads, pieces of a thread
+  auto prep = pt == 1024 ? (ch <= 3 ? gemm_prep_kernel<3, 1024> : gemm_prep_kernel<0, 1024>)
+            : ch <= 1 ? gemm_prep_kernel<1, 256> : ch <= 2 ? gemm_prep_kernel<2, 256> : gemm_prep_kernel<4, 256>;
+  hipLaunchKernelGGL(prep, dim3((unsigned)Mpad, (unsigned)nv), dim3(pt), 0, st, (const uint16_t*)x, ldx, m.cs, xdt, M, m.N, Npad,
                      (uint16_t*)ws, (size_t)Mpad * Npad, row_scale, Mpad);   // one X' per col_scale vector
   GbArgs a;
   a.m = m; a.xp = (const uint16_t*)ws; a.M = M; a.Npad = Npad; a.y = y; a.ydt = ydt; a.ldy = ldy; a.bias = bias;
