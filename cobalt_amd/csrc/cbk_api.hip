@@ -44,9 +44,12 @@ static inline bool gemm_big_takes(const DMat& m, int M) {
 // Two kernels for the fixed-stride layouts: the one that decodes into the registers that multiply
 // (cbk_gemm_skinny.h: few tokens, small matrices) and the 256 x 256 tile (many tokens, whose weight
 // tiles are worth a trip through LDS).  Each knows what a call costs it; the crossover lies between
-// 100 and 600 activation rows, depending on how the matrix fills the chip.
+// 100 and 600 activation rows, depending on how the matrix fills the chip, later for small matrices.  Above 512 rows
+// the first has to be a tenth cheaper, which is what the two models are off by there (3840 x 7424 at 1024 rows: 94 us
+// expected and 98 measured, the tile kernel 94 and 89).
 static inline bool skinny_is_faster(const DMat& m, int M, bool act) {
-  return gemm_skinny_takes(m) && (!gemm_big_takes(m, M) || gemm_skinny_time(m, M) < gemm_big_time(m, M, act));
+  return gemm_skinny_takes(m) &&
+         (!gemm_big_takes(m, M) || gemm_skinny_time(m, M) * (M > 512 ? 1.1 : 1.0) < gemm_big_time(m, M, act));
 }
 // Workspace of run_gemm.  least: what it cannot do without, else what it makes use of.
 static size_t gemm_workspace(const DMat& m, int M, bool least) {

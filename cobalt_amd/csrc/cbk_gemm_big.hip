@@ -144,9 +144,11 @@ static bool gb_fast(const DMat& m) {
 //    take the 256-token tile unless the model below gives the 128-token tile the shorter time,
 //    which it does for small matrices (4096 x 4096 at 256 to 2048 rows: 16 to 128 tiles of 256
 //    tokens): twice the tiles, each 0.8 of the time.
-// Times in microseconds from measurements of this kernel: per 64-column stage 1.1 / 1.25 / 1.7
+// Times in microseconds from measurements of this kernel: per 64-column stage 1.1 / 1.35 / 1.7
 // for the three tiles (the 64-token stage is bound by the weight loads' latency), 8 - 10 per
-// workgroup outside the stage loop, 7 TB/s for the partial tiles, 4 for the reduction kernel.  Over 24 measured calls
+// workgroup outside the stage loop, 4 TB/s for the partial tiles, 5 for the reduction kernel.  (With 1.25 and 7 TB/s,
+// which fit a few small calls better, 4096 x 4096 at 2048 rows went from 92 to 104 us, 3840 x 7424 at 1024 from 89 to
+// 98.)  Over 24 measured calls
 // (eight shapes, 256 / 512 / 2048 rows) the choice is within 2 % of the faster tile; always
 // taking the 256-token tile loses 6 % on average and up to 34 %.
 struct GbPlan { int ti, nsplit; double t; };
@@ -154,7 +156,7 @@ static GbPlan gb_plan_ti(const DMat& m, int M, int ti, int max_split) {
   const int T = 64 * ti;
   const int tiles = ((M + T - 1) / T) * ((m.K + GB_R - 1) / GB_R);
   const int nst = gb_npad(m.N) / GB_K;
-  const double t_stage = ti == 1 ? 1.1 : ti == 2 ? 1.25 : 1.7, t_wg = ti == 1 ? 8.0 : 10.0;
+  const double t_stage = ti == 1 ? 1.1 : ti == 2 ? 1.35 : 1.7, t_wg = ti == 1 ? 8.0 : 10.0;
   GbPlan best{ti, 1, 0.0};
   double t1 = 0;
   const bool may_split = max_split > 1 && m.cs_rows != 2 && gb_fast(m);
@@ -163,7 +165,7 @@ static GbPlan gb_plan_ti(const DMat& m, int M, int ti, int max_split) {
     if (s > 1 && (s - 1) * per >= nst) continue;                    // a part would be empty
     const double rounds = (double)((tiles * s + 255) / 256);
     double t = rounds * (per * t_stage + t_wg);
-    if (s > 1) t += 2.0 * s * (double)M * m.K * 4 / 7.0e6 + 4.0;
+    if (s > 1) t += 2.0 * s * (double)M * m.K * 4 / 4.0e6 + 5.0;
     if (s == 1) { t1 = t; best.t = t; }
     else if (t < best.t) { best.nsplit = s; best.t = t; }
   }
@@ -193,10 +195,14 @@ size_t gemm_big_workspace(const DMat& m, int M, bool least) { return gb_space(m,
 
 // What a call takes, for the choice between this kernel and the one in cbk_gemm_skinny.h: the plan's
 // time, 5 us for the preparation kernel and the launch, 3 more where a gate/up matrix needs the activation
-// kernel behind it (and that kernel's traffic).  Layouts without a decoder of their own are read at a
+// kernel behind it (and that kernel's traffic).  Partial tiles count at 6.5 TB/s here: 4 is what keeps the plan from
+// splitting where it does not pay, calls that are split measure faster (14336 x 4096 at 256 rows 61 us, 3840 x 7424 at
+// 1024 rows 89).  Layouts without a decoder of their own are read at a
 // tenth of the rate.
 double gemm_big_time(const DMat& m, int M, bool act) {
-  const double t = gb_plan(m, M).t * (gb_fast(m) ? 1.0 : 10.0) + 5.0;
+  const GbPlan p = gb_plan(m, M);
+  const double parts = p.nsplit > 1 ? 2.0 * p.nsplit * (double)M * m.K * 4 : 0.0;
+  const double t = (p.t - parts * (1 / 4.0e6 - 1 / 6.5e6)) * (gb_fast(m) ? 1.0 : 10.0) + 5.0;
   return act ? t + 3.0 + (double)M * m.K * (M <= 128 ? 9 : 5) / 5.0e6 : t;
 }
 

@@ -489,6 +489,17 @@ def test_gemv_five_to_eight_rows_equal_single_rows(case):
             assert torch.equal(ops.gemv(pm, x, bias=bias, out_dtype=torch.float32), y)
 
 
+@pytest.mark.parametrize("case", [(F.BLK1632_4, 4, 128, 16), (F.DENSE8, 8, 128, 0), (F.BLKC, 3, 64, 10)], ids=case_id)
+@pytest.mark.parametrize("K,N,M", [(512, 2048, 2000), (130, 1152, 1111), (1000, 512, 3001)])
+def test_gemm_of_many_token_tiles_and_few_row_tiles(case, K, N, M):
+    """Calls whose token tiles are walked in bands, the last one shorter: every tile exactly once."""
+    pm = F.synth_packed(K, N, case[0], case[1], case[2], case[3] or None, seed=K, device=DEV).to_tiled()
+    x = acts(M, N, torch.float16, seed=M).to(DEV)
+    ref = x.double() @ ops.dequant(pm, torch.float32).double().t()
+    y = ops.linear(pm, x, out_dtype=torch.float32).double()
+    assert float(((y - ref).norm(dim=1) / ref.norm(dim=1)).max()) < TOL
+
+
 DECODE_CASES = [(F.BLK1632_6, 6, 128, 16), (F.DENSEB, 8, 64, 0), (F.DENSE8, 8, 128, 0)] + [
     (F.BLKC if k else F.DENSEB, b, g, k) for b in (2, 3, 4) for k in (0, 10, 16, 23) for g in (64, 128)]
 
