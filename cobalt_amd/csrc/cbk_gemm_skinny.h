@@ -499,10 +499,17 @@ static int launch_skinny_ti(const SkArgs& a, int blocks, hipStream_t st) {
   hipLaunchKernelGGL(kern, dim3(blocks), dim3(512), SK_LDS, st, a);
   return hipGetLastError() == hipSuccess ? CBK_OK : CBK_ERR_HIP;
 }
+// Token tiles a code width has.  6-bit codes on tiles of 64 tokens gave sums that differed from run to run in the first
+// 32 of a wavefront's 64 weight rows (relative error 1e-2; 640 x 14336 at 333 rows).  The listing shows no fault, the
+// cause is not known: the instantiation is gone.  Tiles of 32 and 96 tokens are exact and repeat.
+constexpr bool sk_has_tile(int bits, int ti) { return !(bits == 6 && ti == 2); }
 template <int BITS, int KEEP, int GRP>
 static int launch_skinny_cfg(const SkArgs& a, int ti, int blocks, hipStream_t st) {
+  if constexpr (sk_has_tile(BITS, 2)) {
+    if (ti == 2) return launch_skinny_ti<BITS, KEEP, GRP, 2>(a, blocks, st);
+  }
   return ti == 1 ? launch_skinny_ti<BITS, KEEP, GRP, 1>(a, blocks, st)
-       : ti == 2 ? launch_skinny_ti<BITS, KEEP, GRP, 2>(a, blocks, st) : launch_skinny_ti<BITS, KEEP, GRP, 3>(a, blocks, st);
+       : ti == 3 ? launch_skinny_ti<BITS, KEEP, GRP, 3>(a, blocks, st) : CBK_ERR_UNSUPPORTED;
 }
 template <int BITS>
 static int launch_skinny_bits(const SkArgs& a, int keep, int group, int ti, int blocks, hipStream_t st) {

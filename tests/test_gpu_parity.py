@@ -489,6 +489,22 @@ def test_gemv_five_to_eight_rows_equal_single_rows(case):
             assert torch.equal(ops.gemv(pm, x, bias=bias, out_dtype=torch.float32), y)
 
 
+@pytest.mark.parametrize("case", FIXED_CASES, ids=case_id)
+def test_gemm_repeats_and_is_exact_to_its_operands(case):
+    """Every token tile and split of the two prefill kernels, several times over: the same bits each
+    time, and the error of operands of 11 bits."""
+    for (K, N) in ((640, 14336), (1024, 5376), (2048, 14336)):
+        pm = F.synth_packed(K, N, case[0], case[1], case[2], case[3] or None, seed=3, device=DEV).to_tiled()
+        W = ops.dequant(pm, torch.float32).double()
+        for M in (20, 64, 128, 200, 257, 333, 500, 700):
+            x = acts(M, N, torch.float16, seed=M).to(DEV)
+            y = ops.linear(pm, x, out_dtype=torch.float32)
+            ref = x.double() @ W.t()
+            assert float((y.double() - ref).norm() / ref.norm()) < 5e-4, (K, N, M)
+            for _ in range(4):
+                assert torch.equal(ops.linear(pm, x, out_dtype=torch.float32), y), (K, N, M)
+
+
 @pytest.mark.parametrize("case", [(F.BLK1632_4, 4, 128, 16), (F.DENSE8, 8, 128, 0), (F.BLKC, 3, 64, 10)], ids=case_id)
 @pytest.mark.parametrize("K,N,M", [(512, 2048, 2000), (130, 1152, 1111), (1000, 512, 3001)])
 def test_gemm_of_many_token_tiles_and_few_row_tiles(case, K, N, M):
