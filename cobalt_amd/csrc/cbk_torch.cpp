@@ -25,49 +25,49 @@ namespace {
 PyObject* g_error = nullptr;                                        // cobalt_amd._lib.CbkError
 
 // One packed matrix: the image and where its arrays are in it.  The addresses are formed per
-// call, so a tensor whose storage is exchanged (module.to()) is followed.
+// call, so a tensor whose storage is exchanged (module.to()) is followed, and so is a change inside
+// the two containers the Python object owns: the offsets and the row ranges are read from them
+// every time (seven lookups, 0.1 us).
 struct Matrix {
   PyObject_HEAD
   at::Tensor* blob;
+  PyObject* offs;                                                   // dict: byte offset of every array in the image
+  PyObject* splits;                                                 // sequence: cs_split0, cs_split1
   cbk_desc d;
-  int64_t off[5];                                                   // data, row_off, scale, zero, col_scale; -1: none
 };
 
+PyObject* g_key[5];                                                 // "data", "row_off", "scale", "zero", "col_scale"
+
 void matrix_dealloc(PyObject* o) {
-  delete ((Matrix*)o)->blob;
+  Matrix* m = (Matrix*)o;
+  delete m->blob;
+  Py_XDECREF(m->offs);
+  Py_XDECREF(m->splits);
   Py_TYPE(o)->tp_free(o);
 }
 
 PyObject* matrix_new(PyTypeObject* t, PyObject* args, PyObject*) {
-  PyObject *blob, *offs, *ints;
-  if (!PyArg_ParseTuple(args, "OO!O!", &blob, &PyTuple_Type, &offs, &PyTuple_Type, &ints)) return nullptr;
-  if (!THPVariable_Check(blob) || PyTuple_GET_SIZE(offs) != 5 || PyTuple_GET_SIZE(ints) != 10) {
-    PyErr_SetString(PyExc_TypeError, "Matrix(blob tensor, 5 offsets, 10 integers)");
+  PyObject *blob, *offs, *splits, *ints;
+  if (!PyArg_ParseTuple(args, "OO!OO!", &blob, &PyDict_Type, &offs, &splits, &PyTuple_Type, &ints)) return nullptr;
+  if (!THPVariable_Check(blob) || PyTuple_GET_SIZE(ints) != 8) {
+    PyErr_SetString(PyExc_TypeError, "Matrix(blob tensor, offsets, row ranges, 8 integers)");
     return nullptr;
   }
   Matrix* m = (Matrix*)t->tp_alloc(t, 0);
   if (!m) return nullptr;
   m->blob = new at::Tensor(THPVariable_Unpack(blob));
-  long long v[10];
-  for (int i = 0; i < 10; ++i) v[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(ints, i));
-  for (int i = 0; i < 5; ++i) m->off[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(offs, i));
+  Py_INCREF(offs); m->offs = offs;
+  Py_INCREF(splits); m->splits = splits;
+  long long v[8];
+  for (int i = 0; i < 8; ++i) v[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(ints, i));
   if (PyErr_Occurred()) { Py_DECREF(m); return nullptr; }
   m->d = cbk_desc{};
   m->d.K = (int32_t)v[0]; m->d.N = (int32_t)v[1]; m->d.layout = (int32_t)v[2]; m->d.bits = (int32_t)v[3];
-  m->d.group = (int32_t)v[4]; m->d.keep = (int32_t)v[5]; m->d.cs_rows = (int32_t)v[6];
-  m->d.cs_split0 = (int32_t)v[7]; m->d.cs_split1 = (int32_t)v[8]; m->d.flags = (int32_t)v[9];
+  m->d.group = (int32_t)v[4]; m->d.keep = (int32_t)v[5]; m->d.cs_rows = (int32_t)v[6]; m->d.flags = (int32_t)v[7];
   return (PyObject*)m;
 }
 
 PyTypeObject MatrixType = {PyVarObject_HEAD_INIT(nullptr, 0)};
-
-cbk_desc desc_of(const Matrix* m) {
-  cbk_desc d = m->d;
-  const uint8_t* base = (const uint8_t*)m->blob->const_data_ptr();
-  auto at_off = [&](int i) -> const void* { return m->off[i] < 0 ? nullptr : base + m->off[i]; };
-  d.data = at_off(0); d.row_off = at_off(1); d.scale = at_off(2); d.zero = at_off(3); d.col_scale = at_off(4);
-  return d;
-}
 
 struct GilRelease {
   PyThreadState* s = PyEval_SaveThread();
@@ -83,6 +83,35 @@ struct Fail {};                                                     // a Python 
 
 void check(int rc, const char* what) {
   if (rc) fail(g_error, std::string(what) + " failed: " + cbk_strerror(rc) + " (status " + std::to_string(rc) + ")");
+}
+
+// Holds the interpreter lock.
+cbk_desc desc_of(const Matrix* m) {
+  cbk_desc d = m->d;
+  const uint8_t* base = (const uint8_t*)m->blob->const_data_ptr();
+  const void* p[5];
+  for (int i = 0; i < 5; ++i) {
+    PyObject* o = i == 4 && !d.cs_rows ? nullptr : PyDict_GetItemWithError(m->offs, g_key[i]);
+    if (!o) {
+      if (PyErr_Occurred()) throw Fail{};
+      if (i != 1 && !(i == 4 && !d.cs_rows)) { PyErr_SetObject(PyExc_KeyError, g_key[i]); throw Fail{}; }
+      p[i] = nullptr;
+      continue;
+    }
+    const long long off = PyLong_AsLongLong(o);
+    if (off == -1 && PyErr_Occurred()) throw Fail{};
+    p[i] = base + off;
+  }
+  d.data = p[0]; d.row_off = p[1]; d.scale = p[2]; d.zero = p[3]; d.col_scale = p[4];
+  for (int i = 0; i < 2; ++i) {
+    PyObject* o = PySequence_GetItem(m->splits, i);
+    if (!o) throw Fail{};
+    const long long v = PyLong_AsLongLong(o);
+    Py_DECREF(o);
+    if (v == -1 && PyErr_Occurred()) throw Fail{};
+    (i ? d.cs_split1 : d.cs_split0) = (int32_t)v;
+  }
+  return d;
 }
 
 const Matrix* as_matrix(PyObject* o) {
@@ -405,6 +434,9 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods
 }  // namespace
 
 PyMODINIT_FUNC PyInit__native(void) {
+  const char* names[5] = {"data", "row_off", "scale", "zero", "col_scale"};
+  for (int i = 0; i < 5; ++i)
+    if (!(g_key[i] = PyUnicode_InternFromString(names[i]))) return nullptr;
   MatrixType.tp_name = "cobalt_amd._native.Matrix";
   MatrixType.tp_basicsize = sizeof(Matrix);
   MatrixType.tp_dealloc = matrix_dealloc;

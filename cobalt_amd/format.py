@@ -215,15 +215,14 @@ class PackedMatrix:
 
     def native(self):
         """The handle the extension module takes for this matrix, made at the first call after a
-        field was set."""
+        field was set.  It reads `offs` and `cs_splits` at every call, so a change inside them holds
+        at once."""
         h = self._handle
         if h is None:
             from . import _lib
-            o = self.offs
-            h = _lib.native().Matrix(self.blob, (o["data"], o.get("row_off", -1), o["scale"], o["zero"],
-                                                 o["col_scale"] if self.cs_rows else -1),
+            h = _lib.native().Matrix(self.blob, self.offs, self.cs_splits,
                                      (self.K, self.N, self.layout, self.bits, self.group, self.keep or 0, self.cs_rows,
-                                      self.cs_splits[0], self.cs_splits[1], self.flags))
+                                      self.flags))
             object.__setattr__(self, "_handle", h)
         return h
 

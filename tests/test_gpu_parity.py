@@ -53,6 +53,32 @@ def test_dequant_bit_exact(case, tiled):
         assert np.array_equal(_np(ops.dequant(pm, torch.float32, row0=8, nrows=16)), W[8:24])
 
 
+def test_native_handle_follows_changes_inside_the_description():
+    """The offsets and the row ranges of a matrix are containers a caller may change in place: the next
+    call uses what they hold then, as one with a fresh description does."""
+    pm = F.synth_packed(48, 256, F.BLK1632_4, 4, 128, 16, seed=5, device=DEV)
+    extra = pm.array("scale").flip(0).contiguous()
+    pm.blob = torch.cat([pm.blob, extra.view(torch.uint8), torch.zeros(256, dtype=torch.uint8, device=DEV)])
+    ops.dequant(pm)                                                   # the handle exists
+    x = acts(3, 256, torch.float16, seed=1).to(DEV)
+    before = ops.linear(pm, x)
+    at = pm.blob.numel() - 256 - extra.numel() * 2
+    pm.offs["scale"] = at
+    fresh = pm.to(DEV)
+    assert fresh.offs["scale"] == at
+    assert torch.equal(ops.dequant(pm), ops.dequant(fresh)) and torch.equal(ops.linear(pm, x), ops.linear(fresh, x))
+    assert not torch.equal(ops.linear(pm, x), before)
+    del pm.offs["zero"]
+    with pytest.raises(KeyError):
+        ops.linear(pm, x)
+    parts = [F.synth_packed(16 * k, 256, F.BLK1632_4, 4, 128, 16, seed=k, device=DEV) for k in (2, 1, 1)]
+    qkv = F.fuse_rows(parts)
+    qkv.cs_splits = list(qkv.cs_splits)
+    ops.dequant(qkv)
+    qkv.cs_splits[0], qkv.cs_splits[1] = 16, 32
+    assert torch.equal(ops.dequant(qkv), ops.dequant(qkv.to(DEV)))
+
+
 def test_dequant_fused_col_scale_rows_and_subnormal_scales():
     K, N = 48, 512
     raw = R.synth_raw_matrix(K, N, 0.5, 4, seed=3, block=32)
