@@ -1,8 +1,11 @@
 """Builds libcbk_hip.so (the C-ABI HIP library, hipcc for gfx950) and _native.so (its operators for
 Python) in-tree."""
 import os
+import re
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -14,6 +17,64 @@ SOURCES = ["cbk_api.hip", "cbk_dequant.hip", "cbk_gemv_generic.hip", "cbk_gemv.h
 FLAGS = ["-O3", "--offload-arch=gfx950", "-fPIC", "-shared", "-std=c++17",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-Wno-unused-command-line-argument", "-Wno-inline-asm"]
+
+
+def _llvm(tool):
+    return os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "lib", "llvm", "bin", tool)
+
+
+_KD = re.compile(r"\.(agpr_count|vgpr_count|name|symbol):\s+(\S+)")
+_SHIFT64 = re.compile(r"\b(v_(?:lshl|lshr|ashr)rev_[bi]64)\S*\s+v\[\d+:\d+\], v(\d+),")
+
+
+def shift_hazards(code_object):
+    """[(function, instruction, register)]: the 64-bit shifts of a gfx950 code object whose shift amount
+    is in the last vector register its wavefronts are given.
+
+    Measured on gfx950: such a shift can work with another amount (0 in every case seen), in some
+    wavefronts and not in others.  The 64-token tile of 6-bit codes had its amount in v223 of 224
+    registers and returned sums off by 1e-2 that changed from run to run; the same instructions with
+    232 registers given are exact.  The compiler knows the case for gfx90a, where it moves the
+    amount, but does not look for it on gfx950.  Registers are given in blocks of eight."""
+    notes = subprocess.run([_llvm("llvm-readelf"), "--notes", code_object], check=True, capture_output=True, text=True).stdout
+    arch, cur = {}, {}
+    for key, val in _KD.findall(notes):
+        if key == "agpr_count":
+            cur = {"agpr": int(val)}
+        elif key == "symbol":
+            cur["symbol"] = val[:-3] if val.endswith(".kd") else val
+        elif key == "vgpr_count" and "symbol" in cur:                  # (the keys of a kernel come in alphabetical order)
+            arch[cur["symbol"]] = int(val) - cur.get("agpr", 0)
+    out, fn = [], ""
+    dis = subprocess.Popen([_llvm("llvm-objdump"), "-d", "--no-show-raw-insn", code_object], stdout=subprocess.PIPE, text=True)
+    for line in dis.stdout:
+        if line.endswith(">:\n"):
+            fn = line[line.index("<") + 1:-3]
+            continue
+        m = _SHIFT64.search(line)
+        if not m:
+            continue
+        r = int(m.group(2))
+        if r % 8 != 7:
+            continue
+        # a function that is no kernel runs with the registers of any kernel that can hold it
+        n = arch.get(fn, min((v for v in arch.values() if v > r), default=0))
+        if r + 1 >= n or r == 255:
+            out.append((fn, m.group(1), r))
+    if dis.wait() != 0:
+        raise RuntimeError(f"llvm-objdump failed on {code_object}")
+    return out
+
+
+def shift_hazards_of(path):
+    """The same for every gfx950 code object inside an object file or library."""
+    with tempfile.TemporaryDirectory() as tmp:
+        link = os.path.join(tmp, "o")
+        os.symlink(os.path.abspath(path), link)
+        subprocess.run([_llvm("llvm-objdump"), "--offloading", link], check=True, capture_output=True)
+        objs = [os.path.join(tmp, f) for f in sorted(os.listdir(tmp)) if "gfx950" in f]
+        with ThreadPoolExecutor(8) as ex:
+            return [h for hs in ex.map(shift_hazards, objs) for h in hs]
 
 
 def build_lib(verbose=True, extra=()):
@@ -38,6 +99,11 @@ def build_lib(verbose=True, extra=()):
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
+    bad = shift_hazards_of(LIB)
+    if bad:
+        os.remove(LIB)
+        raise RuntimeError("64-bit shifts with their amount in the last register (see shift_hazards):\n" +
+                           "\n".join(f"  {op} amount v{r} in {fn}" for fn, op, r in bad))
     return LIB
 
 

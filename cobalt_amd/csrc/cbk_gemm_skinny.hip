@@ -183,7 +183,6 @@ static SkPlan sk_plan_ti(const DMat& m, int M, int ti, int max_split) {
 static SkPlan sk_plan(const DMat& m, int M, int max_split = 16) {
   SkPlan best = sk_plan_ti(m, M, 1, max_split);
   for (int ti = 2; ti <= 3; ++ti) {
-    if (!sk_has_tile(m.bits, ti)) continue;
     const SkPlan p = sk_plan_ti(m, M, ti, max_split);
     if (p.t < best.t) best = p;
   }
