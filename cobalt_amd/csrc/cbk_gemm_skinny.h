@@ -7,14 +7,17 @@
 //    to.  A wavefront owns 64 weight rows (two such operands) and up to 64 activation rows.  There is no
 //    weight tile in LDS and no barrier in the loop; two wavefronts per SIMD cover each other's waits.
 //  * Everything is a byte permute: codes to their columns, the zero point into the pruned columns (which
-//    so subtract to 0), bytes to halves (0x6400 | code is 1024 + code, exact).
+//    so subtract to 0), bytes to halves BASE + code (SkCfg::BASE), exact.
 //  * Tiles of up to 64 tokens multiply these halves as they are.  Once per quantisation group the float32
-//    sum is corrected by -(1024 + zero) * sum(X' of the group), one more matrix step whose A operand is
+//    sum is corrected by -(BASE + zero) * sum(X' of the group), one more matrix step whose A operand is
 //    that sum (as two halves), and multiplied by the group's scale on its way into the result: 37 vector
 //    instructions per step of 16 columns x 64 rows where a subtraction and a multiplication per weight
-//    need 52, and weights that are not rounded at all; the cancellation costs 2^-24 * 1024 /
-//    |code - zero|, below the 2^-12 of rounding (code - zero) * scale to a half.  Tiles of 96 tokens have
-//    no registers for a second set of sums; they subtract and multiply per weight.
+//    need 52, and weights that are not rounded at all.  BASE is as small as a byte allows, because the matrix pipe
+//    does not round its sums but cuts them off (measured), and what it cuts off a sum of BASE * X' of one sign adds
+//    up: all activations positive, 2-bit codes with 10 of 32 kept in groups of 128, error against float64 2.2e-4
+//    with BASE 1024, 0.7e-4 with 4; operands rounded to halves have 1.3e-4.  (Subnormal halves, code * 2^-24, need
+//    no BASE, but the pipe loses more of those: 1.8e-4 for rows of 14336 columns.)
+//    Tiles of 96 tokens have no registers for a second set of sums; they subtract and multiply per weight.
 //
 // k order.  A step is eight columns of the first half of a group (lanes 0-31) and eight of the second
 // (lanes 32-63): a lane walks half a group of its own row, nothing is loaded or ranked twice.  The
@@ -109,6 +112,9 @@ struct SkCfg {
   // (without spilling: read off the compiler's report)
   static constexpr bool DEFER = TI == 1 || (TI == 2 && 2 * NG * RG <= (DENSE ? 40 : GRP == 128 ? 32 : 24));
   static constexpr int NA = TI == 1 || (TI == 2 && !DEFER) ? 8 : 4; // activation fragments in flight (steps)
+  // A code c becomes the half BASE + c, exactly, from one byte: the low byte of 0x6400 + c (8- and 6-bit codes), of
+  // 0x5400 + (c << 4) (nibbles, kept in the high half of their byte), or the high byte of 0x4400 + (c << 8) (2-bit)
+  static constexpr int BASE = B8 || HI2 ? 1024 : BITS == 2 ? 4 : 64;
   // order of the columns of an octet in a fragment: the order the codes come out of the stream
   static constexpr int ORDER = !DENSE || B8 ? 0 : BITS == 2 ? 2 : 1;
 };
@@ -158,7 +164,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if (tid < 256) {
         const uint2 e = make_selectors((uint32_t)tid, BITS == 2 ? 1 : 0);
         // 6-bit: all ones in the pruned bytes; else the field of a code in the kept ones
-        constexpr uint32_t F = C::HI2 ? 0xFFu : C::SB == 4 ? 0x0Fu : 0x03u;
+        constexpr uint32_t F = C::HI2 ? 0xFFu : C::SB == 4 ? 0xF0u : 0x03u;
         const uint32_t k0 = bits_to_bytes((uint32_t)tid) * F, k1 = bits_to_bytes((uint32_t)tid >> 4) * F;
 #pragma unroll
         for (int j = 0; j < SK_LUT_LANES; ++j) lut[tid * SK_LUT_LANES + j] = make_uint4(e.x, e.y, C::HI2 ? ~k0 : k0, C::HI2 ? ~k1 : k1);
@@ -260,7 +266,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       constexpr int T0 = decltype(t0_tag)::value;
       constexpr bool more = decltype(more_tag)::value;
       uint32_t cw[2][C::ND], st[2][C::NW], z4[2];
-      h2_t off[2], sh[2];                                           // !DEFER: -(1024 + zero) and scale
+      h2_t off[2], sh[2];                                           // -(BASE + zero), and the scale for !DEFER
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         if constexpr (C::WHOLE) {
@@ -269,8 +275,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         } else {
           skew_dwords<C::NL, C::ND, C::HB % 32 == 0>(w[j].raw, ((2u * (uint32_t)g + (uint32_t)half) * (uint32_t)C::HB) & 127u, cw[j]);
         }
-        z4[j] = perm(0, w[j].z, 0);                                 // the zero point in every byte
-        const _Float16 n = (_Float16)(-1024.0f - (float)w[j].z), f = __builtin_bit_cast(_Float16, (uint16_t)w[j].s);
+        // the zero point in every byte, where a code has its bits
+        z4[j] = perm(0, C::BASE == 64 ? w[j].z << 4 : C::BASE == 4 ? w[j].z | 0x44u : w[j].z, 0);
+        const _Float16 n = (_Float16)(-(float)C::BASE - (float)w[j].z), f = __builtin_bit_cast(_Float16, (uint16_t)w[j].s);
         off[j] = h2_t{n, n}; sh[j] = h2_t{f, f};
       }
       uint4 sel[2][2];
@@ -286,12 +293,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const int blk = o >> 2, jj = o & 3;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          const uint32_t k64 = 0x64646464u;
+          const uint32_t kb = C::BASE == 1024 ? 0x64646464u : 0x54545454u;
+          // four bytes -> four halves
+          auto widen = [&](uint32_t b, uint32_t& lo, uint32_t& hi) {
+            if constexpr (C::BASE == 4) { lo = perm(0, b, 0x010C000Cu); hi = perm(0, b, 0x030C020Cu); }
+            else { lo = perm(kb, b, 0x04010400u); hi = perm(kb, b, 0x04030402u); }
+          };
           uint32_t h[4];
           if constexpr (C::B8) {
             const uint32_t b0 = cw[j][2 * o], b1 = cw[j][2 * o + 1];
-            h[0] = perm(k64, b0, 0x04010400u); h[1] = perm(k64, b0, 0x04030402u);
-            h[2] = perm(k64, b1, 0x04010400u); h[3] = perm(k64, b1, 0x04030402u);
+            widen(b0, h[0], h[1]); widen(b1, h[2], h[3]);
           } else {
             if (jj == 0) {
 #pragma unroll
@@ -302,8 +313,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                                   : C::SB == 4 ? st[j][jj] : (st[j][jj >> 1] >> (16 * (jj & 1)));
             if (C::SB == 2) { win &= 0xFFFFu; win |= win << 14; }   // bytes c0 c4 c1 c5; four bits up c2 c6 c3 c7
             if (BITMAP) {
-              // even and odd codes in the low bits of their bytes, the neighbour's bits above them
-              uint32_t q0 = win, q1 = win >> 4, b0, b1;
+              // even and odd codes in the bits they have in a byte, the neighbour's bits beside them
+              uint32_t q0 = C::BASE == 64 ? win << 4 : win, q1 = C::BASE == 64 ? win : win >> 4, b0, b1;
               if (C::HI2) {
                 uint32_t h0, h1;
                 hi2_pools(w[j].h2[C::HI2 ? blk : 0], jj == 0 ? 0u : rank(w[j].m[BITMAP ? blk : 0], jj), h0, h1);
@@ -313,13 +324,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 b0 = mask_select(e[j].z, z4[j], perm(q1, q0, e[j].x));   // in a kept column: it is a code itself)
                 b1 = mask_select(e[j].w, z4[j], perm(q1, q0, e[j].y));
               }
-              h[0] = perm(k64, b0, 0x04010400u); h[1] = perm(k64, b0, 0x04030402u);
-              h[2] = perm(k64, b1, 0x04010400u); h[3] = perm(k64, b1, 0x04030402u);
+              widen(b0, h[0], h[1]); widen(b1, h[2], h[3]);
             } else {                                                // columns in stream order (SkCfg::ORDER)
-              constexpr uint32_t F = C::SB == 4 ? 0x0F0F0F0Fu : 0x03030303u;
-              const uint32_t q0 = win & F, q1 = (win >> 4) & F;
-              h[0] = perm(k64, q0, 0x04010400u); h[1] = perm(k64, q0, 0x04030402u);
-              h[2] = perm(k64, q1, 0x04010400u); h[3] = perm(k64, q1, 0x04030402u);
+              const uint32_t q0 = C::BASE == 64 ? (win << 4) & 0xF0F0F0F0u : (win & 0x03030303u) | 0x44444444u;
+              const uint32_t q1 = C::BASE == 64 ? win & 0xF0F0F0F0u : ((win >> 4) & 0x03030303u) | 0x44444444u;
+              widen(q0, h[0], h[1]); widen(q1, h[2], h[3]);
             }
           }
           if (!DEFER) {
@@ -334,7 +343,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       v8h bf[2][2];
       fetch(0, sel[0]);
       if (ST > 1) fetch(1, sel[1]);
-      // -(1024 + zero) against the sum of this lane's half of the group (as two halfs)
+      // -(BASE + zero) against the sum of this lane's half of the group (as two halfs)
       v16f part[DEFER ? TI : 1][2];
       if constexpr (DEFER) {
         v8h bz[2];

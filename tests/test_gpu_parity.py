@@ -564,6 +564,29 @@ def test_gemv_rows_do_not_depend_on_their_number(case):
                 assert torch.equal(ops.gemv(pm, x, out_dtype=torch.float32, workspace=small), one), (K, N, M, pm is rows)
 
 
+@pytest.mark.parametrize("case", DECODE_CASES, ids=case_id)
+def test_gemm_loses_no_more_than_operands_of_11_bits(case):
+    """The error of the matrix-core GEMM against float64, for activations of both signs and of one, is no
+    larger than that of the product of X' = half(x * col_scale) and half((q - zero) * scale) in exact
+    sums: float32 sums add nothing that shows (2 % are left for them and for the draw).  Sums that carry
+    a large offset of the codes along fail this for activations of one sign."""
+    for K, N in ((200, 4096), (130, 14336)):
+        pm = F.synth_packed(K, N, case[0], case[1], case[2], case[3] or None, seed=N, device=DEV).to_tiled()
+        W = ops.dequant(pm, torch.float32).double()
+        Wh = ops.dequant(pm, torch.float32, with_col_scale=False).half().double()
+        cs = pm.array("col_scale").float()
+        for M in (9, 30, 64, 100):
+            for one_sign in (False, True):
+                x = acts(M, N, torch.float16, seed=M).to(DEV)
+                x = x.abs() if one_sign else x
+                ref = x.double() @ W.t()
+                err = lambda y: float((y - ref).norm() / ref.norm())
+                bound = err((x.float() * cs).half().double() @ Wh.t())
+                got = err(ops.gemm(pm, x, out_dtype=torch.float32).double())
+                assert got <= 1.02 * bound, (K, N, M, one_sign, got, bound)
+
+
+
 @pytest.mark.parametrize("case", [(F.BLK1632_4, 4, 128, 16), (F.DENSE4, 4, 128, 0), (F.BLKC, 3, 128, 10)], ids=case_id)
 def test_gemv_rows_longer_than_the_staging_area(case):
     """Rows whose activation digits do not fit in LDS are staged and multiplied in column slabs, the
