@@ -49,6 +49,9 @@ constexpr size_t SK_LDS = (size_t)SK_WC * SK_WR * 32 * SK_PITCH * 4 + SK_LUT;
 
 typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
 
+// The scale of a token and column part with an infinite activation: above every scale of a finite one (2^120)
+constexpr float SK_INFINITE = 2658455991569831745807614120560689152.f;   // 2^121
+
 struct SkArgs {
   DMat m;
   const uint16_t* xp;      // fragments of X' [vector][token tile][group][steps][TI][64][8]
@@ -254,6 +257,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int i = 0; i < TI; ++i)
         if (DEFER) xs[i] = p[(uint32_t)(lane & 31) + (uint32_t)half * (TI * 32u) + i * 32u];
     };
+    // Does this part of a token of the tile hold an infinity (see SK_INFINITE)?
+    const int rtok = tt * (32 * TI) + (TI == 1 ? lane & 31 : lane);
+    float rs = 0.f;
+    if (DEFER) rs = a.row_scale[(size_t)xv * a.rvs + (size_t)q * a.rss + rtok];
     Grp ring[NG][2];
     load_sums(0);
 #pragma unroll
@@ -261,10 +268,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int t = 0; t < NA - 1; ++t) load_a(t, t);
 
-    // T0: position of the group's first step in the ring of activation fragments
-    auto group = [&](int g, Grp (&w)[2], auto t0_tag, auto more_tag) {
+    // T0: position of the group's first step in the ring of activation fragments.  SUB: the zero point is taken off
+    // every weight instead of off the sum.
+    auto group = [&](int g, Grp (&w)[2], auto t0_tag, auto more_tag, auto sub_tag) {
       constexpr int T0 = decltype(t0_tag)::value;
-      constexpr bool more = decltype(more_tag)::value;
+      constexpr bool more = decltype(more_tag)::value, SUB = decltype(sub_tag)::value;
       uint32_t cw[2][C::ND], st[2][C::NW], z4[2];
       h2_t off[2], sh[2];                                           // -(BASE + zero), and the scale for !DEFER
 #pragma unroll
@@ -331,10 +339,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
               widen(q0, h[0], h[1]); widen(q1, h[2], h[3]);
             }
           }
-          if (!DEFER) {
+          if constexpr (!DEFER || SUB) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-              h[i] = __builtin_bit_cast(uint32_t, (h2_t)((__builtin_bit_cast(h2_t, h[i]) + off[j]) * sh[j]));
+            for (int i = 0; i < 4; ++i) {
+              h2_t v = __builtin_bit_cast(h2_t, h[i]) + off[j];
+              if constexpr (!DEFER) v = v * sh[j];
+              h[i] = __builtin_bit_cast(uint32_t, v);
+            }
           }
           const uint4 hv = make_uint4(h[0], h[1], h[2], h[3]);
           bf[j] = __builtin_bit_cast(v8h, hv);
@@ -360,10 +371,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             v16f zero16;
 #pragma unroll
             for (int e = 0; e < 16; ++e) zero16[e] = 0.f;
-            part[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(az, bz[j], zero16, 0, 0, 0);
+            if constexpr (SUB) part[i][j] = zero16;
+            else part[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(az, bz[j], zero16, 0, 0, 0);
           }
         }
-        load_sums(g - g0 + 1);
+        if constexpr (!SUB) load_sums(g - g0 + 1);
       }
       decode(0, sel[0], bf[0]);
       __builtin_amdgcn_sched_barrier(0);
@@ -409,24 +421,37 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     static_assert(UG % NG == 0 && UG * ST % NA == 0, "both rings turn a whole number of times per trip");
     using Yes = std::true_type; using No = std::false_type;
     int g = g0;
-    for (; g + UG <= g1; g += UG) {
-      group(g, ring[0], std::integral_constant<int, 0>{}, Yes{});
-      group(g + 1, ring[1 % NG], std::integral_constant<int, ST % NA>{}, Yes{});
-      if constexpr (UG > 2) group(g + 2, ring[2 % NG], std::integral_constant<int, 2 * ST % NA>{}, Yes{});
-      if constexpr (UG > 3) {
-        group(g + 3, ring[3 % NG], std::integral_constant<int, 3 * ST % NA>{}, Yes{});
-        group(g + 4, ring[4 % NG], std::integral_constant<int, 4 * ST % NA>{}, Yes{});
-        group(g + 5, ring[5 % NG], std::integral_constant<int, 5 * ST % NA>{}, Yes{});
+    if constexpr (DEFER) {
+      // An infinity: its code times X' and the sum of the group are infinite too, and their difference is NaN where the
+      // weight times it is not.  Such a wavefront takes its groups one at a time with the zero point off every weight.
+      if (__builtin_expect(__ballot(rs == SK_INFINITE && rtok < a.M) != 0, 0)) {
+        for (int h = g0; h < g1; ++h) {
+          load_group(h, ring[0]);
+#pragma unroll
+          for (int t = 0; t < NA - 1; ++t) load_a((h - g0) * ST + t, t);
+          group(h, ring[0], std::integral_constant<int, 0>{}, No{}, Yes{});
+        }
+        g = g1;
       }
     }
-    if (g < g1) group(g, ring[0], std::integral_constant<int, 0>{}, Yes{});
+    for (; g + UG <= g1; g += UG) {
+      group(g, ring[0], std::integral_constant<int, 0>{}, Yes{}, No{});
+      group(g + 1, ring[1 % NG], std::integral_constant<int, ST % NA>{}, Yes{}, No{});
+      if constexpr (UG > 2) group(g + 2, ring[2 % NG], std::integral_constant<int, 2 * ST % NA>{}, Yes{}, No{});
+      if constexpr (UG > 3) {
+        group(g + 3, ring[3 % NG], std::integral_constant<int, 3 * ST % NA>{}, Yes{}, No{});
+        group(g + 4, ring[4 % NG], std::integral_constant<int, 4 * ST % NA>{}, Yes{}, No{});
+        group(g + 5, ring[5 % NG], std::integral_constant<int, 5 * ST % NA>{}, Yes{}, No{});
+      }
+    }
+    if (g < g1) group(g, ring[0], std::integral_constant<int, 0>{}, Yes{}, No{});
     if constexpr (UG > 2) {
-      if (g + 1 < g1) group(g + 1, ring[1 % NG], std::integral_constant<int, ST % NA>{}, Yes{});
+      if (g + 1 < g1) group(g + 1, ring[1 % NG], std::integral_constant<int, ST % NA>{}, Yes{}, No{});
     }
     if constexpr (UG > 3) {
-      if (g + 2 < g1) group(g + 2, ring[2 % NG], std::integral_constant<int, 2 * ST % NA>{}, Yes{});
-      if (g + 3 < g1) group(g + 3, ring[3 % NG], std::integral_constant<int, 3 * ST % NA>{}, Yes{});
-      if (g + 4 < g1) group(g + 4, ring[4 % NG], std::integral_constant<int, 4 * ST % NA>{}, No{});
+      if (g + 2 < g1) group(g + 2, ring[2 % NG], std::integral_constant<int, 2 * ST % NA>{}, Yes{}, No{});
+      if (g + 3 < g1) group(g + 3, ring[3 % NG], std::integral_constant<int, 3 * ST % NA>{}, Yes{}, No{});
+      if (g + 4 < g1) group(g + 4, ring[4 % NG], std::integral_constant<int, 4 * ST % NA>{}, No{}, No{});
     }
   }
 

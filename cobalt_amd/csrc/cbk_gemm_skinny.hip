@@ -18,7 +18,8 @@ int launch_skinny_b68(const SkArgs&, int bits, int group, int ti, int blocks, hi
 // and the write; 0 = any length, read twice.  (A scale per token over the whole row, found by one workgroup per
 // four tokens or by every workgroup again, and half lines: 48 rows of 14336 columns 9 us, 512 rows 31.)
 __device__ inline float skinny_scale(float mx) {                   // the power of two that brings mx into [128, 256)
-  if (!(mx > 0.f) || !(mx <= 3.4028234663852886e38f)) return 1.f;
+  if (!(mx > 0.f)) return 1.f;
+  if (!(mx <= 3.4028234663852886e38f)) return SK_INFINITE;          // (mx is no NaN: fmaxf passes those over)
   int e = (int)((__float_as_uint(mx) >> 23) & 0xffu) - 7;          // its biased exponent
   e = e < 1 ? 1 : e;
   return __uint_as_float((uint32_t)e << 23);

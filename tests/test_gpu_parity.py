@@ -964,6 +964,37 @@ def test_gemm_token_tiles_of_32_64_and_96(case):
             assert err < TOL, f"{case_id(case)} {K}x{N} M={M}: {err}"
 
 
+@pytest.mark.parametrize("case", [(F.BLK1632_4, 4, 128, 16), (F.BLKC, 2, 64, 16), (F.BLKC, 3, 128, 23), (F.BLKC, 2, 128, 10),
+                                  (F.BLK1632_6, 6, 128, 16), (F.DENSE4, 4, 128, 0), (F.DENSE8, 8, 128, 0), (F.DENSEB, 2, 64, 0)],
+                         ids=case_id)
+def test_gemm_of_infinite_activations(case):
+    """A token with infinities gets what sums in IEEE arithmetic give: +-inf, NaN where an infinity meets a
+    weight that is 0 or two of them cancel; NaN stays NaN, the other tokens are untouched.  The same
+    however many tokens the call has, so on every token tile of both kernels; several parts of the columns,
+    values beyond what a half holds beside the infinity, plain and gate/up matrices."""
+    K, N = 192, 4096
+    one = F.synth_packed(K, N, case[0], case[1], case[2], case[3] or None, seed=7, device=DEV)
+    two = F.fuse_rows([one, F.synth_packed(K, N, case[0], case[1], case[2], case[3] or None, seed=8, device=DEV)], interleave=True)
+    for pm in (one.to_tiled(), two.to_tiled()):
+        W = ops.dequant(pm, torch.float32).cpu().double()
+        for M in (9, 30, 60, 90, 130, 400, 1500):
+            x = acts(M, N, torch.bfloat16, seed=M).float()
+            x[1, 7] = float("inf")
+            x[2, 900] = float("nan")
+            x[3, 4090] = float("-inf")
+            x[3, 4000:4090] = 3e5
+            x[5, 130] = x[5, 2000] = float("inf")
+            x[6, 130], x[6, 131] = float("inf"), float("-inf")
+            x[M - 1, N - 1] = float("inf")
+            x = x.to(torch.bfloat16)
+            y = ops.gemm(pm, x.to(DEV), out_dtype=torch.float32).cpu()
+            ref = x.double() @ W.t()
+            assert torch.equal(torch.isnan(y), torch.isnan(ref)), M
+            assert torch.equal(torch.isinf(y), torch.isinf(ref)) and torch.equal(y[torch.isinf(y)] > 0, ref[torch.isinf(ref)] > 0), M
+            ok = torch.isfinite(ref).all(1)
+            assert int((~ok).sum()) == 6 and float((y[ok].double() - ref[ok]).norm() / ref[ok].norm()) < TOL
+
+
 def test_gemm_bias_dtype_and_prune_zero():
     case = (F.BLK1632_4, 4, 128, 16)
     K, N, M = 256, 2048, 300
