@@ -4,6 +4,7 @@
 #include <mutex>
 #include "cbk_internal.h"
 #include "cbk_device.h"
+#include "cbk_gemm_plan.h"
 
 namespace cbk {
 int launch_dequant(const DMat&, int, int, int, void*, int, int64_t, hipStream_t);
@@ -21,25 +22,10 @@ int launch_act_mul(const void* t, int tdt, int64_t ldt, void* y, int ydt, int64_
                    const void* bias, hipStream_t st, bool halves = false);
 int launch_gemm(const DMat&, const void*, int, int, int64_t, void*, int, int64_t, const void*,
                 hipStream_t);
-int launch_gemm_big(const DMat&, const void*, int, int, int64_t, void*, int, int64_t, const void*, void*, size_t,
-                    hipStream_t, bool halves = false);
-size_t gemm_big_workspace(const DMat&, int M, bool least);
-double gemm_big_time(const DMat&, int M, bool act);
-bool gemm_skinny_takes(const DMat&);
-double gemm_skinny_time(const DMat&, int M);
-size_t gemm_skinny_workspace(const DMat&, int M, bool least);
-int launch_gemm_skinny(const DMat&, const void*, int, int, int64_t, void*, int, int64_t, const void*, int act, void*, size_t,
-                       hipStream_t);
 int launch_pack(const DMat&, const void* mask, const void* q, const void* scale, const void* zero, int zero_f16,
                 int fix_zero, int* status, const PackExtra* extra, hipStream_t);
 int launch_repack_dense4(const DMat& sparse, const DMat& dense4, hipStream_t);
 int launch_unpack(const DMat&, void* q, void* mask, hipStream_t);
-// The 256 x 256 tile kernel takes every call of the fixed-stride layouts but q|k|v matrices whose
-// ranges do not start on its row tiles.
-static inline bool gemm_big_takes(const DMat& m, int M) {
-  if (M < 1 || family_of(m.layout) == FAM_SPARSE) return false;
-  return m.cs_rows <= 2 || (m.cs_split0 % 256 == 0 && (m.cs_split0 + m.cs_split1) % 256 == 0);
-}
 
 // Two kernels for the fixed-stride layouts: the one that decodes into the registers that multiply
 // (cbk_gemm_skinny.h: few tokens, small matrices) and the 256 x 256 tile (many tokens, whose weight
@@ -47,26 +33,20 @@ static inline bool gemm_big_takes(const DMat& m, int M) {
 // 100 and 600 activation rows, depending on how the matrix fills the chip, later for small matrices.  Above 512 rows
 // the first has to be a tenth cheaper, which is what the two models are off by there (3840 x 7424 at 1024 rows: 94 us
 // expected and 98 measured, the tile kernel 94 and 89).
-static inline bool skinny_is_faster(const DMat& m, int M, bool act) {
-  return gemm_skinny_takes(m) &&
-         (!gemm_big_takes(m, M) || gemm_skinny_time(m, M) * (M > 512 ? 1.1 : 1.0) < gemm_big_time(m, M, act));
+// act: the call is act(gate) * up, which the first kernel does as it sums the column parts and the tile kernel leaves
+// to the activation kernel: 3 us and that kernel's traffic.
+// GEMM_NONE: a q|k|v matrix whose ranges neither kernel's row tiles fit, or no plan within `room`.
+static GemmPlan gemm_plan(const DMat& m, int M, bool act, size_t room) {
+  const GemmPlan sk = plan_skinny(m, M, room), big = plan_big(m, M, room);
+  if (!sk.kernel || !big.kernel) return sk.kernel ? sk : big;
+  const double t_act = act ? 3.0 + (double)M * m.K * (M <= 128 ? 9 : 5) / 5.0e6 : 0.0;
+  return sk.t * (M > 512 ? 1.1 : 1.0) < big.t + t_act ? sk : big;
 }
-// Workspace of run_gemm.  least: what it cannot do without, else what it makes use of.
-static size_t gemm_workspace(const DMat& m, int M, bool least) {
-  if (M < 1) return 0;
-  const size_t big = gemm_big_takes(m, M) ? gemm_big_workspace(m, M, least) : 0;
-  if (!skinny_is_faster(m, M, false)) return big;
-  const size_t sk = gemm_skinny_workspace(m, M, least);
-  return least && big && big < sk ? big : sk;
+static int run_gemm(const DMat& m, const GemmPlan& p, const void* x, int xdt, int M, int64_t ldx, void* y, int ydt, int64_t ldy,
+                    const void* bias, void* ws, size_t ws_bytes, hipStream_t st) {
+  return p.kernel == GEMM_ROWS ? launch_gemm_skinny(m, p, x, xdt, M, ldx, y, ydt, ldy, bias, -1, ws, ws_bytes, st)
+                               : launch_gemm_big(m, p, x, xdt, M, ldx, y, ydt, ldy, bias, ws, ws_bytes, st);
 }
-static int run_gemm(const DMat& m, const void* x, int xdt, int M, int64_t ldx, void* y, int ydt, int64_t ldy, const void* bias,
-                    void* ws, size_t ws_bytes, hipStream_t st) {
-  if (skinny_is_faster(m, M, false) && (!gemm_big_takes(m, M) || ws_bytes >= gemm_skinny_workspace(m, M, true)))
-    return launch_gemm_skinny(m, x, xdt, M, ldx, y, ydt, ldy, bias, -1, ws, ws_bytes, st);
-  return launch_gemm_big(m, x, xdt, M, ldx, y, ydt, ldy, bias, ws, ws_bytes, st);
-}
-// the matrices run_gemm takes whole
-static inline bool gemm_takes(const DMat& m, int M) { return M >= 1 && (gemm_big_takes(m, M) || gemm_skinny_takes(m)); }
 
 static inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
@@ -232,6 +212,51 @@ static DMat dense4_view(const DMat& m, uint8_t* ws, const Transient& t) {
   return d;
 }
 
+// The workspace a plan may take.  cbk_gemm_static has CBK_STATIC_SCRATCH_BYTES and gives cbk_gemm's results,
+// so the calls it takes run on a plan that fits there under either name: those the tile kernel has room for with
+// its own split of the columns (a q|k|v matrix in one piece; survivor streams with their codes and bitmap beside the
+// dense image).  Every other call may take what the fastest plan takes, and cbk_gemm_static refuses it.
+static size_t gemm_room(const DMat& m, int M) {
+  size_t need = 0, fixed = 0, reserved = 0;
+  if (family_of(m.layout) == FAM_SPARSE) {
+    if (M <= 16 || !sparse_repackable(m)) return (size_t)CBK_STATIC_SCRATCH_BYTES;   // the row kernel, no workspace
+    const Transient t = transient_dense4(m);
+    fixed = t.end;
+    reserved = align_up((size_t)m.K * m.N, 256) + align_up((size_t)m.K * (m.N / 8), 256);
+    need = big_unsplit_space(dense4_view(m, nullptr, t), M);
+  } else {
+    int lo[3], hi[3], row[3];
+    const int nr = fused_ranges(m, lo, hi, row);
+    if (m.cs_rows != 3 || plan_big(m, M, ANY_ROOM).kernel) need = big_unsplit_space(m, M);
+    else
+      for (int i = 0; i < nr; ++i) {
+        const size_t b = big_unsplit_space(row_range(m, lo[i], hi[i], row[i]), M);
+        need = need > b ? need : b;
+      }
+  }
+  return reserved + fixed + need <= (size_t)CBK_STATIC_SCRATCH_BYTES ? (size_t)CBK_STATIC_SCRATCH_BYTES - fixed : ANY_ROOM;
+}
+// What cbk_gemm needs of a workspace.
+static size_t gemm_workspace(const DMat& m, int M) {
+  if (M < 1) return 0;
+  const size_t room = gemm_room(m, M);
+  if (family_of(m.layout) == FAM_SPARSE) {
+    if (M <= 16 || !sparse_repackable(m)) return 0;
+    const Transient t = transient_dense4(m);
+    return t.end + gemm_plan(dense4_view(m, nullptr, t), M, false, room).bytes;
+  }
+  const GemmPlan p = gemm_plan(m, M, false, room);
+  if (p.kernel) return p.bytes;
+  int lo[3], hi[3], row[3];
+  const int nr = fused_ranges(m, lo, hi, row);
+  size_t need = 0;
+  for (int i = 0; i < nr; ++i) {                                    // run one after the other on the same bytes
+    const size_t b = gemm_plan(row_range(m, lo[i], hi[i], row[i]), M, false, room).bytes;
+    need = need > b ? need : b;
+  }
+  return need;
+}
+
 // Room for the part sums of cbk_gemv at M rows (see cbk_workspace_bytes); no other use of a
 // workspace in decode.  A q|k|v matrix runs as its ranges, one launch for all of them.
 static size_t decode_workspace(const DMat& m, int M) {
@@ -308,31 +333,15 @@ size_t cbk_stream_bytes(const cbk_desc* in, size_t sparse_data_bytes) {
   return (size_t)d.K * stride_of(d) + meta;
 }
 
-static size_t workspace_of(const DMat& m, int M, bool least) {
-  if (family_of(m.layout) == FAM_SPARSE) {                          // cbk_gemm / cbk_linear above 16 rows: see Transient
-    if (M <= 16) return least ? 0 : decode_workspace(m, M);         // part sums of long rows split by columns, else none
-    if (!sparse_repackable(m)) return 0;
-    const Transient t = transient_dense4(m);
-    return t.end + gemm_workspace(dense4_view(m, nullptr, t), M, least);
-  }
-  // the most any of the three entry points asks for (cbk_gemm runs the prefill kernel at any M)
-  size_t need = least ? 0 : decode_workspace(m, M);
-  if (gemm_takes(m, M)) {
-    const size_t b = gemm_workspace(m, M, least);
-    return need > b ? need : b;
-  }
-  int lo[3], hi[3], row[3];
-  const int nr = M >= 1 ? fused_ranges(m, lo, hi, row) : 0;
-  for (int i = 0; i < nr; ++i) {                                    // run one after the other on the same bytes
-    const size_t b = gemm_workspace(row_range(m, lo[i], hi[i], row[i]), M, least);
-    need = need > b ? need : b;
-  }
-  return need;
+// the most any of the three entry points asks for (cbk_gemm runs the prefill kernels at any M)
+static size_t workspace_of(const DMat& m, int M) {
+  const size_t a = decode_workspace(m, M), b = gemm_workspace(m, M);
+  return a > b ? a : b;
 }
 
 size_t cbk_workspace_bytes(const cbk_desc* in, int M) {
   DMat m;
-  return to_dmat(in, &m, false) ? 0 : workspace_of(m, M, false);
+  return to_dmat(in, &m, false) ? 0 : workspace_of(m, M);
 }
 
 size_t cbk_gemv_batch_workspace_bytes(int n, const cbk_desc* descs, int M) {
@@ -455,8 +464,7 @@ int cbk_gemm(const cbk_desc* in, const void* x, int x_dtype, int M, int64_t ldx,
     if (M <= 16)                                                    // not worth re-packing: the row kernel
       return cbk_gemv(in, x, x_dtype, M, ldx, y, y_dtype, ldy, bias, workspace, workspace_bytes, stream);
     const Transient t = transient_dense4(m);
-    const bool room = workspace && !((uintptr_t)workspace & 255) &&
-                      workspace_bytes >= t.end + gemm_workspace(dense4_view(m, nullptr, t), M, true);
+    const bool room = workspace && !((uintptr_t)workspace & 255) && workspace_bytes >= gemm_workspace(m, M);
     if (!sparse_repackable(m) || !room) {
       // zero points that are no 4-bit codes, row-fused column scales, or no room for the dense
       // image: the row kernel, sixteen activation rows per pass, without a workspace
@@ -473,19 +481,23 @@ int cbk_gemm(const cbk_desc* in, const void* x, int x_dtype, int M, int64_t ldx,
     const DMat d = dense4_view(m, ws, t);
     rc = launch_repack_dense4(m, d, (hipStream_t)stream);
     if (rc) return rc;
-    return run_gemm(d, x, x_dtype, M, ldx, y, y_dtype, ldy, bias, ws + t.end, workspace_bytes - t.end, (hipStream_t)stream);
+    return run_gemm(d, gemm_plan(d, M, false, gemm_room(m, M)), x, x_dtype, M, ldx, y, y_dtype, ldy, bias, ws + t.end,
+                    workspace_bytes - t.end, (hipStream_t)stream);
   }
-  if (gemm_takes(m, M))
-    return run_gemm(m, x, x_dtype, M, ldx, y, y_dtype, ldy, bias, workspace, workspace_bytes, (hipStream_t)stream);
+  const size_t room = gemm_room(m, M);
+  const GemmPlan plan = gemm_plan(m, M, false, room);
+  if (plan.kernel)
+    return run_gemm(m, plan, x, x_dtype, M, ldx, y, y_dtype, ldy, bias, workspace, workspace_bytes, (hipStream_t)stream);
   int lo[3], hi[3], row[3];
   const int nr = fused_ranges(m, lo, hi, row);
   if (nr) {
     // q|k|v: each range is a matrix with one col_scale vector; the launches share the
     // workspace (pre-scaled activations), which the stream order keeps apart
+    if (!workspace || workspace_bytes < gemm_workspace(m, M)) return CBK_ERR_WORKSPACE;   // before the first of them
     const size_t ysz = y_dtype == CBK_F32 ? 4 : 2;
     for (int i = 0; i < nr; ++i) {
       const DMat s = row_range(m, lo[i], hi[i], row[i]);
-      rc = run_gemm(s, x, x_dtype, M, ldx, (uint8_t*)y + (size_t)lo[i] * ysz, y_dtype, ldy,
+      rc = run_gemm(s, gemm_plan(s, M, false, room), x, x_dtype, M, ldx, (uint8_t*)y + (size_t)lo[i] * ysz, y_dtype, ldy,
                     bias ? (const uint8_t*)bias + (size_t)lo[i] * ysz : nullptr, workspace, workspace_bytes, (hipStream_t)stream);
       if (rc) return rc;
     }
@@ -527,7 +539,7 @@ extern "C" {
 int cbk_gemm_static(const cbk_desc* in, const void* x, int x_dtype, int M, int64_t ldx, void* y, int y_dtype,
                     int64_t ldy, const void* bias, void* stream) {
   DMat m;
-  if (!to_dmat(in, &m, false) && workspace_of(m, M, true) > (size_t)CBK_STATIC_SCRATCH_BYTES) {
+  if (!to_dmat(in, &m, false) && M >= 1 && gemm_room(m, M) == ANY_ROOM) {
     const int rc = to_dmat(in, &m, true);
     return rc ? rc : CBK_ERR_WORKSPACE;                             // more scratch than the array holds
   }
@@ -553,16 +565,19 @@ static size_t act_mid_bytes(int K, int M, int y_dtype) {
   return (b + 255) & ~(size_t)255;
 }
 
-// act(gate) * up in the kernel that sums the column parts (cbk_gemm_skinny.h): no t in memory
-static bool act_fused(const DMat& m, int M) {
-  return M > 8 && family_of(m.layout) != FAM_SPARSE && m.cs_rows <= 2 && skinny_is_faster(m, M, true);
+// How a prefill call of cbk_linear_act runs: GEMM_ROWS, act(gate) * up in the kernel that sums the column parts (no t
+// in memory); GEMM_TILE, a gate/up matrix on the tile kernel; GEMM_NONE, cbk_linear.
+static GemmPlan act_plan(const DMat& m, int M) {
+  if (M <= 8 || family_of(m.layout) == FAM_SPARSE || m.cs_rows == 3) return GemmPlan();
+  const GemmPlan p = gemm_plan(m, M, true, ANY_ROOM);
+  return p.kernel == GEMM_TILE && m.cs_rows != 2 ? GemmPlan() : p;
 }
 
 size_t cbk_linear_act_workspace_bytes(const cbk_desc* in, int M, int y_dtype) {
   DMat m;
   if (M < 1 || to_dmat(in, &m, false)) return 0;
-  if (act_fused(m, M)) return gemm_skinny_workspace(m, M, false);
-  return act_mid_bytes(m.K, M, y_dtype) + workspace_of(m, M, false);
+  const GemmPlan p = act_plan(m, M);
+  return p.kernel == GEMM_ROWS ? p.bytes : act_mid_bytes(m.K, M, y_dtype) + (p.kernel ? p.bytes : workspace_of(m, M));
 }
 
 int cbk_linear_act(const cbk_desc* in, const void* x, int x_dtype, int M, int64_t ldx, void* y, int y_dtype,
@@ -578,19 +593,21 @@ int cbk_linear_act(const cbk_desc* in, const void* x, int x_dtype, int M, int64_
   if ((uintptr_t)y & (y_dtype == CBK_F32 ? 3 : 1)) return CBK_ERR_ALIGN;
   if (!workspace || ((uintptr_t)workspace & 255) || workspace_bytes < cbk_linear_act_workspace_bytes(in, M, y_dtype))
     return CBK_ERR_WORKSPACE;
-  if (act_fused(m, M)) {
+  const GemmPlan plan = act_plan(m, M);
+  if (plan.kernel == GEMM_ROWS) {
     rc = check_io(x, x_dtype, M, ldx, y, y_dtype, ldy, m.N, m.K / 2);
     if (rc) return rc;
-    return launch_gemm_skinny(m, x, x_dtype, M, ldx, y, y_dtype, ldy, bias, act, workspace, workspace_bytes, (hipStream_t)stream);
+    return launch_gemm_skinny(m, plan, x, x_dtype, M, ldx, y, y_dtype, ldy, bias, act, workspace, workspace_bytes,
+                              (hipStream_t)stream);
   }
   const size_t mid = act_mid_bytes(m.K, M, y_dtype);
   const int tdt = act_mid_dtype(M, y_dtype);
-  if (M > 8 && m.cs_rows == 2 && gemm_big_takes(m, M)) {
+  if (plan.kernel == GEMM_TILE) {
     // the tile kernel leaves t as two halves (gate outputs, then up outputs): a workgroup holds
     // one parity of the rows, and interleaved it could only store single elements
     rc = check_io(x, x_dtype, M, ldx, workspace, tdt, m.K, m.N, m.K);
     if (rc) return rc;
-    rc = launch_gemm_big(m, x, x_dtype, M, ldx, workspace, tdt, m.K, nullptr, (uint8_t*)workspace + mid,
+    rc = launch_gemm_big(m, plan, x, x_dtype, M, ldx, workspace, tdt, m.K, nullptr, (uint8_t*)workspace + mid,
                          workspace_bytes - mid, (hipStream_t)stream, true);
     if (rc) return rc;
     return launch_act_mul(workspace, tdt, m.K, y, y_dtype, ldy, M, m.K / 2, act, bias, (hipStream_t)stream, true);

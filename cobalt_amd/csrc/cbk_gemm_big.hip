@@ -2,6 +2,7 @@
 // and the dispatch over the per-code-width instantiations (cbk_gemm_big_b2/3/4.hip).  The
 // kernel itself is in cbk_gemm_big.h.
 #include "cbk_gemm_big.h"
+#include "cbk_gemm_plan.h"
 #include "cbk_prep.h"
 
 namespace cbk {
@@ -151,72 +152,80 @@ static bool gb_fast(const DMat& m) {
 // 98.)  Over 24 measured calls
 // (eight shapes, 256 / 512 / 2048 rows) the choice is within 2 % of the faster tile; always
 // taking the 256-token tile loses 6 % on average and up to 34 %.
-struct GbPlan { int ti, nsplit; double t; };
-static GbPlan gb_plan_ti(const DMat& m, int M, int ti, int max_split) {
-  const int T = 64 * ti;
-  const int tiles = ((M + T - 1) / T) * ((m.K + GB_R - 1) / GB_R);
-  const int nst = gb_npad(m.N) / GB_K;
-  const double t_stage = ti == 1 ? 1.1 : ti == 2 ? 1.35 : 1.7, t_wg = ti == 1 ? 8.0 : 10.0;
-  GbPlan best{ti, 1, 0.0};
-  double t1 = 0;
-  const bool may_split = max_split > 1 && m.cs_rows != 2 && gb_fast(m);
-  for (int s = 1; s <= (may_split ? max_split : 1); ++s) {
-    const int per = ((nst + s - 1) / s + 3) / 4 * 4;                // stages per part, a multiple of 4
-    if (s > 1 && (s - 1) * per >= nst) continue;                    // a part would be empty
-    const double rounds = (double)((tiles * s + 255) / 256);
-    double t = rounds * (per * t_stage + t_wg);
-    if (s > 1) t += 2.0 * s * (double)M * m.K * 4 / 4.0e6 + 5.0;
-    if (s == 1) { t1 = t; best.t = t; }
-    else if (t < best.t) { best.nsplit = s; best.t = t; }
-  }
-  if (best.t > 0.93 * t1) { best.nsplit = 1; best.t = t1; }         // not worth a second kernel
-  return best;
-}
-static GbPlan gb_plan(const DMat& m, int M, int max_split = 16) {
-  if (M <= 64) return gb_plan_ti(m, M, 1, max_split);
-  if (M <= 128) return gb_plan_ti(m, M, 2, max_split);
-  const GbPlan p4 = gb_plan_ti(m, M, 4, max_split), p2 = gb_plan_ti(m, M, 2, max_split);
-  return p2.t < p4.t ? p2 : p4;
-}
-
 static inline size_t gb_kpad(int K) { return (size_t)(K + 7) / 8 * 8; }
-
-static size_t gb_space(const DMat& m, int M, const GbPlan& plan) {
-  const size_t T = 64 * plan.ti, mpad = (size_t)(M + T - 1) / T * T;
+static size_t gb_space(const DMat& m, int M, int ti, int nsplit) {
+  const size_t T = 64 * ti, mpad = (size_t)(M + T - 1) / T * T;
   const size_t nv = m.cs_rows > 1 ? m.cs_rows : 1;
   size_t b = (nv * mpad * gb_npad(m.N) * 2 + 255) & ~(size_t)255;     // X', one per col_scale vector
   b += (nv * mpad * 4 + 255) & ~(size_t)255;                          // and its row scales
-  const int ns = plan.nsplit;
-  if (ns > 1) b += ((size_t)ns * M * gb_kpad(m.K) * 4 + 255) & ~(size_t)255;
+  if (nsplit > 1) b += ((size_t)nsplit * M * gb_kpad(m.K) * 4 + 255) & ~(size_t)255;
   return b;
 }
-// least: without room for partial tiles, i.e. with the column range in one piece
-size_t gemm_big_workspace(const DMat& m, int M, bool least) { return gb_space(m, M, gb_plan(m, M, least ? 1 : 16)); }
+// stages per part, a multiple of 4; 0: a part would be empty
+static int gb_part(const DMat& m, int nsplit) {
+  const int nst = gb_npad(m.N) / GB_K, per = ((nst + nsplit - 1) / nsplit + 3) / 4 * 4;
+  return nsplit > 1 && (nsplit - 1) * per >= nst ? 0 : per;
+}
+static GemmPlan gb_plan_ti(const DMat& m, int M, int ti, int max_split, size_t room) {
+  const int T = 64 * ti;
+  const int tiles = ((M + T - 1) / T) * ((m.K + GB_R - 1) / GB_R);
+  const double t_stage = ti == 1 ? 1.1 : ti == 2 ? 1.35 : 1.7, t_wg = ti == 1 ? 8.0 : 10.0;
+  GemmPlan best, one;
+  const bool may_split = max_split > 1 && m.cs_rows != 2 && gb_fast(m);
+  for (int s = 1; s <= (may_split ? max_split : 1); ++s) {
+    const int per = gb_part(m, s);
+    if (!per) continue;
+    const size_t bytes = gb_space(m, M, ti, s);
+    if (bytes > room) continue;
+    const double rounds = (double)((tiles * s + 255) / 256);
+    double t = rounds * (per * t_stage + t_wg);
+    if (s > 1) t += 2.0 * s * (double)M * m.K * 4 / 4.0e6 + 5.0;
+    if (s == 1) best = one = {GEMM_TILE, ti, 1, t, bytes};
+    else if (t < best.t) best = {GEMM_TILE, ti, s, t, bytes};
+  }
+  return best.t > 0.93 * one.t ? one : best;                        // (not worth a second kernel)
+}
+static GemmPlan gb_plan(const DMat& m, int M, int max_split, size_t room) {
+  if (M <= 64) return gb_plan_ti(m, M, 1, max_split, room);
+  if (M <= 128) return gb_plan_ti(m, M, 2, max_split, room);
+  const GemmPlan p4 = gb_plan_ti(m, M, 4, max_split, room), p2 = gb_plan_ti(m, M, 2, max_split, room);
+  return !p4.kernel || (p2.kernel && p2.t < p4.t) ? p2 : p4;
+}
+// the q|k|v matrices it takes whole: ranges that start on its row tiles
+static bool gb_takes(const DMat& m, int M) {
+  if (M < 1 || family_of(m.layout) == FAM_SPARSE) return false;
+  return m.cs_rows <= 2 || (m.cs_split0 % GB_R == 0 && (m.cs_split0 + m.cs_split1) % GB_R == 0);
+}
+size_t big_unsplit_space(const DMat& m, int M) { return gb_plan(m, M, m.cs_rows <= 1 ? 16 : 1, ANY_ROOM).bytes; }
+GemmPlan fixed_plan_big(const DMat& m, int M, int ti, int nsplit) {
+  GemmPlan p;
+  if (!gb_takes(m, M) || (ti != 1 && ti != 2 && ti != 4) || nsplit < 1 || nsplit > 16 || !gb_part(m, nsplit) ||
+      (nsplit > 1 && (m.cs_rows == 2 || !gb_fast(m))))
+    return p;
+  p.kernel = GEMM_TILE; p.ti = ti; p.nsplit = nsplit; p.bytes = gb_space(m, M, ti, nsplit);
+  return p;
+}
 
-// What a call takes, for the choice between this kernel and the one in cbk_gemm_skinny.h: the plan's
-// time, 5 us for the preparation kernel and the launch, 3 more where a gate/up matrix needs the activation
-// kernel behind it (and that kernel's traffic).  Partial tiles count at 6.5 TB/s here: 4 is what keeps the plan from
+// `t` is what a call takes, for the choice between this kernel and the one in cbk_gemm_skinny.h: the tile's and
+// split's time, 5 us for the preparation kernel and the launch.  Partial tiles count at 6.5 TB/s here: 4 is what keeps the plan from
 // splitting where it does not pay, calls that are split measure faster (14336 x 4096 at 256 rows 61 us, 3840 x 7424 at
 // 1024 rows 89).  Layouts without a decoder of their own are read at a
 // tenth of the rate.
-double gemm_big_time(const DMat& m, int M, bool act) {
-  const GbPlan p = gb_plan(m, M);
+GemmPlan plan_big(const DMat& m, int M, size_t room) {
+  if (!gb_takes(m, M)) return GemmPlan();
+  GemmPlan p = gb_plan(m, M, 16, room);
   const double parts = p.nsplit > 1 ? 2.0 * p.nsplit * (double)M * m.K * 4 : 0.0;
-  const double t = (p.t - parts * (1 / 4.0e6 - 1 / 6.5e6)) * (gb_fast(m) ? 1.0 : 10.0) + 5.0;
-  return act ? t + 3.0 + (double)M * m.K * (M <= 128 ? 9 : 5) / 5.0e6 : t;
+  p.t = (p.t - parts * (1 / 4.0e6 - 1 / 6.5e6)) * (gb_fast(m) ? 1.0 : 10.0) + 5.0;
+  return p;
 }
 
-// halves: a gate/up matrix's outputs as two halves of y (GbArgs::halves) instead of interleaved
-int launch_gemm_big(const DMat& m, const void* x, int xdt, int M, int64_t ldx, void* y, int ydt, int64_t ldy,
-                    const void* bias, void* ws, size_t ws_bytes, hipStream_t st, bool halves) {
+int launch_gemm_big(const DMat& m, const GemmPlan& plan, const void* x, int xdt, int M, int64_t ldx, void* y, int ydt,
+                    int64_t ldy, const void* bias, void* ws, size_t ws_bytes, hipStream_t st, bool halves) {
   if (halves && (m.cs_rows != 2 || (m.K & 1) || bias)) return CBK_ERR_UNSUPPORTED;
-  if (family_of(m.layout) == FAM_SPARSE) return CBK_ERR_UNSUPPORTED;
-  // q|k|v ranges off the row-tile grid: the caller passes them one by one
-  if (m.cs_rows == 3 && (m.cs_split0 % GB_R || (m.cs_split0 + m.cs_split1) % GB_R)) return CBK_ERR_UNSUPPORTED;
+  // (q|k|v ranges off the row-tile grid: the caller passes them one by one)
+  if (plan.kernel != GEMM_TILE || !gb_takes(m, M)) return CBK_ERR_UNSUPPORTED;
   if (ydt != CBK_F32 && ydt != CBK_F16 && ydt != CBK_BF16T) return CBK_ERR_DTYPE;
-  GbPlan plan = gb_plan(m, M);
-  if (ws_bytes < gb_space(m, M, plan)) plan = gb_plan(m, M, 1);     // no room for partial tiles
-  if (!ws || ws_bytes < gb_space(m, M, plan)) return CBK_ERR_WORKSPACE;
+  if (!ws || ws_bytes < gb_space(m, M, plan.ti, plan.nsplit)) return CBK_ERR_WORKSPACE;
   if ((uintptr_t)ws & 255) return CBK_ERR_ALIGN;
   const int T = 64 * plan.ti;
   const int Mpad = (M + T - 1) / T * T;
@@ -238,9 +247,8 @@ int launch_gemm_big(const DMat& m, const void* x, int xdt, int M, int64_t ldx, v
   a.row_scale = row_scale; a.rss = Mpad;
   a.vs0 = m.cs_rows == 3 ? m.cs_split0 : 0x7fffffff;
   a.vs1 = m.cs_rows == 3 ? m.cs_split0 + m.cs_split1 : 0x7fffffff;
-  const int nst_all = Npad / GB_K;
   a.nsplit = plan.nsplit;
-  a.nst_part = ((nst_all + a.nsplit - 1) / a.nsplit + 3) / 4 * 4;
+  a.nst_part = gb_part(m, plan.nsplit);
   a.part_ld = (int64_t)gb_kpad(m.K);
   a.part_stride = (size_t)M * gb_kpad(m.K);
   a.part = (float*)((uint8_t*)ws + xbytes + sbytes);

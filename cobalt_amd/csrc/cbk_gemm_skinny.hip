@@ -1,5 +1,6 @@
 // Preparation kernel, reduction kernels, plan and dispatch of the GEMM in cbk_gemm_skinny.h.
 #include "cbk_gemm_skinny.h"
+#include "cbk_gemm_plan.h"
 #include "cbk_prep.h"
 
 namespace cbk {
@@ -157,71 +158,63 @@ bool gemm_skinny_takes(const DMat& m) {
   return m.keep == 10 || m.keep == 16 || m.keep == 23;
 }
 
-struct SkPlan { int ti, nsplit; double t; };
+struct SkSpace { size_t x, sums, scale, part; int mpad; };
+static SkSpace sk_space(const DMat& m, int M, int ti, int nsplit) {
+  SkSpace s;
+  s.mpad = (M + 32 * ti - 1) / (32 * ti) * (32 * ti);
+  const size_t nv = m.cs_rows > 1 ? m.cs_rows : 1;
+  s.x = sk_up(nv * s.mpad * m.N * 2);
+  s.sums = sk_up(nv * s.mpad * m.G * 8);
+  s.scale = sk_up(nv * s.mpad * nsplit * SK_WC * 4);                // one per part of the column range
+  s.part = nsplit > 1 ? sk_up((size_t)nsplit * M * ((m.K + 7) / 8 * 8) * 4) : 0;
+  return s;
+}
+static inline size_t sk_sum(const SkSpace& s) { return s.x + s.sums + s.scale + s.part; }
 // Times in microseconds, fitted to calls of ten shapes (1024 x 4096 to 43008 x 5376) at 16 to 1700 rows,
 // within a tenth of the measured ones: a group of a wavefront with two wavefronts per SIMD, by token tile
 // (codes that do not start on 16-byte units take a fifth longer, 6-bit codes with their second plane
 // 1.35 times), 5.5 to 10 per workgroup outside the loop, 7.4 for the preparation kernel and the launches and 0.5 per megabyte of X' beyond four (written, and
 // fetched by every XCD: 1024 x 5376 at 4096 rows, 44 MB, took 25 more than without that term), 5.5 and the
 // partial tiles at 4 TB/s for the reduction kernel.
-static SkPlan sk_plan_ti(const DMat& m, int M, int ti, int max_split) {
+static GemmPlan sk_plan_ti(const DMat& m, int M, int ti, size_t room) {
   const int tiles = ((M + 32 * ti - 1) / (32 * ti)) * ((m.K + SK_ROWS * SK_WR - 1) / (SK_ROWS * SK_WR));
   static const double g128[3] = {1.7, 2.2, 2.8}, g64[3] = {1.17, 1.45, 1.53}, wg[3] = {5.5, 7.6, 10.0};
   const bool skewed = family_of(m.layout) == FAM_BLK && (m.keep * m.bits * (m.group / 64)) % 32 != 0;
   const double two = m.cs_rows == 2 ? 1.12 : 1.0;                   // (two sets of X' compete for L2)
   const double t_group = (m.group == 128 ? g128 : g64)[ti - 1] * (skewed ? 1.2 : m.bits == 6 ? 1.35 : 1.0) * two, t_wg = wg[ti - 1] * two;
   const double xmb = 2e-6 * (m.cs_rows > 1 ? m.cs_rows : 1) * (double)M * m.N, t_prep = 7.4 + (xmb > 4.0 ? 0.5 * (xmb - 4.0) : 0.0);
-  SkPlan best{ti, 1, 0};
-  for (int s = 1; s <= max_split; ++s) {
+  GemmPlan best;
+  for (int s = 1; s <= 16; ++s) {
+    const size_t bytes = sk_sum(sk_space(m, M, ti, s));
+    if (bytes > room) break;                                        // (more parts take more)
     const int per = (m.G + SK_WC * s - 1) / (SK_WC * s);
     double t = t_prep + (double)((tiles * s + 255) / 256) * (per * t_group + t_wg);
     if (s > 1) t += 2.0 * s * (double)M * m.K * 4 / 4.0e6 + 5.5;
-    if (s == 1 || t < best.t) { best.nsplit = s; best.t = t; }
+    if (s == 1 || t < best.t) best = {GEMM_ROWS, ti, s, t, bytes};
     if (SK_WC * s >= m.G) break;
   }
   return best;
 }
-static SkPlan sk_plan(const DMat& m, int M, int max_split = 16) {
-  SkPlan best = sk_plan_ti(m, M, 1, max_split);
-  for (int ti = 2; ti <= 3; ++ti) {
-    const SkPlan p = sk_plan_ti(m, M, ti, max_split);
-    if (p.t < best.t) best = p;
+GemmPlan plan_skinny(const DMat& m, int M, size_t room) {
+  GemmPlan best;
+  if (M < 1 || !gemm_skinny_takes(m)) return best;
+  for (int ti = 1; ti <= 3; ++ti) {
+    const GemmPlan p = sk_plan_ti(m, M, ti, room);
+    if (p.kernel && (!best.kernel || p.t < best.t)) best = p;
   }
   return best;
 }
-double gemm_skinny_time(const DMat& m, int M) { return sk_plan(m, M).t; }
-
-struct SkSpace { size_t x, sums, scale, part; int mpad; };
-static SkSpace sk_space(const DMat& m, int M, const SkPlan& p) {
-  SkSpace s;
-  s.mpad = (M + 32 * p.ti - 1) / (32 * p.ti) * (32 * p.ti);
-  const size_t nv = m.cs_rows > 1 ? m.cs_rows : 1;
-  s.x = sk_up(nv * s.mpad * m.N * 2);
-  s.sums = sk_up(nv * s.mpad * m.G * 8);
-  s.scale = sk_up(nv * s.mpad * p.nsplit * SK_WC * 4);              // one per part of the column range
-  s.part = p.nsplit > 1 ? sk_up((size_t)p.nsplit * M * ((m.K + 7) / 8 * 8) * 4) : 0;
-  return s;
-}
-static inline size_t sk_sum(const SkSpace& s) { return s.x + s.sums + s.scale + s.part; }
-// `room`: what the caller has, or (size_t)-1: the split is taken back where its partial tiles do not fit
-static SkPlan sk_fit(const DMat& m, int M, size_t room, SkSpace& s) {
-  SkPlan p = sk_plan(m, M);
-  s = sk_space(m, M, p);
-  if (sk_sum(s) > room) { p = sk_plan(m, M, 1); s = sk_space(m, M, p); }
+GemmPlan fixed_plan_skinny(const DMat& m, int M, int ti, int nsplit) {
+  GemmPlan p;
+  if (M < 1 || !gemm_skinny_takes(m) || ti < 1 || ti > 3 || nsplit < 1 || nsplit > 16) return p;
+  p.kernel = GEMM_ROWS; p.ti = ti; p.nsplit = nsplit; p.bytes = sk_sum(sk_space(m, M, ti, nsplit));
   return p;
 }
-size_t gemm_skinny_workspace(const DMat& m, int M, bool least) {
-  SkSpace s;
-  sk_fit(m, M, least ? 0 : (size_t)-1, s);
-  return sk_sum(s);
-}
 
-// act: -1, or CBK_ACT_*: y = act(gate) * up of a gate/up matrix, [M, K / 2]
-int launch_gemm_skinny(const DMat& m, const void* x, int xdt, int M, int64_t ldx, void* y, int ydt, int64_t ldy,
-                       const void* bias, int act, void* ws, size_t ws_bytes, hipStream_t st) {
-  if (!gemm_skinny_takes(m) || (act >= 0 && ((m.K & 1) || m.cs_rows == 3))) return CBK_ERR_UNSUPPORTED;
-  SkSpace sp;
-  const SkPlan plan = sk_fit(m, M, ws_bytes, sp);
+int launch_gemm_skinny(const DMat& m, const GemmPlan& plan, const void* x, int xdt, int M, int64_t ldx, void* y, int ydt,
+                       int64_t ldy, const void* bias, int act, void* ws, size_t ws_bytes, hipStream_t st) {
+  if (plan.kernel != GEMM_ROWS || !gemm_skinny_takes(m) || (act >= 0 && ((m.K & 1) || m.cs_rows == 3))) return CBK_ERR_UNSUPPORTED;
+  const SkSpace sp = sk_space(m, M, plan.ti, plan.nsplit);
   if (!ws || ws_bytes < sk_sum(sp)) return CBK_ERR_WORKSPACE;
   if ((uintptr_t)ws & 255) return CBK_ERR_ALIGN;
   const int nv = m.cs_rows > 1 ? m.cs_rows : 1;

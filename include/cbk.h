@@ -132,12 +132,13 @@ size_t cbk_row_stride(const cbk_desc* d);
  * (pack_cobalt.write_matrix :431-433 `stream_bytes`); SPARSE layouts need data_bytes. */
 size_t cbk_stream_bytes(const cbk_desc* d, size_t sparse_data_bytes);
 
-/* Device scratch that cbk_gemv / cbk_gemm / cbk_linear make use of for M activation rows.  The prefill
+/* Device scratch needed by cbk_gemv / cbk_gemm / cbk_linear for M activation rows.  The prefill
  * kernels keep their pre-scaled fp16 activations there: ceil(M/256)*256 * ceil(N/256)*256 * 2 bytes
- * per col_scale vector, i.e. times cs_rows for a fused matrix, one float32 scale per activation
- * row and col_scale vector (and a word per activation row and group), plus float32 partial outputs
- * when the library splits the column range of a launch that would not fill the chip; a call with
- * room for the activations only runs in one piece.  The decode kernels need none, with one optional use:
+ * per col_scale vector, i.e. times cs_rows for a fused matrix, at most, float32 scales per activation
+ * row and col_scale vector (and two words per activation row and group), plus float32 partial outputs
+ * when the library splits the column range of a launch that would not fill the chip.  A prefill call with
+ * less is refused (CBK_ERR_WORKSPACE): its results do not depend on what it is given.  The decode
+ * kernels need none, with one optional use:
  * two to eight activation rows of rows whose activations take more than 90 KB of LDS
  * (M * 3 * N bytes) are split over the workgroups by columns when there is room for the float32
  * part sums, K * 16 * M * 4 bytes at most, and so are the rows of SPARSE4X / SPARSE4E matrices on
@@ -224,13 +225,13 @@ int cbk_gemm(const cbk_desc* d, const void* x, int x_dtype, int M, int64_t ldx,
 
 /* cbk_gemm for callers that cannot allocate device memory or pass a workspace: code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in
- * the reference.  Same computation as cbk_gemm, with the scratch (pre-scaled
+ * the reference.  Same computation and same results as cbk_gemm, with the scratch (pre-scaled
  * activations, partial output tiles) in an array of CBK_STATIC_SCRATCH_BYTES that is part of the
  * library's device image: every GPU the library runs on holds one copy until the process ends.
- * The call allocates and frees nothing.  A call whose activations do not fit the array is
- * refused with CBK_ERR_WORKSPACE before anything is launched (16 MiB hold e.g. 1024 activation
- * rows of 5376 columns; prompts beyond that go through cbk_gemm); one whose partial outputs do not
- * fit runs with its column range in one piece (the sums then round differently from cbk_gemm's).  All calls on one GPU share
+ * The call allocates and frees nothing.  A call whose scratch exceeds the array on the 256-row
+ * tile kernel is refused with CBK_ERR_WORKSPACE before anything is launched (16 MiB hold e.g. 1024
+ * activation rows of 5376 columns; prompts beyond that go through cbk_gemm); the others run on the same plan
+ * under both names, one that fits the array.  All calls on one GPU share
  * that GPU's array: calls that overlap in time on one GPU (two streams, two threads) race;
  * calls on one stream are safe.  Nothing in the array needs to start at zero and nothing is
  * carried from one call to the next.  The first call on a GPU looks up the array's address

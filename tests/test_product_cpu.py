@@ -205,6 +205,36 @@ def test_entry_points_reject_bad_arguments_before_any_launch():
     assert L.cbk_gemm_static(ctypes.byref(big), 0x4000, 2, 4096, 21504, 0x5000, 2, 256, None, None) == -6
 
 
+@pytest.mark.skipif(torch.cuda.is_available(), reason="addresses that are none: only where no launch can follow")
+def test_prefill_results_do_not_depend_on_the_workspace():
+    """A prefill call has one plan: a byte less than cbk_workspace_bytes is refused, whatever a plan with fewer
+    parts would need.  cbk_gemm_static, which promises cbk_gemm's results, takes the calls it always took
+    (its answer here is the HIP error of a machine without a GPU) and refuses the others."""
+    L = _lib.lib()
+    fmts = ((F.BLK1632_4, 0, 0, 0), (F.BLKC, 2, 64, 16), (F.BLKC, 3, 64, 10), (F.DENSE4, 0, 0, 0), (F.DENSE8, 0, 0, 0), (F.DENSEB, 2, 64, 0))
+
+    def desc(fmt, K, N, cs, splits=(0, 0)):
+        return F.CbkDesc(K=K, N=N, layout=fmt[0], bits=fmt[1], group=fmt[2], keep=fmt[3], data=0x1000, scale=0x2000, zero=0x3000,
+                         col_scale=0x4000, cs_rows=cs, cs_split0=splits[0], cs_split1=splits[1],
+                         flags=F.FLAG_ZERO_LE_128 | F.FLAG_ZERO_ON_GRID)
+
+    for fmt in fmts:
+        for K, N in ((256, 14336), (1024, 4096), (4096, 4096), (14336, 4096)):
+            for cs, splits in ((1, (0, 0)), (2, (0, 0)), (3, (K // 2, K // 4)), (3, (K // 2 - 48, K // 4 + 16))):
+                for M in (17, 64, 130, 333, 600, 2048):
+                    d = desc(fmt, K, N, cs, splits)
+                    need = L.cbk_workspace_bytes(ctypes.byref(d), M)
+                    for fn in (L.cbk_gemm, L.cbk_linear):
+                        assert fn(ctypes.byref(d), 0x8000, 1, M, N, 0x9000, 1, K, None, 0x10000, need - 1, None) == -6, (fmt, K, N, cs, M)
+    b64_2, b64_3, d8 = fmts[1], fmts[2], fmts[4]
+    for fmt, K, N, M, cs, takes in ((b64_2, 1430, 7040, 405, 2, True), (b64_3, 2602, 4864, 540, 2, True), (d8, 1459, 11264, 486, 1, True),
+                                    (fmts[0], 84, 6016, 577, 2, True), (fmts[0], 21504, 5376, 1024, 1, True),
+                                    (fmts[0], 256, 5376, 1792, 1, False), (d8, 4096, 14336, 512, 1, False)):
+        d = desc(fmt, K, N, cs)
+        assert (L.cbk_gemm_static(ctypes.byref(d), 0x8000, 1, M, N, 0x9000, 1, K, None, None) == -6) == (not takes), (fmt, K, N, M)
+        assert (L.cbk_workspace_bytes(ctypes.byref(d), M) <= 16 << 20) == takes
+
+
 def test_ops_refuse_to_run_without_gpu_tensors():
     from cobalt_amd import ops
     pm = F.synth_packed(16, 256, F.BLK1632_4, seed=1)

@@ -42,6 +42,26 @@ def test_static_scratch_matches_cbk_gemm_twice():
     assert torch.equal(got, ops.gemm(big, x))
 
 
+@pytest.mark.parametrize("layout,bits,group,keep,K,N,M,pair", [
+    (F.BLKC, 2, 64, 16, 715, 7040, 405, True), (F.DENSE8, 8, 128, None, 1459, 11264, 486, False),
+    (F.BLK1632_4, 4, 128, 16, 42, 6016, 577, True), (F.BLKC, 3, 64, 10, 1301, 4864, 540, True)])
+def test_static_scratch_matches_cbk_gemm_near_the_size_of_the_array(layout, bits, group, keep, K, N, M, pair):
+    """Calls whose fastest split of the columns would need more than the array: both entry points run the
+    same plan.  A larger workspace changes nothing, a smaller one is refused."""
+    g = torch.Generator(device=DEV).manual_seed(M)
+    parts = [F.synth_packed(K, N, layout, bits, group, keep, seed=i, device=DEV) for i in range(2 if pair else 1)]
+    pm = (F.fuse_rows(parts, interleave=True) if pair else parts[0]).to_tiled()
+    x = torch.randn(M, N, device=DEV, generator=g).half()
+    want = ops.gemm(pm, x, out_dtype=torch.float32)
+    rc, got = _static(pm, x, torch.float32)
+    assert rc == 0 and torch.equal(got, want)
+    need = _lib.lib().cbk_workspace_bytes(ctypes.byref(pm.desc()), M)
+    room = torch.empty(4 * need, dtype=torch.uint8, device=DEV)
+    assert torch.equal(ops.gemm(pm, x, out_dtype=torch.float32, workspace=room), want)
+    with pytest.raises(_lib.CbkError):
+        ops.gemm(pm, x, out_dtype=torch.float32, workspace=room[:need - 1])
+
+
 def test_static_scratch_call_inside_a_graph_allocates_nothing():
     g = torch.Generator(device=DEV).manual_seed(5)
     pm = F.synth_packed(768, 5376, F.BLK1632_4, seed=13, device=DEV).to_tiled()
