@@ -229,7 +229,7 @@ def test_prefill_results_do_not_depend_on_the_workspace():
     b64_2, b64_3, d8 = fmts[1], fmts[2], fmts[4]
     for fmt, K, N, M, cs, takes in ((b64_2, 1430, 7040, 405, 2, True), (b64_3, 2602, 4864, 540, 2, True), (d8, 1459, 11264, 486, 1, True),
                                     (fmts[0], 84, 6016, 577, 2, True), (fmts[0], 21504, 5376, 1024, 1, True),
-                                    (fmts[0], 256, 5376, 1792, 1, False), (d8, 4096, 14336, 512, 1, False)):
+                                    (fmts[0], 256, 5376, 1792, 1, False), (d8, 4096, 14336, 1024, 1, False)):
         d = desc(fmt, K, N, cs)
         assert (L.cbk_gemm_static(ctypes.byref(d), 0x8000, 1, M, N, 0x9000, 1, K, None, None) == -6) == (not takes), (fmt, K, N, M)
         assert (L.cbk_workspace_bytes(ctypes.byref(d), M) <= 16 << 20) == takes
