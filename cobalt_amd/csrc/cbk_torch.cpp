@@ -69,6 +69,8 @@ PyObject* matrix_new(PyTypeObject* t, PyObject* args, PyObject*) {
 
 PyTypeObject MatrixType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
+// Other Python threads run while this one allocates and launches: a launch waits when its queue is full, an allocation
+// may wait for the device.  No Python object is touched and no Python exception set in its scope.
 struct GilRelease {
   PyThreadState* s = PyEval_SaveThread();
   ~GilRelease() { PyEval_RestoreThread(s); }
@@ -151,11 +153,13 @@ void require_gpu(const Matrix* m, const at::Tensor& x, const at::Tensor& bias) {
       fail(g_error, "tensor on " + t->device().str() + ", packed matrix on " + m->blob->device().str());
 }
 
+void check_features(const at::Tensor& x, int64_t N) {
+  if (x.dim() < 1 || x.size(-1) != N)
+    fail(PyExc_ValueError, "x has " + std::to_string(x.dim() ? x.size(-1) : 1) + " input features, the matrix has N=" + std::to_string(N));
+}
 // x as [M, N] rows of unit stride the kernels can read with 16-byte loads (a copy if it is not)
 struct Rows { at::Tensor keep; const void* p; int64_t M, ld; };
 Rows rows_of(const at::Tensor& x, int64_t N) {
-  if (x.dim() < 1 || x.size(-1) != N)
-    fail(PyExc_ValueError, "x has " + std::to_string(x.dim() ? x.size(-1) : 1) + " input features, the matrix has N=" + std::to_string(N));
   Rows r;
   r.M = x.numel() / N;
   const bool flat = x.is_contiguous();
@@ -215,19 +219,28 @@ PyObject* py_matmul(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!x.defined()) fail(PyExc_TypeError, "x must be a tensor");
     require_gpu(m, x, bias);
     const cbk_desc d = desc_of(m);
-    const Rows r = rows_of(x, d.N);
+    check_features(x, d.N);
     const at::ScalarType odt = out_type(a[4], x);
-    at::Tensor y = out_for(x, d.K, odt);
-    if (r.M == 0) return THPVariable_Wrap(y);
-    const int xdt = dtype_code(x.scalar_type()), ydt = dtype_code(odt), M = (int)r.M;
-    if (bias.defined() && bias.scalar_type() != odt) bias = bias.to(odt);
-    const c10::DeviceGuard guard(x.device());
-    if (!ws.defined())
-      ws = scratch(x, entry == 0 || (entry == 2 && M <= 8) ? cbk::decode_workspace_bytes(&d, M) : cbk_workspace_bytes(&d, M));
-    auto fn = entry == 0 ? cbk_gemv : entry == 1 ? cbk_gemm : cbk_linear;
-    check(fn(&d, r.p, xdt, M, r.ld, y.mutable_data_ptr(), ydt, d.K, bias.defined() ? bias.const_data_ptr() : nullptr,
-             ws.defined() ? ws.mutable_data_ptr() : nullptr, ws.defined() ? ws.nbytes() : 0, stream_of(x)),
-          entry == 0 ? "cbk_gemv" : entry == 1 ? "cbk_gemm" : "cbk_linear");
+    const bool any = x.numel() > 0;
+    const int xdt = any ? dtype_code(x.scalar_type()) : 0, ydt = any ? dtype_code(odt) : 0;
+    at::Tensor y;
+    int rc = CBK_OK;
+    {
+      const GilRelease other_threads_run;
+      y = out_for(x, d.K, odt);
+      if (any) {
+        const Rows r = rows_of(x, d.N);
+        const int M = (int)r.M;
+        if (bias.defined() && bias.scalar_type() != odt) bias = bias.to(odt);
+        const c10::DeviceGuard guard(x.device());
+        if (!ws.defined())
+          ws = scratch(x, entry == 0 || (entry == 2 && M <= 8) ? cbk::decode_workspace_bytes(&d, M) : cbk_workspace_bytes(&d, M));
+        auto fn = entry == 0 ? cbk_gemv : entry == 1 ? cbk_gemm : cbk_linear;
+        rc = fn(&d, r.p, xdt, M, r.ld, y.mutable_data_ptr(), ydt, d.K, bias.defined() ? bias.const_data_ptr() : nullptr,
+                ws.defined() ? ws.mutable_data_ptr() : nullptr, ws.defined() ? ws.nbytes() : 0, stream_of(x));
+      }
+    }
+    check(rc, entry == 0 ? "cbk_gemv" : entry == 1 ? "cbk_gemm" : "cbk_linear");
     return THPVariable_Wrap(y);
   });
 }
@@ -243,19 +256,28 @@ PyObject* py_linear_act(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!x.defined()) fail(PyExc_TypeError, "x must be a tensor");
     require_gpu(m, x, bias);
     const cbk_desc d = desc_of(m);
-    const Rows r = rows_of(x, d.N);
+    check_features(x, d.N);
     if (d.K % 2) fail(PyExc_ValueError, "a gate/up matrix has an even number of rows");
     const at::ScalarType odt = out_type(a[4], x);
-    at::Tensor y = out_for(x, d.K / 2, odt);
-    if (r.M == 0) return THPVariable_Wrap(y);
-    const int xdt = dtype_code(x.scalar_type()), ydt = dtype_code(odt), M = (int)r.M;
-    if (bias.defined() && bias.scalar_type() != odt) bias = bias.to(odt);
-    const c10::DeviceGuard guard(x.device());
-    const at::Tensor ws = scratch(x, cbk_linear_act_workspace_bytes(&d, M, ydt));
-    check(cbk_linear_act(&d, r.p, xdt, M, r.ld, y.mutable_data_ptr(), ydt, d.K / 2,
-                         bias.defined() ? bias.const_data_ptr() : nullptr, act,
-                         ws.defined() ? ws.mutable_data_ptr() : nullptr, ws.defined() ? ws.nbytes() : 0, stream_of(x)),
-          "cbk_linear_act");
+    const bool any = x.numel() > 0;
+    const int xdt = any ? dtype_code(x.scalar_type()) : 0, ydt = any ? dtype_code(odt) : 0;
+    at::Tensor y;
+    int rc = CBK_OK;
+    {
+      const GilRelease other_threads_run;
+      y = out_for(x, d.K / 2, odt);
+      if (any) {
+        const Rows r = rows_of(x, d.N);
+        const int M = (int)r.M;
+        if (bias.defined() && bias.scalar_type() != odt) bias = bias.to(odt);
+        const c10::DeviceGuard guard(x.device());
+        const at::Tensor ws = scratch(x, cbk_linear_act_workspace_bytes(&d, M, ydt));
+        rc = cbk_linear_act(&d, r.p, xdt, M, r.ld, y.mutable_data_ptr(), ydt, d.K / 2,
+                            bias.defined() ? bias.const_data_ptr() : nullptr, act,
+                            ws.defined() ? ws.mutable_data_ptr() : nullptr, ws.defined() ? ws.nbytes() : 0, stream_of(x));
+      }
+    }
+    check(rc, "cbk_linear_act");
     return THPVariable_Wrap(y);
   });
 }
@@ -272,9 +294,17 @@ PyObject* py_dequant(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int cs = PyObject_IsTrue(a[4]);
     if (PyErr_Occurred()) throw Fail{};
     const cbk_desc d = desc_of(m);
-    at::Tensor out = at::empty({(int64_t)nrows, (int64_t)d.N}, m->blob->options().dtype(dt));
-    const c10::DeviceGuard guard(out.device());
-    check(cbk_dequant(&d, (int)row0, (int)nrows, cs, out.mutable_data_ptr(), dtype_code(dt), d.N, stream_of(out)), "cbk_dequant");
+    const int odt = dtype_code(dt);
+    const at::TensorOptions like = m->blob->options().dtype(dt);
+    at::Tensor out;
+    int rc = CBK_OK;
+    {
+      const GilRelease other_threads_run;
+      out = at::empty({(int64_t)nrows, (int64_t)d.N}, like);
+      const c10::DeviceGuard guard(out.device());
+      rc = cbk_dequant(&d, (int)row0, (int)nrows, cs, out.mutable_data_ptr(), odt, d.N, stream_of(out));
+    }
+    check(rc, "cbk_dequant");
     return THPVariable_Wrap(out);
   });
 }
@@ -291,12 +321,7 @@ PyObject* py_gemv_batch(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     if (n > 8) check(CBK_ERR_SHAPE, "cbk_gemv_batch");
     cbk_desc d[8];
     at::Tensor x[8], y[8], b[8];
-    Rows r[8];
-    const void *xp[8], *bp[8];
-    void* yp[8];
-    int64_t ldx[8], ldy[8];
     at::ScalarType odt = at::kHalf;
-    size_t need = 0;
     for (Py_ssize_t i = 0; i < n; ++i) {
       const Matrix* m = as_matrix(PyList_GET_ITEM(a[0], i));
       x[i] = as_tensor(PyList_GET_ITEM(a[1], i), "x");
@@ -304,22 +329,35 @@ PyObject* py_gemv_batch(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
       if (a[2] != Py_None) b[i] = as_tensor(PyList_GET_ITEM(a[2], i), "bias");
       require_gpu(m, x[i], b[i]);
       d[i] = desc_of(m);
-      r[i] = rows_of(x[i], d[i].N);
+      check_features(x[i], d[i].N);
       if (i == 0) odt = out_type(a[3], x[0]);
-      if (r[i].M != r[0].M || x[i].scalar_type() != x[0].scalar_type())
+      if (x[i].numel() / d[i].N != x[0].numel() / d[0].N || x[i].scalar_type() != x[0].scalar_type())
         fail(PyExc_ValueError, "all activations of a batch share the row count and the dtype");
-      y[i] = out_for(x[i], d[i].K, odt);
-      if (b[i].defined() && b[i].scalar_type() != odt) b[i] = b[i].to(odt);
-      xp[i] = r[i].p; ldx[i] = r[i].ld;
-      yp[i] = y[i].mutable_data_ptr(); ldy[i] = d[i].K;
-      bp[i] = b[i].defined() ? b[i].const_data_ptr() : nullptr;
-      need += cbk::decode_workspace_bytes(&d[i], (int)r[0].M);
     }
-    const c10::DeviceGuard guard(x[0].device());
-    const at::Tensor ws = scratch(x[0], need);
-    check(cbk_gemv_batch((int)n, d, xp, ldx, dtype_code(x[0].scalar_type()), (int)r[0].M, yp, ldy, dtype_code(odt), bp,
-                         ws.defined() ? ws.mutable_data_ptr() : nullptr, need, stream_of(x[0])),
-          "cbk_gemv_batch");
+    const int xdt = dtype_code(x[0].scalar_type()), ydt = dtype_code(odt);
+    int rc = CBK_OK;
+    {
+      const GilRelease other_threads_run;
+      Rows r[8];
+      const void *xp[8], *bp[8];
+      void* yp[8];
+      int64_t ldx[8], ldy[8];
+      size_t need = 0;
+      for (Py_ssize_t i = 0; i < n; ++i) {
+        r[i] = rows_of(x[i], d[i].N);
+        y[i] = out_for(x[i], d[i].K, odt);
+        if (b[i].defined() && b[i].scalar_type() != odt) b[i] = b[i].to(odt);
+        xp[i] = r[i].p; ldx[i] = r[i].ld;
+        yp[i] = y[i].mutable_data_ptr(); ldy[i] = d[i].K;
+        bp[i] = b[i].defined() ? b[i].const_data_ptr() : nullptr;
+        need += cbk::decode_workspace_bytes(&d[i], (int)r[0].M);
+      }
+      const c10::DeviceGuard guard(x[0].device());
+      const at::Tensor ws = scratch(x[0], need);
+      rc = cbk_gemv_batch((int)n, d, xp, ldx, xdt, (int)r[0].M, yp, ldy, ydt, bp,
+                          ws.defined() ? ws.mutable_data_ptr() : nullptr, need, stream_of(x[0]));
+    }
+    check(rc, "cbk_gemv_batch");
     PyObject* out = PyList_New(n);
     if (!out) throw Fail{};
     for (Py_ssize_t i = 0; i < n; ++i) PyList_SET_ITEM(out, i, THPVariable_Wrap(y[i]));
@@ -343,49 +381,56 @@ PyObject* py_pack_begin(PyObject*, PyObject* const* a, Py_ssize_t n) {
     d.group = (int)PyLong_AsLong(a[7]); d.keep = (int)PyLong_AsLong(a[8]);
     const bool fix = PyObject_IsTrue(a[9]), tiled = PyObject_IsTrue(a[10]);
     if (PyErr_Occurred()) throw Fail{};
-    const at::Device dev = q.device();
-    const c10::DeviceGuard guard(dev);
-    const int64_t K = q.size(0), N = q.size(1), G = N / d.group;
-    d.K = (int32_t)K; d.N = (int32_t)N; d.flags = tiled ? CBK_FLAG_TILED16 : 0;
-    q = (q.scalar_type() == at::kByte ? q : q.clamp(0, 255).to(at::kByte)).contiguous();
-    if (mask.defined()) mask = mask.to(dev).reshape({K, N / 8}).contiguous();
-    scale = scale.to(dev, at::kHalf).reshape({K, G}).contiguous();
-    zero = zero.to(dev).reshape({K, G});
-    zero = (zero.scalar_type() == at::kByte ? zero : zero.to(at::kHalf)).contiguous();
-    int64_t cs_rows = 0;
-    if (cs.defined()) {
-      cs = cs.to(dev, at::kHalf).reshape({-1, N}).contiguous();
-      if ((uintptr_t)cs.const_data_ptr() & 15) cs = cs.clone(at::MemoryFormat::Contiguous);
-      cs_rows = cs.size(0);
+    const int64_t K = q.size(0), N = q.size(1), G = N / d.group, kr = tiled ? (K + 15) / 16 * 16 : K;
+    int64_t cs_rows = 0, off[4] = {0, 0, 0, -1}, stride = 0;
+    at::Tensor blob, host;
+    int rc = CBK_OK;
+    {
+      const GilRelease other_threads_run;
+      const at::Device dev = q.device();
+      const c10::DeviceGuard guard(dev);
+      d.K = (int32_t)K; d.N = (int32_t)N; d.flags = tiled ? CBK_FLAG_TILED16 : 0;
+      q = (q.scalar_type() == at::kByte ? q : q.clamp(0, 255).to(at::kByte)).contiguous();
+      if (mask.defined()) mask = mask.to(dev).reshape({K, N / 8}).contiguous();
+      scale = scale.to(dev, at::kHalf).reshape({K, G}).contiguous();
+      zero = zero.to(dev).reshape({K, G});
+      zero = (zero.scalar_type() == at::kByte ? zero : zero.to(at::kHalf)).contiguous();
+      if (cs.defined()) {
+        cs = cs.to(dev, at::kHalf).reshape({-1, N}).contiguous();
+        if ((uintptr_t)cs.const_data_ptr() & 15) cs = cs.clone(at::MemoryFormat::Contiguous);
+        cs_rows = cs.size(0);
+      }
+      // the packing kernel reads q with 16-byte and the mask with 4-byte loads
+      if ((uintptr_t)q.const_data_ptr() & 15) q = q.clone(at::MemoryFormat::Contiguous);
+      if (mask.defined() && ((uintptr_t)mask.const_data_ptr() & 3)) mask = mask.clone(at::MemoryFormat::Contiguous);
+      stride = (int64_t)cbk_row_stride(&d);
+      const int64_t size[4] = {kr * stride + (tiled ? 512 : 64), kr * G * 2, kr * G, cs_rows * N * 2};
+      const int na = cs_rows ? 4 : 3;
+      int64_t pos = 0;
+      cbk::PackExtra x{};
+      for (int i = 0; i < na; ++i) { off[i] = pos; pos = (pos + size[i] + 255) / 256 * 256; }
+      const at::TensorOptions bytes = at::TensorOptions().dtype(at::kByte).device(dev);
+      blob = at::empty({pos}, bytes);
+      uint8_t* base = (uint8_t*)blob.mutable_data_ptr();
+      for (int i = 0; i < na; ++i) {
+        x.gap[i] = base + off[i] + size[i];
+        x.gap_bytes[i] = (uint32_t)((i + 1 < na ? off[i + 1] : pos) - off[i] - size[i]);
+      }
+      d.data = base + off[0]; d.scale = base + off[1]; d.zero = base + off[2];
+      if (cs_rows) {
+        x.cs_src = cs.const_data_ptr(); x.cs_dst = base + off[3]; x.cs_units = (uint32_t)(size[3] / 16);
+      }
+      at::Tensor counts = at::zeros({cbk::PACK_SLOTS * cbk::PACK_SLOT_WORDS}, bytes.dtype(at::kInt));
+      x.counts = (uint32_t*)counts.mutable_data_ptr();
+      rc = cbk::pack_image(&d, mask.defined() ? mask.const_data_ptr() : nullptr, q.const_data_ptr(), scale.const_data_ptr(),
+                           zero.const_data_ptr(), zero.scalar_type() == at::kByte ? CBK_U8 : CBK_F16, fix ? 1 : 0, nullptr, &x,
+                           stream_of(q));
+      if (rc == CBK_OK) {
+        host = at::empty(counts.sizes(), at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+        host.copy_(counts, true);
+      }
     }
-    // the packing kernel reads q with 16-byte and the mask with 4-byte loads
-    if ((uintptr_t)q.const_data_ptr() & 15) q = q.clone(at::MemoryFormat::Contiguous);
-    if (mask.defined() && ((uintptr_t)mask.const_data_ptr() & 3)) mask = mask.clone(at::MemoryFormat::Contiguous);
-    const int64_t kr = tiled ? (K + 15) / 16 * 16 : K, stride = (int64_t)cbk_row_stride(&d);
-    const int64_t size[4] = {kr * stride + (tiled ? 512 : 64), kr * G * 2, kr * G, cs_rows * N * 2};
-    const int na = cs_rows ? 4 : 3;
-    int64_t off[4] = {0, 0, 0, -1}, pos = 0;
-    cbk::PackExtra x{};
-    for (int i = 0; i < na; ++i) { off[i] = pos; pos = (pos + size[i] + 255) / 256 * 256; }
-    const at::TensorOptions bytes = at::TensorOptions().dtype(at::kByte).device(dev);
-    at::Tensor blob = at::empty({pos}, bytes);
-    uint8_t* base = (uint8_t*)blob.mutable_data_ptr();
-    for (int i = 0; i < na; ++i) {
-      x.gap[i] = base + off[i] + size[i];
-      x.gap_bytes[i] = (uint32_t)((i + 1 < na ? off[i + 1] : pos) - off[i] - size[i]);
-    }
-    d.data = base + off[0]; d.scale = base + off[1]; d.zero = base + off[2];
-    if (cs_rows) {
-      x.cs_src = cs.const_data_ptr(); x.cs_dst = base + off[3]; x.cs_units = (uint32_t)(size[3] / 16);
-    }
-    at::Tensor counts = at::zeros({cbk::PACK_SLOTS * cbk::PACK_SLOT_WORDS}, bytes.dtype(at::kInt));
-    x.counts = (uint32_t*)counts.mutable_data_ptr();
-    check(cbk::pack_image(&d, mask.defined() ? mask.const_data_ptr() : nullptr, q.const_data_ptr(), scale.const_data_ptr(),
-                          zero.const_data_ptr(), zero.scalar_type() == at::kByte ? CBK_U8 : CBK_F16, fix ? 1 : 0, nullptr, &x,
-                          stream_of(q)),
-          "cbk_pack");
-    at::Tensor host = at::empty(counts.sizes(), at::TensorOptions().dtype(at::kInt).pinned_memory(true));
-    host.copy_(counts, true);
+    check(rc, "cbk_pack");
     return Py_BuildValue("N(LLLL)LLN", THPVariable_Wrap(blob), (long long)off[0], (long long)off[1], (long long)off[2],
                          (long long)off[3], (long long)cs_rows, (long long)(kr * stride),
                          THPVariable_Wrap(host));

@@ -185,3 +185,45 @@ def test_directory_written_by_the_reference_loads_and_runs():
         assert float((gu - ref).abs().max() / ref.abs().max()) < (2e-5 if M < 8 else 2e-3)
     rep = Ct.check_container(os.path.join(gold, "cbk1_dir"), device=DEV)
     assert rep["ok"] and rep["matrices"]["0:gateup"]["pruned_nonzero"] == 0
+
+
+@pytest.mark.parametrize("op", ["linear", "linear_act", "gemv_batch", "dequant", "pack"])
+def test_operators_let_other_threads_run(op):
+    """An operator gives up the interpreter lock while it allocates and launches: with a switch interval no
+    run reaches, another thread moves on only because the calls of this one let go of the lock."""
+    import sys
+    import threading
+    import time
+    from cobalt_amd import format as F, ops
+    pm = F.synth_packed(64, 256, F.BLK1632_4, 4, 128, 16, seed=1, device=DEV)
+    x = torch.randn(4, 256, device=DEV).half()
+    raw = dict(mask_bits=None, q=torch.zeros(64, 256, dtype=torch.uint8, device=DEV), scale=torch.ones(64, 2, device=DEV).half(),
+               zero=torch.zeros(64, 2, dtype=torch.uint8, device=DEV), col_scale=None, layout=F.DENSE4)
+    call = {"linear": lambda: ops.linear(pm, x), "linear_act": lambda: ops.linear_act(pm, x, "silu"),
+            "gemv_batch": lambda: ops.gemv_batch([pm, pm], [x, x]), "dequant": lambda: ops.dequant(pm),
+            "pack": lambda: ops.PackJob(**raw)}[op]
+    call()
+    torch.cuda.synchronize()
+    turns, stop, kept = [0], [False], []                              # (freeing a tensor lets go of the lock as well)
+
+    def other():
+        while not stop[0]:
+            turns[0] += 1
+            time.sleep(0)                                             # waits for the lock again
+
+    t = threading.Thread(target=other)
+    old = sys.getswitchinterval()
+    sys.setswitchinterval(1000.0)
+    try:
+        t.start()
+        start = turns[0]
+        for _ in range(5000 if op != "pack" else 1000):
+            kept.append(call())
+            if turns[0] > start + 3:
+                break
+        seen = turns[0] - start
+    finally:
+        sys.setswitchinterval(old)
+        stop[0] = True
+        t.join()
+    assert seen > 3
