@@ -573,15 +573,18 @@ static GemmPlan act_plan(const DMat& m, int M) {
   return p.kernel == GEMM_TILE && m.cs_rows != 2 ? GemmPlan() : p;
 }
 
-size_t cbk_linear_act_workspace_bytes(const cbk_desc* in, int M, int y_dtype) {
-  DMat m;
-  if (M < 1 || to_dmat(in, &m, false)) return 0;
-  const GemmPlan p = act_plan(m, M);
+static size_t act_workspace(const DMat& m, const GemmPlan& p, int M, int y_dtype) {
   return p.kernel == GEMM_ROWS ? p.bytes : act_mid_bytes(m.K, M, y_dtype) + (p.kernel ? p.bytes : workspace_of(m, M));
 }
 
-int cbk_linear_act(const cbk_desc* in, const void* x, int x_dtype, int M, int64_t ldx, void* y, int y_dtype,
-                   int64_t ldy, const void* bias, int act, void* workspace, size_t workspace_bytes, void* stream) {
+size_t cbk_linear_act_workspace_bytes(const cbk_desc* in, int M, int y_dtype) {
+  DMat m;
+  if (M < 1 || to_dmat(in, &m, false)) return 0;
+  return act_workspace(m, act_plan(m, M), M, y_dtype);
+}
+
+static int linear_act_on(const cbk_desc* in, const GemmPlan* named, const void* x, int x_dtype, int M, int64_t ldx, void* y, int y_dtype,
+                         int64_t ldy, const void* bias, int act, void* workspace, size_t workspace_bytes, void* stream) {
   DMat m;
   int rc = to_dmat(in, &m, true);
   if (rc) return rc;
@@ -591,9 +594,9 @@ int cbk_linear_act(const cbk_desc* in, const void* x, int x_dtype, int M, int64_
   if (!y) return CBK_ERR_NULL;
   if (M < 1 || ldy < m.K / 2) return CBK_ERR_SHAPE;
   if ((uintptr_t)y & (y_dtype == CBK_F32 ? 3 : 1)) return CBK_ERR_ALIGN;
-  if (!workspace || ((uintptr_t)workspace & 255) || workspace_bytes < cbk_linear_act_workspace_bytes(in, M, y_dtype))
+  const GemmPlan plan = named ? *named : act_plan(m, M);
+  if (!workspace || ((uintptr_t)workspace & 255) || workspace_bytes < act_workspace(m, plan, M, y_dtype))
     return CBK_ERR_WORKSPACE;
-  const GemmPlan plan = act_plan(m, M);
   if (plan.kernel == GEMM_ROWS) {
     rc = check_io(x, x_dtype, M, ldx, y, y_dtype, ldy, m.N, m.K / 2);
     if (rc) return rc;
@@ -618,4 +621,45 @@ int cbk_linear_act(const cbk_desc* in, const void* x, int x_dtype, int M, int64_
   return launch_act_mul(workspace, tdt, m.K, y, y_dtype, ldy, M, m.K / 2, act, bias, (hipStream_t)stream);
 }
 
+int cbk_linear_act(const cbk_desc* in, const void* x, int x_dtype, int M, int64_t ldx, void* y, int y_dtype,
+                   int64_t ldy, const void* bias, int act, void* workspace, size_t workspace_bytes, void* stream) {
+  return linear_act_on(in, nullptr, x, x_dtype, M, ldx, y, y_dtype, ldy, bias, act, workspace, workspace_bytes, stream);
+}
+
 }  // extern "C"
+
+namespace cbk {
+
+static GemmPlan named_plan(const DMat& m, int M, const GemmChoice& c) {
+  return c.kernel == GEMM_ROWS ? fixed_plan_skinny(m, M, c.ti, c.nsplit)
+       : c.kernel == GEMM_TILE ? fixed_plan_big(m, M, c.ti, c.nsplit) : GemmPlan();
+}
+
+GemmChoice gemm_choice(const cbk_desc* in, int M, int act) {
+  DMat m;
+  if (M < 1 || to_dmat(in, &m, false) || family_of(m.layout) == FAM_SPARSE) return {GEMM_NONE, 0, 0};
+  const GemmPlan p = act >= 0 ? act_plan(m, M) : gemm_plan(m, M, false, gemm_room(m, M));
+  return {p.kernel, p.ti, p.nsplit};
+}
+
+size_t gemm_as_workspace_bytes(const cbk_desc* in, int M, const GemmChoice& c, int act, int y_dtype) {
+  DMat m;
+  if (M < 1 || to_dmat(in, &m, false)) return 0;
+  const GemmPlan p = named_plan(m, M, c);
+  return !p.kernel ? 0 : act >= 0 ? act_workspace(m, p, M, y_dtype) : p.bytes;
+}
+
+int gemm_as(const cbk_desc* in, const GemmChoice& c, const void* x, int x_dtype, int M, int64_t ldx, void* y, int y_dtype,
+            int64_t ldy, const void* bias, int act, void* workspace, size_t workspace_bytes, void* stream) {
+  DMat m;
+  int rc = to_dmat(in, &m, true);
+  if (rc) return rc;
+  const GemmPlan p = named_plan(m, M, c);
+  if (!p.kernel || (act >= 0 && p.kernel == GEMM_TILE && m.cs_rows != 2)) return CBK_ERR_UNSUPPORTED;
+  if (act >= 0)
+    return linear_act_on(in, &p, x, x_dtype, M, ldx, y, y_dtype, ldy, bias, act, workspace, workspace_bytes, stream);
+  rc = check_io(x, x_dtype, M, ldx, y, y_dtype, ldy, m.N, m.K);
+  return rc ? rc : run_gemm(m, p, x, x_dtype, M, ldx, y, y_dtype, ldy, bias, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+}  // namespace cbk

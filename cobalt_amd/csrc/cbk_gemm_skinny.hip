@@ -206,7 +206,7 @@ GemmPlan plan_skinny(const DMat& m, int M, size_t room) {
 }
 GemmPlan fixed_plan_skinny(const DMat& m, int M, int ti, int nsplit) {
   GemmPlan p;
-  if (M < 1 || !gemm_skinny_takes(m) || ti < 1 || ti > 3 || nsplit < 1 || nsplit > 16) return p;
+  if (M < 1 || !gemm_skinny_takes(m) || ti < 1 || ti > 3 || nsplit < 1 || nsplit > 16 || SK_WC * (nsplit - 1) >= m.G) return p;
   p.kernel = GEMM_ROWS; p.ti = ti; p.nsplit = nsplit; p.bytes = sk_sum(sk_space(m, M, ti, nsplit));
   return p;
 }

@@ -9,6 +9,16 @@ namespace cbk {
 // What cbk_gemv uses of a workspace at M rows (cbk_workspace_bytes covers every entry point).
 size_t decode_workspace_bytes(const cbk_desc*, int M);
 
+// How a prefill call runs, and the same call on a kernel, token tile and split of the columns that the caller
+// names: for tests, which have to know which of the instantiations they run.  kernel: 0 none of the two (cbk_linear in a gated
+// call), 1 the kernel of cbk_gemm_skinny.h (32 ti tokens, ti 1 - 3), 2 that of cbk_gemm_big.h (64 ti tokens, ti 1 / 2 / 4).
+// act: -1 for cbk_gemm, an activation for cbk_linear_act (y_dtype counts only there).
+struct GemmChoice { int kernel, ti, nsplit; };
+GemmChoice gemm_choice(const cbk_desc*, int M, int act);
+size_t gemm_as_workspace_bytes(const cbk_desc*, int M, const GemmChoice&, int act, int y_dtype);   // 0: it cannot be run so
+int gemm_as(const cbk_desc*, const GemmChoice&, const void* x, int x_dtype, int M, int64_t ldx, void* y, int y_dtype, int64_t ldy,
+            const void* bias, int act, void* workspace, size_t workspace_bytes, void* stream);
+
 // The rest of a module's image, written by the packing kernel along with the rows: the column
 // scales, the bytes between the arrays (zero), and two figures about what was packed.
 constexpr int PACK_SLOTS = 64, PACK_SLOT_WORDS = 16;

@@ -282,6 +282,51 @@ PyObject* py_linear_act(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// gemm_plan(matrix, M, act or -1) -> (kernel, ti, nsplit); see cbk::gemm_choice
+PyObject* py_gemm_plan(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (!arity(n, 3)) return nullptr;
+  return guarded([&]() -> PyObject* {
+    const cbk_desc d = desc_of(as_matrix(a[0]));
+    const long M = PyLong_AsLong(a[1]), act = PyLong_AsLong(a[2]);
+    if (PyErr_Occurred()) throw Fail{};
+    const cbk::GemmChoice c = cbk::gemm_choice(&d, (int)M, (int)act);
+    return Py_BuildValue("iii", c.kernel, c.ti, c.nsplit);
+  });
+}
+
+// gemm_as(matrix, x, bias, out_dtype, kernel, ti, nsplit, act or -1) -> y; see cbk::gemm_as
+PyObject* py_gemm_as(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (!arity(n, 8)) return nullptr;
+  return guarded([&]() -> PyObject* {
+    const Matrix* m = as_matrix(a[0]);
+    const at::Tensor x = as_tensor(a[1], "x"), bias = as_tensor(a[2], "bias");
+    if (!x.defined() || !x.numel()) fail(PyExc_TypeError, "x must be a tensor with elements");
+    require_gpu(m, x, bias);
+    const cbk_desc d = desc_of(m);
+    check_features(x, d.N);
+    const at::ScalarType odt = out_type(a[3], x);
+    const int xdt = dtype_code(x.scalar_type()), ydt = dtype_code(odt);
+    const cbk::GemmChoice c{(int)PyLong_AsLong(a[4]), (int)PyLong_AsLong(a[5]), (int)PyLong_AsLong(a[6])};
+    const int act = (int)PyLong_AsLong(a[7]), Ko = act >= 0 ? d.K / 2 : d.K;
+    if (PyErr_Occurred()) throw Fail{};
+    if (bias.defined() && bias.scalar_type() != odt) fail(PyExc_TypeError, "the bias must have the output's type");
+    at::Tensor y;
+    int rc = CBK_OK;
+    {
+      const GilRelease other_threads_run;
+      const Rows r = rows_of(x, d.N);
+      y = out_for(x, Ko, odt);
+      const c10::DeviceGuard guard(x.device());
+      const at::Tensor ws = scratch(x, cbk::gemm_as_workspace_bytes(&d, (int)r.M, c, act, ydt));
+      rc = cbk::gemm_as(&d, c, r.p, xdt, (int)r.M, r.ld, y.mutable_data_ptr(), ydt, Ko,
+                        bias.defined() ? bias.const_data_ptr() : nullptr, act, ws.defined() ? ws.mutable_data_ptr() : nullptr,
+                        ws.defined() ? ws.nbytes() : 0, stream_of(x));
+    }
+    check(rc, "cbk::gemm_as");
+    return THPVariable_Wrap(y);
+  });
+}
+
 // dequant(matrix, dtype, row0, nrows, with_col_scale) -> W_hat[row0 : row0 + nrows]
 PyObject* py_dequant(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!arity(n, 5)) return nullptr;
@@ -468,6 +513,8 @@ PyMethodDef methods[] = {
     {"matmul", (PyCFunction)(void (*)())py_matmul, METH_FASTCALL, nullptr},
     {"linear_act", (PyCFunction)(void (*)())py_linear_act, METH_FASTCALL, nullptr},
     {"gemv_batch", (PyCFunction)(void (*)())py_gemv_batch, METH_FASTCALL, nullptr},
+    {"gemm_plan", (PyCFunction)(void (*)())py_gemm_plan, METH_FASTCALL, nullptr},
+    {"gemm_as", (PyCFunction)(void (*)())py_gemm_as, METH_FASTCALL, nullptr},
     {"dequant", (PyCFunction)(void (*)())py_dequant, METH_FASTCALL, nullptr},
     {"pack_begin", (PyCFunction)(void (*)())py_pack_begin, METH_FASTCALL, nullptr},
     {"pack_end", (PyCFunction)(void (*)())py_pack_end, METH_FASTCALL, nullptr},

@@ -3,7 +3,7 @@ import numpy as np
 import torch
 
 from oracle import cbk_ref as R
-from cobalt_amd import format as F
+from cobalt_amd import _lib, format as F
 
 # (layout, bits, group, keep) of every fixed-stride case the kernels take
 FIXED_CASES = [
@@ -73,3 +73,22 @@ def rel_fro(y, ref):
 def acts(M, N, dtype, seed, scale=1.0):
     g = torch.Generator().manual_seed(seed)
     return (torch.randn(M, N, generator=g) * scale).to(dtype)
+
+
+# The two prefill kernels by name: "rows" (cbk_gemm_skinny.h, tiles of 32, 64 and 96 tokens) and "tile"
+# (cbk_gemm_big.h, 64, 128 and 256 tokens).  A test that is about one of them names it; what a plain call
+# runs on is the library's choice.
+KERNELS = {"rows": 1, "tile": 2}
+TOKENS = {"rows": (32, 64, 96), "tile": (64, 128, 256)}
+
+
+def gemm_as(pm, x, kernel, tokens, nsplit=1, bias=None, out_dtype=None, act=None):
+    """ops.gemm (act: ops.linear_act) on the named kernel, token tile and split of the column range."""
+    return _lib.native().gemm_as(pm.native(), x, bias, out_dtype, KERNELS[kernel], tokens // (32 if kernel == "rows" else 64), nsplit,
+                                 -1 if act is None else _lib.ACT_CODE[act])
+
+
+def gemm_plan(pm, M, act=None):
+    """(kernel, tokens, nsplit) the library runs such a call on; (None, 0, 0): neither."""
+    k, ti, s = _lib.native().gemm_plan(pm.native(), M, -1 if act is None else _lib.ACT_CODE[act])
+    return {0: None, 1: "rows", 2: "tile"}[k], ti * (32 if k == 1 else 64), s

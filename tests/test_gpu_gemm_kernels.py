@@ -1,0 +1,112 @@
+"""Every instantiation of the two prefill kernels by name: code configuration x token tile x column-scale vectors
+(plain, gate/up, q|k|v) x split of the column range x byte order, for activations of both signs and of one.
+Against float64 on the dequantised weights, held to the error of operands of 11 bits in exact sums (2 % for
+float32 sums and the draw); every call twice, bit for bit."""
+import pytest
+import torch
+
+from cobalt_amd import _lib, format as F, ops
+from helpers import TOKENS, acts, case_id, gemm_as, gemm_plan
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+CASES = [(F.BLK1632_6, 6, 128, 16), (F.DENSEB, 8, 64, 0), (F.DENSE8, 8, 128, 0)] + [
+    (F.BLKC if k else F.DENSEB, b, g, k) for b in (2, 3, 4) for k in (0, 10, 16, 23) for g in (64, 128)]
+# (kernel, splits of the column range): 13 groups of 128 columns are 28 stages of the tile kernel
+SPLITS = {"rows": (1, 2, 3), "tile": (1, 2)}
+
+
+def _matrix(case, vectors, N, seed):
+    mk = lambda k, s: F.synth_packed(k, N, case[0], case[1], case[2], case[3] or None, seed=seed + s, device=DEV)
+    if vectors == 1:
+        return mk(267, 0)                                             # two row tiles of 128, ragged
+    if vectors == 2:
+        return F.fuse_rows([mk(131, 0), mk(131, 1)], interleave=True)
+    return F.fuse_rows([mk(256, 0), mk(256, 1), mk(57, 2)])           # ranges on the row tiles of both kernels
+
+
+def _vectors_of_rows(pm):
+    k = torch.arange(pm.K, device=DEV)
+    return k * 0 if pm.cs_rows == 1 else k % 2 if pm.cs_rows == 2 else (k >= pm.cs_splits[0]).long() + (k >= sum(pm.cs_splits)).long()
+
+
+@pytest.mark.parametrize("vectors", [1, 2, 3], ids=["plain", "gate_up", "qkv"])
+@pytest.mark.parametrize("case", CASES, ids=case_id)
+def test_every_instantiation(case, vectors):
+    N = 1664
+    rows = _matrix(case, vectors, N, seed=vectors)
+    W = ops.dequant(rows, torch.float32).double()
+    Wh = ops.dequant(rows, torch.float32, with_col_scale=False).half().double()
+    cs = rows.array("col_scale").view(rows.cs_rows, N).float()
+    vec = _vectors_of_rows(rows)
+    x257 = acts(257, N, torch.float16, seed=case[1]).to(DEV)
+    ran = set()
+    for one_sign in (False, True):
+        x = x257.abs() if one_sign else x257
+        ref = x.double() @ W.t()
+        each = torch.stack([(x.float() * c).half().double() @ Wh.t() for c in cs])       # [vectors, 257, K]
+        rounded = each.gather(0, vec.view(1, 1, -1).expand(1, *ref.shape))[0]
+        for pm in (rows, rows.to_tiled()):
+            for kernel, tiles in TOKENS.items():
+                for tokens in tiles:
+                    M = tokens + 1                                      # a whole tile and one token
+                    bound = float((rounded[:M] - ref[:M]).norm() / ref[:M].norm())
+                    for s in SPLITS[kernel]:
+                        if kernel == "tile" and s > 1 and (vectors == 2 or case[1] == 8):
+                            with pytest.raises(_lib.CbkError):             # gate/up and 8-bit codes are not split there
+                                gemm_as(pm, x[:M], kernel, tokens, s)
+                            continue
+                        y = gemm_as(pm, x[:M], kernel, tokens, s, out_dtype=torch.float32)
+                        err = float((y.double() - ref[:M]).norm() / ref[:M].norm())
+                        assert err <= 1.02 * bound, (kernel, tokens, s, pm is rows, one_sign, err, bound)
+                        assert torch.equal(y, gemm_as(pm, x[:M], kernel, tokens, s, out_dtype=torch.float32)), (kernel, tokens, s)
+                        ran.add((kernel, tokens, s))
+    assert len(ran) == 9 + (3 if vectors == 2 or case[1] == 8 else 6)
+
+
+@pytest.mark.parametrize("act", ["gelu_tanh", "silu"])
+@pytest.mark.parametrize("case", [c for c in CASES if c[2:] in ((128, 16), (64, 10), (128, 0))], ids=case_id)
+def test_gated_call_on_every_tile(case, act):
+    """act(gate) * up where the column parts meet (rows kernel, also over workgroups: the reduction kernel) and
+    from the two halves the tile kernel leaves.  float32 results, the float64 product of the dequantised weights;
+    gate and up carry 3e-4 each, the activations have slopes up to 1.1."""
+    N = 1664
+    pm = _matrix(case, 2, N, seed=9).to_tiled()
+    W = ops.dequant(pm, torch.float32).double()
+    x = acts(257, N, torch.float16, seed=3).to(DEV)
+    bias = acts(1, pm.K, torch.float32, seed=4)[0].to(DEV)
+    t = x.double() @ W.t() + bias.double()
+    g, u = t[:, 0::2], t[:, 1::2]
+    ref = (torch.nn.functional.gelu(g, approximate="tanh") if act == "gelu_tanh" else torch.nn.functional.silu(g)) * u
+    for kernel, tiles in TOKENS.items():
+        for tokens in tiles:
+            M = tokens + 1
+            for s in (1, 2, 3) if kernel == "rows" else (1,):
+                y = gemm_as(pm, x[:M], kernel, tokens, s, bias=bias, out_dtype=torch.float32, act=act)
+                assert y.shape == (M, pm.K // 2)
+                assert float((y.double() - ref[:M]).norm() / ref[:M].norm()) < 1e-3, (kernel, tokens, s)
+                assert torch.equal(y, gemm_as(pm, x[:M], kernel, tokens, s, bias=bias, out_dtype=torch.float32, act=act))
+                yh = gemm_as(pm, x[:M], kernel, tokens, s, bias=bias.bfloat16(), out_dtype=torch.bfloat16, act=act)
+                assert float((yh.double() - ref[:M]).norm() / ref[:M].norm()) < (4e-3 if M <= 128 or kernel == "rows" else 8e-3)
+
+
+def test_a_plain_call_is_the_call_its_plan_names():
+    """What `ops.gemm` and `ops.linear_act` return is the named kernel's result, over sizes that meet both
+    kernels, every token tile and splits."""
+    seen = set()
+    for case, K, N, vectors in (((F.BLK1632_4, 4, 128, 16), 640, 14336, 1), ((F.BLK1632_4, 4, 128, 16), 14336, 4096, 1),
+                                ((F.BLKC, 2, 64, 16), 3072, 4096, 3), ((F.DENSE8, 8, 128, 0), 1024, 5376, 1),
+                                ((F.BLK1632_6, 6, 128, 16), 4096, 4096, 1), ((F.BLKC, 3, 128, 10), 6400, 2048, 2)):
+        mk = lambda k, s: F.synth_packed(k, N, case[0], case[1], case[2], case[3] or None, seed=s, device=DEV)
+        pm = (mk(K, 1) if vectors == 1 else F.fuse_rows([mk(K, 1), mk(K, 2)], interleave=True) if vectors == 2
+              else F.fuse_rows([mk(K // 2, 1), mk(K // 4, 2), mk(K // 4, 3)])).to_tiled()
+        for M in (9, 40, 64, 90, 128, 200, 333, 500, 1100):
+            x = acts(M, N, torch.float16, seed=M).to(DEV)
+            plan = gemm_plan(pm, M)
+            assert torch.equal(ops.gemm(pm, x), gemm_as(pm, x, *plan)), (case, M, plan)
+            seen.add(plan[:2] + (plan[2] > 1,))
+            if vectors == 2:
+                plan = gemm_plan(pm, M, "silu")
+                assert torch.equal(ops.linear_act(pm, x, "silu"), gemm_as(pm, x, *plan, act="silu")), (case, M, plan)
+    kinds = {k[:2] for k in seen}
+    assert {("rows", 32), ("rows", 64), ("rows", 96), ("tile", 256)} <= kinds and {k[2] for k in seen} == {False, True}, sorted(seen)

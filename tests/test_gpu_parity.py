@@ -12,8 +12,8 @@ from oracle import cbk_ref as R
 from cobalt_amd import format as F
 from cobalt_amd import _lib, ops
 from cobalt_amd.linear import CobaltLinear
-from helpers import (FIXED_CASES, SPARSE_CASES, acts, case_id, kw_of, make_raw, oracle_pack, packed_from_oracle,
-                     product_pack, rel_fro)
+from helpers import (FIXED_CASES, SPARSE_CASES, TOKENS, acts, case_id, gemm_as, kw_of, make_raw, oracle_pack,
+                     packed_from_oracle, product_pack, rel_fro)
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -517,8 +517,9 @@ def test_gemv_five_to_eight_rows_equal_single_rows(case):
 
 @pytest.mark.parametrize("case", FIXED_CASES, ids=case_id)
 def test_gemm_repeats_and_is_exact_to_its_operands(case):
-    """Every token tile and split of the two prefill kernels, several times over: the same bits each
-    time, and the error of operands of 11 bits."""
+    """Long and short rows at 20 to 700 activation rows on the plans the library picks for them (several tiles
+    and splits of the kernel for few rows), several times over: the same bits each time, and the
+    error of operands of 11 bits."""
     for (K, N) in ((640, 14336), (1024, 5376), (2048, 14336)):
         pm = F.synth_packed(K, N, case[0], case[1], case[2], case[3] or None, seed=3, device=DEV).to_tiled()
         W = ops.dequant(pm, torch.float32).double()
@@ -534,7 +535,7 @@ def test_gemm_repeats_and_is_exact_to_its_operands(case):
 @pytest.mark.parametrize("case", [(F.BLK1632_4, 4, 128, 16), (F.DENSE8, 8, 128, 0), (F.BLKC, 3, 64, 10)], ids=case_id)
 @pytest.mark.parametrize("K,N,M", [(512, 2048, 2000), (130, 1152, 1111), (1000, 512, 3001)])
 def test_gemm_of_many_token_tiles_and_few_row_tiles(case, K, N, M):
-    """Calls whose token tiles are walked in bands, the last one shorter: every tile exactly once."""
+    """A thousand and more tokens over one to eight row tiles, the last of both ragged: every tile exactly once."""
     pm = F.synth_packed(K, N, case[0], case[1], case[2], case[3] or None, seed=K, device=DEV).to_tiled()
     x = acts(M, N, torch.float16, seed=M).to(DEV)
     ref = x.double() @ ops.dequant(pm, torch.float32).double().t()
@@ -731,8 +732,9 @@ def test_gemv_fused_rows_equal_their_unfused_parts_bit_for_bit():
 
 @pytest.mark.parametrize("case", FUSED_CASES[:2] + FUSED_CASES[4:], ids=case_id)
 def test_gemm_fused_col_scale_rows(case):
-    """Prefill on fused matrices: q|k|v ranges run the 256 x 256 kernel range by range, gate/up
-    (row parity) as workgroups of one parity; ranges off the 16-row grid the 128 x 128 kernel."""
+    """Prefill on fused matrices: q|k|v ranges whole where they fit the row tiles of a kernel, else range
+    by range, gate/up (row parity) as workgroups of one parity; ranges off the 16-row grid on the 128 x 128
+    kernel.  What a plain call takes, and the tile kernel by name where it takes the matrix whole."""
     K, N = 640, 1024
     # (40, 24): ranges off the 16-row grid, which only the 128 x 128 fallback kernel takes
     for cs_rows, splits in ((3, (256, 128)), (3, (48, 16)), (3, (40, 24)), (2, (0, 0))):
@@ -744,6 +746,10 @@ def test_gemm_fused_col_scale_rows(case):
             y = ops.gemm(pm, x.to(DEV), bias=bias.to(DEV), out_dtype=torch.float32)
             err = rel_fro(_np(y), ref)
             assert err < TOL, f"{case_id(case)} cs_rows={cs_rows} splits={splits} M={M}: {err}"
+            if cs_rows == 2:
+                for tokens in TOKENS["tile"]:
+                    y = gemm_as(pm, x.to(DEV), "tile", tokens, bias=bias.to(DEV), out_dtype=torch.float32)
+                    assert rel_fro(_np(y), ref) < TOL, f"{case_id(case)} M={M} {tokens} tokens"
 
 
 def _gated_ref(t, act):
@@ -781,6 +787,9 @@ def test_linear_act_gated_epilogue(case, act):
         err = rel_fro(_np(y), ref)
         tol = 4e-3 if odt == torch.bfloat16 else TOL
         assert err < tol, f"{case_id(case)} {act} M={M} {dtype}->{odt}: {err}"
+        if M > 8:                                                     # and on the tile kernel, whichever a plain call takes
+            yt = gemm_as(pm, x.to(DEV), "tile", 64 if M <= 64 else 256, bias=None if b is None else b.to(DEV), out_dtype=odt, act=act)
+            assert rel_fro(_np(yt), ref) < tol, f"{case_id(case)} {act} M={M} {dtype}->{odt}"
     # the first half of an MLP equals the two-step form on the same kernels
     x = acts(8, N, torch.float16, seed=3).to(DEV)
     t = ops.linear(pm, x, out_dtype=torch.float32)
@@ -792,8 +801,8 @@ def test_linear_act_gated_epilogue(case, act):
 
 @pytest.mark.parametrize("act", ["gelu_tanh", "silu"])
 def test_linear_act_for_nine_to_128_rows(act):
-    """Between 9 and 128 activation rows (the 64- and 128-token tiles of the matrix kernel, a float32
-    intermediate and one rounding of the result).  Row counts on and off the tile sizes, more than
+    """Between 9 and 128 activation rows: what a plain call takes, and the 64- and 128-token tiles of the tile
+    kernel by name (a float32 intermediate and one rounding of the result).  Row counts on and off the tile sizes, more than
     one row tile with a ragged last one (K = 2 * 331), with and without bias, every output type,
     both byte orders, and a y with a leading dimension beyond K / 2; against the oracle's float64
     gate/up product."""
@@ -817,6 +826,8 @@ def test_linear_act_for_nine_to_128_rows(act):
                 tol = 4e-3 if odt == torch.bfloat16 else TOL
                 assert err < tol, f"{case_id(case)} {act} tiled={tiled} M={M} {dtype}->{odt}: {err}"
                 assert torch.equal(ops.linear_act(pm, x.to(DEV), act, bias=None if b is None else b.to(DEV), out_dtype=odt), y)
+                yt = gemm_as(pm, x.to(DEV), "tile", 64 if M <= 64 else 128, bias=None if b is None else b.to(DEV), out_dtype=odt, act=act)
+                assert rel_fro(_np(yt), ref) < tol, f"{case_id(case)} {act} tiled={tiled} M={M} {dtype}->{odt}"
     # through the C ABI into a y with a leading dimension larger than K / 2: the columns beyond stay untouched
     pm, W = _fused(FUSED_CASES[0], 256, 512, 2, (0, 0), seed=3, tiled=True)
     M, ldy = 20, 136
@@ -867,6 +878,9 @@ def test_gemm_matches_oracle(case, dtype, tiled):
         y = ops.gemm(pm, x.to(DEV), out_dtype=torch.float32)
         err = rel_fro(_np(y), ref)
         assert err < TOL, f"{case_id(case)} M={M}: {err}"
+        for kernel, tokens in (("rows", 96), ("tile", 64), ("tile", 256)):
+            y = gemm_as(pm, x.to(DEV), kernel, tokens, out_dtype=torch.float32)
+            assert rel_fro(_np(y), ref) < TOL, f"{case_id(case)} M={M} {kernel} {tokens}"
 
 
 @pytest.mark.parametrize("cs_rows", [1, 2, 3])
@@ -914,16 +928,22 @@ def test_gemm_odd_chunk_count_and_ragged_tiles(case):
             assert y.dtype == odt and rel_fro(_np(y), ref) < (TOL if odt != torch.bfloat16 else 3e-3)
         xs = torch.zeros(M, N + 8, dtype=torch.float16); xs[:, :N] = x
         assert rel_fro(_np(ops.gemm(pm, xs.to(DEV)[:, :N], out_dtype=torch.float32)), ref) < TOL
-        for m in (1, 37, 64, 65):                               # the 64-token tile, ragged, and just past it
+        for m in (1, 37, 64, 65):                               # a 64-token tile, ragged, and just past it
             y = ops.gemm(pm, x[:m].to(DEV), out_dtype=torch.float32)
             assert rel_fro(_np(y), ref[:m]) < TOL, (m, tiled)
+            y = gemm_as(pm, x[:m].to(DEV), "tile", 64 if m <= 64 else 128, out_dtype=torch.float32)
+            assert rel_fro(_np(y), ref[:m]) < TOL, (m, tiled)
+        for odt in (torch.float32, torch.float16, torch.bfloat16):
+            y = gemm_as(pm, xs.to(DEV)[:, :N], "tile", 256, out_dtype=odt)
+            assert y.dtype == odt and rel_fro(_np(y), ref) < (TOL if odt != torch.bfloat16 else 3e-3)
 
 
 @pytest.mark.parametrize("case", ALL_MFMA_CASES, ids=case_id)
 def test_gemm_every_kernel_configuration(case):
-    """Every instantiation of the prefill kernel's byte-permute decoder (code width x survivors
-    per block x group size, bitmap and dense), both byte orders, five 128-column chunks so that
-    code bits straddle 16-byte units at every skew, run twice."""
+    """Every instantiation of the byte-permute decoders (code width x survivors per block x group
+    size, bitmap and dense) on the tile kernel's 256- and 64-token tiles and on what a plain call takes,
+    both byte orders, five 128-column chunks so that code bits straddle 16-byte units at every
+    skew, run twice."""
     K, N, M = 272, 640, 260
     raw = make_raw(case, K, N, seed=5 * case[1] + case[3])
     pk = oracle_pack(case, raw)
@@ -936,9 +956,13 @@ def test_gemm_every_kernel_configuration(case):
         err = rel_fro(_np(y), ref)
         assert err < TOL, f"{case_id(case)} tiled={tiled}: {err}"
         assert torch.equal(y, ops.gemm(pm, x.to(DEV), out_dtype=torch.float32))
-        y64 = ops.gemm(pm, x[:50].to(DEV), out_dtype=torch.float32)     # the 64-token instantiation
+        y64 = ops.gemm(pm, x[:50].to(DEV), out_dtype=torch.float32)
         assert rel_fro(_np(y64), ref[:50]) < TOL, f"{case_id(case)} tiled={tiled} M=50"
         assert torch.equal(y64, ops.gemm(pm, x[:50].to(DEV), out_dtype=torch.float32))
+        for m, tokens in ((M, 256), (50, 64)):
+            yt = gemm_as(pm, x[:m].to(DEV), "tile", tokens, out_dtype=torch.float32)
+            assert rel_fro(_np(yt), ref[:m]) < TOL, f"{case_id(case)} tiled={tiled} {tokens} tokens"
+            assert torch.equal(yt, gemm_as(pm, x[:m].to(DEV), "tile", tokens, out_dtype=torch.float32))
 
 
 @pytest.mark.parametrize("case", [(F.BLK1632_4, 4, 128, 16), (F.BLKC, 2, 64, 16), (F.BLKC, 3, 128, 23), (F.BLK1632_6, 6, 128, 16),
@@ -948,7 +972,7 @@ def test_gemm_token_tiles_of_32_64_and_96(case):
     64 and 128 and one more or less, one group of columns (fewer than the parts of a row), group counts
     that are no multiple of what is in flight, both byte orders.  Against the oracle's float64 product:
     two roundings to eleven bits, 2^-12 each, give 3e-4, so the layer tolerance holds with room; also for
-    activations of one sign, whose group sums are what 1024 + zero is taken off again from."""
+    activations of one sign, whose group sums are what the codes' offset and the zero point are taken off again from."""
     for K, N, tiled in ((1, 128, True), (63, 384, False), (129, 1152, True), (191, 2304, False)):
         raw = make_raw(case, K, N, seed=K + N)
         pk = oracle_pack(case, raw)
@@ -959,9 +983,10 @@ def test_gemm_token_tiles_of_32_64_and_96(case):
             x = acts(M, N, dtype, seed=M)
             if M in (33, 96):
                 x = (x.float() * 0.05 + 1.0).to(dtype)
-            y = ops.gemm(pm, x.to(DEV), out_dtype=torch.float32)
-            err = rel_fro(_np(y), R.forward_ref(W, _np(x)))
-            assert err < TOL, f"{case_id(case)} {K}x{N} M={M}: {err}"
+            ref = R.forward_ref(W, _np(x))
+            for tokens in TOKENS["rows"]:
+                err = rel_fro(_np(gemm_as(pm, x.to(DEV), "rows", tokens, out_dtype=torch.float32)), ref)
+                assert err < TOL, f"{case_id(case)} {K}x{N} M={M} {tokens} tokens: {err}"
 
 
 @pytest.mark.parametrize("case", [(F.BLK1632_4, 4, 128, 16), (F.BLKC, 2, 64, 16), (F.BLKC, 3, 128, 23), (F.BLKC, 2, 128, 10),
@@ -970,14 +995,14 @@ def test_gemm_token_tiles_of_32_64_and_96(case):
 def test_gemm_of_infinite_activations(case):
     """A token with infinities gets what sums in IEEE arithmetic give: +-inf, NaN where an infinity meets a
     weight that is 0 or two of them cancel; NaN stays NaN, the other tokens are untouched.  The same
-    however many tokens the call has, so on every token tile of both kernels; several parts of the columns,
-    values beyond what a half holds beside the infinity, plain and gate/up matrices."""
+    however many tokens the call has: every token tile of both kernels by name, one and two parts of the
+    columns over workgroups, values beyond what a half holds beside the infinity, plain and gate/up matrices."""
     K, N = 192, 4096
     one = F.synth_packed(K, N, case[0], case[1], case[2], case[3] or None, seed=7, device=DEV)
     two = F.fuse_rows([one, F.synth_packed(K, N, case[0], case[1], case[2], case[3] or None, seed=8, device=DEV)], interleave=True)
     for pm in (one.to_tiled(), two.to_tiled()):
         W = ops.dequant(pm, torch.float32).cpu().double()
-        for M in (9, 30, 60, 90, 130, 400, 1500):
+        for kernel, tokens, M in [("rows", t, m) for t in TOKENS["rows"] for m in (9, 100)] + [("tile", t, 300) for t in TOKENS["tile"]]:
             x = acts(M, N, torch.bfloat16, seed=M).float()
             x[1, 7] = float("inf")
             x[2, 900] = float("nan")
@@ -987,12 +1012,15 @@ def test_gemm_of_infinite_activations(case):
             x[6, 130], x[6, 131] = float("inf"), float("-inf")
             x[M - 1, N - 1] = float("inf")
             x = x.to(torch.bfloat16)
-            y = ops.gemm(pm, x.to(DEV), out_dtype=torch.float32).cpu()
             ref = x.double() @ W.t()
-            assert torch.equal(torch.isnan(y), torch.isnan(ref)), M
-            assert torch.equal(torch.isinf(y), torch.isinf(ref)) and torch.equal(y[torch.isinf(y)] > 0, ref[torch.isinf(ref)] > 0), M
             ok = torch.isfinite(ref).all(1)
-            assert int((~ok).sum()) == 6 and float((y[ok].double() - ref[ok]).norm() / ref[ok].norm()) < TOL
+            assert int((~ok).sum()) == 6
+            for s in (1, 2) if kernel == "rows" else (1,):
+                y = gemm_as(pm, x.to(DEV), kernel, tokens, s, out_dtype=torch.float32).cpu()
+                assert torch.equal(torch.isnan(y), torch.isnan(ref)), (kernel, tokens, M, s)
+                assert torch.equal(torch.isinf(y), torch.isinf(ref)), (kernel, tokens, M, s)
+                assert torch.equal(y[torch.isinf(y)] > 0, ref[torch.isinf(ref)] > 0), (kernel, tokens, M, s)
+                assert float((y[ok].double() - ref[ok]).norm() / ref[ok].norm()) < TOL
 
 
 def test_gemm_bias_dtype_and_prune_zero():
@@ -1047,9 +1075,15 @@ def test_gemm_activations_beyond_fp16_range():
                 assert err < TOL, f"cs_rows={cs_rows} splits={splits} {dtype} token {tok}: {err}"
             keep = [t for t in range(M) if t not in (1, 70, 200, 299)]
             assert torch.equal(y[keep], small[keep])
-            y64 = ops.gemm(pm, xb[:40].to(DEV), out_dtype=torch.float32)          # the 64-token instantiation
+            y64 = ops.gemm(pm, xb[:40].to(DEV), out_dtype=torch.float32)
             small64 = ops.gemm(pm, x[:40].to(DEV), out_dtype=torch.float32)
             assert rel_fro(_np(y64[1:2]), ref[1:2]) < TOL and torch.equal(y64[2:], small64[2:])
+            if cs_rows < 3:
+                for kernel, tokens in (("rows", 32), ("rows", 64), ("rows", 96), ("tile", 64), ("tile", 256)):
+                    yk, sk = (gemm_as(pm, v.to(DEV), kernel, tokens, out_dtype=torch.float32) for v in (xb, x))
+                    for tok in (1, 70, 200, 299):
+                        assert rel_fro(_np(yk[tok:tok + 1]), ref[tok:tok + 1]) < TOL, (cs_rows, dtype, kernel, tokens, tok)
+                    assert torch.equal(yk[keep], sk[keep])
 
 
 # ------------------------------------------------------------------ the module seam

@@ -1,5 +1,5 @@
 """Seeded random sweep over shapes, layouts, byte orders, activation counts and types: every call
-of the layer (`cbk_linear`: decode kernel up to eight rows, tile kernels above) and of the gated
+of the layer (`cbk_linear`: decode kernel up to eight rows, the two prefill kernels above) and of the gated
 MLP's first half (`cbk_linear_act`) against the CPU oracle's dequantised weights in float64.
 The fixed cases elsewhere pin known corners; this sweep is there for the ones nobody listed
 (row counts off the 16-row tiles, column counts off the 512-column step, rows longer than the
@@ -11,7 +11,7 @@ import torch
 from oracle import cbk_ref as R
 from cobalt_amd import format as F
 from cobalt_amd import ops
-from helpers import FIXED_CASES, SPARSE_CASES, acts, case_id, kw_of, make_raw, oracle_pack, packed_from_oracle, rel_fro
+from helpers import FIXED_CASES, SPARSE_CASES, acts, case_id, gemm_as, kw_of, make_raw, oracle_pack, packed_from_oracle, rel_fro
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -53,8 +53,9 @@ def test_linear_random_shapes(case):
 @pytest.mark.parametrize("case", [(F.BLK1632_4, 4, 128, 16), (F.BLKC, 3, 64, 10), (F.DENSE4, 4, 128, 0)], ids=case_id)
 def test_linear_act_random_shapes(case):
     """gate/up matrices (rows 2i gate, 2i+1 up, one column-scale vector per parity): act(gate) * up
-    from the decode kernel (interleaved float32 intermediate), the 64-token and the 256-token tile
-    kernels (intermediate in two halves), tanh-GELU and SiLU, with and without a bias."""
+    from the decode kernel (interleaved float32 intermediate), what a plain call above eight rows takes, and by
+    name the 64-token and the 256-token tile kernels (intermediate in two halves), tanh-GELU and SiLU, with
+    and without a bias."""
     rng = np.random.default_rng(5)
     for (K2, N, M, act) in ((24, 384, 3, "silu"), (130, 640, 8, "gelu_tanh"), (77, 1152, 9, "silu"), (256, 512, 64, "gelu_tanh"),
                             (300, 256, 65, "silu"), (129, 1408, 300, "gelu_tanh"), (512, 128, 257, "silu")):
@@ -81,6 +82,10 @@ def test_linear_act_random_shapes(case):
             err = rel_fro(_np(y), ref.astype(np.float32))
             # above 128 rows the intermediate is rounded to the output type before the activation
             assert err < (4e-3 if M > 128 else TOL), f"{case_id(case)} {K}x{N} M={M} tiled={tiled} {act}: {err}"
+            if M > 8:
+                y = gemm_as(pm, x.to(DEV), "tile", 64 if M <= 64 else 256, bias=None if bias is None else bias.to(DEV),
+                            out_dtype=torch.float32, act=act)
+                assert rel_fro(_np(y), ref.astype(np.float32)) < TOL, f"{case_id(case)} {K}x{N} M={M} tiled={tiled} {act} tile"
 
 
 def test_gemv_between_one_and_two_tiles_per_workgroup():
