@@ -173,15 +173,15 @@ static inline size_t sk_sum(const SkSpace& s) { return s.x + s.sums + s.scale + 
 // Times in microseconds, fitted to calls of ten shapes (1024 x 4096 to 43008 x 5376) at 16 to 1700 rows,
 // within a tenth of the measured ones: a group of a wavefront with two wavefronts per SIMD, by token tile
 // (codes that do not start on 16-byte units take a fifth longer, 6-bit codes with their second plane
-// 1.35 times), 5.5 to 10 per workgroup outside the loop, 7.4 for the preparation kernel and the launches and 0.5 per megabyte of X' beyond four (written, and
+// 1.35, 1.27 and 1.07 times on the three tiles: 21504 x 5376 at 32, 64 and 96 rows 38.0, 45.7 and 50.3), 5.5 to 10 per workgroup outside the loop, 7.4 for the preparation kernel and the launches and 0.5 per megabyte of X' beyond four (written, and
 // fetched by every XCD: 1024 x 5376 at 4096 rows, 44 MB, took 25 more than without that term), 5.5 and the
 // partial tiles at 4 TB/s for the reduction kernel.
 static GemmPlan sk_plan_ti(const DMat& m, int M, int ti, size_t room) {
   const int tiles = ((M + 32 * ti - 1) / (32 * ti)) * ((m.K + SK_ROWS * SK_WR - 1) / (SK_ROWS * SK_WR));
-  static const double g128[3] = {1.7, 2.2, 2.8}, g64[3] = {1.17, 1.45, 1.53}, wg[3] = {5.5, 7.6, 10.0};
+  static const double g128[3] = {1.7, 2.2, 2.8}, g64[3] = {1.17, 1.45, 1.53}, wg[3] = {5.5, 7.6, 10.0}, six[3] = {1.35, 1.27, 1.07};
   const bool skewed = family_of(m.layout) == FAM_BLK && (m.keep * m.bits * (m.group / 64)) % 32 != 0;
   const double two = m.cs_rows == 2 ? 1.12 : 1.0;                   // (two sets of X' compete for L2)
-  const double t_group = (m.group == 128 ? g128 : g64)[ti - 1] * (skewed ? 1.2 : m.bits == 6 ? 1.35 : 1.0) * two, t_wg = wg[ti - 1] * two;
+  const double t_group = (m.group == 128 ? g128 : g64)[ti - 1] * (skewed ? 1.2 : m.bits == 6 ? six[ti - 1] : 1.0) * two, t_wg = wg[ti - 1] * two;
   const double xmb = 2e-6 * (m.cs_rows > 1 ? m.cs_rows : 1) * (double)M * m.N, t_prep = 7.4 + (xmb > 4.0 ? 0.5 * (xmb - 4.0) : 0.0);
   GemmPlan best;
   for (int s = 1; s <= 16; ++s) {
