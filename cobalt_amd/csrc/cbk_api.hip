@@ -177,7 +177,7 @@ static int check_io(const void* x, int xdt, int M, int64_t ldx, const void* y, i
 }
 
 // A survivor-stream matrix (SPARSE4, SPARSE4X, SPARSE4E: rows of different lengths) has no
-// matrix-core kernel of its own.  A prefill call re-packs it, in the caller's workspace and for
+// prefill kernel of its own.  A prefill call re-packs it, in the caller's workspace and for
 // the duration of the call, as the dense 4-bit layout in tiled order (pruned columns hold the
 // zero point, so every weight dequantises to the same value) and runs the prefill kernel on that:
 // one small kernel in front of the matrix product.
@@ -550,11 +550,12 @@ int cbk_gemm_static(const cbk_desc* in, const void* x, int x_dtype, int M, int64
 
 int cbk_linear(const cbk_desc* in, const void* x, int x_dtype, int M, int64_t ldx, void* y, int y_dtype,
                int64_t ldy, const void* bias, void* workspace, size_t workspace_bytes, void* stream) {
-  // up to 8 rows (one or two passes of the decode kernel) the weights are streamed faster than the
-  // prefill kernel's 64-token tile decodes them (14336 x 4096: 28 us against 31 us; 54 us at 16 rows)
+  // up to 8 rows (one pass of the decode kernel) the weights are streamed faster than the prefill kernel for few
+  // tokens decodes them; from 9 on it takes two (BLK1632_4, 14336 x 4096: 13.8 against 19.4 us at 8 rows, 26.4 against
+  // 20.0 at 16; 5376 x 21504: 18.8 / 25.2 and 36.5 / 25.9)
   if (M <= 8) return cbk_gemv(in, x, x_dtype, M, ldx, y, y_dtype, ldy, bias, workspace, workspace_bytes, stream);
-  // (the variable-length layouts have no matrix-core path of their own: cbk_gemm sends them to the
-  // row kernel or re-packs them for the call)
+  // (the variable-length layouts have no prefill kernel of their own: cbk_gemm sends them to the
+  // decode kernels or re-packs them for the call)
   return cbk_gemm(in, x, x_dtype, M, ldx, y, y_dtype, ldy, bias, workspace, workspace_bytes, stream);
 }
 

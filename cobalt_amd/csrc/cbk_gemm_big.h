@@ -1,4 +1,5 @@
-// Prefill GEMM:  Y[M, K] = X[M, N] . W_hat[K, N]^T on the gfx950 matrix cores.
+// Prefill GEMM for many tokens:  Y[M, K] = X[M, N] . W_hat[K, N]^T on the gfx950 matrix cores.  (Calls of nine to a
+// few hundred rows and small matrices: cbk_gemm_skinny.h, which has a decoder for 8-bit codes too.)
 //
 // Workgroup tile 256 tokens x 256 weight rows, 64 input columns per stage, four wavefronts
 // each owning a 128 x 128 sub-tile (4 x 4 blocks of v_mfma_f32_32x32x16_f16, 256 accumulator
@@ -60,7 +61,7 @@ struct GbArgs {
   int tiles_t, tiles_r;
   int halves;              // gate/up matrix (par): 1 = write the gate outputs to columns [0, K/2) and the up outputs to
                            // [K/2, K) of y instead of interleaving them (whole 16-byte stores; for cbk_linear_act)
-  int ti;                  // 32-token blocks per wavefront: 4 (256-token tiles) or 1 (64-token tiles)
+  int ti;                  // 32-token blocks per wavefront: 4, 2 or 1 (tiles of 256, 128 or 64 tokens)
   // par = 1: gate/up matrix, two col_scale vectors by row parity.  A workgroup then takes 256
   // rows of one parity out of 512 (rows r0 + 2 i + p), and X' of that parity's vector, which
   // starts xps elements after the other one.

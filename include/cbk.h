@@ -210,9 +210,12 @@ int cbk_gemv_batch(int n, const cbk_desc* descs, const void* const* xs, const in
                    int x_dtype, int M, void* const* ys, const int64_t* ldys, int y_dtype,
                    const void* const* biases, void* workspace, size_t workspace_bytes, void* stream);
 
-/* Prefill path, any M >= 1 (256-token tiles; a 128-token tile up to 128 rows, a 64-token tile up to 64).  Same contract as
+/* Prefill path, any M >= 1.  Two kernels, chosen by what each expects a call to take: one for few
+ * tokens or small matrices (tiles of 32, 64 and 96 tokens, weights decoded in the registers that
+ * multiply them) and one for many (tiles of 64, 128 and 256 tokens x 256 rows).  Same contract as
  * cbk_gemv; activations are carried as fp16 inside, a token whose values leave fp16's range
- * scaled by a power of two on the way in and back on the way out.  The survivor-stream layouts
+ * scaled by a power of two on the way in and back on the way out; an infinite one gives +-inf, or NaN
+ * where it meets a weight that is 0.  The survivor-stream layouts
  * (SPARSE4, SPARSE4X, SPARSE4E) are re-packed for the call, above 16 rows, into the dense 4-bit
  * layout inside the workspace (cbk_workspace_bytes counts it) when the descriptor carries
  * CBK_FLAG_ZERO_ON_GRID, has at most one col_scale vector and the workspace is large enough;
