@@ -8,7 +8,8 @@
 // v_mfma_i32_16x16x64_i8 as the B operand.  The A operand is the activation vector in
 // block fixed point: per 128-column chunk, x' = x * col_scale is written as
 // delta * (65536*d2 + 256*d1 + d0) with three int8 digits (|x' - delta*X| <= max|x'| / 2^24,
-// i.e. float32 resolution relative to the largest activation of the chunk).  The
+// i.e. float32 resolution relative to the largest activation of the chunk; 8-bit codes: four
+// digits, see digits_of).  The
 // matrix core produces exact int32 dot products per (row, chunk, digit); one float FMA per
 // row and quantisation group applies scale * delta.  A pruned column multiplies a literal
 // zero byte, so it contributes exactly 0 whatever the zero point holds.
@@ -55,11 +56,15 @@ constexpr int LUT_BYTES = 256 * LUT_LANES * 8;
 constexpr int ZERO_BYTES = 256;
 constexpr int CNT_SLOTS = 64;                 // most reduction slots (arrival counters)
 constexpr int CNT_BYTES = CNT_SLOTS * 4;       // at a fixed place: zeroed before the arguments are read
-constexpr int X_LDS_BUDGET = 112 * 1024;      // activation digits of one column slab: M * 3 * columns bytes (of 160 KB LDS)
+constexpr int X_LDS_BUDGET = 112 * 1024;      // activation digits of one row: 3 (8-bit codes: 4) * columns bytes (of 160 KB LDS)
 constexpr int DELTA_LDS_BUDGET = 16 * 1024;   // one float per 128-column chunk and activation row (eight rows of 65024
                                               // columns; the digits take what is left: a part of 4096 columns of
                                               // eight rows, 96 KB, still fits beside 24 KB of reduction slots)
 constexpr int NDIG = 3;                       // int8 digits per activation
+// 8-bit codes have four on the matrix-core kernels (the A operand has four rows per activation row anyway): some of
+// these layouts come from the float row kernel, and 24 bits below a chunk's largest activation lose more than it
+// does (groups of 64, 384 columns, eight rows: error against float64 3.0e-7, the row kernel 1.3e-7; 5.9e-8 with four).
+__host__ __device__ constexpr int digits_of(int bits) { return bits == 8 ? 4 : NDIG; }
 // The digit rows of the matrix-core kernels lie X_PAD bytes further apart than their length.  The
 // sixteen lanes of a quarter read sixteen bytes each from up to twelve different rows (activation
 // row, digit) at the same column; row lengths are multiples of 128 bytes, and unpadded rows would
@@ -144,7 +149,7 @@ __host__ __device__ constexpr bool block_loads(int bits, int keep) {
 __host__ __device__ constexpr int digit_order(int bits, bool dense) { return !dense || bits == 8 ? 0 : bits == 2 ? 2 : 1; }
 
 // ------------------------------------------------------------------ activation prep
-// x' = x * col_scale per 128-column chunk -> delta and three signed int8 digits per column:
+// x' = x * col_scale per 128-column chunk -> delta and three (ND = 4: four) signed int8 digits per column:
 // x' ~= delta * (65536*d2 + 256*d1 + d0),  delta = max|x'| / (127 * 65536).  Every workgroup
 // converts the activations it needs into its own LDS (a few hundred instructions per thread,
 // overlapped with the first weight loads).  One thread converts 16 columns at a time; the
@@ -170,7 +175,10 @@ __device__ inline void stage_load(const uint16_t* x, int64_t ldx, const uint16_t
 // chunk are always active together (the item count is a multiple of 8)
 // (digits at row stride Ns = 16 * n16 + pad bytes, deltas at the chunk's index in the whole row: ch0 is
 // the slab's first chunk)
-template <int ORDER>
+// ND = 4: x' = delta * (2^24 d3 + ...) with delta a power of two, 2^29 of them to the power of two at or below the largest: products
+// with the column scale are represented as they are, down to 2^-6 of it, and to 2^-30 of it below that.
+// HALVES (groups of 64): the delta of a chunk with infinities says which half has them, see group_delta.
+template <int ORDER, int ND = NDIG, bool HALVES = false>
 __device__ inline void stage_convert(const XLoad& r, bool has_cs, int xdt, int N, int ch0, int n16, int it, bool one_row,
                                      int8_t* xq, float* delta, int pad = 0) {
   const int NCH = N >> 7, Ns = n16 * 16 + pad;
@@ -189,35 +197,67 @@ __device__ inline void stage_convert(const XLoad& r, bool has_cs, int xdt, int N
 #pragma unroll
     for (int e = 0; e < 16; ++e) xv[e] *= h2f((uint16_t)(cw[e >> 1] >> (16 * (e & 1))));
   }
+  // (ND 4: magnitudes compare as their bits, which puts a NaN above an infinity; fmaxf passes NaN over)
+  auto larger = [](float a, float b) {
+    if constexpr (ND == 4) {
+      const uint32_t ab = __float_as_uint(a), bb = __float_as_uint(b);
+      return __uint_as_float(ab > bb ? ab : bb);
+    } else {
+      return fmaxf(a, b);
+    }
+  };
   float mx = 0.f;
 #pragma unroll
-  for (int e = 0; e < 16; ++e) mx = fmaxf(mx, fabsf(xv[e]));
+  for (int e = 0; e < 16; ++e) mx = larger(mx, fabsf(xv[e]));
   // maximum over the eight lanes of the chunk with register-to-register lane moves: swap
   // neighbours, swap pairs, mirror the eight-lane half row (every lane of a quad holds the
   // quad's maximum by then, so the mirror image is the other quad's)
-  mx = fmaxf(mx, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, mx), 0xB1, 0xF, 0xF, true)));
-  mx = fmaxf(mx, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, mx), 0x4E, 0xF, 0xF, true)));
-  mx = fmaxf(mx, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, mx), 0x141, 0xF, 0xF, true)));
+  mx = larger(mx, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, mx), 0xB1, 0xF, 0xF, true)));
+  mx = larger(mx, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, mx), 0x4E, 0xF, 0xF, true)));
+  const float here = mx, there = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, mx), 0x141, 0xF, 0xF, true));
+  mx = larger(here, there);
   // delta = max|x'| / 8323072 (= 127 * 65536: 24 signed bits) by a multiplication, its reciprocal by the
   // hardware approximation and one Newton step; two divisions were a tenth of this function.
   // (24 bits, not 23 with a cheaper rounding: activations of 1e4 at the pruned columns of a chunk,
   // the reference's own probe, leave the ordinary ones 10 bits less, and the result must still
   // meet the layer tolerance.)
-  const float d = mx > 1e-30f ? mx * (1.f / 8323072.f) : 1.f;
-  float inv = __builtin_amdgcn_rcpf(d);
-  inv = inv * fmaf(-d, inv, 2.f);
+  float d, inv;
+  bool none = false;                                               // ND 4: no finite maximum
+  if constexpr (ND == 4) {
+    const uint32_t e = __float_as_uint(mx) & 0x7f800000u;
+    none = e == 0x7f800000u;
+    d = none ? mx : mx > 1e-30f ? __uint_as_float(e) * 0x1p-29f : 1.f;
+    inv = none ? 0.f : 1.f / d;
+  } else {
+    d = mx > 1e-30f ? mx * (1.f / 8323072.f) : 1.f;
+    inv = __builtin_amdgcn_rcpf(d);
+    inv = inv * fmaf(-d, inv, 2.f);
+  }
   // X + 0x808080 has the bytes d0 + 128, d1 + 128, d2 + 128 of the balanced base-256 digits
   // (X = d0 + 256 d1 + 65536 d2, -128 <= d < 128), so the digits of four columns are byte
   // permutes of the four biased integers and one xor per digit plane
-  uint32_t dw[NDIG][4];
+  uint32_t dw[ND][4];
   uint32_t xb[16];
 #pragma unroll
   for (int bi = 0; bi < 16; ++bi) {
     const float v = ORDER == 0 ? xv[bi] : ORDER == 1 ? xv[frag_col(4, true, bi)] : xv[frag_col(2, true, bi)];
-    xb[bi] = (uint32_t)((int)rintf(v * inv) + 0x808080);          // |X| <= 127 * 65536 (+ 2 from the rounding of inv)
+    // ND 3: |X| <= 127 * 65536 (+ 2 from the rounding of inv); ND 4: |X| < 2^30
+    int X = (int)rintf(v * inv);
+    // A NaN makes delta one.  An infinity makes delta infinite and has +-1 for a digit (several in a chunk: their sum)
+    if (ND == 4 && none) X = fabsf(v) == mx ? (v > 0.f ? 1 : -1) : 0;
+    xb[bi] = (uint32_t)X + (ND == 4 ? 0x80808080u : 0x808080u);
   }
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
+    if constexpr (ND == 4) {
+      const uint32_t a = perm(xb[4 * q + 1], xb[4 * q], 0x05010400u), a2 = perm(xb[4 * q + 1], xb[4 * q], 0x07030602u);
+      const uint32_t b = perm(xb[4 * q + 3], xb[4 * q + 2], 0x05010400u), b2 = perm(xb[4 * q + 3], xb[4 * q + 2], 0x07030602u);
+      dw[0][q] = perm(b2, a2, 0x07060302u) ^ 0x80808080u;
+      dw[1][q] = perm(b2, a2, 0x05040100u) ^ 0x80808080u;
+      dw[2][q] = perm(b, a, 0x07060302u) ^ 0x80808080u;
+      dw[ND - 1][q] = perm(b, a, 0x05040100u) ^ 0x80808080u;
+      continue;
+    }
     const uint32_t a = perm(xb[4 * q + 1], xb[4 * q], 0x05010400u);       // d0 d0 d1 d1 of columns 0, 1
     const uint32_t b = perm(xb[4 * q + 3], xb[4 * q + 2], 0x05010400u);   // and of columns 2, 3
     const uint32_t c01 = perm(xb[4 * q + 1], xb[4 * q], 0x0C0C0602u);     // d2 d2 0 0
@@ -227,10 +267,34 @@ __device__ inline void stage_convert(const XLoad& r, bool has_cs, int xdt, int N
     dw[2][q] = perm(b, a, 0x05040100u) ^ 0x80808080u;
   }
 #pragma unroll
-  for (int k = 0; k < NDIG; ++k)
-    *(uint4*)(xq + ((size_t)row * NDIG + k) * Ns + c16 * 16) = make_uint4(dw[k][0], dw[k][1], dw[k][2], dw[k][3]);
+  for (int k = 0; k < ND; ++k)
+    *(uint4*)(xq + ((size_t)row * ND + k) * Ns + c16 * 16) = make_uint4(dw[k][0], dw[k][1], dw[k][2], dw[k][3]);
+  if (HALVES && none && mx == __builtin_inff())                     // (the writing lane is one of the first half)
+    d = here != mx ? -3.4028234663852886e38f : there != mx ? -mx : mx;
   if ((c16 & 7) == 0) delta[row * (NCH + 4) + ch0 + (c16 >> 3)] = d;
   if (ch0 == 0 && c16 < 4) delta[row * (NCH + 4) + NCH + c16] = 0.f;   // chunks past N
+}
+
+// The sum of a group from its digit sums (128 columns: below 2^22 each, so two of them meet in an int32).
+template <int ND>
+__device__ inline float digits_value(const v4i a) {
+  if (ND == 4) return fmaf((float)(a[0] * 256 + a[1]), 65536.f, (float)(a[2] * 256 + a[3]));
+  return fmaf((float)(a[0] * 256 + a[1]), 256.f, (float)a[2]);
+}
+
+// Delta of group h of a chunk of two groups: stage_convert leaves -infinity where only the first one holds an
+// infinity, the lowest float where only the second does; the other one's digits are 0 then.
+__device__ inline float group_delta(float dl, int h) {
+  return dl < 0.f ? ((dl < -3.4028234663852886e38f) == (h == 0) ? __builtin_inff() : 0.f) : dl;
+}
+
+// Four part sums more.  Those of 8-bit codes meet among themselves first: for activations of one sign sixteen sums one
+// after the other round more than the float row kernel did that served some of these layouts before (14336 columns
+// 9.5e-8 against 6.8e-8; 8.5e-8 so).  (All sixteen as a tree would need registers the kernel does not have: 21504 x 5376
+// at 4 rows 26 -> 33 us.)
+template <bool FOURS>
+__device__ inline float parts_add(float v, float p0, float p1, float p2, float p3) {
+  return FOURS ? v + ((p0 + p1) + (p2 + p3)) : (((v + p0) + p1) + p2) + p3;
 }
 
 // y(l) + y(l ^ 16), then that + the same of lane l ^ 32: the sum over the four lane quarters, in
@@ -460,7 +524,7 @@ struct XDigits { uint32_t xq_off, z_off; const float* delta; int Ns, ch0, NCH, M
 template <class C, int BITS, int NG, bool TURN>
 __device__ inline void block_step(const Loads<C>& cur, const uint8_t* smem, const uint2* lut, uint32_t l16, int lane, int S,
                                   const XDigits& x, float (&ysum)[4 * NG]) {
-  constexpr int NGC = C::NGC;
+  constexpr int NGC = C::NGC, ND = digits_of(BITS);
   const int wr = lane & 15, kq = lane >> 4;
   const int a_m = wr >> 2, a_dig = wr & 3;                          // activation row and digit of this lane's A row
   uint32_t st4[4][C::NW], mk4[4], hw4[4];
@@ -493,8 +557,8 @@ __device__ inline void block_step(const Loads<C>& cur, const uint8_t* smem, cons
   int dm[NG];                                                       // the activation rows this quarter sums
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
-    a_on[g] = a_dig < NDIG && a_m + 4 * g < x.M;
-    a_base[g] = x.xq_off + (uint32_t)(((a_m + 4 * g) * NDIG + a_dig) * (x.Ns + X_PAD) + kq * 32);
+    a_on[g] = a_dig < ND && a_m + 4 * g < x.M;
+    a_base[g] = x.xq_off + (uint32_t)(((a_m + 4 * g) * ND + a_dig) * (x.Ns + X_PAD) + kq * 32);
     dm[g] = kq + 4 * g < x.M ? kq + 4 * g : 0;
   }
 #pragma unroll
@@ -550,8 +614,9 @@ __device__ inline void block_step(const Loads<C>& cur, const uint8_t* smem, cons
       const float dl = x.delta[dm[g] * (x.NCH + 4) + chunk];        // 0 past the last chunk
 #pragma unroll
       for (int h = 0; h < NGC; ++h) {
-        const float f = fmaf((float)(acc[g][h][0] * 256 + acc[g][h][1]), 256.f, (float)acc[g][h][2]);
-        ysum[4 * g + c] = fmaf(f, h2f((uint16_t)(zs[c][h] >> 8)) * dl, ysum[4 * g + c]);
+        const float f = digits_value<ND>(acc[g][h]);
+        const float dg = ND == 4 && NGC == 2 ? group_delta(dl, h) : dl;
+        ysum[4 * g + c] = fmaf(f, h2f((uint16_t)(zs[c][h] >> 8)) * dg, ysum[4 * g + c]);
       }
     }
   }
@@ -563,6 +628,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
   static_assert(MP == 1 || MP == 2 || MP == 4 || MP == 8, "single activation rows, or row groups of four");
   constexpr bool QB = MP >= 4, TURN = QB && !block_loads(BITS, KEEP);
   constexpr int NG = MP == 8 ? 2 : 1;                  // groups of four activation rows, one MFMA each per fragment
+  constexpr int ND = digits_of(BITS);
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);     // in a scalar register: positions are scalar work
@@ -605,7 +671,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
   const int wr = lane & 15, kq = lane >> 4;            // weight row in tile / lane quarter
   const uint32_t l16 = lane & (LUT_LANES - 1);
   // role of this lane's row in the A operand: variant i = lane%16 = 4 * quarter + digit
-  // (digit 3 is an all-zero row); in the result, lane quarter kq holds the three digit sums
+  // (digit 3 is an all-zero row where there are three); in the result, lane quarter kq holds the three digit sums
   // of its own chunk, so every lane post-processes exactly the chunk it decoded
   const int a_slice = wr >> 2, a_dig = wr & 3;
   const uint32_t xq_off = (uint32_t)((uint8_t*)xq - smem), z_off = (uint32_t)(zreg - smem);
@@ -734,12 +800,12 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
     if (!first) __syncthreads();                                  // previous matrix fully consumed
     first = false;
     constexpr int XORD = digit_order(BITS, C::DENSE);
-    if (xit < xitems) stage_convert<XORD>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, xit, MP == 1, xq, delta, X_PAD);
+    if (xit < xitems) stage_convert<XORD, ND, ND == 4 && C::NGC == 2>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, xit, MP == 1, xq, delta, X_PAD);
     if (PRE2 && xit + GV_THREADS < xitems)
-      stage_convert<XORD>(xl2, m.cs != nullptr, h.xdt, N, ch0, n16, xit + GV_THREADS, MP == 1, xq, delta, X_PAD);
+      stage_convert<XORD, ND, ND == 4 && C::NGC == 2>(xl2, m.cs != nullptr, h.xdt, N, ch0, n16, xit + GV_THREADS, MP == 1, xq, delta, X_PAD);
     for (xit += (PRE2 ? 2 : 1) * GV_THREADS; xit < xitems; xit += GV_THREADS) {
       stage_load(gm.x, gm.ldx, m.cs, N, col0, n16, xit, MP == 1, gm.par, xl);
-      stage_convert<XORD>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, xit, MP == 1, xq, delta, X_PAD);
+      stage_convert<XORD, ND, ND == 4 && C::NGC == 2>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, xit, MP == 1, xq, delta, X_PAD);
     }
     __syncthreads();
 
@@ -767,8 +833,8 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
         uint32_t aaddr[MP];
 #pragma unroll
         for (int p = 0; p < MP; ++p) {
-          const bool on = valid && a_slice == kq && a_dig < NDIG && p < h.M;
-          aaddr[p] = on ? xq_off + (uint32_t)((p * NDIG + a_dig) * (Ns + X_PAD) + (chunk - ch0) * 128) : z_off;
+          const bool on = valid && a_slice == kq && a_dig < ND && p < h.M;
+          aaddr[p] = on ? xq_off + (uint32_t)((p * ND + a_dig) * (Ns + X_PAD) + (chunk - ch0) * 128) : z_off;
         }
         // ---- bring the chunk's first code bit to bit 0 of cw[0]
         uint32_t cw[C::ND];
@@ -817,8 +883,9 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
 #pragma unroll
               for (int p = 0; p < MP; ++p) {
                 const float dl = delta[(p < h.M ? p : 0) * (NCH + 4) + chunk];      // 0 past the last chunk
-                const float f = fmaf((float)(acc[p][0] * 256 + acc[p][1]), 256.f, (float)acc[p][2]);
-                ysum[p] = fmaf(f, h2f((uint16_t)cur.sc[g]) * dl, ysum[p]);
+                const float f = digits_value<ND>(acc[p]);
+                const float dg = ND == 4 && C::NGC == 2 ? group_delta(dl, g) : dl;
+                ysum[p] = fmaf(f, h2f((uint16_t)cur.sc[g]) * dg, ysum[p]);
                 acc[p] = (v4i){0, 0, 0, 0};
               }
             }
@@ -897,7 +964,8 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) pv[j] = rs[((j0 + j < SK ? j0 + j : SK - 1) * h.M + am) * 16 + wr];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) v += j0 + j < SK ? pv[j] : 0.f;
+                for (int j = 0; j < 4; ++j) pv[j] = j0 + j < SK ? pv[j] : 0.f;
+                v = parts_add<ND == 4>(v, pv[0], pv[1], pv[2], pv[3]);
               }
               store(am, wr, v);
             }
@@ -1047,16 +1115,16 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
   Pos p1 = p0; bool v1 = v0 && advance(p1);
 
   // ---- stage the slab's digits (the activation loads go out before the first weight loads)
-  constexpr int XORD = digit_order(BITS, C::DENSE);
+  constexpr int XORD = digit_order(BITS, C::DENSE), ND = digits_of(BITS);
   const int n16 = Ns >> 4, xitems = M * n16;                        // a multiple of 8
   XLoad xl;
   if (tid < xitems) stage_load(gm.x, gm.ldx, m.cs, N, col0, n16, tid, false, gm.par, xl);
   Loads<C> LA, LB;
   issue(T_lo + p0.tl, p0.S, LA);
-  if (tid < xitems) stage_convert<XORD>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, tid, false, xq, delta, X_PAD);
+  if (tid < xitems) stage_convert<XORD, ND, ND == 4 && C::NGC == 2>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, tid, false, xq, delta, X_PAD);
   for (int xit = tid + GV_THREADS; xit < xitems; xit += GV_THREADS) {
     stage_load(gm.x, gm.ldx, m.cs, N, col0, n16, xit, false, gm.par, xl);
-    stage_convert<XORD>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, xit, false, xq, delta, X_PAD);
+    stage_convert<XORD, ND, ND == 4 && C::NGC == 2>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, xit, false, xq, delta, X_PAD);
   }
   __syncthreads();
 
@@ -1117,7 +1185,14 @@ __global__ __launch_bounds__(GS_RED_THREADS) void gemv_split_reduce_kernel(GsArg
   for (int j = 0; j < 16; ++j) pv[j] = gs.part[((size_t)(tile * SK + (j < SK ? j : SK - 1)) * M + am) * 16 + wr];
   float v = 0.f;
 #pragma unroll
-  for (int j = 0; j < 16; ++j) v += j < SK ? pv[j] : 0.f;
+  for (int j = 0; j < 16; ++j) pv[j] = j < SK ? pv[j] : 0.f;
+  if (gm.m.bits == 8) {                                             // (the order of the main kernel)
+#pragma unroll
+    for (int j = 0; j < 16; j += 4) v = parts_add<true>(v, pv[j], pv[j + 1], pv[j + 2], pv[j + 3]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 16; j += 4) v = parts_add<false>(v, pv[j], pv[j + 1], pv[j + 2], pv[j + 3]);
+  }
   if (gm.bias) v += (h.ydt == CBK_F32) ? ((const float*)gm.bias)[k]
                   : (h.ydt == CBK_F16) ? h2f(((const uint16_t*)gm.bias)[k]) : bf2f(((const uint16_t*)gm.bias)[k]);
   const size_t o = (size_t)om * gm.ldy + k;
@@ -2187,6 +2262,8 @@ int launch_gemv_dense8(const DMat& m, const void* x, int xdt, int M, int64_t ldx
 
 // ------------------------------------------------------------------ host side
 
+// (four digits of 28672 columns are 64 bytes over the budget of three of 38213)
+static inline size_t x_lds_budget(int bits) { return X_LDS_BUDGET + (bits == 8 ? 1024 : 0); }
 static bool keep_supported(int keep) { return keep == 10 || keep == 16 || keep == 23; }
 
 bool gemv_fast_takes(const DMat& m, int M) {
@@ -2208,7 +2285,7 @@ bool gemv_fast_takes(const DMat& m, int M) {
   if ((uint64_t)((m.K + 15) / 16 * 16) * m.G * 2 >= (1ull << 32)) return false;
   // the digits are staged in column slabs where a whole row does not fit; the per-chunk deltas
   // of all rows stay in LDS for the whole matrix
-  if (M == 1) return (size_t)NDIG * (m.N + X_PAD) <= (size_t)X_LDS_BUDGET;   // (the one-row kernels stage whole rows only)
+  if (M == 1) return (size_t)digits_of(m.bits) * (m.N + X_PAD) <= x_lds_budget(m.bits);   // (the one-row kernels stage whole rows only)
   return (size_t)M * (m.N / 128 + 4) * 4 <= (size_t)DELTA_LDS_BUDGET;
 }
 
@@ -2220,9 +2297,10 @@ bool gemv_same_config(const DMat& a, const DMat& b) {
 // Macro-steps per work item of a launch of `cost` tile-steps on `blocks` workgroups: about one and
 // a half items per wavefront over the whole launch (the end of an item costs about as many
 // instructions as a step; measured best between one and two).
-static inline int launch_spi(long long cost, int blocks) {
-  const int spi = (int)(cost * 2 / ((long long)blocks * GV_WAVES * 3));
-  return spi < 1 ? 1 : (spi > 8 ? 8 : spi);
+// (8-bit codes: at most seven, so that one part of eight rows, four digits, always fits in LDS beside two reduction slots)
+static inline int launch_spi(long long cost, int blocks, int bits) {
+  const int spi = (int)(cost * 2 / ((long long)blocks * GV_WAVES * 3)), most = bits == 8 ? 7 : 8;
+  return spi < 1 ? 1 : (spi > most ? most : spi);
 }
 // The parts of a row of nS macro-steps: at most 16, a power of two of them where the row is long
 // enough (the items then spread evenly over the four SIMDs), of equal length.
@@ -2265,12 +2343,12 @@ static inline int kernel_rows(const DMat& m, int M) {            // activation r
 size_t gemv_fast_workspace(const DMat& m, int M) {
   const int Mk = kernel_rows(m, M);
   if (Mk < 2) return 0;
-  const size_t digits = (size_t)Mk * NDIG * (m.N + X_PAD);
+  const size_t digits = (size_t)Mk * digits_of(m.bits) * (m.N + X_PAD);
   if (digits <= split_min_bytes(m, Mk)) return 0;
   // what a call with this matrix alone would do
   const int ntiles = (m.K + 15) / 16, nS = (m.N / 128 + 3) / 4;
   int spi, sk;
-  row_parts(nS, launch_spi((long long)ntiles * nS, ntiles < 256 ? ntiles : 256), spi, sk);
+  row_parts(nS, launch_spi((long long)ntiles * nS, ntiles < 256 ? ntiles : 256, m.bits), spi, sk);
   if (digits <= main_x_budget(Mk, Mk * (m.N / 128 + 4), sk) && ntiles > SPLIT_MAX_TILES) return 0;
   if (ntiles < 256) sk = nS < 16 ? nS : 16;                       // (in a batch a small matrix may be cut finer)
   return up256(split_part_bytes(ntiles + 3, sk, Mk));             // (+3: a q|k|v matrix is run as its three ranges)
@@ -2392,7 +2470,8 @@ static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt,
     total += (long long)mats[i].ntiles * mats[i].nS;
     delta_cap = delta_cap > M * (mats[i].m.N / 128 + 4) ? delta_cap : M * (mats[i].m.N / 128 + 4);
   }
-  const size_t fixed = (size_t)LUT_BYTES + ZERO_BYTES + (size_t)delta_cap * 4 + (size_t)M * NDIG * X_PAD;
+  const int ND = digits_of(mats[0].m.bits);
+  const size_t fixed = (size_t)LUT_BYTES + ZERO_BYTES + (size_t)delta_cap * 4 + (size_t)M * ND * X_PAD;
   int xq_cap = 0, wg = 0, th = 0;
   size_t off = 0;
   for (int i = 0; i < n; ++i) {
@@ -2404,7 +2483,7 @@ static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt,
     // this matrix's share of the 256 workgroups
     int budget = (int)((long long)256 * g.ntiles * g.nS / total);
     budget = budget < 1 ? 1 : budget;
-    const size_t per_part = (size_t)M * NDIG * g.spi * 512;
+    const size_t per_part = (size_t)M * ND * g.spi * 512;
     if (fixed + per_part > 160 * 1024) return CBK_ERR_UNSUPPORTED;
     int pps_max = (int)((160 * 1024 - fixed) / per_part);
     pps_max = pps_max < g.sk ? pps_max : g.sk;
@@ -2430,7 +2509,7 @@ static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt,
     q.g.inv_sp = (uint32_t)((65536 + best_pps - 1) / best_pps);
     q.g.dq_t = GV_WAVES / best_pps; q.g.dq_p = GV_WAVES % best_pps;
     const int cols = best_pps * g.spi * 512 < g.m.N ? best_pps * g.spi * 512 : g.m.N;
-    xq_cap = xq_cap > M * NDIG * (cols + X_PAD) ? xq_cap : M * NDIG * (cols + X_PAD);
+    xq_cap = xq_cap > M * ND * (cols + X_PAD) ? xq_cap : M * ND * (cols + X_PAD);
     q.wg0 = wg; wg += q.nslab * q.wps; a.h.wg_end[i] = wg;
     q.th0 = th; th += (g.ntiles * M * 16 + GS_RED_THREADS - 1) / GS_RED_THREADS * GS_RED_THREADS; a.h.th_end[i] = th;
   }
@@ -2468,19 +2547,20 @@ static int launch_main_batch(GvBatch& gb, hipStream_t st) {
   // eight rows always fits).
   const size_t slot_bytes = (size_t)sk_cap * M * 16 * 4;
   const size_t fixed = (size_t)LUT_BYTES + ZERO_BYTES + CNT_BYTES + (size_t)delta_cap * 4;
-  const size_t x_budget = M == 1 ? (size_t)X_LDS_BUDGET : main_x_budget(M, delta_cap, sk_cap);
+  const int ND = digits_of(gb.mat[0].m.bits);
+  const size_t x_budget = M == 1 ? x_lds_budget(gb.mat[0].m.bits) : main_x_budget(M, delta_cap, sk_cap);
   for (int i = 0; i < n; ++i) {
     GvMat& g = gb.mat[i];
     const int N = g.m.N;
     g.sp = g.sk;
-    if ((size_t)M * NDIG * (N + X_PAD) > x_budget) {
-      g.sp = (int)((x_budget - (size_t)M * NDIG * X_PAD) / ((size_t)M * NDIG * g.spi * 512));
+    if ((size_t)M * ND * (N + X_PAD) > x_budget) {
+      g.sp = (int)((x_budget - (size_t)M * ND * X_PAD) / ((size_t)M * ND * g.spi * 512));
       if (g.sp < 1 || M == 1) return CBK_ERR_UNSUPPORTED;         // (the one-row kernels stage whole rows only)
       const int nsl = (g.sk + g.sp - 1) / g.sp;                   // slabs of equal length, not a short last one
       g.sp = (g.sk + nsl - 1) / nsl;
     }
     const int slab_cols = g.sp >= g.sk ? N : g.sp * g.spi * 512;
-    xq_cap = xq_cap > M * NDIG * (slab_cols + X_PAD) ? xq_cap : M * NDIG * (slab_cols + X_PAD);
+    xq_cap = xq_cap > M * ND * (slab_cols + X_PAD) ? xq_cap : M * ND * (slab_cols + X_PAD);
     if (g.sp > g.sk) g.sp = g.sk;
     // exact for every a the kernel divides (a < cost + nS) when (cost + nS) * nS < 2^32
     g.inv_nS = g.nS > 1 && (uint64_t)(cost + g.nS) * g.nS < (1ull << 32) ? (uint32_t)(((1ull << 32) + g.nS - 1) / g.nS) : 0u;
@@ -2539,7 +2619,7 @@ int launch_gemv_fast_batch(int n, const GvCall* calls, int xdt, int M, int ydt, 
   const int blocks = gemv_blocks(gb, n, tiles);
   // The parts depend on the matrices of the call only, not on M: they fix the order of every
   // row's partial sums.
-  const int spi = launch_spi(cost, blocks);
+  const int spi = launch_spi(cost, blocks, calls[0].m.bits);
   int sk_cap = 1;
   for (int i = 0; i < n; ++i) {
     GvMat& g = gb.mat[i];
@@ -2556,7 +2636,7 @@ int launch_gemv_fast_batch(int n, const GvCall* calls, int xdt, int M, int ydt, 
   if (M > 1) {
     const size_t x_budget = main_x_budget(M, delta_cap, sk_cap);
     auto splits = [&](const GvMat& g) {
-      const size_t digits = (size_t)M * NDIG * (g.m.N + X_PAD);
+      const size_t digits = (size_t)M * digits_of(g.m.bits) * (g.m.N + X_PAD);
       return digits > x_budget || (digits > split_min_bytes(g.m, M) && tiles <= SPLIT_MAX_TILES);
     };
     GvMat split[GV_MAX_BATCH];

@@ -140,7 +140,7 @@ size_t cbk_stream_bytes(const cbk_desc* d, size_t sparse_data_bytes);
  * less is refused (CBK_ERR_WORKSPACE): its results do not depend on what it is given.  The decode
  * kernels need none, with one optional use:
  * two to eight activation rows of rows whose activations take more than 90 KB of LDS
- * (M * 3 * N bytes) are split over the workgroups by columns when there is room for the float32
+ * (M * 3 * N bytes; 8-bit codes M * 4 * N) are split over the workgroups by columns when there is room for the float32
  * part sums, K * 16 * M * 4 bytes at most, and so are the rows of SPARSE4X / SPARSE4E matrices on
  * the matrix-core stream kernel when the activation rows of a pass (up to eight) do not fit in
  * LDS as whole rows (M * 3 * N bytes beyond about 140 KB); with a smaller workspace, or none,

@@ -565,6 +565,67 @@ def test_gemv_rows_do_not_depend_on_their_number(case):
                 assert torch.equal(ops.gemv(pm, x, out_dtype=torch.float32, workspace=small), one), (K, N, M, pm is rows)
 
 
+EIGHT_BIT = [(F.DENSE8, 8, 128, 0), (F.DENSEB, 8, 64, 0), (F.DENSEB, 8, 128, 0)]
+
+
+def _eight_bit(case, K, N, vectors, seed):
+    mk = lambda k, s: F.synth_packed(k, N, case[0], case[1], case[2], None, seed=seed + s, device=DEV)
+    return (mk(K, 0) if vectors == 1 else F.fuse_rows([mk(K // 2, 0), mk(K // 2, 1)], interleave=True) if vectors == 2
+            else F.fuse_rows([mk(32, 0), mk(16, 1), mk(K - 48, 2)])).to_tiled()
+
+
+@pytest.mark.parametrize("vectors", [1, 2, 3], ids=["plain", "gate_up", "qkv"])
+@pytest.mark.parametrize("case", EIGHT_BIT, ids=case_id)
+def test_gemv_of_8bit_codes_is_a_float32_sum(case, vectors):
+    """Decode of 8-bit codes: float32 sums of products that are not rounded first.  Two units of 2^-24 (1.2e-7) in
+    the 2-norm, for activations with outliers sixteen times the rest; digits of 24 bits below a chunk's
+    largest value have 2e-7 and more.  Short rows, the longest the matrix-core kernel takes (28672
+    columns) and one it does not take; main, column-split and slab arrangements, row m whatever M."""
+    for K, N in ((96, 384), (96, 2048), (112, 14336), (64, 28672)):
+        pm = _eight_bit(case, K, N, vectors, seed=N)
+        W = ops.dequant(pm, torch.float32).double()
+        x = acts(8, N, torch.float16, seed=N)
+        x[:, ::61] *= 16
+        x = x.to(DEV)
+        ref = x.double() @ W.t()
+        one = torch.cat([ops.gemv(pm, x[i:i + 1], out_dtype=torch.float32) for i in range(8)])
+        assert float((one.double() - ref).norm() / ref.norm()) < 1.2e-7, (K, N)
+        small = torch.empty(256, dtype=torch.uint8, device=DEV)
+        for M in (2, 3, 5, 8):
+            assert torch.equal(ops.gemv(pm, x[:M], out_dtype=torch.float32), one[:M]), (K, N, M)
+            assert torch.equal(ops.gemv(pm, x[:M], out_dtype=torch.float32, workspace=small), one[:M]), (K, N, M)
+    pm = _eight_bit(case, 64, 28800, vectors, seed=1)
+    x = acts(3, 28800, torch.float16, seed=2).to(DEV)
+    ref = x.double() @ ops.dequant(pm, torch.float32).double().t()
+    assert float((ops.gemv(pm, x, out_dtype=torch.float32).double() - ref).norm() / ref.norm()) < 1e-6
+
+
+@pytest.mark.parametrize("case", EIGHT_BIT[1:], ids=case_id)
+def test_gemv_of_8bit_codes_with_infinities_and_nan(case):
+    """An infinite activation gives +-inf, or NaN where it meets a weight that is 0; a NaN gives NaN; the
+    other rows are untouched.  Infinities in different chunks of a row, values at the ends of a chunk."""
+    K, N = 100, 2048
+    pm = _eight_bit(case, K, N, 1, seed=3)
+    W = ops.dequant(pm, torch.float32).double().cpu()
+    W[W == 0] = 0.0
+    clean = acts(8, N, torch.bfloat16, seed=5)
+    x = clean.clone()
+    x[1, 0] = float("inf")
+    x[2, 700] = float("nan")
+    x[3, 127] = float("-inf")
+    x[4, 128], x[4, 2047] = float("inf"), float("inf")
+    x[6, 5], x[6, 1500] = float("inf"), float("-inf")
+    ref = x.double() @ W.t()
+    for rows in ([1], [2], [3, 0], [0, 1, 2, 3], list(range(8))):
+        y = ops.gemv(pm, x[rows].to(DEV), out_dtype=torch.float32).cpu()
+        r = ref[rows]
+        assert torch.equal(torch.isnan(y), torch.isnan(r)) and torch.equal(torch.isinf(y), torch.isinf(r)), rows
+        assert torch.equal(y[torch.isinf(y)] > 0, r[torch.isinf(r)] > 0), rows
+        for i, m in enumerate(rows):
+            if bool(torch.isfinite(r[i]).all()):
+                assert torch.equal(y[i], ops.gemv(pm, clean[m:m + 1].to(DEV), out_dtype=torch.float32)[0].cpu())
+
+
 @pytest.mark.parametrize("case", DECODE_CASES, ids=case_id)
 def test_gemm_loses_no_more_than_operands_of_11_bits(case):
     """The error of the matrix-core GEMM against float64, for activations of both signs and of one, is no
