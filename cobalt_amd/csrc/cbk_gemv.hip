@@ -1162,6 +1162,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
 constexpr int GS_RED_THREADS = 256;
 static inline size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
 static inline size_t split_part_bytes(int ntiles, int sk, int Mk) { return (size_t)ntiles * sk * Mk * 16 * 4; }   // [tiles][parts][M][16] floats
+template <bool FOURS>                                                // 8-bit codes: the order of their main kernel, see parts_add
 __global__ __launch_bounds__(GS_RED_THREADS) void gemv_split_reduce_kernel(GsArgs a) {
   const GsHead& h = a.h;
   int idx = (int)blockIdx.x * GS_RED_THREADS + (int)threadIdx.x, mi = 0;
@@ -1184,14 +1185,14 @@ __global__ __launch_bounds__(GS_RED_THREADS) void gemv_split_reduce_kernel(GsArg
 #pragma unroll
   for (int j = 0; j < 16; ++j) pv[j] = gs.part[((size_t)(tile * SK + (j < SK ? j : SK - 1)) * M + am) * 16 + wr];
   float v = 0.f;
+  if constexpr (FOURS) {
 #pragma unroll
-  for (int j = 0; j < 16; ++j) pv[j] = j < SK ? pv[j] : 0.f;
-  if (gm.m.bits == 8) {                                             // (the order of the main kernel)
+    for (int j = 0; j < 16; ++j) pv[j] = j < SK ? pv[j] : 0.f;
 #pragma unroll
     for (int j = 0; j < 16; j += 4) v = parts_add<true>(v, pv[j], pv[j + 1], pv[j + 2], pv[j + 3]);
   } else {
 #pragma unroll
-    for (int j = 0; j < 16; j += 4) v = parts_add<false>(v, pv[j], pv[j + 1], pv[j + 2], pv[j + 3]);
+    for (int j = 0; j < 16; ++j) v += j < SK ? pv[j] : 0.f;
   }
   if (gm.bias) v += (h.ydt == CBK_F32) ? ((const float*)gm.bias)[k]
                   : (h.ydt == CBK_F16) ? h2f(((const uint16_t*)gm.bias)[k]) : bf2f(((const uint16_t*)gm.bias)[k]);
@@ -1994,7 +1995,7 @@ static int launch_gemv_stream_mfma(const DMat& m, const void* x, int xdt, int M,
           q.g.y = (uint8_t*)y + (size_t)m0 * ldy * ysz;
           const int th = (p.ntiles * mp * 16 + GS_RED_THREADS - 1) / GS_RED_THREADS * GS_RED_THREADS;
           r.h.th_end[0] = th;
-          hipLaunchKernelGGL(gemv_split_reduce_kernel, dim3(th / GS_RED_THREADS), dim3(GS_RED_THREADS), 0, st, r);
+          hipLaunchKernelGGL(gemv_split_reduce_kernel<false>, dim3(th / GS_RED_THREADS), dim3(GS_RED_THREADS), 0, st, r);
           if (hipGetLastError() != hipSuccess) return CBK_ERR_HIP;
         }
         return CBK_OK;
@@ -2432,7 +2433,7 @@ static int launch_split_cfg(const GsArgs& a, size_t lds, int blocks, int red_blo
   }
   hipLaunchKernelGGL(kern, dim3(blocks), dim3(GV_THREADS), lds, st, a);
   if (hipGetLastError() != hipSuccess) return CBK_ERR_HIP;
-  hipLaunchKernelGGL(gemv_split_reduce_kernel, dim3(red_blocks), dim3(GS_RED_THREADS), 0, st, a);
+  hipLaunchKernelGGL(gemv_split_reduce_kernel<(digits_of(BITS) == 4)>, dim3(red_blocks), dim3(GS_RED_THREADS), 0, st, a);
   return hipGetLastError() == hipSuccess ? CBK_OK : CBK_ERR_HIP;
 }
 template <int BITS, int KEEP>
