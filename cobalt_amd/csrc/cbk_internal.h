@@ -21,11 +21,15 @@ int gemm_as(const cbk_desc*, const GemmChoice&, const void* x, int x_dtype, int 
 
 // The rest of a module's image, written by the packing kernel along with the rows: the column
 // scales, the bytes between the arrays (zero), and two figures about what was packed.
-constexpr int PACK_SLOTS = 64, PACK_SLOT_WORDS = 16;
+constexpr int PACK_ROWS = 16, PACK_COLS = 4096, PACK_RECORDS = 4096;  // a workgroup's slab; workgroups at most
+inline int pack_records(int64_t K, int64_t N) {
+  const int64_t b = (K + PACK_ROWS - 1) / PACK_ROWS * ((N + PACK_COLS - 1) / PACK_COLS);
+  return (int)(b < PACK_RECORDS ? b : PACK_RECORDS);
+}
 struct PackExtra {
-  // PACK_SLOTS x PACK_SLOT_WORDS, zeroed by the caller: status bits, groups re-derived, largest zero
-  // point stored, survivors in the mask.  Workgroup b adds to slot b % PACK_SLOTS, a cache line each:
-  // all workgroups on one address cost 25 us of a 50 us kernel.
+  // pack_records(K, N) x 4 words, one record per workgroup: status bits, groups re-derived, largest zero
+  // point stored, survivors in the mask.  Plain stores that the host adds up: nothing has to be cleared before the
+  // kernel, and no cache line is shared (atomics of all workgroups on one line cost 25 us of a 50 us kernel).
   uint32_t* counts;
   const void* cs_src;          // column scales to copy (16-byte aligned), or nullptr
   void* cs_dst;

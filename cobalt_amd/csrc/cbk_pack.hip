@@ -26,6 +26,7 @@ struct PackArgs {
   uint8_t* ozero;
   int K, N, G, group, keep, tiled, zero_f16, fix_zero;
   uint32_t stride;
+  int slabs, blocks;       // slabs of a row tile, and of the image
   int krows;               // rows of the image: K, or K padded to a multiple of 16 in the tiled order
   uint32_t tail;           // readable bytes behind the last row, zeroed
   int* status;             // see below, or nullptr
@@ -81,7 +82,7 @@ __device__ inline GroupQ group_quant(const PackArgs& a, float nl, uint32_t sz, c
   return r;
 }
 
-constexpr int PK_ROWS = 16, PK_COLS = 4096, PK_THREADS = 512;
+constexpr int PK_ROWS = PACK_ROWS, PK_COLS = PACK_COLS, PK_THREADS = 512;
 
 // permute selectors that move the survivors of eight bytes together: output byte i takes the i-th
 // survivor (zero past the last)
@@ -102,6 +103,8 @@ __device__ inline uint2 compress_selectors(uint32_t mb) {
 template <int bits>
 __device__ inline uint64_t narrow8(uint32_t lo, uint32_t hi) {
   if (bits == 8) return (uint64_t)lo | ((uint64_t)hi << 32);
+  // (bytes 0 and 2 of x | x >> 4 are the pairs of nibbles, as no code has bits above them)
+  if (bits == 4) return (uint64_t)perm(hi | (hi >> 4), lo | (lo >> 4), 0x06040200u);
   auto four = [&](uint32_t x) -> uint32_t {                         // four bytes -> 4 * bits bits
     const uint32_t mask = ((1u << bits) - 1u) * 0x00010001u;
     const uint32_t y = (x & mask) | (((x >> 8) & mask) << bits);    // pairs at bits 0 and 16
@@ -117,13 +120,14 @@ template <int FAM, int BITS>
 __global__ __launch_bounds__(PK_THREADS) void pack_rows_kernel(PackArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint32_t img[];   // [PK_ROWS][code bytes of a slab (+ its BLK6 high plane)]
   __shared__ uint2 lut[256];
-  __shared__ uint32_t tot[4];                                      // status bits, groups re-derived, largest zero, survivors
+  __shared__ uint4 tot[PK_THREADS / 64];                            // status bits, groups re-derived, largest zero, survivors
   const int tid = threadIdx.x;
   constexpr bool dense = FAM == FAM_DENSE, blk6 = FAM == FAM_BLK6;
   if (tid < 256) lut[tid] = compress_selectors((uint32_t)tid);
-  if (tid < 4) tot[tid] = 0;
-  const int slabs = (a.N + PK_COLS - 1) / PK_COLS;
-  const int rt = blockIdx.x / slabs, c0 = (blockIdx.x % slabs) * PK_COLS, k0 = rt * PK_ROWS;
+  uint32_t st = 0, fixed = 0, zmax = 0, surv = 0;
+  // (one slab per workgroup but for images of more than PACK_RECORDS slabs)
+  for (int slab = blockIdx.x; slab < a.blocks; slab += gridDim.x) {
+  const int rt = slab / a.slabs, c0 = (slab % a.slabs) * PK_COLS, k0 = rt * PK_ROWS;
   const int cols = a.N - c0 < PK_COLS ? a.N - c0 : PK_COLS, nb = cols >> 5;
   constexpr int pb = blk6 ? 4 : BITS;                               // bits per code of the code plane
   const int cb = (dense ? 32 : a.keep) * pb;                       // code bits of a block
@@ -135,32 +139,39 @@ __global__ __launch_bounds__(PK_THREADS) void pack_rows_kernel(PackArgs a) {
   __syncthreads();
   const float nl = (float)((1u << BITS) - 1u);
   const uint32_t over = ~((uint32_t)nl * 0x01010101u);             // bits that no code of this width has
-  uint32_t st = 0, fixed = 0, zmax = 0, surv = 0;
   // codes, mask, scale and zero point of the next block are in flight while one is packed
   struct In { uint4 qa, qb; uint32_t m, sz; };
-  const int items = (a.K - k0 < PK_ROWS ? a.K - k0 : PK_ROWS) * nb;  // (padding rows have no blocks)
-  auto load = [&](int it) -> In {
-    it = it < items ? it : items - 1;
-    const int k = k0 + it / nb, c = c0 + 32 * (it % nb);
-    const size_t gi = (size_t)k * a.G + (uint32_t)c / (uint32_t)a.group;
-    const uint8_t* qp = a.q + (size_t)k * a.N + c;
+  const int rows_in = a.K - k0 < PK_ROWS ? a.K - k0 : PK_ROWS;      // (padding rows have no blocks)
+  // a thread's blocks: every PK_THREADS-th of the slab's, row by row
+  const int drow = PK_THREADS / nb, dt = PK_THREADS % nb, lg = a.group == 64 ? 6 : 7;
+  const uint8_t* qb = a.q + (size_t)k0 * a.N + c0;
+  const uint8_t* mb = a.mask ? a.mask + (size_t)k0 * plane + (c0 >> 3) : nullptr;
+  const size_t gb = (size_t)k0 * a.G + (c0 >> lg);
+  const uint16_t* sb = a.scale + gb;
+  const uint8_t* zb = (const uint8_t*)a.zero + (a.zero_f16 ? 2 * gb : gb);
+  auto load = [&](int row, int t) -> In {
+    if (row >= rows_in) { row = rows_in - 1; t = 0; }
+    // (sixteen rows: 32-bit offsets from an address all threads share)
+    const uint32_t gi = (uint32_t)row * (uint32_t)a.G + (((uint32_t)t * 32u) >> lg), qo = (uint32_t)row * (uint32_t)a.N + (uint32_t)t * 32u;
     In x;
-    x.qa = *(const uint4*)qp; x.qb = *(const uint4*)(qp + 16);
-    x.m = a.mask ? *(const uint32_t*)(a.mask + (size_t)k * plane + (c >> 3)) : 0xffffffffu;
-    x.sz = (uint32_t)a.scale[gi] | ((a.zero_f16 ? (uint32_t)((const uint16_t*)a.zero)[gi] : (uint32_t)((const uint8_t*)a.zero)[gi]) << 16);
+    x.qa = *(const uint4*)(qb + qo); x.qb = *(const uint4*)(qb + 16 + qo);
+    x.m = mb ? *(const uint32_t*)(mb + (uint32_t)row * plane + (uint32_t)t * 4u) : 0xffffffffu;
+    x.sz = (uint32_t)sb[gi] | ((a.zero_f16 ? (uint32_t)((const uint16_t*)zb)[gi] : (uint32_t)zb[gi]) << 16);
     return x;
   };
-  In nx = load(tid);
-  for (int it = tid; it < items; it += PK_THREADS) {
+  int row = tid / nb, t = tid % nb;
+  In nx = load(row, t);
+  for (int nrow, nt; row < rows_in; row = nrow, t = nt) {
     const In cur = nx;
-    nx = load(it + PK_THREADS);
-    const int row = it / nb, t = it % nb, k = k0 + row;
-    const int c = c0 + 32 * t, g = (uint32_t)c / (uint32_t)a.group;
+    nrow = row + drow; nt = t + dt;
+    if (nt >= nb) { nt -= nb; ++nrow; }
+    nx = load(nrow, nt);
+    const int k = k0 + row, c = c0 + 32 * t, g = c >> lg;
     uint32_t q[8] = {cur.qa.x, cur.qa.y, cur.qa.z, cur.qa.w, cur.qb.x, cur.qb.y, cur.qb.z, cur.qb.w};
     const uint32_t m = cur.m;
     surv += (uint32_t)__popc(m);
     const GroupQ gq = group_quant(a, nl, cur.sz, q, m);
-    if (c % a.group == 0) {                                        // the group's first block stores its quantisation
+    if ((c & (a.group - 1)) == 0) {                                // the group's first block stores its quantisation
       const size_t mi = a.tiled ? ((size_t)rt * a.G + g) * 16 + row : (size_t)k * a.G + g;
       a.oscale[mi] = gq.s_out;
       a.ozero[mi] = (uint8_t)gq.z_out;
@@ -282,27 +293,34 @@ __global__ __launch_bounds__(PK_THREADS) void pack_rows_kernel(PackArgs a) {
       a.oscale[mi] = 0;
       a.ozero[mi] = 0;
     }
+  if (slab + (int)gridDim.x < a.blocks) __syncthreads();           // the image has been read
+  }
   if (blockIdx.x == 0 && tid < (int)(a.tail >> 4)) ((uint4*)(a.data + (size_t)a.krows * a.stride))[tid] = make_uint4(0, 0, 0, 0);
   for (uint32_t i = blockIdx.x * (uint32_t)PK_THREADS + tid; i < a.extra.cs_units; i += gridDim.x * (uint32_t)PK_THREADS)
     ((uint4*)a.extra.cs_dst)[i] = ((const uint4*)a.extra.cs_src)[i];
   if (blockIdx.x == 0)
     for (int i = 0; i < 4; ++i)
       if (tid < (int)a.extra.gap_bytes[i]) a.extra.gap[i][tid] = 0;
-  if (a.status || a.extra.counts) {                                       // one update per workgroup
-    if (st) atomicOr(&tot[0], st);
-    if (fixed) atomicAdd(&tot[1], fixed);
-    if (a.extra.counts) { atomicMax(&tot[2], zmax); atomicAdd(&tot[3], surv); }
+  if (a.status || a.extra.counts) {                                 // one record per workgroup, added over lanes, then wavefronts
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      st |= (uint32_t)__shfl_xor((int)st, o);
+      fixed += (uint32_t)__shfl_xor((int)fixed, o);
+      const uint32_t z = (uint32_t)__shfl_xor((int)zmax, o);
+      zmax = zmax > z ? zmax : z;
+      surv += (uint32_t)__shfl_xor((int)surv, o);
+    }
+    if ((tid & 63) == 0) tot[tid >> 6] = make_uint4(st, fixed, zmax, surv);
     __syncthreads();
     if (tid == 0) {
-      if (a.status && tot[0]) atomicOr(a.status, (int)tot[0]);
-      if (a.status && tot[1]) atomicAdd(a.status + 1, (int)tot[1]);
-      if (a.extra.counts) {
-        uint32_t* c = a.extra.counts + (blockIdx.x % PACK_SLOTS) * PACK_SLOT_WORDS;
-        if (tot[0]) atomicOr(c, tot[0]);
-        if (tot[1]) atomicAdd(c + 1, tot[1]);
-        atomicMax(c + 2, tot[2]);
-        atomicAdd(c + 3, tot[3]);
+      uint4 t = tot[0];
+      for (int w = 1; w < PK_THREADS / 64; ++w) {
+        const uint4 u = tot[w];
+        t.x |= u.x; t.y += u.y; t.z = t.z > u.z ? t.z : u.z; t.w += u.w;
       }
+      if (a.status && t.x) atomicOr(a.status, (int)t.x);
+      if (a.status && t.y) atomicAdd(a.status + 1, (int)t.y);
+      if (a.extra.counts) ((uint4*)a.extra.counts)[blockIdx.x] = t;
     }
   }
 }
@@ -481,7 +499,7 @@ int launch_repack_dense4(const DMat& m, const DMat& d, hipStream_t st) {
 }
 
 template <int FAM, int BITS>
-static int launch_pack_cfg(const PackArgs& a, int64_t blocks, size_t lds, hipStream_t st) {
+static int launch_pack_cfg(const PackArgs& a, size_t lds, hipStream_t st) {
   auto kern = pack_rows_kernel<FAM, BITS>;
   static std::atomic<int> configured{0};
   if (!configured.load(std::memory_order_acquire)) {               // 64 KB for a slab of 8-bit codes, and the table
@@ -489,7 +507,7 @@ static int launch_pack_cfg(const PackArgs& a, int64_t blocks, size_t lds, hipStr
       return CBK_ERR_HIP;
     configured.store(1, std::memory_order_release);
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(PK_THREADS), lds, st, a);
+  hipLaunchKernelGGL(kern, dim3((unsigned)pack_records(a.K, a.N)), dim3(PK_THREADS), lds, st, a);
   return hipGetLastError() == hipSuccess ? CBK_OK : CBK_ERR_HIP;
 }
 
@@ -507,19 +525,20 @@ int launch_pack(const DMat& m, const void* mask, const void* q, const void* scal
   a.tail = m.tiled ? 512 : 64;
   a.status = status;
   a.extra = extra ? *extra : PackExtra{};
-  const int64_t blocks = (int64_t)((m.K + PK_ROWS - 1) / PK_ROWS) * ((m.N + PK_COLS - 1) / PK_COLS);
+  a.slabs = (m.N + PK_COLS - 1) / PK_COLS;
+  a.blocks = (m.K + PK_ROWS - 1) / PK_ROWS * a.slabs;
   const int cols = m.N < PK_COLS ? m.N : PK_COLS, pb = fam == FAM_BLK6 ? 4 : m.bits;
   const size_t row = (size_t)((cols / 32) * (fam == FAM_DENSE ? 32 : m.keep) * pb + 127) / 128 * 16 +
                      (fam == FAM_BLK6 ? (size_t)cols / 8 : 0);
-  if (fam == FAM_BLK6) return launch_pack_cfg<FAM_BLK6, 6>(a, blocks, PK_ROWS * row, st);
+  if (fam == FAM_BLK6) return launch_pack_cfg<FAM_BLK6, 6>(a, PK_ROWS * row, st);
   if (fam == FAM_DENSE)
-    return m.bits == 2 ? launch_pack_cfg<FAM_DENSE, 2>(a, blocks, PK_ROWS * row, st)
-         : m.bits == 3 ? launch_pack_cfg<FAM_DENSE, 3>(a, blocks, PK_ROWS * row, st)
-         : m.bits == 4 ? launch_pack_cfg<FAM_DENSE, 4>(a, blocks, PK_ROWS * row, st)
-                       : launch_pack_cfg<FAM_DENSE, 8>(a, blocks, PK_ROWS * row, st);
-  return m.bits == 2 ? launch_pack_cfg<FAM_BLK, 2>(a, blocks, PK_ROWS * row, st)
-       : m.bits == 3 ? launch_pack_cfg<FAM_BLK, 3>(a, blocks, PK_ROWS * row, st)
-                     : launch_pack_cfg<FAM_BLK, 4>(a, blocks, PK_ROWS * row, st);
+    return m.bits == 2 ? launch_pack_cfg<FAM_DENSE, 2>(a, PK_ROWS * row, st)
+         : m.bits == 3 ? launch_pack_cfg<FAM_DENSE, 3>(a, PK_ROWS * row, st)
+         : m.bits == 4 ? launch_pack_cfg<FAM_DENSE, 4>(a, PK_ROWS * row, st)
+                       : launch_pack_cfg<FAM_DENSE, 8>(a, PK_ROWS * row, st);
+  return m.bits == 2 ? launch_pack_cfg<FAM_BLK, 2>(a, PK_ROWS * row, st)
+       : m.bits == 3 ? launch_pack_cfg<FAM_BLK, 3>(a, PK_ROWS * row, st)
+                     : launch_pack_cfg<FAM_BLK, 4>(a, PK_ROWS * row, st);
 }
 
 }  // namespace cbk

@@ -465,7 +465,7 @@ PyObject* py_pack_begin(PyObject*, PyObject* const* a, Py_ssize_t n) {
       if (cs_rows) {
         x.cs_src = cs.const_data_ptr(); x.cs_dst = base + off[3]; x.cs_units = (uint32_t)(size[3] / 16);
       }
-      at::Tensor counts = at::zeros({cbk::PACK_SLOTS * cbk::PACK_SLOT_WORDS}, bytes.dtype(at::kInt));
+      at::Tensor counts = at::empty({cbk::pack_records(K, N), 4}, bytes.dtype(at::kInt));
       x.counts = (uint32_t*)counts.mutable_data_ptr();
       rc = cbk::pack_image(&d, mask.defined() ? mask.const_data_ptr() : nullptr, q.const_data_ptr(), scale.const_data_ptr(),
                            zero.const_data_ptr(), zero.scalar_type() == at::kByte ? CBK_U8 : CBK_F16, fix ? 1 : 0, nullptr, &x,
@@ -495,7 +495,7 @@ PyObject* py_pack_end(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const uint32_t* h = (const uint32_t*)host.const_data_ptr();
     uint32_t status = 0, fixed = 0, zmax = 0;
     unsigned long long surv = 0;
-    for (int i = 0; i < cbk::PACK_SLOTS; ++i, h += cbk::PACK_SLOT_WORDS) {
+    for (int64_t i = 0, n = host.size(0); i < n; ++i, h += 4) {
       status |= h[0]; fixed += h[1]; surv += h[3];
       zmax = zmax > h[2] ? zmax : h[2];
     }

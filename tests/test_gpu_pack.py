@@ -318,3 +318,20 @@ def test_pack_and_unpack_at_the_smallest_and_ragged_shapes():
                                     pm.to_rowmajor().array("zero").view(K, -1), _t(raw["col_scale"]), layout, bits, group,
                                     keep or None, fix_zero=False, tiled=tiled)
                 assert torch.equal(back.blob, pm.blob), (case_id(case), K, N, tiled)
+
+
+@pytest.mark.parametrize("K,N", [(16 * 4096 + 19, 128), (35, 4096 + 384)], ids=["more_slabs_than_workgroups", "two_slabs_of_columns"])
+def test_pack_walks_every_slab_and_adds_their_records(K, N):
+    """A workgroup packs sixteen rows of 4096 columns at a time; from 4097 such slabs on it takes several.  The bytes and the
+    figures gathered on the way (groups re-derived, zero-point flags) are those of the torch packer."""
+    g = torch.Generator().manual_seed(K + N)
+    kept = torch.zeros(K, N // 32, 32, dtype=torch.bool).scatter_(-1, torch.rand(K, N // 32, 32, generator=g).topk(10, -1).indices, True)
+    zero = torch.randint(0, 8, (K, N // 64), generator=g)
+    zero[K - 1, -1] = 11                                              # off the grid of 3-bit codes: the last slab's
+    zero[K // 2, 0] = 9
+    args = (F.pack_mask(kept.view(K, N)), torch.randint(0, 8, (K, N), generator=g).to(torch.uint8),
+            (torch.rand(K, N // 64, generator=g) * 0.01 + 1e-3).half(), zero.half(), torch.rand(N, generator=g).half())
+    want = F.pack_raw(*args, F.BLKC, 3, 64, 10).to_tiled()
+    got = ops.pack_raw(*[a.to(DEV) for a in args], F.BLKC, 3, 64, 10, tiled=True)
+    assert torch.equal(got.blob.cpu(), want.blob)
+    assert (got.n_zero_fixed, got.flags, got.n_survivors) == (2, want.flags, want.n_survivors)
