@@ -211,7 +211,7 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
   if (BITMAP) {
     const uint2 e = make_selectors((uint32_t)tid, C::SEL_KIND);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) lut[tid * 8 + j] = e;
+    for (int j = 0; j < 8; ++j) lut[table_slot<8, 8>(tid, j)] = e;
   }
   const uint32_t l8 = lane & 7;
 

@@ -170,7 +170,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         constexpr uint32_t F = C::HI2 ? 0xFFu : C::SB == 4 ? 0xF0u : 0x03u;
         const uint32_t k0 = bits_to_bytes((uint32_t)tid) * F, k1 = bits_to_bytes((uint32_t)tid >> 4) * F;
 #pragma unroll
-        for (int j = 0; j < SK_LUT_LANES; ++j) lut[tid * SK_LUT_LANES + j] = make_uint4(e.x, e.y, C::HI2 ? ~k0 : k0, C::HI2 ? ~k1 : k1);
+        for (int j = 0; j < SK_LUT_LANES; ++j) lut[table_slot<SK_LUT_LANES, 16>(tid, j)] = make_uint4(e.x, e.y, C::HI2 ? ~k0 : k0, C::HI2 ? ~k1 : k1);
       }
       // (a barrier over LDS only: __syncthreads() would wait for the loads in flight)
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");

@@ -656,7 +656,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
     if (tid < 256) {
       const uint2 e = make_selectors((uint32_t)tid, C0::SEL_KIND);
 #pragma unroll
-      for (int j = 0; j < LUT_LANES; ++j) lut[tid * LUT_LANES + j] = e;
+      for (int j = 0; j < LUT_LANES; ++j) lut[table_slot<LUT_LANES, 8>(tid, j)] = e;
     } else if (tid < 256 + ZERO_BYTES / 4) {
       ((uint32_t*)zreg)[tid - 256] = 0u;
     } else if (tid < 256 + ZERO_BYTES / 4 + CNT_SLOTS) {
@@ -1057,7 +1057,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
   if (tid < 256) {
     const uint2 e = make_selectors((uint32_t)tid, C::SEL_KIND);
 #pragma unroll
-    for (int j = 0; j < LUT_LANES; ++j) lut[tid * LUT_LANES + j] = e;
+    for (int j = 0; j < LUT_LANES; ++j) lut[table_slot<LUT_LANES, 8>(tid, j)] = e;
   } else if (tid < 256 + ZERO_BYTES / 4) {
     ((uint32_t*)zreg)[tid - 256] = 0u;
   } else if (tid < 256 + ZERO_BYTES / 4 + 4 * M) {                  // deltas of the chunks past N
@@ -1382,7 +1382,7 @@ __global__ __launch_bounds__(ST_THREADS) void gemv_stream_kernel(DMat m, const u
   if (tid < 256) {
     const uint2 e = make_selectors((uint32_t)tid, 0);
 #pragma unroll
-    for (int j = 0; j < ST_LUT_LANES; ++j) lut[tid * ST_LUT_LANES + j] = e;
+    for (int j = 0; j < ST_LUT_LANES; ++j) lut[table_slot<ST_LUT_LANES, 8>(tid, j)] = e;
   }
   const int n16 = N >> 4, xitems = M * n16;                      // a multiple of 8
   for (int it = tid; it < xitems; it += ST_THREADS) {
@@ -1786,7 +1786,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_stream_mfma_kernel(SmArgs a) 
   if (tid < 256) {
     const uint2 e = make_selectors((uint32_t)tid, 0);
 #pragma unroll
-    for (int j = 0; j < LUT_LANES; ++j) lut[tid * LUT_LANES + j] = e;
+    for (int j = 0; j < LUT_LANES; ++j) lut[table_slot<LUT_LANES, 8>(tid, j)] = e;
   } else if (tid < 256 + (ZERO_BYTES + CNT_BYTES) / 4) {
     ((uint32_t*)zreg)[tid - 256] = 0u;                             // zero row and counters
   } else if (SPLIT && tid < 256 + (ZERO_BYTES + CNT_BYTES) / 4 + 4 * M) {       // deltas of the chunks past N

@@ -12,7 +12,7 @@ constexpr int OCT_LUT_LANES = 4;                                    // lane-priv
 __device__ inline void octet_table(uint2 (&lut)[256 * OCT_LUT_LANES]) {   // 256 threads; the caller synchronises
   const uint2 e = make_selectors(threadIdx.x, 0);
 #pragma unroll
-  for (int j = 0; j < OCT_LUT_LANES; ++j) lut[threadIdx.x * OCT_LUT_LANES + j] = e;
+  for (int j = 0; j < OCT_LUT_LANES; ++j) lut[table_slot<OCT_LUT_LANES, 8>(threadIdx.x, j)] = e;
 }
 
 // eight 2-bit codes -> eight nibbles
