@@ -53,6 +53,7 @@ constexpr int GV_THREADS = GV_WAVES * 64;
 #endif
 constexpr int LUT_LANES = CBK_LUT_LANES;      // lane-private copies of the selector table
 constexpr int LUT_BYTES = 256 * LUT_LANES * 8;
+constexpr int WIDE_LUT_LANES = 16, WIDE_LUT_BYTES = 256 * WIDE_LUT_LANES * 16;   // one activation row: see fetch_selectors
 constexpr int ZERO_BYTES = 256;
 constexpr int CNT_SLOTS = 64;                 // most reduction slots (arrival counters)
 constexpr int CNT_BYTES = CNT_SLOTS * 4;       // at a fixed place: zeroed before the arguments are read
@@ -332,14 +333,56 @@ __device__ inline void split_mask(uint32_t mw, uint32_t (&mb)[4], uint32_t (&rk)
   }
 }
 
-// ranks and table reads of one block
-template <class C>
-__device__ inline void fetch_selectors(uint32_t mw, const uint2* lut, uint32_t l16, uint32_t (&rk)[4], uint2 (&sel4)[4]) {
-  uint32_t mb[4];
-  split_mask<C>(mw, mb, rk);
-  if (!C::DENSE) {
+template <bool WT>
+__device__ inline uint32_t table_lane(int lane) {                   // offset of this lane's copy in an entry
+  return WT ? (uint32_t)(lane & (WIDE_LUT_LANES - 1)) * 16u : (uint32_t)(lane & (LUT_LANES - 1)) * 8u;
+}
+// (the wide one by the last wavefronts: the first ones convert the activations)
+template <class C, bool WT>
+__device__ inline void build_table(uint8_t* lut, int tid) {
+  if (C::DENSE) return;
+  if (WT && tid >= GV_THREADS - 256) {
+    const uint32_t mb = (uint32_t)tid & 255u;
+    const uint2 e = make_selectors(mb, C::SEL_KIND);
+    const uint4 w = make_uint4(e.x, e.y, (uint32_t)__builtin_popcount(mb) * C::SB, 0u);
 #pragma unroll
-    for (int jj = 0; jj < 4; ++jj) sel4[jj] = lut[mb[jj] * LUT_LANES + l16];
+    for (int j = 0; j < WIDE_LUT_LANES; ++j) ((uint4*)lut)[table_slot<WIDE_LUT_LANES, 16>(mb, j)] = w;
+  } else if (!WT && tid < 256) {
+    const uint2 e = make_selectors((uint32_t)tid, C::SEL_KIND);
+#pragma unroll
+    for (int j = 0; j < LUT_LANES; ++j) ((uint2*)lut)[table_slot<LUT_LANES, 8>(tid, j)] = e;
+  }
+}
+
+// Table reads of one block: selectors, and in `sh` the bits of the code stream before each mask byte.
+// WT: the wide table, 16-byte entries of selectors and the stream bits of the byte's survivors, 256 bytes (sixteen
+// copies) apart, so that one permute of mask word and lane offset is an entry's address and the counting is done by
+// the table.  The small one has 8-byte entries, eight copies: an address takes a field extract and a shift and add,
+// the counts a population count and a shift.  Per mask byte, four wavefronts per SIMD: 42 cycles of vector
+// instructions with the small table, 34 with the wide one; a wavefront's table read takes the LDS 5.9 cycles (eight
+// copies of 8 bytes: conflicts) and 4.3.  Two layers of 5376 / 21504 columns at one row, weights from memory, 112.3 ->
+// 110.6 us, of which the launches that are long enough (see launch_main_batch) take 0.3 - 0.7 less each; what is left of
+// those is memory.
+template <class C, bool WT>
+__device__ inline void fetch_selectors(uint32_t mw, const uint8_t* lut, uint32_t lane_off, uint32_t (&sh)[4], uint2 (&sel4)[4]) {
+  if constexpr (WT) {
+    sh[0] = 0;
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) {                                // mask byte in byte 1, this lane's copy in byte 0
+      const uint4 e = *(const uint4*)(lut + perm(mw, lane_off, 0x0C0C0400u + ((uint32_t)jj << 8)));
+      sel4[jj] = make_uint2(e.x, e.y);
+      if (jj < 3) sh[jj + 1] = sh[jj] + e.z;
+    }
+  } else {
+    uint32_t mb[4], rk[4];
+    split_mask<C>(mw, mb, rk);
+    if (!C::DENSE) {
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {
+        sel4[jj] = *(const uint2*)(lut + mb[jj] * (LUT_LANES * 8) + lane_off);
+        sh[jj] = rk[jj] * C::SB;
+      }
+    }
   }
 }
 
@@ -347,7 +390,7 @@ __device__ inline void fetch_selectors(uint32_t mw, const uint2* lut, uint32_t l
 // pruned columns 0: the B operand of one MFMA.
 // sel4: the selectors of the block's four mask bytes, read from the table by fetch_selectors.
 template <class C, int BITS>
-__device__ inline void decode_half(const uint32_t (&st)[C::NW], const uint32_t (&rk)[4], const uint2 (&sel4)[4],
+__device__ inline void decode_half(const uint32_t (&st)[C::NW], const uint32_t (&sh)[4], const uint2 (&sel4)[4],
                                    uint32_t nz, int half, uint32_t (&bfrag)[4], uint32_t hw = 0) {
   if constexpr (BITS == 8) {                             // q - 128; the zero point is a second operand (zero8)
 #pragma unroll
@@ -372,10 +415,10 @@ __device__ inline void decode_half(const uint32_t (&st)[C::NW], const uint32_t (
     } else {
       uint32_t w;
       if (jj == 0) w = st[0];
-      else w = window<C::NW>(st, rk[jj] * C::SB);
+      else w = window<C::NW>(st, sh[jj]);
       if (C::HI2) {
         uint32_t h0, h1;
-        hi2_pools(hw, jj == 0 ? 0u : rk[jj], h0, h1);
+        hi2_pools(hw, jj == 0 ? 0u : sh[jj] / C::SB, h0, h1);
         p0 = bias_pool((w & 0x0F0F0F0Fu) | h0, nz);
         p1 = bias_pool(((w >> 4) & 0x0F0F0F0Fu) | h1, nz);
       } else if (C::SB == 4) {
@@ -521,8 +564,8 @@ __device__ inline void load_chunk(const StepAt& p, int S4, int kq, Loads<C>& L) 
 // launches, 3-bit codes, 10 of 32 kept: 21504 x 5376 23.4 -> 21.3 us at M = 4, 45.6 -> 23.0 at M = 8; 5376 x 21504, rows
 // split by columns now, 35.2 -> 19.6 and 69.5 -> 21.4.)
 struct XDigits { uint32_t xq_off, z_off; const float* delta; int Ns, ch0, NCH, M; };   // staged digits and deltas
-template <class C, int BITS, int NG, bool TURN>
-__device__ inline void block_step(const Loads<C>& cur, const uint8_t* smem, const uint2* lut, uint32_t l16, int lane, int S,
+template <class C, int BITS, int NG, bool TURN, bool WT>
+__device__ inline void block_step(const Loads<C>& cur, const uint8_t* smem, const uint8_t* lut, uint32_t lane_off, int lane, int S,
                                   const XDigits& x, float (&ysum)[4 * NG]) {
   constexpr int NGC = C::NGC, ND = digits_of(BITS);
   const int wr = lane & 15, kq = lane >> 4;
@@ -570,9 +613,9 @@ __device__ inline void block_step(const Loads<C>& cur, const uint8_t* smem, cons
 #pragma unroll
       for (int h = 0; h < NGC; ++h)
         aaddr[g][h] = (a_on[g] && chunk < x.NCH && (NGC == 1 || (kq >> 1) == h)) ? a_base[g] + (uint32_t)(chunk - x.ch0) * 128u : x.z_off;
-    uint32_t rkc[4];
+    uint32_t shc[4];
     uint2 selc[4];
-    fetch_selectors<C>(TURN ? mk4[c] : cur.mk[c], lut, l16, rkc, selc);
+    fetch_selectors<C, WT>(TURN ? mk4[c] : cur.mk[c], lut, lane_off, shc, selc);
     uint32_t st[C::NW];
 #pragma unroll
     for (int k = 0; k < C::NW; ++k) {
@@ -589,7 +632,7 @@ __device__ inline void block_step(const Loads<C>& cur, const uint8_t* smem, cons
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       uint32_t bfrag[4];
-      decode_half<C, BITS>(st, rkc, selc, nz, half, bfrag, TURN && C::HI2 ? hw4[c] : 0u);
+      decode_half<C, BITS>(st, shc, selc, nz, half, bfrag, TURN && C::HI2 ? hw4[c] : 0u);
       const v4i bv = (v4i){(int)bfrag[0], (int)bfrag[1], (int)bfrag[2], (int)bfrag[3]};
 #pragma unroll
       for (int g = 0; g < NG; ++g)
@@ -622,7 +665,7 @@ __device__ inline void block_step(const Loads<C>& cur, const uint8_t* smem, cons
   }
 }
 
-template <int BITS, int KEEP, int GRP, int MP>
+template <int BITS, int KEEP, int GRP, int MP, bool WT>
 __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
   using C = Cfg<BITS, KEEP, GRP, MP>;
   static_assert(MP == 1 || MP == 2 || MP == 4 || MP == 8, "single activation rows, or row groups of four");
@@ -632,8 +675,8 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);     // in a scalar register: positions are scalar work
-  uint2* lut = (uint2*)smem;
-  uint8_t* zreg = smem + LUT_BYTES;
+  uint8_t* lut = smem;
+  uint8_t* zreg = smem + (WT ? WIDE_LUT_BYTES : LUT_BYTES);
   int* cnt = (int*)(zreg + ZERO_BYTES);                // [CNT_SLOTS] arrival counters
   int8_t* xq = (int8_t*)cnt + CNT_BYTES;
   // The argument block is read in two dependent steps (header, then the record of the first
@@ -653,10 +696,8 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
   // staging of the first matrix's activations (nothing reads them before).
   {
     using C0 = Cfg<BITS, KEEP, GRP, MP>;
+    build_table<C0, WT>(lut, tid);
     if (tid < 256) {
-      const uint2 e = make_selectors((uint32_t)tid, C0::SEL_KIND);
-#pragma unroll
-      for (int j = 0; j < LUT_LANES; ++j) lut[table_slot<LUT_LANES, 8>(tid, j)] = e;
     } else if (tid < 256 + ZERO_BYTES / 4) {
       ((uint32_t*)zreg)[tid - 256] = 0u;
     } else if (tid < 256 + ZERO_BYTES / 4 + CNT_SLOTS) {
@@ -669,7 +710,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
   float* red = delta + h.delta_cap;                    // [nslot][sk_cap][M][16] partial sums
 
   const int wr = lane & 15, kq = lane >> 4;            // weight row in tile / lane quarter
-  const uint32_t l16 = lane & (LUT_LANES - 1);
+  const uint32_t lane_off = table_lane<WT>(lane);
   // role of this lane's row in the A operand: variant i = lane%16 = 4 * quarter + digit
   // (digit 3 is an all-zero row where there are three); in the result, lane quarter kq holds the three digit sums
   // of its own chunk, so every lane post-processes exactly the chunk it decoded
@@ -825,7 +866,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
       // the compiler no longer spreads them over the decode, and every launch was 2-6 % slower)
       issue(t_lo + p1.tl, p1.S, tgt);
       if constexpr (QB) {
-        block_step<C, BITS, NG, TURN>(cur, smem, lut, l16, lane, S, XDigits{xq_off, z_off, delta, Ns, ch0, NCH, h.M}, ysum);
+        block_step<C, BITS, NG, TURN, WT>(cur, smem, lut, lane_off, lane, S, XDigits{xq_off, z_off, delta, Ns, ch0, NCH, h.M}, ysum);
       } else
       {
         const int chunk = 4 * S + kq;
@@ -846,9 +887,9 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
 
 #pragma unroll
         for (int jb = 0; jb < 4; ++jb) {
-          uint32_t rkc[4];
+          uint32_t shc[4];
           uint2 selc[4];
-          fetch_selectors<C>(cur.mk[jb], lut, l16, rkc, selc);
+          fetch_selectors<C, WT>(cur.mk[jb], lut, lane_off, shc, selc);
           uint32_t st[C::NW];                                     // code stream of block jb
           block_stream<C, BITS>(cw, jb, st);
           const uint32_t z = (C::NGC == 1) ? cur.zraw : ((cur.zraw >> (8 * (jb >> 1))) & 0xFFu);
@@ -857,7 +898,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
           for (int half = 0; half < 2; ++half) {
             const int t = 2 * jb + half;                            // fragment index in the chunk
             uint32_t bfrag[4];
-            decode_half<C, BITS>(st, rkc, selc, nz, half, bfrag, C::HI2 ? cur.h2[C::HI2 ? jb : 0] : 0u);
+            decode_half<C, BITS>(st, shc, selc, nz, half, bfrag, C::HI2 ? cur.h2[C::HI2 ? jb : 0] : 0u);
             const v4i bv = (v4i){(int)bfrag[0], (int)bfrag[1], (int)bfrag[2], (int)bfrag[3]};
 #pragma unroll
             for (int p = 0; p < MP; ++p) {
@@ -1031,7 +1072,7 @@ struct GsArgs {
 };
 static_assert(sizeof(GsArgs) <= 4096 && sizeof(GvBatch) <= 4096, "kernel argument blocks are at most 4 KB");
 
-template <int BITS, int KEEP, int GRP, int MP>
+template <int BITS, int KEEP, int GRP, int MP, bool WT>
 __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
   using C = Cfg<BITS, KEEP, GRP, MP>;
   static_assert(MP == 4 || MP == 8, "row groups of four");
@@ -1040,8 +1081,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  uint2* lut = (uint2*)smem;
-  uint8_t* zreg = smem + LUT_BYTES;
+  uint8_t* zreg = smem + (WT ? WIDE_LUT_BYTES : LUT_BYTES);
   int8_t* xq = (int8_t*)zreg + ZERO_BYTES;
   const GsHead h = a.h;
   float* delta = (float*)(xq + h.xq_cap);
@@ -1054,10 +1094,8 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
   const GvMat& gm = gs.g;
   const DMat& m = gm.m;
   const int M = h.M, N = m.N, NCH = N >> 7, nS = gm.nS, spi = gm.spi, SK = gm.sk;
+  build_table<C, WT>(smem, tid);
   if (tid < 256) {
-    const uint2 e = make_selectors((uint32_t)tid, C::SEL_KIND);
-#pragma unroll
-    for (int j = 0; j < LUT_LANES; ++j) lut[table_slot<LUT_LANES, 8>(tid, j)] = e;
   } else if (tid < 256 + ZERO_BYTES / 4) {
     ((uint32_t*)zreg)[tid - 256] = 0u;
   } else if (tid < 256 + ZERO_BYTES / 4 + 4 * M) {                  // deltas of the chunks past N
@@ -1065,7 +1103,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
     delta[(i >> 2) * (NCH + 4) + NCH + (i & 3)] = 0.f;
   }
   const int wr = lane & 15, kq = lane >> 4;
-  const uint32_t l16 = lane & (LUT_LANES - 1);
+  const uint32_t lane_off = table_lane<WT>(lane);
   const uint32_t xq_off = (uint32_t)((uint8_t*)xq - smem), z_off = (uint32_t)(zreg - smem);
 
   // this workgroup: slab sl, tiles [T_lo, T_hi)
@@ -1138,7 +1176,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
       for (int p = 0; p < MP; ++p) ysum[p] = 0.f;
     }
     issue(T_lo + p1.tl, p1.S, tgt);
-    block_step<C, BITS, NG, TURN>(cur, smem, lut, l16, lane, S, XDigits{xq_off, z_off, delta, Ns, ch0, NCH, M}, ysum);
+    block_step<C, BITS, NG, TURN, WT>(cur, smem, smem, lane_off, lane, S, XDigits{xq_off, z_off, delta, Ns, ch0, NCH, M}, ysum);
     if (S + 1 == s_end) {
       // the part is done: lane quarter kq holds activation row 4g + kq of weight row wr
 #pragma unroll
@@ -2365,9 +2403,9 @@ struct GvCall {           // one matrix of a batched call, host side
   int par;                  // gate/up matrix: M counts real activation rows, the kernel sees 2 M
 };
 
-template <int BITS, int KEEP, int GRP, int MP>
-static int launch_cfg(const GvBatch& b, size_t lds, int blocks, hipStream_t st) {
-  auto kern = gemv_mfma_kernel<BITS, KEEP, GRP, MP>;
+template <int BITS, int KEEP, int GRP, int MP, bool WT>
+static int launch_as(const GvBatch& b, size_t lds, int blocks, hipStream_t st) {
+  auto kern = gemv_mfma_kernel<BITS, KEEP, GRP, MP, WT>;
   static std::atomic<int> configured{0};
   if (!configured.load(std::memory_order_acquire)) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
@@ -2378,32 +2416,40 @@ static int launch_cfg(const GvBatch& b, size_t lds, int blocks, hipStream_t st) 
   return hipGetLastError() == hipSuccess ? CBK_OK : CBK_ERR_HIP;
 }
 
+template <int BITS, int KEEP, int GRP, int MP>
+static int launch_cfg(const GvBatch& b, size_t lds, int blocks, bool wide, hipStream_t st) {
+  if constexpr (KEEP != 0) {
+    if (wide) return launch_as<BITS, KEEP, GRP, MP, true>(b, lds, blocks, st);
+  }
+  return launch_as<BITS, KEEP, GRP, MP, false>(b, lds, blocks, st);
+}
+
 template <int BITS, int KEEP, int GRP>
-static int launch_mp(const GvBatch& b, size_t lds, int blocks, hipStream_t st) {
-  if (b.h.M == 1) return launch_cfg<BITS, KEEP, GRP, 1>(b, lds, blocks, st);
+static int launch_mp(const GvBatch& b, size_t lds, int blocks, bool wide, hipStream_t st) {
+  if (b.h.M == 1) return launch_cfg<BITS, KEEP, GRP, 1>(b, lds, blocks, wide, st);
   // (two rows: a pass each costs less than turning the blocks or halving the operands, 21504 x 5376 3-bit keep 10: 19.7
   // against 20.7 us)
   if constexpr (!block_loads(BITS, KEEP) || GRP == 64) {
-    if (b.h.M == 2) return launch_cfg<BITS, KEEP, GRP, 2>(b, lds, blocks, st);
+    if (b.h.M == 2) return launch_cfg<BITS, KEEP, GRP, 2>(b, lds, blocks, wide, st);
   }
-  if (b.h.M > 4) return launch_cfg<BITS, KEEP, GRP, 8>(b, lds, blocks, st);
-  return launch_cfg<BITS, KEEP, GRP, 4>(b, lds, blocks, st);
+  if (b.h.M > 4) return launch_cfg<BITS, KEEP, GRP, 8>(b, lds, blocks, wide, st);
+  return launch_cfg<BITS, KEEP, GRP, 4>(b, lds, blocks, wide, st);
 }
 
 template <int BITS, int KEEP>
-static int launch_grp(const GvBatch& b, size_t lds, int blocks, hipStream_t st) {
-  return b.mat[0].m.group == 64 ? launch_mp<BITS, KEEP, 64>(b, lds, blocks, st)
-                                : launch_mp<BITS, KEEP, 128>(b, lds, blocks, st);
+static int launch_grp(const GvBatch& b, size_t lds, int blocks, bool wide, hipStream_t st) {
+  return b.mat[0].m.group == 64 ? launch_mp<BITS, KEEP, 64>(b, lds, blocks, wide, st)
+                                : launch_mp<BITS, KEEP, 128>(b, lds, blocks, wide, st);
 }
 
 template <int BITS>
-static int launch_keep(const GvBatch& b, size_t lds, int blocks, hipStream_t st) {
+static int launch_keep(const GvBatch& b, size_t lds, int blocks, bool wide, hipStream_t st) {
   const DMat& m = b.mat[0].m;
   switch (family_of(m.layout) == FAM_DENSE ? 0 : m.keep) {
-    case 0: return launch_grp<BITS, 0>(b, lds, blocks, st);
-    case 10: return launch_grp<BITS, 10>(b, lds, blocks, st);
-    case 16: return launch_grp<BITS, 16>(b, lds, blocks, st);
-    case 23: return launch_grp<BITS, 23>(b, lds, blocks, st);
+    case 0: return launch_grp<BITS, 0>(b, lds, blocks, wide, st);
+    case 10: return launch_grp<BITS, 10>(b, lds, blocks, wide, st);
+    case 16: return launch_grp<BITS, 16>(b, lds, blocks, wide, st);
+    case 23: return launch_grp<BITS, 23>(b, lds, blocks, wide, st);
     default: return CBK_ERR_UNSUPPORTED;
   }
 }
@@ -2422,9 +2468,9 @@ static int gemv_blocks(const GvBatch& gb, int n, int tiles) {
   return blocks;
 }
 
-template <int BITS, int KEEP, int GRP, int MP>
-static int launch_split_cfg(const GsArgs& a, size_t lds, int blocks, int red_blocks, hipStream_t st) {
-  auto kern = gemv_split_kernel<BITS, KEEP, GRP, MP>;
+template <int BITS, int KEEP, int GRP, int MP, bool WT>
+static int launch_split_as(const GsArgs& a, size_t lds, int blocks, int red_blocks, hipStream_t st) {
+  auto kern = gemv_split_kernel<BITS, KEEP, GRP, MP, WT>;
   static std::atomic<int> configured{0};
   if (!configured.load(std::memory_order_acquire)) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
@@ -2435,6 +2481,14 @@ static int launch_split_cfg(const GsArgs& a, size_t lds, int blocks, int red_blo
   if (hipGetLastError() != hipSuccess) return CBK_ERR_HIP;
   hipLaunchKernelGGL(gemv_split_reduce_kernel<(digits_of(BITS) == 4)>, dim3(red_blocks), dim3(GS_RED_THREADS), 0, st, a);
   return hipGetLastError() == hipSuccess ? CBK_OK : CBK_ERR_HIP;
+}
+template <int BITS, int KEEP, int GRP, int MP>
+static int launch_split_cfg(const GsArgs& a, size_t lds, int blocks, int red_blocks, hipStream_t st) {
+  if constexpr (KEEP != 0) {
+    if (lds + WIDE_LUT_BYTES - LUT_BYTES <= 160 * 1024)
+      return launch_split_as<BITS, KEEP, GRP, MP, true>(a, lds + WIDE_LUT_BYTES - LUT_BYTES, blocks, red_blocks, st);
+  }
+  return launch_split_as<BITS, KEEP, GRP, MP, false>(a, lds, blocks, red_blocks, st);
 }
 template <int BITS, int KEEP>
 static int launch_split_grp(const GsArgs& a, size_t lds, int blocks, int red_blocks, hipStream_t st) {
@@ -2486,7 +2540,8 @@ static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt,
     budget = budget < 1 ? 1 : budget;
     const size_t per_part = (size_t)M * ND * g.spi * 512;
     if (fixed + per_part > 160 * 1024) return CBK_ERR_UNSUPPORTED;
-    int pps_max = (int)((160 * 1024 - fixed) / per_part);
+    const bool wide = family_of(g.m.layout) != FAM_DENSE && fixed + WIDE_LUT_BYTES - LUT_BYTES + per_part <= 160 * 1024;
+    int pps_max = (int)((160 * 1024 - fixed - (wide ? WIDE_LUT_BYTES - LUT_BYTES : 0)) / per_part);
     pps_max = pps_max < g.sk ? pps_max : g.sk;
     // Parts per slab: a workgroup runs ceil(items / 16) rounds of one part per wavefront after
     // staging its slab (a 512-column step of M = 8 rows costs about 0.15 rounds of one step)
@@ -2571,20 +2626,28 @@ static int launch_main_batch(GvBatch& gb, hipStream_t st) {
   gb.h.xq_cap = xq_cap; gb.h.delta_cap = delta_cap;
   // reduction slots: as many as fit what is left, at most 24 KB: a power of two between 2 and 64
   const int slot_floats = sk_cap * M * 16;
-  size_t red_room = 160 * 1024 - fixed - (size_t)xq_cap;
+  // Bitmap layouts take the wide selector table where it leaves room for the slots and the wavefronts have five
+  // quarters of a step each: below that its writing and the longer way to a block's first window cost more than its
+  // shorter steps give (M = 1, us, small / wide: 0.5 steps, 3-bit 4096 x 4096 5.8 / 6.0; 1 step, 3-bit q,k,v of 4096 columns
+  // 7.2 / 7.5; 1.4 steps, 4-bit q,k,v of 5376 columns 8.5 / 8.0; 28672 columns, 3.5 steps, 14.4 / 13.8).
+  constexpr size_t more = WIDE_LUT_BYTES - LUT_BYTES;
+  const size_t slots = 8 * slot_bytes < 24 * 1024 ? 8 * slot_bytes : 2 * slot_bytes < 24 * 1024 ? 24 * 1024 : 2 * slot_bytes;
+  const bool wide = family_of(gb.mat[0].m.layout) != FAM_DENSE && 4LL * cost >= 5LL * blocks * GV_WAVES &&
+                    fixed + more + xq_cap + slots <= 160 * 1024;
+  const size_t table = wide ? more : 0;
+  size_t red_room = 160 * 1024 - fixed - table - (size_t)xq_cap;
   red_room = red_room < 24 * 1024 ? red_room : 24 * 1024;
   int nslot = 64;
   while (nslot > 2 && (size_t)nslot * slot_bytes > red_room) nslot >>= 1;
   gb.h.sk_cap = sk_cap; gb.h.nslot = nslot; gb.h.red_floats = nslot * slot_floats;
   gb.h.cq = cost / blocks; gb.h.cr = cost % blocks;
-  const size_t lds = (size_t)LUT_BYTES + ZERO_BYTES + CNT_BYTES + xq_cap + (size_t)delta_cap * 4 +
-                     (size_t)gb.h.red_floats * 4;
+  const size_t lds = fixed + table + xq_cap + (size_t)gb.h.red_floats * 4;
   if (lds > 160 * 1024) return CBK_ERR_UNSUPPORTED;
   const int bits = gb.mat[0].m.bits;
-  if (bits == 6) return launch_mp<6, 16, 128>(gb, lds, blocks, st);   // BLK1632_6: one configuration
-  if (bits == 8) return launch_grp<8, 0>(gb, lds, blocks, st);
-  return bits == 2 ? launch_keep<2>(gb, lds, blocks, st) : bits == 3 ? launch_keep<3>(gb, lds, blocks, st)
-       : bits == 4 ? launch_keep<4>(gb, lds, blocks, st) : CBK_ERR_UNSUPPORTED;
+  if (bits == 6) return launch_mp<6, 16, 128>(gb, lds, blocks, wide, st);   // BLK1632_6: one configuration
+  if (bits == 8) return launch_grp<8, 0>(gb, lds, blocks, false, st);
+  return bits == 2 ? launch_keep<2>(gb, lds, blocks, wide, st) : bits == 3 ? launch_keep<3>(gb, lds, blocks, wide, st)
+       : bits == 4 ? launch_keep<4>(gb, lds, blocks, wide, st) : CBK_ERR_UNSUPPORTED;
 }
 
 // All matrices share one kernel configuration (checked by the caller) and 1 <= M <= 8 (more than

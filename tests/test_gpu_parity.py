@@ -336,6 +336,26 @@ def test_gemv_every_kernel_configuration(case, tiled):
             assert torch.equal(ops.gemv(pm, x.to(DEV), out_dtype=torch.float32), y)
 
 
+@pytest.mark.parametrize("case", [(F.BLK1632_4, 4, 128, 16), (F.BLKC, 3, 64, 10), (F.BLKC, 2, 128, 23), (F.BLK1632_6, 6, 128, 16)],
+                         ids=case_id)
+@pytest.mark.parametrize("K,N,rows", [(24, 9728, (1, 2)), (24, 10240, (1, 2, 5)), (24, 29440, (1, 2)), (24, 31232, (1, 2)),
+                                      (12304, 4096, (1, 4, 5))],
+                         ids=["under_five_quarters_of_a_step", "five_quarters", "last_with_room", "no_room", "tall"])
+def test_gemv_on_either_side_of_the_wide_table(case, K, N, rows):
+    """The selector table of the decode kernels has two forms; a launch takes the wide one from five quarters of a step
+    per wavefront on (two tiles of sixteen rows: 10240 columns) where LDS has room for it (one row: up to about 30000
+    columns).  Shapes on both sides of either line, and tall ones for the kernels of several rows: the float64 product to
+    the decode bar, and row m of M bit for bit what it is alone."""
+    pm = F.synth_packed(K, N, *case[:3], case[3], seed=N, device=DEV).to_tiled()
+    W = ops.dequant(pm, torch.float32).double()
+    x = acts(max(rows), N, torch.float16, seed=N).to(DEV)
+    ref = x.double() @ W.T
+    alone = torch.cat([ops.gemv(pm, x[m:m + 1], out_dtype=torch.float32) for m in range(max(rows))])
+    assert float((alone - ref).abs().max() / ref.abs().max()) < 2e-5
+    for M in rows:
+        assert torch.equal(ops.gemv(pm, x[:M], out_dtype=torch.float32), alone[:M]), M
+
+
 def test_gemv_batch_matches_single_calls():
     """A batched launch against one call per matrix.  How a row is cut into parts depends on the
     launch as a whole (its tiles against the 256 workgroups), so the two agree to float32 rounding
