@@ -18,6 +18,16 @@
 //    with BASE 1024, 0.7e-4 with 4; operands rounded to halves have 1.3e-4.  (Subnormal halves, code * 2^-24, need
 //    no BASE, but the pipe loses more of those: 1.8e-4 for rows of 14336 columns.)
 //    Tiles of 96 tokens have no registers for a second set of sums; they subtract and multiply per weight.
+//  * What a step costs is counted in vector instructions at their price: with two or more wavefronts on a SIMD and, or,
+//    xor, add, right shift, three-input logic, v_fma_f32 and v_mul_f32 on registers take 2.3 to 2.7 cycles, permutes, left
+//    and 64-bit shifts, counts, packed halves, v_fma_mix_f32 and anything with a scalar operand 4.4.  So memory is read
+//    through buffer descriptors (lane offset + scalar offset, no vector addition), the table starts LDS (an entry's
+//    offset is its address), and scales are floats before they multiply: 4-bit codes, 64 tokens, 168 -> 135 cycles per
+//    step of 16 columns x 64 rows beside 144 of matrix instructions.  With the preparation, before and after: feed-forward
+//    block 14336 x 4096 at 48 rows 61.7 -> 58.9 us, 2-bit 6144 x 4096 at 333 rows 43.2 -> 41.6, fixed-stride 8-bit down
+//    projection 4096 x 14336 at 512 rows 90.0 -> 85.3.  At the last the clock falls to 1.6 - 1.7 GHz: what is left there
+//    is the power of the matrix instructions, which no schedule changes (the older
+//    of the two wavefronts of a SIMD ends 25 % early; priorities that keep them level leave the end where it is).
 //
 // k order.  A step is eight columns of the first half of a group (lanes 0-31) and eight of the second
 // (lanes 32-63): a lane walks half a group of its own row, nothing is loaded or ranked twice.  The
@@ -48,6 +58,21 @@ constexpr int SK_LUT = 256 * SK_LUT_LANES * 16;
 constexpr size_t SK_LDS = (size_t)SK_WC * SK_WR * 32 * SK_PITCH * 4 + SK_LUT;
 
 typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+
+// A wavefront's view of global memory: base in scalar registers, loads at lane offset + scalar offset (32 bits each).
+__device__ inline __amdgpu_buffer_rsrc_t sk_buffer(const void* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, -1, 0x00027000);
+}
+template <typename T>
+__device__ inline T sk_load(__amdgpu_buffer_rsrc_t b, uint32_t lane_off, uint32_t off) {
+  if constexpr (sizeof(T) == 16) return __builtin_amdgcn_raw_buffer_load_b128(b, lane_off, off, 0);
+  else if constexpr (sizeof(T) == 8) return __builtin_amdgcn_raw_buffer_load_b64(b, lane_off, off, 0);
+  else if constexpr (sizeof(T) == 4) return __builtin_amdgcn_raw_buffer_load_b32(b, lane_off, off, 0);
+  else if constexpr (sizeof(T) == 2) return __builtin_amdgcn_raw_buffer_load_b16(b, lane_off, off, 0);
+  else return __builtin_amdgcn_raw_buffer_load_b8(b, lane_off, off, 0);
+}
 
 // The scale of a token and column part with an infinite activation: above every scale of a finite one (2^120)
 constexpr float SK_INFINITE = 2658455991569831745807614120560689152.f;   // 2^121
@@ -135,8 +160,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   constexpr bool DEFER = C::DEFER;
   constexpr int ST = C::ST, NG = C::NG, NA = C::NA;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  float* red = (float*)smem;
-  uint4* lut = (uint4*)(smem + (size_t)SK_WC * SK_WR * 32 * SK_PITCH * 4);   // [256][copies]: selectors, byte masks
+  uint4* lut = (uint4*)smem;                                        // [256][copies]: selectors, byte masks (first: an entry's
+  float* red = (float*)(smem + SK_LUT);                             // address is its offset)
   const DMat& m = a.m;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = wave & 1, wc = wave >> 1, half = lane >> 5;
@@ -195,6 +220,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       moff[j] = m.tiled ? (uint32_t)((rc >> 4) - (rb >> 4)) * (uint32_t)m.G * 16u + (uint32_t)(rc & 15) : (uint32_t)(rc - rb) * (uint32_t)m.G;
     }
     const uint32_t lut_lane = (uint32_t)(lane & (SK_LUT_LANES - 1)) * 16u;
+    // Read as buffers: a scalar offset that moves with the group and a lane's that does not cost no vector instruction
+    // (as pointers, every group's base and every step's went through a 64-bit vector addition)
+    const auto data_b = sk_buffer(dbase), zero_b = sk_buffer(m.zero + mbase), scale_b = sk_buffer(m.scale + mbase);
     struct Grp {
       uint32_t m[BITMAP ? C::PBLK : 1];
       uint32_t raw[C::NL];
@@ -208,34 +236,32 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const uint32_t go8 = C::PBLK == 2 ? ug * ush : (ug >> 1) * ush + (ug & 1u) * 8u, lo8 = (uint32_t)half * (C::PBLK * 4u);
       // first unit of a skewed run
       const uint32_t uskew = ((2u * ug + (uint32_t)half) * (uint32_t)C::HB >> 7) * ush;
+      const uint32_t plane = (m.code_off >> 4) * ush;               // (the mask plane is whole units)
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         if (BITMAP) {
-          const uint8_t* p = dbase + go8 + (roff[j] + lo8);
-          if (C::PBLK == 2) { const uint2 v = *(const uint2*)p; w[j].m[0] = v.x; w[j].m[C::PBLK - 1] = v.y; }
-          else w[j].m[0] = *(const uint32_t*)p;
+          if (C::PBLK == 2) { const v2u v = sk_load<v2u>(data_b, roff[j] + lo8, go8); w[j].m[0] = v[0]; w[j].m[C::PBLK - 1] = v[1]; }
+          else w[j].m[0] = sk_load<uint32_t>(data_b, roff[j] + lo8, go8);
         }
         if (C::HI2) {                                               // behind the mask and nibble planes
-          const uint2 v = *(const uint2*)(dbase + (size_t)(m.N * 3 >> 7) * ush + ug * ush + (roff[j] + (uint32_t)half * 8u));
-          w[j].h2[0] = v.x; w[j].h2[C::HI2 ? C::PBLK - 1 : 0] = v.y;
+          const v2u v = sk_load<v2u>(data_b, roff[j] + (uint32_t)half * 8u, (uint32_t)(m.N * 3 >> 7) * ush + ug * ush);
+          w[j].h2[0] = v[0]; w[j].h2[C::HI2 ? C::PBLK - 1 : 0] = v[1];
         }
-        const uint8_t* cbase = dbase + (m.code_off >> 4) * ush;     // the mask plane is whole units
-        if constexpr (C::HB == 32) w[j].raw[0] = *(const uint32_t*)(cbase + go8 + (roff[j] + lo8));
+        if constexpr (C::HB == 32) w[j].raw[0] = sk_load<uint32_t>(data_b, roff[j] + lo8, plane + go8);
         else if constexpr (C::HB == 64) {
-          const uint2 v = *(const uint2*)(cbase + ug * ush + (roff[j] + (uint32_t)half * 8u));
-          w[j].raw[0] = v.x; w[j].raw[1] = v.y;
+          const v2u v = sk_load<v2u>(data_b, roff[j] + (uint32_t)half * 8u, plane + ug * ush);
+          w[j].raw[0] = v[0]; w[j].raw[1] = v[1];
         } else {
 #pragma unroll
           for (int i = 0; i < C::NL / 4; ++i) {
-            const uint8_t* p = C::WHOLE ? cbase + (ug * (2 * C::HB / 128) + i) * ush + (roff[j] + (uint32_t)half * (C::HB / 128) * ush)
-                                        : cbase + i * ush + (roff[j] + uskew);
-            const uint4 v = *(const uint4*)p;
-            w[j].raw[4 * i] = v.x; w[j].raw[4 * i + 1] = v.y; w[j].raw[4 * i + 2] = v.z; w[j].raw[4 * i + 3] = v.w;
+            const v4u v = C::WHOLE ? sk_load<v4u>(data_b, roff[j] + (uint32_t)half * (C::HB / 128) * ush, plane + (ug * (2 * C::HB / 128) + i) * ush)
+                                   : sk_load<v4u>(data_b, roff[j] + uskew, plane + i * ush);
+            w[j].raw[4 * i] = v[0]; w[j].raw[4 * i + 1] = v[1]; w[j].raw[4 * i + 2] = v[2]; w[j].raw[4 * i + 3] = v[3];
           }
         }
-        const size_t mg = mbase + (m.tiled ? ug * 16u : ug);
-        w[j].z = (m.zero + mg)[moff[j]];
-        w[j].s = (m.scale + mg)[moff[j]];
+        const uint32_t mg = m.tiled ? ug * 16u : ug;
+        w[j].z = sk_load<uint8_t>(zero_b, moff[j], mg);
+        w[j].s = sk_load<uint16_t>(scale_b, moff[j] * 2u, mg * 2u);
       }
     };
     // activation fragments of step t and group sums of group g (counted from the wavefront's first)
@@ -243,13 +269,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const uint32_t* xcb = a.xc + (size_t)xv * a.xcs + ((size_t)tt * m.G + g0) * (2 * TI * 32);
     v8h af[NA][TI];
     uint32_t xs[TI];
-    uint32_t lane16 = (uint32_t)lane * 16u;
-    asm("" : "+v"(lane16));                                         // keep it an offset of its own: scalar base + 32-bit offset loads
+    const uint32_t lane16 = (uint32_t)lane * 16u;
+    const auto act_b = sk_buffer(xb);
     const int steps = (g1 - g0) * ST;
     auto load_a = [&](int t, int buf) {
-      const uint8_t* p = xb + (size_t)((uint32_t)(t < steps ? t : steps - 1) * (TI * 1024u));
+      const uint32_t at = (uint32_t)(t < steps ? t : steps - 1) * (TI * 1024u);
 #pragma unroll
-      for (int i = 0; i < TI; ++i) af[buf][i] = *(const v8h*)(p + i * 1024 + lane16);
+      for (int i = 0; i < TI; ++i) af[buf][i] = __builtin_bit_cast(v8h, sk_load<v4u>(act_b, lane16, at + i * 1024u));
     };
     auto load_sums = [&](int g) {
       const uint32_t* p = xcb + (size_t)((uint32_t)(g < g1 - g0 ? g : g1 - g0 - 1) * (2u * TI * 32u));
@@ -293,8 +319,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       auto fetch = [&](int o, uint4 (&e)[2]) {
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-          if (BITMAP)                                               // entry address: mask byte in byte 1, this lane's copy in byte 0
-            e[j] = *(const uint4*)((const uint8_t*)lut + perm(w[j].m[BITMAP ? o >> 2 : 0], lut_lane, 0x0C0C0400u + ((uint32_t)(o & 3) << 8)));
+          if (BITMAP) {                                             // entry address: mask byte in byte 1, this lane's copy in byte 0
+            const v4u v = *(const __attribute__((address_space(3))) v4u*)(uintptr_t)perm(w[j].m[BITMAP ? o >> 2 : 0], lut_lane, 0x0C0C0400u + ((uint32_t)(o & 3) << 8));
+            e[j] = make_uint4(v[0], v[1], v[2], v[3]);
+          }
       };
       // octet o of both rows -> the B operands of a step
       auto decode = [&](int o, const uint4 (&e)[2], v8h (&bf)[2]) {
@@ -402,7 +430,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
       float sc[2];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) sc[j] = h2f((uint16_t)w[j].s);
+      for (int j = 0; j < 2; ++j) {
+        sc[j] = h2f((uint16_t)w[j].s);
+        asm("" : "+v"(sc[j]));                                      // (or the conversion is folded into v_fma_mix_f32, see below)
+      }
       if (more) load_group(g + NG, w);
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (DEFER) {
