@@ -12,6 +12,7 @@ namespace cbk {
 // 0x0C, the constant 0x00.
 // kind 0: pool = {even-rank codes (bytes 0-3), odd-rank codes (bytes 4-7)}   (4-bit codes)
 // kind 1: pool = {c0,c4,c1,c5 | c2,c6,c3,c7}                                   (2-bit codes)
+template <uint32_t REMOVED = 0x0C0C0C0Cu>                  // selector of a pruned column, in every byte; 0x0C: a zero byte
 __device__ inline uint2 make_selectors(uint32_t mb, int kind) {
   uint32_t sel[2], before = 0;                           // survivors of the lower four columns, in every byte
 #pragma unroll
@@ -21,7 +22,7 @@ __device__ inline uint2 make_selectors(uint32_t mb, int kind) {
     before = ((b * 0x01010101u) >> 24) * 0x01010101u;
     const uint32_t idx = kind == 0 ? ((r >> 1) & 0x03030303u) + ((r & 0x01010101u) << 2)
                                    : ((r & 0x03030303u) << 1) | ((r >> 2) & 0x01010101u);
-    sel[h] = (idx & kept) | (0x0C0C0C0Cu & ~kept);
+    sel[h] = (idx & kept) | (REMOVED & ~kept);
   }
   return make_uint2(sel[0], sel[1]);
 }

@@ -24,7 +24,17 @@
 // and the dense layouts) and for BLK1632_6, zero points <= 128, this is the byte-permute decoder
 // of the decode kernel (selector table in LDS) followed by two packed-half operations per column
 // pair; the remaining layouts (8-bit codes, larger zero points) go through the generic
-// 32-column reader.
+// 32-column reader.  One wavefront per SIMD issues a vector instruction every five to seven
+// cycles beside its matrix instructions, whatever its kind, so the decode is counted in
+// instructions: an entry's address is one four-byte dot product of the mask dword, codes stay
+// unsigned until the exact subtraction of 1024 + zero point, and a pruned column reads the zero
+// point from the place of the eighth survivor, which only a full byte asks for.  4-bit, 16 of 32:
+// 932 -> 764 vector instructions per 256 of the matrix cores (1028 -> 764 with two or three
+// column-scale vectors, whose activation base had stayed in vector registers).  Gated block of
+// 21504 x 5376 at 2048 tokens 1457 -> 1436 us.  More would have to come out of the energy of the
+// matrix instructions and of LDS: the clock falls with the load (one tile on every eighth CU
+// takes 132 us, one on every CU 167), spreading the copies over the stage changes nothing, a
+// second copy of each activation line costs 12 %.
 //
 // Workgroups are ordered so that those running at the same time on one XCD (blockIdx % 8)
 // share their token tile, which then stays in that XCD's L2.
@@ -47,6 +57,7 @@ constexpr int gb_xbuf(int ti) { return 64 * ti * GB_K * 2; }
 constexpr size_t gb_lds(int ti) { return (size_t)2 * gb_xbuf(ti) + (size_t)2 * GB_R * GB_P * 2 + GB_LUT; }
 
 typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 
 struct GbArgs {
   DMat m;
@@ -91,18 +102,16 @@ __device__ inline void dma_x16(const void* base, uint32_t voff, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds) : "memory", "m0");
 }
 
-// eight signed bytes (q - z for a kept column, 0 for a pruned one) -> eight halfs times scale
-__device__ inline uint4 bytes_to_halfs(uint32_t b0, uint32_t b1, h2_t s2) {
-  // byte b (two's complement) -> u = b ^ 0x80 = b + 128 -> half bits 0x6400 | u = 1024 + 128 + b
-  const uint32_t u0 = b0 ^ 0x80808080u, u1 = b1 ^ 0x80808080u;
+// eight codes (the zero point z for a pruned column) -> eight halfs (q - z) * scale; off2 = -(1024 + z) twice.
+// A code in the low byte of 0x64xx is the half 1024 + q; the difference is exact, the product rounds once.
+__device__ inline uint4 bytes_to_halfs(uint32_t b0, uint32_t b1, h2_t off2, h2_t s2) {
   const uint32_t k = 0x64646464u;
-  uint32_t w[4] = {__builtin_amdgcn_perm(k, u0, 0x04010400u), __builtin_amdgcn_perm(k, u0, 0x04030402u),
-                   __builtin_amdgcn_perm(k, u1, 0x04010400u), __builtin_amdgcn_perm(k, u1, 0x04030402u)};
-  const h2_t off = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+  uint32_t w[4] = {__builtin_amdgcn_perm(k, b0, 0x04010400u), __builtin_amdgcn_perm(k, b0, 0x04030402u),
+                   __builtin_amdgcn_perm(k, b1, 0x04010400u), __builtin_amdgcn_perm(k, b1, 0x04030402u)};
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     h2_t v = __builtin_bit_cast(h2_t, w[i]);
-    v = (v + off) * s2;
+    v = (v + off2) * s2;
     w[i] = __builtin_bit_cast(uint32_t, v);
   }
   return make_uint4(w[0], w[1], w[2], w[3]);
@@ -209,11 +218,12 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
   const int nch = N >> 7;                                         // 128-column chunks of the weight rows
 
   if (BITMAP) {
-    const uint2 e = make_selectors((uint32_t)tid, C::SEL_KIND);
+    const uint2 e = make_selectors<0x07070707u>((uint32_t)tid, C::SEL_KIND);   // a pruned column reads rank 7's byte
 #pragma unroll
     for (int j = 0; j < 8; ++j) lut[table_slot<8, 8>(tid, j)] = e;
   }
-  const uint32_t l8 = lane & 7;
+  const uint32_t lut_lane = (uint32_t)(uintptr_t)lut + 8 * (lane & 7);       // LDS address of this lane's copy of entry 0
+  const uint32_t lut_full = (uint32_t)(uintptr_t)lut + 255 * 64;             // and of the first copy of entry 255
 
   v16f acc[TI][4];
 #pragma unroll
@@ -238,6 +248,9 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
   const uint32_t xvo_o = (uint32_t)((lane >> 3) * Npad * 2 + (((lane & 7) ^ (4 + (lane >> 4))) * 16));
   const int xv = PAR == 1 ? pp : PAR >= 2 ? (r0 >= a.vs0 ? 1 : 0) + (r0 >= a.vs1 ? 1 : 0) : 0;   // which col_scale vector
   const uint8_t* xsb = (const uint8_t*)(a.xp + (size_t)xv * a.xps + (size_t)(t0 + 16 * TI * wv) * Npad + (size_t)s_begin * GB_K);
+  // the same in every lane: kept in scalar registers from here on, or each copy below reads it out of vector registers
+  xsb = (const uint8_t*)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uint64_t)xsb) |
+                         ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)xsb >> 32)) << 32));
   const uint32_t xlds0 = (uint32_t)(uintptr_t)Xs + (uint32_t)wv * (2048u * TI);
   auto dma_x = [&](int s, int buf) {                              // stage s -> Xs[buf]
     const uint8_t* sb = xsb + (size_t)s * (GB_K * 2);
@@ -294,14 +307,17 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
   };
 
   // selectors of mask byte b8 (0..7) of half h of a chunk (bitmap layouts only)
-  auto fetch_sel = [&](const WChunk& w, int h, int b8) -> uint2 {
-    if (!BITMAP) return make_uint2(0, 0);
+  struct Sel { uint32_t x, y; bool full; };                         // full: all eight columns kept
+  auto fetch_sel = [&](const WChunk& w, int h, int b8) -> Sel {
+    if (!BITMAP) return Sel{0, 0, false};
     const int jb = 8 * h + b8;                                     // mask byte of the chunk, 0..15
-    const uint32_t mb = (w.m[jb >> 2] >> (8 * (jb & 3))) & 0xFFu;
-    return lut[mb * 8 + l8];
+    // byte jb % 4 of the mask dword, times 64 bytes per entry, plus the base
+    const uint32_t at = __builtin_amdgcn_udot4(w.m[jb >> 2], 64u << (8 * (jb & 3)), lut_lane, false);
+    const v2u e = *(const __attribute__((address_space(3))) v2u*)(uintptr_t)at;
+    return Sel{e[0], e[1], at >= lut_full};
   };
   // decode mask byte b8 (8 columns) of stage s = half h of chunk w into Ws[buf]
-  auto store_w_byte = [&](int s, WChunk& w, int h, int buf, int b8, uint2 sel) {
+  auto store_w_byte = [&](int s, WChunk& w, int h, int buf, int b8, Sel sel) {
     _Float16* dst = Ws + (size_t)buf * GB_R * GB_P + tid * GB_P + b8 * 8;
     if (!FASTD) {
       if (b8 & 3) return;                                         // the generic reader works on 32 columns
@@ -337,43 +353,51 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
     const int gi = C::NGC == 2 ? h : 0;                             // quantisation group of this stage
     const _Float16 sh = (_Float16)(wok ? w.s[gi] : 0.f);
     const h2_t s2 = {sh, sh};
-    const uint32_t nz = 0x80808080u - ((w.z >> (8 * gi)) & 0xFFu) * 0x01010101u;
+    const uint32_t z = (w.z >> (8 * gi)) & 0xFFu;
+    const h2_t off2 = __builtin_bit_cast(h2_t, 0xE400E400u + z * 0x00010001u);
     uint32_t p0, p1, b0, b1;
     if (BITMAP) {
       const uint32_t mw = w.m[blk];
       const uint32_t r = jj == 0 ? 0u : (uint32_t)__builtin_popcount(mw & ((1u << (8 * jj)) - 1u));
       const uint32_t cwin = jj == 0 ? st[0] : window<C::NW>(st, r * C::SB);
+      // p0 | p1: the codes of the survivors from this byte's first on, even and odd ranks (four bits), or 0 2 .. and 4 6 ..
+      // Rank 7, the top byte of p1, is asked for only if all eight columns are kept: otherwise the zero point takes its
+      // place, which is what a pruned column reads (bits above a code in that byte are zeros already).
+      const uint32_t zt = z << 24;
       if (C::HI2) {
         uint32_t h0, h1;
         hi2_pools(w.h2[C::HI2 ? blk : 0], r, h0, h1);
-        p0 = bias_pool((cwin & 0x0F0F0F0Fu) | h0, nz);
-        p1 = bias_pool(((cwin >> 4) & 0x0F0F0F0Fu) | h1, nz);
+        p0 = (cwin & 0x0F0F0F0Fu) | h0;
+        const uint32_t of = sel.full ? 0xFFFFFFFFu : 0x00FFFFFFu;
+        p1 = ((((cwin >> 4) & 0x0F0F0F0Fu) | h1) & of) | (zt & ~of);
       } else if (C::SB == 4) {
-        p0 = bias_pool(cwin & 0x0F0F0F0Fu, nz);
-        p1 = bias_pool((cwin >> 4) & 0x0F0F0F0Fu, nz);
+        p0 = cwin & 0x0F0F0F0Fu;
+        const uint32_t of = sel.full ? 0xFF0F0F0Fu : 0x000F0F0Fu;
+        p1 = ((cwin >> 4) & of) | (zt & ~of);
       } else {
         const uint32_t lo16 = cwin & 0xFFFFu;
         const uint32_t t2 = (lo16 << 14) | lo16;
-        p0 = bias_pool(t2 & 0x03030303u, nz);
-        p1 = bias_pool((t2 >> 4) & 0x03030303u, nz);
+        p0 = t2 & 0x03030303u;
+        const uint32_t of = sel.full ? 0xFF030303u : 0x00030303u;
+        p1 = ((t2 >> 4) & of) | (zt & ~of);
       }
       b0 = perm(p1, p0, sel.x);
       b1 = perm(p1, p0, sel.y);
     } else if (C::SB == 4) {                                       // dense 4-bit, or 3-bit widened to nibbles
       const uint32_t cwin = st[jj];
-      p0 = bias_pool(cwin & 0x0F0F0F0Fu, nz);                      // even columns
-      p1 = bias_pool((cwin >> 4) & 0x0F0F0F0Fu, nz);               // odd columns
+      p0 = cwin & 0x0F0F0F0Fu;                                     // even columns
+      p1 = (cwin >> 4) & 0x0F0F0F0Fu;                              // odd columns
       b0 = perm(p1, p0, 0x05010400u);
       b1 = perm(p1, p0, 0x07030602u);
     } else {                                                       // dense 2-bit: 16 codes per dword
       const uint32_t lo16 = (st[jj >> 1] >> (16 * (jj & 1))) & 0xFFFFu;
       const uint32_t t2 = (lo16 << 14) | lo16;
-      p0 = bias_pool(t2 & 0x03030303u, nz);                        // c0 c4 c1 c5
-      p1 = bias_pool((t2 >> 4) & 0x03030303u, nz);                 // c2 c6 c3 c7
+      p0 = t2 & 0x03030303u;                                       // c0 c4 c1 c5
+      p1 = (t2 >> 4) & 0x03030303u;                                // c2 c6 c3 c7
       b0 = perm(p1, p0, 0x06040200u);
       b1 = perm(p1, p0, 0x07050301u);
     }
-    *(uint4*)dst = bytes_to_halfs(b0, b1, s2);
+    *(uint4*)dst = bytes_to_halfs(b0, b1, off2, s2);
   };
 
   // fragment registers, two sets; set 0 of the next stage is loaded at the end of the current one
@@ -399,7 +423,7 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
   read_frags(0, 0, 0);
   dma_x(nst > 1 ? 1 : 0, 1);
   load_chunk(1, wB);
-  uint2 selc[3];                                                  // selectors of the mask bytes decoded next
+  Sel selc[3];                                                    // selectors of the mask bytes decoded next
 #pragma unroll
   for (int i = 0; i < 3; ++i) selc[i] = fetch_sel(wA, 1, i);
 
@@ -421,7 +445,7 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
       const int c = kk & 1, n = c ^ 1;
       if (kk < 3) {
         read_frags(buf, kk + 1, n);
-        uint2 seln[3];
+        Sel seln[3];
         if (kk == 0) {
 #pragma unroll
           for (int i = 0; i < NB1; ++i) seln[i] = fetch_sel(wd, HD, NB0 + i);

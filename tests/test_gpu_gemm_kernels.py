@@ -64,6 +64,31 @@ def test_every_instantiation(case, vectors):
     assert len(ran) == 9 + (3 if vectors == 2 or case[1] == 8 else 6)
 
 
+@pytest.mark.parametrize("case", [c for c in CASES if c[3]], ids=case_id)
+def test_runs_of_kept_columns(case):
+    """Mask bytes with all eight columns kept beside bytes with none: in the tile kernel the eighth survivor's place
+    holds the zero point unless the byte is full.  Zero points on the grid's ends and at 128.  Bound as above."""
+    N, keep = 1664, case[3]
+    pm = _matrix(case, 1, N, seed=5)
+    turn = (torch.arange(pm.K, device=DEV)[:, None] + torch.arange(N // 32, device=DEV)) % 32
+    run = ((((1 << keep) - 1) << turn) | (((1 << keep) - 1) >> (32 - turn))) & 0xFFFFFFFF    # a run that starts at column `turn`
+    mask = pm.array("data")[: pm.data_bytes].view(pm.K, -1)[:, : N // 8]
+    mask[:] = ((run[..., None] >> torch.arange(0, 32, 8, device=DEV)) & 255).to(torch.uint8).view(pm.K, N // 8)
+    zero = pm.array("zero")
+    zero[:] = torch.tensor([0, 2 ** case[1] - 1, 128], dtype=torch.uint8, device=DEV)[torch.arange(zero.numel(), device=DEV) % 3].view(zero.shape)
+    pm.flags = F.FLAG_ZERO_LE_128
+    W = ops.dequant(pm, torch.float32).double()
+    kept = F.unpack_mask(mask, N)
+    assert bool((W[~kept] == 0).all()) and int(kept.sum()) == pm.K * N * keep // 32
+    Wh = ops.dequant(pm, torch.float32, with_col_scale=False).half().double()
+    x = acts(257, N, torch.float16, seed=case[1]).to(DEV)
+    ref = x.double() @ W.t()
+    bound = float(((x.float() * pm.array("col_scale").view(-1, N).float()).half().double() @ Wh.t() - ref).norm() / ref.norm())
+    for tokens in TOKENS["tile"]:
+        y = gemm_as(pm.to_tiled(), x, "tile", tokens, out_dtype=torch.float32)
+        assert float((y.double() - ref).norm() / ref.norm()) <= 1.02 * bound, tokens
+
+
 @pytest.mark.parametrize("act", ["gelu_tanh", "silu"])
 @pytest.mark.parametrize("case", [c for c in CASES if c[2:] in ((128, 16), (64, 10), (128, 0))], ids=case_id)
 def test_gated_call_on_every_tile(case, act):
