@@ -69,7 +69,8 @@ struct GbArgs {
   int ydt;
   int64_t ldy;
   const void* bias;
-  int tiles_t, tiles_r;
+  int tiles_t, tiles_r;    // token tiles, row tiles of this launch
+  int tr0;                 // its first row tile
   int halves;              // gate/up matrix (par): 1 = write the gate outputs to columns [0, K/2) and the up outputs to
                            // [K/2, K) of y instead of interleaving them (whole 16-byte stores; for cbk_linear_act)
   int ti;                  // 32-token blocks per wavefront: 4, 2 or 1 (tiles of 256, 128 or 64 tokens)
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
   const int lin = xcd * per + idx;                                 // token-tile-major linear id
   if (lin >= nb) return;
   const int part = SPLIT ? lin % a.nsplit : 0, tile = SPLIT ? lin / a.nsplit : lin;
-  const int tt = tile / a.tiles_r, tr = tile % a.tiles_r;
+  const int tt = tile / a.tiles_r, tr = tile % a.tiles_r + a.tr0;
   constexpr int kstep = PAR == 1 ? 2 : 1;                         // row stride of this workgroup's rows
   const int pp = PAR == 1 ? (tr & 1) : 0;                         // and their parity
   const int t0 = tt * (64 * TI), r0 = PAR == 1 ? (tr >> 1) * (2 * GB_R) + pp : tr * GB_R;

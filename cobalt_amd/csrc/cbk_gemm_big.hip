@@ -166,6 +166,22 @@ static int gb_part(const DMat& m, int nsplit) {
   const int nst = gb_npad(m.N) / GB_K, per = ((nst + nsplit - 1) / nsplit + 3) / 4 * 4;
   return nsplit > 1 && (nsplit - 1) * per >= nst ? 0 : per;
 }
+// Last round of a launch of 256-token tiles.  Tiles beyond a whole number of rounds over the 256 CUs keep a few CUs busy
+// for a whole tile time; the row tiles that hold them go into a second launch of 64- or 128-token tiles if those fit one
+// round.  Every output is the same sum in the same order whatever its tile.  Measured, N = 5376 at 2048 tokens, with the
+// preparation: 64 tiles of 256 tokens 134 us, as 128 of 128 103, as 256 of 64 88; 128 tiles 135, as 256 of 128 109, as
+// 512 of 64 162 (two rounds: not taken).
+struct GbTail { int rows, ti; };                                    // row tiles of the second launch (0: none), its tile
+static GbTail gb_tail(int tiles_r, int M, bool pairs) {
+  const int tiles_t = (M + GB_T - 1) / GB_T, full = tiles_t * tiles_r / 256, left = tiles_t * tiles_r - 256 * full;
+  if (!full || !left) return {0, 4};
+  int rows = (left + tiles_t - 1) / tiles_t;
+  if (pairs) rows += rows & 1;                                      // both parities of a row range
+  if (rows >= tiles_r) return {0, 4};
+  for (int ti = 1; ti <= 2; ++ti)
+    if ((M + 64 * ti - 1) / (64 * ti) * rows <= 256) return {rows, ti};
+  return {0, 4};
+}
 static GemmPlan gb_plan_ti(const DMat& m, int M, int ti, int max_split, size_t room) {
   const int T = 64 * ti;
   const int tiles = ((M + T - 1) / T) * ((m.K + GB_R - 1) / GB_R);
@@ -177,7 +193,11 @@ static GemmPlan gb_plan_ti(const DMat& m, int M, int ti, int max_split, size_t r
     if (!per) continue;
     const size_t bytes = gb_space(m, M, ti, s);
     if (bytes > room) continue;
-    const double rounds = (double)((tiles * s + 255) / 256);
+    double rounds = (double)((tiles * s + 255) / 256);
+    if (s == 1 && ti == 4 && gb_fast(m)) {                          // (shares of a tile time that the smaller tiles take)
+      const GbTail tail = gb_tail((m.K + GB_R - 1) / GB_R, M, m.cs_rows == 2);
+      if (tail.rows) rounds -= tail.ti == 1 ? 0.30 : 0.20;
+    }
     double t = rounds * (per * t_stage + t_wg);
     if (s > 1) t += 2.0 * s * (double)M * m.K * 4 / 4.0e6 + 5.0;
     if (s == 1) best = one = {GEMM_TILE, ti, 1, t, bytes};
@@ -219,6 +239,28 @@ GemmPlan plan_big(const DMat& m, int M, size_t room) {
   return p;
 }
 
+static int gb_launch(const GbArgs& a, hipStream_t st) {
+  const DMat& m = a.m;
+  const int nb = a.tiles_t * a.tiles_r * a.nsplit;
+  const int blocks = ((nb + 7) / 8) * 8;
+  const bool le128 = (m.flags & CBK_FLAG_ZERO_LE_128) != 0;
+  const int fam = family_of(m.layout);
+  int rc = CBK_ERR_UNSUPPORTED;
+  if (le128 && (fam == FAM_BLK || fam == FAM_DENSE)) {
+    const int keep = fam == FAM_DENSE ? 0 : m.keep;
+    if (m.bits == 2) rc = launch_gemm_big_b2(a, keep, m.group, blocks, st);
+    else if (m.bits == 3) rc = launch_gemm_big_b3(a, keep, m.group, blocks, st);
+    else if (m.bits == 4) rc = launch_gemm_big_b4(a, keep, m.group, blocks, st);
+  } else if (le128 && fam == FAM_BLK6 && m.bits == 6 && m.keep == 16 && m.group == 128) {
+    rc = launch_gemm_big_b6(a, blocks, st);
+  }
+  if (rc == CBK_ERR_UNSUPPORTED) {
+    if (a.nsplit > 1) return CBK_ERR_UNSUPPORTED;                   // (only what the cases above take is ever split)
+    rc = launch_big_cfg<0, 0, 128>(a, blocks, st);                  // generic reader
+  }
+  return rc;
+}
+
 int launch_gemm_big(const DMat& m, const GemmPlan& plan, const void* x, int xdt, int M, int64_t ldx, void* y, int ydt,
                     int64_t ldy, const void* bias, void* ws, size_t ws_bytes, hipStream_t st, bool halves) {
   if (halves && (m.cs_rows != 2 || (m.K & 1) || bias)) return CBK_ERR_UNSUPPORTED;
@@ -253,24 +295,18 @@ int launch_gemm_big(const DMat& m, const GemmPlan& plan, const void* x, int xdt,
   a.part_stride = (size_t)M * gb_kpad(m.K);
   a.part = (float*)((uint8_t*)ws + xbytes + sbytes);
   a.ti = plan.ti;
+  a.tr0 = 0;
   a.tiles_t = (M + T - 1) / T;
   a.tiles_r = par ? 2 * ((m.K + 2 * GB_R - 1) / (2 * GB_R)) : (m.K + GB_R - 1) / GB_R;
-  const int nb = a.tiles_t * a.tiles_r * a.nsplit;
-  const int blocks = ((nb + 7) / 8) * 8;
-  const bool le128 = (m.flags & CBK_FLAG_ZERO_LE_128) != 0;
-  const int fam = family_of(m.layout);
-  int rc = CBK_ERR_UNSUPPORTED;
-  if (le128 && (fam == FAM_BLK || fam == FAM_DENSE)) {
-    const int keep = fam == FAM_DENSE ? 0 : m.keep;
-    if (m.bits == 2) rc = launch_gemm_big_b2(a, keep, m.group, blocks, st);
-    else if (m.bits == 3) rc = launch_gemm_big_b3(a, keep, m.group, blocks, st);
-    else if (m.bits == 4) rc = launch_gemm_big_b4(a, keep, m.group, blocks, st);
-  } else if (le128 && fam == FAM_BLK6 && m.bits == 6 && m.keep == 16 && m.group == 128) {
-    rc = launch_gemm_big_b6(a, blocks, st);
-  }
-  if (rc == CBK_ERR_UNSUPPORTED) {
-    if (a.nsplit > 1) return CBK_ERR_UNSUPPORTED;                   // (only what the cases above take is ever split)
-    rc = launch_big_cfg<0, 0, 128>(a, blocks, st);                  // generic reader
+  const GbTail tail = a.ti == 4 && a.nsplit == 1 && gb_fast(m) ? gb_tail(a.tiles_r, M, par != 0) : GbTail{0, 4};
+  a.tiles_r -= tail.rows;
+  int rc = gb_launch(a, st);
+  if (rc == CBK_OK && tail.rows) {
+    a.tr0 = a.tiles_r;
+    a.tiles_r = tail.rows;
+    a.ti = tail.ti;
+    a.tiles_t = (M + 64 * a.ti - 1) / (64 * a.ti);
+    rc = gb_launch(a, st);
   }
   if (rc == CBK_OK && a.nsplit > 1) {
     const int64_t items = (int64_t)M * ((m.K + 7) / 8);

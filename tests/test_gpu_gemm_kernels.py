@@ -89,6 +89,26 @@ def test_runs_of_kept_columns(case):
         assert float((y.double() - ref).norm() / ref.norm()) <= 1.02 * bound, tokens
 
 
+@pytest.mark.parametrize("vectors", [1, 2, 3], ids=["plain", "gate_up", "qkv"])
+@pytest.mark.parametrize("rows", [7423, 7700, 10300, 14800], ids=["64 tokens", "64 tokens, ragged", "128 tokens", "none"])
+def test_last_round_in_smaller_tiles(rows, vectors):
+    """More than 256 tiles of 256 tokens: the row tiles past the last whole round run as smaller tiles in a launch of
+    their own if that fits one round.  Bit for bit what slices of 700 tokens, at most 174 tiles, give."""
+    N, M = 256, 2100                                                    # nine token tiles, 29 / 31 / 41 / 58 row tiles
+    mk = lambda k, s: F.synth_packed(k, N, F.BLKC, 4, 128, 16, seed=s, device=DEV)
+    if vectors == 1:
+        pm = mk(rows, 0)
+    elif vectors == 2:
+        pm = F.fuse_rows([mk(rows // 2, 0), mk(rows // 2, 1)], interleave=True)
+    else:
+        pm = F.fuse_rows([mk(rows // 512 * 256, 0), mk(256, 1), mk(rows - rows // 512 * 256 - 256, 2)])
+    pm = pm.to_tiled()
+    x = acts(M, N, torch.float16, seed=7).to(DEV)
+    for act in (None, "silu") if vectors == 2 else (None,):
+        y = gemm_as(pm, x, "tile", 256, act=act)
+        assert torch.equal(y, torch.cat([gemm_as(pm, x[i:i + 700], "tile", 256, act=act) for i in range(0, M, 700)])), act
+
+
 @pytest.mark.parametrize("act", ["gelu_tanh", "silu"])
 @pytest.mark.parametrize("case", [c for c in CASES if c[2:] in ((128, 16), (64, 10), (128, 0))], ids=case_id)
 def test_gated_call_on_every_tile(case, act):
