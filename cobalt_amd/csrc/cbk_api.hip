@@ -643,6 +643,13 @@ GemmChoice gemm_choice(const cbk_desc* in, int M, int act) {
   return {p.kernel, p.ti, p.nsplit};
 }
 
+void gemm_last_round(const cbk_desc* in, int M, const GemmChoice& c, int* row_tiles, int* ti) {
+  DMat m;
+  const LastRound r = M < 1 || to_dmat(in, &m, false) ? LastRound() : last_round_big(m, named_plan(m, M, c), M);
+  *row_tiles = r.rows;
+  *ti = r.ti;
+}
+
 size_t gemm_as_workspace_bytes(const cbk_desc* in, int M, const GemmChoice& c, int act, int y_dtype) {
   DMat m;
   if (M < 1 || to_dmat(in, &m, false)) return 0;

@@ -166,22 +166,6 @@ static int gb_part(const DMat& m, int nsplit) {
   const int nst = gb_npad(m.N) / GB_K, per = ((nst + nsplit - 1) / nsplit + 3) / 4 * 4;
   return nsplit > 1 && (nsplit - 1) * per >= nst ? 0 : per;
 }
-// Last round of a launch of 256-token tiles.  Tiles beyond a whole number of rounds over the 256 CUs keep a few CUs busy
-// for a whole tile time; the row tiles that hold them go into a second launch of 64- or 128-token tiles if those fit one
-// round.  Every output is the same sum in the same order whatever its tile.  Measured, N = 5376 at 2048 tokens, with the
-// preparation: 64 tiles of 256 tokens 134 us, as 128 of 128 103, as 256 of 64 88; 128 tiles 135, as 256 of 128 109, as
-// 512 of 64 162 (two rounds: not taken).
-struct GbTail { int rows, ti; };                                    // row tiles of the second launch (0: none), its tile
-static GbTail gb_tail(int tiles_r, int M, bool pairs) {
-  const int tiles_t = (M + GB_T - 1) / GB_T, full = tiles_t * tiles_r / 256, left = tiles_t * tiles_r - 256 * full;
-  if (!full || !left) return {0, 4};
-  int rows = (left + tiles_t - 1) / tiles_t;
-  if (pairs) rows += rows & 1;                                      // both parities of a row range
-  if (rows >= tiles_r) return {0, 4};
-  for (int ti = 1; ti <= 2; ++ti)
-    if ((M + 64 * ti - 1) / (64 * ti) * rows <= 256) return {rows, ti};
-  return {0, 4};
-}
 static GemmPlan gb_plan_ti(const DMat& m, int M, int ti, int max_split, size_t room) {
   const int T = 64 * ti;
   const int tiles = ((M + T - 1) / T) * ((m.K + GB_R - 1) / GB_R);
@@ -193,11 +177,7 @@ static GemmPlan gb_plan_ti(const DMat& m, int M, int ti, int max_split, size_t r
     if (!per) continue;
     const size_t bytes = gb_space(m, M, ti, s);
     if (bytes > room) continue;
-    double rounds = (double)((tiles * s + 255) / 256);
-    if (s == 1 && ti == 4 && gb_fast(m)) {                          // (shares of a tile time that the smaller tiles take)
-      const GbTail tail = gb_tail((m.K + GB_R - 1) / GB_R, M, m.cs_rows == 2);
-      if (tail.rows) rounds -= tail.ti == 1 ? 0.30 : 0.20;
-    }
+    const double rounds = (double)((tiles * s + 255) / 256);
     double t = rounds * (per * t_stage + t_wg);
     if (s > 1) t += 2.0 * s * (double)M * m.K * 4 / 4.0e6 + 5.0;
     if (s == 1) best = one = {GEMM_TILE, ti, 1, t, bytes};
@@ -237,6 +217,31 @@ GemmPlan plan_big(const DMat& m, int M, size_t room) {
   const double parts = p.nsplit > 1 ? 2.0 * p.nsplit * (double)M * m.K * 4 : 0.0;
   p.t = (p.t - parts * (1 / 4.0e6 - 1 / 6.5e6)) * (gb_fast(m) ? 1.0 : 10.0) + 5.0;
   return p;
+}
+
+// Last round of a launch of 256-token tiles.  Tiles beyond a whole number of rounds over the 256 CUs keep a few CUs busy
+// for a whole tile time; the row tiles that hold them go into a second launch of 64- or 128-token tiles if those fit one
+// round.  Every output is the same sum in the same order whatever its tile.  Measured, N = 5376 at 2048 tokens, with the
+// preparation: 64 tiles of 256 tokens 134 us, as 128 of 128 103, as 256 of 64 88; 128 tiles 135, as 256 of 128 109, as
+// 512 of 64 162 (two rounds: not taken).
+// The plan does not count it: a share of a tile time taken off the unsplit 256-token plan moved calls onto it that ran
+// faster where they were (us before / after: 38323 x 256 at 294 tokens, 128-token tile, 44 / 54; 30878 x 7680 at 587,
+// 96-token rows, 351 / 380; 5376 x 21504 at 3600, three parts, 923 / 946), off the 64-token rows kernel, which does not
+// round weights, and within the room of cbk_gemm_static.
+static int gb_row_tiles(const DMat& m) {                            // (gate/up: both parities of each range of rows)
+  return m.cs_rows == 2 ? 2 * ((m.K + 2 * GB_R - 1) / (2 * GB_R)) : (m.K + GB_R - 1) / GB_R;
+}
+LastRound last_round_big(const DMat& m, const GemmPlan& p, int M) {
+  if (p.kernel != GEMM_TILE || p.ti != 4 || p.nsplit != 1 || !gb_fast(m)) return LastRound();
+  const int tiles_r = gb_row_tiles(m), tiles_t = (M + GB_T - 1) / GB_T;
+  const int full = tiles_t * tiles_r / 256, left = tiles_t * tiles_r - 256 * full;
+  if (!full || !left) return LastRound();
+  int rows = (left + tiles_t - 1) / tiles_t;
+  if (m.cs_rows == 2) rows += rows & 1;
+  if (rows >= tiles_r) return LastRound();
+  for (int ti = 1; ti <= 2; ++ti)
+    if ((M + 64 * ti - 1) / (64 * ti) * rows <= 256) return {rows, ti};
+  return LastRound();
 }
 
 static int gb_launch(const GbArgs& a, hipStream_t st) {
@@ -297,9 +302,8 @@ int launch_gemm_big(const DMat& m, const GemmPlan& plan, const void* x, int xdt,
   a.ti = plan.ti;
   a.tr0 = 0;
   a.tiles_t = (M + T - 1) / T;
-  a.tiles_r = par ? 2 * ((m.K + 2 * GB_R - 1) / (2 * GB_R)) : (m.K + GB_R - 1) / GB_R;
-  const GbTail tail = a.ti == 4 && a.nsplit == 1 && gb_fast(m) ? gb_tail(a.tiles_r, M, par != 0) : GbTail{0, 4};
-  a.tiles_r -= tail.rows;
+  const LastRound tail = last_round_big(m, plan, M);
+  a.tiles_r = gb_row_tiles(m) - tail.rows;
   int rc = gb_launch(a, st);
   if (rc == CBK_OK && tail.rows) {
     a.tr0 = a.tiles_r;

@@ -22,6 +22,9 @@ GemmPlan plan_big(const DMat&, int M, size_t room);
 // A given tile and split as a plan, for callers that name one; GEMM_NONE where the kernel cannot run it.
 GemmPlan fixed_plan_skinny(const DMat&, int M, int ti, int nsplit);
 GemmPlan fixed_plan_big(const DMat&, int M, int ti, int nsplit);
+// The row tiles of a plan of 256-token tiles that run as smaller tiles (64 ti tokens) in a launch of their own; rows 0: none.
+struct LastRound { int rows = 0, ti = 0; };
+LastRound last_round_big(const DMat&, const GemmPlan&, int M);
 // What the tile kernel takes with every q|k|v matrix in one piece (see gemm_room in cbk_api.hip).
 size_t big_unsplit_space(const DMat&, int M);
 bool gemm_skinny_takes(const DMat&);

@@ -15,6 +15,7 @@ size_t decode_workspace_bytes(const cbk_desc*, int M);
 // act: -1 for cbk_gemm, an activation for cbk_linear_act (y_dtype counts only there).
 struct GemmChoice { int kernel, ti, nsplit; };
 GemmChoice gemm_choice(const cbk_desc*, int M, int act);
+void gemm_last_round(const cbk_desc*, int M, const GemmChoice&, int* row_tiles, int* ti);   // of such a call: LastRound in cbk_gemm_plan.h
 size_t gemm_as_workspace_bytes(const cbk_desc*, int M, const GemmChoice&, int act, int y_dtype);   // 0: it cannot be run so
 int gemm_as(const cbk_desc*, const GemmChoice&, const void* x, int x_dtype, int M, int64_t ldx, void* y, int y_dtype, int64_t ldy,
             const void* bias, int act, void* workspace, size_t workspace_bytes, void* stream);

@@ -294,6 +294,20 @@ PyObject* py_gemm_plan(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// gemm_last_round(matrix, M, kernel, ti, nsplit) -> (row tiles, ti); see cbk::gemm_last_round
+PyObject* py_gemm_last_round(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (!arity(n, 5)) return nullptr;
+  return guarded([&]() -> PyObject* {
+    const cbk_desc d = desc_of(as_matrix(a[0]));
+    const long M = PyLong_AsLong(a[1]);
+    const cbk::GemmChoice c{(int)PyLong_AsLong(a[2]), (int)PyLong_AsLong(a[3]), (int)PyLong_AsLong(a[4])};
+    if (PyErr_Occurred()) throw Fail{};
+    int rows, ti;
+    cbk::gemm_last_round(&d, (int)M, c, &rows, &ti);
+    return Py_BuildValue("ii", rows, ti);
+  });
+}
+
 // gemm_as(matrix, x, bias, out_dtype, kernel, ti, nsplit, act or -1) -> y; see cbk::gemm_as
 PyObject* py_gemm_as(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!arity(n, 8)) return nullptr;
@@ -514,6 +528,7 @@ PyMethodDef methods[] = {
     {"linear_act", (PyCFunction)(void (*)())py_linear_act, METH_FASTCALL, nullptr},
     {"gemv_batch", (PyCFunction)(void (*)())py_gemv_batch, METH_FASTCALL, nullptr},
     {"gemm_plan", (PyCFunction)(void (*)())py_gemm_plan, METH_FASTCALL, nullptr},
+    {"gemm_last_round", (PyCFunction)(void (*)())py_gemm_last_round, METH_FASTCALL, nullptr},
     {"gemm_as", (PyCFunction)(void (*)())py_gemm_as, METH_FASTCALL, nullptr},
     {"dequant", (PyCFunction)(void (*)())py_dequant, METH_FASTCALL, nullptr},
     {"pack_begin", (PyCFunction)(void (*)())py_pack_begin, METH_FASTCALL, nullptr},

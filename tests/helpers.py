@@ -92,3 +92,9 @@ def gemm_plan(pm, M, act=None):
     """(kernel, tokens, nsplit) the library runs such a call on; (None, 0, 0): neither."""
     k, ti, s = _lib.native().gemm_plan(pm.native(), M, -1 if act is None else _lib.ACT_CODE[act])
     return {0: None, 1: "rows", 2: "tile"}[k], ti * (32 if k == 1 else 64), s
+
+
+def last_round(pm, M, kernel, tokens, nsplit=1):
+    """(row tiles, tokens) of the second launch such a call ends with; (0, 0): it is one launch."""
+    rows, ti = _lib.native().gemm_last_round(pm.native(), M, KERNELS[kernel], tokens // (32 if kernel == "rows" else 64), nsplit)
+    return rows, 64 * ti

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from cobalt_amd import _lib, format as F, ops
-from helpers import TOKENS, acts, case_id, gemm_as, gemm_plan
+from helpers import TOKENS, acts, case_id, gemm_as, gemm_plan, last_round
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -90,11 +90,14 @@ def test_runs_of_kept_columns(case):
 
 
 @pytest.mark.parametrize("vectors", [1, 2, 3], ids=["plain", "gate_up", "qkv"])
-@pytest.mark.parametrize("rows", [7423, 7700, 10300, 14800], ids=["64 tokens", "64 tokens, ragged", "128 tokens", "none"])
-def test_last_round_in_smaller_tiles(rows, vectors):
+@pytest.mark.parametrize("rows,tail", [(7423, {1: (1, 64), 2: (2, 64), 3: (1, 64)}), (7700, {1: (3, 64), 2: (4, 64), 3: (3, 64)}),
+                                       (10300, {1: (13, 128), 2: (14, 128), 3: (13, 128)}), (14800, {1: (2, 64), 2: (2, 64), 3: (2, 64)}),
+                                       (12800, {1: (0, 0), 2: (0, 0), 3: (0, 0)})],
+                         ids=["64 tokens", "64 tokens, ragged", "128 tokens", "third round", "none"])
+def test_last_round_in_smaller_tiles(rows, tail, vectors):
     """More than 256 tiles of 256 tokens: the row tiles past the last whole round run as smaller tiles in a launch of
-    their own if that fits one round.  Bit for bit what slices of 700 tokens, at most 174 tiles, give."""
-    N, M = 256, 2100                                                    # nine token tiles, 29 / 31 / 41 / 58 row tiles
+    their own if that fits one round (`tail`).  Bit for bit what slices of 700 tokens, at most 174 tiles, give."""
+    N, M = 256, 2100                                                    # nine token tiles, 29 / 31 / 41 / 58 / 50 row tiles
     mk = lambda k, s: F.synth_packed(k, N, F.BLKC, 4, 128, 16, seed=s, device=DEV)
     if vectors == 1:
         pm = mk(rows, 0)
@@ -104,6 +107,7 @@ def test_last_round_in_smaller_tiles(rows, vectors):
         pm = F.fuse_rows([mk(rows // 512 * 256, 0), mk(256, 1), mk(rows - rows // 512 * 256 - 256, 2)])
     pm = pm.to_tiled()
     x = acts(M, N, torch.float16, seed=7).to(DEV)
+    assert last_round(pm, M, "tile", 256) == tail[vectors] and last_round(pm, 700, "tile", 256) == (0, 0)
     for act in (None, "silu") if vectors == 2 else (None,):
         y = gemm_as(pm, x, "tile", 256, act=act)
         assert torch.equal(y, torch.cat([gemm_as(pm, x[i:i + 700], "tile", 256, act=act) for i in range(0, M, 700)])), act

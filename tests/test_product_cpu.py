@@ -233,6 +233,32 @@ def test_prefill_results_do_not_depend_on_the_workspace():
         d = desc(fmt, K, N, cs)
         assert (L.cbk_gemm_static(ctypes.byref(d), 0x8000, 1, M, N, 0x9000, 1, K, None, None) == -6) == (not takes), (fmt, K, N, M)
         assert (L.cbk_workspace_bytes(ctypes.byref(d), M) <= 16 << 20) == takes
+    # the tile kernel's split of these does not fit, whatever the plan that the call then runs on takes
+    for fmt, K, N, M in ((b64_2, 44547, 13184, 320), (fmts[5], 45932, 9600, 270)):
+        assert L.cbk_gemm_static(ctypes.byref(desc(fmt, K, N, 1)), 0x8000, 1, M, N, 0x9000, 1, K, None, None) == -6, (fmt, K, N, M)
+
+
+def _sizes_only(K, N, case, cs_rows=1):
+    """A matrix for questions about sizes: no memory behind its arrays."""
+    return _lib.native().Matrix(torch.empty(0, dtype=torch.uint8), dict.fromkeys(("data", "scale", "zero", "col_scale"), 0), (0, 0),
+                                (K, N, *case, cs_rows, F.FLAG_ZERO_LE_128 | F.FLAG_ZERO_ON_GRID))
+
+
+@pytest.mark.parametrize("K,N,cs_rows,M,plan,tail", [
+    (5376, 21504, 1, 3485, (2, 4, 4), (3, 1)), (5376, 21504, 1, 3600, (2, 4, 3), (4, 1)), (21504, 5376, 1, 816, (1, 3, 1), (20, 2)),
+    (21504, 5376, 1, 864, (1, 3, 1), (20, 2)), (14336, 4096, 1, 1200, (1, 3, 1), (5, 1)), (44224, 2176, 1, 289, (1, 2, 1), (45, 1)),
+    (38323, 256, 1, 294, (2, 2, 1), (22, 1)), (36612, 768, 2, 278, (2, 2, 1), (16, 1)), (21504, 5376, 1, 1024, (2, 4, 1), (20, 2)),
+    (43008, 5376, 2, 2048, (2, 4, 1), (8, 1)), (34516, 256, 2, 519, (2, 4, 1), (0, 0)), (21716, 256, 2, 519, (2, 4, 1), (2, 1))])
+def test_the_last_round_of_smaller_tiles_does_not_choose_the_plan(K, N, cs_rows, M, plan, tail):
+    """Kernel, token tile and split of a call (1: rows kernel, 2: tile kernel) go by whole rounds.  `tail`, the row tiles
+    and the 64-token units of the second launch that a call on unsplit 256-token tiles ends with, takes no part: counted
+    as a share of a round, it moved the calls of the first eight cases to that plan, where most run slower, some
+    with weights rounded to a half that were not.  Gate/up row tiles (cs_rows 2) count in pairs, as they are launched."""
+    h = _sizes_only(K, N, (F.BLK1632_4, 4, 128, 16), cs_rows)
+    assert _lib.native().gemm_plan(h, M, -1) == plan
+    assert _lib.native().gemm_last_round(h, M, 2, 4, 1) == tail
+    for other in ((2, 2, 1), (2, 4, 2), (1, 3, 1)):
+        assert _lib.native().gemm_last_round(h, M, *other) == (0, 0)
 
 
 def test_ops_refuse_to_run_without_gpu_tensors():
