@@ -53,7 +53,7 @@ constexpr int GV_THREADS = GV_WAVES * 64;
 #endif
 constexpr int LUT_LANES = CBK_LUT_LANES;      // lane-private copies of the selector table
 constexpr int LUT_BYTES = 256 * LUT_LANES * 8;
-constexpr int WIDE_LUT_LANES = 16, WIDE_LUT_BYTES = 256 * WIDE_LUT_LANES * 16;   // one activation row: see fetch_selectors
+constexpr int WIDE_LUT_LANES = 16, WIDE_LUT_BYTES = 256 * WIDE_LUT_LANES * 16;   // see fetch_selectors
 constexpr int ZERO_BYTES = 256;
 constexpr int CNT_SLOTS = 64;                 // most reduction slots (arrival counters)
 constexpr int CNT_BYTES = CNT_SLOTS * 4;       // at a fixed place: zeroed before the arguments are read
@@ -361,8 +361,8 @@ __device__ inline void build_table(uint8_t* lut, int tid) {
 // the counts a population count and a shift.  Per mask byte, four wavefronts per SIMD: 42 cycles of vector
 // instructions with the small table, 34 with the wide one; a wavefront's table read takes the LDS 5.9 cycles (eight
 // copies of 8 bytes: conflicts) and 4.3.  Two layers of 5376 / 21504 columns at one row, weights from memory, 112.3 ->
-// 110.6 us, of which the launches that are long enough (see launch_main_batch) take 0.3 - 0.7 less each; what is left of
-// those is memory.
+// 110.6 us, of which the launches that are long enough (see launch_main_batch and launch_split_batch) take 0.3 - 0.7
+// less each.
 template <class C, bool WT>
 __device__ inline void fetch_selectors(uint32_t mw, const uint8_t* lut, uint32_t lane_off, uint32_t (&sh)[4], uint2 (&sel4)[4]) {
   if constexpr (WT) {
@@ -2483,31 +2483,30 @@ static int launch_split_as(const GsArgs& a, size_t lds, int blocks, int red_bloc
   return hipGetLastError() == hipSuccess ? CBK_OK : CBK_ERR_HIP;
 }
 template <int BITS, int KEEP, int GRP, int MP>
-static int launch_split_cfg(const GsArgs& a, size_t lds, int blocks, int red_blocks, hipStream_t st) {
+static int launch_split_cfg(const GsArgs& a, size_t lds, int blocks, int red_blocks, bool wide, hipStream_t st) {
   if constexpr (KEEP != 0) {
-    if (lds + WIDE_LUT_BYTES - LUT_BYTES <= 160 * 1024)
-      return launch_split_as<BITS, KEEP, GRP, MP, true>(a, lds + WIDE_LUT_BYTES - LUT_BYTES, blocks, red_blocks, st);
+    if (wide) return launch_split_as<BITS, KEEP, GRP, MP, true>(a, lds, blocks, red_blocks, st);
   }
   return launch_split_as<BITS, KEEP, GRP, MP, false>(a, lds, blocks, red_blocks, st);
 }
 template <int BITS, int KEEP>
-static int launch_split_grp(const GsArgs& a, size_t lds, int blocks, int red_blocks, hipStream_t st) {
+static int launch_split_grp(const GsArgs& a, size_t lds, int blocks, int red_blocks, bool wide, hipStream_t st) {
   if constexpr (BITS != 6) {
     if (a.mat[0].g.m.group == 64)
-      return a.h.M > 4 ? launch_split_cfg<BITS, KEEP, 64, 8>(a, lds, blocks, red_blocks, st)
-                       : launch_split_cfg<BITS, KEEP, 64, 4>(a, lds, blocks, red_blocks, st);
+      return a.h.M > 4 ? launch_split_cfg<BITS, KEEP, 64, 8>(a, lds, blocks, red_blocks, wide, st)
+                       : launch_split_cfg<BITS, KEEP, 64, 4>(a, lds, blocks, red_blocks, wide, st);
   }
-  return a.h.M > 4 ? launch_split_cfg<BITS, KEEP, 128, 8>(a, lds, blocks, red_blocks, st)
-                   : launch_split_cfg<BITS, KEEP, 128, 4>(a, lds, blocks, red_blocks, st);
+  return a.h.M > 4 ? launch_split_cfg<BITS, KEEP, 128, 8>(a, lds, blocks, red_blocks, wide, st)
+                   : launch_split_cfg<BITS, KEEP, 128, 4>(a, lds, blocks, red_blocks, wide, st);
 }
 template <int BITS>
-static int launch_split_keep(const GsArgs& a, size_t lds, int blocks, int red_blocks, hipStream_t st) {
+static int launch_split_keep(const GsArgs& a, size_t lds, int blocks, int red_blocks, bool wide, hipStream_t st) {
   const DMat& m = a.mat[0].g.m;
   switch (family_of(m.layout) == FAM_DENSE ? 0 : m.keep) {
-    case 0: return launch_split_grp<BITS, 0>(a, lds, blocks, red_blocks, st);
-    case 10: return launch_split_grp<BITS, 10>(a, lds, blocks, red_blocks, st);
-    case 16: return launch_split_grp<BITS, 16>(a, lds, blocks, red_blocks, st);
-    case 23: return launch_split_grp<BITS, 23>(a, lds, blocks, red_blocks, st);
+    case 0: return launch_split_grp<BITS, 0>(a, lds, blocks, red_blocks, wide, st);
+    case 10: return launch_split_grp<BITS, 10>(a, lds, blocks, red_blocks, wide, st);
+    case 16: return launch_split_grp<BITS, 16>(a, lds, blocks, red_blocks, wide, st);
+    case 23: return launch_split_grp<BITS, 23>(a, lds, blocks, red_blocks, wide, st);
     default: return CBK_ERR_UNSUPPORTED;
   }
 }
@@ -2526,7 +2525,17 @@ static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt,
     delta_cap = delta_cap > M * (mats[i].m.N / 128 + 4) ? delta_cap : M * (mats[i].m.N / 128 + 4);
   }
   const int ND = digits_of(mats[0].m.bits);
-  const size_t fixed = (size_t)LUT_BYTES + ZERO_BYTES + (size_t)delta_cap * 4 + (size_t)M * ND * X_PAD;
+  // The wide selector table, for all matrices of the launch or none: where a part of each still fits beside it and the
+  // wavefronts have half a step each.  Below that its writing is not won back (us at eight rows, small / wide: 1024 x 5376,
+  // a sixth of a step, BLK1632_4 8.6 / 8.7, 3-bit keep 10 8.4 / 8.75; half a step, 2048 x 8192, 10.2 / 10.1 and 9.7 / 9.8;
+  // 1.75 steps, 4096 x 14336, 14.6 / 14.1 and 16.1 / 15.4) but by blocks whose codes are one dword, 2-bit with 16 of 32 kept,
+  // which gain at every size (1024 x 5376 9.6 / 9.2).  The slabs are the shorter for it.
+  constexpr size_t more = WIDE_LUT_BYTES - LUT_BYTES;
+  const DMat& m0 = mats[0].m;
+  const size_t small = (size_t)LUT_BYTES + ZERO_BYTES + (size_t)delta_cap * 4 + (size_t)M * ND * X_PAD;
+  bool wide = family_of(m0.layout) != FAM_DENSE && (2 * total >= 256 * GV_WAVES || m0.bits * m0.keep == BLOCK);
+  for (int i = 0; i < n; ++i) wide = wide && small + more + (size_t)M * ND * mats[i].spi * 512 <= 160 * 1024;
+  const size_t table = wide ? more : 0, fixed = small + table;
   int xq_cap = 0, wg = 0, th = 0;
   size_t off = 0;
   for (int i = 0; i < n; ++i) {
@@ -2540,8 +2549,7 @@ static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt,
     budget = budget < 1 ? 1 : budget;
     const size_t per_part = (size_t)M * ND * g.spi * 512;
     if (fixed + per_part > 160 * 1024) return CBK_ERR_UNSUPPORTED;
-    const bool wide = family_of(g.m.layout) != FAM_DENSE && fixed + WIDE_LUT_BYTES - LUT_BYTES + per_part <= 160 * 1024;
-    int pps_max = (int)((160 * 1024 - fixed - (wide ? WIDE_LUT_BYTES - LUT_BYTES : 0)) / per_part);
+    int pps_max = (int)((160 * 1024 - fixed) / per_part);
     pps_max = pps_max < g.sk ? pps_max : g.sk;
     // Parts per slab: a workgroup runs ceil(items / 16) rounds of one part per wavefront after
     // staging its slab (a 512-column step of M = 8 rows costs about 0.15 rounds of one step)
@@ -2571,13 +2579,13 @@ static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt,
   }
   for (int i = n; i < GV_MAX_BATCH; ++i) { a.h.wg_end[i] = 0x7fffffff; a.h.th_end[i] = 0x7fffffff; }
   a.h.xq_cap = xq_cap; a.h.delta_cap = delta_cap;
-  const size_t lds = (size_t)LUT_BYTES + ZERO_BYTES + xq_cap + (size_t)delta_cap * 4;
+  const size_t lds = (size_t)LUT_BYTES + table + ZERO_BYTES + xq_cap + (size_t)delta_cap * 4;
   if (lds > 160 * 1024) return CBK_ERR_UNSUPPORTED;
   const int bits = mats[0].m.bits, rb = th / GS_RED_THREADS;
-  if (bits == 6) return launch_split_grp<6, 16>(a, lds, wg, rb, st);  // BLK1632_6: one configuration
-  if (bits == 8) return launch_split_grp<8, 0>(a, lds, wg, rb, st);
-  return bits == 2 ? launch_split_keep<2>(a, lds, wg, rb, st) : bits == 3 ? launch_split_keep<3>(a, lds, wg, rb, st)
-       : bits == 4 ? launch_split_keep<4>(a, lds, wg, rb, st) : CBK_ERR_UNSUPPORTED;
+  if (bits == 6) return launch_split_grp<6, 16>(a, lds, wg, rb, wide, st);  // BLK1632_6: one configuration
+  if (bits == 8) return launch_split_grp<8, 0>(a, lds, wg, rb, wide, st);
+  return bits == 2 ? launch_split_keep<2>(a, lds, wg, rb, wide, st) : bits == 3 ? launch_split_keep<3>(a, lds, wg, rb, wide, st)
+       : bits == 4 ? launch_split_keep<4>(a, lds, wg, rb, wide, st) : CBK_ERR_UNSUPPORTED;
 }
 
 // Distribution over the workgroups, LDS and launch of the matrices of `gb` (spi and sk set).

@@ -342,8 +342,8 @@ def test_gemv_every_kernel_configuration(case, tiled):
                                       (12304, 4096, (1, 4, 5))],
                          ids=["under_five_quarters_of_a_step", "five_quarters", "last_with_room", "no_room", "tall"])
 def test_gemv_on_either_side_of_the_wide_table(case, K, N, rows):
-    """The selector table of the decode kernels has two forms; a launch takes the wide one from five quarters of a step
-    per wavefront on (two tiles of sixteen rows: 10240 columns) where LDS has room for it (one row: up to about 30000
+    """The selector table of the decode kernels has two forms; a launch of the main kernel takes the wide one from five
+    quarters of a step per wavefront on (two tiles of sixteen rows: 10240 columns) where LDS has room for it (one row: up to about 30000
     columns).  Shapes on both sides of either line, and tall ones for the kernels of several rows: the float64 product to
     the decode bar, and row m of M bit for bit what it is alone."""
     pm = F.synth_packed(K, N, *case[:3], case[3], seed=N, device=DEV).to_tiled()
@@ -354,6 +354,26 @@ def test_gemv_on_either_side_of_the_wide_table(case, K, N, rows):
     assert float((alone - ref).abs().max() / ref.abs().max()) < 2e-5
     for M in rows:
         assert torch.equal(ops.gemv(pm, x[:M], out_dtype=torch.float32), alone[:M]), M
+
+
+@pytest.mark.parametrize("case", [(F.BLK1632_4, 4, 128, 16), (F.BLKC, 3, 64, 10), (F.BLKC, 2, 64, 16), (F.BLKC, 3, 64, 23), (F.BLK1632_6, 6, 128, 16)],
+                         ids=case_id)
+@pytest.mark.parametrize("shapes", [[(2976, 5376)], [(2992, 5376)], [(2992, 5376), (40, 65024)]], ids=["under_half_a_step", "half_a_step", "no_room"])
+def test_split_gemv_on_either_side_of_the_wide_table(case, shapes):
+    """The column-split decode kernels take the wide table from half a step per wavefront on (2048 tile-steps; 186 tiles
+    of 11 steps are 2046), for all matrices of a launch or none: beside eight rows of a part of 65024 columns there is no
+    room for it.  The float64 product to the decode bar, and the rows of eight bit for bit what pairs of them give (the
+    main kernel, but for 65024 columns)."""
+    pms = [F.synth_packed(K, N, *case[:3], case[3], seed=K, device=DEV).to_tiled() for K, N in shapes]
+    xs = [acts(8, N, torch.float16, seed=N).to(DEV) for _, N in shapes]
+    assert all(8 * 3 * N > 90 * 1024 for _, N in shapes)
+    ys = ops.gemv_batch(pms, xs, out_dtype=torch.float32)
+    pairs = [ops.gemv_batch(pms, [x[m:m + 2] for x in xs], out_dtype=torch.float32) for m in range(0, 8, 2)]
+    for i, (pm, x) in enumerate(zip(pms, xs)):
+        ref = x.double() @ ops.dequant(pm, torch.float32).double().T
+        assert float((ys[i] - ref).abs().max() / ref.abs().max()) < 2e-5
+        assert torch.equal(ys[i], torch.cat([p[i] for p in pairs]))
+    assert all(torch.equal(a, b) for a, b in zip(ys, ops.gemv_batch(pms, xs, out_dtype=torch.float32)))
 
 
 def test_gemv_batch_matches_single_calls():
