@@ -23,8 +23,24 @@ def _llvm(tool):
     return os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "lib", "llvm", "bin", tool)
 
 
-_KD = re.compile(r"\.(agpr_count|vgpr_count|name|symbol):\s+(\S+)")
+_KD = re.compile(r"\.(agpr_count|group_segment_fixed_size|vgpr_count|symbol):\s+(\S+)")
 _SHIFT64 = re.compile(r"\b(v_(?:lshl|lshr|ashr)rev_[bi]64)\S*\s+v\[\d+:\d+\], v(\d+),")
+
+
+def _kernels(code_object):
+    """{kernel: its architectural vector registers and bytes of static LDS}, from the notes of a code object."""
+    notes = subprocess.run([_llvm("llvm-readelf"), "--notes", code_object], check=True, capture_output=True, text=True).stdout
+    out, cur = {}, {}
+    for key, val in _KD.findall(notes):                                # (the keys of a kernel come in alphabetical order)
+        if key == "agpr_count":
+            cur = {"agpr": int(val)}
+        elif key == "group_segment_fixed_size":
+            cur["lds"] = int(val)
+        elif key == "symbol":
+            cur["symbol"] = val[:-3] if val.endswith(".kd") else val
+        elif key == "vgpr_count" and "symbol" in cur:
+            out[cur["symbol"]] = (int(val) - cur.get("agpr", 0), cur.get("lds", 0))
+    return out
 
 
 def shift_hazards(code_object):
@@ -36,15 +52,7 @@ def shift_hazards(code_object):
     registers and returned sums off by 1e-2 that changed from run to run; the same instructions with
     232 registers given are exact.  The compiler knows the case for gfx90a, where it moves the
     amount, but does not look for it on gfx950.  Registers are given in blocks of eight."""
-    notes = subprocess.run([_llvm("llvm-readelf"), "--notes", code_object], check=True, capture_output=True, text=True).stdout
-    arch, cur = {}, {}
-    for key, val in _KD.findall(notes):
-        if key == "agpr_count":
-            cur = {"agpr": int(val)}
-        elif key == "symbol":
-            cur["symbol"] = val[:-3] if val.endswith(".kd") else val
-        elif key == "vgpr_count" and "symbol" in cur:                  # (the keys of a kernel come in alphabetical order)
-            arch[cur["symbol"]] = int(val) - cur.get("agpr", 0)
+    arch = {k: v[0] for k, v in _kernels(code_object).items()}
     out, fn = [], ""
     dis = subprocess.Popen([_llvm("llvm-objdump"), "-d", "--no-show-raw-insn", code_object], stdout=subprocess.PIPE, text=True)
     for line in dis.stdout:
@@ -66,15 +74,33 @@ def shift_hazards(code_object):
     return out
 
 
-def shift_hazards_of(path):
-    """The same for every gfx950 code object inside an object file or library."""
+# Kernels whose table reads take an entry's offset in dynamic LDS as its address: nothing else may lie before it.
+LDS_FROM_ZERO = ("gemm_skinny_kernel",)
+
+
+def static_lds(code_object):
+    """[(kernel, bytes)]: the kernels of LDS_FROM_ZERO that have static LDS, which would move their table off address 0
+    and have them multiply with wrong weights."""
+    return [(k, lds) for k, (_, lds) in _kernels(code_object).items() if lds and any(n in k for n in LDS_FROM_ZERO)]
+
+
+def _of_every_code_object(check, path):
+    """What `check` finds in every gfx950 code object inside an object file or library."""
     with tempfile.TemporaryDirectory() as tmp:
         link = os.path.join(tmp, "o")
         os.symlink(os.path.abspath(path), link)
         subprocess.run([_llvm("llvm-objdump"), "--offloading", link], check=True, capture_output=True)
         objs = [os.path.join(tmp, f) for f in sorted(os.listdir(tmp)) if "gfx950" in f]
         with ThreadPoolExecutor(8) as ex:
-            return [h for hs in ex.map(shift_hazards, objs) for h in hs]
+            return [h for hs in ex.map(check, objs) for h in hs]
+
+
+def shift_hazards_of(path):
+    return _of_every_code_object(shift_hazards, path)
+
+
+def static_lds_of(path):
+    return _of_every_code_object(static_lds, path)
 
 
 def build_lib(verbose=True, extra=()):
@@ -99,6 +125,11 @@ def build_lib(verbose=True, extra=()):
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
+    bad = static_lds_of(LIB)
+    if bad:
+        os.remove(LIB)
+        raise RuntimeError("static LDS in kernels that read from LDS address 0 (see static_lds):\n" +
+                           "\n".join(f"  {n} bytes in {fn}" for fn, n in bad))
     bad = shift_hazards_of(LIB)
     if bad:
         os.remove(LIB)

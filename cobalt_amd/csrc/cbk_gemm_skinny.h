@@ -160,8 +160,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   constexpr bool DEFER = C::DEFER;
   constexpr int ST = C::ST, NG = C::NG, NA = C::NA;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  uint4* lut = (uint4*)smem;                                        // [256][copies]: selectors, byte masks (first: an entry's
-  float* red = (float*)(smem + SK_LUT);                             // address is its offset)
+  // [256][copies]: selectors, byte masks.  First: an entry's address is its offset, so this kernel and what it inlines have
+  // no static __shared__ (the build refuses one)
+  uint4* lut = (uint4*)smem;
+  float* red = (float*)(smem + SK_LUT);
   const DMat& m = a.m;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = wave & 1, wc = wave >> 1, half = lane >> 5;

@@ -62,3 +62,23 @@ def test_no_kernel_of_the_library_has_one():
     if not os.path.exists(B.LIB):
         pytest.skip("the library is not built")
     assert B.shift_hazards_of(B.LIB) == []
+
+
+@pytest.mark.parametrize("name,lds,hit", [("_ZN3cbk18gemm_skinny_kernelILi4EEEvNS_6SkArgsE", 16, True),
+                                          ("_ZN3cbk18gemm_skinny_kernelILi4EEEvNS_6SkArgsE", 0, False), ("other", 16, False)])
+def test_static_lds_before_a_table_at_address_0_is_found(tmp_path, name, lds, hit):
+    src, obj = tmp_path / "k.s", str(tmp_path / "k.co")
+    text = KERNEL.format(op="v_lshrrev_b64", amount=6, n=8, agpr=0, accum=8)
+    text = text.replace(".group_segment_fixed_size: 0", f".group_segment_fixed_size: {lds}").replace(" .name: k", f" .name: {name}")
+    src.write_text(text.replace(".symbol: k.kd", f".symbol: {name}.kd"))
+    subprocess.run([B._llvm("clang"), "-target", "amdgcn-amd-amdhsa", "-mcpu=gfx950", str(src), "-o", obj], check=True)
+    assert B.static_lds(obj) == ([(name, lds)] if hit else [])
+
+
+def test_kernels_that_read_from_lds_address_0_have_no_static_lds():
+    """And the library holds kernels of the names that are looked for."""
+    if not os.path.exists(B.LIB):
+        pytest.skip("the library is not built")
+    assert B.static_lds_of(B.LIB) == []
+    names = B._of_every_code_object(B._kernels, B.LIB)
+    assert all(any(n in k for k in names) for n in B.LDS_FROM_ZERO)
