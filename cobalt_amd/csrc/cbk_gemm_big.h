@@ -32,9 +32,10 @@
 // 932 -> 764 vector instructions per 256 of the matrix cores (1028 -> 764 with two or three
 // column-scale vectors, whose activation base had stayed in vector registers).  Gated block of
 // 21504 x 5376 at 2048 tokens 1457 -> 1436 us.  More would have to come out of the energy of the
-// matrix instructions and of LDS: the clock falls with the load (one tile on every eighth CU
-// takes 132 us, one on every CU 167), spreading the copies over the stage changes nothing, a
-// second copy of each activation line costs 12 %.
+// matrix instructions and of LDS: the clock falls with the load (N = 5376, 256 tokens: one tile on
+// every eighth CU takes 126 us, one on every CU 163, both 296 thousand cycles of a wavefront's life),
+// spreading the copies over the stage changes nothing, a second copy of each activation line
+// costs 12 %.
 //
 // Workgroups are ordered so that those running at the same time on one XCD (blockIdx % 8)
 // share their token tile, which then stays in that XCD's L2.

@@ -25,9 +25,12 @@
 //    offset is its address), and scales are floats before they multiply: 4-bit codes, 64 tokens, 168 -> 135 cycles per
 //    step of 16 columns x 64 rows beside 144 of matrix instructions.  With the preparation, before and after: feed-forward
 //    block 14336 x 4096 at 48 rows 61.7 -> 58.9 us, 2-bit 6144 x 4096 at 333 rows 43.2 -> 41.6, fixed-stride 8-bit down
-//    projection 4096 x 14336 at 512 rows 90.0 -> 85.3.  At the last the clock falls to 1.6 - 1.7 GHz: what is left there
-//    is the power of the matrix instructions, which no schedule changes (the older
-//    of the two wavefronts of a SIMD ends 25 % early; priorities that keep them level leave the end where it is).
+//    projection 4096 x 14336 at 512 rows 90.0 -> 85.3.
+//  * No one unit is full.  Of a SIMD's cycles at 48, 333 and 512 rows of these three calls the matrix instructions take
+//    34, 35 and 46 %, the other vector instructions (four cycles each) 42, 42 and 39 %, both at once 15, 17 and 22 %; a
+//    wavefront waits at a counter or a barrier for 31, 33 and 25 % of its life; L2 sends a CU 28, 20 and 38 bytes per cycle.
+//    The clock falls as the matrix share grows (1.8, 1.9 and 1.6 GHz, life over duration).  (The older of the two
+//    wavefronts of a SIMD ends 25 % early; priorities that keep them level leave the end where it is.)
 //
 // k order.  A step is eight columns of the first half of a group (lanes 0-31) and eight of the second
 // (lanes 32-63): a lane walks half a group of its own row, nothing is loaded or ranked twice.  The

@@ -358,11 +358,11 @@ __device__ inline void build_table(uint8_t* lut, int tid) {
 // WT: the wide table, 16-byte entries of selectors and the stream bits of the byte's survivors, 256 bytes (sixteen
 // copies) apart, so that one permute of mask word and lane offset is an entry's address and the counting is done by
 // the table.  The small one has 8-byte entries, eight copies: an address takes a field extract and a shift and add,
-// the counts a population count and a shift.  Per mask byte, four wavefronts per SIMD: 42 cycles of vector
-// instructions with the small table, 34 with the wide one; a wavefront's table read takes the LDS 5.9 cycles (eight
-// copies of 8 bytes: conflicts) and 4.3.  Two layers of 5376 / 21504 columns at one row, weights from memory, 112.3 ->
-// 110.6 us, of which the launches that are long enough (see launch_main_batch and launch_split_batch) take 0.3 - 0.7
-// less each.
+// the counts a population count and a shift.  Gate and up of 21504 x 5376 (BLK1632_4, one row, weights from memory), small
+// and wide: 290 and 277 vector instructions per step of 16 rows x 512 columns, 2.3 and 0.7 million LDS bank conflicts, a
+// wavefront's life 35.8 and 34.8 thousand cycles, 23.8 and 22.6 us; 14336 x 4096, 3-bit keep 10: 438 and 429
+// instructions, 16.0 and 15.3 us.  Two layers of 5376 / 21504 columns 112.3 -> 110.6 us.  (Launches that are long
+// enough take it: launch_main_batch, launch_split_batch.)
 template <class C, bool WT>
 __device__ inline void fetch_selectors(uint32_t mw, const uint8_t* lut, uint32_t lane_off, uint32_t (&sh)[4], uint2 (&sel4)[4]) {
   if constexpr (WT) {
