@@ -13,7 +13,7 @@ int launch_gemv_generic(const DMat&, const void*, int, int, int64_t, void*, int,
 size_t gemv_stream_workspace(const DMat&, int M);
 struct GvCall { DMat m; const void* x; int64_t ldx; void* y; int64_t ldy; const void* bias; int par; };
 int launch_gemv_fast_batch(int n, const GvCall* calls, int xdt, int M, int ydt, void* ws, size_t ws_bytes,
-                           hipStream_t);
+                           hipStream_t, DecodeChoice* ask = nullptr);
 bool gemv_fast_takes(const DMat&, int M);
 bool gemv_same_config(const DMat&, const DMat&);
 size_t gemv_fast_workspace(const DMat&, int M);
@@ -641,6 +641,21 @@ GemmChoice gemm_choice(const cbk_desc* in, int M, int act) {
   if (M < 1 || to_dmat(in, &m, false) || family_of(m.layout) == FAM_SPARSE) return {GEMM_NONE, 0, 0};
   const GemmPlan p = act >= 0 ? act_plan(m, M) : gemm_plan(m, M, false, gemm_room(m, M));
   return {p.kernel, p.ti, p.nsplit};
+}
+
+int decode_choice(int n, const cbk_desc* descs, int M, DecodeChoice* out) {
+  if (n < 1 || n > kMaxBatch || M < 1) return CBK_ERR_SHAPE;
+  *out = DecodeChoice();
+  GvCall c[kMaxBatch];
+  for (int i = 0; i < n; ++i) {
+    c[i] = GvCall{};
+    const int rc = to_dmat(descs + i, &c[i].m, false);
+    if (rc) return rc;
+    c[i].par = c[i].m.cs_rows == 2 ? 1 : 0;
+    c[i].ldx = c[i].m.N; c[i].ldy = c[i].m.K;
+    if (!gemv_fast_takes(c[i].m, M * (c[i].par + 1)) || !gemv_same_config(c[0].m, c[i].m)) return CBK_ERR_UNSUPPORTED;
+  }
+  return launch_gemv_fast_batch(n, c, CBK_F16, M, CBK_F32, (void*)256, (size_t)1 << 60, nullptr, out);
 }
 
 void gemm_last_round(const cbk_desc* in, int M, const GemmChoice& c, int* row_tiles, int* ti) {

@@ -43,6 +43,7 @@
 // (src/cobaltkernel/csrc/cobalt_gemv.cuh:617-712, :839-1123): same sums, other machinery.
 #include <atomic>
 #include "cbk_decode.h"
+#include "cbk_internal.h"
 
 namespace cbk {
 
@@ -2515,7 +2516,7 @@ static int launch_split_keep(const GsArgs& a, size_t lds, int blocks, int red_bl
 // reduce kernel: workgroups per matrix by its share of the work, parts per slab, workgroups per
 // slab, LDS.  `ws` holds the part sums of the matrices one after the other, each
 // up256(split_part_bytes(ntiles, sk, M)).
-static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt, uint8_t* ws, hipStream_t st) {
+static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt, uint8_t* ws, hipStream_t st, DecodeChoice* ask) {
   GsArgs a;
   a.h.n = n; a.h.M = M; a.h.xdt = xdt; a.h.ydt = ydt;
   long long total = 0;
@@ -2581,6 +2582,7 @@ static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt,
   a.h.xq_cap = xq_cap; a.h.delta_cap = delta_cap;
   const size_t lds = (size_t)LUT_BYTES + table + ZERO_BYTES + xq_cap + (size_t)delta_cap * 4;
   if (lds > 160 * 1024) return CBK_ERR_UNSUPPORTED;
+  if (ask) { ask->split_table = wide ? 1 : 0; return CBK_OK; }
   const int bits = mats[0].m.bits, rb = th / GS_RED_THREADS;
   if (bits == 6) return launch_split_grp<6, 16>(a, lds, wg, rb, wide, st);  // BLK1632_6: one configuration
   if (bits == 8) return launch_split_grp<8, 0>(a, lds, wg, rb, wide, st);
@@ -2589,7 +2591,7 @@ static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt,
 }
 
 // Distribution over the workgroups, LDS and launch of the matrices of `gb` (spi and sk set).
-static int launch_main_batch(GvBatch& gb, hipStream_t st) {
+static int launch_main_batch(GvBatch& gb, hipStream_t st, DecodeChoice* ask) {
   const int n = gb.h.n, M = gb.h.M;
   int cost = 0, tiles = 0, delta_cap = 0, sk_cap = 1, xq_cap = 0;
   for (int i = 0; i < n; ++i) {
@@ -2634,23 +2636,33 @@ static int launch_main_batch(GvBatch& gb, hipStream_t st) {
   gb.h.xq_cap = xq_cap; gb.h.delta_cap = delta_cap;
   // reduction slots: as many as fit what is left, at most 24 KB: a power of two between 2 and 64
   const int slot_floats = sk_cap * M * 16;
-  // Bitmap layouts take the wide selector table where it leaves room for the slots and the wavefronts have five
-  // quarters of a step each: below that its writing and the longer way to a block's first window cost more than its
-  // shorter steps give (M = 1, us, small / wide: 0.5 steps, 3-bit 4096 x 4096 5.8 / 6.0; 1 step, 3-bit q,k,v of 4096 columns
-  // 7.2 / 7.5; 1.4 steps, 4-bit q,k,v of 5376 columns 8.5 / 8.0; 28672 columns, 3.5 steps, 14.4 / 13.8).
+  auto slots_beside = [&](size_t table) -> int {
+    if (fixed + table + (size_t)xq_cap + 2 * slot_bytes > 160 * 1024) return 0;
+    size_t room = 160 * 1024 - fixed - table - (size_t)xq_cap;
+    room = room < 24 * 1024 ? room : 24 * 1024;
+    int n = 64;
+    while (n > 2 && (size_t)n * slot_bytes > room) n >>= 1;
+    return n;
+  };
+  // Bitmap layouts take the wide selector table where the wavefronts have five quarters of a step each: below that its
+  // writing and the longer way to a block's first window cost more than its shorter steps give (M = 1, us, small / wide:
+  // 0.5 steps, 3-bit 4096 x 4096 5.8 / 6.0; 1 step, 3-bit q,k,v of 4096 columns 7.2 / 7.5; 1.4 steps, 4-bit q,k,v of 5376
+  // columns 8.5 / 8.0; 28672 columns, 3.5 steps, 14.4 / 13.8).
+  // And where it leaves the slots alone, or eight of them that hold six rounds of the wavefronts' parts: a wavefront
+  // that runs ahead waits for a slot.  Wide against small over nineteen formats, mean: sixteen slots still, eight rows,
+  // 65536 x 2944 0.98; eight instead of sixteen slots, 65536 x 3584 at eight rows (one round) 1.12, 32768 x 3072 (one and a
+  // half) 1.09, 28672 x 7168 at four rows (two) 1.07, 4096 x 27648 at one row (eight) 0.98.
   constexpr size_t more = WIDE_LUT_BYTES - LUT_BYTES;
-  const size_t slots = 8 * slot_bytes < 24 * 1024 ? 8 * slot_bytes : 2 * slot_bytes < 24 * 1024 ? 24 * 1024 : 2 * slot_bytes;
-  const bool wide = family_of(gb.mat[0].m.layout) != FAM_DENSE && 4LL * cost >= 5LL * blocks * GV_WAVES &&
-                    fixed + more + xq_cap + slots <= 160 * 1024;
-  const size_t table = wide ? more : 0;
-  size_t red_room = 160 * 1024 - fixed - table - (size_t)xq_cap;
-  red_room = red_room < 24 * 1024 ? red_room : 24 * 1024;
-  int nslot = 64;
-  while (nslot > 2 && (size_t)nslot * slot_bytes > red_room) nslot >>= 1;
+  const int small_slots = slots_beside(0), wide_slots = slots_beside(more);
+  if (!small_slots) return CBK_ERR_UNSUPPORTED;
+  const bool wide = family_of(gb.mat[0].m.layout) != FAM_DENSE && 4LL * cost >= 5LL * blocks * GV_WAVES && wide_slots &&
+                    (wide_slots == small_slots || (wide_slots >= 8 && wide_slots * sk_cap >= 6 * GV_WAVES));
+  const int nslot = wide ? wide_slots : small_slots;
   gb.h.sk_cap = sk_cap; gb.h.nslot = nslot; gb.h.red_floats = nslot * slot_floats;
   gb.h.cq = cost / blocks; gb.h.cr = cost % blocks;
-  const size_t lds = fixed + table + xq_cap + (size_t)gb.h.red_floats * 4;
+  const size_t lds = fixed + (wide ? more : 0) + xq_cap + (size_t)gb.h.red_floats * 4;
   if (lds > 160 * 1024) return CBK_ERR_UNSUPPORTED;
+  if (ask) { ask->main_table = wide ? 1 : 0; ask->main_slots = nslot; return CBK_OK; }
   const int bits = gb.mat[0].m.bits;
   if (bits == 6) return launch_mp<6, 16, 128>(gb, lds, blocks, wide, st);   // BLK1632_6: one configuration
   if (bits == 8) return launch_grp<8, 0>(gb, lds, blocks, false, st);
@@ -2660,8 +2672,9 @@ static int launch_main_batch(GvBatch& gb, hipStream_t st) {
 
 // All matrices share one kernel configuration (checked by the caller) and 1 <= M <= 8 (more than
 // four only where gemv_fast_takes says so).
+// ask: no launch, what it would be.
 int launch_gemv_fast_batch(int n, const GvCall* calls, int xdt, int M, int ydt, void* workspace, size_t ws_bytes,
-                           hipStream_t st) {
+                           hipStream_t st, DecodeChoice* ask) {
   if (n < 1 || n > GV_MAX_BATCH) return CBK_ERR_SHAPE;
   GvBatch gb;
   const int par = calls[0].par ? 1 : 0;
@@ -2728,13 +2741,13 @@ int launch_gemv_fast_batch(int n, const GvCall* calls, int xdt, int M, int ydt, 
       }
       gb.h.n = na;
       if (na > 0) {
-        const int rc = launch_main_batch(gb, st);
+        const int rc = launch_main_batch(gb, st, ask);
         if (rc != CBK_OK) return rc;
       }
-      return launch_split_batch(split, ns, M, xdt, ydt, (uint8_t*)workspace, st);
+      return launch_split_batch(split, ns, M, xdt, ydt, (uint8_t*)workspace, st, ask);
     }
   }
-  return launch_main_batch(gb, st);
+  return launch_main_batch(gb, st, ask);
 }
 
 }  // namespace cbk

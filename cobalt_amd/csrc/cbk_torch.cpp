@@ -282,6 +282,23 @@ PyObject* py_linear_act(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// decode_choice([matrix], M) -> (table of the main kernel, its slots, table of the split kernel); see cbk::decode_choice
+PyObject* py_decode_choice(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (!arity(n, 2)) return nullptr;
+  return guarded([&]() -> PyObject* {
+    if (!PyList_Check(a[0]) || PyList_GET_SIZE(a[0]) < 1 || PyList_GET_SIZE(a[0]) > 8)
+      fail(PyExc_TypeError, "a list of one to eight matrices is expected");
+    const int k = (int)PyList_GET_SIZE(a[0]);
+    cbk_desc d[8];
+    for (int i = 0; i < k; ++i) d[i] = desc_of(as_matrix(PyList_GET_ITEM(a[0], i)));
+    const long M = PyLong_AsLong(a[1]);
+    if (PyErr_Occurred()) throw Fail{};
+    cbk::DecodeChoice c;
+    check(cbk::decode_choice(k, d, (int)M, &c), "cbk::decode_choice");
+    return Py_BuildValue("iii", c.main_table, c.main_slots, c.split_table);
+  });
+}
+
 // gemm_plan(matrix, M, act or -1) -> (kernel, ti, nsplit); see cbk::gemm_choice
 PyObject* py_gemm_plan(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!arity(n, 3)) return nullptr;
@@ -527,6 +544,7 @@ PyMethodDef methods[] = {
     {"matmul", (PyCFunction)(void (*)())py_matmul, METH_FASTCALL, nullptr},
     {"linear_act", (PyCFunction)(void (*)())py_linear_act, METH_FASTCALL, nullptr},
     {"gemv_batch", (PyCFunction)(void (*)())py_gemv_batch, METH_FASTCALL, nullptr},
+    {"decode_choice", (PyCFunction)(void (*)())py_decode_choice, METH_FASTCALL, nullptr},
     {"gemm_plan", (PyCFunction)(void (*)())py_gemm_plan, METH_FASTCALL, nullptr},
     {"gemm_last_round", (PyCFunction)(void (*)())py_gemm_last_round, METH_FASTCALL, nullptr},
     {"gemm_as", (PyCFunction)(void (*)())py_gemm_as, METH_FASTCALL, nullptr},

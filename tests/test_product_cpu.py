@@ -241,7 +241,7 @@ def test_prefill_results_do_not_depend_on_the_workspace():
 def _sizes_only(K, N, case, cs_rows=1):
     """A matrix for questions about sizes: no memory behind its arrays."""
     return _lib.native().Matrix(torch.empty(0, dtype=torch.uint8), dict.fromkeys(("data", "scale", "zero", "col_scale"), 0), (0, 0),
-                                (K, N, *case, cs_rows, F.FLAG_ZERO_LE_128 | F.FLAG_ZERO_ON_GRID))
+                                (K, N, *case[:3], case[3] or 0, cs_rows, F.FLAG_ZERO_LE_128 | F.FLAG_ZERO_ON_GRID))
 
 
 @pytest.mark.parametrize("K,N,cs_rows,M,plan,tail", [
@@ -259,6 +259,25 @@ def test_the_last_round_of_smaller_tiles_does_not_choose_the_plan(K, N, cs_rows,
     assert _lib.native().gemm_last_round(h, M, 2, 4, 1) == tail
     for other in ((2, 2, 1), (2, 4, 2), (1, 3, 1)):
         assert _lib.native().gemm_last_round(h, M, *other) == (0, 0)
+
+
+@pytest.mark.parametrize("shapes,M,main,slots,split", [
+    # main kernel: one row on both sides of five quarters of a step per wavefront and of the room in LDS
+    ([(24, 9728)], 1, 0, 32, -1), ([(24, 10240)], 1, 1, 32, -1), ([(24, 29440)], 1, 1, 8, -1), ([(24, 31232)], 1, 0, 16, -1),
+    # several rows: the wide table beside as many slots, or beside eight that hold six rounds of parts; not for fewer
+    ([(65536, 2944)], 8, 1, 16, -1), ([(65536, 3584)], 8, 0, 16, -1), ([(32768, 3072)], 8, 0, 16, -1), ([(28672, 7168)], 4, 0, 16, -1),
+    ([(21504, 5376)], 4, 1, 16, -1), ([(8192, 28672)], 1, 1, 8, -1),
+    # split kernel: both sides of half a step; one choice for matrices that have room for it and one that has none
+    ([(2976, 5376)], 8, -1, 0, 0), ([(2992, 5376)], 8, -1, 0, 1), ([(2992, 5376), (40, 65024)], 8, -1, 0, 0)])
+def test_which_selector_table_a_decode_call_takes(shapes, M, main, slots, split):
+    h = [_sizes_only(K, N, (F.BLK1632_4, 4, 128, 16)) for K, N in shapes]
+    assert _lib.native().decode_choice(h, M) == (main, slots, split)
+
+
+def test_selector_table_of_one_dword_blocks_and_of_dense_layouts():
+    choice = lambda case, K: _lib.native().decode_choice([_sizes_only(K, 5376, case)], 8)[2]
+    assert [choice((F.BLKC, 2, 64, keep), 1024) for keep in (10, 16, 23)] == [0, 1, 0]
+    assert choice((F.BLKC, 2, 64, 10), 8192) == 1 and choice((F.DENSEB, 2, 64, None), 8192) == 0
 
 
 def test_ops_refuse_to_run_without_gpu_tensors():
