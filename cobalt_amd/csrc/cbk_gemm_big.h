@@ -2,7 +2,7 @@
 // few hundred rows and small matrices: cbk_gemm_skinny.h, which has a decoder for 8-bit codes too.)
 //
 // Workgroup tile 256 tokens x 256 weight rows, 64 input columns per stage, four wavefronts
-// each owning a 128 x 128 sub-tile (4 x 4 blocks of v_mfma_f32_32x32x16_f16, 256 accumulator
+// each owning a 128 x 128 sub-tile (8 x 8 blocks of v_mfma_f32_16x16x32_f16, 256 accumulator
 // registers), one wavefront per SIMD.  Both operands are double-buffered in LDS (64 KB of
 // activations, 72 KB of weights): while the matrix cores work on stage s, the same wavefronts
 // dequantise the weights of stage s + 1 into the other buffer, and the activation tile is
@@ -24,18 +24,20 @@
 // and the dense layouts) and for BLK1632_6, zero points <= 128, this is the byte-permute decoder
 // of the decode kernel (selector table in LDS) followed by two packed-half operations per column
 // pair; the remaining layouts (8-bit codes, larger zero points) go through the generic
-// 32-column reader.  One wavefront per SIMD issues a vector instruction every five to seven
-// cycles beside its matrix instructions, whatever its kind, so the decode is counted in
-// instructions: an entry's address is one four-byte dot product of the mask dword, codes stay
-// unsigned until the exact subtraction of 1024 + zero point, and a pruned column reads the zero
-// point from the place of the eighth survivor, which only a full byte asks for.  4-bit, 16 of 32:
-// 932 -> 764 vector instructions per 256 of the matrix cores (1028 -> 764 with two or three
-// column-scale vectors, whose activation base had stayed in vector registers).  Gated block of
-// 21504 x 5376 at 2048 tokens 1457 -> 1436 us.  More would have to come out of the energy of the
-// matrix instructions and of LDS: the clock falls with the load (N = 5376, 256 tokens: one tile on
-// every eighth CU takes 126 us, one on every CU 163, both 296 thousand cycles of a wavefront's life),
-// spreading the copies over the stage changes nothing, a second copy of each activation line
-// costs 12 %.
+// 32-column reader.  One wavefront per SIMD issues an instruction every five cycles, later if it waits
+// for the one before, and two fit beside a matrix instruction of 16 cycles.  So the decode is counted in
+// instructions (an entry's address is one four-byte dot product of the mask dword, the entry holds what
+// would be counted or compared, codes stay unsigned until the exact subtraction of 1024 + zero point, a
+// pruned column reads the zero point from the place of the eighth survivor) and dealt out by hand, at most
+// two independent ones beside each matrix instruction: 4-bit, 16 of 32: 1.4 per matrix instruction.
+//
+// What bounds it: power.  The clock falls with the load: a loop of nothing but these matrix instructions on
+// halves, half of one operand zeros, runs at 2.08 PFLOP/s, of v_mfma_f32_32x32x16_f16 (a fourth of the sums moved per
+// product, but twice as often) at 1.85 at the same operands: hence the 16 x 16 x 32 form here.  N = 5376, 2048 tokens,
+// 8192 rows (one tile on every CU), 4-bit, 16 of 32, one box: 181 us with 32 x 32 blocks and the decode left to the
+// compiler's interleave, 169 now, 141 with the decode taken out, 119 with the matrix instructions alone (266, 196 and 183
+// thousand cycles of the loop at about 1.6 GHz).  Gated block of 21504 x 5376 at 2048 tokens with both its products
+// 1421 -> 1346 us.
 //
 // Workgroups are ordered so that those running at the same time on one XCD (blockIdx % 8)
 // share their token tile, which then stays in that XCD's L2.
@@ -44,6 +46,7 @@
 #pragma once
 #include <atomic>
 #include <type_traits>
+#include <utility>
 #include "cbk_decode.h"
 
 namespace cbk {
@@ -51,14 +54,14 @@ namespace cbk {
 constexpr int GB_T = 256;       // tokens per workgroup tile (TI = 4); the TI = 1 kernels take 64
 constexpr int GB_R = 256;       // weight rows per workgroup tile
 constexpr int GB_K = 64;        // input columns per stage
-constexpr int GB_P = GB_K + 8;  // LDS row pitch of the weight tile in halfs (144 B): conflict-free 16-byte reads
-constexpr int GB_LUT = 256 * 8 * 8;   // selector table, 8 lane-private copies of 256 x 8 B
-// one activation stage in LDS: 64 TI rows x 128 B, unpadded, swizzled
+constexpr int GB_LUT = 256 * 8 * 16;  // selector table, 8 lane-private copies of 256 x 16 B
+// one stage of either operand in LDS: rows of 128 B, unpadded, swizzled
 constexpr int gb_xbuf(int ti) { return 64 * ti * GB_K * 2; }
-constexpr size_t gb_lds(int ti) { return (size_t)2 * gb_xbuf(ti) + (size_t)2 * GB_R * GB_P * 2 + GB_LUT; }
+constexpr int GB_WBUF = GB_R * GB_K * 2;
+constexpr size_t gb_lds(int ti) { return (size_t)2 * gb_xbuf(ti) + (size_t)2 * GB_WBUF + GB_LUT; }
 
 typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
-typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 
 struct GbArgs {
   DMat m;
@@ -92,70 +95,74 @@ struct GbArgs {
 };
 
 // One wavefront-wide copy of 64 x 16 bytes from global memory straight into LDS (no VGPRs, no
-// ds_write): lane l reads base + voff and its 16 bytes land at LDS byte lds + 16 * l.  The
+// ds_write): lane l reads base + soff + voff and its 16 bytes land at LDS byte lds + AT + 16 * l.  The
 // compiler does not know that this instruction counts on vmcnt or that it writes LDS; the
 // kernel waits for it by hand before the barrier that publishes the stage.
-__device__ inline void dma_x16(const void* base, uint32_t voff, uint32_t lds) {
-  // base and lds are the same in every lane; say so, or they may arrive in vector registers
-  const uint64_t b64 = (uint64_t)base;
-  const uint64_t sbase = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b64) |
-                         ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b64 >> 32)) << 32);
-  lds = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds) : "memory", "m0");
+template <int AT>
+__device__ inline void dma_x16(v4u buffer, uint32_t voff, uint32_t soff, uint32_t lds) {
+  asm volatile("s_add_u32 m0, %3, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(buffer), "s"(soff), "s"(lds), "i"(AT) : "memory", "m0", "scc");
 }
+// the same in every lane, in a scalar register
+__device__ inline uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 
-// eight codes (the zero point z for a pruned column) -> eight halfs (q - z) * scale; off2 = -(1024 + z) twice.
-// A code in the low byte of 0x64xx is the half 1024 + q; the difference is exact, the product rounds once.
-__device__ inline uint4 bytes_to_halfs(uint32_t b0, uint32_t b1, h2_t off2, h2_t s2) {
-  const uint32_t k = 0x64646464u;
-  uint32_t w[4] = {__builtin_amdgcn_perm(k, b0, 0x04010400u), __builtin_amdgcn_perm(k, b0, 0x04030402u),
-                   __builtin_amdgcn_perm(k, b1, 0x04010400u), __builtin_amdgcn_perm(k, b1, 0x04030402u)};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    h2_t v = __builtin_bit_cast(h2_t, w[i]);
-    v = (v + off2) * s2;
-    w[i] = __builtin_bit_cast(uint32_t, v);
-  }
-  return make_uint4(w[0], w[1], w[2], w[3]);
+// f(integral_constant 0), f(1), ... f(N - 1)
+template <typename F, int... I>
+__device__ inline void static_for_seq(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, typename F>
+__device__ inline void static_for(F&& f) { static_for_seq(f, std::make_integer_sequence<int, N>{}); }
+
+// d += w . x^T of 16 weight rows, 16 tokens and 32 columns.  Written as the instruction, with the sum in place in
+// accumulation registers: the compiler's own choice of a destination beside the addend left 912 register copies in
+// a trip of the loop (the gated block of the header 1395 -> 1663 us).  What reads the sums waits (gb_mfma_done).
+__device__ inline void gb_mfma(v4f& d, const v8h& w, const v8h& x) {
+  asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(d) : "v"(w), "v"(x));
 }
+__device__ inline void gb_mfma_done() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
 
 // One wavefront's 128 x 128 accumulators -> y, 32 tokens at a time through LDS.  D[i][j] holds, in
-// lane l and register r, token 8*(r/4) + 4*(l/32) + r%4 and weight row l%32 of its 32 x 32 block;
-// turning the tile around in LDS makes the global stores whole 16-byte pieces of consecutive
-// output columns: 256 B (f16) or 512 B (f32) per token.  Compile-time indexed and branch-free
-// per element: the 256 accumulators make this straight-line code, and it has to stay small.
+// lane l and register r, token l%16 and weight row 4*(l/16) + r of its 16 x 16 block: four consecutive
+// output columns, one LDS store.  Turning the tile around in LDS makes the global stores whole 16-byte
+// pieces of consecutive output columns: 256 B (f16) or 512 B (f32) per token.  Compile-time indexed and
+// branch-free per element: the 256 accumulators make this straight-line code, and it has to stay small.
 template <int YDT, int kstep, int TI>                            // local row i is output column row0 + kstep * i
-__device__ inline void gb_epilogue(const GbArgs& a, v16f (&acc)[TI][4], uint8_t* smem, int lane, int wave, int tok0,
+__device__ inline void gb_epilogue(const GbArgs& a, v4f (&acc)[2 * TI][8], uint8_t* smem, int lane, int wave, int tok0,
                                    int row0, const float* rs) {   // rs: the row scales of this tile's X'
   constexpr int ESZ = YDT == CBK_F32 ? 4 : 2;
   constexpr int PITCH = 128 * ESZ + 16;                          // bytes per token row in LDS
   constexpr int EPP = 16 / ESZ, PPR = 128 / EPP;                 // elements per 16-byte piece, pieces per row
   const int K = a.m.K;
   uint8_t* ep = smem + (size_t)wave * (32 * (128 * 4 + 16));
-  uint8_t* epl = ep + 4 * (lane >> 5) * PITCH + (lane & 31) * ESZ;
-  float bv[4];
+  uint8_t* epl = ep + (lane & 15) * PITCH + 4 * (lane >> 4) * ESZ;
+  float bv[8][4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int k = row0 + kstep * (32 * j + (lane & 31));
-    bv[j] = 0.f;
-    if (a.bias && k < K) bv[j] = load_act<YDT>(a.bias, k);
-  }
+  for (int j = 0; j < 8; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int k = row0 + kstep * (16 * j + 4 * (lane >> 4) + r);
+      bv[j][r] = 0.f;
+      if (a.bias && k < K) bv[j][r] = load_act<YDT>(a.bias, k);
+    }
   const bool vec_ok = ((a.ldy * ESZ) & 15) == 0 && (((uintptr_t)a.y) & 15) == 0;
 #pragma unroll
   for (int i = 0; i < TI; ++i) {
-    float ts[16];                                                  // token of register r: see above
 #pragma unroll
-    for (int r = 0; r < 16; ++r) ts[r] = rs[tok0 + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)];
+    for (int h = 0; h < 2; ++h) {
+      const float ts = rs[tok0 + 32 * i + 16 * h + (lane & 15)];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < 8; ++j) {
+        float v[4];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float v = acc[i][j][r] * ts[r] + bv[j];
-        uint8_t* d = epl + (8 * (r >> 2) + (r & 3)) * PITCH + 32 * j * ESZ;
-        if (YDT == CBK_F32) *(float*)d = v;
-        else if (YDT == CBK_F16) *(uint16_t*)d = f2h(v);
-        else *(__bf16*)d = (__bf16)v;                              // v_cvt_pk_bf16_f32: round to nearest even
+        for (int r = 0; r < 4; ++r) v[r] = acc[2 * i + h][j][r] * ts + bv[j][r];
+        uint8_t* d = epl + 16 * h * PITCH + 16 * j * ESZ;
+        if (YDT == CBK_F32) *(float4*)d = make_float4(v[0], v[1], v[2], v[3]);
+        else if (YDT == CBK_F16) *(uint2*)d = make_uint2((uint32_t)f2h(v[0]) | ((uint32_t)f2h(v[1]) << 16), (uint32_t)f2h(v[2]) | ((uint32_t)f2h(v[3]) << 16));
+        else {                                                     // v_cvt_pk_bf16_f32: round to nearest even
+          typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+          const b2 lo = {(__bf16)v[0], (__bf16)v[1]}, hi = {(__bf16)v[2], (__bf16)v[3]};
+          *(uint2*)d = make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
+        }
       }
+    }
 #pragma unroll
     for (int t = 0; t < 32 * PPR / 64; ++t) {
       const int pc = t * 64 + lane;
@@ -186,16 +193,21 @@ __device__ inline void gb_epilogue(const GbArgs& a, v16f (&acc)[TI][4], uint8_t*
 // the weight decode: a quarter of the matrix instructions per stage, the same decode.
 template <int BITS, int KEEP, int GRP, int PAR, int TI = 4>
 __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
+  // All 256 registers of a wavefront (LDS holds one workgroup per CU either way), so that the shift amounts of the decode
+  // are not in the last one (build.py, shift_hazards, which found two 64-token kernels with theirs in v127 of 128).
+  asm volatile("" ::: "v255");
   constexpr int GB_XBUF = gb_xbuf(TI);
   constexpr bool FASTD = BITS != 0;
   using C = CodeCfg<FASTD ? BITS : 4, KEEP, FASTD ? GRP : 128>;
   constexpr bool BITMAP = FASTD && !C::DENSE;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  // Xs [2][GB_T][64 halfs]: row r, logical 16-byte piece c at physical piece c ^ ((r >> 1) & 7)
-  // (conflict-free 16-byte fragment reads without padding, which the direct copies cannot make)
+  // Xs [2][GB_T][64 halfs], Ws [2][GB_R][64 halfs]: row r, logical 16-byte piece c at physical piece c ^ ((r >> 1) & 7).
+  // A 16-byte read or write goes through LDS in sets of sixteen lanes, 0-3 12-15 20-27 and so on: with the fragments' rows
+  // (l % 16) and pieces (l / 16) as with one piece of 64 rows, a set's pieces so lie in different banks.  (Rows padded to
+  // 144 bytes, which serve fragments of 32 rows and one piece, triple the conflicts of the call: 14 -> 43 million cycles.)
   _Float16* Xs = (_Float16*)smem;
-  _Float16* Ws = (_Float16*)(smem + 2 * GB_XBUF);                 // [2][GB_R][GB_P]
-  uint2* lut = (uint2*)(Ws + 2 * GB_R * GB_P);                    // [256][8]
+  uint8_t* Ws = smem + 2 * GB_XBUF;
+  uint4* lut = (uint4*)(Ws + 2 * GB_WBUF);                        // [256][8]
   const DMat& m = a.m;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wt = wave >> 1, wr = wave & 1;
@@ -220,20 +232,23 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
   const int nch = N >> 7;                                         // 128-column chunks of the weight rows
 
   if (BITMAP) {
-    const uint2 e = make_selectors<0x07070707u>((uint32_t)tid, C::SEL_KIND);   // a pruned column reads rank 7's byte
+    // an entry: the two selectors (a pruned column reads rank 7's byte); which bits of the upper pool are the codes' (rank 7's
+    // byte only if all eight columns are kept); the bits its survivors take in the code stream
+    const uint2 e = make_selectors<0x07070707u>((uint32_t)tid, C::SEL_KIND);
+    const uint32_t full = C::HI2 ? 0x00FFFFFFu : C::SB == 4 ? 0x000F0F0Fu : 0x00030303u;
+    const uint4 v = make_uint4(e.x, e.y, tid == 255 ? full | 0xFF000000u : full, (uint32_t)__builtin_popcount(tid) * C::SB);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) lut[table_slot<8, 8>(tid, j)] = e;
+    for (int j = 0; j < 8; ++j) lut[table_slot<8, 16>(tid, j)] = v;
   }
-  const uint32_t lut_lane = (uint32_t)(uintptr_t)lut + 8 * (lane & 7);       // LDS address of this lane's copy of entry 0
-  const uint32_t lut_full = (uint32_t)(uintptr_t)lut + 255 * 64;             // and of the first copy of entry 255
+  const uint32_t lut_lane = (uint32_t)(uintptr_t)lut + 16 * (lane & 7);      // LDS address of this lane's copy of entry 0
 
-  v16f acc[TI][4];
+  v4f acc[2 * TI][8];                                             // 16 tokens x 16 weight rows each
 #pragma unroll
-  for (int i = 0; i < TI; ++i)
+  for (int i = 0; i < 2 * TI; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 8; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+      for (int e = 0; e < 4; ++e) acc[i][j][e] = 0.f;
 
   // this thread's weight row
   const int wrow = r0 + kstep * tid;
@@ -249,23 +264,25 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
   const uint32_t xvo_e = (uint32_t)((lane >> 3) * Npad * 2 + (((lane & 7) ^ (lane >> 4)) * 16));
   const uint32_t xvo_o = (uint32_t)((lane >> 3) * Npad * 2 + (((lane & 7) ^ (4 + (lane >> 4))) * 16));
   const int xv = PAR == 1 ? pp : PAR >= 2 ? (r0 >= a.vs0 ? 1 : 0) + (r0 >= a.vs1 ? 1 : 0) : 0;   // which col_scale vector
-  const uint8_t* xsb = (const uint8_t*)(a.xp + (size_t)xv * a.xps + (size_t)(t0 + 16 * TI * wv) * Npad + (size_t)s_begin * GB_K);
-  // the same in every lane: kept in scalar registers from here on, or each copy below reads it out of vector registers
-  xsb = (const uint8_t*)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uint64_t)xsb) |
-                         ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)xsb >> 32)) << 32));
-  const uint32_t xlds0 = (uint32_t)(uintptr_t)Xs + (uint32_t)wv * (2048u * TI);
-  auto dma_x = [&](int s, int buf) {                              // stage s -> Xs[buf]
-    const uint8_t* sb = xsb + (size_t)s * (GB_K * 2);
-    const uint32_t ld = xlds0 + (uint32_t)buf * GB_XBUF;
-#pragma unroll
-    for (int q = 0; q < 2 * TI; ++q)
-      dma_x16(sb + (size_t)q * 8 * Npad * 2, (q & 1) ? xvo_o : xvo_e, ld + q * 1024);
+  const uint64_t xsb = (uint64_t)(a.xp + (size_t)xv * a.xps + (size_t)(t0 + 16 * TI * wv) * Npad + (size_t)s_begin * GB_K);
+  const uint64_t xsu = (uint64_t)uniform((uint32_t)xsb) | ((uint64_t)uniform((uint32_t)(xsb >> 32)) << 32);
+  const uint32_t xlds0 = uniform((uint32_t)(uintptr_t)Xs + (uint32_t)wv * (2048u * TI)), xrow8 = uniform(16u * Npad);
+  v4u xbuf;                                                       // the stage that is being copied, as a buffer
+  auto dma_stage = [&](int s) {
+    const uint64_t b = xsu + (uint64_t)(uint32_t)((s < nst ? s : nst - 1) * (GB_K * 2));
+    xbuf = v4u{uniform((uint32_t)b), uniform((uint32_t)(b >> 32)), 0xFFFFFFFFu, 0x00027000u};
   };
-  // fragment reads: this lane's row inside a 32-row block and its four swizzled piece offsets
-  const uint32_t xsw = ((lane & 31) >> 1) & 7;
-  uint32_t xpc[4];
+  auto dma_x = [&](auto buf_, auto q_) {                          // copy q of that stage -> Xs[buf]
+    constexpr int q = decltype(q_)::value;
+    dma_x16<decltype(buf_)::value * GB_XBUF + q * 1024>(xbuf, (q & 1) ? xvo_o : xvo_e, q * xrow8, xlds0);
+  };
+  // fragment reads: this lane's row inside a 16-row block of either operand and its two swizzled piece offsets
+  uint32_t xpc[2], wpc[2];
 #pragma unroll
-  for (int kk = 0; kk < 4; ++kk) xpc[kk] = (((2 * kk + (lane >> 5)) ^ xsw) * 16);
+  for (int kk = 0; kk < 2; ++kk) {
+    xpc[kk] = ((4 * kk + (lane >> 4)) ^ ((lane & 15) >> 1)) * 16;
+    wpc[kk] = ((4 * kk + (lane >> 4)) ^ (lane & 7)) * 16;
+  }
 
   // one 128-column chunk of this thread's weight row: two stages' worth
   struct WChunk {
@@ -308,21 +325,25 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
     }
   };
 
-  // selectors of mask byte b8 (0..7) of half h of a chunk (bitmap layouts only)
-  struct Sel { uint32_t x, y; bool full; };                         // full: all eight columns kept
-  auto fetch_sel = [&](const WChunk& w, int h, int b8) -> Sel {
-    if (!BITMAP) return Sel{0, 0, false};
-    const int jb = 8 * h + b8;                                     // mask byte of the chunk, 0..15
-    // byte jb % 4 of the mask dword, times 64 bytes per entry, plus the base
-    const uint32_t at = __builtin_amdgcn_udot4(w.m[jb >> 2], 64u << (8 * (jb & 3)), lut_lane, false);
-    const v2u e = *(const __attribute__((address_space(3))) v2u*)(uintptr_t)at;
-    return Sel{e[0], e[1], at >= lut_full};
-  };
-  // decode mask byte b8 (8 columns) of stage s = half h of chunk w into Ws[buf]
-  auto store_w_byte = [&](int s, WChunk& w, int h, int buf, int b8, Sel sel) {
-    _Float16* dst = Ws + (size_t)buf * GB_R * GB_P + tid * GB_P + b8 * 8;
+  // Decode of mask byte b8 (8 columns) of a stage = half h of chunk w into Ws[buf], in PIECES pieces of at most two vector
+  // instructions that do not depend on each other, one piece beside each matrix instruction of a 256-token tile: with one
+  // wavefront on a SIMD an instruction that waits for the one before it takes eight cycles and more, and of the rest two fit
+  // beside a 16-cycle matrix instruction.  Pieces 0 and 1 fetch the table entry of the byte two ahead (half ha of chunk wa).
+  constexpr int PIECES = 16;
+  constexpr bool CHAIN = C::NW <= 2 && !C::HI2;                     // the stream is shifted on from byte to byte
+  struct Sel { uint32_t x, y, full, bits; };
+  Sel sel[4];                                                       // by byte mod 4
+  uint32_t sel_at = 0;
+  struct Dec { uint32_t win, rank, p0, p1, t, b0, b1, o[4]; } de;
+  uint32_t wdst[8];                                                 // 16-byte pieces of this thread's row in Ws[0]
+#pragma unroll
+  for (int c = 0; c < 8; ++c) wdst[c] = (uint32_t)(uintptr_t)Ws + (uint32_t)tid * 128u + (((uint32_t)tid & 7u) ^ c) * 16u;
+  auto decode_piece = [&](int s, WChunk& w, int h, int buf, int b8, int piece, const WChunk& wa, int ha) {
+    auto put = [&](int c, uint32_t x, uint32_t y, uint32_t z, uint32_t v) {
+      *(__attribute__((address_space(3))) v4u*)(uintptr_t)(wdst[c] + (uint32_t)buf * GB_WBUF) = v4u{x, y, z, v};
+    };
     if (!FASTD) {
-      if (b8 & 3) return;                                         // the generic reader works on 32 columns
+      if ((b8 & 3) || piece) return;                              // the generic reader works on 32 columns
       uint32_t packed[16];
       if (wok) {
         int q[32];
@@ -345,172 +366,203 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
       }
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        ((uint4*)dst)[e] = make_uint4(packed[4 * e], packed[4 * e + 1], packed[4 * e + 2], packed[4 * e + 3]);
+        put(b8 + e, packed[4 * e], packed[4 * e + 1], packed[4 * e + 2], packed[4 * e + 3]);
       return;
     }
-    if (h == 0 && b8 == 0) align_chunk_codes<C>(w.raw, w.ci, w.c);  // once per chunk, at its first use
     const int blk = 2 * h + (b8 >> 2);                              // 32-column block of the chunk
     const int jj = b8 & 3;                                          // mask byte inside the block
-    if (jj == 0) block_stream<C, BITS>(w.c, blk, st);               // once per block
     const int gi = C::NGC == 2 ? h : 0;                             // quantisation group of this stage
     const _Float16 sh = (_Float16)(wok ? w.s[gi] : 0.f);
     const h2_t s2 = {sh, sh};
     const uint32_t z = (w.z >> (8 * gi)) & 0xFFu;
+    // eight codes (the zero point z for a pruned column) -> eight halfs (q - z) * scale: a code in the low byte of
+    // 0x64xx is the half 1024 + q; the difference to 1024 + z is exact, the product rounds once
     const h2_t off2 = __builtin_bit_cast(h2_t, 0xE400E400u + z * 0x00010001u);
-    uint32_t p0, p1, b0, b1;
-    if (BITMAP) {
-      const uint32_t mw = w.m[blk];
-      const uint32_t r = jj == 0 ? 0u : (uint32_t)__builtin_popcount(mw & ((1u << (8 * jj)) - 1u));
-      const uint32_t cwin = jj == 0 ? st[0] : window<C::NW>(st, r * C::SB);
+    if (piece == 0) {
+      if (h == 0 && b8 == 0) align_chunk_codes<C>(w.raw, w.ci, w.c);  // once per chunk, at its first use
+      if (jj == 0) block_stream<C, BITS>(w.c, blk, st);               // once per block
+      if (BITMAP) {
+        const int ja = 8 * ha + ((b8 + 2) & 7);                       // mask byte of the chunk, 0..15
+        // byte ja % 4 of the mask dword, times 128 bytes per entry, plus the base
+        sel_at = __builtin_amdgcn_udot4(wa.m[ja >> 2], 128u << (8 * (ja & 3)), lut_lane, false);
+      }
+    } else if (piece == 1) {
+      if (BITMAP) {
+        const v4u e = *(const __attribute__((address_space(3))) v4u*)(uintptr_t)sel_at;
+        sel[(b8 + 2) & 3] = Sel{e[0], e[1], e[2], e[3]};
+      }
+    } else if (piece == 2) {
+      if (BITMAP) {                                                   // past the survivors of the byte before
+        const uint32_t n = sel[(b8 - 1) & 3].bits;
+        if (!CHAIN) de.rank = jj == 0 ? 0u : jj == 1 ? n : de.rank + n;
+        else if (jj && C::NW == 1) st[0] >>= n;
+        else if (jj) {
+          const uint64_t v = (((uint64_t)st[C::NW - 1] << 32) | st[0]) >> n;
+          st[0] = (uint32_t)v; st[C::NW - 1] = (uint32_t)(v >> 32);
+        }
+      }
+    } else if (piece == 3) {
+      if (BITMAP) de.win = CHAIN || jj == 0 ? st[0] : window<C::NW>(st, de.rank);
+      else de.win = C::SB == 4 ? st[jj] : (st[jj >> 1] >> (16 * (jj & 1)));
+    } else if (piece == 4) {
+      if (C::SB == 2) { const uint32_t lo16 = de.win & 0xFFFFu; de.win = (lo16 << 14) | lo16; }   // bytes c0 c4 c1 c5; four bits up c2 c6 c3 c7
+    } else if (piece == 5) {
+      de.p0 = de.win & (C::SB == 4 ? 0x0F0F0F0Fu : 0x03030303u);      // even codes (of two bits: c0 c4 c1 c5)
+      de.t = de.win >> 4;
+    } else if (piece == 6) {
       // p0 | p1: the codes of the survivors from this byte's first on, even and odd ranks (four bits), or 0 2 .. and 4 6 ..
       // Rank 7, the top byte of p1, is asked for only if all eight columns are kept: otherwise the zero point takes its
-      // place, which is what a pruned column reads (bits above a code in that byte are zeros already).
-      const uint32_t zt = z << 24;
+      // place, which is what a pruned column reads.
       if (C::HI2) {
         uint32_t h0, h1;
-        hi2_pools(w.h2[C::HI2 ? blk : 0], r, h0, h1);
-        p0 = (cwin & 0x0F0F0F0Fu) | h0;
-        const uint32_t of = sel.full ? 0xFFFFFFFFu : 0x00FFFFFFu;
-        p1 = ((((cwin >> 4) & 0x0F0F0F0Fu) | h1) & of) | (zt & ~of);
-      } else if (C::SB == 4) {
-        p0 = cwin & 0x0F0F0F0Fu;
-        const uint32_t of = sel.full ? 0xFF0F0F0Fu : 0x000F0F0Fu;
-        p1 = ((cwin >> 4) & of) | (zt & ~of);
-      } else {
-        const uint32_t lo16 = cwin & 0xFFFFu;
-        const uint32_t t2 = (lo16 << 14) | lo16;
-        p0 = t2 & 0x03030303u;
-        const uint32_t of = sel.full ? 0xFF030303u : 0x00030303u;
-        p1 = ((t2 >> 4) & of) | (zt & ~of);
+        hi2_pools(w.h2[C::HI2 ? blk : 0], de.rank >> 2, h0, h1);
+        de.p0 |= h0;
+        de.t = (de.t & 0x0F0F0F0Fu) | h1;
       }
-      b0 = perm(p1, p0, sel.x);
-      b1 = perm(p1, p0, sel.y);
-    } else if (C::SB == 4) {                                       // dense 4-bit, or 3-bit widened to nibbles
-      const uint32_t cwin = st[jj];
-      p0 = cwin & 0x0F0F0F0Fu;                                     // even columns
-      p1 = (cwin >> 4) & 0x0F0F0F0Fu;                              // odd columns
-      b0 = perm(p1, p0, 0x05010400u);
-      b1 = perm(p1, p0, 0x07030602u);
-    } else {                                                       // dense 2-bit: 16 codes per dword
-      const uint32_t lo16 = (st[jj >> 1] >> (16 * (jj & 1))) & 0xFFFFu;
-      const uint32_t t2 = (lo16 << 14) | lo16;
-      p0 = t2 & 0x03030303u;                                       // c0 c4 c1 c5
-      p1 = (t2 >> 4) & 0x03030303u;                                // c2 c6 c3 c7
-      b0 = perm(p1, p0, 0x06040200u);
-      b1 = perm(p1, p0, 0x07050301u);
+    } else if (piece == 7) {
+      if (BITMAP) de.p1 = (de.t & sel[b8 & 3].full) | ((z << 24) & ~sel[b8 & 3].full);
+      else de.p1 = de.t & (C::SB == 4 ? 0x0F0F0F0Fu : 0x03030303u);
+    } else if (piece == 8) {
+      de.b0 = perm(de.p1, de.p0, BITMAP ? sel[b8 & 3].x : C::SB == 4 ? 0x05010400u : 0x06040200u);
+      de.b1 = perm(de.p1, de.p0, BITMAP ? sel[b8 & 3].y : C::SB == 4 ? 0x07030602u : 0x07050301u);
+    } else if (piece < 15) {
+      const int i = piece < 11 ? 2 * (piece - 9) : 2 * ((piece - 11) & 1);
+#pragma unroll
+      for (int e = i; e < i + 2; ++e) {
+        if (piece < 11) de.o[e] = __builtin_amdgcn_perm(0x64646464u, e < 2 ? de.b0 : de.b1, e & 1 ? 0x04030402u : 0x04010400u);
+        else {
+          const h2_t v = __builtin_bit_cast(h2_t, de.o[e]);
+          de.o[e] = __builtin_bit_cast(uint32_t, piece < 13 ? v + off2 : v * s2);
+        }
+      }
+    } else {
+      put(b8, de.o[0], de.o[1], de.o[2], de.o[3]);
     }
-    *(uint4*)dst = bytes_to_halfs(b0, b1, off2, s2);
   };
 
-  // fragment registers, two sets; set 0 of the next stage is loaded at the end of the current one
-  v8h af[2][TI], bf[2][4];
-  auto read_frags = [&](int buf, int kk, int set) {
-    const uint8_t* xb = (const uint8_t*)Xs + (size_t)buf * GB_XBUF + (32 * TI * wt + (lane & 31)) * 128;
-    const _Float16* wb = Ws + (size_t)buf * GB_R * GB_P + (128 * wr + (lane & 31)) * GB_P + 8 * (lane >> 5);
-#pragma unroll
-    for (int i = 0; i < TI; ++i) af[set][i] = *(const v8h*)(xb + 4096 * i + xpc[kk]);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) bf[set][j] = *(const v8h*)(wb + 32 * j * GB_P + 16 * kk);
+  // Fragment registers: the two halves of the tile's token blocks and of its row blocks, 32 columns each.  The 64-token tile
+  // has registers for both 32-column steps of a stage (DEEP): a phase of its four matrix instructions is shorter than the
+  // LDS latency (4096 x 14336, 2-bit dense, 64 rows: 216 us with the half that the next phase needs read one phase ahead as in
+  // the larger tiles, 189 so; the 128-token tile gains nothing by it).
+  constexpr bool DEEP = TI == 1;
+  constexpr int BP = DEEP ? 4 : 6;                                // the phase that begins with the barrier
+  v8h af[DEEP ? 2 : 1][2][TI], bf[DEEP ? 2 : 1][2][4];
+  auto read_x = [&](int buf, int kk, int h, int i) {
+    const uint8_t* xb = (const uint8_t*)Xs + (size_t)buf * GB_XBUF + (32 * TI * wt + 16 * TI * h + (lane & 15)) * 128;
+    af[DEEP ? kk : 0][h][i] = *(const v8h*)(xb + 2048 * i + xpc[kk]);
   };
+  auto read_w = [&](int buf, int kk, int h, int j) {
+    const uint8_t* wb = Ws + (size_t)buf * GB_WBUF + (128 * wr + 64 * h + (lane & 15)) * 128;
+    bf[DEEP ? kk : 0][h][j] = *(const v8h*)(wb + 2048 * j + wpc[kk]);
+  };
+  auto read_all = [&](int buf, int kk) {
+    static_for<2 * TI>([&](auto i_) { constexpr int i = decltype(i_)::value; read_x(buf, kk, i / TI, i % TI); });
+    static_for<8>([&](auto j_) { constexpr int j = decltype(j_)::value; read_w(buf, kk, j / 4, j % 4); });
+  };
+
+  // Decode of a stage: mask byte d / PIECES, piece d % PIECES; the first DEC0 pieces run behind the barrier of the stage
+  // before the one that precedes it.
+  constexpr int MF = 32 * TI, DEC0 = PIECES * (8 - BP);            // MFMAs of a stage
+  // The copies of a stage start there too, one every DMAX MFMAs: a wavefront that issues the next before the last one's
+  // 1 KB has passed waits for it (all eight behind the barrier: 1840 -> 2000 thousand cycles for the call)
+  constexpr int DMAX = 12, DMA0 = (4 * TI * (8 - BP) - 3) / DMAX + 1;
+  auto decode_step = [&](int s, auto d_, WChunk& wd, auto hd_tag, const WChunk& wn, auto hn_tag, int buf) {
+    constexpr int d = decltype(d_)::value, b8 = d / PIECES, HD = decltype(hd_tag)::value, HN = decltype(hn_tag)::value;
+    decode_piece(s, wd, HD, buf, b8, d % PIECES, b8 < 6 ? wd : wn, b8 < 6 ? HD : HN);
+  };
+  using T = std::true_type; using Fl = std::false_type;
+  using H0 = std::integral_constant<int, 0>; using H1 = std::integral_constant<int, 1>;
 
   // ---- prologue: chunk 0 into registers and stage 0 into buffer 0; then, in the order every
-  // stage leaves them, the copies of stage 1 and the loads of chunk 1
-  dma_x(0, 0);
+  // stage leaves them, the copies of stage 1, the loads of chunk 1 and the first pieces of stage 1
+  dma_stage(0);
+  static_for<2 * TI>([&](auto q_) { dma_x(std::integral_constant<int, 0>{}, q_); });
   load_chunk(0, wA);
+  load_chunk(1, wB);
   __syncthreads();                                                // selector table visible
-#pragma unroll
-  for (int b8 = 0; b8 < 8; ++b8) store_w_byte(0, wA, 0, 0, b8, fetch_sel(wA, 0, b8));
+  if (FASTD) {                                                    // selectors of bytes 0 and 1: as bytes 6 and 7 before them leave them
+    decode_piece(0, wA, 0, 0, 6, 0, wA, 0); decode_piece(0, wA, 0, 0, 6, 1, wA, 0);
+    decode_piece(0, wA, 0, 0, 7, 0, wA, 0); decode_piece(0, wA, 0, 0, 7, 1, wA, 0);
+  }
+  static_for<8 * PIECES>([&](auto d_) { decode_step(0, d_, wA, H0{}, wA, H1{}, 0); });
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  read_frags(0, 0, 0);
-  dma_x(nst > 1 ? 1 : 0, 1);
-  load_chunk(1, wB);
-  Sel selc[3];                                                    // selectors of the mask bytes decoded next
+  if constexpr (DEEP) read_all(0, 0);
+  else {
 #pragma unroll
-  for (int i = 0; i < 3; ++i) selc[i] = fetch_sel(wA, 1, i);
+    for (int i = 0; i < TI; ++i) read_x(0, 0, 0, i);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) read_w(0, 0, 0, j);
+  }
+  dma_stage(1);
+  static_for<DMA0>([&](auto q_) { dma_x(std::integral_constant<int, 1>{}, q_); });
+  static_for<DEC0>([&](auto d_) { decode_step(1, d_, wA, H1{}, wB, H0{}, 1); });
 
-  // One stage = four phases of 16 MFMAs on buffer s % 2.  Phases 0-2 also decode the weights of
-  // stage s + 1 (half HD of chunk wd; mask bytes 0-2, 3-5, 6-7) into the other buffer between
-  // their MFMAs, fetching the selectors of the following phase (at the end: of bytes 0-2 of half
-  // HN of chunk wn) a phase early.  Phase 3 first waits for the direct copies of stage s + 1
-  // (issued a stage ago) and passes the barrier, then starts the fragment reads of stage s + 1,
-  // the direct copies of stage s + 2 and, with LOADW, the loads of weight chunk `cl`, and only
-  // then issues its 16 MFMAs from registers: the LDS latency of the next stage hides under them.
+  // One stage = eight phases of 4 TI MFMAs on buffer s % 2: for each 32 columns the four quarters (half of the
+  // token blocks) x (half of the row blocks), in an order in which every phase needs one new half, read a phase
+  // early into the registers that have just become free.  Phase BP first waits for the direct copies of stage
+  // s + 1 (issued a stage ago) and passes the barrier; nobody reads buffer s % 2 after it, so the copies of
+  // stage s + 2 start there and its weights begin to be decoded; the phases before it decode the rest
+  // of stage s + 1: the same number of vector instructions beside every MFMA.
+  // Stage s + 1 is half HD of chunk wd, stage s + 2 half HN of chunk wn; the stage behind that begins with chunk wo, half
+  // HD.  With LOADW, phase BP loads chunk `cl` into wd, which is decoded.
   // No branches inside.
-  constexpr int NB0 = 3, NB1 = 3;                                 // mask bytes decoded in phases 0 and 1
-  auto stage = [&](int s, auto loadw_tag, WChunk& wd, auto hd_tag, const WChunk& wn, auto hn_tag, WChunk& wl, int cl) {
+  auto stage = [&](int s, auto buf_, auto loadw_tag, WChunk& wd, auto hd_tag, WChunk& wn, auto hn_tag, WChunk& wo, int cl) {
     constexpr bool LOADW = decltype(loadw_tag)::value;
-    constexpr int HD = decltype(hd_tag)::value, HN = decltype(hn_tag)::value;
-    const int buf = s & 1;
-#pragma unroll
-    for (int kk = 0; kk < GB_K / 16; ++kk) {
-      const int c = kk & 1, n = c ^ 1;
-      if (kk < 3) {
-        read_frags(buf, kk + 1, n);
-        Sel seln[3];
-        if (kk == 0) {
-#pragma unroll
-          for (int i = 0; i < NB1; ++i) seln[i] = fetch_sel(wd, HD, NB0 + i);
-#pragma unroll
-          for (int i = 0; i < NB0; ++i) store_w_byte(s + 1, wd, HD, buf ^ 1, i, selc[i]);
-        } else if (kk == 1) {
-#pragma unroll
-          for (int i = 0; i < 8 - NB0 - NB1; ++i) seln[i] = fetch_sel(wd, HD, NB0 + NB1 + i);
-#pragma unroll
-          for (int i = 0; i < NB1; ++i) store_w_byte(s + 1, wd, HD, buf ^ 1, NB0 + i, selc[i]);
-        } else {
-#pragma unroll
-          for (int i = 0; i < NB0; ++i) seln[i] = fetch_sel(wn, HN, i);
-#pragma unroll
-          for (int i = 0; i < 8 - NB0 - NB1; ++i) store_w_byte(s + 1, wd, HD, buf ^ 1, NB0 + NB1 + i, selc[i]);
-        }
-#pragma unroll
-        for (int i = 0; i < 3; ++i) selc[i] = seln[i];
-      } else {
+    constexpr int BUF = decltype(buf_)::value, buf = BUF;
+    static_for<8>([&](auto p_) {
+      constexpr int p = decltype(p_)::value, kk = p >> 2, q = p & 3;
+      constexpr int hx = q >> 1, hw = (q == 1 || q == 2) ? 1 - kk : kk;
+      if constexpr (p == BP) {
         // the direct copies of stage s + 1 must have landed before the barrier publishes them
         // (the weight chunk loads of the previous stage wait here as well: they were issued a
         // whole stage ago, and counting them out of the wait would rest on how many load
         // instructions the compiler keeps)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        read_frags(buf ^ 1, 0, 0);
-        dma_x(s + 2 < nst ? s + 2 : nst - 1, buf);
-        if (LOADW) load_chunk(cl, wl);
+        if (LOADW) load_chunk(cl, wd);
       }
-#pragma unroll
-      for (int i = 0; i < TI; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[c][i], bf[c][j], acc[i][j], 0, 0, 0);
-      if (kk < 3) {
-#pragma unroll
-        for (int g = 0; g < 4 * TI; ++g) {                        // one MFMA, then a slice of the decode
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          if (kk == 2) __builtin_amdgcn_sched_group_barrier(0x002, 16 / TI, 0);
-          else __builtin_amdgcn_sched_group_barrier(0x002, 20 / TI, 0);
+      static_for<4 * TI>([&](auto t_) {
+        constexpr int t = decltype(t_)::value, i = t / 4, j = t % 4, at = 4 * TI * p + t;
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (DEEP) {
+          if constexpr (p == 0 && t == 0) read_all(buf, 1);
+          if constexpr (p == BP && t == 0) read_all(buf ^ 1, 0);
+        } else if constexpr (q == 1 || q == 2) {                    // the half that the next phase needs
+          if constexpr (t < TI) read_x(p == 6 ? buf ^ 1 : buf, p == 2 ? 1 : kk & (p != 6), q == 1, t);
+        } else if constexpr (t < 4) {
+          if constexpr (q == 0) read_w(buf, kk, 1 - kk, t);
+          else read_w(p == 7 ? buf ^ 1 : buf, p == 3, p == 3, t);
         }
-      }
+        constexpr int g = p >= BP ? at - 4 * TI * BP : at + 4 * TI * (8 - BP);      // MFMAs since the barrier
+        if constexpr (g == 0) dma_stage(s + 2);
+        if constexpr (g % DMAX == 2 && g / DMAX < 2 * TI) dma_x(std::integral_constant<int, p >= BP ? BUF : 1 - BUF>{}, std::integral_constant<int, g / DMAX>{});
+        gb_mfma(acc[TI * hx + i][4 * hw + j], bf[DEEP ? kk : 0][hw][j], af[DEEP ? kk : 0][hx][i]);
+        if constexpr (p < BP) {
+          constexpr int d0 = DEC0 + at * 8 * PIECES / MF, d1 = DEC0 + (at + 1) * 8 * PIECES / MF;
+          static_for<d1 - d0>([&](auto d_) { decode_step(s + 1, std::integral_constant<int, d0 + decltype(d_)::value>{}, wd, hd_tag, wn, hn_tag, buf ^ 1); });
+        } else {
+          constexpr int a6 = at - 4 * TI * BP, d0 = a6 * 8 * PIECES / MF, d1 = (a6 + 1) * 8 * PIECES / MF;
+          static_for<d1 - d0>([&](auto d_) { decode_step(s + 2, std::integral_constant<int, d0 + decltype(d_)::value>{}, wn, hn_tag, wo, hd_tag, buf); });
+        }
+      });
       __builtin_amdgcn_sched_barrier(0);
-    }
+    });
   };
-  // Four stages per trip (two chunks): stage 2p decodes the upper half of chunk p and, in its
-  // last phase, loads chunk p+2 into the registers chunk p has just left; stage 2p+1 decodes the
-  // lower half of chunk p+1.  The loads so have a stage and three phases until their first use
-  // (the selectors of chunk p+2 at the end of stage 2p+2); issued a stage later, where the
-  // kernel first had them, their latency from HBM showed: 3-4 % of the run time.
-  using T = std::true_type; using Fl = std::false_type;
-  using H0 = std::integral_constant<int, 0>; using H1 = std::integral_constant<int, 1>;
+  // Four stages per trip (two chunks): stage 2p decodes the rest of the upper half of chunk p and, behind its
+  // barrier, loads chunk p+2 into the registers chunk p has just left, two stages before their first use.
   for (int s = 0; s < nst; s += 4) {
     const int p = s >> 1;
-    stage(s,     T{},  wA, H1{}, wB, H0{}, wA, p + 2);
-    stage(s + 1, Fl{}, wB, H0{}, wB, H1{}, wA, 0);
-    stage(s + 2, T{},  wB, H1{}, wA, H0{}, wB, p + 3);
-    stage(s + 3, Fl{}, wA, H0{}, wA, H1{}, wB, 0);
+    stage(s,     H0{}, T{},  wA, H1{}, wB, H0{}, wB, p + 2);
+    stage(s + 1, H1{}, Fl{}, wB, H0{}, wB, H1{}, wA, 0);
+    stage(s + 2, H0{}, T{},  wB, H1{}, wA, H0{}, wA, p + 3);
+    stage(s + 3, H1{}, Fl{}, wA, H0{}, wA, H1{}, wB, 0);
   }
   // the last stage issued copies of a stage that does not exist: let them land before the
   // epilogue reuses LDS
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
+  gb_mfma_done();
 
   const int tok0 = t0 + 32 * TI * wt, row0 = r0 + kstep * 128 * wr;
   const float* rs = a.row_scale + (size_t)xv * a.rss;
