@@ -92,6 +92,17 @@ __device__ inline float token_scale(float mx) {
   return __uint_as_float(e << 23);
 }
 
+// A 16-byte store that goes on to memory at once instead of staying in the XCD's L2 (sc1), to `base` (the same in every
+// lane) + `off`.  What a kernel leaves dirty in the L2s is written back when it ends, and the next kernel waits for
+// that: kernels whose output another one reads, mostly from other XCDs, store this way.
+__device__ inline __amdgpu_buffer_rsrc_t through_buffer(void* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(base, 0, -1, 0x00027000);
+}
+__device__ inline void store16_through(__amdgpu_buffer_rsrc_t base, uint32_t off, const uint4 v) {
+  typedef uint32_t v4 __attribute__((ext_vector_type(4)));
+  __builtin_amdgcn_raw_buffer_store_b128(v4{v.x, v.y, v.z, v.w}, base, off, 0, 16);
+}
+
 template <int DT> __device__ inline float load_act(const void* p, size_t i) {
   if (DT == CBK_F16) return h2f(((const uint16_t*)p)[i]);
   if (DT == CBK_BF16T) return bf2f(((const uint16_t*)p)[i]);

@@ -18,6 +18,11 @@ int launch_skinny_b68(const SkArgs&, int bits, int group, int ti, int blocks, hi
 // outputs are never stored.  CH: pieces of the part a thread keeps in registers between the range pass
 // and the write; 0 = any length, read twice.  (A scale per token over the whole row, found by one workgroup per
 // four tokens or by every workgroup again, and half lines: 48 rows of 14336 columns 9 us, 512 rows 31.)
+// Bound: latency at 48 rows, the write of X' at hundreds: without its stores the launch of 333 rows of 4096 columns and three
+// vectors (8.2 MB) takes 4.9 us, with them 10.4, most of it the write-back of the L2s at its end, so the stores go on to
+// memory (store16_through; non-temporal ones take 9.1, but the GEMM then reads X' 2 us slower).  The type of x and the
+// order are compiled in, no load stands behind a condition of its own, sums go over lanes in registers: 333 rows 11.8 -> 9.7 us,
+// 512 rows of 14336 columns 12.8 -> 9.0, 48 rows 5.9 -> 4.8.  Sixteen tokens per workgroup, stores of 256 bytes: 10.1, 13.6, 5.2.
 __device__ inline float skinny_scale(float mx) {                   // the power of two that brings mx into [128, 256)
   if (!(mx > 0.f)) return 1.f;
   if (!(mx <= 3.4028234663852886e38f)) return SK_INFINITE;          // (mx is no NaN: fmaxf passes those over)
@@ -25,88 +30,121 @@ __device__ inline float skinny_scale(float mx) {                   // the power 
   e = e < 1 ? 1 : e;
   return __uint_as_float((uint32_t)e << 23);
 }
-template <int CH>
-__global__ __launch_bounds__(1024) void skinny_prep_kernel(const uint16_t* x, int64_t ldx, const uint16_t* cs, int xdt,
-                                                           int M, int N, int lg, int order, int ti, uint16_t* out,
-                                                           size_t xps, uint32_t* sums, size_t xcs, float* scale, int rss) {
+// f of a lane's value and that of lane ^ 8, ^ 16, ^ 32, without a trip through LDS; f is commutative
+template <typename F>
+__device__ inline float lanes8(float v, F f) {                      // (a row of sixteen lanes turned by eight)
+  return f(v, __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0x128, 0xf, 0xf, false)));
+}
+template <typename F>
+__device__ inline float lanes16(float v, F f) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+template <typename F>
+__device__ inline float lanes32(float v, F f) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+template <int CH, int XDT, int ORDER>
+__global__ __launch_bounds__(1024) void skinny_prep_kernel(const uint16_t* x, int64_t ldx, const uint16_t* cs, int M, int N,
+                                                           int lg, int ti, uint32_t inv_nq, uint16_t* out, size_t xps,
+                                                           uint32_t* sums, size_t xcs, float* scale, int rss) {
   __shared__ float red[16][8];
   const int tid = threadIdx.x, tl = tid & 7, v = blockIdx.z, q = blockIdx.y, nq = gridDim.y;
   const int tok = blockIdx.x * 8 + tl;
   const bool ok = tok < M;
-  // groups of 1 << lg columns; nothing per lane is divided (the four divisions by the group size alone took 6 us)
+  // groups of 1 << lg columns; nothing is divided here (the part's bounds by the host's reciprocal)
   const int G = N >> lg, T8 = blockDim.x >> 3;
-  const int b8 = G * q / nq << (lg - 3), e8 = G * (q + 1) / nq << (lg - 3);
+  const int b8 = (int)__umulhi((uint32_t)(G * q), inv_nq) << (lg - 3), e8 = (int)__umulhi((uint32_t)(G * (q + 1)), inv_nq) << (lg - 3);
+  if (b8 == e8) {                                                   // (more parts than groups)
+    if (ok && tid < 8) scale[((size_t)v * nq + q) * rss + tok] = 1.f;
+    return;
+  }
   const uint16_t* xr = x + (size_t)(ok ? tok : M - 1) * ldx;
   const uint16_t* cv = cs ? cs + (size_t)v * N : nullptr;
   const uint4 one = make_uint4(0x3c003c00u, 0x3c003c00u, 0x3c003c00u, 0x3c003c00u);
-  uint4 xk[CH ? CH : 1], ck[CH ? CH : 1];
+  float a[CH ? CH : 1][8];
   float mx = 0.f;
-  auto range = [&](const uint4 xq, const uint4 cq) {
-    float a[8];
-    prep8(xq, cq, xdt, a);
+  auto range = [&](const float (&f)[8]) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(a[e]));
+    for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(f[e]));
   };
+  const int c0 = b8 + (tid >> 3);
   if (CH) {
+    uint4 xk[CH ? CH : 1], ck[CH ? CH : 1];
 #pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      const int c8 = b8 + (tid >> 3) + T8 * i;
-      xk[i] = make_uint4(0, 0, 0, 0); ck[i] = one;
-      if (c8 < e8) { xk[i] = *(const uint4*)(xr + c8 * 8); if (cv) ck[i] = *(const uint4*)(cv + c8 * 8); }
+    for (int i = 0; i < CH; ++i) {                                  // pieces past the part: its last one again
+      const int c8 = c0 + T8 * i < e8 ? c0 + T8 * i : e8 - 1;
+      xk[i] = *(const uint4*)(xr + c8 * 8);
+      ck[i] = one;
     }
+    if (cv)
 #pragma unroll
-    for (int i = 0; i < CH; ++i) range(xk[i], ck[i]);
+      for (int i = 0; i < CH; ++i) ck[i] = *(const uint4*)(cv + (c0 + T8 * i < e8 ? c0 + T8 * i : e8 - 1) * 8);
+#pragma unroll
+    for (int i = 0; i < CH; ++i) { prep8(xk[i], ck[i], XDT, a[i]); range(a[i]); }
   } else {
-    for (int c8 = b8 + (tid >> 3); c8 < e8; c8 += T8) range(*(const uint4*)(xr + c8 * 8), cv ? *(const uint4*)(cv + c8 * 8) : one);
+    for (int c8 = c0; c8 < e8; c8 += T8) {
+      prep8(*(const uint4*)(xr + c8 * 8), cv ? *(const uint4*)(cv + c8 * 8) : one, XDT, a[0]);
+      range(a[0]);
+    }
   }
-#pragma unroll
-  for (int o = 8; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+  auto larger = [](float l, float r) { return fmaxf(l, r); };
+  auto plus = [](float l, float r) { return l + r; };
+  mx = lanes32(lanes16(lanes8(mx, larger), larger), larger);
   if ((tid & 63) < 8) red[tid >> 6][tl] = mx;
   __syncthreads();
+  const int nw = blockDim.x >> 6;
   float all = red[0][tl];
-  for (int w = 1; w < (int)(blockDim.x >> 6); ++w) all = fmaxf(all, red[w][tl]);
+#pragma unroll
+  for (int w = 1; w < 16; ++w) all = fmaxf(all, red[w < nw ? w : 0][tl]);
   const float s = skinny_scale(all), inv = 1.f / s;                 // powers of two
   if (ok && tid < 8) scale[((size_t)v * nq + q) * rss + tok] = s;
-  const int t32 = blockIdx.x >> 2, tile = t32 / ti, i32 = t32 % ti, l = tok & 31;
-  uint16_t* o0 = out + (size_t)v * xps + ((size_t)tile * (N >> 4) * ti + i32) * 512 + l * 8;
+  const uint32_t t32 = blockIdx.x >> 2, tile = ti == 1 ? t32 : ti == 2 ? t32 >> 1 : __umulhi(t32, 0xAAAAAAABu) >> 1;
+  const uint32_t i32 = t32 - tile * ti, l = tok & 31;
+  const auto o0 = through_buffer(out + (size_t)v * xps + ((size_t)tile * (N >> 4) * ti + i32) * 512);
   uint32_t* s0 = sums + (size_t)v * xcs + (size_t)tile * G * 2 * ti * 32 + i32 * 32 + l;
-  auto emit = [&](int c8, const uint4 xq, const uint4 cq) {         // (the pieces of half a group emit together: its sum needs all of them)
-    float a[8];
-    prep8(xq, cq, xdt, a);
+  auto emit = [&](int c8, const float (&f)[8]) {                    // (the pieces of half a group emit together: its sum needs all of them)
     uint16_t h[8];
     float sum = 0.f;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) { h[e] = f2h(a[e] * inv); sum += h2f(h[e]); }
+    for (int e = 0; e < 8; ++e) { h[e] = f2h(f[e] * inv); sum += h2f(h[e]); }
     uint32_t o[4];
-    if (order == 0) {
+    auto pair = [&](int lo, int hi) { return (uint32_t)h[lo] | ((uint32_t)h[hi] << 16); };
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = (uint32_t)h[2 * e] | ((uint32_t)h[2 * e + 1] << 16);
-    } else if (order == 1) {                                        // even columns, then odd ones
-      o[0] = (uint32_t)h[0] | ((uint32_t)h[2] << 16); o[1] = (uint32_t)h[4] | ((uint32_t)h[6] << 16);
-      o[2] = (uint32_t)h[1] | ((uint32_t)h[3] << 16); o[3] = (uint32_t)h[5] | ((uint32_t)h[7] << 16);
-    } else {                                                        // 0 4 1 5 2 6 3 7
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = (uint32_t)h[e] | ((uint32_t)h[e + 4] << 16);
-    }
-    const int run = c8 >> (lg - 4), t = c8 & ((1 << (lg - 4)) - 1);   // half group, step in it
-    if (ok) *(uint4*)(o0 + (size_t)((run >> 1 << (lg - 4)) + t) * (ti * 512) + (run & 1) * 256) = make_uint4(o[0], o[1], o[2], o[3]);
-    sum += __shfl_xor(sum, 8);                                      // the pieces of half a group: 32 or 64 columns
-    sum += __shfl_xor(sum, 16);
-    if (lg == 7) sum += __shfl_xor(sum, 32);
-    if (ok && t == 0) {
-      const uint16_t hi = f2h(sum), lo = f2h(sum - h2f(hi));
-      s0[(size_t)run * ti * 32] = (uint32_t)hi | ((uint32_t)lo << 16);
+    for (int e = 0; e < 4; ++e)                                     // SkCfg::ORDER: as they are; even columns, then odd ones; 0 4 1 5 2 6 3 7
+      o[e] = ORDER == 0 ? pair(2 * e, 2 * e + 1) : ORDER == 1 ? pair((4 * e + (e >> 1)) & 7, (4 * e + (e >> 1) + 2) & 7) : pair(e, e + 4);
+    sum = lanes16(lanes8(sum, plus), plus);                         // the pieces of half a group: 32 or 64 columns
+    const float both = lanes32(sum, plus);
+    if (lg == 7) sum = both;
+    const uint32_t run = (uint32_t)c8 >> (lg - 4), t = c8 & ((1 << (lg - 4)) - 1);   // half group, step in it
+    if (ok && c8 < e8) {
+      store16_through(o0, ((run >> 1 << (lg - 4)) + t) * (uint32_t)ti * 1024u + (run & 1) * 512u + l * 16u, make_uint4(o[0], o[1], o[2], o[3]));
+      if (t == 0) {
+        const uint16_t hi = f2h(sum), lo = f2h(sum - h2f(hi));
+        s0[(size_t)run * ti * 32] = (uint32_t)hi | ((uint32_t)lo << 16);
+      }
     }
   };
   if (CH) {
 #pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      const int c8 = b8 + (tid >> 3) + T8 * i;
-      if (c8 < e8) emit(c8, xk[i], ck[i]);
-    }
+    for (int i = 0; i < CH; ++i) emit(c0 + T8 * i, a[i]);
   } else {
-    for (int c8 = b8 + (tid >> 3); c8 < e8; c8 += T8) emit(c8, *(const uint4*)(xr + c8 * 8), cv ? *(const uint4*)(cv + c8 * 8) : one);
+    // (no wavefront has both pieces of the part and pieces past it in one half group)
+    for (int c8 = c0; c8 < e8; c8 += T8) {
+      prep8(*(const uint4*)(xr + c8 * 8), cv ? *(const uint4*)(cv + c8 * 8) : one, XDT, a[0]);
+      emit(c8, a[0]);
+    }
   }
+}
+
+template <int CH, int XDT>
+static auto skinny_prep_of(int order) {
+  return order == 0 ? skinny_prep_kernel<CH, XDT, 0> : order == 1 ? skinny_prep_kernel<CH, XDT, 1> : skinny_prep_kernel<CH, XDT, 2>;
+}
+template <int XDT>
+static auto skinny_prep_of(int ch, int order) {
+  return ch <= 4 ? skinny_prep_of<4, XDT>(order) : ch <= 8 ? skinny_prep_of<8, XDT>(order) : skinny_prep_of<0, XDT>(order);
 }
 
 // y = sum of the float32 partial tiles in part order (+ bias); ACT: act(gate) * up of the interleaved
@@ -242,10 +280,10 @@ int launch_gemm_skinny(const DMat& m, const GemmPlan& plan, const void* x, int x
   const int nq = plan.nsplit * SK_WC, p8 = (m.G + nq - 1) / nq * (m.group / 8);   // parts, 16-byte pieces of the longest
   const int want = (2 * p8 + 63) / 64 * 64;                         // four pieces per thread
   const int threads = want > 1024 ? 1024 : want, ch = (8 * p8 + threads - 1) / threads;
-  auto prep = ch <= 4 ? skinny_prep_kernel<4> : ch <= 8 ? skinny_prep_kernel<8> : skinny_prep_kernel<0>;
+  auto prep = xdt == CBK_F16 ? skinny_prep_of<CBK_F16>(ch, order) : skinny_prep_of<CBK_BF16T>(ch, order);
   hipLaunchKernelGGL(prep, dim3((unsigned)((M + 7) / 8), (unsigned)nq, (unsigned)nv), dim3(threads), 0, st, (const uint16_t*)x,
-                     ldx, m.cs, xdt, M, m.N, m.group == 64 ? 6 : 7, order, plan.ti, (uint16_t*)ws, a.xps, (uint32_t*)a.xc, a.xcs,
-                     (float*)a.row_scale, a.rss);
+                     ldx, m.cs, M, m.N, m.group == 64 ? 6 : 7, plan.ti, (uint32_t)(((1ull << 32) + nq - 1) / nq), (uint16_t*)ws, a.xps,
+                     (uint32_t*)a.xc, a.xcs, (float*)a.row_scale, a.rss);
   const int nb = a.tiles_t * a.tiles_r * a.nsplit, blocks = (nb + 7) / 8 * 8;
   const int fam = family_of(m.layout), keep = fam == FAM_DENSE ? 0 : m.keep;
   int rc;
