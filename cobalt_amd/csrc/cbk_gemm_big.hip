@@ -18,14 +18,13 @@ int launch_gemm_big_b6(const GbArgs&, int blocks, hipStream_t);
 // row's outputs by it.  Rows M..Mpad-1 and columns N..Npad-1 are zero.
 // One workgroup of T threads per row.  CH: 16-byte pieces of the row a thread keeps in
 // registers between the two passes (the row is read from memory once); 0 = any row length, the
-// second pass reads the row again.  Rows of up to 8192 columns take 256 threads, so that a CU has eight
-// of them in flight and a row's chain of load, exchange and store hides behind the others (1024 threads:
-// two in flight; 2 x 2048 rows of 5376 columns 23 -> 18 us); longer rows would need 200 registers
-// at that width (2048 rows of 21504 columns: 68 us, with 1024 threads 40).
-template <int CH, int T>
-__global__ __launch_bounds__(T) void gemm_prep_kernel(const uint16_t* x, int64_t ldx, const uint16_t* cs, int xdt,
-                                                         int M, int N, int Npad, uint16_t* out, size_t out_vs, float* row_scale,
-                                                         int scale_vs) {
+// second pass reads the row again.  Bound: reading x and writing X'.  The type of x is compiled in and no load stands behind a
+// condition of its own (a wavefront waited for each piece before it asked for the next); long rows take 512 threads and
+// six pieces rather than 1024 and three (four workgroups on a CU, so one's loads run beside another's stores); stores go on to
+// memory (store16_through).  2048 rows of 21504 columns (176 MB moved) 40.0 -> 32.7 us, 2 x 2048 of 5376 17.9 -> 15.5.
+template <int CH, int T, int XDT>
+__global__ __launch_bounds__(T) void gemm_prep_kernel(const uint16_t* x, int64_t ldx, const uint16_t* cs, int M, int N, int Npad,
+                                                      uint16_t* out, size_t out_vs, float* row_scale, int scale_vs) {
   __shared__ float red[T / 64];
   const int row = blockIdx.x, tid = threadIdx.x;
   const int n8 = Npad >> 3, nv = N >> 3;                           // N is a multiple of 128
@@ -39,28 +38,26 @@ __global__ __launch_bounds__(T) void gemm_prep_kernel(const uint16_t* x, int64_t
   }
   const uint16_t* xr = x + (size_t)row * ldx;
   const uint4 one = make_uint4(0x3c003c00u, 0x3c003c00u, 0x3c003c00u, 0x3c003c00u);
-  uint4 xv[CH ? CH : 1], cv[CH ? CH : 1];
+  float a[CH ? CH : 1][8];
   float mx = 0.f;
+  auto range = [&](const float (&f)[8]) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(f[e]));
+  };
   if (CH) {
+    // Pieces past the row: its last one again.  No load behind a condition of its own, which would wait for the one before.
+    uint4 xv[CH ? CH : 1], cv[CH ? CH : 1];
 #pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      const int c8 = tid + T * i;
-      xv[i] = make_uint4(0, 0, 0, 0); cv[i] = one;
-      if (c8 < nv) { xv[i] = *(const uint4*)(xr + c8 * 8); if (cs) cv[i] = *(const uint4*)(cs + c8 * 8); }
-    }
+    for (int i = 0; i < CH; ++i) { xv[i] = *(const uint4*)(xr + (tid + T * i < nv ? tid + T * i : nv - 1) * 8); cv[i] = one; }
+    if (cs)
 #pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      float a[8];
-      prep8(xv[i], cv[i], xdt, a);
+      for (int i = 0; i < CH; ++i) cv[i] = *(const uint4*)(cs + (tid + T * i < nv ? tid + T * i : nv - 1) * 8);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(a[e]));
-    }
+    for (int i = 0; i < CH; ++i) { prep8(xv[i], cv[i], XDT, a[i]); range(a[i]); }
   } else {
     for (int c8 = tid; c8 < nv; c8 += T) {
-      float a[8];
-      prep8(*(const uint4*)(xr + c8 * 8), cs ? *(const uint4*)(cs + c8 * 8) : one, xdt, a);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(a[e]));
+      prep8(*(const uint4*)(xr + c8 * 8), cs ? *(const uint4*)(cs + c8 * 8) : one, XDT, a[0]);
+      range(a[0]);
     }
   }
 #pragma unroll
@@ -73,26 +70,38 @@ __global__ __launch_bounds__(T) void gemm_prep_kernel(const uint16_t* x, int64_t
   const float s = token_scale(all);
   const float inv = 1.f / s;                                       // a power of two: exact
   if (tid == 0) row_scale[row] = s;
-  auto emit = [&](int c8, const uint4 xq, const uint4 cq) {
-    uint4 o4 = make_uint4(0, 0, 0, 0);
-    if (c8 < nv) {
-      float a[8];
-      prep8(xq, cq, xdt, a);
-      uint32_t o[4];
+  const auto dst = through_buffer(orow);
+  auto emit = [&](int c8, const float (&f)[8]) {
+    uint32_t o[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = (uint32_t)f2h(a[2 * e] * inv) | ((uint32_t)f2h(a[2 * e + 1] * inv) << 16);
-      o4 = make_uint4(o[0], o[1], o[2], o[3]);
-    }
-    *(uint4*)(orow + c8 * 8) = o4;
+    for (int e = 0; e < 4; ++e) o[e] = (uint32_t)f2h(f[2 * e] * inv) | ((uint32_t)f2h(f[2 * e + 1] * inv) << 16);
+    const bool in = c8 < nv;
+    store16_through(dst, (uint32_t)c8 * 16u, make_uint4(in ? o[0] : 0u, in ? o[1] : 0u, in ? o[2] : 0u, in ? o[3] : 0u));
   };
   if (CH) {
 #pragma unroll
     for (int i = 0; i < CH; ++i)
-      if (tid + T * i < n8) emit(tid + T * i, xv[i], cv[i]);
+      if (tid + T * i < n8) emit(tid + T * i, a[i]);
   } else {
-    for (int c8 = tid; c8 < n8; c8 += T)
-      emit(c8, c8 < nv ? *(const uint4*)(xr + c8 * 8) : one, (cs && c8 < nv) ? *(const uint4*)(cs + c8 * 8) : one);
+    for (int c8 = tid; c8 < n8; c8 += T) {
+      const int c = c8 < nv ? c8 : nv - 1;
+      prep8(*(const uint4*)(xr + c * 8), cs ? *(const uint4*)(cs + c * 8) : one, XDT, a[0]);
+      emit(c8, a[0]);
+    }
   }
+}
+
+typedef decltype(&gemm_prep_kernel<1, 256, CBK_F16>) PrepKernel;
+template <int XDT>
+static PrepKernel prep_of(int p8, int* threads) {                  // p8: 16-byte pieces of a row
+  if (p8 <= 1024) {
+    *threads = 256;
+    return p8 <= 256 ? gemm_prep_kernel<1, 256, XDT> : p8 <= 512 ? gemm_prep_kernel<2, 256, XDT>
+         : p8 <= 768 ? gemm_prep_kernel<3, 256, XDT> : gemm_prep_kernel<4, 256, XDT>;
+  }
+  *threads = 512;
+  return p8 <= 2048 ? gemm_prep_kernel<4, 512, XDT> : p8 <= 3072 ? gemm_prep_kernel<6, 512, XDT>
+       : p8 <= 4096 ? gemm_prep_kernel<8, 512, XDT> : gemm_prep_kernel<0, 512, XDT>;
 }
 
 static inline int gb_npad(int N) { return (N + 255) / 256 * 256; }
@@ -282,10 +291,9 @@ int launch_gemm_big(const DMat& m, const GemmPlan& plan, const void* x, int xdt,
   const size_t xbytes = ((size_t)nv * Mpad * Npad * 2 + 255) & ~(size_t)255;
   const size_t sbytes = ((size_t)nv * Mpad * 4 + 255) & ~(size_t)255;
   float* row_scale = (float*)((uint8_t*)ws + xbytes);
-  const int p8 = Npad / 8, pt = p8 <= 1024 ? 256 : 1024, ch = (p8 + pt - 1) / pt;   // 16-byte pieces of a row, threads, pieces of a thread
-  auto prep = pt == 1024 ? (ch <= 3 ? gemm_prep_kernel<3, 1024> : gemm_prep_kernel<0, 1024>)
-            : ch <= 1 ? gemm_prep_kernel<1, 256> : ch <= 2 ? gemm_prep_kernel<2, 256> : gemm_prep_kernel<4, 256>;
-  hipLaunchKernelGGL(prep, dim3((unsigned)Mpad, (unsigned)nv), dim3(pt), 0, st, (const uint16_t*)x, ldx, m.cs, xdt, M, m.N, Npad,
+  int threads;
+  const PrepKernel prep = xdt == CBK_F16 ? prep_of<CBK_F16>(Npad / 8, &threads) : prep_of<CBK_BF16T>(Npad / 8, &threads);
+  hipLaunchKernelGGL(prep, dim3((unsigned)Mpad, (unsigned)nv), dim3(threads), 0, st, (const uint16_t*)x, ldx, m.cs, M, m.N, Npad,
                      (uint16_t*)ws, (size_t)Mpad * Npad, row_scale, Mpad);   // one X' per col_scale vector
   GbArgs a;
   a.m = m; a.xp = (const uint16_t*)ws; a.M = M; a.Npad = Npad; a.y = y; a.ydt = ydt; a.ldy = ldy; a.bias = bias;
