@@ -96,7 +96,7 @@ class PackJob:
     def finish(self) -> PackedMatrix:
         from . import format as F
         pm = self.pm
-        wrong, pm.n_zero_fixed, z_max, n_mask = _lib.native().pack_end(self._pending, pm.blob.device.index)
+        wrong, pm.n_zero_fixed, z_max, n_mask = _lib.native().pack_end(self._pending)
         if wrong & 2:
             raise ValueError(f"{F.LAYOUT_NAME[pm.layout]} stores the zero point as the code of a pruned column, and a zero point "
                              f"of this matrix is above {(1 << pm.bits) - 1}: such a column would not dequantise to 0 (pack with "
