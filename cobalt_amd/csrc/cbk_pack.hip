@@ -42,6 +42,8 @@ struct GroupQ {
   float z_raw, s_raw, s_new, z_new;
   uint32_t z_out;
   uint16_t s_out;
+  bool small;                                                       // redo, and codes of the group: at most 15, map[c / 4] byte c % 4 is the new one
+  uint32_t map[4];
   __device__ inline uint32_t code(uint32_t q, float nl) const {
     if (!redo) return q > (uint32_t)nl ? (uint32_t)nl : q;
     const float v = __fmul_rn((float)q - z_raw, s_raw);
@@ -50,8 +52,15 @@ struct GroupQ {
 };
 
 // sz: the group's scale and, in the upper half, its zero point as given.  q, m: codes and mask of one 32-column block of the group; the blocks of a group are in consecutive
-// lanes (four or two of them, all active), which agree on the hull by lane exchanges.
-__device__ inline GroupQ group_quant(const PackArgs& a, float nl, uint32_t sz, const uint32_t (&q)[8], uint32_t m) {
+// lanes (four or two of them, all active), which agree on the hull by lane exchanges.  any: bits of q that no code has.
+//
+// A group that is re-derived costs its whole workgroup the time, as the others wait for it (one group in 500 off the grid
+// is two workgroups in three).  So its lanes do not take its 32 codes each through the arithmetic, a division apiece:
+// where all codes are at most 2^BITS - 1, the dequantised values are monotonic in the code and none is NaN (the zero
+// point is no code), so the hull is that of the smallest and the largest kept one; and the lanes work out the new code of the 16
+// there are between them and look theirs up by byte permutes.  14336 x 4096, one group in 500: 28.8 -> 25.7 us (23 without such groups), 24.4 with stores that go on to memory.
+template <int BITS>
+__device__ inline GroupQ group_quant(const PackArgs& a, float nl, uint32_t sz, const uint32_t (&q)[8], uint32_t m, uint32_t any) {
   GroupQ r;
   r.s_out = (uint16_t)sz;
   r.s_raw = h2f(r.s_out);
@@ -60,25 +69,74 @@ __device__ inline GroupQ group_quant(const PackArgs& a, float nl, uint32_t sz, c
   r.redo = a.fix_zero && (zi < 0 || zi > (int)nl);
   r.z_out = (uint32_t)zi & 0xffu;
   r.s_new = r.s_raw; r.z_new = r.z_raw;
+  r.small = false;
   if (!r.redo) return r;
   constexpr float BIG = 3.4028234663852886e38f;
+  const int lanes = a.group >> 5;
   float vmin = BIG, vmax = -BIG;
-#pragma unroll
-  for (int j = 0; j < 32; ++j) {
-    const float v = __fmul_rn((float)((q[j >> 2] >> (8 * (j & 3))) & 0xFFu) - r.z_raw, r.s_raw);
-    const bool kept = (m >> j) & 1u;
-    vmin = kept ? fminf(vmin, v) : vmin;
-    vmax = kept ? fmaxf(vmax, v) : vmax;
+  if (BITS <= 4) {
+    for (int o = 1; o < lanes; o <<= 1) any |= (uint32_t)__shfl_xor((int)any, o);
+    r.small = any == 0;
   }
-  for (int o = 1; o < a.group >> 5; o <<= 1) {
-    vmin = fminf(vmin, __shfl_xor(vmin, o));
-    vmax = fmaxf(vmax, __shfl_xor(vmax, o));
+  if (r.small) {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    u16x2 lo = {255, 255}, hi = {0, 0};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t kp = bits_to_bytes(m >> (4 * i)) * 0xFFu, l = q[i] | ~kp, h = q[i] & kp;
+      lo = __builtin_elementwise_min(lo, __builtin_bit_cast(u16x2, l & 0x00FF00FFu));
+      lo = __builtin_elementwise_min(lo, __builtin_bit_cast(u16x2, (l >> 8) & 0x00FF00FFu));
+      hi = __builtin_elementwise_max(hi, __builtin_bit_cast(u16x2, h & 0x00FF00FFu));
+      hi = __builtin_elementwise_max(hi, __builtin_bit_cast(u16x2, (h >> 8) & 0x00FF00FFu));
+    }
+    int least = lo[0] < lo[1] ? lo[0] : lo[1], most = hi[0] > hi[1] ? hi[0] : hi[1];
+    for (int o = 1; o < lanes; o <<= 1) {
+      const int l = __shfl_xor(least, o), h = __shfl_xor(most, o);
+      least = least < l ? least : l; most = most > h ? most : h;
+    }
+    if (least != 255) {                                             // (a kept code is at most 15)
+      const float v0 = __fmul_rn((float)least - r.z_raw, r.s_raw), v1 = __fmul_rn((float)most - r.z_raw, r.s_raw);
+      vmin = fminf(v0, v1); vmax = fmaxf(v0, v1);                   // (the scale may be negative)
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 32; ++j) {
+      const float v = __fmul_rn((float)((q[j >> 2] >> (8 * (j & 3))) & 0xFFu) - r.z_raw, r.s_raw);
+      const bool kept = (m >> j) & 1u;
+      vmin = kept ? fminf(vmin, v) : vmin;
+      vmax = kept ? fmaxf(vmax, v) : vmax;
+    }
+    for (int o = 1; o < lanes; o <<= 1) {
+      vmin = fminf(vmin, __shfl_xor(vmin, o));
+      vmax = fmaxf(vmax, __shfl_xor(vmax, o));
+    }
   }
   vmin = fminf(vmin, 0.f); vmax = fmaxf(vmax, 0.f);                // (a group without survivors: 0 and 0)
   r.s_new = fmaxf(__fdiv_rn(__fsub_rn(vmax, vmin), nl), 1e-12f);
   r.z_new = fminf(fmaxf(rintf(__fdiv_rn(-vmin, r.s_new)), 0.f), nl);
   r.z_out = (uint32_t)r.z_new;
   r.s_out = f2h(r.s_new);
+  if (r.small) {
+    auto four = [&](uint32_t c) {
+      uint32_t w = 0;
+      for (uint32_t e = 0; e < 4; ++e) w |= r.code(c + e, nl) << (8 * e);
+      return w;
+    };
+    const uint32_t at = threadIdx.x & (uint32_t)(lanes - 1);
+    if (lanes == 4) {                                               // lane i of the four: codes 4 i ... 4 i + 3
+      const int w = (int)four(4 * at);
+      r.map[0] = (uint32_t)__builtin_amdgcn_update_dpp(0, w, 0x00, 0xf, 0xf, false);
+      r.map[1] = (uint32_t)__builtin_amdgcn_update_dpp(0, w, 0x55, 0xf, 0xf, false);
+      r.map[2] = (uint32_t)__builtin_amdgcn_update_dpp(0, w, 0xAA, 0xf, 0xf, false);
+      r.map[3] = (uint32_t)__builtin_amdgcn_update_dpp(0, w, 0xFF, 0xf, 0xf, false);
+    } else {                                                        // of the two: eight each
+      const int w0 = (int)four(8 * at), w1 = (int)four(8 * at + 4);
+      r.map[0] = (uint32_t)__builtin_amdgcn_update_dpp(0, w0, 0xA0, 0xf, 0xf, false);
+      r.map[1] = (uint32_t)__builtin_amdgcn_update_dpp(0, w1, 0xA0, 0xf, 0xf, false);
+      r.map[2] = (uint32_t)__builtin_amdgcn_update_dpp(0, w0, 0xF5, 0xf, 0xf, false);
+      r.map[3] = (uint32_t)__builtin_amdgcn_update_dpp(0, w1, 0xF5, 0xf, 0xf, false);
+    }
+  }
   return r;
 }
 
@@ -170,7 +228,10 @@ __global__ __launch_bounds__(PK_THREADS) void pack_rows_kernel(PackArgs a) {
     uint32_t q[8] = {cur.qa.x, cur.qa.y, cur.qa.z, cur.qa.w, cur.qb.x, cur.qb.y, cur.qb.z, cur.qb.w};
     const uint32_t m = cur.m;
     surv += (uint32_t)__popc(m);
-    const GroupQ gq = group_quant(a, nl, cur.sz, q, m);
+    uint32_t any = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) any |= q[i] & over;
+    const GroupQ gq = group_quant<BITS>(a, nl, cur.sz, q, m, any);
     if ((c & (a.group - 1)) == 0) {                                // the group's first block stores its quantisation
       const size_t mi = a.tiled ? ((size_t)rt * a.G + g) * 16 + row : (size_t)k * a.G + g;
       a.oscale[mi] = gq.s_out;
@@ -178,10 +239,13 @@ __global__ __launch_bounds__(PK_THREADS) void pack_rows_kernel(PackArgs a) {
       fixed += gq.redo ? 1u : 0u;
       zmax = zmax > gq.z_out ? zmax : gq.z_out;
     }
-    uint32_t any = 0;
+    if (BITS <= 4 && gq.small) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) any |= q[i] & over;
-    if (gq.redo || any) {
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t sel = q[i] & 0x07070707u, up = ((q[i] >> 3) & 0x01010101u) * 0xFFu;
+        q[i] = (perm(gq.map[1], gq.map[0], sel) & ~up) | (perm(gq.map[3], gq.map[2], sel) & up);
+      }
+    } else if (gq.redo || any) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         uint32_t w = 0;
@@ -218,8 +282,8 @@ __global__ __launch_bounds__(PK_THREADS) void pack_rows_kernel(PackArgs a) {
     }
     if (__popc(m) != a.keep) st |= 1u;
     // survivors of the block, at most `keep` of them, as one bit string of at most 128 bits
-    uint64_t s0 = 0, s1 = 0;
-    uint32_t hw = 0;
+    static_assert(dense || pb <= 4, "the codes of a mask byte are at most 32 bits");
+    uint32_t hw = 0, w[4], at[4];                                  // codes of a mask byte, bits of those before it
     int r = 0;
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
@@ -234,12 +298,13 @@ __global__ __launch_bounds__(PK_THREADS) void pack_rows_kernel(PackArgs a) {
         }
         lo &= 0x0F0F0F0Fu; hi &= 0x0F0F0F0Fu;
       }
-      const uint64_t w = narrow8<pb>(lo, hi);
-      const int at = r * pb;
-      if (at < 64) { s0 |= w << at; if (at) s1 |= w >> (64 - at); }
-      else if (at < 128) s1 |= w << (at - 64);
+      w[b] = (uint32_t)narrow8<pb>(lo, hi);
+      at[b] = (uint32_t)(r * pb);
       r += __popc(mb);
     }
+    // two mask bytes at a time (at most 64 bits), then the second two behind the first
+    const uint64_t front = w[0] | ((uint64_t)w[1] << at[1]), back = w[2] | ((uint64_t)w[3] << (at[3] - at[2]));
+    uint64_t s0 = front | (at[2] < 64 ? back << (at[2] & 63u) : 0), s1 = at[2] == 0 ? 0 : at[2] < 64 ? back >> ((64u - at[2]) & 63u) : back;
     if (cb < 64) { s0 &= (1ull << (cb & 63)) - 1ull; s1 = 0; }            // (too many survivors: an error, but never into the next block)
     else if (cb < 128) s1 &= (1ull << (cb & 63)) - 1ull;
     const uint32_t bit = (uint32_t)t * cb, sh = bit & 31u;
@@ -263,16 +328,16 @@ __global__ __launch_bounds__(PK_THREADS) void pack_rows_kernel(PackArgs a) {
   }
   __syncthreads();
   // the image, unit by unit: consecutive threads write the rows of a unit (tiled: a 256-byte run) or the units of a row
-  auto unit_addr = [&](int row, uint32_t o) -> uint4* {            // o: byte offset in the row, a multiple of 16
-    return a.tiled ? (uint4*)(a.data + (size_t)rt * 16 * a.stride + (size_t)o * 16 + row * 16)
-                   : (uint4*)(a.data + (size_t)(k0 + row) * a.stride + o);
+  const auto rows_at = through_buffer(a.data + (size_t)rt * 16 * a.stride);
+  auto unit_at = [&](int row, uint32_t o) -> uint32_t {            // o: byte offset in the row, a multiple of 16
+    return a.tiled ? o * 16 + (uint32_t)row * 16 : (uint32_t)row * a.stride + o;
   };
   const int rows = a.krows - k0 < PK_ROWS ? a.krows - k0 : PK_ROWS;
   auto put = [&](uint32_t units, uint32_t o0, auto&& get) {
     for (uint32_t i = tid; i < PK_ROWS * units; i += PK_THREADS) {
       const int row = a.tiled ? (int)(i & 15u) : (int)(i / units);
       const uint32_t u = a.tiled ? i >> 4 : i % units;
-      if (row < rows) *unit_addr(row, o0 + u * 16) = get(row, u);
+      if (row < rows) store16_through(rows_at, unit_at(row, o0 + u * 16), get(row, u));
     }
   };
   put(cbytes >> 4, (dense ? 0u : plane) + (uint32_t)(c0 >> 5) * (uint32_t)cb / 8,

@@ -335,3 +335,36 @@ def test_pack_walks_every_slab_and_adds_their_records(K, N):
     got = ops.pack_raw(*[a.to(DEV) for a in args], F.BLKC, 3, 64, 10, tiled=True)
     assert torch.equal(got.blob.cpu(), want.blob)
     assert (got.n_zero_fixed, got.flags, got.n_survivors) == (2, want.flags, want.n_survivors)
+
+
+@pytest.mark.parametrize("case", FIXED_CASES, ids=case_id)
+def test_groups_off_the_grid_are_rederived_to_the_byte(case):
+    """Two groups in five off the code grid, by one and by far, on either side: in a wavefront beside groups that are not, scales of
+    both signs and zero, a group without survivors (dense), codes above the grid in some of the groups (those take
+    their codes one by one; the others look them up).  Byte for byte what the torch packer makes of it on the CPU."""
+    layout, bits, group, keep = case
+    K, N, nl = 35, 4096 + 640, (1 << bits) - 1
+    g = torch.Generator().manual_seed(bits * 100 + group + keep)
+    if keep:
+        mask = F.pack_mask(torch.zeros(K, N // 32, 32, dtype=torch.bool).scatter_(
+            -1, torch.rand(K, N // 32, 32, generator=g).topk(keep, -1).indices, True).view(K, N))
+    else:
+        kept = torch.rand(K, N, generator=g) < 0.5
+        kept[7, :group] = False
+        mask = F.pack_mask(kept)
+    q = torch.randint(0, nl + 1, (K, N), generator=g)
+    if bits < 8:
+        over = torch.rand(K, N // group, 1, generator=g) < 0.2
+        q = torch.where(over & (torch.rand(K, N // group, group, generator=g) < 0.1), nl + 1 + q.view(K, -1, group), q.view(K, -1, group)).view(K, N)
+    zero = torch.randint(0, nl + 1, (K, N // group), generator=g).float()
+    off = torch.rand(K, N // group, generator=g)
+    zero = torch.where(off < 0.1, -1 - zero, torch.where(off < 0.2, nl + 1 + zero, torch.where(off < 0.3, zero * 0 + nl + 1, torch.where(off < 0.4, zero * 0 - 1, zero))))
+    scale = (torch.rand(K, N // group, generator=g) * 0.02 - 0.01).half()
+    scale[3, :5] = 0
+    zero[7, 0] = -3
+    args = (mask, q.to(torch.uint8), scale, zero.half(), torch.rand(N, generator=g).half(), layout, bits, group, keep or None)
+    want = F.pack_raw(*args)
+    got = ops.pack_raw(*[a.to(DEV) for a in args[:5]], *args[5:], tiled=False)
+    assert got.n_zero_fixed == want.n_zero_fixed > K * (N // group) // 4
+    assert torch.equal(got.blob.cpu(), want.blob)
+    assert torch.equal(ops.pack_raw(*[a.to(DEV) for a in args[:5]], *args[5:], tiled=True).blob.cpu(), want.to_tiled().blob)
