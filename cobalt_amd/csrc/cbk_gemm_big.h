@@ -87,8 +87,8 @@ struct GbArgs {
   // vs1 on the third (both INT_MAX for any other matrix)
   int vs0, vs1;
   // split of the column range (PAR 3): nsplit workgroups per output tile take nst_part stages
-  // each and leave float32 partial tiles [nsplit][.][part_ld] at part; a second kernel adds them
-  int nsplit, nst_part;
+  // each, the first one nst_first, and leave float32 partial tiles [nsplit][.][part_ld] at part; a second kernel adds them
+  int nsplit, nst_part, nst_first;
   float* part;
   size_t part_stride;      // elements between the partial matrices
   int64_t part_ld;
@@ -216,12 +216,18 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
   const int wt = wave >> 1, wr = wave & 1;
   // XCD-aware order: blockIdx % 8 picks the XCD; give each XCD whole token tiles
   constexpr bool SPLIT = PAR == 3;
-  const int nb = a.tiles_t * a.tiles_r * (SPLIT ? a.nsplit : 1);
   const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-  const int per = (nb + 7) >> 3;
-  const int lin = xcd * per + idx;                                 // token-tile-major linear id
-  if (lin >= nb) return;
-  const int part = SPLIT ? lin % a.nsplit : 0, tile = SPLIT ? lin / a.nsplit : lin;
+  int part = 0, tile;                                              // token-tile-major tile
+  if (SPLIT && a.nst_first == a.nst_part) {                        // equal parts: side by side
+    const int nb = a.tiles_t * a.tiles_r * a.nsplit, lin = xcd * ((nb + 7) >> 3) + idx;
+    if (lin >= nb) return;
+    tile = lin / a.nsplit; part = lin - tile * a.nsplit;
+  } else {                                                         // the first parts of all of an XCD's tiles, then the second ones
+    const int nb = a.tiles_t * a.tiles_r, per = (nb + 7) >> 3;
+    if (SPLIT) part = idx >= per ? 1 : 0;
+    tile = xcd * per + idx - part * per;
+    if (tile >= nb) return;
+  }
   const int tt = tile / a.tiles_r, tr = tile % a.tiles_r + a.tr0;
   constexpr int kstep = PAR == 1 ? 2 : 1;                         // row stride of this workgroup's rows
   const int pp = PAR == 1 ? (tr & 1) : 0;                         // and their parity
@@ -229,8 +235,8 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
   const int N = m.N, Npad = a.Npad;
   // stages of this workgroup: all of them, or its part of them; a multiple of 4 either way;
   // stages past N see X' = 0
-  const int s_begin = SPLIT ? part * a.nst_part : 0;
-  const int nst = SPLIT ? (Npad / GB_K - s_begin < a.nst_part ? Npad / GB_K - s_begin : a.nst_part) : Npad / GB_K;
+  const int s_begin = SPLIT && part ? a.nst_first + (part - 1) * a.nst_part : 0, s_len = part ? a.nst_part : a.nst_first;
+  const int nst = SPLIT && s_len < Npad / GB_K - s_begin ? s_len : Npad / GB_K - s_begin;
   const int c_begin = s_begin >> 1;                               // first 128-column chunk
   const int nch = N >> 7;                                         // 128-column chunks of the weight rows
 

@@ -161,6 +161,8 @@ static bool gb_fast(const DMat& m) {
 // 98.)  Over 24 measured calls
 // (eight shapes, 256 / 512 / 2048 rows) the choice is within 2 % of the faster tile; always
 // taking the 256-token tile loses 6 % on average and up to 34 %.
+static inline double gb_t_stage(int ti) { return ti == 1 ? 1.1 : ti == 2 ? 1.35 : 1.7; }
+static inline double gb_t_wg(int ti) { return ti == 1 ? 8.0 : 10.0; }
 static inline size_t gb_kpad(int K) { return (size_t)(K + 7) / 8 * 8; }
 static size_t gb_space(const DMat& m, int M, int ti, int nsplit) {
   const size_t T = 64 * ti, mpad = (size_t)(M + T - 1) / T * T;
@@ -175,10 +177,34 @@ static int gb_part(const DMat& m, int nsplit) {
   const int nst = gb_npad(m.N) / GB_K, per = ((nst + nsplit - 1) / nsplit + 3) / 4 * 4;
   return nsplit > 1 && (nsplit - 1) * per >= nst ? 0 : per;
 }
+// The parts of a launch whose plan is `nsplit` parts of `tiles` tiles.  They are equal, but where a plan cuts 129 tiles or more
+// in n >= 3 parts to fill n - 1 rounds: there two parts may do, the first ones, a workgroup each on its CU from the start,
+// so long that the CUs without one need as long for all the second ones.  The same CU time with fewer partial tiles, and a
+// workgroup's start and end less for most.  Workgroups go to the eight XCDs in turn and to the four shader engines of one in turn, and stay there:
+// it is the eight CUs of an engine that share its second parts (168 tiles, 228 + 108 stages, as 256 CUs would
+// share them: three turns instead of two, 5376 x 21504 at 2048 tokens 447 -> 574 us).  Equal and unequal parts, us, with preparation
+// and reduction: 160 tiles 5120 x 20480 426 -> 408, 4096 x 14336 320 -> 307; 144 tiles 4608 x 18432 374 -> 360; 192 tiles
+// 6144 x 24576 578 -> 552.
+// (The plan does not count it: calls keep their kernel and room.)
+struct GbCut { int nsplit, first, part; };
+static GbCut gb_cut(const DMat& m, int tiles, int ti, int nsplit) {
+  const int per = gb_part(m, nsplit), nst = gb_npad(m.N) / GB_K;
+  GbCut c = {nsplit, per, per};
+  const int held = ((tiles + 7) / 8 + 3) / 4, left = 8 - held;      // CUs of a shader engine with and without a first part
+  if (nsplit < 3 || tiles <= 128 || left < 1) return c;
+  const double t_stage = gb_t_stage(ti), t_wg = gb_t_wg(ti);
+  const int turns = (held + left - 1) / left;                       // second parts of a CU without a first one
+  double best = (double)((tiles * nsplit + 255) / 256) * (per * t_stage + t_wg);
+  for (int s = 4; 2 * s < nst; s += 4) {
+    const double first = (nst - s) * t_stage + t_wg, rest = turns * (s * t_stage + t_wg), t = first > rest ? first : rest;
+    if (t < best) { best = t; c = {2, nst - s, s}; }
+  }
+  return c;
+}
 static GemmPlan gb_plan_ti(const DMat& m, int M, int ti, int max_split, size_t room) {
   const int T = 64 * ti;
   const int tiles = ((M + T - 1) / T) * ((m.K + GB_R - 1) / GB_R);
-  const double t_stage = ti == 1 ? 1.1 : ti == 2 ? 1.35 : 1.7, t_wg = ti == 1 ? 8.0 : 10.0;
+  const double t_stage = gb_t_stage(ti), t_wg = gb_t_wg(ti);
   GemmPlan best, one;
   const bool may_split = max_split > 1 && m.cs_rows != 2 && gb_fast(m);
   for (int s = 1; s <= (may_split ? max_split : 1); ++s) {
@@ -255,8 +281,8 @@ LastRound last_round_big(const DMat& m, const GemmPlan& p, int M) {
 
 static int gb_launch(const GbArgs& a, hipStream_t st) {
   const DMat& m = a.m;
-  const int nb = a.tiles_t * a.tiles_r * a.nsplit;
-  const int blocks = ((nb + 7) / 8) * 8;
+  const int tiles = a.tiles_t * a.tiles_r;
+  const int blocks = a.nst_first == a.nst_part ? (tiles * a.nsplit + 7) / 8 * 8 : (tiles + 7) / 8 * 8 * a.nsplit;
   const bool le128 = (m.flags & CBK_FLAG_ZERO_LE_128) != 0;
   const int fam = family_of(m.layout);
   int rc = CBK_ERR_UNSUPPORTED;
@@ -302,8 +328,6 @@ int launch_gemm_big(const DMat& m, const GemmPlan& plan, const void* x, int xdt,
   a.row_scale = row_scale; a.rss = Mpad;
   a.vs0 = m.cs_rows == 3 ? m.cs_split0 : 0x7fffffff;
   a.vs1 = m.cs_rows == 3 ? m.cs_split0 + m.cs_split1 : 0x7fffffff;
-  a.nsplit = plan.nsplit;
-  a.nst_part = gb_part(m, plan.nsplit);
   a.part_ld = (int64_t)gb_kpad(m.K);
   a.part_stride = (size_t)M * gb_kpad(m.K);
   a.part = (float*)((uint8_t*)ws + xbytes + sbytes);
@@ -312,6 +336,8 @@ int launch_gemm_big(const DMat& m, const GemmPlan& plan, const void* x, int xdt,
   a.tiles_t = (M + T - 1) / T;
   const LastRound tail = last_round_big(m, plan, M);
   a.tiles_r = gb_row_tiles(m) - tail.rows;
+  const GbCut cut = gb_cut(m, a.tiles_t * a.tiles_r, plan.ti, plan.nsplit);
+  a.nsplit = cut.nsplit; a.nst_first = cut.first; a.nst_part = cut.part;
   int rc = gb_launch(a, st);
   if (rc == CBK_OK && tail.rows) {
     a.tr0 = a.tiles_r;

@@ -159,3 +159,22 @@ def test_a_plain_call_is_the_call_its_plan_names():
                 assert torch.equal(ops.linear_act(pm, x, "silu"), gemm_as(pm, x, *plan, act="silu")), (case, M, plan)
     kinds = {k[:2] for k in seen}
     assert {("rows", 32), ("rows", 64), ("rows", 96), ("tile", 256)} <= kinds and {k[2] for k in seen} == {False, True}, sorted(seen)
+
+
+@pytest.mark.parametrize("tokens", [64, 128, 256])
+@pytest.mark.parametrize("row_tiles,parts,N", [(9, 3, 1536), (10, 3, 1664), (12, 4, 2048)])
+def test_columns_in_two_unequal_parts(row_tiles, parts, N, tokens):
+    """144, 160 and 192 tiles whose plan is three or four parts run as a long and a short one (the last
+    tiles ragged on both sides, a padded last chunk of columns).  Operands are rounded to 2^-12 twice: 3e-4, as everywhere on this
+    kernel; against the unsplit call only the order of float32 sums differs."""
+    K, M = 256 * row_tiles - 7, 16 * tokens - 5
+    pm = F.synth_packed(K, N, F.BLK1632_4, 4, 128, 16, seed=row_tiles, device=DEV).to_tiled()
+    x = acts(M, N, torch.float16, seed=tokens).to(DEV)
+    y = gemm_as(pm, x, "tile", tokens, parts, out_dtype=torch.float32).double()
+    ref = x.double() @ ops.dequant(pm, torch.float32).double().t()
+    assert float((y - ref).norm() / ref.norm()) < 5e-4
+    one = gemm_as(pm, x, "tile", tokens, out_dtype=torch.float32).double()
+    assert float((y - one).norm() / one.norm()) < 1e-5
+    assert torch.equal(y, gemm_as(pm, x, "tile", tokens, parts, out_dtype=torch.float32).double())
+    bias = acts(1, K, torch.float32, seed=4)[0].to(DEV)
+    assert torch.equal(gemm_as(pm, x, "tile", tokens, parts, bias=bias, out_dtype=torch.float32), y.float() + bias)
