@@ -178,3 +178,18 @@ def test_columns_in_two_unequal_parts(row_tiles, parts, N, tokens):
     assert torch.equal(y, gemm_as(pm, x, "tile", tokens, parts, out_dtype=torch.float32).double())
     bias = acts(1, K, torch.float32, seed=4)[0].to(DEV)
     assert torch.equal(gemm_as(pm, x, "tile", tokens, parts, bias=bias, out_dtype=torch.float32), y.float() + bias)
+
+
+@pytest.mark.parametrize("tokens", [64, 128, 256])
+@pytest.mark.parametrize("K", [256, 260, 262, 263, 129])
+def test_rows_of_y_that_start_anywhere(K, tokens):
+    """Heights that are multiples of 8, 4, 2 and 1: whole 16-byte pieces, dwords of two outputs, single elements.  Every
+    output of a 16-bit call is the float32 call's rounded once."""
+    M = tokens + 37
+    pm = F.synth_packed(K, 512, F.BLK1632_4, 4, 128, 16, seed=K, device=DEV).to_tiled()
+    x = acts(M, 512, torch.float16, seed=tokens).to(DEV)
+    y = gemm_as(pm, x, "tile", tokens, out_dtype=torch.float32)
+    ref = x.double() @ ops.dequant(pm, torch.float32).double().t()
+    assert float((y.double() - ref).norm() / ref.norm()) < 5e-4
+    for dt in (torch.float16, torch.bfloat16):
+        assert torch.equal(gemm_as(pm, x, "tile", tokens, out_dtype=dt), y.to(dt)), dt
