@@ -1,11 +1,12 @@
 """Builds libcbk_hip.so (the C-ABI HIP library, hipcc for gfx950) and _native.so (its operators for
 Python) in-tree."""
+import multiprocessing
 import os
 import re
 import subprocess
 import sys
 import tempfile
-from concurrent.futures import ThreadPoolExecutor
+from concurrent.futures import ProcessPoolExecutor, ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -74,6 +75,91 @@ def shift_hazards(code_object):
     return out
 
 
+# Wait states between two instructions that the hardware does not keep apart.  The compiler fills them in, but not around
+# instructions written by hand (cbk_gemm_big.h): the values are those it leaves on gfx950 around its own.  An instruction
+# is one wait state, s_nop n is n + 1.
+VALU_TO_VMEM = 5                                                       # a scalar register written by a vector instruction -> a memory instruction reads it
+_REG = re.compile(r"(?<![\w])([vas])(?:(\d+)\b|\[(\d+):(\d+)\])")
+_TARGET = re.compile(r"<(\S+?)(?:\+0x([0-9a-f]+))?>$")
+
+
+def _registers(text):
+    return {(k, r) for k, n, lo, hi in _REG.findall(text) for r in (range(int(lo), int(hi) + 1) if lo else (int(n),))}
+
+
+def _functions(code_object):
+    """(name, [(address, mnemonic, operands, branch target or None)]) of every function of a code object."""
+    dis = subprocess.Popen([_llvm("llvm-objdump"), "-d", "--no-show-raw-insn", code_object], stdout=subprocess.PIPE, text=True)
+    name, start, body = "", 0, []
+    for line in dis.stdout:
+        if line.endswith(">:\n"):
+            if body:
+                yield name, body
+            name, start, body = line[line.index("<") + 1:-3], int(line[:line.index(" ")], 16), []
+            continue
+        text, _, note = line.partition("//")
+        op, _, args = text.strip().partition(" ")
+        if not op or not note:
+            continue
+        target = None
+        if op.startswith(("s_cbranch", "s_branch")):
+            m = _TARGET.search(note.strip())
+            if m and m.group(1) == name:
+                target = start + int(m.group(2) or "0", 16)
+        body.append((int(note[:note.index(":")], 16), op, args.strip(), target))
+    if body:
+        yield name, body
+    if dis.wait() != 0:
+        raise RuntimeError(f"llvm-objdump failed on {code_object}")
+
+
+def wait_hazards(code_object):
+    """[(function, address, instruction, register, instruction that follows too soon)] of a gfx950 code object: the pairs
+    above that lie closer together, along any path of branches inside a function."""
+    out = []
+    for fn, body in _functions(code_object):
+        at = {b[0]: i for i, b in enumerate(body)}
+        regs = [None] * len(body)
+
+        def touched(i):
+            if regs[i] is None:
+                regs[i] = _registers(body[i][2])
+            return regs[i]
+
+        def followers(i, states):
+            """Instructions that can begin fewer than `states` wait states after instruction i."""
+            todo, seen = [(i, states)], {}
+            while todo:
+                j, left = todo.pop()
+                _, op, args, target = body[j]
+                if j != i:
+                    left -= int(args, 0) + 1 if op == "s_nop" else 1
+                nxt = [] if op in ("s_branch", "s_endpgm", "s_setpc_b64") else [j + 1]
+                if target is not None and target in at:
+                    nxt.append(at[target])
+                for n in nxt:
+                    if left > 0 and n < len(body) and seen.get(n, 0) < left:
+                        if n not in seen:
+                            yield n
+                        seen[n] = left
+                        todo.append((n, left))
+
+        for i, (addr, op, args, _) in enumerate(body):
+            if not op.startswith("v_") or op.startswith("v_mfma"):
+                continue
+            dst = args.split(", ", 2)
+            first = _registers(dst[0])
+            if len(dst) > 1 and any(o in op for o in ("_co_", "v_div_scale", "v_mad_u64", "v_mad_i64")):
+                first |= _registers(dst[1])
+            if any(k == "s" for k, _ in first):
+                for j in followers(i, VALU_TO_VMEM):
+                    if body[j][1].startswith(("buffer_", "global_", "scratch_", "flat_")):
+                        hit = {r for r in first if r[0] == "s"} & touched(j)
+                        if hit:
+                            out.append((fn, addr, op, "%s%d" % min(hit), body[j][1]))
+    return out
+
+
 # Kernels whose table reads take an entry's offset in dynamic LDS as its address: nothing else may lie before it.
 LDS_FROM_ZERO = ("gemm_skinny_kernel",)
 
@@ -84,19 +170,24 @@ def static_lds(code_object):
     return [(k, lds) for k, (_, lds) in _kernels(code_object).items() if lds and any(n in k for n in LDS_FROM_ZERO)]
 
 
-def _of_every_code_object(check, path):
+def _of_every_code_object(check, path, executor=ThreadPoolExecutor):
     """What `check` finds in every gfx950 code object inside an object file or library."""
     with tempfile.TemporaryDirectory() as tmp:
         link = os.path.join(tmp, "o")
         os.symlink(os.path.abspath(path), link)
         subprocess.run([_llvm("llvm-objdump"), "--offloading", link], check=True, capture_output=True)
         objs = [os.path.join(tmp, f) for f in sorted(os.listdir(tmp)) if "gfx950" in f]
-        with ThreadPoolExecutor(8) as ex:
+        with executor(8) as ex:
             return [h for hs in ex.map(check, objs) for h in hs]
 
 
 def shift_hazards_of(path):
     return _of_every_code_object(shift_hazards, path)
+
+
+def wait_hazards_of(path):
+    # (python's own work: processes)
+    return _of_every_code_object(wait_hazards, path, lambda n: ProcessPoolExecutor(n, multiprocessing.get_context("fork")))
 
 
 def static_lds_of(path):
@@ -135,6 +226,11 @@ def build_lib(verbose=True, extra=()):
         os.remove(LIB)
         raise RuntimeError("64-bit shifts with their amount in the last register (see shift_hazards):\n" +
                            "\n".join(f"  {op} amount v{r} in {fn}" for fn, op, r in bad))
+    bad = wait_hazards_of(LIB)
+    if bad:
+        os.remove(LIB)
+        raise RuntimeError("instructions that follow each other too soon (see wait_hazards):\n" +
+                           "\n".join(f"  {op} of {r}, then {then}, at {at:#x} of {fn}" for fn, at, op, r, then in bad))
     return LIB
 
 

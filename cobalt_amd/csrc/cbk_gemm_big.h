@@ -98,9 +98,14 @@ struct GbArgs {
 // ds_write): lane l reads base + soff + voff and its 16 bytes land at LDS byte lds + AT + 16 * l.  The
 // compiler does not know that this instruction counts on vmcnt or that it writes LDS; the
 // kernel waits for it by hand before the barrier that publishes the stage.
-template <int AT>
+// Nor does it put the five wait states between a vector instruction that writes a scalar register and a memory instruction
+// that reads it, as it does around its own.  SPILLS: kernels that keep the descriptor or an offset in vector registers
+// and read it back right before (the generic reader's): the wait is here.  The others have them in scalar registers from
+// long before, which build.py (wait_hazards) looks at.
+template <int AT, bool SPILLS>
 __device__ inline void dma_x16(v4u buffer, uint32_t voff, uint32_t soff, uint32_t lds) {
-  asm volatile("s_add_u32 m0, %3, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(buffer), "s"(soff), "s"(lds), "i"(AT) : "memory", "m0", "scc");
+  asm volatile("s_add_u32 m0, %3, %4\n\ts_nop %5\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+               ::"v"(voff), "s"(buffer), "s"(soff), "s"(lds), "i"(AT), "i"(SPILLS ? 4 : 0) : "memory", "m0", "scc");
 }
 // the same in every lane, in a scalar register
 __device__ inline uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
@@ -306,7 +311,7 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
   };
   auto dma_x = [&](auto buf_, auto q_) {                          // copy q of that stage -> Xs[buf]
     constexpr int q = decltype(q_)::value;
-    dma_x16<decltype(buf_)::value * GB_XBUF + q * 1024>(xbuf, (q & 1) ? xvo_o : xvo_e, q * xrow8, xlds0);
+    dma_x16<decltype(buf_)::value * GB_XBUF + q * 1024, !FASTD>(xbuf, (q & 1) ? xvo_o : xvo_e, q * xrow8, xlds0);
   };
   // fragment reads: this lane's row inside a 16-row block of either operand and its two swizzled piece offsets
   uint32_t xpc[2], wpc[2];

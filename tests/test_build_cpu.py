@@ -82,3 +82,37 @@ def test_kernels_that_read_from_lds_address_0_have_no_static_lds():
     assert B.static_lds_of(B.LIB) == []
     names = B._of_every_code_object(B._kernels, B.LIB)
     assert all(any(n in k for k in names) for n in B.LDS_FROM_ZERO)
+
+
+def assembled(tmp_path, code):
+    """A kernel of these instructions, assembled and never run."""
+    src, obj = tmp_path / "k.s", str(tmp_path / "k.co")
+    text = KERNEL.format(op="v_lshrrev_b64", amount=6, n=264, agpr=8, accum=256)
+    begin, end = text.index("  v_mov_b32_e32"), text.index("  s_endpgm")
+    src.write_text(text[:begin] + "".join(f"  {c}\n" for c in code) + text[end:])
+    subprocess.run([B._llvm("clang"), "-target", "amdgcn-amd-amdhsa", "-mcpu=gfx950", str(src), "-o", obj], check=True)
+    return obj
+
+
+LDS_COPY = "buffer_load_dwordx4 v2, s[4:7], s9 offen lds"
+
+
+@pytest.mark.parametrize("code,hit", [
+    (["v_readfirstlane_b32 s4, v0", "s_add_u32 m0, s8, 16", "s_nop 0", LDS_COPY], "s4"),
+    (["v_readfirstlane_b32 s4, v0", "s_add_u32 m0, s8, 16", "s_nop 4", LDS_COPY], None),
+    (["v_readlane_b32 s9, v0, 3", "s_nop 3", LDS_COPY], "s9"),           # the offset, one state short
+    (["v_readlane_b32 s9, v0, 3", "s_nop 3", "s_nop 0", LDS_COPY], None),
+    (["v_readfirstlane_b32 s10, v0", LDS_COPY], None),                 # another register
+    (["v_cmp_lt_u32_e64 s[4:5], v0, v1", "v_mov_b32_e32 v3, 0", LDS_COPY], "s4"),
+    (["v_readfirstlane_b32 s4, v0", "s_cbranch_scc1 2", "s_nop 7", "s_nop 7", LDS_COPY], "s4"),   # only on the path that jumps
+    (["v_readfirstlane_b32 s4, v0", "s_branch 2", LDS_COPY, "s_endpgm", "s_nop 3", LDS_COPY], None),
+    (["s_nop 7", LDS_COPY, "s_nop 7", "v_readfirstlane_b32 s4, v0", "s_cbranch_scc1 65531"], "s4")])   # around a loop (to the copy)
+def test_scalar_registers_read_too_soon_are_found(tmp_path, code, hit):
+    found = B.wait_hazards(assembled(tmp_path, code))
+    assert [f[3] for f in found] == ([hit] if hit else [])
+
+
+def test_no_kernel_of_the_library_reads_a_register_too_soon():
+    if not os.path.exists(B.LIB):
+        pytest.skip("the library is not built")
+    assert B.wait_hazards_of(B.LIB) == []
