@@ -78,6 +78,8 @@ def shift_hazards(code_object):
 # Wait states between two instructions that the hardware does not keep apart.  The compiler fills them in, but not around
 # instructions written by hand (cbk_gemm_big.h): the values are those it leaves on gfx950 around its own.  An instruction
 # is one wait state, s_nop n is n + 1.
+MFMA_TO_READ = {"v_mfma_f32_16x16x32_f16": 8, "v_mfma_f32_32x32x16_f16": 12}   # until anything but the next product of the same sums touches them
+VALU_TO_MFMA = 2                                                       # a vector register written -> a matrix instruction reads it
 VALU_TO_VMEM = 5                                                       # a scalar register written by a vector instruction -> a memory instruction reads it
 _REG = re.compile(r"(?<![\w])([vas])(?:(\d+)\b|\[(\d+):(\d+)\])")
 _TARGET = re.compile(r"<(\S+?)(?:\+0x([0-9a-f]+))?>$")
@@ -145,16 +147,35 @@ def wait_hazards(code_object):
                         todo.append((n, left))
 
         for i, (addr, op, args, _) in enumerate(body):
-            if not op.startswith("v_") or op.startswith("v_mfma"):
+            if not op.startswith("v_"):
                 continue
-            dst = args.split(", ", 2)
-            first = _registers(dst[0])
-            if len(dst) > 1 and any(o in op for o in ("_co_", "v_div_scale", "v_mad_u64", "v_mad_i64")):
-                first |= _registers(dst[1])
-            if any(k == "s" for k, _ in first):
-                for j in followers(i, VALU_TO_VMEM):
-                    if body[j][1].startswith(("buffer_", "global_", "scratch_", "flat_")):
-                        hit = {r for r in first if r[0] == "s"} & touched(j)
+            if op in MFMA_TO_READ:
+                sums = args.partition(", ")[0]
+                dst = _registers(sums)
+                for j in followers(i, MFMA_TO_READ[op]):
+                    hit = dst & touched(j)
+                    if hit and body[j][1] == op:
+                        d, a, b, c = body[j][2].split(", ")[:4]
+                        if c == d == sums:                             # the next product of the same sums: chained by the hardware
+                            hit = dst & _registers(a + " " + b)
+                    if hit:
+                        out.append((fn, addr, op, "%s%d" % min(hit), body[j][1]))
+            elif op.startswith("v_mfma") or op.startswith("v_smfma"):
+                continue
+            else:
+                dst = args.split(", ", 2)
+                first = _registers(dst[0])
+                if len(dst) > 1 and any(o in op for o in ("_co_", "v_div_scale", "v_mad_u64", "v_mad_i64")):
+                    first |= _registers(dst[1])
+                if any(k == "s" for k, _ in first):
+                    for j in followers(i, VALU_TO_VMEM):
+                        if body[j][1].startswith(("buffer_", "global_", "scratch_", "flat_")):
+                            hit = {r for r in first if r[0] == "s"} & touched(j)
+                            if hit:
+                                out.append((fn, addr, op, "%s%d" % min(hit), body[j][1]))
+                if any(k != "s" for k, _ in first) and any(b[1] in MFMA_TO_READ for b in body[i + 1:i + 1 + VALU_TO_MFMA]):
+                    for j in followers(i, VALU_TO_MFMA):
+                        hit = first & _registers(body[j][2].partition(", ")[2]) if body[j][1] in MFMA_TO_READ else None
                         if hit:
                             out.append((fn, addr, op, "%s%d" % min(hit), body[j][1]))
     return out

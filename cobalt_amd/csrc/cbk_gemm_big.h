@@ -118,11 +118,23 @@ __device__ inline void static_for(F&& f) { static_for_seq(f, std::make_integer_s
 
 // d += w . x^T of 16 weight rows, 16 tokens and 32 columns.  Written as the instruction, with the sum in place in
 // accumulation registers: the compiler's own choice of a destination beside the addend left 912 register copies in
-// a trip of the loop (the gated block of the header 1395 -> 1663 us).  What reads the sums waits (gb_mfma_done).
+// a trip of the loop (the gated block of the header 1395 -> 1663 us).  So the compiler knows of no wait states: two behind what
+// writes an operand, eight before anything else reads a sum.  The sums are tied to the wait behind the loop (gb_mfma_done); that nothing
+// comes between, a copy or a spill, is looked at in every build (build.py, wait_hazards).  SPILLS: the generic reader's kernels, which
+// move sums around the calls of their decoder, leave it to the compiler.
+template <bool SPILLS>
 __device__ inline void gb_mfma(v4f& d, const v8h& w, const v8h& x) {
-  asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(d) : "v"(w), "v"(x));
+  if (SPILLS) d = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, x, d, 0, 0, 0);
+  else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(d) : "v"(w), "v"(x));
 }
-__device__ inline void gb_mfma_done() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
+template <int N>
+__device__ inline void gb_mfma_done(v4f (&acc)[N][8]) {
+  asm volatile("s_nop 15" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) asm volatile("" : "+a"(acc[i][j]));
+}
 
 // One wavefront's 128 x 128 accumulators -> y, 32 tokens at a time through LDS.  D[i][j] holds, in
 // lane l and register r, token l%16 and weight row 4*(l/16) + r of its 16 x 16 block: four consecutive
@@ -574,7 +586,7 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
         constexpr int g = p >= BP ? at - 4 * TI * BP : at + 4 * TI * (8 - BP);      // MFMAs since the barrier
         if constexpr (g == 0) dma_stage(s + 2);
         if constexpr (g % DMAX == 2 && g / DMAX < 2 * TI) dma_x(std::integral_constant<int, p >= BP ? BUF : 1 - BUF>{}, std::integral_constant<int, g / DMAX>{});
-        gb_mfma(acc[TI * hx + i][4 * hw + j], bf[DEEP ? kk : 0][hw][j], af[DEEP ? kk : 0][hx][i]);
+        gb_mfma<!FASTD>(acc[TI * hx + i][4 * hw + j], bf[DEEP ? kk : 0][hw][j], af[DEEP ? kk : 0][hx][i]);
         if constexpr (p < BP) {
           constexpr int d0 = DEC0 + at * 8 * PIECES / MF, d1 = DEC0 + (at + 1) * 8 * PIECES / MF;
           static_for<d1 - d0>([&](auto d_) { decode_step(s + 1, std::integral_constant<int, d0 + decltype(d_)::value>{}, wd, hd_tag, wn, hn_tag, buf ^ 1); });
@@ -595,11 +607,11 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
     stage(s + 2, H0{}, T{},  wB, H1{}, wA, H0{}, wA, p + 3);
     stage(s + 3, H1{}, Fl{}, wA, H0{}, wA, H1{}, wB, 0);
   }
+  gb_mfma_done(acc);
   // the last stage issued copies of a stage that does not exist: let them land before the
   // epilogue reuses LDS
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  gb_mfma_done();
 
   const int tok0 = t0 + 32 * TI * wt, row0 = r0 + kstep * 128 * wr;
   const float* rs = a.row_scale + (size_t)xv * a.rss;

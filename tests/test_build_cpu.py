@@ -112,6 +112,58 @@ def test_scalar_registers_read_too_soon_are_found(tmp_path, code, hit):
     assert [f[3] for f in found] == ([hit] if hit else [])
 
 
+MFMA = "v_mfma_f32_16x16x32_f16 a[0:3], v[4:7], v[8:11], a[0:3]"
+READ = "v_accvgpr_read_b32 v0, a3"
+
+
+@pytest.mark.parametrize("code,hit", [
+    ([MFMA, "s_nop 6", READ], "a3"), ([MFMA, "s_nop 7", READ], None),
+    ([MFMA, "s_nop 6", "v_accvgpr_write_b32 a2, 0"], "a2"),
+    ([MFMA, "s_nop 6", "v_accvgpr_read_b32 v0, a4"], None),
+    ([MFMA, MFMA, "s_nop 7", READ], None),                              # the same sums again: chained
+    ([MFMA, "s_nop 6", "v_mfma_f32_16x16x32_f16 a[4:7], v[4:7], v[8:11], a[0:3]"], "a0"),
+    ([MFMA, "s_nop 6", "v_mfma_f32_16x16x32_f16 a[4:7], a[0:3], v[8:11], a[4:7]"], "a0"),
+    ([MFMA, "s_nop 7", "v_mfma_f32_16x16x32_f16 a[4:7], a[0:3], v[8:11], a[4:7]"], None),
+    ([MFMA, "s_cbranch_scc1 1", "s_nop 7", READ], "a3"),
+    (["s_nop 0", READ, "s_nop 7", MFMA, "s_cbranch_scc0 65530"], "a3"),    # around a loop
+    (["v_mfma_f32_32x32x16_f16 a[0:15], v[4:7], v[8:11], a[0:15]", "s_nop 10", "v_accvgpr_read_b32 v0, a15"], "a15"),
+    (["v_mfma_f32_32x32x16_f16 a[0:15], v[4:7], v[8:11], a[0:15]", "s_nop 11", "v_accvgpr_read_b32 v0, a15"], None),
+    (["v_mov_b32_e32 v5, 0", "s_nop 0", MFMA, "s_nop 7"], "v5"), (["v_mov_b32_e32 v5, 0", "s_nop 1", MFMA, "s_nop 7"], None),
+    (["v_accvgpr_write_b32 a1, 0", MFMA, "s_nop 7"], "a1"), (["v_mov_b32_e32 v12, 0", MFMA, "s_nop 7"], None)])
+def test_wait_states_around_matrix_instructions_are_looked_for(tmp_path, code, hit):
+    found = B.wait_hazards(assembled(tmp_path, code))
+    assert [f[3] for f in found] == ([hit] if hit else [])
+
+
+def test_the_wait_states_are_the_compilers_own(tmp_path):
+    """The figures of build.py against what the compiler leaves around its own instructions: a source that needs every one of them
+    has no hazard, and would have with one state more."""
+    src, obj = tmp_path / "k.hip", str(tmp_path / "k.o")
+    src.write_text("""
+#include <hip/hip_runtime.h>
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+__global__ void read4(const v8h* p, v4f* o) { const v4f c = __builtin_amdgcn_mfma_f32_16x16x32_f16(p[threadIdx.x], p[64], o[threadIdx.x], 0, 0, 0); o[64 + threadIdx.x] = c + 1.f; }
+__global__ void read16(const v8h* p, v16f* o) { const v16f c = __builtin_amdgcn_mfma_f32_32x32x16_f16(p[threadIdx.x], p[64], o[threadIdx.x], 0, 0, 0); o[64 + threadIdx.x] = c + 1.f; }
+__global__ void write(const v8h* p, v4f* o) { const v8h a = p[threadIdx.x]; o[64 + threadIdx.x] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a + a, p[64], o[threadIdx.x], 0, 0, 0); }
+__global__ void scalar(const int* q, int* o) {
+  const int s = __builtin_amdgcn_readfirstlane(q[threadIdx.x]);
+  o[threadIdx.x] = __builtin_amdgcn_raw_buffer_load_b32(__builtin_amdgcn_make_buffer_rsrc((void*)q, 0, -1, 0x27000), threadIdx.x * 4, s, 0);
+}
+""")
+    subprocess.run(["/opt/rocm/bin/hipcc"] + [f for f in B.FLAGS if f != "-shared"] + ["-c", str(src), "-o", obj], check=True, capture_output=True)
+    assert B._of_every_code_object(B.wait_hazards, obj) == []
+    kept = B.MFMA_TO_READ, B.VALU_TO_MFMA, B.VALU_TO_VMEM
+    try:
+        B.MFMA_TO_READ = {k: v + 1 for k, v in kept[0].items()}
+        assert {f[2] for f in B._of_every_code_object(B.wait_hazards, obj)} == set(kept[0])
+        B.MFMA_TO_READ, B.VALU_TO_MFMA, B.VALU_TO_VMEM = kept[0], kept[1], kept[2] + 1
+        assert {f[4] for f in B._of_every_code_object(B.wait_hazards, obj)} == {"buffer_load_dword"}
+    finally:
+        B.MFMA_TO_READ, B.VALU_TO_MFMA, B.VALU_TO_VMEM = kept
+
+
 def test_no_kernel_of_the_library_reads_a_register_too_soon():
     if not os.path.exists(B.LIB):
         pytest.skip("the library is not built")
