@@ -206,9 +206,12 @@ def shift_hazards_of(path):
     return _of_every_code_object(shift_hazards, path)
 
 
+def _in_processes(check, path):                                       # (for what takes python itself long)
+    return _of_every_code_object(check, path, lambda n: ProcessPoolExecutor(n, multiprocessing.get_context("fork")))
+
+
 def wait_hazards_of(path):
-    # (python's own work: processes)
-    return _of_every_code_object(wait_hazards, path, lambda n: ProcessPoolExecutor(n, multiprocessing.get_context("fork")))
+    return _in_processes(wait_hazards, path)
 
 
 def static_lds_of(path):

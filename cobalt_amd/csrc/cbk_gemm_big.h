@@ -224,6 +224,34 @@ __device__ inline void gb_epilogue(const GbArgs& a, v4f (&acc)[2 * TI][8], uint8
   }
 }
 
+// The generic reader: block t (32 columns) of row wrc as halfs, into pieces c ... c + 3 of the weight tile's row at LDS address
+// `row` (swizzled with `sw`).  Long, and called from many places, so a function; it is given values and not, as a closure would,
+// the caller's variables, which would then live in memory around every call.
+static __device__ __attribute__((noinline)) void gb_generic_block(const DMat& m, const RowView rv, int wrc, bool wok, int t, uint32_t row,
+                                                                  uint32_t sw, uint32_t c) {
+  uint32_t packed[16];
+  if (wok) {
+    int q[32];
+    const uint32_t keep = decode_block32(m, rv, t, q);
+    const int g = (t * BLOCK) / m.group;
+    const float sc = h2f(m.scale[meta_index(m, wrc, g)]);
+    const float z = (float)m.zero[meta_index(m, wrc, g)];
+    const bool dense = family_of(m.layout) == FAM_DENSE;
+#pragma unroll
+    for (int p = 0; p < 32; p += 2) {
+      float v0 = __fmul_rn((float)q[p] - z, sc), v1 = __fmul_rn((float)q[p + 1] - z, sc);
+      if (!dense) { v0 = ((keep >> p) & 1u) ? v0 : 0.f; v1 = ((keep >> (p + 1)) & 1u) ? v1 : 0.f; }
+      packed[p >> 1] = (uint32_t)f2h(v0) | ((uint32_t)f2h(v1) << 16);
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) packed[e] = 0;
+  }
+#pragma unroll
+  for (uint32_t e = 0; e < 4; ++e)
+    *(__attribute__((address_space(3))) v4u*)(uintptr_t)(row + (sw ^ (c + e)) * 16u) = v4u{packed[4 * e], packed[4 * e + 1], packed[4 * e + 2], packed[4 * e + 3]};
+}
+
 // BITS 2 / 3 / 4: byte-permute decoder for (BITS, KEEP, GRP), KEEP = 0 for the dense layouts.
 // BITS 0: generic 32-column reader, any fixed-stride layout.
 // PAR 0: one col_scale vector.  1: gate/up matrix (GbArgs::par).  2: q|k|v matrix (GbArgs::vs0, vs1).
@@ -393,29 +421,9 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
     };
     if (!FASTD) {
       if ((b8 & 3) || piece) return;                              // the generic reader works on 32 columns
-      uint32_t packed[16];
-      if (wok) {
-        int q[32];
-        int t = ((s + s_begin) * GB_K >> 5) + (b8 >> 2);
-        t = t < (N >> 5) ? t : (N >> 5) - 1;
-        const uint32_t keep = decode_block32(m, rv, t, q);
-        const int g = (t * BLOCK) / m.group;
-        const float sc = h2f(m.scale[meta_index(m, wrc, g)]);
-        const float z = (float)m.zero[meta_index(m, wrc, g)];
-        const bool dense = family_of(m.layout) == FAM_DENSE;
-#pragma unroll
-        for (int p = 0; p < 32; p += 2) {
-          float v0 = __fmul_rn((float)q[p] - z, sc), v1 = __fmul_rn((float)q[p + 1] - z, sc);
-          if (!dense) { v0 = ((keep >> p) & 1u) ? v0 : 0.f; v1 = ((keep >> (p + 1)) & 1u) ? v1 : 0.f; }
-          packed[p >> 1] = (uint32_t)f2h(v0) | ((uint32_t)f2h(v1) << 16);
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) packed[e] = 0;
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        put(b8 + e, packed[4 * e], packed[4 * e + 1], packed[4 * e + 2], packed[4 * e + 3]);
+      const int t = ((s + s_begin) * GB_K >> 5) + (b8 >> 2);
+      gb_generic_block(m, rv, wrc, wok, t < (N >> 5) ? t : (N >> 5) - 1,
+                       (uint32_t)(uintptr_t)Ws + (uint32_t)buf * GB_WBUF + (uint32_t)tid * 128u, (uint32_t)tid & 7u, (uint32_t)b8);
       return;
     }
     const int blk = 2 * h + (b8 >> 2);                              // 32-column block of the chunk

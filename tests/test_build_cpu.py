@@ -168,3 +168,29 @@ def test_no_kernel_of_the_library_reads_a_register_too_soon():
     if not os.path.exists(B.LIB):
         pytest.skip("the library is not built")
     assert B.wait_hazards_of(B.LIB) == []
+
+
+def main_loop(body):
+    """Of a function's instructions, those of the loop with most matrix instructions."""
+    at = {b[0]: i for i, b in enumerate(body)}
+    loops = [body[at[b[3]]:i + 1] for i, b in enumerate(body) if b[3] in at and at[b[3]] < i]
+    return max(loops, key=lambda l: sum("mfma" in b[1] for b in l), default=[])
+
+
+def tile_loops(code_object):
+    return [(fn, [(b[1], b[2]) for b in main_loop(body)]) for fn, body in B._functions(code_object) if "gemm_big_kernel" in fn]
+
+
+@pytest.fixture(scope="module")
+def loops():
+    if not os.path.exists(B.LIB):
+        pytest.skip("the library is not built")
+    return dict(B._in_processes(tile_loops, B.LIB))
+
+
+def test_tile_kernels_keep_their_state_in_registers(loops):
+    """Every function named after one is a kernel with its matrix instructions in a loop: none calls a closure, which has its
+    variables in memory (as the generic reader did, a quarter of its time)."""
+    assert len(loops) > 300
+    assert [fn for fn, l in loops.items() if sum(op.startswith("v_mfma") for op, _ in l) not in (128, 256, 512)] == []
+    assert [fn for fn, l in loops.items() if any(op.startswith("scratch_") for op, _ in l)] == []
