@@ -366,8 +366,8 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
     uint32_t m[4];                       // bitmap
     uint32_t raw[C::NL];                 // code dwords as loaded (whole 16-byte units)
     uint32_t c[C::ND];                   // code bits, first bit of the chunk at bit 0
-    uint32_t z;                          // zero points of the chunk's groups, one per byte
-    float s[C::NGC];
+    uint32_t z[C::NGC];                  // zero points of the chunk's groups, and scales as loaded: nothing that needs
+    uint32_t s[C::NGC];                  // their values may stand beside the loads, where it would wait for them
     uint32_t ci;                         // chunk index the units were loaded for
     uint32_t h2[C::HI2 ? 4 : 1];         // BLK1632_6: high bit pairs, one dword per block
   };
@@ -394,11 +394,10 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
       w.h2[0] = v.x; w.h2[1] = v.y; w.h2[2] = v.z; w.h2[3] = v.w;
     }
     const size_t mi = meta0 + (size_t)c * C::NGC * meta_step;
-    w.z = m.zero[mi];
-    w.s[0] = h2f(m.scale[mi]);
-    if (C::NGC == 2) {
-      w.z |= (uint32_t)m.zero[mi + meta_step] << 8;
-      w.s[1] = h2f(m.scale[mi + meta_step]);
+#pragma unroll
+    for (int g = 0; g < C::NGC; ++g) {
+      w.z[g] = m.zero[mi + g * meta_step];
+      w.s[g] = m.scale[mi + g * meta_step];
     }
   };
 
@@ -429,9 +428,9 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
     const int blk = 2 * h + (b8 >> 2);                              // 32-column block of the chunk
     const int jj = b8 & 3;                                          // mask byte inside the block
     const int gi = C::NGC == 2 ? h : 0;                             // quantisation group of this stage
-    const _Float16 sh = (_Float16)(wok ? w.s[gi] : 0.f);
+    const _Float16 sh = __builtin_bit_cast(_Float16, (uint16_t)(wok ? w.s[gi] : 0u));
     const h2_t s2 = {sh, sh};
-    const uint32_t z = (w.z >> (8 * gi)) & 0xFFu;
+    const uint32_t z = w.z[gi];
     // eight codes (the zero point z for a pruned column) -> eight halfs (q - z) * scale: a code in the low byte of
     // 0x64xx is the half 1024 + q; the difference to 1024 + z is exact, the product rounds once
     const h2_t off2 = __builtin_bit_cast(h2_t, 0xE400E400u + z * 0x00010001u);

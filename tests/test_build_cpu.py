@@ -194,3 +194,25 @@ def test_tile_kernels_keep_their_state_in_registers(loops):
     assert len(loops) > 300
     assert [fn for fn, l in loops.items() if sum(op.startswith("v_mfma") for op, _ in l) not in (128, 256, 512)] == []
     assert [fn for fn, l in loops.items() if any(op.startswith("scratch_") for op, _ in l)] == []
+
+
+def waits(loop):
+    """(matrix instructions so far, loads since the barrier and whether one of those lies behind the last matrix instruction, the
+    count that is waited for, whether a barrier follows) of every wait for loads in a loop."""
+    mfma, loads, fresh, out = 0, 0, False, []
+    for i, (op, args) in enumerate(loop):
+        if op.startswith("v_mfma"):
+            mfma, fresh = mfma + 1, False
+        elif op == "s_barrier":
+            loads = 0
+        elif op.startswith("global_load"):
+            loads, fresh = loads + 1, True
+        elif op == "s_waitcnt" and "vmcnt" in args:
+            count = int(args[args.index("vmcnt(") + 6:].partition(")")[0])
+            out.append((mfma, loads, fresh, count, any(o == "s_barrier" for o, _ in loop[i:i + 4])))
+    return out
+
+
+def test_tile_kernels_do_not_wait_for_loads_where_they_issue_them(loops):
+    """A chunk of weights is loaded two stages before its use: nothing beside its loads may need what they load."""
+    assert [(fn, w) for fn, l in loops.items() for w in waits(l) if w[2] and w[3] < w[1]] == []
