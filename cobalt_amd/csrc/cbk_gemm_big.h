@@ -107,6 +107,12 @@ __device__ inline void dma_x16(v4u buffer, uint32_t voff, uint32_t soff, uint32_
   asm volatile("s_add_u32 m0, %3, %4\n\ts_nop %5\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
                ::"v"(voff), "s"(buffer), "s"(soff), "s"(lds), "i"(AT), "i"(SPILLS ? 4 : 0) : "memory", "m0", "scc");
 }
+// Waits for all of a wavefront's loads and direct copies, in a form that the compiler's own count of loads takes in: behind an assembly
+// statement it still holds its loads for outstanding, and at their first use waits for the copies issued since
+__device__ inline void wait_loads() {
+  __builtin_amdgcn_s_waitcnt(0x0F70);                               // vmcnt 0, the other counters at their largest
+  asm volatile("" ::: "memory");
+}
 // the same in every lane, in a scalar register
 __device__ inline uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 
@@ -541,7 +547,7 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
     decode_piece(0, wA, 0, 0, 7, 0, wA, 0); decode_piece(0, wA, 0, 0, 7, 1, wA, 0);
   }
   static_for<8 * PIECES>([&](auto d_) { decode_step(0, d_, wA, H0{}, wA, H1{}, 0); });
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  wait_loads();
   __syncthreads();
   if constexpr (DEEP) read_all(0, 0);
   else {
@@ -574,7 +580,7 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
         // (the weight chunk loads of the previous stage wait here as well: they were issued a
         // whole stage ago, and counting them out of the wait would rest on how many load
         // instructions the compiler keeps)
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        wait_loads();
         __syncthreads();
         if (LOADW) load_chunk(cl, wd);
       }
@@ -617,7 +623,7 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
   gb_mfma_done(acc);
   // the last stage issued copies of a stage that does not exist: let them land before the
   // epilogue reuses LDS
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  wait_loads();
   __syncthreads();
 
   const int tok0 = t0 + 32 * TI * wt, row0 = r0 + kstep * 128 * wr;

@@ -216,3 +216,11 @@ def waits(loop):
 def test_tile_kernels_do_not_wait_for_loads_where_they_issue_them(loops):
     """A chunk of weights is loaded two stages before its use: nothing beside its loads may need what they load."""
     assert [(fn, w) for fn, l in loops.items() for w in waits(l) if w[2] and w[3] < w[1]] == []
+
+
+def test_tile_kernels_wait_for_loads_at_their_barriers_only(loops):
+    """Four waits for everything in a trip of four stages, each before a barrier, and none that the compiler adds: such a one
+    would wait for the direct copies of the next stage."""
+    for fn, l in loops.items():
+        if "gemm_big_kernelILi0E" not in fn:                              # (calls of the generic reader wait for what they load)
+            assert [w[3:] for w in waits(l)] == [(0, True)] * 4, fn
