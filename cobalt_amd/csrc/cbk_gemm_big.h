@@ -412,7 +412,10 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
   // wavefront on a SIMD an instruction that waits for the one before it takes eight cycles and more, and of the rest two fit
   // beside a 16-cycle matrix instruction.  Pieces 0 and 1 fetch the table entry of the byte two ahead (half ha of chunk wa).
   constexpr int PIECES = 16;
-  constexpr bool CHAIN = C::NW <= 2 && !C::HI2;                     // the stream is shifted on from byte to byte
+  // The stream is shifted on from byte to byte, of three dwords as two 64-bit pieces (a byte's survivors take at most 32 bits): five
+  // shifts a block, 18 instructions fewer than windows at a running position (8192 x 5376, 4-bit, 23 of 32, 512 / 1024 / 2048 tokens on
+  // the 64- / 128- / 256-token tile: 104 / 120 / 166 -> 92 / 110 / 162 us).
+  constexpr bool CHAIN = !C::HI2;
   struct Sel { uint32_t x, y, full, bits; };
   Sel sel[4];                                                       // by byte mod 4
   uint32_t sel_at = 0;
@@ -459,8 +462,14 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
         if (!CHAIN) de.rank = jj == 0 ? 0u : jj == 1 ? n : de.rank + n;
         else if (jj && C::NW == 1) st[0] >>= n;
         else if (jj) {
-          const uint64_t v = (((uint64_t)st[C::NW - 1] << 32) | st[0]) >> n;
-          st[0] = (uint32_t)v; st[C::NW - 1] = (uint32_t)(v >> 32);
+          constexpr int B = C::NW > 1 ? 1 : 0, E = C::NW - 1;
+          const uint64_t v = (((uint64_t)st[B] << 32) | st[0]) >> n;
+          st[0] = (uint32_t)v;
+          if (C::NW == 2) st[B] = (uint32_t)(v >> 32);
+          else {
+            const uint64_t u = (((uint64_t)st[E] << 32) | st[B]) >> n;
+            st[B] = (uint32_t)u; st[E] = (uint32_t)(u >> 32);
+          }
         }
       }
     } else if (piece == 3) {

@@ -1,5 +1,6 @@
 """What the build looks for in the compiled kernels."""
 import os
+import re
 import subprocess
 
 import pytest
@@ -224,3 +225,16 @@ def test_tile_kernels_wait_for_loads_at_their_barriers_only(loops):
     for fn, l in loops.items():
         if "gemm_big_kernelILi0E" not in fn:                              # (calls of the generic reader wait for what they load)
             assert [w[3:] for w in waits(l)] == [(0, True)] * 4, fn
+
+
+def test_streams_of_three_dwords_are_shifted_on(loops):
+    """23 of 32 codes of four bits (three widened) fill three dwords.  Shifted on from byte to byte they take at most 30 vector
+    instructions a block (eight in a trip) more than the two dwords of 16 codes: reading, widening and shifting the third.  Windows at
+    a running position took 36 and 42."""
+    vector = {}
+    for fn, l in loops.items():
+        key = tuple(map(int, re.search(r"gemm_big_kernelILi(\d)ELi(\d+)ELi(\d+)ELi(\d)ELi(\d)E", fn).groups()))
+        vector[key] = sum(op.startswith("v_") and "mfma" not in op for op, _ in l)
+    for (bits, keep, group, vectors, tile), n in vector.items():
+        if keep == 23 and bits > 2:
+            assert n - vector[bits, 16, group, vectors, tile] <= 8 * 30, (bits, group, vectors, tile)
