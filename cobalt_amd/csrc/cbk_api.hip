@@ -665,6 +665,16 @@ void gemm_last_round(const cbk_desc* in, int M, const GemmChoice& c, int* row_ti
   *ti = r.ti;
 }
 
+void gemm_column_parts(const cbk_desc* in, int M, const GemmChoice& c, int* parts, int* first, int* rest) {
+  DMat m;
+  GbCut cut = {0, 0, 0};
+  if (M >= 1 && !to_dmat(in, &m, false)) {
+    const GemmPlan p = named_plan(m, M, c);
+    if (p.kernel == GEMM_TILE) cut = cut_big(m, p, M);
+  }
+  *parts = cut.nsplit; *first = cut.first; *rest = cut.part;
+}
+
 size_t gemm_as_workspace_bytes(const cbk_desc* in, int M, const GemmChoice& c, int act, int y_dtype) {
   DMat m;
   if (M < 1 || to_dmat(in, &m, false)) return 0;

@@ -679,7 +679,10 @@ static int launch_big_par(const GbArgs& a, int blocks, hipStream_t st) {
 template <int BITS, int KEEP, int GRP, int TI>
 static int launch_big_ti(const GbArgs& a, int blocks, hipStream_t st) {
   if (a.par) return launch_big_par<BITS, KEEP, GRP, 1, TI>(a, blocks, st);
-  if (a.nsplit > 1) return launch_big_par<BITS, KEEP, GRP, 3, TI>(a, blocks, st);
+  if (a.nsplit > 1) {
+    if constexpr (BITS == 0) return CBK_ERR_UNSUPPORTED;             // (the generic reader's launches are never split)
+    else return launch_big_par<BITS, KEEP, GRP, 3, TI>(a, blocks, st);
+  }
   if (a.vs0 != 0x7fffffff) return launch_big_par<BITS, KEEP, GRP, 2, TI>(a, blocks, st);
   return launch_big_par<BITS, KEEP, GRP, 0, TI>(a, blocks, st);
 }

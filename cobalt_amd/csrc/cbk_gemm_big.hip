@@ -177,21 +177,20 @@ static int gb_part(const DMat& m, int nsplit) {
   const int nst = gb_npad(m.N) / GB_K, per = ((nst + nsplit - 1) / nsplit + 3) / 4 * 4;
   return nsplit > 1 && (nsplit - 1) * per >= nst ? 0 : per;
 }
-// The parts of a launch whose plan is `nsplit` parts of `tiles` tiles.  They are equal, but where a plan cuts 129 tiles or more
+// The parts of a launch whose plan is `nsplit` parts of `tiles` tiles.  They are equal, but where a plan cuts 129 to 192 tiles
 // in n >= 3 parts to fill n - 1 rounds: there two parts may do, the first ones, a workgroup each on its CU from the start,
 // so long that the CUs without one need as long for all the second ones.  The same CU time with fewer partial tiles, and a
 // workgroup's start and end less for most.  Workgroups go to the eight XCDs in turn and to the four shader engines of one in turn, and stay there:
 // it is the eight CUs of an engine that share its second parts (168 tiles, 228 + 108 stages, as 256 CUs would
 // share them: three turns instead of two, 5376 x 21504 at 2048 tokens 447 -> 574 us).  Equal and unequal parts, us, with preparation
 // and reduction: 160 tiles 5120 x 20480 426 -> 408, 4096 x 14336 320 -> 307; 144 tiles 4608 x 18432 374 -> 360; 192 tiles
-// 6144 x 24576 578 -> 552.
+// 6144 x 24576 578 -> 552.  Above 192 tiles one CU of an engine would run seven second parts in turn: equal parts.
 // (The plan does not count it: calls keep their kernel and room.)
-struct GbCut { int nsplit, first, part; };
 static GbCut gb_cut(const DMat& m, int tiles, int ti, int nsplit) {
   const int per = gb_part(m, nsplit), nst = gb_npad(m.N) / GB_K;
   GbCut c = {nsplit, per, per};
   const int held = ((tiles + 7) / 8 + 3) / 4, left = 8 - held;      // CUs of a shader engine with and without a first part
-  if (nsplit < 3 || tiles <= 128 || left < 1) return c;
+  if (nsplit < 3 || tiles <= 128 || left < 2) return c;
   const double t_stage = gb_t_stage(ti), t_wg = gb_t_wg(ti);
   const int turns = (held + left - 1) / left;                       // second parts of a CU without a first one
   double best = (double)((tiles * nsplit + 255) / 256) * (per * t_stage + t_wg);
@@ -279,6 +278,10 @@ LastRound last_round_big(const DMat& m, const GemmPlan& p, int M) {
   return LastRound();
 }
 
+GbCut cut_big(const DMat& m, const GemmPlan& p, int M) {            // (only unsplit plans have a last round of their own)
+  return gb_cut(m, (M + 64 * p.ti - 1) / (64 * p.ti) * gb_row_tiles(m), p.ti, p.nsplit);
+}
+
 static int gb_launch(const GbArgs& a, hipStream_t st) {
   const DMat& m = a.m;
   const int tiles = a.tiles_t * a.tiles_r;
@@ -336,7 +339,7 @@ int launch_gemm_big(const DMat& m, const GemmPlan& plan, const void* x, int xdt,
   a.tiles_t = (M + T - 1) / T;
   const LastRound tail = last_round_big(m, plan, M);
   a.tiles_r = gb_row_tiles(m) - tail.rows;
-  const GbCut cut = gb_cut(m, a.tiles_t * a.tiles_r, plan.ti, plan.nsplit);
+  const GbCut cut = cut_big(m, plan, M);
   a.nsplit = cut.nsplit; a.nst_first = cut.first; a.nst_part = cut.part;
   int rc = gb_launch(a, st);
   if (rc == CBK_OK && tail.rows) {

@@ -25,6 +25,10 @@ GemmPlan fixed_plan_big(const DMat&, int M, int ti, int nsplit);
 // The row tiles of a plan of 256-token tiles that run as smaller tiles (64 ti tokens) in a launch of their own; rows 0: none.
 struct LastRound { int rows = 0, ti = 0; };
 LastRound last_round_big(const DMat&, const GemmPlan&, int M);
+// The column parts of a launch of the tile kernel: nsplit of them, in 64-column stages `first` for the first and `part` for
+// each further one (the last takes what is left).
+struct GbCut { int nsplit, first, part; };
+GbCut cut_big(const DMat&, const GemmPlan&, int M);
 // What the tile kernel takes with every q|k|v matrix in one piece (see gemm_room in cbk_api.hip).
 size_t big_unsplit_space(const DMat&, int M);
 bool gemm_skinny_takes(const DMat&);

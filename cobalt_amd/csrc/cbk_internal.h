@@ -21,6 +21,7 @@ int decode_choice(int n, const cbk_desc* descs, int M, DecodeChoice*);   // CBK_
 struct GemmChoice { int kernel, ti, nsplit; };
 GemmChoice gemm_choice(const cbk_desc*, int M, int act);
 void gemm_last_round(const cbk_desc*, int M, const GemmChoice&, int* row_tiles, int* ti);   // of such a call: LastRound in cbk_gemm_plan.h
+void gemm_column_parts(const cbk_desc*, int M, const GemmChoice&, int* parts, int* first, int* rest);   // of such a call: GbCut there; parts 0: not that kernel's
 size_t gemm_as_workspace_bytes(const cbk_desc*, int M, const GemmChoice&, int act, int y_dtype);   // 0: it cannot be run so
 int gemm_as(const cbk_desc*, const GemmChoice&, const void* x, int x_dtype, int M, int64_t ldx, void* y, int y_dtype, int64_t ldy,
             const void* bias, int act, void* workspace, size_t workspace_bytes, void* stream);

@@ -326,6 +326,20 @@ PyObject* py_gemm_last_round(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// gemm_column_parts(matrix, M, kernel, ti, nsplit) -> (parts, stages of the first, of a further one); see cbk::gemm_column_parts
+PyObject* py_gemm_column_parts(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (!arity(n, 5)) return nullptr;
+  return guarded([&]() -> PyObject* {
+    const cbk_desc d = desc_of(as_matrix(a[0]));
+    const long M = PyLong_AsLong(a[1]);
+    const cbk::GemmChoice c{(int)PyLong_AsLong(a[2]), (int)PyLong_AsLong(a[3]), (int)PyLong_AsLong(a[4])};
+    if (PyErr_Occurred()) throw Fail{};
+    int parts, first, rest;
+    cbk::gemm_column_parts(&d, (int)M, c, &parts, &first, &rest);
+    return Py_BuildValue("iii", parts, first, rest);
+  });
+}
+
 // gemm_as(matrix, x, bias, out_dtype, kernel, ti, nsplit, act or -1) -> y; see cbk::gemm_as
 PyObject* py_gemm_as(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!arity(n, 8)) return nullptr;
@@ -560,6 +574,7 @@ PyMethodDef methods[] = {
     {"gemv_batch", (PyCFunction)(void (*)())py_gemv_batch, METH_FASTCALL, nullptr},
     {"decode_choice", (PyCFunction)(void (*)())py_decode_choice, METH_FASTCALL, nullptr},
     {"gemm_plan", (PyCFunction)(void (*)())py_gemm_plan, METH_FASTCALL, nullptr},
+    {"gemm_column_parts", (PyCFunction)(void (*)())py_gemm_column_parts, METH_FASTCALL, nullptr},
     {"gemm_last_round", (PyCFunction)(void (*)())py_gemm_last_round, METH_FASTCALL, nullptr},
     {"gemm_as", (PyCFunction)(void (*)())py_gemm_as, METH_FASTCALL, nullptr},
     {"dequant", (PyCFunction)(void (*)())py_dequant, METH_FASTCALL, nullptr},

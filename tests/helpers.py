@@ -98,3 +98,8 @@ def last_round(pm, M, kernel, tokens, nsplit=1):
     """(row tiles, tokens) of the second launch such a call ends with; (0, 0): it is one launch."""
     rows, ti = _lib.native().gemm_last_round(pm.native(), M, KERNELS[kernel], tokens // (32 if kernel == "rows" else 64), nsplit)
     return rows, 64 * ti
+
+
+def column_parts(pm, M, tokens, nsplit):
+    """(parts, 64-column stages of the first, of each further one) of such a call on the tile kernel."""
+    return _lib.native().gemm_column_parts(pm.native(), M, KERNELS["tile"], tokens // 64, nsplit)

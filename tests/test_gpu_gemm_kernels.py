@@ -2,11 +2,13 @@
 (plain, gate/up, q|k|v) x split of the column range x byte order, for activations of both signs and of one.
 Against float64 on the dequantised weights, held to the error of operands of 11 bits in exact sums (2 % for
 float32 sums and the draw); every call twice, bit for bit."""
+import ctypes
+
 import pytest
 import torch
 
 from cobalt_amd import _lib, format as F, ops
-from helpers import TOKENS, acts, case_id, gemm_as, gemm_plan, last_round
+from helpers import TOKENS, acts, case_id, column_parts, gemm_as, gemm_plan, last_round
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -162,13 +164,17 @@ def test_a_plain_call_is_the_call_its_plan_names():
 
 
 @pytest.mark.parametrize("tokens", [64, 128, 256])
-@pytest.mark.parametrize("row_tiles,parts,N", [(9, 3, 1536), (10, 3, 1664), (12, 4, 2048)])
-def test_columns_in_two_unequal_parts(row_tiles, parts, N, tokens):
-    """144, 160 and 192 tiles whose plan is three or four parts run as a long and a short one (the last
+@pytest.mark.parametrize("row_tiles,token_tiles,parts,N,runs", [(9, 16, 3, 1536, 2), (10, 16, 3, 1664, 2), (12, 16, 4, 2048, 2),
+                                                                (11, 13, 3, 1664, 2), (13, 13, 3, 1664, 2), (13, 15, 4, 4096, 4)])
+def test_columns_in_two_unequal_parts(row_tiles, token_tiles, parts, N, runs, tokens):
+    """144, 160, 192, 143 and 169 tiles (the last two no multiple of the XCDs) whose plan is three or four parts run as a long and a
+    short one, 195 tiles as four equal ones (the last
     tiles ragged on both sides, a padded last chunk of columns).  Operands are rounded to 2^-12 twice: 3e-4, as everywhere on this
     kernel; against the unsplit call only the order of float32 sums differs."""
-    K, M = 256 * row_tiles - 7, 16 * tokens - 5
+    K, M = 256 * row_tiles - 7, token_tiles * tokens - 5
     pm = F.synth_packed(K, N, F.BLK1632_4, 4, 128, 16, seed=row_tiles, device=DEV).to_tiled()
+    ran, first, rest = column_parts(pm, M, tokens, parts)
+    assert ran == runs and ((first > rest) if runs == 2 else (first == rest)), (ran, first, rest)
     x = acts(M, N, torch.float16, seed=tokens).to(DEV)
     y = gemm_as(pm, x, "tile", tokens, parts, out_dtype=torch.float32).double()
     ref = x.double() @ ops.dequant(pm, torch.float32).double().t()
@@ -193,3 +199,44 @@ def test_rows_of_y_that_start_anywhere(K, tokens):
     assert float((y.double() - ref).norm() / ref.norm()) < 5e-4
     for dt in (torch.float16, torch.bfloat16):
         assert torch.equal(gemm_as(pm, x, "tile", tokens, out_dtype=dt), y.to(dt)), dt
+
+
+@pytest.mark.parametrize("half", [256, 260, 262, 263])
+def test_halves_that_start_anywhere(half):
+    """A gate/up call on the tile kernel leaves its up outputs `half` elements behind its gate outputs.  Each half is the
+    plain product of its matrix, bit for bit; the activation of those, rounded once (float32: an exponential and two divisions)."""
+    N, M = 512, 293
+    rounded = {torch.float16: 1.01 * 2 ** -11, torch.bfloat16: 1.01 * 2 ** -8, torch.float32: 4e-6}   # significands of 11 and 8 bits
+    parts = [F.synth_packed(half, N, F.BLK1632_4, 4, 128, 16, seed=half + s, device=DEV) for s in (0, 1)]
+    pm = F.fuse_rows(parts, interleave=True).to_tiled()
+    x = acts(M, N, torch.float16, seed=half).to(DEV)
+    for tokens in TOKENS["tile"]:
+        for dt in (torch.float16, torch.bfloat16, torch.float32):
+            g, u = (gemm_as(p.to_tiled(), x, "tile", tokens, out_dtype=dt) for p in parts)
+            both = torch.stack((g, u), -1).view(M, 2 * half)
+            assert torch.equal(gemm_as(pm, x, "tile", tokens, out_dtype=dt), both), (tokens, dt)
+            ref = torch.nn.functional.silu(g.double()) * u.double()
+            err = (gemm_as(pm, x, "tile", tokens, out_dtype=dt, act="silu").double() - ref).abs()
+            assert bool((err <= rounded[dt] * ref.abs() + 1e-7).all()), (tokens, dt)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("at,pitch", [(0, 0), (1, 0), (2, 8), (8, 0), (8, 8), (0, (1 << 22) - 8200), (0, (1 << 22) - 8192)],
+                         ids=["as it is", "one element on", "two", "a piece", "a piece and wider", "32-bit offsets end", "and past it"])
+def test_y_that_starts_anywhere(dtype, at, pitch):
+    """y from any element on, rows any distance apart: the same outputs, and nothing else written.  8192 outputs of 520 tokens
+    at strides below and from 4 M elements, where a tile's offsets no longer fit 32 bits."""
+    K, N, M = 8192, 512, 520
+    pm = F.synth_packed(K, N, F.BLK1632_4, 4, 128, 16, seed=3, device=DEV).to_tiled()
+    assert gemm_plan(pm, M)[0] == "tile"
+    x = acts(M, N, torch.float16, seed=3).to(DEV)
+    ref = ops.gemm(pm, x, out_dtype=dtype)
+    ld = K + pitch
+    y = torch.full((M * ld + 16,), 7.0, dtype=dtype, device=DEV)
+    d, L = pm.desc(), _lib.lib()
+    ws = torch.empty(L.cbk_workspace_bytes(ctypes.byref(d), M), dtype=torch.uint8, device=DEV)
+    _lib.check(L.cbk_gemm(ctypes.byref(d), x.data_ptr(), F.dtype_code(x.dtype), M, N, y.data_ptr() + at * y.element_size(), F.dtype_code(dtype), ld,
+                          None, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream), "cbk_gemm")
+    rows = y[at:at + M * ld].view(M, ld)
+    assert torch.equal(rows[:, :K], ref)
+    assert bool((rows[:, K:] == 7).all()) and bool((y[:at] == 7).all()) and bool((y[at + M * ld:] == 7).all())
