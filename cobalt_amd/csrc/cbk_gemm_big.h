@@ -258,6 +258,24 @@ static __device__ __attribute__((noinline)) void gb_generic_block(const DMat& m,
     *(__attribute__((address_space(3))) v4u*)(uintptr_t)(row + (sw ^ (c + e)) * 16u) = v4u{packed[4 * e], packed[4 * e + 1], packed[4 * e + 2], packed[4 * e + 3]};
 }
 
+// Code stream of 32-column block jb of a chunk (block_stream in cbk_decode.h).  3-bit codes are widened by three shifts and three
+// selects, which leaves bits of a neighbour above every code; a dense block takes them off with the mask that it needs
+// anyway (CODES), a bitmap's rank 7 has none.  Few instructions less, but a shorter chain, which shows where a block has three dwords
+// or four (8192 x 5376, 512 tokens on the 64-token tile: dense 80.7 -> 75.3 us, group 64 80.1 -> 77.3; 23 of 32 100 -> 96, 103 -> 97) and not
+// where it has two (10 of 32 88.4 -> 91.3, 16 of 32 86.5 -> 88.6: those keep the general form).
+template <class C, int BITS>
+__device__ inline void gb_block_stream(const uint32_t (&cw)[C::ND], int jb, uint32_t (&st)[C::NW]) {
+  if (BITS != 3 || C::NW < 3) { block_stream<C, BITS>(cw, jb, st); return; }
+#pragma unroll
+  for (int k = 0; k < C::NW; ++k) {
+    uint32_t x = get32<C::ND>(cw, jb * C::CB + 24 * k);
+    x = mask_select(0x00000FFFu, x << 4, x);
+    x = mask_select(0x003F003Fu, x << 2, x);
+    x = mask_select(0x07070707u, x << 1, x);
+    st[k] = C::DENSE ? x : x & 0x77777777u;
+  }
+}
+
 // BITS 2 / 3 / 4: byte-permute decoder for (BITS, KEEP, GRP), KEEP = 0 for the dense layouts.
 // BITS 0: generic 32-column reader, any fixed-stride layout.
 // PAR 0: one col_scale vector.  1: gate/up matrix (GbArgs::par).  2: q|k|v matrix (GbArgs::vs0, vs1).
@@ -412,6 +430,7 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
   // wavefront on a SIMD an instruction that waits for the one before it takes eight cycles and more, and of the rest two fit
   // beside a 16-cycle matrix instruction.  Pieces 0 and 1 fetch the table entry of the byte two ahead (half ha of chunk wa).
   constexpr int PIECES = 16;
+  constexpr uint32_t CODES = BITS == 3 ? 0x07070707u : C::SB == 4 ? 0x0F0F0F0Fu : 0x03030303u;
   // The stream is shifted on from byte to byte, of three dwords as two 64-bit pieces (a byte's survivors take at most 32 bits): five
   // shifts a block, 18 instructions fewer than windows at a running position (8192 x 5376, 4-bit, 23 of 32, 512 / 1024 / 2048 tokens on
   // the 64- / 128- / 256-token tile: 104 / 120 / 166 -> 92 / 110 / 162 us).
@@ -445,7 +464,7 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
     const h2_t off2 = __builtin_bit_cast(h2_t, 0xE400E400u + z * 0x00010001u);
     if (piece == 0) {
       if (h == 0 && b8 == 0) align_chunk_codes<C>(w.raw, w.ci, w.c);  // once per chunk, at its first use
-      if (jj == 0) block_stream<C, BITS>(w.c, blk, st);               // once per block
+      if (jj == 0) gb_block_stream<C, BITS>(w.c, blk, st);            // once per block
       if (BITMAP) {
         const int ja = 8 * ha + ((b8 + 2) & 7);                       // mask byte of the chunk, 0..15
         // byte ja % 4 of the mask dword, times 128 bytes per entry, plus the base
@@ -478,7 +497,7 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
     } else if (piece == 4) {
       if (C::SB == 2) { const uint32_t lo16 = de.win & 0xFFFFu; de.win = (lo16 << 14) | lo16; }   // bytes c0 c4 c1 c5; four bits up c2 c6 c3 c7
     } else if (piece == 5) {
-      de.p0 = de.win & (C::SB == 4 ? 0x0F0F0F0Fu : 0x03030303u);      // even codes (of two bits: c0 c4 c1 c5)
+      de.p0 = de.win & CODES;                                         // even codes (of two bits: c0 c4 c1 c5)
       de.t = de.win >> 4;
     } else if (piece == 6) {
       // p0 | p1: the codes of the survivors from this byte's first on, even and odd ranks (four bits), or 0 2 .. and 4 6 ..
@@ -492,7 +511,7 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
       }
     } else if (piece == 7) {
       if (BITMAP) de.p1 = (de.t & sel[b8 & 3].full) | ((z << 24) & ~sel[b8 & 3].full);
-      else de.p1 = de.t & (C::SB == 4 ? 0x0F0F0F0Fu : 0x03030303u);
+      else de.p1 = de.t & CODES;
     } else if (piece == 8) {
       de.b0 = perm(de.p1, de.p0, BITMAP ? sel[b8 & 3].x : C::SB == 4 ? 0x05010400u : 0x06040200u);
       de.b1 = perm(de.p1, de.p0, BITMAP ? sel[b8 & 3].y : C::SB == 4 ? 0x07030602u : 0x07050301u);
