@@ -28,8 +28,13 @@
 // for the one before, and two fit beside a matrix instruction of 16 cycles.  So the decode is counted in
 // instructions (an entry's address is one four-byte dot product of the mask dword, the entry holds what
 // would be counted or compared, codes stay unsigned until the exact subtraction of 1024 + zero point, a
-// pruned column reads the zero point from the place of the eighth survivor) and dealt out by hand, at most
-// two independent ones beside each matrix instruction: 4-bit, 16 of 32: 1.4 per matrix instruction.
+// pruned column reads the zero point from the place of the eighth survivor) and dealt out by hand, two independent
+// ones beside a matrix instruction; but what a chunk and a block take once (the alignment and widening of their codes) and the
+// high bit pairs of 6-bit codes stand in one place, up to forty.  Vector instructions per matrix instruction of the 256-token tile: 4-bit,
+// 16 of 32 1.2, dense 1.1, 3-bit 23 of 32 2.0, 6-bit 2.3; of the 128- and 64-token tiles two and four times that, and there
+// they bind.  (The 64-token tile in 32 x 32 blocks, half as many products: with the same decode 0.5 to 2 % slower in the mean of 24 decoders.
+// Over these, plain, gate/up, q|k|v and split, 8192 x 5376: the 256- / 128- / 64-token tile 1.07 - 1.12 / 1.04 - 1.10 / 1.00 - 1.07 times as
+// fast in the mean as the kernel with 32 x 32 blocks throughout, on five boxes.)
 //
 // What bounds it: power.  The clock falls with the load: a loop of nothing but these matrix instructions on
 // halves, half of one operand zeros, runs at 2.08 PFLOP/s, of v_mfma_f32_32x32x16_f16 (a fourth of the sums moved per
@@ -37,7 +42,7 @@
 // 8192 rows (one tile on every CU), 4-bit, 16 of 32, one box: 181 us with 32 x 32 blocks and the decode left to the
 // compiler's interleave, 169 now, 141 with the decode taken out, 119 with the matrix instructions alone (266, 196 and 183
 // thousand cycles of the loop at about 1.6 GHz).  Gated block of 21504 x 5376 at 2048 tokens with both its products
-// 1421 -> 1346 us.
+// 1421 -> 1346 us; since the wait before a barrier is one that the compiler counts (wait_loads) 1.6 % less again.
 //
 // Workgroups are ordered so that those running at the same time on one XCD (blockIdx % 8)
 // share their token tile, which then stays in that XCD's L2.
@@ -296,8 +301,8 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(GbArgs a) {
   using C = CodeCfg<FASTD ? BITS : 4, KEEP, FASTD ? GRP : 128>;
   constexpr bool BITMAP = FASTD && !C::DENSE;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  // Xs [2][GB_T][64 halfs], Ws [2][GB_R][64 halfs]: row r, logical 16-byte piece c at physical piece c ^ ((r >> 1) & 7).
-  // A 16-byte read or write goes through LDS in sets of sixteen lanes, 0-3 12-15 20-27 and so on: with the fragments' rows
+  // Xs [2][GB_T][64 halfs], Ws [2][GB_R][64 halfs]: row r, logical 16-byte piece c at physical piece c ^ ((r >> 1) & 7),
+  // of Ws at c ^ (r & 7).  A 16-byte read or write goes through LDS in sets of sixteen lanes, 0-3 12-15 20-27 and so on: with the fragments' rows
   // (l % 16) and pieces (l / 16) as with one piece of 64 rows, a set's pieces so lie in different banks.  (Rows padded to
   // 144 bytes, which serve fragments of 32 rows and one piece, triple the conflicts of the call: 14 -> 43 million cycles.)
   _Float16* Xs = (_Float16*)smem;

@@ -154,13 +154,15 @@ static bool gb_fast(const DMat& m) {
 //    take the 256-token tile unless the model below gives the 128-token tile the shorter time,
 //    which it does for small matrices (4096 x 4096 at 256 to 2048 rows: 16 to 128 tiles of 256
 //    tokens): twice the tiles, each 0.8 of the time.
-// Times in microseconds from measurements of this kernel: per 64-column stage 1.1 / 1.35 / 1.7
-// for the three tiles (the 64-token stage is bound by the weight loads' latency), 8 - 10 per
-// workgroup outside the stage loop, 4 TB/s for the partial tiles, 5 for the reduction kernel.  (With 1.25 and 7 TB/s,
-// which fit a few small calls better, 4096 x 4096 at 2048 rows went from 92 to 104 us, 3840 x 7424 at 1024 from 89 to
-// 98.)  Over 24 measured calls
-// (eight shapes, 256 / 512 / 2048 rows) the choice is within 2 % of the faster tile; always
-// taking the 256-token tile loses 6 % on average and up to 34 %.
+// Times in microseconds, as measured when the kernel had 32 x 32 x 16 instructions: per 64-column stage 1.1 / 1.35 / 1.7
+// for the three tiles, 8 - 10 per workgroup outside the stage loop, 4 TB/s for the partial tiles, 5 for the reduction kernel.  (With 1.25 and
+// 7 TB/s, which fit a few small calls better, 4096 x 4096 at 2048 rows went from 92 to 104 us, 3840 x 7424 at 1024 from 89 to
+// 98.)  Over 24 calls measured then
+// (eight shapes, 256 / 512 / 2048 rows) the choice was within 2 % of the faster tile; always
+// taking the 256-token tile lost 6 % on average and up to 34 %.
+// The present kernel, a tile on every CU without a pause: 4-bit, 16 of 32 0.84 / 1.09 / 1.77; dense 0.73 - 0.89 / 1.00 - 1.22 /
+// 1.52 - 1.95; 3-bit, 23 of 32 1.09 / 1.31 / 1.94; 6-bit 1.04 / 1.32 / 1.98; outside the loop 5 - 14.  So the model takes the
+// smaller tiles for up to a third slower than they are and knows no code width.
 static inline double gb_t_stage(int ti) { return ti == 1 ? 1.1 : ti == 2 ? 1.35 : 1.7; }
 static inline double gb_t_wg(int ti) { return ti == 1 ? 8.0 : 10.0; }
 static inline size_t gb_kpad(int K) { return (size_t)(K + 7) / 8 * 8; }
