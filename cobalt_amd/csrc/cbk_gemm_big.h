@@ -34,7 +34,7 @@
 // 16 of 32 1.2, dense 1.1, 3-bit 23 of 32 2.0, 6-bit 2.3; of the 128- and 64-token tiles two and four times that, and there
 // they bind.  (The 64-token tile in 32 x 32 blocks, half as many products: with the same decode 0.5 to 2 % slower in the mean of 24 decoders.
 // Over these, plain, gate/up, q|k|v and split, 8192 x 5376: the 256- / 128- / 64-token tile 1.07 - 1.12 / 1.04 - 1.10 / 1.00 - 1.07 times as
-// fast in the mean as the kernel with 32 x 32 blocks throughout, on five boxes.)
+// fast in the mean as the kernel with 32 x 32 blocks throughout, on five GPUs.)
 //
 // What bounds it: power.  The clock falls with the load: a loop of nothing but these matrix instructions on
 // halves, half of one operand zeros, runs at 2.08 PFLOP/s, of v_mfma_f32_32x32x16_f16 (a fourth of the sums moved per
