@@ -182,7 +182,7 @@ def wait_hazards(code_object):
 
 
 # Kernels whose table reads take an entry's offset in dynamic LDS as its address: nothing else may lie before it.
-LDS_FROM_ZERO = ("gemm_skinny_kernel",)
+LDS_FROM_ZERO = ("gemm_skinny_kernel", "gemv_mfma_kernel", "gemv_split_kernel")
 
 
 def static_lds(code_object):

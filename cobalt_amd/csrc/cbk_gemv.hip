@@ -3,16 +3,17 @@
 // Idea.  At 8 TB/s and ~3 bits per weight the chip must consume ~20e12 weights per second,
 // which leaves about two vector-ALU instructions per weight: a per-weight convert + FMA
 // dequantiser cannot keep up.  So the weights stay integers.  Every lane decodes 128
-// consecutive columns of ONE weight row into signed bytes (q - zero for a kept column, 0
-// for a pruned one) sixteen at a time, and hands each 16-byte fragment to
+// consecutive columns of ONE weight row into signed bytes (a code less 128 for a kept column, the
+// zero point less 128 for a pruned one) sixteen at a time, and hands each 16-byte fragment to
 // v_mfma_i32_16x16x64_i8 as the B operand.  The A operand is the activation vector in
 // block fixed point: per 128-column chunk, x' = x * col_scale is written as
 // delta * (65536*d2 + 256*d1 + d0) with three int8 digits (|x' - delta*X| <= max|x'| / 2^24,
 // i.e. float32 resolution relative to the largest activation of the chunk; 8-bit codes: four
 // digits, see digits_of).  The
 // matrix core produces exact int32 dot products per (row, chunk, digit); one float FMA per
-// row and quantisation group applies scale * delta.  A pruned column multiplies a literal
-// zero byte, so it contributes exactly 0 whatever the zero point holds.
+// row and quantisation group applies scale * delta, after (128 - zero) times the sum of the group's
+// digits, integers too, has been added.  A pruned column's byte is the zero point's, so its two shares
+// cancel exactly and it contributes 0 whatever the zero point holds.
 //
 // Work decomposition.  A wavefront owns a tile of 16 weight rows; lane l works on row l%16
 // and on the 128-column chunk 4*S + l/16 of macro-step S (512 columns).  The four lane
@@ -35,9 +36,10 @@
 //
 // Expansion of the bitmap.  For one mask byte (8 columns, r survivors before it in its
 // 32-column block) the survivor codes r .. r+7 are shifted out of the block's code bits,
-// spread to one code per byte (two dwords = the 8-byte pool of v_perm_b32), biased to
-// q - zero, and v_perm_b32 with a selector from a 256-entry table (indexed by the mask
-// byte) drops each survivor into its column and a constant 0 into every pruned column.
+// spread to one code per byte less 128 (two dwords = the 8-byte pool of v_perm_b32), and
+// v_perm_b32 with a selector from a 256-entry table (indexed by the mask byte) drops each
+// survivor into its column and the pool's last byte, the zero point less 128 unless all eight
+// columns are kept, into every pruned column.
 //
 // Reference semantics: cbk::gemv_blk1632_multi / gemv_dense4_multi
 // (src/cobaltkernel/csrc/cobalt_gemv.cuh:617-712, :839-1123): same sums, other machinery.
@@ -55,7 +57,7 @@ constexpr int GV_THREADS = GV_WAVES * 64;
 constexpr int LUT_LANES = CBK_LUT_LANES;      // lane-private copies of the selector table
 constexpr int LUT_BYTES = 256 * LUT_LANES * 8;
 constexpr int WIDE_LUT_LANES = 16, WIDE_LUT_BYTES = 256 * WIDE_LUT_LANES * 16;   // see fetch_selectors
-constexpr int ZERO_BYTES = 256;
+constexpr int ZERO_BYTES = 128;               // a chunk of a digit row
 constexpr int CNT_SLOTS = 64;                 // most reduction slots (arrival counters)
 constexpr int CNT_BYTES = CNT_SLOTS * 4;       // at a fixed place: zeroed before the arguments are read
 constexpr int X_LDS_BUDGET = 112 * 1024;      // activation digits of one row: 3 (8-bit codes: 4) * columns bytes (of 160 KB LDS)
@@ -158,6 +160,31 @@ __host__ __device__ constexpr int digit_order(int bits, bool dense) { return !de
 // eight threads of a chunk agree on its maximum with three lane exchanges.
 struct XLoad { uint4 x[2], c[2]; };
 
+// What the end of a quantisation group reads of an activation row, three digits: the sum P of X = 65536 d2 + 256 d1 + d0 over the group
+// and the chunk's delta, [row][group of the slab], whole macro-steps (chunks past N: zeros).  Quarter-per-block: P as P >> 8 and P & 255, in
+// sixteen bytes.
+template <bool QB> constexpr int REC_BYTES = QB ? 16 : 8;
+__host__ __device__ constexpr int rec_stride(int cols, int group) { return (cols / 128 + 3) / 4 * 4 * (128 / group); }
+// Bytes between two digit rows.  Linear order (quarter-per-chunk), or whole macro-steps of 512 columns in the order of the quarters 0, 2,
+// 1, 3 (quarter-per-block): a read of sixteen bytes goes through LDS in sets of sixteen lanes, 0-3 12-15 20-27 and so on, which
+// mix the quarters 0 and 1 or 2 and 3 of all twelve digit rows; 256 bytes apart, and rows 16 bytes off 256, no two of a set meet in a
+// bank (in linear order two did in every set: 72 of 264 LDS cycles of a step at eight rows).
+template <bool QB>
+__host__ __device__ constexpr int x_stride(int cols) { return (QB ? (cols + 511) / 512 * 512 : cols) + X_PAD; }
+// offset of the sixteen columns c16 of a slab in a digit row
+template <bool QB>
+__device__ inline int x_place(int c16) {
+  return QB ? (c16 >> 5) * 512 + (c16 & 2) * 128 + (c16 & 4) * 32 + (c16 & 24) * 4 + (c16 & 1) * 16 : c16 * 16;
+}
+// LDS bytes of an activation row's digits, and what is set aside for them with the records, for `cols` columns (a multiple of 128)
+static inline size_t x_digit_bytes(int bits, int cols) { return (size_t)digits_of(bits) * (cols + X_PAD); }
+static inline size_t x_row_bytes(int bits, int group, int cols, int M) {
+  return digits_of(bits) * (size_t)(M == 1 ? x_stride<false>(cols) : x_stride<true>(cols)) +
+         (bits == 8 ? 0 : rec_stride(cols, group) * (M == 1 ? REC_BYTES<false> : REC_BYTES<true>));
+}
+// 8-bit codes have their deltas alone, of all chunks of M rows: floats
+static inline int delta_floats(const DMat& m, int M) { return m.bits == 8 ? M * (m.N / 128 + 4) : 0; }
+
 // global loads of staging item `it` of the column slab that starts at column col0 and is n16 * 16
 // columns wide (activation row it / n16, columns col0 + 16 * (it % n16) ...)
 __device__ inline void stage_load(const uint16_t* x, int64_t ldx, const uint16_t* cs, int N, int col0, int n16, int it,
@@ -180,10 +207,11 @@ __device__ inline void stage_load(const uint16_t* x, int64_t ldx, const uint16_t
 // ND = 4: x' = delta * (2^24 d3 + ...) with delta a power of two, 2^29 of them to the power of two at or below the largest: products
 // with the column scale are represented as they are, down to 2^-6 of it, and to 2^-30 of it below that.
 // HALVES (groups of 64): the delta of a chunk with infinities says which half has them, see group_delta.
-template <int ORDER, int ND = NDIG, bool HALVES = false>
+// SUMG (64 or 128, three digits only): the group size; what a group's end reads goes to `recs`, and nothing to `delta`.
+template <int ORDER, int ND = NDIG, bool HALVES = false, int SUMG = 0, bool QB = false>
 __device__ inline void stage_convert(const XLoad& r, bool has_cs, int xdt, int N, int ch0, int n16, int it, bool one_row,
-                                     int8_t* xq, float* delta, int pad = 0) {
-  const int NCH = N >> 7, Ns = n16 * 16 + pad;
+                                     int8_t* xq, float* delta, int pad = 0, void* recs = nullptr) {
+  const int NCH = N >> 7, Ns = QB ? x_stride<true>(n16 * 16) : n16 * 16 + pad;
   const int row = one_row ? 0 : it / n16, c16 = it - row * n16;
   const uint32_t* xw = (const uint32_t*)r.x;
   const uint32_t* cw = (const uint32_t*)r.c;
@@ -239,38 +267,58 @@ __device__ inline void stage_convert(const XLoad& r, bool has_cs, int xdt, int N
   // (X = d0 + 256 d1 + 65536 d2, -128 <= d < 128), so the digits of four columns are byte
   // permutes of the four biased integers and one xor per digit plane
   uint32_t dw[ND][4];
-  uint32_t xb[16];
-#pragma unroll
-  for (int bi = 0; bi < 16; ++bi) {
-    const float v = ORDER == 0 ? xv[bi] : ORDER == 1 ? xv[frag_col(4, true, bi)] : xv[frag_col(2, true, bi)];
-    // ND 3: |X| <= 127 * 65536 (+ 2 from the rounding of inv); ND 4: |X| < 2^30
-    int X = (int)rintf(v * inv);
-    // A NaN makes delta one.  An infinity makes delta infinite and has +-1 for a digit (several in a chunk: their sum)
-    if (ND == 4 && none) X = fabsf(v) == mx ? (v > 0.f ? 1 : -1) : 0;
-    xb[bi] = (uint32_t)X + (ND == 4 ? 0x80808080u : 0x808080u);
-  }
+  uint32_t sum = 0u - 16u * 0x808080u;                              // SUMG: of X
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
+    uint32_t xb[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int bi = 4 * q + i;
+      const float v = ORDER == 0 ? xv[bi] : ORDER == 1 ? xv[frag_col(4, true, bi)] : xv[frag_col(2, true, bi)];
+      // ND 3: |X| <= 127 * 65536 (+ 2 from the rounding of inv); ND 4: |X| < 2^30
+      int X = (int)rintf(v * inv);
+      // A NaN makes delta one.  An infinity makes delta infinite and has +-1 for a digit (several in a chunk: their sum)
+      if (ND == 4 && none) X = fabsf(v) == mx ? (v > 0.f ? 1 : -1) : 0;
+      xb[i] = (uint32_t)X + (ND == 4 ? 0x80808080u : 0x808080u);
+    }
     if constexpr (ND == 4) {
-      const uint32_t a = perm(xb[4 * q + 1], xb[4 * q], 0x05010400u), a2 = perm(xb[4 * q + 1], xb[4 * q], 0x07030602u);
-      const uint32_t b = perm(xb[4 * q + 3], xb[4 * q + 2], 0x05010400u), b2 = perm(xb[4 * q + 3], xb[4 * q + 2], 0x07030602u);
+      const uint32_t a = perm(xb[1], xb[0], 0x05010400u), a2 = perm(xb[1], xb[0], 0x07030602u);
+      const uint32_t b = perm(xb[3], xb[2], 0x05010400u), b2 = perm(xb[3], xb[2], 0x07030602u);
       dw[0][q] = perm(b2, a2, 0x07060302u) ^ 0x80808080u;
       dw[1][q] = perm(b2, a2, 0x05040100u) ^ 0x80808080u;
       dw[2][q] = perm(b, a, 0x07060302u) ^ 0x80808080u;
       dw[ND - 1][q] = perm(b, a, 0x05040100u) ^ 0x80808080u;
-      continue;
+    } else {
+      const uint32_t a = perm(xb[1], xb[0], 0x05010400u);               // d0 d0 d1 d1 of columns 0, 1
+      const uint32_t b = perm(xb[3], xb[2], 0x05010400u);               // and of columns 2, 3
+      const uint32_t c01 = perm(xb[1], xb[0], 0x0C0C0602u);             // d2 d2 0 0
+      const uint32_t c23 = perm(xb[3], xb[2], 0x06020C0Cu);             // 0 0 d2 d2
+      dw[0][q] = (c01 | c23) ^ 0x80808080u;
+      dw[1][q] = perm(b, a, 0x07060302u) ^ 0x80808080u;
+      dw[2][q] = perm(b, a, 0x05040100u) ^ 0x80808080u;
+      if constexpr (SUMG != 0) sum += (xb[0] + xb[1]) + (xb[2] + xb[3]);
     }
-    const uint32_t a = perm(xb[4 * q + 1], xb[4 * q], 0x05010400u);       // d0 d0 d1 d1 of columns 0, 1
-    const uint32_t b = perm(xb[4 * q + 3], xb[4 * q + 2], 0x05010400u);   // and of columns 2, 3
-    const uint32_t c01 = perm(xb[4 * q + 1], xb[4 * q], 0x0C0C0602u);     // d2 d2 0 0
-    const uint32_t c23 = perm(xb[4 * q + 3], xb[4 * q + 2], 0x06020C0Cu); // 0 0 d2 d2
-    dw[0][q] = (c01 | c23) ^ 0x80808080u;
-    dw[1][q] = perm(b, a, 0x07060302u) ^ 0x80808080u;
-    dw[2][q] = perm(b, a, 0x05040100u) ^ 0x80808080u;
+    if constexpr (QB) __builtin_amdgcn_sched_barrier(0);            // (four columns at a time: registers)
   }
 #pragma unroll
   for (int k = 0; k < ND; ++k)
-    *(uint4*)(xq + ((size_t)row * ND + k) * Ns + c16 * 16) = make_uint4(dw[k][0], dw[k][1], dw[k][2], dw[k][3]);
+    *(uint4*)(xq + ((size_t)row * ND + k) * Ns + x_place<QB>(c16)) = make_uint4(dw[k][0], dw[k][1], dw[k][2], dw[k][3]);
+  if constexpr (SUMG != 0) {                                        // |P| <= 128 * 127 * 65536 and a little
+    static_assert(ND == 3, "three digits");
+    constexpr int PG = SUMG / 16, NGC = 128 / SUMG;
+    int P = (int)sum;
+    P += __builtin_amdgcn_mov_dpp(P, 0xB1, 0xF, 0xF, true);
+    P += __builtin_amdgcn_mov_dpp(P, 0x4E, 0xF, 0xF, true);
+    if (SUMG == 128) P += __builtin_amdgcn_mov_dpp(P, 0x141, 0xF, 0xF, true);
+    const int rs = rec_stride(n16 * 16, SUMG), r0 = row * rs, past = rs - n16 / PG;
+    auto put = [&](int g, int p, float dl) {
+      if (QB) ((int4*)recs)[r0 + g] = make_int4(p >> 8, p & 255, __float_as_int(dl), 0);
+      else ((int2*)recs)[r0 + g] = make_int2(p, __float_as_int(dl));
+    };
+    if ((c16 & (PG - 1)) == 0) put(c16 / PG, P, d);
+    if (past > 0 && c16 < past) put(n16 / PG + c16, 0, 0.f);
+    return;
+  }
   if (HALVES && none && mx == __builtin_inff())                     // (the writing lane is one of the first half)
     d = here != mx ? -3.4028234663852886e38f : there != mx ? -mx : mx;
   if ((c16 & 7) == 0) delta[row * (NCH + 4) + ch0 + (c16 >> 3)] = d;
@@ -324,16 +372,15 @@ __device__ inline float wave_sum_dpp(float v) {
 }
 
 // ------------------------------------------------------------------ one 32-column block
-// mask bytes of a block and the number of survivors before each of them
+// The eight-byte pool of a permute in the bitmap layouts: BIAS in every byte takes 128 off a code
 template <class C>
-__device__ inline void split_mask(uint32_t mw, uint32_t (&mb)[4], uint32_t (&rk)[4]) {
-  if (!C::DENSE) {
-    mb[0] = mw & 0xFFu; mb[1] = __builtin_amdgcn_ubfe(mw, 8, 8); mb[2] = __builtin_amdgcn_ubfe(mw, 16, 8); mb[3] = mw >> 24;
-    rk[0] = 0; rk[1] = (uint32_t)__builtin_popcount(mb[0]);
-    rk[2] = rk[1] + (uint32_t)__builtin_popcount(mb[1]); rk[3] = rk[2] + (uint32_t)__builtin_popcount(mb[2]);
+struct Pool {
+  static constexpr uint32_t BIAS = 0x80808080u;
+  static __device__ inline uint32_t full(uint32_t mb) {
+    constexpr uint32_t f = C::HI2 ? 0x00FFFFFFu : C::SB == 4 ? 0x000F0F0Fu : 0x00030303u;
+    return mb == 255u ? f | 0xFF000000u : f;
   }
-}
-
+};
 template <bool WT>
 __device__ inline uint32_t table_lane(int lane) {                   // offset of this lane's copy in an entry
   return WT ? (uint32_t)(lane & (WIDE_LUT_LANES - 1)) * 16u : (uint32_t)(lane & (LUT_LANES - 1)) * 8u;
@@ -344,98 +391,156 @@ __device__ inline void build_table(uint8_t* lut, int tid) {
   if (C::DENSE) return;
   if (WT && tid >= GV_THREADS - 256) {
     const uint32_t mb = (uint32_t)tid & 255u;
-    const uint2 e = make_selectors(mb, C::SEL_KIND);
-    const uint4 w = make_uint4(e.x, e.y, (uint32_t)__builtin_popcount(mb) * C::SB, 0u);
+    const uint2 e = make_selectors<0x07070707u>(mb, C::SEL_KIND);
+    const uint4 w = make_uint4(e.x, e.y, Pool<C>::full(mb), (uint32_t)__builtin_popcount(mb) * C::SB);
 #pragma unroll
     for (int j = 0; j < WIDE_LUT_LANES; ++j) ((uint4*)lut)[table_slot<WIDE_LUT_LANES, 16>(mb, j)] = w;
   } else if (!WT && tid < 256) {
-    const uint2 e = make_selectors((uint32_t)tid, C::SEL_KIND);
+    const uint2 e = make_selectors<0x07070707u>((uint32_t)tid, C::SEL_KIND);
 #pragma unroll
     for (int j = 0; j < LUT_LANES; ++j) ((uint2*)lut)[table_slot<LUT_LANES, 8>(tid, j)] = e;
   }
 }
 
-// Table reads of one block: selectors, and in `sh` the bits of the code stream before each mask byte.
-// WT: the wide table, 16-byte entries of selectors and the stream bits of the byte's survivors, 256 bytes (sixteen
-// copies) apart, so that one permute of mask word and lane offset is an entry's address and the counting is done by
-// the table.  The small one has 8-byte entries, eight copies: an address takes a field extract and a shift and add,
-// the counts a population count and a shift.  Gate and up of 21504 x 5376 (BLK1632_4, one row, weights from memory), small
-// and wide: 290 and 277 vector instructions per step of 16 rows x 512 columns, 2.3 and 0.7 million LDS bank conflicts, a
-// wavefront's life 35.8 and 34.8 thousand cycles, 23.8 and 22.6 us; 14336 x 4096, 3-bit keep 10: 438 and 429
-// instructions, 16.0 and 15.3 us.  Two layers of 5376 / 21504 columns 112.3 -> 110.6 us.  (Launches that are long
-// enough take it: launch_main_batch, launch_split_batch.)
+// Table reads of half a block.  WT: the wide table, 16-byte entries, 256 bytes (sixteen copies) apart, so that one permute of mask
+// word and lane offset is an entry's address, and mask and count are the table's.  The small one has 8-byte entries, eight copies: an address
+// takes a field extract and a shift and add, the count a population count and a shift, the mask a comparison and a
+// select.  (Launches that are long enough take the wide one: launch_main_batch, launch_split_batch.)
+// Read by LDS address: the table is the first thing in LDS and nothing is added to an entry's offset (the build refuses static LDS).
+template <typename T>
+__device__ inline T lds_at(uint32_t at) { return *(const __attribute__((address_space(3))) T*)(uintptr_t)at; }
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+struct Sel {
+  uint32_t x, y;       // selectors of the eight columns; a pruned column reads the last byte of the pool
+  uint32_t full;       // the bits of the pool's second half that are codes: rank 7's byte only if all eight columns are kept
+  uint32_t bits;       // what the byte's survivors take in the code stream
+};
 template <class C, bool WT>
-__device__ inline void fetch_selectors(uint32_t mw, const uint8_t* lut, uint32_t lane_off, uint32_t (&sh)[4], uint2 (&sel4)[4]) {
+__device__ inline void fetch_selectors(uint32_t mw, uint32_t lane_off, int half, Sel (&sel)[2]) {
+  if constexpr (C::DENSE) return;
   if constexpr (WT) {
-    sh[0] = 0;
 #pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {                                // mask byte in byte 1, this lane's copy in byte 0
-      const uint4 e = *(const uint4*)(lut + perm(mw, lane_off, 0x0C0C0400u + ((uint32_t)jj << 8)));
-      sel4[jj] = make_uint2(e.x, e.y);
-      if (jj < 3) sh[jj + 1] = sh[jj] + e.z;
+    for (int j = 0; j < 2; ++j) {                                   // mask byte in byte 1, this lane's copy in byte 0
+      const v4u e = lds_at<v4u>(perm(mw, lane_off, 0x0C0C0400u + ((uint32_t)(2 * half + j) << 8)));
+      sel[j] = Sel{e[0], e[1], e[2], e[3]};
     }
   } else {
-    uint32_t mb[4], rk[4];
-    split_mask<C>(mw, mb, rk);
-    if (!C::DENSE) {
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        sel4[jj] = *(const uint2*)(lut + mb[jj] * (LUT_LANES * 8) + lane_off);
-        sh[jj] = rk[jj] * C::SB;
-      }
+    for (int j = 0; j < 2; ++j) {
+      const uint32_t mb = __builtin_amdgcn_ubfe(mw, 16 * half + 8 * j, 8);
+      const v2u e = lds_at<v2u>(mb * (LUT_LANES * 8) + lane_off);
+      sel[j] = Sel{e[0], e[1], Pool<C>::full(mb), (uint32_t)__builtin_popcount(mb) * C::SB};
     }
   }
 }
 
-// Sixteen columns (half `half` of the block whose code stream is st) as signed bytes q - zero,
-// pruned columns 0: the B operand of one MFMA.
-// sel4: the selectors of the block's four mask bytes, read from the table by fetch_selectors.
+// align_chunk_codes with a 24-bit multiplication (a chunk's index is below 2^13)
+template <class C>
+__device__ inline void gv_align_codes(const uint32_t (&raw)[C::NL], uint32_t chunk, uint32_t (&cw)[C::ND]) {
+  if constexpr (C::VEC16) align_chunk_codes<C>(raw, chunk, cw);
+  else skew_dwords<C::NL, C::ND, C::ALIGNED>(raw, (uint32_t)__umul24(chunk, (uint32_t)C::CHB) & 127u, cw);
+}
+
+// Code stream of 32-column block jb of a chunk; 3-bit codes widened to nibbles by three shifts and selects, which leave
+// bits of a neighbour above every code: the dense pools take them off with the mask they need anyway.
 template <class C, int BITS>
-__device__ inline void decode_half(const uint32_t (&st)[C::NW], const uint32_t (&sh)[4], const uint2 (&sel4)[4],
-                                   uint32_t nz, int half, uint32_t (&bfrag)[4], uint32_t hw = 0) {
+__device__ inline void gv_block_stream(const uint32_t (&cw)[C::ND], int jb, uint32_t (&st)[C::NW]) {
+  if constexpr (BITS != 3) block_stream<C, BITS>(cw, jb, st);
+  else
+#pragma unroll
+    for (int k = 0; k < C::NW; ++k) {
+      uint32_t x = get32<C::ND>(cw, jb * C::CB + 24 * k);
+      x = mask_select(0x00000FFFu, x << 4, x);
+      x = mask_select(0x003F003Fu, x << 2, x);
+      x = mask_select(0x07070707u, x << 1, x);
+      st[k] = C::DENSE ? x : x & 0x77777777u;
+    }
+}
+
+// Sixteen columns (half `half` of the block whose code stream is st) as signed bytes, the B operand of one MFMA.  Dense
+// layouts: the codes.  Bitmap layouts: codes less 128, and in a pruned column the zero point less 128, which is put in the place of
+// the eighth survivor (`zero`: that byte, and what Pool<C>::BIAS is in the others).  So no weight has its zero point taken off: the
+// sums are put right by (128 - zero), or -zero, times the sum of the group's digits (group_value), and are the same integers.
+// What bounds the kernel is the issue of vector instructions; the zero point off every pool, two instructions for each of its two
+// halves, was the part of them that the sums can carry.  The layers of a decode step that take the wide table gain (one row, 16 x
+// 4096 x 14336 and the others of such a layer, see the table of calls); a matrix of a few steps per wavefront at five
+// to eight rows pays for the sums without a gain.
+// The stream is shifted on by what a byte's survivors took of it, so halves are decoded in order; `taken` is their sum (6-bit codes).
+template <class C, int BITS>
+__device__ inline void decode_half(uint32_t (&st)[C::NW], uint32_t& taken, const Sel (&sel)[2], uint32_t zero, uint32_t bias, int half,
+                                   uint32_t (&bfrag)[4], uint32_t hw = 0) {
   if constexpr (BITS == 8) {                             // q - 128; the zero point is a second operand (zero8)
 #pragma unroll
     for (int k = 0; k < 4; ++k) bfrag[k] = st[4 * half + k] ^ 0x80808080u;
     return;
   }
+  constexpr uint32_t CODE = C::SB == 2 ? 0x03030303u : BITS == 3 ? 0x07070707u : 0x0F0F0F0Fu;
 #pragma unroll
   for (int jj2 = 0; jj2 < 2; ++jj2) {
     const int jj = 2 * half + jj2;                       // mask byte inside the block
-    uint32_t p0, p1;
-    if (C::DENSE) {
-      if (C::SB == 4) {
-        const uint32_t w = st[jj];
-        p0 = bias_pool(w & 0x0F0F0F0Fu, nz);
-        p1 = bias_pool((w >> 4) & 0x0F0F0F0Fu, nz);
-      } else {                                           // 2-bit: 16 codes per dword
-        const uint32_t w = st[half] >> (4 * jj2);
-        p0 = bias_pool(w & 0x03030303u, nz);
-        p1 = bias_pool((w >> 2) & 0x03030303u, nz);
-      }
-      bfrag[2 * jj2] = p0; bfrag[2 * jj2 + 1] = p1;
+    if constexpr (C::DENSE) {
+      const uint32_t w = C::SB == 4 ? st[jj] : st[half] >> (4 * jj2);     // 2-bit: 16 codes per dword
+      bfrag[2 * jj2] = w & CODE; bfrag[2 * jj2 + 1] = (w >> C::SB) & CODE;
     } else {
-      uint32_t w;
-      if (jj == 0) w = st[0];
-      else w = window<C::NW>(st, sh[jj]);
-      if (C::HI2) {
+      // the pool: its second half's top byte has no code bits of a neighbour above rank 7
+      uint32_t w = st[0];
+      if constexpr (C::SB == 2) { const uint32_t lo16 = w & 0xFFFFu; w = (lo16 << 14) | lo16; }
+      uint32_t p0, p1;
+      if constexpr (C::HI2) {
         uint32_t h0, h1;
-        hi2_pools(hw, jj == 0 ? 0u : sh[jj] / C::SB, h0, h1);
-        p0 = bias_pool((w & 0x0F0F0F0Fu) | h0, nz);
-        p1 = bias_pool(((w >> 4) & 0x0F0F0F0Fu) | h1, nz);
-      } else if (C::SB == 4) {
-        p0 = bias_pool(w & 0x0F0F0F0Fu, nz);
-        p1 = bias_pool((w >> 4) & 0x0F0F0F0Fu, nz);
+        hi2_pools(hw, jj == 0 ? 0u : taken / C::SB, h0, h1);
+        taken = jj == 0 ? sel[0].bits : taken + sel[jj2].bits;
+        p0 = (w & CODE) | (h0 | bias);
+        p1 = ((w >> 4) & CODE) | (h1 | bias);
       } else {
-        const uint32_t lo16 = w & 0xFFFFu;
-        const uint32_t t2 = (lo16 << 14) | lo16;
-        p0 = bias_pool(t2 & 0x03030303u, nz);
-        p1 = bias_pool((t2 >> 4) & 0x03030303u, nz);
+        p0 = (w & CODE) | bias;
+        p1 = __builtin_amdgcn_alignbit(Pool<C>::BIAS >> 28, w, 4);
       }
-      const uint2 sel = sel4[jj];
-      bfrag[2 * jj2] = perm(p1, p0, sel.x);
-      bfrag[2 * jj2 + 1] = perm(p1, p0, sel.y);
+      p1 = mask_select(sel[jj2].full, zero, p1);
+      bfrag[2 * jj2] = perm(p1, p0, sel[jj2].x);
+      bfrag[2 * jj2 + 1] = perm(p1, p0, sel[jj2].y);
+      if (jj < 3) {                                      // past this byte's survivors
+        const uint32_t n = sel[jj2].bits;
+        if constexpr (C::NW == 1) st[0] >>= n;
+        else {
+          constexpr int E = C::NW - 1;
+          const uint64_t v = (((uint64_t)st[1] << 32) | st[0]) >> n;
+          st[0] = (uint32_t)v;
+          if constexpr (C::NW == 2) st[1] = (uint32_t)(v >> 32);
+          else {
+            const uint64_t u = (((uint64_t)st[E] << 32) | st[1]) >> n;
+            st[1] = (uint32_t)u; st[E] = (uint32_t)(u >> 32);
+          }
+        }
+      }
     }
   }
+}
+// The byte of a pruned column, as decode_half takes it
+template <class C>
+__device__ inline uint32_t zero_byte(uint32_t z) { return C::DENSE ? 0u : (Pool<C>::BIAS & 0x00FFFFFFu) | ((z ^ 0x80u) << 24); }
+// The value of a group from its digit sums, which become those of codes less zero point z (p8, p0: P >> 8 and P & 255 of its record)
+template <class C>
+__device__ inline float group_value(const v4i& acc, int p8, int p0, uint32_t z) {
+  const int f = (C::DENSE ? 0 : 128) - (int)z;
+  return fmaf((float)(acc[0] * 256 + acc[1] + __mul24(p8, f)), 256.f, (float)(acc[2] + __mul24(p0, f)));
+}
+// What lane n of each sixteen holds; n is a constant after unrolling
+__device__ inline int row_lane(int v, int n) {
+  switch (n) {
+#define CBK_ROW_LANE(N) case N: return __builtin_amdgcn_mov_dpp(v, 0x150 + N, 0xF, 0xF, true);
+    CBK_ROW_LANE(0) CBK_ROW_LANE(1) CBK_ROW_LANE(2) CBK_ROW_LANE(3) CBK_ROW_LANE(4) CBK_ROW_LANE(5) CBK_ROW_LANE(6) CBK_ROW_LANE(7)
+    CBK_ROW_LANE(8) CBK_ROW_LANE(9) CBK_ROW_LANE(10) CBK_ROW_LANE(11) CBK_ROW_LANE(12) CBK_ROW_LANE(13) CBK_ROW_LANE(14)
+#undef CBK_ROW_LANE
+    default: return __builtin_amdgcn_mov_dpp(v, 0x15F, 0xF, 0xF, true);
+  }
+}
+// Pool<C>::BIAS in a register of its own: and-or with two literals is two instructions
+__device__ inline uint32_t bias_register() {
+  uint32_t b = 0x80808080u;
+  asm("" : "+v"(b));
+  return b;
 }
 
 // 8-bit codes: q - z needs nine bits, so the matrix instruction gets q - 128 and, in two more, the two halves of
@@ -543,7 +648,7 @@ __device__ inline void load_chunk(const StepAt& p, int S4, int kq, Loads<C>& L) 
       L.raw[4 * i] = v.x; L.raw[4 * i + 1] = v.y; L.raw[4 * i + 2] = v.z; L.raw[4 * i + 3] = v.w;
     }
   } else {
-    const uint32_t u = (((uint32_t)S4 + chl) * (uint32_t)C::CHB) >> 7;
+    const uint32_t u = __umul24((uint32_t)S4 + chl, (uint32_t)C::CHB) >> 7;
     const uint32_t voff = p.lane_off + (u << p.ush);
 #pragma unroll
     for (int i = 0; i < C::NL / 4; ++i) {
@@ -564,9 +669,9 @@ __device__ inline void load_chunk(const StepAt& p, int S4, int kq, Loads<C>& L) 
 // mask, 12 to 24 of a step's ~ 350 instructions.  (A pass of quarter-per-chunk per row, five to eight rows in two
 // launches, 3-bit codes, 10 of 32 kept: 21504 x 5376 23.4 -> 21.3 us at M = 4, 45.6 -> 23.0 at M = 8; 5376 x 21504, rows
 // split by columns now, 35.2 -> 19.6 and 69.5 -> 21.4.)
-struct XDigits { uint32_t xq_off, z_off; const float* delta; int Ns, ch0, NCH, M; };   // staged digits and deltas
+struct XDigits { uint32_t xq_off, z_off, rec_off; const float* delta; int Ns, ch0, NCH, M; };   // staged digits and what goes with them
 template <class C, int BITS, int NG, bool TURN, bool WT>
-__device__ inline void block_step(const Loads<C>& cur, const uint8_t* smem, const uint8_t* lut, uint32_t lane_off, int lane, int S,
+__device__ inline void block_step(const Loads<C>& cur, uint32_t lane_off, uint32_t bias, int lane, int S,
                                   const XDigits& x, float (&ysum)[4 * NG]) {
   constexpr int NGC = C::NGC, ND = digits_of(BITS);
   const int wr = lane & 15, kq = lane >> 4;
@@ -575,10 +680,10 @@ __device__ inline void block_step(const Loads<C>& cur, const uint8_t* smem, cons
   if constexpr (TURN) {
     uint32_t cw[C::ND];
     const int chunk = 4 * S + kq;
-    align_chunk_codes<C>(cur.raw, (uint32_t)(chunk < x.NCH ? chunk : x.NCH - 1), cw);
+    gv_align_codes<C>(cur.raw, (uint32_t)(chunk < x.NCH ? chunk : x.NCH - 1), cw);
 #pragma unroll
     for (int jb = 0; jb < 4; ++jb) {
-      block_stream<C, BITS>(cw, jb, st4[jb]);
+      gv_block_stream<C, BITS>(cw, jb, st4[jb]);
       mk4[jb] = C::DENSE ? 0u : cur.mk[jb];
       hw4[jb] = cur.h2[C::HI2 ? jb : 0];
     }
@@ -587,59 +692,61 @@ __device__ inline void block_step(const Loads<C>& cur, const uint8_t* smem, cons
     if (!C::DENSE) transpose4(mk4[0], mk4[1], mk4[2], mk4[3]);
     if (C::HI2) transpose4(hw4[0], hw4[1], hw4[2], hw4[3]);
   }
-  uint32_t zs[4][NGC];                                              // zero | scale << 8 of the groups of the chunks 4S .. 4S+3
+  uint32_t own[NGC];                                                // zero | scale << 8 of the groups of chunk 4S + kq
 #pragma unroll
-  for (int g = 0; g < NGC; ++g) {
-    const uint32_t own = ((cur.zraw >> (8 * g)) & 0xFFu) | (cur.sc[g] << 8);
-#pragma unroll
-    for (int c = 0; c < 4; ++c) zs[c][g] = (uint32_t)__shfl((int)own, wr + 16 * c, 64);
-  }
-  // row group g holds activation rows 4g .. 4g+3: its A operand, and in the result lane
-  // quarter kq the three digit sums of activation row 4g + kq
-  bool a_on[NG];
-  uint32_t a_base[NG];
-  int dm[NG];                                                       // the activation rows this quarter sums
+  for (int g = 0; g < NGC; ++g) own[g] = ((cur.zraw >> (8 * g)) & 0xFFu) | (cur.sc[g] << 8);
+  // Row group g holds activation rows 4g .. 4g + 3: its A operand (for a digit or row there is not, any other: nothing reads those
+  // rows of the result), in groups of 64 that of each half, zeros in the other two quarters
+  uint32_t aaddr[NG][NGC];
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
-    a_on[g] = a_dig < ND && a_m + 4 * g < x.M;
-    a_base[g] = x.xq_off + (uint32_t)(((a_m + 4 * g) * ND + a_dig) * (x.Ns + X_PAD) + kq * 32);
-    dm[g] = kq + 4 * g < x.M ? kq + 4 * g : 0;
+    const int am = a_m + 4 * g < x.M ? a_m + 4 * g : 0, ad = a_dig < ND ? a_dig : ND - 1;
+    const uint32_t a = x.xq_off + (uint32_t)((am * ND + ad) * x_stride<true>(x.Ns) + (kq & 1) * 256 + (kq >> 1) * 128) + (uint32_t)(4 * S - x.ch0) * 128u;
+#pragma unroll
+    for (int h = 0; h < NGC; ++h) aaddr[g][h] = NGC == 1 || (kq >> 1) == h ? a : x.z_off;
   }
+  // The records of the step's groups: in the result lane quarter kq holds the three digit sums of activation rows 4g + kq, and lane n of
+  // its sixteen fetches record n of (chunk, g, half).  Groups of 64 fetch those of a chunk when it ends, for want of registers.
+  constexpr int RC = NGC == 1 ? 4 : 1;                              // chunks at a time
+  auto fetch_rec = [&](int c) -> v4i {
+    if constexpr (BITS == 8) return v4i{0, 0, 0, 0};
+    const int n = wr & (RC * NG * NGC - 1), g = NG == 2 ? (n / NGC) & 1 : 0, am = kq + 4 * g < x.M ? kq + 4 * g : 0;
+    return lds_at<v4i>(x.rec_off + (uint32_t)(am * rec_stride(x.Ns, 128 / NGC) + (4 * S - x.ch0 + n / (NG * NGC)) * NGC + n % NGC) * 16u + (uint32_t)(c * NGC * 16));
+  };
+  v4i rec;
+  if constexpr (RC == 4) rec = fetch_rec(0);
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     const int chunk = 4 * S + c;
-    uint32_t aaddr[NG][NGC];
+    uint32_t zs[NGC];
 #pragma unroll
-    for (int g = 0; g < NG; ++g)
-#pragma unroll
-      for (int h = 0; h < NGC; ++h)
-        aaddr[g][h] = (a_on[g] && chunk < x.NCH && (NGC == 1 || (kq >> 1) == h)) ? a_base[g] + (uint32_t)(chunk - x.ch0) * 128u : x.z_off;
-    uint32_t shc[4];
-    uint2 selc[4];
-    fetch_selectors<C, WT>(TURN ? mk4[c] : cur.mk[c], lut, lane_off, shc, selc);
+    for (int g = 0; g < NGC; ++g) zs[g] = (uint32_t)__shfl((int)own[g], wr + 16 * c, 64);
+    uint32_t taken = 0;
     uint32_t st[C::NW];
 #pragma unroll
     for (int k = 0; k < C::NW; ++k) {
       if constexpr (TURN) st[k] = st4[c][k];
       else st[k] = cur.raw[c * C::NW + k];
     }
-    const uint32_t z = (NGC == 1 || kq < 2 ? zs[c][0] : zs[c][NGC - 1]) & 0xFFu;
-    const uint32_t nz = 0x80808080u - z * 0x01010101u;
+    const uint32_t z = (NGC == 1 || kq < 2 ? zs[0] : zs[NGC - 1]) & 0xFFu;
     v4i acc[NG][NGC];
 #pragma unroll
     for (int g = 0; g < NG; ++g)
 #pragma unroll
-      for (int h = 0; h < NGC; ++h) acc[g][h] = (v4i){0, 0, 0, 0};
+      for (int h = 0; h < NGC; ++h)
+        acc[g][h] = (v4i){0, 0, 0, 0};
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       uint32_t bfrag[4];
-      decode_half<C, BITS>(st, shc, selc, nz, half, bfrag, TURN && C::HI2 ? hw4[c] : 0u);
+      Sel sel[2];
+      fetch_selectors<C, WT>(TURN ? mk4[c] : cur.mk[c], lane_off, half, sel);
+      decode_half<C, BITS>(st, taken, sel, zero_byte<C>(z), bias, half, bfrag, TURN && C::HI2 ? hw4[c] : 0u);
       const v4i bv = (v4i){(int)bfrag[0], (int)bfrag[1], (int)bfrag[2], (int)bfrag[3]};
 #pragma unroll
       for (int g = 0; g < NG; ++g)
 #pragma unroll
         for (int h = 0; h < NGC; ++h) {
-          const v4i av = *(const v4i*)(smem + aaddr[g][h] + 16 * half);
+          const v4i av = lds_at<v4i>(aaddr[g][h] + 32 * c + 16 * half);
           acc[g][h] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bv, acc[g][h], 0, 0, 0);
           asm("s_nop 1" : "+v"(acc[g][h]));                         // see the decode path of one activation row
           if constexpr (BITS == 8) {
@@ -651,16 +758,28 @@ __device__ inline void block_step(const Loads<C>& cur, const uint8_t* smem, cons
           }
         }
     }
+    if constexpr (RC == 1) {
+      __builtin_amdgcn_sched_barrier(0);                            // (and not before the decode has done with its registers)
+      rec = fetch_rec(c);
+    }
     // the 128 columns of the chunk are complete: rows 4 kq .. 4 kq + 2 of the result are the three digit
     // sums of activation row 4g + kq
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
-      const float dl = x.delta[dm[g] * (x.NCH + 4) + chunk];        // 0 past the last chunk
+      // (every delta is 0 past the last chunk)
+      const float dl = BITS == 8 ? x.delta[(kq + 4 * g < x.M ? kq + 4 * g : 0) * (x.NCH + 4) + chunk] : 0.f;
 #pragma unroll
       for (int h = 0; h < NGC; ++h) {
-        const float f = digits_value<ND>(acc[g][h]);
-        const float dg = ND == 4 && NGC == 2 ? group_delta(dl, h) : dl;
-        ysum[4 * g + c] = fmaf(f, h2f((uint16_t)(zs[c][h] >> 8)) * dg, ysum[4 * g + c]);
+        float f, dg;
+        if constexpr (BITS == 8) {
+          f = digits_value<ND>(acc[g][h]);
+          dg = NGC == 2 ? group_delta(dl, h) : dl;
+        } else {
+          const int n = ((RC == 4 ? c : 0) * NG + g) * NGC + h;
+          f = group_value<C>(acc[g][h], row_lane(rec[0], n), row_lane(rec[1], n), zs[h] & 0xFFu);
+          dg = __int_as_float(row_lane(rec[2], n));
+        }
+        ysum[4 * g + c] = fmaf(f, h2f((uint16_t)(zs[h] >> 8)) * dg, ysum[4 * g + c]);
       }
     }
   }
@@ -711,7 +830,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
   float* red = delta + h.delta_cap;                    // [nslot][sk_cap][M][16] partial sums
 
   const int wr = lane & 15, kq = lane >> 4;            // weight row in tile / lane quarter
-  const uint32_t lane_off = table_lane<WT>(lane);
+  const uint32_t lane_off = table_lane<WT>(lane), bias = bias_register();
   // role of this lane's row in the A operand: variant i = lane%16 = 4 * quarter + digit
   // (digit 3 is an all-zero row where there are three); in the result, lane quarter kq holds the three digit sums
   // of its own chunk, so every lane post-processes exactly the chunk it decoded
@@ -756,13 +875,14 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
     // the rest of the set-up, which is a few hundred scalar instructions on the one scalar unit
     // the sixteen wavefronts share.
     const int n16 = Ns >> 4, xitems = h.M * n16;                  // a multiple of 8
+    const uint32_t recs = xq_off + (uint32_t)(h.M * ND * x_stride<QB>(Ns));   // LDS offset of the records, behind the digits
     // The first two items of a thread (all there are, but for the longest rows) are loaded here
     // and converted outside the loop further down: inside it the compiler's wait for an item's
     // loads has to allow for the trip in which they were issued after the weight loads, and so
     // waits for the weight loads as well; the conversion would start only once the first weights
     // have arrived instead of running while they are on their way.
     // (The second item only where its sixteen registers do not push the kernel into scratch.)
-    constexpr bool PRE2 = BITS != 8 && (MP == 1 || (MP == 4 && QB));
+    constexpr bool PRE2 = BITS != 8 && (MP == 1 || (MP == 4 && QB && GRP == 128 && !C::HI2)) && (C::DENSE || C::NL < 16);
     int xit = tid;
     XLoad xl, xl2;
     if (xit < xitems) stage_load(gm.x, gm.ldx, m.cs, N, col0, n16, xit, MP == 1, gm.par, xl);
@@ -842,15 +962,15 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
     if (!first) __syncthreads();                                  // previous matrix fully consumed
     first = false;
     constexpr int XORD = digit_order(BITS, C::DENSE);
-    if (xit < xitems) stage_convert<XORD, ND, ND == 4 && C::NGC == 2>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, xit, MP == 1, xq, delta, X_PAD);
+    if (xit < xitems) stage_convert<XORD, ND, ND == 4 && C::NGC == 2, ND == 4 ? 0 : GRP, QB>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, xit, MP == 1, xq, delta, X_PAD, smem + recs);
     if (PRE2 && xit + GV_THREADS < xitems)
-      stage_convert<XORD, ND, ND == 4 && C::NGC == 2>(xl2, m.cs != nullptr, h.xdt, N, ch0, n16, xit + GV_THREADS, MP == 1, xq, delta, X_PAD);
+      stage_convert<XORD, ND, ND == 4 && C::NGC == 2, ND == 4 ? 0 : GRP, QB>(xl2, m.cs != nullptr, h.xdt, N, ch0, n16, xit + GV_THREADS, MP == 1, xq, delta, X_PAD, smem + recs);
     for (xit += (PRE2 ? 2 : 1) * GV_THREADS; xit < xitems; xit += GV_THREADS) {
       stage_load(gm.x, gm.ldx, m.cs, N, col0, n16, xit, MP == 1, gm.par, xl);
-      stage_convert<XORD, ND, ND == 4 && C::NGC == 2>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, xit, MP == 1, xq, delta, X_PAD);
+      stage_convert<XORD, ND, ND == 4 && C::NGC == 2, ND == 4 ? 0 : GRP, QB>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, xit, MP == 1, xq, delta, X_PAD, smem + recs);
     }
     __syncthreads();
-
+    const int dlane = lane;
     int bars = 0;                                                 // group barriers passed so far
     float ysum[MP];
     auto do_step = [&](Loads<C>& cur, Loads<C>& tgt) {             // decode `cur`, load the next step into `tgt`
@@ -867,7 +987,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
       // the compiler no longer spreads them over the decode, and every launch was 2-6 % slower)
       issue(t_lo + p1.tl, p1.S, tgt);
       if constexpr (QB) {
-        block_step<C, BITS, NG, TURN, WT>(cur, smem, lut, lane_off, lane, S, XDigits{xq_off, z_off, delta, Ns, ch0, NCH, h.M}, ysum);
+        block_step<C, BITS, NG, TURN, WT>(cur, lane_off, bias, dlane, S, XDigits{xq_off, z_off, recs, delta, Ns, ch0, NCH, h.M}, ysum);
       } else
       {
         const int chunk = 4 * S + kq;
@@ -876,11 +996,11 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
 #pragma unroll
         for (int p = 0; p < MP; ++p) {
           const bool on = valid && a_slice == kq && a_dig < ND && p < h.M;
-          aaddr[p] = on ? xq_off + (uint32_t)((p * ND + a_dig) * (Ns + X_PAD) + (chunk - ch0) * 128) : z_off;
+          aaddr[p] = on ? xq_off + (uint32_t)((p * ND + a_dig) * x_stride<false>(Ns) + (chunk - ch0) * 128) : z_off;
         }
         // ---- bring the chunk's first code bit to bit 0 of cw[0]
         uint32_t cw[C::ND];
-        align_chunk_codes<C>(cur.raw, (uint32_t)(valid ? chunk : NCH - 1), cw);
+        gv_align_codes<C>(cur.raw, (uint32_t)(valid ? chunk : NCH - 1), cw);
 
         v4i acc[MP];
 #pragma unroll
@@ -888,22 +1008,21 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
 
 #pragma unroll
         for (int jb = 0; jb < 4; ++jb) {
-          uint32_t shc[4];
-          uint2 selc[4];
-          fetch_selectors<C, WT>(cur.mk[jb], lut, lane_off, shc, selc);
+          uint32_t taken = 0;
           uint32_t st[C::NW];                                     // code stream of block jb
-          block_stream<C, BITS>(cw, jb, st);
+          gv_block_stream<C, BITS>(cw, jb, st);
           const uint32_t z = (C::NGC == 1) ? cur.zraw : ((cur.zraw >> (8 * (jb >> 1))) & 0xFFu);
-          const uint32_t nz = 0x80808080u - z * 0x01010101u;
 #pragma unroll
           for (int half = 0; half < 2; ++half) {
             const int t = 2 * jb + half;                            // fragment index in the chunk
             uint32_t bfrag[4];
-            decode_half<C, BITS>(st, shc, selc, nz, half, bfrag, C::HI2 ? cur.h2[C::HI2 ? jb : 0] : 0u);
+            Sel sel[2];
+            fetch_selectors<C, WT>(cur.mk[jb], lane_off, half, sel);
+            decode_half<C, BITS>(st, taken, sel, zero_byte<C>(z), bias, half, bfrag, C::HI2 ? cur.h2[C::HI2 ? jb : 0] : 0u);
             const v4i bv = (v4i){(int)bfrag[0], (int)bfrag[1], (int)bfrag[2], (int)bfrag[3]};
 #pragma unroll
             for (int p = 0; p < MP; ++p) {
-              const v4i av = *(const v4i*)(smem + aaddr[p] + 16 * t);
+              const v4i av = lds_at<v4i>(aaddr[p] + 16 * t);
               acc[p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bv, acc[p], 0, 0, 0);
               // One idle issue slot after every MFMA.  Without it some instantiations of this
               // kernel (register allocations in which the accumulator chain changes registers)
@@ -924,9 +1043,17 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
               const int g = (C::NGC == 2 && t == 7) ? 1 : 0;
 #pragma unroll
               for (int p = 0; p < MP; ++p) {
-                const float dl = delta[(p < h.M ? p : 0) * (NCH + 4) + chunk];      // 0 past the last chunk
-                const float f = digits_value<ND>(acc[p]);
-                const float dg = ND == 4 && C::NGC == 2 ? group_delta(dl, g) : dl;
+                const int pr = p < h.M ? p : 0;                     // (every delta is 0 past the last chunk)
+                float f, dg;
+                if constexpr (BITS == 8) {
+                  const float dl = delta[pr * (NCH + 4) + chunk];
+                  f = digits_value<ND>(acc[p]);
+                  dg = C::NGC == 2 ? group_delta(dl, g) : dl;
+                } else {
+                  const v2u r = lds_at<v2u>(recs + (uint32_t)(pr * rec_stride(Ns, GRP) + (chunk - ch0) * C::NGC + g) * (uint32_t)REC_BYTES<false>);
+                  f = group_value<C>(acc[p], (int)r[0] >> 8, (int)(r[0] & 255u), (cur.zraw >> (8 * g)) & 0xFFu);
+                  dg = __uint_as_float(r[1]);
+                }
                 ysum[p] = fmaf(f, h2f((uint16_t)cur.sc[g]) * dg, ysum[p]);
                 acc[p] = (v4i){0, 0, 0, 0};
               }
@@ -957,6 +1084,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
         }
         if (gm.bias) v += (h.ydt == CBK_F32) ? ((const float*)gm.bias)[k]
                         : (h.ydt == CBK_F16) ? h2f(((const uint16_t*)gm.bias)[k]) : bf2f(((const uint16_t*)gm.bias)[k]);
+        asm volatile("" : "+v"(om));                                // (or its row's offset is kept in registers across the loop)
         const size_t o = (size_t)om * gm.ldy + k;
         if (h.ydt == CBK_F32) ((float*)gm.y)[o] = v;
         else if (h.ydt == CBK_F16) ((uint16_t*)gm.y)[o] = f2h(v);
@@ -1099,12 +1227,12 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
   if (tid < 256) {
   } else if (tid < 256 + ZERO_BYTES / 4) {
     ((uint32_t*)zreg)[tid - 256] = 0u;
-  } else if (tid < 256 + ZERO_BYTES / 4 + 4 * M) {                  // deltas of the chunks past N
+  } else if (BITS == 8 && tid < 256 + ZERO_BYTES / 4 + 4 * M) {     // deltas of the chunks past N
     const int i = tid - 256 - ZERO_BYTES / 4;
     delta[(i >> 2) * (NCH + 4) + NCH + (i & 3)] = 0.f;
   }
   const int wr = lane & 15, kq = lane >> 4;
-  const uint32_t lane_off = table_lane<WT>(lane);
+  const uint32_t lane_off = table_lane<WT>(lane), bias = bias_register();
   const uint32_t xq_off = (uint32_t)((uint8_t*)xq - smem), z_off = (uint32_t)(zreg - smem);
 
   // this workgroup: slab sl, tiles [T_lo, T_hi)
@@ -1156,16 +1284,19 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
   // ---- stage the slab's digits (the activation loads go out before the first weight loads)
   constexpr int XORD = digit_order(BITS, C::DENSE), ND = digits_of(BITS);
   const int n16 = Ns >> 4, xitems = M * n16;                        // a multiple of 8
+  const uint32_t recs = xq_off + (uint32_t)(M * ND * x_stride<true>(Ns));  // LDS offset of the records, behind the digits
   XLoad xl;
   if (tid < xitems) stage_load(gm.x, gm.ldx, m.cs, N, col0, n16, tid, false, gm.par, xl);
   Loads<C> LA, LB;
   issue(T_lo + p0.tl, p0.S, LA);
-  if (tid < xitems) stage_convert<XORD, ND, ND == 4 && C::NGC == 2>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, tid, false, xq, delta, X_PAD);
+  if (tid < xitems) stage_convert<XORD, ND, ND == 4 && C::NGC == 2, ND == 4 ? 0 : GRP, true>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, tid, false, xq, delta, X_PAD, smem + recs);
   for (int xit = tid + GV_THREADS; xit < xitems; xit += GV_THREADS) {
     stage_load(gm.x, gm.ldx, m.cs, N, col0, n16, xit, false, gm.par, xl);
-    stage_convert<XORD, ND, ND == 4 && C::NGC == 2>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, xit, false, xq, delta, X_PAD);
+    stage_convert<XORD, ND, ND == 4 && C::NGC == 2, ND == 4 ? 0 : GRP, true>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, xit, false, xq, delta, X_PAD, smem + recs);
   }
   __syncthreads();
+  int dlane = lane;                                                 // (as in the kernel above)
+  asm volatile("" : "+v"(dlane));
 
   float ysum[MP];
   auto do_step = [&](Loads<C>& cur, Loads<C>& tgt) {               // decode `cur`, load the next step into `tgt`
@@ -1177,7 +1308,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
       for (int p = 0; p < MP; ++p) ysum[p] = 0.f;
     }
     issue(T_lo + p1.tl, p1.S, tgt);
-    block_step<C, BITS, NG, TURN, WT>(cur, smem, smem, lane_off, lane, S, XDigits{xq_off, z_off, delta, Ns, ch0, NCH, M}, ysum);
+    block_step<C, BITS, NG, TURN, WT>(cur, lane_off, bias, dlane, S, XDigits{xq_off, z_off, recs, delta, Ns, ch0, NCH, M}, ysum);
     if (S + 1 == s_end) {
       // the part is done: lane quarter kq holds activation row 4g + kq of weight row wr
 #pragma unroll
@@ -2371,10 +2502,16 @@ constexpr size_t SPLIT_MIN_BYTES = 90 * 1024;  // digits of a row (M * 3 * N byt
 // 8-bit codes at five to eight rows are split from two million weights on: two buffers of 32 dwords beside the sums of
 // eight rows spill registers in the main kernel (us at eight rows, main / split: 512 x 1024 7.1 / 8.0, 2048 x 2048
 // 9.4 / 8.0, 4096 x 4096 17.5 / 10.3, 1024 x 16384 39 / 11).
-static inline size_t split_min_bytes(const DMat& m, int M) {
-  return m.bits == 8 && M > 4 && (size_t)m.K * m.N >= (2u << 20) ? 0 : SPLIT_MIN_BYTES;
-}
+// Five to eight rows of codes of up to six bits are split from SPLIT_MIN_BYTES_TALL on where the matrix has SPLIT_TALL to
+// SPLIT_TALL_MAX tiles of 16 rows: the second launch is hidden and the reduction slots matter (4-bit codes, 10 of 32, 4096 columns, us main / split:
+// 28672 rows 18.9 / 18.4 at six and 20.3 / 18.0 at seven, 14336 rows 14.8 / 13.5 and 15.1 / 13.7; 4096 rows 9.2 / 10.7).
+constexpr size_t SPLIT_MIN_BYTES_TALL = 70 * 1024;
+constexpr int SPLIT_TALL = 512, SPLIT_TALL_MAX = 2047;   // (from 2048 on the main kernel has several rounds of tiles)
 constexpr int SPLIT_MAX_TILES = 4096;          // (rows that fit are split only in launches of at most this many tiles)
+static inline size_t split_min_bytes(const DMat& m, int M) {
+  if (M > 4 && m.bits == 8) return (size_t)m.K * m.N >= (2u << 20) ? 0 : SPLIT_MIN_BYTES;
+  return M > 4 && m.K >= SPLIT_TALL * 16 && m.K <= SPLIT_TALL_MAX * 16 ? SPLIT_MIN_BYTES_TALL : SPLIT_MIN_BYTES;
+}
 static inline int kernel_rows(const DMat& m, int M) {            // activation rows as the kernel counts them, per pass
   const int v = m.cs_rows == 2 ? 2 : 1;
   return M * v > GV_MAX_M ? GV_MAX_M : M * v;
@@ -2383,13 +2520,12 @@ static inline int kernel_rows(const DMat& m, int M) {            // activation r
 size_t gemv_fast_workspace(const DMat& m, int M) {
   const int Mk = kernel_rows(m, M);
   if (Mk < 2) return 0;
-  const size_t digits = (size_t)Mk * digits_of(m.bits) * (m.N + X_PAD);
-  if (digits <= split_min_bytes(m, Mk)) return 0;
+  if (Mk * x_digit_bytes(m.bits, m.N) <= split_min_bytes(m, Mk)) return 0;
   // what a call with this matrix alone would do
   const int ntiles = (m.K + 15) / 16, nS = (m.N / 128 + 3) / 4;
   int spi, sk;
   row_parts(nS, launch_spi((long long)ntiles * nS, ntiles < 256 ? ntiles : 256, m.bits), spi, sk);
-  if (digits <= main_x_budget(Mk, Mk * (m.N / 128 + 4), sk) && ntiles > SPLIT_MAX_TILES) return 0;
+  if (Mk * x_row_bytes(m.bits, m.group, m.N, Mk) <= main_x_budget(Mk, delta_floats(m, Mk), sk) && ntiles > SPLIT_MAX_TILES) return 0;
   if (ntiles < 256) sk = nS < 16 ? nS : 16;                       // (in a batch a small matrix may be cut finer)
   return up256(split_part_bytes(ntiles + 3, sk, Mk));             // (+3: a q|k|v matrix is run as its three ranges)
 }
@@ -2523,7 +2659,7 @@ static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt,
   int delta_cap = 0;
   for (int i = 0; i < n; ++i) {
     total += (long long)mats[i].ntiles * mats[i].nS;
-    delta_cap = delta_cap > M * (mats[i].m.N / 128 + 4) ? delta_cap : M * (mats[i].m.N / 128 + 4);
+    delta_cap = delta_cap > delta_floats(mats[i].m, M) ? delta_cap : delta_floats(mats[i].m, M);
   }
   const int ND = digits_of(mats[0].m.bits);
   // The wide selector table, for all matrices of the launch or none: where a part of each still fits beside it and the
@@ -2535,7 +2671,8 @@ static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt,
   const DMat& m0 = mats[0].m;
   const size_t small = (size_t)LUT_BYTES + ZERO_BYTES + (size_t)delta_cap * 4 + (size_t)M * ND * X_PAD;
   bool wide = family_of(m0.layout) != FAM_DENSE && (2 * total >= 256 * GV_WAVES || m0.bits * m0.keep == BLOCK);
-  for (int i = 0; i < n; ++i) wide = wide && small + more + (size_t)M * ND * mats[i].spi * 512 <= 160 * 1024;
+  auto part_bytes = [&](const GvMat& g) { return M * (x_row_bytes(g.m.bits, g.m.group, g.spi * 512, M) - (size_t)ND * X_PAD); };
+  for (int i = 0; i < n; ++i) wide = wide && small + more + part_bytes(mats[i]) <= 160 * 1024;
   const size_t table = wide ? more : 0, fixed = small + table;
   int xq_cap = 0, wg = 0, th = 0;
   size_t off = 0;
@@ -2548,7 +2685,7 @@ static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt,
     // this matrix's share of the 256 workgroups
     int budget = (int)((long long)256 * g.ntiles * g.nS / total);
     budget = budget < 1 ? 1 : budget;
-    const size_t per_part = (size_t)M * ND * g.spi * 512;
+    const size_t per_part = part_bytes(g);
     if (fixed + per_part > 160 * 1024) return CBK_ERR_UNSUPPORTED;
     int pps_max = (int)((160 * 1024 - fixed) / per_part);
     pps_max = pps_max < g.sk ? pps_max : g.sk;
@@ -2574,7 +2711,8 @@ static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt,
     q.g.inv_sp = (uint32_t)((65536 + best_pps - 1) / best_pps);
     q.g.dq_t = GV_WAVES / best_pps; q.g.dq_p = GV_WAVES % best_pps;
     const int cols = best_pps * g.spi * 512 < g.m.N ? best_pps * g.spi * 512 : g.m.N;
-    xq_cap = xq_cap > M * ND * (cols + X_PAD) ? xq_cap : M * ND * (cols + X_PAD);
+    const int xb = M * (int)x_row_bytes(g.m.bits, g.m.group, cols, M);
+    xq_cap = xq_cap > xb ? xq_cap : xb;
     q.wg0 = wg; wg += q.nslab * q.wps; a.h.wg_end[i] = wg;
     q.th0 = th; th += (g.ntiles * M * 16 + GS_RED_THREADS - 1) / GS_RED_THREADS * GS_RED_THREADS; a.h.th_end[i] = th;
   }
@@ -2600,7 +2738,7 @@ static int launch_main_batch(GvBatch& gb, hipStream_t st, DecodeChoice* ask) {
     cost += g.ntiles * g.nS;
     gb.h.cost_end[i] = cost;
     tiles += g.ntiles;
-    delta_cap = delta_cap > M * (g.m.N / 128 + 4) ? delta_cap : M * (g.m.N / 128 + 4);
+    delta_cap = delta_cap > delta_floats(g.m, M) ? delta_cap : delta_floats(g.m, M);
     sk_cap = sk_cap > g.sk ? sk_cap : g.sk;
   }
   for (int i = n; i < GV_MAX_BATCH; ++i) gb.h.cost_end[i] = 0x7fffffff;
@@ -2619,14 +2757,16 @@ static int launch_main_batch(GvBatch& gb, hipStream_t st, DecodeChoice* ask) {
     GvMat& g = gb.mat[i];
     const int N = g.m.N;
     g.sp = g.sk;
-    if ((size_t)M * ND * (N + X_PAD) > x_budget) {
-      g.sp = (int)((x_budget - (size_t)M * ND * X_PAD) / ((size_t)M * ND * g.spi * 512));
+    // (one row: the digits alone count, as in gemv_fast_takes; its budget leaves room for their sums)
+    if ((M == 1 ? x_digit_bytes(g.m.bits, N) : M * x_row_bytes(g.m.bits, g.m.group, N, M)) > x_budget) {
+      g.sp = (int)((x_budget - (size_t)M * ND * X_PAD) / (M * (x_row_bytes(g.m.bits, g.m.group, g.spi * 512, M) - (size_t)ND * X_PAD)));
       if (g.sp < 1 || M == 1) return CBK_ERR_UNSUPPORTED;         // (the one-row kernels stage whole rows only)
       const int nsl = (g.sk + g.sp - 1) / g.sp;                   // slabs of equal length, not a short last one
       g.sp = (g.sk + nsl - 1) / nsl;
     }
     const int slab_cols = g.sp >= g.sk ? N : g.sp * g.spi * 512;
-    xq_cap = xq_cap > M * ND * (slab_cols + X_PAD) ? xq_cap : M * ND * (slab_cols + X_PAD);
+    const int xb = M * (int)x_row_bytes(g.m.bits, g.m.group, slab_cols, M);
+    xq_cap = xq_cap > xb ? xq_cap : xb;
     if (g.sp > g.sk) g.sp = g.sk;
     // exact for every a the kernel divides (a < cost + nS) when (cost + nS) * nS < 2^32
     g.inv_nS = g.nS > 1 && (uint64_t)(cost + g.nS) * g.nS < (1ull << 32) ? (uint32_t)(((1ull << 32) + g.nS - 1) / g.nS) : 0u;
@@ -2699,7 +2839,7 @@ int launch_gemv_fast_batch(int n, const GvCall* calls, int xdt, int M, int ydt, 
     g.ush = m.tiled ? 8 : 4; g.csh = m.tiled ? 4 : 0;
     cost += g.ntiles * g.nS;
     tiles += g.ntiles;
-    delta_cap = delta_cap > M * (m.N / 128 + 4) ? delta_cap : M * (m.N / 128 + 4);
+    delta_cap = delta_cap > delta_floats(m, M) ? delta_cap : delta_floats(m, M);
   }
   const int blocks = gemv_blocks(gb, n, tiles);
   // The parts depend on the matrices of the call only, not on M: they fix the order of every
@@ -2721,8 +2861,8 @@ int launch_gemv_fast_batch(int n, const GvCall* calls, int xdt, int M, int ydt, 
   if (M > 1) {
     const size_t x_budget = main_x_budget(M, delta_cap, sk_cap);
     auto splits = [&](const GvMat& g) {
-      const size_t digits = (size_t)M * digits_of(g.m.bits) * (g.m.N + X_PAD);
-      return digits > x_budget || (digits > split_min_bytes(g.m, M) && tiles <= SPLIT_MAX_TILES);
+      return M * x_row_bytes(g.m.bits, g.m.group, g.m.N, M) > x_budget ||
+             (M * x_digit_bytes(g.m.bits, g.m.N) > split_min_bytes(g.m, M) && tiles <= SPLIT_MAX_TILES);
     };
     GvMat split[GV_MAX_BATCH];
     int ns = 0;

@@ -605,6 +605,42 @@ def test_gemv_rows_do_not_depend_on_their_number(case):
                 assert torch.equal(ops.gemv(pm, x, out_dtype=torch.float32, workspace=small), one), (K, N, M, pm is rows)
 
 
+@pytest.mark.parametrize("case", [(F.BLK1632_4, 4, 128, 16), (F.BLK1632_6, 6, 128, 16), (F.DENSEB, 4, 64, 0)] + [
+    (F.BLKC, b, g, k) for b in (2, 3, 4) for k, g in ((10, 64), (16, 128), (23, 64), (23, 128))], ids=case_id)
+@pytest.mark.parametrize("N", [1024, 10240], ids=["small_table", "wide_table"])
+def test_gemv_zero_points_at_the_ends_of_their_range(case, N):
+    """A pruned column reads its zero point from the place of the eighth survivor, and the sums are put right from the digits'
+    own: mask bytes that keep all eight columns, none, and the survivors a block has left; zero points 0, the largest
+    code, 127 and 128; one to eight rows.  An activation is off by at most 2^-24 of its chunk's largest, and a sum of n float32
+    terms by n 2^-24 of their magnitudes (here fewer than 80)."""
+    layout, bits, group, keep = case
+    K, nl = 256, (1 << bits) - 1
+    rng = np.random.default_rng(N + bits)
+    mask = np.ones((K, N // 32, 32), bool)
+    if keep:                                                          # whole bytes first, in every order of the four; the rest in one byte
+        order = np.argsort(rng.random((K, N // 32, 4)), axis=2)
+        left = np.argsort(rng.random((K, N // 32, 8)), axis=2)
+        mask = np.zeros((K, N // 32, 4, 8), bool)
+        for i in range(4):
+            n = min(8, max(0, keep - 8 * i))
+            np.put_along_axis(mask, order[:, :, i:i + 1, None], (left < n)[:, :, None, :], axis=2)
+        mask = mask.reshape(K, N // 32, 32)
+        assert (mask.sum(2) == keep).all()
+    q = rng.integers(0, nl + 1, (K, N)).astype(np.uint8)
+    scale = (rng.random((K, N // group)) * 0.01 + 1e-3).astype(np.float16)
+    zero = rng.choice([0, nl, 127, 128], (K, N // group)).astype(np.float16)
+    pk = R.pack_matrix(R.pack_bits(mask.reshape(K, N)), q, scale, zero, layout, fix_zero=False, **kw_of(case))
+    W = R.dequant(pk, K, N, layout, **kw_of(case)).astype(np.float64)
+    pm = packed_from_oracle(case, pk, None, K, N, DEV, tiled=True)
+    x = acts(8, N, torch.float16, seed=N)
+    xd = x.double().numpy()
+    ref, mag = xd @ W.T, np.abs(xd) @ np.abs(W).T
+    bound = 2.0 ** -24 * (np.abs(xd).max(1)[:, None] * np.abs(W).sum(1)[None] + 80 * mag)
+    for M in (1, 2, 4, 8):
+        y = _np(ops.gemv(pm, x[:M].to(DEV), out_dtype=torch.float32)).astype(np.float64)
+        assert (np.abs(y - ref[:M]) <= bound[:M]).all(), (M, float((np.abs(y - ref[:M]) / bound[:M]).max()))
+
+
 EIGHT_BIT = [(F.DENSE8, 8, 128, 0), (F.DENSEB, 8, 64, 0), (F.DENSEB, 8, 128, 0)]
 
 
