@@ -643,7 +643,7 @@ GemmChoice gemm_choice(const cbk_desc* in, int M, int act) {
   return {p.kernel, p.ti, p.nsplit};
 }
 
-int decode_choice(int n, const cbk_desc* descs, int M, DecodeChoice* out) {
+int decode_choice(int n, const cbk_desc* descs, int M, bool room, DecodeChoice* out) {
   if (n < 1 || n > kMaxBatch || M < 1) return CBK_ERR_SHAPE;
   *out = DecodeChoice();
   GvCall c[kMaxBatch];
@@ -655,7 +655,7 @@ int decode_choice(int n, const cbk_desc* descs, int M, DecodeChoice* out) {
     c[i].ldx = c[i].m.N; c[i].ldy = c[i].m.K;
     if (!gemv_fast_takes(c[i].m, M * (c[i].par + 1)) || !gemv_same_config(c[0].m, c[i].m)) return CBK_ERR_UNSUPPORTED;
   }
-  return launch_gemv_fast_batch(n, c, CBK_F16, M, CBK_F32, (void*)256, (size_t)1 << 60, nullptr, out);
+  return launch_gemv_fast_batch(n, c, CBK_F16, M, CBK_F32, room ? (void*)256 : nullptr, room ? (size_t)1 << 60 : 0, nullptr, out);
 }
 
 void gemm_last_round(const cbk_desc* in, int M, const GemmChoice& c, int* row_tiles, int* ti) {

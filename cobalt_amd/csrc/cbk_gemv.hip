@@ -58,6 +58,11 @@ constexpr int LUT_LANES = CBK_LUT_LANES;      // lane-private copies of the sele
 constexpr int LUT_BYTES = 256 * LUT_LANES * 8;
 constexpr int WIDE_LUT_LANES = 16, WIDE_LUT_BYTES = 256 * WIDE_LUT_LANES * 16;   // see fetch_selectors
 constexpr int ZERO_BYTES = 128;               // a chunk of a digit row
+__host__ __device__ constexpr bool split_placed(int bits) { return bits != 8; }   // see x_stride
+// quarter-per-block, groups of 64: digits in column order want a macro-step of zeros (8-bit codes: one chunk, see block_step)
+__host__ __device__ constexpr int zero_bytes(int bits, int group, int rows, bool placed = false) {
+  return bits != 8 && group == 64 && rows > 2 && !placed ? 512 : ZERO_BYTES;
+}
 constexpr int CNT_SLOTS = 64;                 // most reduction slots (arrival counters)
 constexpr int CNT_BYTES = CNT_SLOTS * 4;       // at a fixed place: zeroed before the arguments are read
 constexpr int X_LDS_BUDGET = 112 * 1024;      // activation digits of one row: 3 (8-bit codes: 4) * columns bytes (of 160 KB LDS)
@@ -161,26 +166,33 @@ __host__ __device__ constexpr int digit_order(int bits, bool dense) { return !de
 struct XLoad { uint4 x[2], c[2]; };
 
 // What the end of a quantisation group reads of an activation row, three digits: the sum P of X = 65536 d2 + 256 d1 + d0 over the group
-// and the chunk's delta, [row][group of the slab], whole macro-steps (chunks past N: zeros).  Quarter-per-block: P as P >> 8 and P & 255, in
-// sixteen bytes.
-template <bool QB> constexpr int REC_BYTES = QB ? 16 : 8;
+// and the chunk's delta, [row][group of the slab], whole macro-steps (chunks past N: zeros).
+constexpr int REC_BYTES = 8;
 __host__ __device__ constexpr int rec_stride(int cols, int group) { return (cols / 128 + 3) / 4 * 4 * (128 / group); }
-// Bytes between two digit rows.  Linear order (quarter-per-chunk), or whole macro-steps of 512 columns in the order of the quarters 0, 2,
-// 1, 3 (quarter-per-block): a read of sixteen bytes goes through LDS in sets of sixteen lanes, 0-3 12-15 20-27 and so on, which
-// mix the quarters 0 and 1 or 2 and 3 of all twelve digit rows; 256 bytes apart, and rows 16 bytes off 256, no two of a set meet in a
-// bank (in linear order two did in every set: 72 of 264 LDS cycles of a step at eight rows).
-template <bool QB>
-__host__ __device__ constexpr int x_stride(int cols) { return (QB ? (cols + 511) / 512 * 512 : cols) + X_PAD; }
+// Bytes between two digit rows.  In column order, or PLACED (column-split kernel, codes of up to six bits): whole macro-steps of 512 columns
+// in the order of the quarters 0, 2, 1, 3.  A read of sixteen bytes goes through LDS in sets of sixteen lanes, 0-3 12-15 20-27 and so on,
+// which mix the quarters 0 and 1 or 2 and 3 of all twelve digit rows; 256 bytes apart, and rows 16 bytes off 256, no two of a set meet in a
+// bank (in column order two did in every set: 72 of 264 LDS cycles of a step at eight rows), but every two stores of a chunk do.  There it
+// gains (q,k,v of 5376 columns at eight rows 13.05 -> 12.6 us, larger matrices nothing).  The main kernel keeps column order: its rows are not
+// padded, so that all that fitted before there were records still fit, and fewer registers hold its addresses (placed: 98 more spilled over all
+// instantiations; at eight rows 28672 x 2816 dense 4-bit 15.2 us against 14.3, 4096 x 2304 4-bit keep 10 in groups of 64 10.6 against 9.8).
+template <bool PLACED>
+__host__ __device__ constexpr int x_stride(int cols) { return (PLACED ? (cols + 511) / 512 * 512 : cols) + X_PAD; }
 // offset of the sixteen columns c16 of a slab in a digit row
-template <bool QB>
+template <bool PLACED>
 __device__ inline int x_place(int c16) {
-  return QB ? (c16 >> 5) * 512 + (c16 & 2) * 128 + (c16 & 4) * 32 + (c16 & 24) * 4 + (c16 & 1) * 16 : c16 * 16;
+  return PLACED ? (c16 >> 5) * 512 + (c16 & 2) * 128 + (c16 & 4) * 32 + (c16 & 24) * 4 + (c16 & 1) * 16 : c16 * 16;
 }
 // LDS bytes of an activation row's digits, and what is set aside for them with the records, for `cols` columns (a multiple of 128)
-static inline size_t x_digit_bytes(int bits, int cols) { return (size_t)digits_of(bits) * (cols + X_PAD); }
-static inline size_t x_row_bytes(int bits, int group, int cols, int M) {
-  return digits_of(bits) * (size_t)(M == 1 ? x_stride<false>(cols) : x_stride<true>(cols)) +
-         (bits == 8 ? 0 : rec_stride(cols, group) * (M == 1 ? REC_BYTES<false> : REC_BYTES<true>));
+static inline size_t x_digit_bytes(int bits, int cols) { return (size_t)digits_of(bits) * x_stride<false>(cols); }
+static inline size_t x_rec_bytes(int bits, int group, int cols) { return bits == 8 ? 0 : (size_t)rec_stride(cols, group) * REC_BYTES; }
+static inline size_t x_row_bytes(int bits, int group, int cols) { return x_digit_bytes(bits, cols) + x_rec_bytes(bits, group, cols); }
+static inline size_t x_split_row_bytes(int bits, int group, int cols) {
+  return split_placed(bits) ? digits_of(bits) * (size_t)x_stride<true>(cols) + x_rec_bytes(bits, group, cols) : x_row_bytes(bits, group, cols);
+}
+// Reads of several rows in column order go on to the end of the last macro-step, over what follows (all of it meets a delta of 0)
+static inline size_t x_read_end(int bits, int cols, int M) {
+  return M * x_digit_bytes(bits, cols) - X_PAD + (size_t)(M > 1 ? (512 - cols % 512) % 512 : 0);
 }
 // 8-bit codes have their deltas alone, of all chunks of M rows: floats
 static inline int delta_floats(const DMat& m, int M) { return m.bits == 8 ? M * (m.N / 128 + 4) : 0; }
@@ -208,10 +220,10 @@ __device__ inline void stage_load(const uint16_t* x, int64_t ldx, const uint16_t
 // with the column scale are represented as they are, down to 2^-6 of it, and to 2^-30 of it below that.
 // HALVES (groups of 64): the delta of a chunk with infinities says which half has them, see group_delta.
 // SUMG (64 or 128, three digits only): the group size; what a group's end reads goes to `recs`, and nothing to `delta`.
-template <int ORDER, int ND = NDIG, bool HALVES = false, int SUMG = 0, bool QB = false>
+template <int ORDER, int ND = NDIG, bool HALVES = false, int SUMG = 0, bool QB = false, bool PLACED = false>
 __device__ inline void stage_convert(const XLoad& r, bool has_cs, int xdt, int N, int ch0, int n16, int it, bool one_row,
                                      int8_t* xq, float* delta, int pad = 0, void* recs = nullptr) {
-  const int NCH = N >> 7, Ns = QB ? x_stride<true>(n16 * 16) : n16 * 16 + pad;
+  const int NCH = N >> 7, Ns = PLACED ? x_stride<true>(n16 * 16) : n16 * 16 + pad;
   const int row = one_row ? 0 : it / n16, c16 = it - row * n16;
   const uint32_t* xw = (const uint32_t*)r.x;
   const uint32_t* cw = (const uint32_t*)r.c;
@@ -302,7 +314,7 @@ __device__ inline void stage_convert(const XLoad& r, bool has_cs, int xdt, int N
   }
 #pragma unroll
   for (int k = 0; k < ND; ++k)
-    *(uint4*)(xq + ((size_t)row * ND + k) * Ns + x_place<QB>(c16)) = make_uint4(dw[k][0], dw[k][1], dw[k][2], dw[k][3]);
+    *(uint4*)(xq + ((size_t)row * ND + k) * Ns + x_place<PLACED>(c16)) = make_uint4(dw[k][0], dw[k][1], dw[k][2], dw[k][3]);
   if constexpr (SUMG != 0) {                                        // |P| <= 128 * 127 * 65536 and a little
     static_assert(ND == 3, "three digits");
     constexpr int PG = SUMG / 16, NGC = 128 / SUMG;
@@ -311,10 +323,7 @@ __device__ inline void stage_convert(const XLoad& r, bool has_cs, int xdt, int N
     P += __builtin_amdgcn_mov_dpp(P, 0x4E, 0xF, 0xF, true);
     if (SUMG == 128) P += __builtin_amdgcn_mov_dpp(P, 0x141, 0xF, 0xF, true);
     const int rs = rec_stride(n16 * 16, SUMG), r0 = row * rs, past = rs - n16 / PG;
-    auto put = [&](int g, int p, float dl) {
-      if (QB) ((int4*)recs)[r0 + g] = make_int4(p >> 8, p & 255, __float_as_int(dl), 0);
-      else ((int2*)recs)[r0 + g] = make_int2(p, __float_as_int(dl));
-    };
+    auto put = [&](int g, int p, float dl) { ((int2*)recs)[r0 + g] = make_int2(p, __float_as_int(dl)); };
     if ((c16 & (PG - 1)) == 0) put(c16 / PG, P, d);
     if (past > 0 && c16 < past) put(n16 / PG + c16, 0, 0.f);
     return;
@@ -670,7 +679,7 @@ __device__ inline void load_chunk(const StepAt& p, int S4, int kq, Loads<C>& L) 
 // launches, 3-bit codes, 10 of 32 kept: 21504 x 5376 23.4 -> 21.3 us at M = 4, 45.6 -> 23.0 at M = 8; 5376 x 21504, rows
 // split by columns now, 35.2 -> 19.6 and 69.5 -> 21.4.)
 struct XDigits { uint32_t xq_off, z_off, rec_off; const float* delta; int Ns, ch0, NCH, M; };   // staged digits and what goes with them
-template <class C, int BITS, int NG, bool TURN, bool WT>
+template <class C, int BITS, int NG, bool TURN, bool WT, bool PLACED>
 __device__ inline void block_step(const Loads<C>& cur, uint32_t lane_off, uint32_t bias, int lane, int S,
                                   const XDigits& x, float (&ysum)[4 * NG]) {
   constexpr int NGC = C::NGC, ND = digits_of(BITS);
@@ -701,9 +710,10 @@ __device__ inline void block_step(const Loads<C>& cur, uint32_t lane_off, uint32
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
     const int am = a_m + 4 * g < x.M ? a_m + 4 * g : 0, ad = a_dig < ND ? a_dig : ND - 1;
-    const uint32_t a = x.xq_off + (uint32_t)((am * ND + ad) * x_stride<true>(x.Ns) + (kq & 1) * 256 + (kq >> 1) * 128) + (uint32_t)(4 * S - x.ch0) * 128u;
+    const uint32_t a = x.xq_off + (uint32_t)((am * ND + ad) * x_stride<PLACED>(x.Ns) + (PLACED ? (kq & 1) * 256 + (kq >> 1) * 128 : kq * 32)) +
+                       (uint32_t)(4 * S - x.ch0) * 128u;
 #pragma unroll
-    for (int h = 0; h < NGC; ++h) aaddr[g][h] = NGC == 1 || (kq >> 1) == h ? a : x.z_off;
+    for (int h = 0; h < NGC; ++h) aaddr[g][h] = NGC == 1 || BITS == 8 || (kq >> 1) == h ? a : x.z_off;
   }
   // The records of the step's groups: in the result lane quarter kq holds the three digit sums of activation rows 4g + kq, and lane n of
   // its sixteen fetches record n of (chunk, g, half).  Groups of 64 fetch those of a chunk when it ends, for want of registers.
@@ -711,7 +721,9 @@ __device__ inline void block_step(const Loads<C>& cur, uint32_t lane_off, uint32
   auto fetch_rec = [&](int c) -> v4i {
     if constexpr (BITS == 8) return v4i{0, 0, 0, 0};
     const int n = wr & (RC * NG * NGC - 1), g = NG == 2 ? (n / NGC) & 1 : 0, am = kq + 4 * g < x.M ? kq + 4 * g : 0;
-    return lds_at<v4i>(x.rec_off + (uint32_t)(am * rec_stride(x.Ns, 128 / NGC) + (4 * S - x.ch0 + n / (NG * NGC)) * NGC + n % NGC) * 16u + (uint32_t)(c * NGC * 16));
+    const v2u r = lds_at<v2u>(x.rec_off + (uint32_t)(am * rec_stride(x.Ns, 128 / NGC) + (4 * S - x.ch0 + n / (NG * NGC)) * NGC + n % NGC) * (uint32_t)REC_BYTES +
+                              (uint32_t)(c * NGC * REC_BYTES));
+    return v4i{(int)r[0] >> 8, (int)(r[0] & 255u), (int)r[1], 0};
   };
   v4i rec;
   if constexpr (RC == 4) rec = fetch_rec(0);
@@ -746,7 +758,9 @@ __device__ inline void block_step(const Loads<C>& cur, uint32_t lane_off, uint32
       for (int g = 0; g < NG; ++g)
 #pragma unroll
         for (int h = 0; h < NGC; ++h) {
-          const v4i av = lds_at<v4i>(aaddr[g][h] + 32 * c + 16 * half);
+          // (8-bit codes: one address and a selection; a second one kept is a register too many)
+          const uint32_t at = BITS == 8 && NGC == 2 ? ((kq >> 1) == h && chunk < x.NCH ? aaddr[g][0] + 128 * c : x.z_off) : aaddr[g][h] + (PLACED ? 32 : 128) * c;
+          const v4i av = lds_at<v4i>(at + 16 * half);
           acc[g][h] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bv, acc[g][h], 0, 0, 0);
           asm("s_nop 1" : "+v"(acc[g][h]));                         // see the decode path of one activation row
           if constexpr (BITS == 8) {
@@ -797,7 +811,8 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);     // in a scalar register: positions are scalar work
   uint8_t* lut = smem;
   uint8_t* zreg = smem + (WT ? WIDE_LUT_BYTES : LUT_BYTES);
-  int* cnt = (int*)(zreg + ZERO_BYTES);                // [CNT_SLOTS] arrival counters
+  constexpr int ZB = zero_bytes(BITS, GRP, MP);
+  int* cnt = (int*)(zreg + ZB);                        // [CNT_SLOTS] arrival counters
   int8_t* xq = (int8_t*)cnt + CNT_BYTES;
   // The argument block is read in two dependent steps (header, then the record of the first
   // matrix), each a round trip to memory for the first wavefronts that ask.  Touch its first
@@ -818,10 +833,10 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
     using C0 = Cfg<BITS, KEEP, GRP, MP>;
     build_table<C0, WT>(lut, tid);
     if (tid < 256) {
-    } else if (tid < 256 + ZERO_BYTES / 4) {
+    } else if (tid < 256 + ZB / 4) {
       ((uint32_t*)zreg)[tid - 256] = 0u;
-    } else if (tid < 256 + ZERO_BYTES / 4 + CNT_SLOTS) {
-      cnt[tid - 256 - ZERO_BYTES / 4] = 0;
+    } else if (tid < 256 + ZB / 4 + CNT_SLOTS) {
+      cnt[tid - 256 - ZB / 4] = 0;
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::"s"(ka[0]), "s"(ka[1]), "s"(ka[2]), "s"(ka[3]), "s"(ka[4]));
   }
@@ -875,7 +890,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
     // the rest of the set-up, which is a few hundred scalar instructions on the one scalar unit
     // the sixteen wavefronts share.
     const int n16 = Ns >> 4, xitems = h.M * n16;                  // a multiple of 8
-    const uint32_t recs = xq_off + (uint32_t)(h.M * ND * x_stride<QB>(Ns));   // LDS offset of the records, behind the digits
+    const uint32_t recs = xq_off + (uint32_t)(h.M * ND * x_stride<false>(Ns));   // LDS offset of the records, behind the digits
     // The first two items of a thread (all there are, but for the longest rows) are loaded here
     // and converted outside the loop further down: inside it the compiler's wait for an item's
     // loads has to allow for the trip in which they were issued after the weight loads, and so
@@ -970,7 +985,6 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
       stage_convert<XORD, ND, ND == 4 && C::NGC == 2, ND == 4 ? 0 : GRP, QB>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, xit, MP == 1, xq, delta, X_PAD, smem + recs);
     }
     __syncthreads();
-    const int dlane = lane;
     int bars = 0;                                                 // group barriers passed so far
     float ysum[MP];
     auto do_step = [&](Loads<C>& cur, Loads<C>& tgt) {             // decode `cur`, load the next step into `tgt`
@@ -987,7 +1001,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
       // the compiler no longer spreads them over the decode, and every launch was 2-6 % slower)
       issue(t_lo + p1.tl, p1.S, tgt);
       if constexpr (QB) {
-        block_step<C, BITS, NG, TURN, WT>(cur, lane_off, bias, dlane, S, XDigits{xq_off, z_off, recs, delta, Ns, ch0, NCH, h.M}, ysum);
+        block_step<C, BITS, NG, TURN, WT, false>(cur, lane_off, bias, lane, S, XDigits{xq_off, z_off, recs, delta, Ns, ch0, NCH, h.M}, ysum);
       } else
       {
         const int chunk = 4 * S + kq;
@@ -1050,7 +1064,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
                   f = digits_value<ND>(acc[p]);
                   dg = C::NGC == 2 ? group_delta(dl, g) : dl;
                 } else {
-                  const v2u r = lds_at<v2u>(recs + (uint32_t)(pr * rec_stride(Ns, GRP) + (chunk - ch0) * C::NGC + g) * (uint32_t)REC_BYTES<false>);
+                  const v2u r = lds_at<v2u>(recs + (uint32_t)(pr * rec_stride(Ns, GRP) + (chunk - ch0) * C::NGC + g) * (uint32_t)REC_BYTES);
                   f = group_value<C>(acc[p], (int)r[0] >> 8, (int)(r[0] & 255u), (cur.zraw >> (8 * g)) & 0xFFu);
                   dg = __uint_as_float(r[1]);
                 }
@@ -1211,7 +1225,8 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   uint8_t* zreg = smem + (WT ? WIDE_LUT_BYTES : LUT_BYTES);
-  int8_t* xq = (int8_t*)zreg + ZERO_BYTES;
+  constexpr int ZB = zero_bytes(BITS, GRP, MP, split_placed(BITS));
+  int8_t* xq = (int8_t*)zreg + ZB;
   const GsHead h = a.h;
   float* delta = (float*)(xq + h.xq_cap);
   // the matrix of this workgroup
@@ -1225,10 +1240,10 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
   const int M = h.M, N = m.N, NCH = N >> 7, nS = gm.nS, spi = gm.spi, SK = gm.sk;
   build_table<C, WT>(smem, tid);
   if (tid < 256) {
-  } else if (tid < 256 + ZERO_BYTES / 4) {
+  } else if (tid < 256 + ZB / 4) {
     ((uint32_t*)zreg)[tid - 256] = 0u;
-  } else if (BITS == 8 && tid < 256 + ZERO_BYTES / 4 + 4 * M) {     // deltas of the chunks past N
-    const int i = tid - 256 - ZERO_BYTES / 4;
+  } else if (BITS == 8 && tid < 256 + ZB / 4 + 4 * M) {             // deltas of the chunks past N
+    const int i = tid - 256 - ZB / 4;
     delta[(i >> 2) * (NCH + 4) + NCH + (i & 3)] = 0.f;
   }
   const int wr = lane & 15, kq = lane >> 4;
@@ -1283,16 +1298,17 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
 
   // ---- stage the slab's digits (the activation loads go out before the first weight loads)
   constexpr int XORD = digit_order(BITS, C::DENSE), ND = digits_of(BITS);
+  constexpr bool PLACED = split_placed(BITS);
   const int n16 = Ns >> 4, xitems = M * n16;                        // a multiple of 8
-  const uint32_t recs = xq_off + (uint32_t)(M * ND * x_stride<true>(Ns));  // LDS offset of the records, behind the digits
+  const uint32_t recs = xq_off + (uint32_t)(M * ND * x_stride<PLACED>(Ns));  // LDS offset of the records, behind the digits
   XLoad xl;
   if (tid < xitems) stage_load(gm.x, gm.ldx, m.cs, N, col0, n16, tid, false, gm.par, xl);
   Loads<C> LA, LB;
   issue(T_lo + p0.tl, p0.S, LA);
-  if (tid < xitems) stage_convert<XORD, ND, ND == 4 && C::NGC == 2, ND == 4 ? 0 : GRP, true>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, tid, false, xq, delta, X_PAD, smem + recs);
+  if (tid < xitems) stage_convert<XORD, ND, ND == 4 && C::NGC == 2, ND == 4 ? 0 : GRP, true, PLACED>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, tid, false, xq, delta, X_PAD, smem + recs);
   for (int xit = tid + GV_THREADS; xit < xitems; xit += GV_THREADS) {
     stage_load(gm.x, gm.ldx, m.cs, N, col0, n16, xit, false, gm.par, xl);
-    stage_convert<XORD, ND, ND == 4 && C::NGC == 2, ND == 4 ? 0 : GRP, true>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, xit, false, xq, delta, X_PAD, smem + recs);
+    stage_convert<XORD, ND, ND == 4 && C::NGC == 2, ND == 4 ? 0 : GRP, true, PLACED>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, xit, false, xq, delta, X_PAD, smem + recs);
   }
   __syncthreads();
   int dlane = lane;                                                 // (as in the kernel above)
@@ -1308,7 +1324,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
       for (int p = 0; p < MP; ++p) ysum[p] = 0.f;
     }
     issue(T_lo + p1.tl, p1.S, tgt);
-    block_step<C, BITS, NG, TURN, WT>(cur, lane_off, bias, dlane, S, XDigits{xq_off, z_off, recs, delta, Ns, ch0, NCH, M}, ysum);
+    block_step<C, BITS, NG, TURN, WT, PLACED>(cur, lane_off, bias, dlane, S, XDigits{xq_off, z_off, recs, delta, Ns, ch0, NCH, M}, ysum);
     if (S + 1 == s_end) {
       // the part is done: lane quarter kq holds activation row 4g + kq of weight row wr
 #pragma unroll
@@ -2487,9 +2503,9 @@ static inline void row_parts(int nS, int spi_launch, int& spi, int& sk) {
 }
 // LDS left for the activation digits of M rows beside the selector table, the deltas and two
 // reduction slots (up to 24 KB of slots where there is room)
-static inline size_t main_x_budget(int M, int delta_cap, int sk_cap) {
+static inline size_t main_x_budget(int M, const DMat& m, int delta_cap, int sk_cap) {
   const size_t slot_bytes = (size_t)sk_cap * M * 16 * 4;
-  const size_t fixed = (size_t)LUT_BYTES + ZERO_BYTES + CNT_BYTES + (size_t)delta_cap * 4;
+  const size_t fixed = (size_t)LUT_BYTES + zero_bytes(m.bits, m.group, M) + CNT_BYTES + (size_t)delta_cap * 4;
   const size_t red_floor = 2 * slot_bytes < 24 * 1024 ? 2 * slot_bytes : 24 * 1024;
   return 160 * 1024 - fixed - red_floor;
 }
@@ -2507,10 +2523,22 @@ constexpr size_t SPLIT_MIN_BYTES = 90 * 1024;  // digits of a row (M * 3 * N byt
 // 28672 rows 18.9 / 18.4 at six and 20.3 / 18.0 at seven, 14336 rows 14.8 / 13.5 and 15.1 / 13.7; 4096 rows 9.2 / 10.7).
 constexpr size_t SPLIT_MIN_BYTES_TALL = 70 * 1024;
 constexpr int SPLIT_TALL = 512, SPLIT_TALL_MAX = 2047;   // (from 2048 on the main kernel has several rounds of tiles)
-constexpr int SPLIT_MAX_TILES = 4096;          // (rows that fit are split only in launches of at most this many tiles)
+// Launches of more than SPLIT_MAX_TILES tiles: rows that fit are split where the layout has a bitmap and they take more than SPLIT_TALLEST_BYTES.
+// Split / main at 66000 to 262144 rows: eight activation rows of 5376 columns BLK1632_4 0.83 to 0.89, 4-bit keep 10 in groups of 64 0.71 to
+// 0.78, dense 4-bit 0.99 to 1.20; seven of 6144 0.97 to 0.98, 0.80 to 0.82 and 1.10; five of 8192 0.83 to 0.95 and 0.91 to 1.05; three of
+// 15360 0.53 to 0.85 and 1.04; two of 22528 0.91 to 1.02.  At 96 KB the main kernel wins (eight of 4096 1.01 to 1.13).  Between the two (eight
+// of 4608 and 4992 0.82 to 0.98) it is kept where it was.
+constexpr int SPLIT_MAX_TILES = 4096;
+constexpr size_t SPLIT_TALLEST_BYTES = 120 * 1024;
 static inline size_t split_min_bytes(const DMat& m, int M) {
   if (M > 4 && m.bits == 8) return (size_t)m.K * m.N >= (2u << 20) ? 0 : SPLIT_MIN_BYTES;
   return M > 4 && m.K >= SPLIT_TALL * 16 && m.K <= SPLIT_TALL_MAX * 16 ? SPLIT_MIN_BYTES_TALL : SPLIT_MIN_BYTES;
+}
+// whether the digits of M rows are split in a launch of `tiles` tiles where whole rows of them fit
+static inline bool split_pays(const DMat& m, int M, long long tiles) {
+  const size_t digits = M * x_digit_bytes(m.bits, m.N);
+  if (tiles > SPLIT_MAX_TILES) return m.bits != 8 && family_of(m.layout) != FAM_DENSE && digits > SPLIT_TALLEST_BYTES;
+  return digits > split_min_bytes(m, M);
 }
 static inline int kernel_rows(const DMat& m, int M) {            // activation rows as the kernel counts them, per pass
   const int v = m.cs_rows == 2 ? 2 : 1;
@@ -2520,12 +2548,11 @@ static inline int kernel_rows(const DMat& m, int M) {            // activation r
 size_t gemv_fast_workspace(const DMat& m, int M) {
   const int Mk = kernel_rows(m, M);
   if (Mk < 2) return 0;
-  if (Mk * x_digit_bytes(m.bits, m.N) <= split_min_bytes(m, Mk)) return 0;
   // what a call with this matrix alone would do
   const int ntiles = (m.K + 15) / 16, nS = (m.N / 128 + 3) / 4;
   int spi, sk;
   row_parts(nS, launch_spi((long long)ntiles * nS, ntiles < 256 ? ntiles : 256, m.bits), spi, sk);
-  if (Mk * x_row_bytes(m.bits, m.group, m.N, Mk) <= main_x_budget(Mk, delta_floats(m, Mk), sk) && ntiles > SPLIT_MAX_TILES) return 0;
+  if (Mk * x_row_bytes(m.bits, m.group, m.N) <= main_x_budget(Mk, m, delta_floats(m, Mk), sk) && !split_pays(m, Mk, ntiles)) return 0;
   if (ntiles < 256) sk = nS < 16 ? nS : 16;                       // (in a batch a small matrix may be cut finer)
   return up256(split_part_bytes(ntiles + 3, sk, Mk));             // (+3: a q|k|v matrix is run as its three ranges)
 }
@@ -2669,12 +2696,13 @@ static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt,
   // which gain at every size (1024 x 5376 9.6 / 9.2).  The slabs are the shorter for it.
   constexpr size_t more = WIDE_LUT_BYTES - LUT_BYTES;
   const DMat& m0 = mats[0].m;
-  const size_t small = (size_t)LUT_BYTES + ZERO_BYTES + (size_t)delta_cap * 4 + (size_t)M * ND * X_PAD;
+  const size_t zeros = zero_bytes(m0.bits, m0.group, M > 4 ? 8 : 4, split_placed(m0.bits));
+  const size_t small = (size_t)LUT_BYTES + zeros + (size_t)delta_cap * 4 + (size_t)M * ND * X_PAD;
   bool wide = family_of(m0.layout) != FAM_DENSE && (2 * total >= 256 * GV_WAVES || m0.bits * m0.keep == BLOCK);
-  auto part_bytes = [&](const GvMat& g) { return M * (x_row_bytes(g.m.bits, g.m.group, g.spi * 512, M) - (size_t)ND * X_PAD); };
+  auto part_bytes = [&](const GvMat& g) { return M * (x_split_row_bytes(g.m.bits, g.m.group, g.spi * 512) - (size_t)ND * X_PAD); };
   for (int i = 0; i < n; ++i) wide = wide && small + more + part_bytes(mats[i]) <= 160 * 1024;
   const size_t table = wide ? more : 0, fixed = small + table;
-  int xq_cap = 0, wg = 0, th = 0;
+  int xq_cap = 0, read_end = 0, wg = 0, th = 0;
   size_t off = 0;
   for (int i = 0; i < n; ++i) {
     GsMat& q = a.mat[i];
@@ -2711,14 +2739,16 @@ static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt,
     q.g.inv_sp = (uint32_t)((65536 + best_pps - 1) / best_pps);
     q.g.dq_t = GV_WAVES / best_pps; q.g.dq_p = GV_WAVES % best_pps;
     const int cols = best_pps * g.spi * 512 < g.m.N ? best_pps * g.spi * 512 : g.m.N;
-    const int xb = M * (int)x_row_bytes(g.m.bits, g.m.group, cols, M);
+    const int xb = M * (int)x_split_row_bytes(g.m.bits, g.m.group, cols);
+    if (!split_placed(g.m.bits) && (int)x_read_end(g.m.bits, cols, M) > read_end) read_end = (int)x_read_end(g.m.bits, cols, M);
     xq_cap = xq_cap > xb ? xq_cap : xb;
     q.wg0 = wg; wg += q.nslab * q.wps; a.h.wg_end[i] = wg;
     q.th0 = th; th += (g.ntiles * M * 16 + GS_RED_THREADS - 1) / GS_RED_THREADS * GS_RED_THREADS; a.h.th_end[i] = th;
   }
   for (int i = n; i < GV_MAX_BATCH; ++i) { a.h.wg_end[i] = 0x7fffffff; a.h.th_end[i] = 0x7fffffff; }
   a.h.xq_cap = xq_cap; a.h.delta_cap = delta_cap;
-  const size_t lds = (size_t)LUT_BYTES + table + ZERO_BYTES + xq_cap + (size_t)delta_cap * 4;
+  const size_t behind = xq_cap + (size_t)delta_cap * 4;
+  const size_t lds = LUT_BYTES + table + zeros + (behind > (size_t)read_end ? behind : (size_t)read_end);
   if (lds > 160 * 1024) return CBK_ERR_UNSUPPORTED;
   if (ask) { ask->split_table = wide ? 1 : 0; return CBK_OK; }
   const int bits = mats[0].m.bits, rb = th / GS_RED_THREADS;
@@ -2731,7 +2761,7 @@ static int launch_split_batch(const GvMat* mats, int n, int M, int xdt, int ydt,
 // Distribution over the workgroups, LDS and launch of the matrices of `gb` (spi and sk set).
 static int launch_main_batch(GvBatch& gb, hipStream_t st, DecodeChoice* ask) {
   const int n = gb.h.n, M = gb.h.M;
-  int cost = 0, tiles = 0, delta_cap = 0, sk_cap = 1, xq_cap = 0;
+  int cost = 0, tiles = 0, delta_cap = 0, sk_cap = 1, xq_cap = 0, read_end = 0;
   for (int i = 0; i < n; ++i) {
     GvMat& g = gb.mat[i];
     g.cost0 = cost;
@@ -2745,28 +2775,30 @@ static int launch_main_batch(GvBatch& gb, hipStream_t st, DecodeChoice* ask) {
   const int blocks = gemv_blocks(gb, n, tiles);
   // LDS: selector table, zero row and counters, the deltas, the reduction slots, and the activation
   // digits, which get what the others leave: at least two reduction slots are kept back (up to 24 KB
-  // of them where there is room), so that eight rows of 5376 columns (126 KB of digits) are still
-  // staged whole.  Rows whose digits do not fit are staged in column slabs: as many whole parts as the
+  // of them where there is room), so that eight rows of 5376 columns (126 KB of digits, 5.5 KB of
+  // records in groups of 64) are still staged whole.  Rows whose digits do not fit are staged in column slabs: as many whole parts as the
   // budget holds (a part is at most 8 steps = 4096 columns, 12 KB per activation row, so one part of
   // eight rows always fits).
   const size_t slot_bytes = (size_t)sk_cap * M * 16 * 4;
-  const size_t fixed = (size_t)LUT_BYTES + ZERO_BYTES + CNT_BYTES + (size_t)delta_cap * 4;
+  const DMat& m0 = gb.mat[0].m;
+  const size_t fixed = (size_t)LUT_BYTES + zero_bytes(m0.bits, m0.group, M) + CNT_BYTES + (size_t)delta_cap * 4;
   const int ND = digits_of(gb.mat[0].m.bits);
-  const size_t x_budget = M == 1 ? x_lds_budget(gb.mat[0].m.bits) : main_x_budget(M, delta_cap, sk_cap);
+  const size_t x_budget = M == 1 ? x_lds_budget(gb.mat[0].m.bits) : main_x_budget(M, m0, delta_cap, sk_cap);
   for (int i = 0; i < n; ++i) {
     GvMat& g = gb.mat[i];
     const int N = g.m.N;
     g.sp = g.sk;
     // (one row: the digits alone count, as in gemv_fast_takes; its budget leaves room for their sums)
-    if ((M == 1 ? x_digit_bytes(g.m.bits, N) : M * x_row_bytes(g.m.bits, g.m.group, N, M)) > x_budget) {
-      g.sp = (int)((x_budget - (size_t)M * ND * X_PAD) / (M * (x_row_bytes(g.m.bits, g.m.group, g.spi * 512, M) - (size_t)ND * X_PAD)));
+    if ((M == 1 ? x_digit_bytes(g.m.bits, N) : M * x_row_bytes(g.m.bits, g.m.group, N)) > x_budget) {
+      g.sp = (int)((x_budget - (size_t)M * ND * X_PAD) / (M * (x_row_bytes(g.m.bits, g.m.group, g.spi * 512) - (size_t)ND * X_PAD)));
       if (g.sp < 1 || M == 1) return CBK_ERR_UNSUPPORTED;         // (the one-row kernels stage whole rows only)
       const int nsl = (g.sk + g.sp - 1) / g.sp;                   // slabs of equal length, not a short last one
       g.sp = (g.sk + nsl - 1) / nsl;
     }
     const int slab_cols = g.sp >= g.sk ? N : g.sp * g.spi * 512;
-    const int xb = M * (int)x_row_bytes(g.m.bits, g.m.group, slab_cols, M);
+    const int xb = M * (int)x_row_bytes(g.m.bits, g.m.group, slab_cols), re = (int)x_read_end(g.m.bits, slab_cols, M);
     xq_cap = xq_cap > xb ? xq_cap : xb;
+    read_end = read_end > re ? read_end : re;
     if (g.sp > g.sk) g.sp = g.sk;
     // exact for every a the kernel divides (a < cost + nS) when (cost + nS) * nS < 2^32
     g.inv_nS = g.nS > 1 && (uint64_t)(cost + g.nS) * g.nS < (1ull << 32) ? (uint32_t)(((1ull << 32) + g.nS - 1) / g.nS) : 0u;
@@ -2800,9 +2832,17 @@ static int launch_main_batch(GvBatch& gb, hipStream_t st, DecodeChoice* ask) {
   const int nslot = wide ? wide_slots : small_slots;
   gb.h.sk_cap = sk_cap; gb.h.nslot = nslot; gb.h.red_floats = nslot * slot_floats;
   gb.h.cq = cost / blocks; gb.h.cr = cost % blocks;
-  const size_t lds = fixed + (wide ? more : 0) + xq_cap + (size_t)gb.h.red_floats * 4;
+  const size_t behind = xq_cap + (size_t)delta_cap * 4 + (size_t)gb.h.red_floats * 4;
+  const size_t lds = fixed - (size_t)delta_cap * 4 + (wide ? more : 0) + (behind > (size_t)read_end ? behind : (size_t)read_end);
   if (lds > 160 * 1024) return CBK_ERR_UNSUPPORTED;
-  if (ask) { ask->main_table = wide ? 1 : 0; ask->main_slots = nslot; return CBK_OK; }
+  if (ask) {
+    ask->main_table = wide ? 1 : 0; ask->main_slots = nslot;
+    for (int i = 0; i < n; ++i) {
+      const int nsl = (gb.mat[i].sk + gb.mat[i].sp - 1) / gb.mat[i].sp;
+      ask->main_slabs = ask->main_slabs > nsl ? ask->main_slabs : nsl;
+    }
+    return CBK_OK;
+  }
   const int bits = gb.mat[0].m.bits;
   if (bits == 6) return launch_mp<6, 16, 128>(gb, lds, blocks, wide, st);   // BLK1632_6: one configuration
   if (bits == 8) return launch_grp<8, 0>(gb, lds, blocks, false, st);
@@ -2853,16 +2893,14 @@ int launch_gemv_fast_batch(int n, const GvCall* calls, int xdt, int M, int ydt, 
   }
   // Matrices for the column-split kernel (one launch pair for all of them, behind the others),
   // where the caller has left room for the part sums: rows whose
-  // digits do not fit the staging area of the main kernel, and, in launches of at most
-  // SPLIT_MAX_TILES tiles, rows whose digits take more than SPLIT_MIN_BYTES of it (eight rows of
-  // 5376 columns: every workgroup of the main kernel converts all of them before its first step
+  // digits do not fit the staging area of the main kernel, and those of which split_pays says so
+  // (eight rows of 5376 columns: every workgroup of the main kernel converts all of them before its first step
   // and is left with four reduction slots; gate,up of that shape 43 us there, 30 + 5 us split).
   // Otherwise the main kernel stages long rows slab by slab.
   if (M > 1) {
-    const size_t x_budget = main_x_budget(M, delta_cap, sk_cap);
+    const size_t x_budget = main_x_budget(M, calls[0].m, delta_cap, sk_cap);
     auto splits = [&](const GvMat& g) {
-      return M * x_row_bytes(g.m.bits, g.m.group, g.m.N, M) > x_budget ||
-             (M * x_digit_bytes(g.m.bits, g.m.N) > split_min_bytes(g.m, M) && tiles <= SPLIT_MAX_TILES);
+      return M * x_row_bytes(g.m.bits, g.m.group, g.m.N) > x_budget || split_pays(g.m, M, tiles);
     };
     GvMat split[GV_MAX_BATCH];
     int ns = 0;

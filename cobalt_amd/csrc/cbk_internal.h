@@ -9,10 +9,11 @@ namespace cbk {
 // What cbk_gemv uses of a workspace at M rows (cbk_workspace_bytes covers every entry point).
 size_t decode_workspace_bytes(const cbk_desc*, int M);
 
-// What a decode call of M rows launches when it has a workspace: the selector table (0 the small one, 1 the wide one, -1:
-// no such launch) of the main and of the column-split kernel, and the main kernel's reduction slots.  For tests.
-struct DecodeChoice { int main_table = -1, main_slots = 0, split_table = -1; };
-int decode_choice(int n, const cbk_desc* descs, int M, DecodeChoice*);   // CBK_ERR_UNSUPPORTED: not in one pass of these kernels
+// What a decode call of M rows launches when it has a workspace, or none: the selector table (0 the small one, 1 the wide one, -1:
+// no such launch) of the main and of the column-split kernel, the main kernel's reduction slots, and the column slabs it stages a row in.
+// For tests.
+struct DecodeChoice { int main_table = -1, main_slots = 0, split_table = -1, main_slabs = 0; };
+int decode_choice(int n, const cbk_desc* descs, int M, bool room, DecodeChoice*);   // CBK_ERR_UNSUPPORTED: not in one pass of these kernels
 
 // How a prefill call runs, and the same call on a kernel, token tile and split of the columns that the caller
 // names: for tests, which have to know which of the instantiations they run.  kernel: 0 none of the two (cbk_linear in a gated

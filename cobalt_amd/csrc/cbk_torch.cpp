@@ -283,21 +283,31 @@ PyObject* py_linear_act(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
-// decode_choice([matrix], M) -> (table of the main kernel, its slots, table of the split kernel); see cbk::decode_choice
+// what a decode call of the matrices launches; see cbk::decode_choice
+cbk::DecodeChoice choice_of(PyObject* const* a, bool room) {
+  if (!PyList_Check(a[0]) || PyList_GET_SIZE(a[0]) < 1 || PyList_GET_SIZE(a[0]) > 8)
+    fail(PyExc_TypeError, "a list of one to eight matrices is expected");
+  const int k = (int)PyList_GET_SIZE(a[0]);
+  cbk_desc d[8];
+  for (int i = 0; i < k; ++i) d[i] = desc_of(as_matrix(PyList_GET_ITEM(a[0], i)));
+  const long M = PyLong_AsLong(a[1]);
+  if (PyErr_Occurred()) throw Fail{};
+  cbk::DecodeChoice c;
+  check(cbk::decode_choice(k, d, (int)M, room, &c), "cbk::decode_choice");
+  return c;
+}
+// decode_choice([matrix], M) -> (table of the main kernel, its slots, table of the split kernel)
 PyObject* py_decode_choice(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!arity(n, 2)) return nullptr;
   return guarded([&]() -> PyObject* {
-    if (!PyList_Check(a[0]) || PyList_GET_SIZE(a[0]) < 1 || PyList_GET_SIZE(a[0]) > 8)
-      fail(PyExc_TypeError, "a list of one to eight matrices is expected");
-    const int k = (int)PyList_GET_SIZE(a[0]);
-    cbk_desc d[8];
-    for (int i = 0; i < k; ++i) d[i] = desc_of(as_matrix(PyList_GET_ITEM(a[0], i)));
-    const long M = PyLong_AsLong(a[1]);
-    if (PyErr_Occurred()) throw Fail{};
-    cbk::DecodeChoice c;
-    check(cbk::decode_choice(k, d, (int)M, &c), "cbk::decode_choice");
+    const cbk::DecodeChoice c = choice_of(a, true);
     return Py_BuildValue("iii", c.main_table, c.main_slots, c.split_table);
   });
+}
+// decode_slabs([matrix], M) -> column slabs a row is staged in where there is no workspace (1: whole)
+PyObject* py_decode_slabs(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (!arity(n, 2)) return nullptr;
+  return guarded([&]() -> PyObject* { return PyLong_FromLong(choice_of(a, false).main_slabs); });
 }
 
 // gemm_plan(matrix, M, act or -1) -> (kernel, ti, nsplit); see cbk::gemm_choice
@@ -573,6 +583,7 @@ PyMethodDef methods[] = {
     {"linear_act", (PyCFunction)(void (*)())py_linear_act, METH_FASTCALL, nullptr},
     {"gemv_batch", (PyCFunction)(void (*)())py_gemv_batch, METH_FASTCALL, nullptr},
     {"decode_choice", (PyCFunction)(void (*)())py_decode_choice, METH_FASTCALL, nullptr},
+    {"decode_slabs", (PyCFunction)(void (*)())py_decode_slabs, METH_FASTCALL, nullptr},
     {"gemm_plan", (PyCFunction)(void (*)())py_gemm_plan, METH_FASTCALL, nullptr},
     {"gemm_column_parts", (PyCFunction)(void (*)())py_gemm_column_parts, METH_FASTCALL, nullptr},
     {"gemm_last_round", (PyCFunction)(void (*)())py_gemm_last_round, METH_FASTCALL, nullptr},

@@ -280,6 +280,29 @@ def test_selector_table_of_one_dword_blocks_and_of_dense_layouts():
     assert choice((F.BLKC, 2, 64, 10), 8192) == 1 and choice((F.DENSEB, 2, 64, None), 8192) == 0
 
 
+@pytest.mark.parametrize("K,N,case,M", [
+    # the longest rows of eight and seven activation rows beside the main kernel's table and two slots of sixteen, and of two, parts
+    (21504, 5376, (F.BLKC, 4, 64, 10), 8), (21504, 5376, (F.BLK1632_4, 4, 128, 16), 8), (262144, 5888, (F.BLK1632_4, 4, 128, 16), 8),
+    (262144, 6656, (F.BLK1632_4, 4, 128, 16), 7), (262144, 5760, (F.DENSEB, 3, 128, None), 8), (65536, 4352, (F.DENSEB, 8, 64, None), 8)])
+def test_rows_that_fit_are_staged_whole(K, N, case, M):
+    """Without a workspace a row whose digits do not fit in LDS is staged slab by slab, once per few tiles."""
+    assert _lib.native().decode_slabs([_sizes_only(K, N, case)], M) == 1
+    assert _lib.native().decode_slabs([_sizes_only(K, 2 * N, case)], M) > 1
+
+
+@pytest.mark.parametrize("case,K,N,M,split", [
+    ((F.BLKC, 4, 64, 10), 65552, 5248, 8, True), ((F.BLKC, 4, 64, 10), 65552, 5120 - 128, 8, False), ((F.BLK1632_4, 4, 128, 16), 262144, 5888, 8, True),
+    ((F.BLK1632_4, 4, 128, 16), 65552, 4096, 8, False), ((F.DENSEB, 3, 128, None), 262144, 5888, 8, False), ((F.DENSEB, 3, 128, None), 262144, 6016, 8, True)])
+def test_which_tall_matrices_are_split_by_columns(case, K, N, M, split):
+    """More than 4096 tiles: bitmap layouts above 120 KB of digits, dense ones where the rows do not fit; the workspace goes with it."""
+    h = _sizes_only(K, N, case)
+    assert (_lib.native().decode_choice([h], M)[0] < 0) == split
+    d = F.synth_packed(16, N, *case, seed=1).desc()
+    d.K = K
+    need = _lib.lib().cbk_workspace_bytes(ctypes.byref(d), M)
+    assert (need >= K * 2 * M * 4) == split
+
+
 def test_ops_refuse_to_run_without_gpu_tensors():
     from cobalt_amd import ops
     pm = F.synth_packed(16, 256, F.BLK1632_4, seed=1)
