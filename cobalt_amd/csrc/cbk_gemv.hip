@@ -678,8 +678,14 @@ __device__ inline void load_chunk(const StepAt& p, int S4, int kq, Loads<C>& L) 
 // mask, 12 to 24 of a step's ~ 350 instructions.  (A pass of quarter-per-chunk per row, five to eight rows in two
 // launches, 3-bit codes, 10 of 32 kept: 21504 x 5376 23.4 -> 21.3 us at M = 4, 45.6 -> 23.0 at M = 8; 5376 x 21504, rows
 // split by columns now, 35.2 -> 19.6 and 69.5 -> 21.4.)
+// The lane, from no register that would have to be kept for it
+__device__ inline int lane_anew() {
+  int l;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+  return l;
+}
 struct XDigits { uint32_t xq_off, z_off, rec_off; const float* delta; int Ns, ch0, NCH, M; };   // staged digits and what goes with them
-template <class C, int BITS, int NG, bool TURN, bool WT, bool PLACED>
+template <class C, int BITS, int NG, bool TURN, bool WT, bool PLACED, int RC>
 __device__ inline void block_step(const Loads<C>& cur, uint32_t lane_off, uint32_t bias, int lane, int S,
                                   const XDigits& x, float (&ysum)[4 * NG]) {
   constexpr int NGC = C::NGC, ND = digits_of(BITS);
@@ -716,8 +722,8 @@ __device__ inline void block_step(const Loads<C>& cur, uint32_t lane_off, uint32
     for (int h = 0; h < NGC; ++h) aaddr[g][h] = NGC == 1 || BITS == 8 || (kq >> 1) == h ? a : x.z_off;
   }
   // The records of the step's groups: in the result lane quarter kq holds the three digit sums of activation rows 4g + kq, and lane n of
-  // its sixteen fetches record n of (chunk, g, half).  Groups of 64 fetch those of a chunk when it ends, for want of registers.
-  constexpr int RC = NGC == 1 ? 4 : 1;                              // chunks at a time
+  // its sixteen fetches record n of (chunk, g, half), those of RC chunks at a time.
+  static_assert(RC * NG * NGC <= 16, "one record per lane");
   auto fetch_rec = [&](int c) -> v4i {
     if constexpr (BITS == 8) return v4i{0, 0, 0, 0};
     const int n = wr & (RC * NG * NGC - 1), g = NG == 2 ? (n / NGC) & 1 : 0, am = kq + 4 * g < x.M ? kq + 4 * g : 0;
@@ -772,10 +778,8 @@ __device__ inline void block_step(const Loads<C>& cur, uint32_t lane_off, uint32
           }
         }
     }
-    if constexpr (RC == 1) {
-      __builtin_amdgcn_sched_barrier(0);                            // (and not before the decode has done with its registers)
-      rec = fetch_rec(c);
-    }
+    if constexpr (RC == 1) __builtin_amdgcn_sched_barrier(0);       // (and not before the decode has done with its registers)
+    if (RC < 4 && (c & (RC - 1)) == 0) rec = fetch_rec(c);
     // the 128 columns of the chunk are complete: rows 4 kq .. 4 kq + 2 of the result are the three digit
     // sums of activation row 4g + kq
 #pragma unroll
@@ -789,7 +793,7 @@ __device__ inline void block_step(const Loads<C>& cur, uint32_t lane_off, uint32
           f = digits_value<ND>(acc[g][h]);
           dg = NGC == 2 ? group_delta(dl, h) : dl;
         } else {
-          const int n = ((RC == 4 ? c : 0) * NG + g) * NGC + h;
+          const int n = ((c & (RC - 1)) * NG + g) * NGC + h;
           f = group_value<C>(acc[g][h], row_lane(rec[0], n), row_lane(rec[1], n), zs[h] & 0xFFu);
           dg = __int_as_float(row_lane(rec[2], n));
         }
@@ -1001,7 +1005,12 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
       // the compiler no longer spreads them over the decode, and every launch was 2-6 % slower)
       issue(t_lo + p1.tl, p1.S, tgt);
       if constexpr (QB) {
-        block_step<C, BITS, NG, TURN, WT, false>(cur, lane_off, bias, lane, S, XDigits{xq_off, z_off, recs, delta, Ns, ch0, NCH, h.M}, ysum);
+        // Groups of 64 at five to eight rows are at the end of the registers: what follows from the lane is made anew in every step, and
+        // records are fetched for two chunks at a time (kept over the steps, and one at a time: 223 registers spilled over all
+        // instantiations against 93; 28672 x 2816 at eight rows, 4-bit keep 23 28.4 us against 21.4, keep 10 20.0 and 19.7).
+        constexpr bool TIGHT = MP == 8 && GRP == 64;
+        const int slane = TIGHT ? lane_anew() : lane;
+        block_step<C, BITS, NG, TURN, WT, false, TIGHT ? 2 : 4>(cur, lane_off, bias, slane, S, XDigits{xq_off, z_off, recs, delta, Ns, ch0, NCH, h.M}, ysum);
       } else
       {
         const int chunk = 4 * S + kq;
@@ -1267,8 +1276,12 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
   const uint32_t tile_a = gm.tile_a, lane_mul = gm.lane_mul, sz_mul = gm.sz_mul, code_u0 = m.code_off >> 4;
   const int last_S = nS - 1, last_tile = T_hi - 1;
 
+  // 8-bit codes in groups of 64, five to eight rows: two values of the lane were kept in scratch memory, and reading them back
+  // waited for the weights on their way (4096 x 14336 at six rows 27.0 us, 24.0 before there were records, 22.8 now)
+  constexpr bool TIGHT = BITS == 8 && GRP == 64 && MP == 8;
   // loads of one (tile, macro-step) position
   auto issue = [&](int tile, int S, Loads<C>& L) {
+    const int ln = TIGHT ? lane_anew() : lane, wr = ln & 15, kq = ln >> 4;
     tile = tile < last_tile ? tile : last_tile;
     S = S < last_S ? S : last_S;
     const int rlim = m_K - 1 - tile * 16;                           // rows past K repeat row K - 1
@@ -1311,8 +1324,6 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
     stage_convert<XORD, ND, ND == 4 && C::NGC == 2, ND == 4 ? 0 : GRP, true, PLACED>(xl, m.cs != nullptr, h.xdt, N, ch0, n16, xit, false, xq, delta, X_PAD, smem + recs);
   }
   __syncthreads();
-  int dlane = lane;                                                 // (as in the kernel above)
-  asm volatile("" : "+v"(dlane));
 
   float ysum[MP];
   auto do_step = [&](Loads<C>& cur, Loads<C>& tgt) {               // decode `cur`, load the next step into `tgt`
@@ -1324,7 +1335,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
       for (int p = 0; p < MP; ++p) ysum[p] = 0.f;
     }
     issue(T_lo + p1.tl, p1.S, tgt);
-    block_step<C, BITS, NG, TURN, WT, PLACED>(cur, lane_off, bias, dlane, S, XDigits{xq_off, z_off, recs, delta, Ns, ch0, NCH, M}, ysum);
+    block_step<C, BITS, NG, TURN, WT, PLACED, GRP == 64 ? 1 : 4>(cur, lane_off, bias, TIGHT ? lane_anew() : lane, S, XDigits{xq_off, z_off, recs, delta, Ns, ch0, NCH, M}, ysum);
     if (S + 1 == s_end) {
       // the part is done: lane quarter kq holds activation row 4g + kq of weight row wr
 #pragma unroll

@@ -238,3 +238,36 @@ def test_streams_of_three_dwords_are_shifted_on(loops):
     for (bits, keep, group, vectors, tile), n in vector.items():
         if keep == 23 and bits > 2:
             assert n - vector[bits, 16, group, vectors, tile] <= 8 * 30, (bits, group, vectors, tile)
+
+
+def decode_kernels(code_object):
+    """[(kernel, bits, group, rows, wide table, instructions, of those the blocks that have matrix instructions)] of the decode kernels."""
+    out = []
+    for fn, body in B._functions(code_object):
+        m = re.search(r"gemv_(mfma|split)_kernelILi(\d)ELi(\d+)ELi(\d+)ELi(\d)ELb(\d)", fn)
+        if not m:
+            continue
+        ops, steps, block = [b[1] for b in body], [], []
+        for op in ops:
+            block.append(op)
+            if op.startswith(("s_cbranch", "s_branch", "s_endpgm")):
+                if any(o.startswith("v_mfma") for o in block):
+                    steps.append(block)
+                block = []
+        out.append((m.group(1), *map(int, m.groups()[1:]), ops, steps))
+    return out
+
+
+@pytest.fixture(scope="module")
+def decoders():
+    if not os.path.exists(B.LIB):
+        pytest.skip("the library is not built")
+    return B._in_processes(decode_kernels, B.LIB)
+
+
+def test_decode_steps_keep_their_state_in_registers(decoders):
+    """A value of the loop that lies in scratch memory is read back behind the weights on their way, and waits for them."""
+    assert len(decoders) > 200
+    scratch = lambda ops: any(op.startswith("scratch_") for op in ops)
+    assert [d[:6] for d in decoders if any(map(scratch, d[7])) and (d[1] != 8 or d[0] == "split")] == []
+    assert [d[:6] for d in decoders if scratch(d[6]) and d[0] == "mfma" and d[1] != 8 and d[3] == 128] == []
