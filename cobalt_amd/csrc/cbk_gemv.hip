@@ -467,6 +467,18 @@ __device__ inline void gv_block_stream(const uint32_t (&cw)[C::ND], int jb, uint
     }
 }
 
+// Constants of a pool.  The bias in a register of its own: and-or with two literals is two instructions.  With the small table and up to four
+// rows the mask of the codes too: a literal of such an instruction is a scalar register, and launches of a step or two per wavefront pay for
+// scalars that are kept in lanes (3-bit keep 10, 1024 x 4096 at one row, 5.48 us against 5.39; with the wide table q,k,v of 5376 columns 8.0 against 7.87).
+struct PoolRegs { uint32_t bias, code; };
+template <class C, int BITS, bool REG>
+__device__ inline PoolRegs pool_regs() {
+  PoolRegs k{0x80808080u, C::SB == 2 ? 0x03030303u : BITS == 3 ? 0x07070707u : 0x0F0F0F0Fu};
+  asm("" : "+v"(k.bias));
+  if constexpr (REG) asm("" : "+v"(k.code));
+  return k;
+}
+
 // Sixteen columns (half `half` of the block whose code stream is st) as signed bytes, the B operand of one MFMA.  Dense
 // layouts: the codes.  Bitmap layouts: codes less 128, and in a pruned column the zero point less 128, which is put in the place of
 // the eighth survivor (`zero`: that byte, and what Pool<C>::BIAS is in the others).  So no weight has its zero point taken off: the
@@ -477,14 +489,14 @@ __device__ inline void gv_block_stream(const uint32_t (&cw)[C::ND], int jb, uint
 // to eight rows pays for the sums without a gain.
 // The stream is shifted on by what a byte's survivors took of it, so halves are decoded in order; `taken` is their sum (6-bit codes).
 template <class C, int BITS>
-__device__ inline void decode_half(uint32_t (&st)[C::NW], uint32_t& taken, const Sel (&sel)[2], uint32_t zero, uint32_t bias, int half,
+__device__ inline void decode_half(uint32_t (&st)[C::NW], uint32_t& taken, const Sel (&sel)[2], uint32_t zero, const PoolRegs& k, int half,
                                    uint32_t (&bfrag)[4], uint32_t hw = 0) {
   if constexpr (BITS == 8) {                             // q - 128; the zero point is a second operand (zero8)
 #pragma unroll
     for (int k = 0; k < 4; ++k) bfrag[k] = st[4 * half + k] ^ 0x80808080u;
     return;
   }
-  constexpr uint32_t CODE = C::SB == 2 ? 0x03030303u : BITS == 3 ? 0x07070707u : 0x0F0F0F0Fu;
+  const uint32_t CODE = k.code;
 #pragma unroll
   for (int jj2 = 0; jj2 < 2; ++jj2) {
     const int jj = 2 * half + jj2;                       // mask byte inside the block
@@ -500,10 +512,10 @@ __device__ inline void decode_half(uint32_t (&st)[C::NW], uint32_t& taken, const
         uint32_t h0, h1;
         hi2_pools(hw, jj == 0 ? 0u : taken / C::SB, h0, h1);
         taken = jj == 0 ? sel[0].bits : taken + sel[jj2].bits;
-        p0 = (w & CODE) | (h0 | bias);
-        p1 = ((w >> 4) & CODE) | (h1 | bias);
+        p0 = (w & CODE) | (h0 | k.bias);
+        p1 = ((w >> 4) & CODE) | (h1 | k.bias);
       } else {
-        p0 = (w & CODE) | bias;
+        p0 = (w & CODE) | k.bias;
         p1 = __builtin_amdgcn_alignbit(Pool<C>::BIAS >> 28, w, 4);
       }
       p1 = mask_select(sel[jj2].full, zero, p1);
@@ -545,13 +557,6 @@ __device__ inline int row_lane(int v, int n) {
     default: return __builtin_amdgcn_mov_dpp(v, 0x15F, 0xF, 0xF, true);
   }
 }
-// Pool<C>::BIAS in a register of its own: and-or with two literals is two instructions
-__device__ inline uint32_t bias_register() {
-  uint32_t b = 0x80808080u;
-  asm("" : "+v"(b));
-  return b;
-}
-
 // 8-bit codes: q - z needs nine bits, so the matrix instruction gets q - 128 and, in two more, the two halves of
 // 128 - z (-63 ... 64), into the same exact sums.  (The decode of such a fragment is four xors; sums of their own
 // for one constant z - 128 would take the registers that the second buffer of 32 dwords needs.)  On the row kernel below, a
@@ -685,8 +690,8 @@ __device__ inline int lane_anew() {
   return l;
 }
 struct XDigits { uint32_t xq_off, z_off, rec_off; const float* delta; int Ns, ch0, NCH, M; };   // staged digits and what goes with them
-template <class C, int BITS, int NG, bool TURN, bool WT, bool PLACED, int RC>
-__device__ inline void block_step(const Loads<C>& cur, uint32_t lane_off, uint32_t bias, int lane, int S,
+template <class C, int BITS, int NG, bool TURN, bool WT, bool PLACED, int RC, bool ZS_ALL>
+__device__ inline void block_step(const Loads<C>& cur, uint32_t lane_off, const PoolRegs& pool, int lane, int S,
                                   const XDigits& x, float (&ysum)[4 * NG]) {
   constexpr int NGC = C::NGC, ND = digits_of(BITS);
   const int wr = lane & 15, kq = lane >> 4;
@@ -707,9 +712,18 @@ __device__ inline void block_step(const Loads<C>& cur, uint32_t lane_off, uint32
     if (!C::DENSE) transpose4(mk4[0], mk4[1], mk4[2], mk4[3]);
     if (C::HI2) transpose4(hw4[0], hw4[1], hw4[2], hw4[3]);
   }
-  uint32_t own[NGC];                                                // zero | scale << 8 of the groups of chunk 4S + kq
+  // zero | scale << 8 of the groups of the step's chunks.  All of them at once where there are registers for it: a launch of one step per
+  // wavefront waits for four lane exchanges one after the other otherwise (4096 x 2304 at four rows, 7.1 us against 6.85).
+  uint32_t zall[4][NGC];
+  auto zs_of = [&](int c, int g) {
+    const uint32_t own = ((cur.zraw >> (8 * g)) & 0xFFu) | (cur.sc[g] << 8);      // of chunk 4S + kq
+    return (uint32_t)__shfl((int)own, wr + 16 * c, 64);
+  };
+  if constexpr (ZS_ALL)
 #pragma unroll
-  for (int g = 0; g < NGC; ++g) own[g] = ((cur.zraw >> (8 * g)) & 0xFFu) | (cur.sc[g] << 8);
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int g = 0; g < NGC; ++g) zall[c][g] = zs_of(c, g);
   // Row group g holds activation rows 4g .. 4g + 3: its A operand (for a digit or row there is not, any other: nothing reads those
   // rows of the result), in groups of 64 that of each half, zeros in the other two quarters
   uint32_t aaddr[NG][NGC];
@@ -738,7 +752,7 @@ __device__ inline void block_step(const Loads<C>& cur, uint32_t lane_off, uint32
     const int chunk = 4 * S + c;
     uint32_t zs[NGC];
 #pragma unroll
-    for (int g = 0; g < NGC; ++g) zs[g] = (uint32_t)__shfl((int)own[g], wr + 16 * c, 64);
+    for (int g = 0; g < NGC; ++g) zs[g] = ZS_ALL ? zall[c][g] : zs_of(c, g);
     uint32_t taken = 0;
     uint32_t st[C::NW];
 #pragma unroll
@@ -758,7 +772,7 @@ __device__ inline void block_step(const Loads<C>& cur, uint32_t lane_off, uint32
       uint32_t bfrag[4];
       Sel sel[2];
       fetch_selectors<C, WT>(TURN ? mk4[c] : cur.mk[c], lane_off, half, sel);
-      decode_half<C, BITS>(st, taken, sel, zero_byte<C>(z), bias, half, bfrag, TURN && C::HI2 ? hw4[c] : 0u);
+      decode_half<C, BITS>(st, taken, sel, zero_byte<C>(z), pool, half, bfrag, TURN && C::HI2 ? hw4[c] : 0u);
       const v4i bv = (v4i){(int)bfrag[0], (int)bfrag[1], (int)bfrag[2], (int)bfrag[3]};
 #pragma unroll
       for (int g = 0; g < NG; ++g)
@@ -849,7 +863,8 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
   float* red = delta + h.delta_cap;                    // [nslot][sk_cap][M][16] partial sums
 
   const int wr = lane & 15, kq = lane >> 4;            // weight row in tile / lane quarter
-  const uint32_t lane_off = table_lane<WT>(lane), bias = bias_register();
+  const uint32_t lane_off = table_lane<WT>(lane);
+  const PoolRegs pool = pool_regs<Cfg<BITS, KEEP, GRP, MP>, BITS, KEEP != 0 && !WT && MP <= 4>();
   // role of this lane's row in the A operand: variant i = lane%16 = 4 * quarter + digit
   // (digit 3 is an all-zero row where there are three); in the result, lane quarter kq holds the three digit sums
   // of its own chunk, so every lane post-processes exactly the chunk it decoded
@@ -1010,7 +1025,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
         // instantiations against 93; 28672 x 2816 at eight rows, 4-bit keep 23 28.4 us against 21.4, keep 10 20.0 and 19.7).
         constexpr bool TIGHT = MP == 8 && GRP == 64;
         const int slane = TIGHT ? lane_anew() : lane;
-        block_step<C, BITS, NG, TURN, WT, false, TIGHT ? 2 : 4>(cur, lane_off, bias, slane, S, XDigits{xq_off, z_off, recs, delta, Ns, ch0, NCH, h.M}, ysum);
+        block_step<C, BITS, NG, TURN, WT, false, TIGHT ? 2 : 4, BITS != 8 && !TIGHT>(cur, lane_off, pool, slane, S, XDigits{xq_off, z_off, recs, delta, Ns, ch0, NCH, h.M}, ysum);
       } else
       {
         const int chunk = 4 * S + kq;
@@ -1025,6 +1040,15 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
         uint32_t cw[C::ND];
         gv_align_codes<C>(cur.raw, (uint32_t)(valid ? chunk : NCH - 1), cw);
 
+        // (one row, groups of 64: the records with the step and not at a group's end, 1024 x 4096 2-bit 5.28 -> 5.16 us)
+        constexpr bool REC_FIRST = MP == 1 && C::NGC == 2 && BITS != 8;
+        auto rec_of = [&](int p, int g) {
+          return lds_at<v2u>(recs + (uint32_t)(p * rec_stride(Ns, GRP) + (chunk - ch0) * C::NGC + g) * (uint32_t)REC_BYTES);
+        };
+        v2u first_rec[C::NGC];
+        if constexpr (REC_FIRST)
+#pragma unroll
+          for (int g = 0; g < C::NGC; ++g) first_rec[g] = rec_of(0, g);
         v4i acc[MP];
 #pragma unroll
         for (int p = 0; p < MP; ++p) acc[p] = (v4i){0, 0, 0, 0};
@@ -1041,7 +1065,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
             uint32_t bfrag[4];
             Sel sel[2];
             fetch_selectors<C, WT>(cur.mk[jb], lane_off, half, sel);
-            decode_half<C, BITS>(st, taken, sel, zero_byte<C>(z), bias, half, bfrag, C::HI2 ? cur.h2[C::HI2 ? jb : 0] : 0u);
+            decode_half<C, BITS>(st, taken, sel, zero_byte<C>(z), pool, half, bfrag, C::HI2 ? cur.h2[C::HI2 ? jb : 0] : 0u);
             const v4i bv = (v4i){(int)bfrag[0], (int)bfrag[1], (int)bfrag[2], (int)bfrag[3]};
 #pragma unroll
             for (int p = 0; p < MP; ++p) {
@@ -1073,7 +1097,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
                   f = digits_value<ND>(acc[p]);
                   dg = C::NGC == 2 ? group_delta(dl, g) : dl;
                 } else {
-                  const v2u r = lds_at<v2u>(recs + (uint32_t)(pr * rec_stride(Ns, GRP) + (chunk - ch0) * C::NGC + g) * (uint32_t)REC_BYTES);
+                  const v2u r = REC_FIRST ? first_rec[g] : rec_of(pr, g);
                   f = group_value<C>(acc[p], (int)r[0] >> 8, (int)(r[0] & 255u), (cur.zraw >> (8 * g)) & 0xFFu);
                   dg = __uint_as_float(r[1]);
                 }
@@ -1107,7 +1131,9 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
         }
         if (gm.bias) v += (h.ydt == CBK_F32) ? ((const float*)gm.bias)[k]
                         : (h.ydt == CBK_F16) ? h2f(((const uint16_t*)gm.bias)[k]) : bf2f(((const uint16_t*)gm.bias)[k]);
-        asm volatile("" : "+v"(om));                                // (or its row's offset is kept in registers across the loop)
+        // (or its row's offset is kept in registers across the loop: groups of 64 spill, and with the wide table q,k,v of 5376 columns at
+        // one row take 8.0 us against 7.9; elsewhere it only makes the end of a launch longer, 1024 x 4096 at one row 5.06 against 4.93)
+        if constexpr (WT || (MP == 8 && GRP == 64) || BITS == 8) asm volatile("" : "+v"(om));
         const size_t o = (size_t)om * gm.ldy + k;
         if (h.ydt == CBK_F32) ((float*)gm.y)[o] = v;
         else if (h.ydt == CBK_F16) ((uint16_t*)gm.y)[o] = f2h(v);
@@ -1256,7 +1282,8 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
     delta[(i >> 2) * (NCH + 4) + NCH + (i & 3)] = 0.f;
   }
   const int wr = lane & 15, kq = lane >> 4;
-  const uint32_t lane_off = table_lane<WT>(lane), bias = bias_register();
+  const uint32_t lane_off = table_lane<WT>(lane);
+  const PoolRegs pool = pool_regs<C, BITS, false>();
   const uint32_t xq_off = (uint32_t)((uint8_t*)xq - smem), z_off = (uint32_t)(zreg - smem);
 
   // this workgroup: slab sl, tiles [T_lo, T_hi)
@@ -1335,7 +1362,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
       for (int p = 0; p < MP; ++p) ysum[p] = 0.f;
     }
     issue(T_lo + p1.tl, p1.S, tgt);
-    block_step<C, BITS, NG, TURN, WT, PLACED, GRP == 64 ? 1 : 4>(cur, lane_off, bias, TIGHT ? lane_anew() : lane, S, XDigits{xq_off, z_off, recs, delta, Ns, ch0, NCH, M}, ysum);
+    block_step<C, BITS, NG, TURN, WT, PLACED, GRP == 64 ? 1 : 4, BITS == 8 ? GRP == 64 && MP == 4 : GRP == 128 || MP == 4>(cur, lane_off, pool, TIGHT ? lane_anew() : lane, S, XDigits{xq_off, z_off, recs, delta, Ns, ch0, NCH, M}, ysum);
     if (S + 1 == s_end) {
       // the part is done: lane quarter kq holds activation row 4g + kq of weight row wr
 #pragma unroll

@@ -271,3 +271,10 @@ def test_decode_steps_keep_their_state_in_registers(decoders):
     scratch = lambda ops: any(op.startswith("scratch_") for op in ops)
     assert [d[:6] for d in decoders if any(map(scratch, d[7])) and (d[1] != 8 or d[0] == "split")] == []
     assert [d[:6] for d in decoders if scratch(d[6]) and d[0] == "mfma" and d[1] != 8 and d[3] == 128] == []
+
+
+def test_small_launches_end_without_spilled_scalars(decoders):
+    """One activation row, small table: a launch of a step or two per wavefront is as long as what stands before and after
+    them.  With more scalars spilled than there are here, every store of the end reads its pointers back from vector lanes."""
+    small = [d for d in decoders if d[0] == "mfma" and d[4] == 1 and not d[5] and d[1] in (2, 4) and d[2] in (10, 16)]
+    assert len(small) == 8 and max(d[6].count("v_readlane_b32") for d in small) <= 50
