@@ -16,7 +16,7 @@ int launch_gemv_fast_batch(int n, const GvCall* calls, int xdt, int M, int ydt, 
                            hipStream_t, DecodeChoice* ask = nullptr);
 bool gemv_fast_takes(const DMat&, int M);
 bool gemv_same_config(const DMat&, const DMat&);
-size_t gemv_fast_workspace(const DMat&, int M);
+size_t gemv_fast_workspace(const DMat&, int M, long long tiles);
 constexpr int kMaxBatch = 8;
 int launch_act_mul(const void* t, int tdt, int64_t ldt, void* y, int ydt, int64_t ldy, int M, int K2, int act,
                    const void* bias, hipStream_t st, bool halves = false);
@@ -257,18 +257,29 @@ static size_t gemm_workspace(const DMat& m, int M) {
   return need;
 }
 
+// 16-row tiles of a matrix, of each range by itself
+static long long matrix_tiles(const DMat& m) {
+  if (m.cs_rows != 3) return (m.K + 15) / 16;
+  int lo[3], hi[3], row[3];
+  const int nr = fused_ranges(m, lo, hi, row);
+  long long t = 0;
+  for (int i = 0; i < nr; ++i) t += (hi[i] - lo[i] + 15) / 16;
+  return t;
+}
+
 // Room for the part sums of cbk_gemv at M rows (see cbk_workspace_bytes); no other use of a
 // workspace in decode.  A q|k|v matrix runs as its ranges, one launch for all of them.
-static size_t decode_workspace(const DMat& m, int M) {
+// tiles: of the launch, all its matrices together.
+static size_t decode_workspace(const DMat& m, int M, long long tiles) {
   if (M < 1 || M > 16) return 0;
   if (family_of(m.layout) == FAM_SPARSE) return gemv_stream_workspace(m, M);
-  if (m.cs_rows != 3) return gemv_fast_takes(m, 1) ? gemv_fast_workspace(m, M) : 0;
+  if (m.cs_rows != 3) return gemv_fast_takes(m, 1) ? gemv_fast_workspace(m, M, tiles) : 0;
   int lo[3], hi[3], row[3];
   const int nr = fused_ranges(m, lo, hi, row);
   size_t need = 0;
   for (int i = 0; i < nr; ++i) {
     const DMat r = row_range(m, lo[i], hi[i], row[i]);
-    if (gemv_fast_takes(r, 1)) need += gemv_fast_workspace(r, M);
+    if (gemv_fast_takes(r, 1)) need += gemv_fast_workspace(r, M, tiles);
   }
   return need;
 }
@@ -277,7 +288,16 @@ static size_t decode_workspace(const DMat& m, int M) {
 // operators that know they will decode ask for this.
 size_t decode_workspace_bytes(const cbk_desc* in, int M) {
   DMat m;
-  return to_dmat(in, &m, false) ? 0 : decode_workspace(m, M);
+  return to_dmat(in, &m, false) ? 0 : decode_workspace(m, M, matrix_tiles(m));
+}
+
+size_t decode_batch_workspace_bytes(int n, const cbk_desc* descs, int M) {
+  long long tiles = 0;
+  DMat m;
+  for (int i = 0; i < n; ++i) tiles += to_dmat(descs + i, &m, false) ? 0 : matrix_tiles(m);
+  size_t need = 0;
+  for (int i = 0; i < n; ++i) need += to_dmat(descs + i, &m, false) ? 0 : decode_workspace(m, M, tiles);
+  return need;
 }
 
 int pack_image(const cbk_desc* dst, const void* mask_bits, const void* q, const void* scale, const void* zero,
@@ -335,7 +355,7 @@ size_t cbk_stream_bytes(const cbk_desc* in, size_t sparse_data_bytes) {
 
 // the most any of the three entry points asks for (cbk_gemm runs the prefill kernels at any M)
 static size_t workspace_of(const DMat& m, int M) {
-  const size_t a = decode_workspace(m, M), b = gemm_workspace(m, M);
+  const size_t a = decode_workspace(m, M, matrix_tiles(m)), b = gemm_workspace(m, M);
   return a > b ? a : b;
 }
 
@@ -347,7 +367,8 @@ size_t cbk_workspace_bytes(const cbk_desc* in, int M) {
 size_t cbk_gemv_batch_workspace_bytes(int n, const cbk_desc* descs, int M) {
   size_t total = 0;
   for (int i = 0; i < n; ++i) total += cbk_workspace_bytes(descs + i, M);
-  return total;
+  const size_t launch = decode_batch_workspace_bytes(n, descs, M);   // (a launch splits rows that a call of one of its matrices does not)
+  return total > launch ? total : launch;
 }
 
 int cbk_dequant(const cbk_desc* in, int row0, int nrows, int with_col_scale, void* out, int out_dtype,

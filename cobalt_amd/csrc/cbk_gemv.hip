@@ -2548,19 +2548,18 @@ static inline size_t main_x_budget(int M, const DMat& m, int delta_cap, int sk_c
   return 160 * 1024 - fixed - red_floor;
 }
 
-// Rows whose digits (M * 3 * N bytes) stay within SPLIT_MIN_BYTES need no workspace; longer ones (two
-// to eight activation rows) are split over the workgroups by
-// columns when the caller provides room for the part sums: [tiles][parts <= 16][M][16] floats.
-constexpr size_t SPLIT_MIN_BYTES = 90 * 1024;  // digits of a row (M * 3 * N bytes) from which it is split (measured on both layer sets
-                                               // at 56, 72, 90 and 112 KB: six rows of 5376 and eight of 4096 columns gain, seven of 4096 lose)
-// 8-bit codes at five to eight rows are split from two million weights on: two buffers of 32 dwords beside the sums of
-// eight rows spill registers in the main kernel (us at eight rows, main / split: 512 x 1024 7.1 / 8.0, 2048 x 2048
-// 9.4 / 8.0, 4096 x 4096 17.5 / 10.3, 1024 x 16384 39 / 11).
-// Five to eight rows of codes of up to six bits are split from SPLIT_MIN_BYTES_TALL on where the matrix has SPLIT_TALL to
-// SPLIT_TALL_MAX tiles of 16 rows: the second launch is hidden and the reduction slots matter (4-bit codes, 10 of 32, 4096 columns, us main / split:
-// 28672 rows 18.9 / 18.4 at six and 20.3 / 18.0 at seven, 14336 rows 14.8 / 13.5 and 15.1 / 13.7; 4096 rows 9.2 / 10.7).
+// Rows of two to eight activation rows whose digits (M * 3 * N bytes) take more than a limit are split over the workgroups by
+// columns when the caller provides room for the part sums: [tiles][parts <= 16][M][16] floats.  The limit is SPLIT_MIN_BYTES (measured
+// on both layer sets at 56, 72, 90 and 112 KB: six rows of 5376 and eight of 4096 columns gain), and for five to eight rows of codes of up to
+// six bits SPLIT_MIN_BYTES_TALL in launches of SPLIT_TALL to SPLIT_TALL_MAX tiles, all matrices together, if it would split all of them: a
+// batch is not broken up for it (one more launch pair).  Split / main over five formats, 70 to 80 KB (4736 to 5120 columns at five rows, 3968
+// and 4096 at six, 3456 to 3712 at seven, 3072 to 3200 at eight): 512 tiles 0.94 to 1.07, 688 0.81 to 1.02, 896 0.82 to 1.06, 1280 0.86 to
+// 1.01, 1792 0.93 to 1.06, 2047 0.88 to 1.08; above 80 KB 0.77 to 1.05.  So it gains between the ends (a seventh of the tiles of a workgroup
+// more or less is most of a round there) and little at them; at 60 to 67 KB the same heights are 0.88 to 1.13.  q,k,v of
+// 8192 + 1024 + 1024 rows and 4096 columns, 3-bit keep 10, us main / split: 17.5 / 12.7 at six rows, 19.6 / 13.0 at eight.
+constexpr size_t SPLIT_MIN_BYTES = 90 * 1024;
 constexpr size_t SPLIT_MIN_BYTES_TALL = 70 * 1024;
-constexpr int SPLIT_TALL = 512, SPLIT_TALL_MAX = 2047;   // (from 2048 on the main kernel has several rounds of tiles)
+constexpr int SPLIT_TALL = 512, SPLIT_TALL_MAX = 2047;
 // Launches of more than SPLIT_MAX_TILES tiles: rows that fit are split where the layout has a bitmap and they take more than SPLIT_TALLEST_BYTES.
 // Split / main at 66000 to 262144 rows: eight activation rows of 5376 columns BLK1632_4 0.83 to 0.89, 4-bit keep 10 in groups of 64 0.71 to
 // 0.78, dense 4-bit 0.99 to 1.20; seven of 6144 0.97 to 0.98, 0.80 to 0.82 and 1.10; five of 8192 0.83 to 0.95 and 0.91 to 1.05; three of
@@ -2568,29 +2567,34 @@ constexpr int SPLIT_TALL = 512, SPLIT_TALL_MAX = 2047;   // (from 2048 on the ma
 // of 4608 and 4992 0.82 to 0.98) it is kept where it was.
 constexpr int SPLIT_MAX_TILES = 4096;
 constexpr size_t SPLIT_TALLEST_BYTES = 120 * 1024;
-static inline size_t split_min_bytes(const DMat& m, int M) {
-  if (M > 4 && m.bits == 8) return (size_t)m.K * m.N >= (2u << 20) ? 0 : SPLIT_MIN_BYTES;
-  return M > 4 && m.K >= SPLIT_TALL * 16 && m.K <= SPLIT_TALL_MAX * 16 ? SPLIT_MIN_BYTES_TALL : SPLIT_MIN_BYTES;
+// 8-bit codes at five to eight rows are split from two million weights on: two buffers of 32 dwords beside the sums of
+// eight rows spill registers in the main kernel (us at eight rows, main / split: 512 x 1024 7.1 / 8.0, 2048 x 2048
+// 9.4 / 8.0, 4096 x 4096 17.5 / 10.3, 1024 x 16384 39 / 11).
+static inline bool split_tall(const DMat& m, int M, long long tiles) {      // the lower limit, for one matrix of a launch of `tiles` tiles
+  return M > 4 && m.bits != 8 && tiles >= SPLIT_TALL && tiles <= SPLIT_TALL_MAX && M * x_digit_bytes(m.bits, m.N) > SPLIT_MIN_BYTES_TALL;
 }
-// whether the digits of M rows are split in a launch of `tiles` tiles where whole rows of them fit
-static inline bool split_pays(const DMat& m, int M, long long tiles) {
+// whether the digits of M rows are split in a launch of `tiles` tiles where whole rows of them fit.  tall: split_tall of every matrix of it
+static inline bool split_pays(const DMat& m, int M, long long tiles, bool tall) {
   const size_t digits = M * x_digit_bytes(m.bits, m.N);
   if (tiles > SPLIT_MAX_TILES) return m.bits != 8 && family_of(m.layout) != FAM_DENSE && digits > SPLIT_TALLEST_BYTES;
-  return digits > split_min_bytes(m, M);
+  if (M > 4 && m.bits == 8 && (size_t)m.K * m.N >= (2u << 20)) return true;
+  return tall || digits > SPLIT_MIN_BYTES;
 }
 static inline int kernel_rows(const DMat& m, int M) {            // activation rows as the kernel counts them, per pass
   const int v = m.cs_rows == 2 ? 2 : 1;
   return M * v > GV_MAX_M ? GV_MAX_M : M * v;
 }
 
-size_t gemv_fast_workspace(const DMat& m, int M) {
+// What a matrix of a launch of `tiles` tiles may use at M activation rows
+size_t gemv_fast_workspace(const DMat& m, int M, long long tiles) {
   const int Mk = kernel_rows(m, M);
   if (Mk < 2) return 0;
-  // what a call with this matrix alone would do
+  // what a call with this matrix alone would do, or the launch
   const int ntiles = (m.K + 15) / 16, nS = (m.N / 128 + 3) / 4;
   int spi, sk;
   row_parts(nS, launch_spi((long long)ntiles * nS, ntiles < 256 ? ntiles : 256, m.bits), spi, sk);
-  if (Mk * x_row_bytes(m.bits, m.group, m.N) <= main_x_budget(Mk, m, delta_floats(m, Mk), sk) && !split_pays(m, Mk, ntiles)) return 0;
+  if (Mk * x_row_bytes(m.bits, m.group, m.N) <= main_x_budget(Mk, m, delta_floats(m, Mk), sk) && !split_pays(m, Mk, ntiles, split_tall(m, Mk, ntiles)) &&
+      !split_pays(m, Mk, tiles, split_tall(m, Mk, tiles))) return 0;
   if (ntiles < 256) sk = nS < 16 ? nS : 16;                       // (in a batch a small matrix may be cut finer)
   return up256(split_part_bytes(ntiles + 3, sk, Mk));             // (+3: a q|k|v matrix is run as its three ranges)
 }
@@ -2937,8 +2941,10 @@ int launch_gemv_fast_batch(int n, const GvCall* calls, int xdt, int M, int ydt, 
   // Otherwise the main kernel stages long rows slab by slab.
   if (M > 1) {
     const size_t x_budget = main_x_budget(M, calls[0].m, delta_cap, sk_cap);
+    bool tall = true;
+    for (int i = 0; i < n; ++i) tall = tall && split_tall(gb.mat[i].m, M, tiles);
     auto splits = [&](const GvMat& g) {
-      return M * x_row_bytes(g.m.bits, g.m.group, g.m.N) > x_budget || split_pays(g.m, M, tiles);
+      return M * x_row_bytes(g.m.bits, g.m.group, g.m.N) > x_budget || split_pays(g.m, M, tiles, tall);
     };
     GvMat split[GV_MAX_BATCH];
     int ns = 0;

@@ -8,6 +8,7 @@ namespace cbk {
 
 // What cbk_gemv uses of a workspace at M rows (cbk_workspace_bytes covers every entry point).
 size_t decode_workspace_bytes(const cbk_desc*, int M);
+size_t decode_batch_workspace_bytes(int n, const cbk_desc* descs, int M);   // and cbk_gemv_batch
 
 // What a decode call of M rows launches when it has a workspace, or none: the selector table (0 the small one, 1 the wide one, -1:
 // no such launch) of the main and of the column-split kernel, the main kernel's reduction slots, and the column slabs it stages a row in.

@@ -451,8 +451,8 @@ PyObject* py_gemv_batch(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         xp[i] = r[i].p; ldx[i] = r[i].ld;
         yp[i] = y[i].mutable_data_ptr(); ldy[i] = d[i].K;
         bp[i] = b[i].defined() ? b[i].const_data_ptr() : nullptr;
-        need += cbk::decode_workspace_bytes(&d[i], (int)r[0].M);
       }
+      need = cbk::decode_batch_workspace_bytes((int)n, d, (int)r[0].M);
       const c10::DeviceGuard guard(x[0].device());
       const at::Tensor ws = scratch(x[0], need);
       rc = cbk_gemv_batch((int)n, d, xp, ldx, xdt, (int)r[0].M, yp, ldy, ydt, bp,

@@ -280,6 +280,26 @@ def test_selector_table_of_one_dword_blocks_and_of_dense_layouts():
     assert choice((F.BLKC, 2, 64, 10), 8192) == 1 and choice((F.DENSEB, 2, 64, None), 8192) == 0
 
 
+@pytest.mark.parametrize("shapes,M,split", [
+    # both ends of the heights that have the lower limit, and of the limit; eight rows of 3072 columns take 72 KB
+    ([(8176, 4096)], 6, False), ([(8192, 4096)], 6, True), ([(32752, 4096)], 6, True), ([(32768, 4096)], 6, False),
+    ([(14336, 3840)], 6, False), ([(14336, 3968)], 6, True), ([(14336, 4096)], 4, False), ([(14336, 3072)], 8, True),
+    # matrices of unequal height go by the tiles of the launch, all one way; one that is not long enough keeps the others
+    ([(8192, 4096), (1024, 4096), (1024, 4096)], 6, True), ([(6144, 4096), (1024, 4096), (1008, 4096)], 6, False),
+    ([(6144, 4096), (1024, 4096), (1024, 4096)], 6, True), ([(8192, 5120), (1024, 5120), (1024, 5120)], 5, True),
+    ([(14336, 4096), (14336, 4096)], 6, True), ([(16384, 4096), (16384, 4096)], 6, False), ([(14336, 4096), (1024, 2048)], 6, False)])
+def test_a_launch_is_split_by_columns_as_a_whole(shapes, M, split):
+    h = [_sizes_only(K, N, (F.BLK1632_4, 4, 128, 16)) for K, N in shapes]
+    main, _, other = _lib.native().decode_choice(h, M)
+    assert (main < 0, other >= 0) == (split, split)
+    d = (type(F.synth_packed(16, 128, F.BLK1632_4, seed=1).desc()) * len(shapes))()
+    for i, (K, N) in enumerate(shapes):
+        d[i] = F.synth_packed(16, N, F.BLK1632_4, seed=1).desc()
+        d[i].K = K
+    parts = sum(K * 2 * M * 4 for K, _ in shapes)                   # two parts of a row at least
+    assert not split or _lib.lib().cbk_gemv_batch_workspace_bytes(len(shapes), d, M) >= parts
+
+
 @pytest.mark.parametrize("K,N,case,M", [
     # the longest rows of eight and seven activation rows beside the main kernel's table and two slots of sixteen, and of two, parts
     (21504, 5376, (F.BLKC, 4, 64, 10), 8), (21504, 5376, (F.BLK1632_4, 4, 128, 16), 8), (262144, 5888, (F.BLK1632_4, 4, 128, 16), 8),
