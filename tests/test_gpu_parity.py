@@ -641,6 +641,35 @@ def test_gemv_zero_points_at_the_ends_of_their_range(case, N):
         assert (np.abs(y - ref[:M]) <= bound[:M]).all(), (M, float((np.abs(y - ref[:M]) / bound[:M]).max()))
 
 
+@pytest.mark.parametrize("K,N,M,choice", [(2999, 5504, 8, (-1, 1)), (2975, 5504, 6, (-1, 0)), (8199, 5248, 4, (1, -1)), (1999, 3200, 8, (0, -1))],
+                         ids=["split_wide", "split_small", "main_wide", "main_small"])
+@pytest.mark.parametrize("case", [(F.BLK1632_4, 4, 128, 16), (F.BLK1632_6, 6, 128, 16), (F.DENSE4, 4, 128, None), (F.DENSEB, 3, 128, None),
+                                  (F.DENSEB, 2, 64, None)] + [
+    (F.BLKC, b, g, k) for b, g, k in ((3, 64, 10), (4, 64, 23), (4, 128, 23), (2, 64, 10), (3, 128, 16))], ids=case_id)
+def test_zero_points_in_both_kernels_with_both_tables(case, K, N, M, choice):
+    """Zero points at the ends of their range where several activation rows read them: either kernel, either selector table,
+    ragged heights, rows that end inside a macro-step.  An activation is off by at most 2^-24 of its chunk's largest; a group's
+    value is rounded four times, and a row adds N / group of them."""
+    layout, bits, group, keep = case
+    pm = F.synth_packed(K, N, layout, bits, group, keep, seed=N + bits, device=DEV)
+    ends = torch.tensor([0, (1 << bits) - 1, 127, 128], dtype=torch.uint8, device=DEV)
+    g = torch.Generator(device=DEV).manual_seed(K)
+    zero = pm.array("zero")
+    zero.copy_(ends[torch.randint(0, 4, zero.shape, generator=g, device=DEV)])
+    W = ops.dequant(pm, torch.float32, with_col_scale=False).double()
+    cs = pm.array("col_scale").double()
+    pm = pm.to_tiled()
+    dense = layout in F._DENSE
+    main, _, split = _lib.native().decode_choice([pm.native()], M)
+    assert (main, split) == (choice if not dense else tuple(min(c, 0) for c in choice)) or bits == 2 and keep == 16
+    x = acts(M, N, torch.float16, seed=N).to(DEV)
+    xs = x.double() * cs
+    ref, mag = xs @ W.T, xs.abs() @ W.abs().T
+    bound = 2.0 ** -24 * (xs.abs().amax(1)[:, None] * W.abs().sum(1)[None] + (N // group + 4) * mag)
+    y = ops.gemv(pm, x, out_dtype=torch.float32).double()
+    assert ((y - ref).abs() <= bound).all(), float(((y - ref).abs() / bound).max())
+
+
 EIGHT_BIT = [(F.DENSE8, 8, 128, 0), (F.DENSEB, 8, 64, 0), (F.DENSEB, 8, 128, 0)]
 
 
