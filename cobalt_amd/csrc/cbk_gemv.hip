@@ -488,7 +488,9 @@ __device__ inline PoolRegs pool_regs() {
 // 4096 x 14336 and the others of such a layer, see the table of calls); a matrix of a few steps per wavefront at five
 // to eight rows pays for the sums without a gain.
 // The stream is shifted on by what a byte's survivors took of it, so halves are decoded in order; `taken` is their sum (6-bit codes).
-template <class C, int BITS>
+// CHAIN off (6-bit codes with the small table, which counts no bits): windows at the ranks, which their high bits want anyway (1024 x 4096
+// at one row 5.87 -> 5.80 us).
+template <class C, int BITS, bool CHAIN>
 __device__ inline void decode_half(uint32_t (&st)[C::NW], uint32_t& taken, const Sel (&sel)[2], uint32_t zero, const PoolRegs& k, int half,
                                    uint32_t (&bfrag)[4], uint32_t hw = 0) {
   if constexpr (BITS == 8) {                             // q - 128; the zero point is a second operand (zero8)
@@ -505,7 +507,7 @@ __device__ inline void decode_half(uint32_t (&st)[C::NW], uint32_t& taken, const
       bfrag[2 * jj2] = w & CODE; bfrag[2 * jj2 + 1] = (w >> C::SB) & CODE;
     } else {
       // the pool: its second half's top byte has no code bits of a neighbour above rank 7
-      uint32_t w = st[0];
+      uint32_t w = CHAIN || jj == 0 ? st[0] : window<C::NW>(st, taken);
       if constexpr (C::SB == 2) { const uint32_t lo16 = w & 0xFFFFu; w = (lo16 << 14) | lo16; }
       uint32_t p0, p1;
       if constexpr (C::HI2) {
@@ -521,7 +523,7 @@ __device__ inline void decode_half(uint32_t (&st)[C::NW], uint32_t& taken, const
       p1 = mask_select(sel[jj2].full, zero, p1);
       bfrag[2 * jj2] = perm(p1, p0, sel[jj2].x);
       bfrag[2 * jj2 + 1] = perm(p1, p0, sel[jj2].y);
-      if (jj < 3) {                                      // past this byte's survivors
+      if (CHAIN && jj < 3) {                             // past this byte's survivors
         const uint32_t n = sel[jj2].bits;
         if constexpr (C::NW == 1) st[0] >>= n;
         else {
@@ -772,14 +774,14 @@ __device__ inline void block_step(const Loads<C>& cur, uint32_t lane_off, const 
       uint32_t bfrag[4];
       Sel sel[2];
       fetch_selectors<C, WT>(TURN ? mk4[c] : cur.mk[c], lane_off, half, sel);
-      decode_half<C, BITS>(st, taken, sel, zero_byte<C>(z), pool, half, bfrag, TURN && C::HI2 ? hw4[c] : 0u);
+      decode_half<C, BITS, WT || !C::HI2>(st, taken, sel, zero_byte<C>(z), pool, half, bfrag, TURN && C::HI2 ? hw4[c] : 0u);
       const v4i bv = (v4i){(int)bfrag[0], (int)bfrag[1], (int)bfrag[2], (int)bfrag[3]};
 #pragma unroll
       for (int g = 0; g < NG; ++g)
 #pragma unroll
         for (int h = 0; h < NGC; ++h) {
           // (8-bit codes: one address and a selection; a second one kept is a register too many)
-          const uint32_t at = BITS == 8 && NGC == 2 ? ((kq >> 1) == h && chunk < x.NCH ? aaddr[g][0] + 128 * c : x.z_off) : aaddr[g][h] + (PLACED ? 32 : 128) * c;
+          const uint32_t at = BITS == 8 && NGC == 2 ? ((kq >> 1) == h ? aaddr[g][0] + 128 * c : x.z_off) : aaddr[g][h] + (PLACED ? 32 : 128) * c;
           const v4i av = lds_at<v4i>(at + 16 * half);
           acc[g][h] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bv, acc[g][h], 0, 0, 0);
           asm("s_nop 1" : "+v"(acc[g][h]));                         // see the decode path of one activation row
@@ -1065,7 +1067,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
             uint32_t bfrag[4];
             Sel sel[2];
             fetch_selectors<C, WT>(cur.mk[jb], lane_off, half, sel);
-            decode_half<C, BITS>(st, taken, sel, zero_byte<C>(z), pool, half, bfrag, C::HI2 ? cur.h2[C::HI2 ? jb : 0] : 0u);
+            decode_half<C, BITS, WT || !C::HI2>(st, taken, sel, zero_byte<C>(z), pool, half, bfrag, C::HI2 ? cur.h2[C::HI2 ? jb : 0] : 0u);
             const v4i bv = (v4i){(int)bfrag[0], (int)bfrag[1], (int)bfrag[2], (int)bfrag[3]};
 #pragma unroll
             for (int p = 0; p < MP; ++p) {
@@ -1122,22 +1124,28 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
         }
         part_sum[p] = quarter_sum(ysum[p]);
       }
+      // One row: where an output goes is read again here, from the scalar cache.  Kept over the steps it took scalars that were then spilled to
+      // vector lanes, and a launch of a few steps per wavefront ends with reading them back (one row, us, kept / read again: 1024 x 4096
+      // BLK1632_4 4.97 / 4.87, 4-bit keep 10 5.18 / 4.99, keep 23 5.43 / 5.30; q,k,v of 5376 columns 8.0 / 7.25; several rows gain nothing).
+      int at_end = mi;
+      if constexpr (MP == 1) asm volatile("" : "+s"(at_end));
+      const GvMat& go = MP == 1 ? b.mat[at_end] : gm;
       auto store = [&](int om, int r, float v) {
         const int k = tile * 16 + r;
-        if (k >= m.K) return;
-        if (gm.par) {                                             // the sum scaled for the other parity is dropped
+        if (k >= go.m.K) return;
+        if (go.par) {                                             // the sum scaled for the other parity is dropped
           if ((om ^ k) & 1) return;
           om >>= 1;
         }
-        if (gm.bias) v += (h.ydt == CBK_F32) ? ((const float*)gm.bias)[k]
-                        : (h.ydt == CBK_F16) ? h2f(((const uint16_t*)gm.bias)[k]) : bf2f(((const uint16_t*)gm.bias)[k]);
+        if (go.bias) v += (h.ydt == CBK_F32) ? ((const float*)go.bias)[k]
+                        : (h.ydt == CBK_F16) ? h2f(((const uint16_t*)go.bias)[k]) : bf2f(((const uint16_t*)go.bias)[k]);
         // (or its row's offset is kept in registers across the loop: groups of 64 spill, and with the wide table q,k,v of 5376 columns at
         // one row take 8.0 us against 7.9; elsewhere it only makes the end of a launch longer, 1024 x 4096 at one row 5.06 against 4.93)
         if constexpr (WT || (MP == 8 && GRP == 64) || BITS == 8) asm volatile("" : "+v"(om));
-        const size_t o = (size_t)om * gm.ldy + k;
-        if (h.ydt == CBK_F32) ((float*)gm.y)[o] = v;
-        else if (h.ydt == CBK_F16) ((uint16_t*)gm.y)[o] = f2h(v);
-        else ((uint16_t*)gm.y)[o] = f2bf(v);
+        const size_t o = (size_t)om * go.ldy + k;
+        if (h.ydt == CBK_F32) ((float*)go.y)[o] = v;
+        else if (h.ydt == CBK_F16) ((uint16_t*)go.y)[o] = f2h(v);
+        else ((uint16_t*)go.y)[o] = f2bf(v);
       };
       if (SK == 1) {
         if (QB) {
@@ -1362,7 +1370,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_split_kernel(GsArgs a) {
       for (int p = 0; p < MP; ++p) ysum[p] = 0.f;
     }
     issue(T_lo + p1.tl, p1.S, tgt);
-    block_step<C, BITS, NG, TURN, WT, PLACED, GRP == 64 ? 1 : 4, BITS == 8 ? GRP == 64 && MP == 4 : GRP == 128 || MP == 4>(cur, lane_off, pool, TIGHT ? lane_anew() : lane, S, XDigits{xq_off, z_off, recs, delta, Ns, ch0, NCH, M}, ysum);
+    block_step<C, BITS, NG, TURN, WT, PLACED, GRP == 64 ? 1 : 4, BITS != 8 && (GRP == 128 || MP == 4)>(cur, lane_off, pool, TIGHT ? lane_anew() : lane, S, XDigits{xq_off, z_off, recs, delta, Ns, ch0, NCH, M}, ysum);
     if (S + 1 == s_end) {
       // the part is done: lane quarter kq holds activation row 4g + kq of weight row wr
 #pragma unroll
