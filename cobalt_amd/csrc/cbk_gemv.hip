@@ -1126,11 +1126,9 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
       }
       // One row: where an output goes is read again here, from the scalar cache.  Kept over the steps it took scalars that were then spilled to
       // vector lanes, and a launch of a few steps per wavefront ends with reading them back (one row, us, kept / read again: 1024 x 4096
-      // BLK1632_4 4.97 / 4.87, 4-bit keep 10 5.18 / 4.99, keep 23 5.43 / 5.30; q,k,v of 5376 columns 8.0 / 7.25; several rows gain nothing).
-      int at_end = mi;
-      if constexpr (MP == 1) asm volatile("" : "+s"(at_end));
-      const GvMat& go = MP == 1 ? b.mat[at_end] : gm;
-      auto store = [&](int om, int r, float v) {
+      // BLK1632_4 4.97 / 4.87, 4-bit keep 10 5.18 / 4.99, keep 23 5.43 / 5.30; q,k,v of 5376 columns 8.0 / 7.25; several rows gain nothing, and lose
+      // 1 to 3 % if their end so much as goes through the same reference: 4096 x 2304 at four rows 6.82 / 7.03).
+      auto store_at = [&](const GvMat& go, int om, int r, float v) {
         const int k = tile * 16 + r;
         if (k >= go.m.K) return;
         if (go.par) {                                             // the sum scaled for the other parity is dropped
@@ -1146,6 +1144,15 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_mfma_kernel(GvBatch b) {
         if (h.ydt == CBK_F32) ((float*)go.y)[o] = v;
         else if (h.ydt == CBK_F16) ((uint16_t*)go.y)[o] = f2h(v);
         else ((uint16_t*)go.y)[o] = f2bf(v);
+      };
+      auto store = [&](int om, int r, float v) {
+        if constexpr (MP == 1) {
+          int at_end = mi;
+          asm volatile("" : "+s"(at_end));
+          store_at(b.mat[at_end], om, r, v);
+        } else {
+          store_at(gm, om, r, v);
+        }
       };
       if (SK == 1) {
         if (QB) {

@@ -275,12 +275,13 @@ def test_decode_steps_keep_their_state_in_registers(decoders):
 
 def test_small_launches_end_without_spilled_scalars(decoders):
     """One activation row, small table: a launch of a step or two per wavefront is as long as what stands before and after
-    them.  With more scalars spilled than there are here, every store of the end reads its pointers back from vector lanes."""
+    them.  With more scalars spilled than there are here, every store of the end reads its pointers back from vector lanes:
+    130 reads and more in a kernel, 33 to 51 without."""
     small = [d for d in decoders if d[0] == "mfma" and d[4] == 1 and not d[5] and d[1] in (2, 4) and d[2] in (10, 16)]
-    assert len(small) == 8 and max(d[6].count("v_readlane_b32") for d in small) <= 50
+    assert len(small) == 8 and max(d[6].count("v_readlane_b32") for d in small) <= 64
 
 
 def test_small_launches_of_every_format_end_without_spilled_scalars(decoders):
     """The same of 3- and 6-bit codes, 23 of 32 kept and dense layouts: where an output goes is read from the arguments at the end."""
     small = [d for d in decoders if d[0] == "mfma" and d[4] == 1 and not d[5]]
-    assert len(small) > 25 and [d[:6] for d in small if d[6].count("v_readlane_b32") > 50] == []
+    assert len(small) > 25 and [d[:6] for d in small if d[6].count("v_readlane_b32") > 64] == []
