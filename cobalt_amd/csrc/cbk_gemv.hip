@@ -12,8 +12,9 @@
 // digits, see digits_of).  The
 // matrix core produces exact int32 dot products per (row, chunk, digit); one float FMA per
 // row and quantisation group applies scale * delta, after (128 - zero) times the sum of the group's
-// digits, integers too, has been added.  A pruned column's byte is the zero point's, so its two shares
-// cancel exactly and it contributes 0 whatever the zero point holds.
+// digits has been added: integers too, in two halves like the products, so nothing is lost before the
+// one conversion.  A pruned column's byte is the zero point's, so its two shares cancel exactly and it
+// contributes 0 whatever the zero point holds.
 //
 // Work decomposition.  A wavefront owns a tile of 16 weight rows; lane l works on row l%16
 // and on the 128-column chunk 4*S + l/16 of macro-step S (512 columns).  The four lane
@@ -66,9 +67,11 @@ __host__ __device__ constexpr int zero_bytes(int bits, int group, int rows, bool
 constexpr int CNT_SLOTS = 64;                 // most reduction slots (arrival counters)
 constexpr int CNT_BYTES = CNT_SLOTS * 4;       // at a fixed place: zeroed before the arguments are read
 constexpr int X_LDS_BUDGET = 112 * 1024;      // activation digits of one row: 3 (8-bit codes: 4) * columns bytes (of 160 KB LDS)
-constexpr int DELTA_LDS_BUDGET = 16 * 1024;   // one float per 128-column chunk and activation row (eight rows of 65024
-                                              // columns; the digits take what is left: a part of 4096 columns of
-                                              // eight rows, 96 KB, still fits beside 24 KB of reduction slots)
+constexpr int DELTA_LDS_BUDGET = 16 * 1024;   // longest rows of several activation rows, as the deltas of 8-bit codes: one float per
+                                              // 128-column chunk and activation row (eight rows of 65024 columns; the digits
+                                              // take what is left: a part of 4096 columns of eight rows, 96 KB, still fits
+                                              // beside 24 KB of reduction slots).  Codes of up to six bits have their deltas in the
+                                              // records of the columns that are staged, and the same limit.
 constexpr int NDIG = 3;                       // int8 digits per activation
 // 8-bit codes have four on the matrix-core kernels (the A operand has four rows per activation row anyway): some of
 // these layouts come from the float row kernel, and 24 bits below a chunk's largest activation lose more than it
@@ -2510,7 +2513,7 @@ bool gemv_fast_takes(const DMat& m, int M) {
   if (M < 1 || M > GV_MAX_M) return false;
   if (m.cs_rows == 3) return false;                              // the caller splits q|k|v into its ranges
   const int fam = family_of(m.layout);
-  // (q - z in a signed byte; 8-bit codes keep the zero point apart)
+  // (for zero points up to 128 the sums of a group are known to fit, see group_value; 8-bit codes keep the zero point apart)
   const bool dense8 = fam == FAM_DENSE && m.bits == 8;
   if (!(m.flags & CBK_FLAG_ZERO_LE_128) && !dense8) return false;
   // Row-major 8-bit rows stay on their row kernel, whose wavefront reads 2 KB of one row at a time: here sixteen rows
@@ -2523,8 +2526,8 @@ bool gemv_fast_takes(const DMat& m, int M) {
   // 32-bit offsets inside the kernel: every array of the matrix below 4 GB
   if ((uint64_t)((m.K + 15) / 16 * 16) * m.stride + 1024 >= (1ull << 32)) return false;
   if ((uint64_t)((m.K + 15) / 16 * 16) * m.G * 2 >= (1ull << 32)) return false;
-  // the digits are staged in column slabs where a whole row does not fit; the per-chunk deltas
-  // of all rows stay in LDS for the whole matrix
+  // the digits are staged in column slabs where a whole row does not fit; the per-chunk deltas of 8-bit codes
+  // stay in LDS for the whole matrix
   if (M == 1) return (size_t)digits_of(m.bits) * (m.N + X_PAD) <= x_lds_budget(m.bits);   // (the one-row kernels stage whole rows only)
   return (size_t)M * (m.N / 128 + 4) * 4 <= (size_t)DELTA_LDS_BUDGET;
 }
@@ -2554,12 +2557,17 @@ static inline void row_parts(int nS, int spi_launch, int& spi, int& sk) {
   spi = (nS + sk - 1) / sk;
   sk = (nS + spi - 1) / spi;
 }
-// LDS left for the activation digits of M rows beside the selector table, the deltas and two
-// reduction slots (up to 24 KB of slots where there is room)
+// LDS left for the activation digits of M rows beside the selector table, the deltas and the reduction slots: so many (a power of two) that
+// every wavefront can have a part of its own in them, two at least, up to 24 KB.  With fewer the wavefronts wait for each other: 21504 x 5376, 4-bit
+// keep 10 in groups of 64, eight rows without a workspace, whole rows beside two slots of six parts 43.8 us, in two slabs 32; 262144 x 5376,
+// BLK1632_4, whole rows beside four slots of two parts 253 us, eight 165 to 183.
 static inline size_t main_x_budget(int M, const DMat& m, int delta_cap, int sk_cap) {
   const size_t slot_bytes = (size_t)sk_cap * M * 16 * 4;
   const size_t fixed = (size_t)LUT_BYTES + zero_bytes(m.bits, m.group, M) + CNT_BYTES + (size_t)delta_cap * 4;
-  const size_t red_floor = 2 * slot_bytes < 24 * 1024 ? 2 * slot_bytes : 24 * 1024;
+  int slots = 2;
+  while (slots * sk_cap < GV_WAVES) slots <<= 1;
+  size_t red_floor = slots * slot_bytes;
+  if (red_floor > 24 * 1024) red_floor = 2 * slot_bytes < 24 * 1024 ? 2 * slot_bytes : 24 * 1024;
   return 160 * 1024 - fixed - red_floor;
 }
 
@@ -2575,24 +2583,26 @@ static inline size_t main_x_budget(int M, const DMat& m, int delta_cap, int sk_c
 constexpr size_t SPLIT_MIN_BYTES = 90 * 1024;
 constexpr size_t SPLIT_MIN_BYTES_TALL = 70 * 1024;
 constexpr int SPLIT_TALL = 512, SPLIT_TALL_MAX = 2047;
-// Launches of more than SPLIT_MAX_TILES tiles: rows that fit are split where the layout has a bitmap and they take more than SPLIT_TALLEST_BYTES.
-// Split / main at 66000 to 262144 rows: eight activation rows of 5376 columns BLK1632_4 0.83 to 0.89, 4-bit keep 10 in groups of 64 0.71 to
-// 0.78, dense 4-bit 0.99 to 1.20; seven of 6144 0.97 to 0.98, 0.80 to 0.82 and 1.10; five of 8192 0.83 to 0.95 and 0.91 to 1.05; three of
-// 15360 0.53 to 0.85 and 1.04; two of 22528 0.91 to 1.02.  At 96 KB the main kernel wins (eight of 4096 1.01 to 1.13).  Between the two (eight
-// of 4608 and 4992 0.82 to 0.98) it is kept where it was.
+// Launches of more than SPLIT_MAX_TILES tiles: rows that fit are split where they take more than SPLIT_TALLEST_BYTES, but those of
+// dense 4-bit codes and of 8-bit codes in groups of 128, which the main kernel reads nearly at the rate of the memory.  Split / main at 66000
+// to 262144 rows: eight activation rows of 5376 columns BLK1632_4 0.83 to 0.89, 4-bit keep 10 in groups of 64 0.71 to 0.78, dense 4-bit 0.99
+// to 1.20; eight of 5504 and 5632 dense 2-bit 0.76, 3-bit 0.88 to 0.93, 4-bit 1.03 to 1.11; seven of 6144 0.97 to 0.98, 0.80 to 0.82, dense 4-bit
+// 1.10; four of 8832 8-bit in groups of 64 0.87, of 128 1.05; three of 15360 0.53 to 0.85, dense 4-bit 1.04; two of 22528 0.91 to 1.02.
+// At 96 KB the main kernel wins (eight of 4096 1.01 to 1.13).  Between the two (eight of 4608 and 4992 0.82 to 0.98) it is kept where it was.
 constexpr int SPLIT_MAX_TILES = 4096;
 constexpr size_t SPLIT_TALLEST_BYTES = 120 * 1024;
 // 8-bit codes at five to eight rows are split from two million weights on: two buffers of 32 dwords beside the sums of
 // eight rows spill registers in the main kernel (us at eight rows, main / split: 512 x 1024 7.1 / 8.0, 2048 x 2048
-// 9.4 / 8.0, 4096 x 4096 17.5 / 10.3, 1024 x 16384 39 / 11).
+// 9.4 / 8.0, 4096 x 4096 17.5 / 10.3, 1024 x 16384 39 / 11; 65552 x 4352 in groups of 64 233 / 87).
 static inline bool split_tall(const DMat& m, int M, long long tiles) {      // the lower limit, for one matrix of a launch of `tiles` tiles
   return M > 4 && m.bits != 8 && tiles >= SPLIT_TALL && tiles <= SPLIT_TALL_MAX && M * x_digit_bytes(m.bits, m.N) > SPLIT_MIN_BYTES_TALL;
 }
 // whether the digits of M rows are split in a launch of `tiles` tiles where whole rows of them fit.  tall: split_tall of every matrix of it
 static inline bool split_pays(const DMat& m, int M, long long tiles, bool tall) {
   const size_t digits = M * x_digit_bytes(m.bits, m.N);
-  if (tiles > SPLIT_MAX_TILES) return m.bits != 8 && family_of(m.layout) != FAM_DENSE && digits > SPLIT_TALLEST_BYTES;
   if (M > 4 && m.bits == 8 && (size_t)m.K * m.N >= (2u << 20)) return true;
+  const bool read_bound = family_of(m.layout) == FAM_DENSE && (m.bits == 4 || (m.bits == 8 && m.group == 128));
+  if (tiles > SPLIT_MAX_TILES) return !read_bound && digits > SPLIT_TALLEST_BYTES;
   return tall || digits > SPLIT_MIN_BYTES;
 }
 static inline int kernel_rows(const DMat& m, int M) {            // activation rows as the kernel counts them, per pass
@@ -2831,11 +2841,10 @@ static int launch_main_batch(GvBatch& gb, hipStream_t st, DecodeChoice* ask) {
   for (int i = n; i < GV_MAX_BATCH; ++i) gb.h.cost_end[i] = 0x7fffffff;
   const int blocks = gemv_blocks(gb, n, tiles);
   // LDS: selector table, zero row and counters, the deltas, the reduction slots, and the activation
-  // digits, which get what the others leave: at least two reduction slots are kept back (up to 24 KB
-  // of them where there is room), so that eight rows of 5376 columns (126 KB of digits, 5.5 KB of
-  // records in groups of 64) are still staged whole.  Rows whose digits do not fit are staged in column slabs: as many whole parts as the
-  // budget holds (a part is at most 8 steps = 4096 columns, 12 KB per activation row, so one part of
-  // eight rows always fits).
+  // digits, which get what the others leave (main_x_budget): eight rows of 5376 columns (126 KB of digits, 2.75 KB of
+  // records, 5.5 in groups of 64) are still staged whole, in groups of 64 where a row has two parts only.  Rows
+  // whose digits do not fit are staged in column slabs: as many whole parts as the budget holds (a part is at most
+  // 8 steps = 4096 columns, 12 KB per activation row, so one part of eight rows always fits).
   const size_t slot_bytes = (size_t)sk_cap * M * 16 * 4;
   const DMat& m0 = gb.mat[0].m;
   const size_t fixed = (size_t)LUT_BYTES + zero_bytes(m0.bits, m0.group, M) + CNT_BYTES + (size_t)delta_cap * 4;
