@@ -139,8 +139,9 @@ size_t cbk_stream_bytes(const cbk_desc* d, size_t sparse_data_bytes);
  * when the library splits the column range of a launch that would not fill the chip.  A prefill call with
  * less is refused (CBK_ERR_WORKSPACE): its results do not depend on what it is given.  The decode
  * kernels need none, with one optional use:
- * two to eight activation rows of rows whose activations take more than 90 KB of LDS
- * (M * 3 * N bytes; 8-bit codes M * 4 * N) are split over the workgroups by columns when there is room for the float32
+ * two to eight activation rows of rows whose activations take more than 70 to 120 KB of LDS
+ * (M * 3 * N bytes, 8-bit codes M * 4 * N, the limit by the format and by the rows of the launch; 8-bit codes at
+ * five to eight rows: nearly all) are split over the workgroups by columns when there is room for the float32
  * part sums, K * 16 * M * 4 bytes at most, and so are the rows of SPARSE4X / SPARSE4E matrices on
  * the matrix-core stream kernel when the activation rows of a pass (up to eight) do not fit in
  * LDS as whole rows (M * 3 * N bytes beyond about 140 KB); with a smaller workspace, or none,
